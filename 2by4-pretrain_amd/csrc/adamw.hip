@@ -8,7 +8,9 @@
 //     m  = m * beta1 + (1 - beta1) * g
 //     v  = v * beta2 + ((1 - beta2) * g) * g
 //     p  = p + (-(lr / bc1)) * (m / (sqrt(v) / sqrt(bc2) + eps))
-// The gradient is only read.  Lane owns 4 consecutive elements (16-byte accesses of the float32
+// The gradient is only read.  One launch updates a whole list of tensors: a block owns kBlockElems consecutive
+// elements of one of them and finds it by a binary search of the list, which travels in the kernel arguments
+// (every step of the search is a scalar load).  Lane owns 4 consecutive elements (16-byte accesses of the float32
 // operands).
 #include "tf24_common.hpp"
 
@@ -45,15 +47,6 @@ __host__ __device__ inline AdamArgs adam_args(const AdamHyper& h, int64_t step) 
   return a;
 }
 
-// step_dev == nullptr: `a` holds the step's scalars; otherwise they are formed here from *step_dev
-__device__ __forceinline__ AdamArgs block_args(const AdamArgs& a, const AdamHyper& h, const int64_t* step_dev) {
-  if (!step_dev) return a;
-  __shared__ AdamArgs shared;
-  if (threadIdx.x == 0) shared = adam_args(h, *step_dev);
-  __syncthreads();
-  return shared;
-}
-
 __device__ __forceinline__ void adam_element(float& p, float g, float& m, float& v, bool decay, const AdamArgs& a) {
   if (decay) g = g + p * a.alpha;
   p = p * a.decay_mul;
@@ -63,103 +56,153 @@ __device__ __forceinline__ void adam_element(float& p, float g, float& m, float&
   p = p + a.neg_step_size * (m / denom);
 }
 
-template <typename G, typename M, bool HAS_MASK>
+constexpr int kBlockElems = kThreads * 4;
+constexpr int kMaxTensors = 56;         // 64 bytes each: the list and the scalars stay below the 4 KB of a launch's arguments
+
+struct AdamTensor {
+  float *p, *m, *v;
+  const void *grad, *mask;              // mask == nullptr: no decay
+  const int64_t* step;                  // step count in device memory, or nullptr: the launch's scalars hold
+  int64_t n;
+  uint32_t first_block;                 // blocks of the launch before this tensor's
+  uint32_t vec;                         // 16-byte accesses: every pointer is aligned for them
+};
+struct AdamList {
+  AdamTensor t[kMaxTensors];
+  int count;
+};
+
+// Bound by memory: 29 bytes per element (float32 gradient, byte mask).  24 weights of 3072 x 768 and their 24 biases,
+// 56.6 M elements: 254 us = 6.47 TB/s in one launch, against 16 us per weight (4.3 TB/s: too short to fill the memory
+// pipeline and drain it again) and 3.8 us per bias, 442 us in all, with a launch per tensor.  The moments and the
+// parameter are loaded AND stored with the streaming forms: ordinary accesses 295 us, streaming stores alone 295 us.
+// Two rounds of 1024 elements per block are slower (262 us).
+template <typename G, typename M>
 __global__ void __launch_bounds__(kThreads)
-adamw_vec(float* __restrict__ p, const G* __restrict__ grad, float* __restrict__ m, float* __restrict__ v,
-          const M* __restrict__ mask, int64_t n4, AdamArgs a_host, AdamHyper h, const int64_t* __restrict__ step_dev) {
-  const AdamArgs a = block_args(a_host, h, step_dev);
-  const int64_t u = (int64_t)blockIdx.x * kThreads + threadIdx.x;
-  if (u >= n4) return;
-  Pack<float, 4> pv, mv, vv;
-  Pack<G, 4> gv;
-  Pack<M, 4> mk;
-  pv.load(p + u * 4); mv.load(m + u * 4); vv.load(v + u * 4); gv.load_stream(grad + u * 4);
-  if constexpr (HAS_MASK) mk.load_stream(mask + u * 4);
+adamw_list(const AdamList list, const AdamArgs a_host, const AdamHyper h) {
+  int lo = 0, hi = list.count;          // the last tensor whose first_block is not behind this block
+  while (hi - lo > 1) {
+    const int mid = (lo + hi) >> 1;
+    if (list.t[mid].first_block <= blockIdx.x) lo = mid; else hi = mid;
+  }
+  const AdamTensor& t = list.t[lo];
+  AdamArgs a = a_host;
+  if (t.step) {                         // (uniform over the block)
+    __shared__ AdamArgs shared;
+    if (threadIdx.x == 0) shared = adam_args(h, *t.step);
+    __syncthreads();
+    a = shared;
+  }
+  const int64_t base = (int64_t)(blockIdx.x - t.first_block) * kBlockElems;
+  float* const p = t.p + base;
+  float* const m = t.m + base;
+  float* const v = t.v + base;
+  const G* const grad = (const G*)t.grad + base;
+  const M* const mask = t.mask ? (const M*)t.mask + base : nullptr;
+  const int64_t left = t.n - base;
+  if (t.vec && left >= kBlockElems) {
+    const int u = threadIdx.x * 4;
+    Pack<float, 4> pv, mv, vv;
+    Pack<G, 4> gv;
+    Pack<M, 4> mk;
+    pv.load_stream(p + u); mv.load_stream(m + u); vv.load_stream(v + u); gv.load_stream(grad + u);
+    if (mask) mk.load_stream(mask + u);
 #pragma unroll
-  for (int i = 0; i < 4; i++) {
-    bool decay = false;
-    if constexpr (HAS_MASK) decay = to_float(mk.v[i]) == 0.0f;
-    adam_element(pv.v[i], to_float(gv.v[i]), mv.v[i], vv.v[i], decay, a);
+    for (int i = 0; i < 4; i++) adam_element(pv.v[i], to_float(gv.v[i]), mv.v[i], vv.v[i], mask && to_float(mk.v[i]) == 0.0f, a);
+    pv.store_stream(p + u); mv.store_stream(m + u); vv.store_stream(v + u);
+  } else {                              // the last block of a tensor, or unaligned pointers
+    const int n = (int)(left < kBlockElems ? left : kBlockElems);
+    for (int i = threadIdx.x; i < n; i += kThreads) {
+      float pi = p[i], mi = m[i], vi = v[i];
+      adam_element(pi, to_float(grad[i]), mi, vi, mask && to_float(mask[i]) == 0.0f, a);
+      p[i] = pi; m[i] = mi; v[i] = vi;
+    }
   }
-  pv.store(p + u * 4); mv.store(m + u * 4); vv.store(v + u * 4);
 }
 
-template <typename G, typename M, bool HAS_MASK>
-__global__ void __launch_bounds__(kThreads)
-adamw_scalar(float* __restrict__ p, const G* __restrict__ grad, float* __restrict__ m, float* __restrict__ v,
-             const M* __restrict__ mask, int64_t begin, int64_t n, AdamArgs a_host, AdamHyper h, const int64_t* __restrict__ step_dev) {
-  const AdamArgs a = block_args(a_host, h, step_dev);
-  const int64_t i = begin + (int64_t)blockIdx.x * kThreads + threadIdx.x;
-  if (i >= n) return;
-  bool decay = false;
-  if constexpr (HAS_MASK) decay = to_float(mask[i]) == 0.0f;
-  float pi = p[i], mi = m[i], vi = v[i];
-  adam_element(pi, to_float(grad[i]), mi, vi, decay, a);
-  p[i] = pi; m[i] = mi; v[i] = vi;
-}
-
-template <typename G, typename M, bool HAS_MASK>
-int launch(float* p, const void* grad, float* m, float* v, const void* mask, int64_t n, const AdamArgs& a, const AdamHyper& h,
-           const int64_t* step_dev, hipStream_t s) {
-  const bool aligned = ((uintptr_t)p % 16 == 0) && ((uintptr_t)m % 16 == 0) && ((uintptr_t)v % 16 == 0) &&
-                       ((uintptr_t)grad % (4 * sizeof(G)) == 0) && (!HAS_MASK || (uintptr_t)mask % (4 * sizeof(M)) == 0);
-  const int64_t n4 = aligned ? n / 4 : 0;
-  if (n4 > 0) {
-    dim3 grid((unsigned)((n4 + kThreads - 1) / kThreads));
-    hipLaunchKernelGGL((adamw_vec<G, M, HAS_MASK>), grid, dim3(kThreads), 0, s, p, (const G*)grad, m, v, (const M*)mask, n4, a, h, step_dev);
+template <typename G, typename M>
+int launch(const char* fn, AdamList& list, const AdamArgs& a, const AdamHyper& h, hipStream_t s) {
+  int64_t blocks = 0;
+  for (int i = 0; i < list.count; i++) {
+    AdamTensor& t = list.t[i];
+    t.first_block = (uint32_t)blocks;
+    t.vec = (uintptr_t)t.p % 16 == 0 && (uintptr_t)t.m % 16 == 0 && (uintptr_t)t.v % 16 == 0 &&
+            (uintptr_t)t.grad % (4 * sizeof(G)) == 0 && (uintptr_t)t.mask % (4 * sizeof(M)) == 0;
+    blocks += (t.n + kBlockElems - 1) / kBlockElems;
   }
-  const int64_t begin = n4 * 4;
-  if (begin < n) {
-    dim3 grid((unsigned)((n - begin + kThreads - 1) / kThreads));
-    hipLaunchKernelGGL((adamw_scalar<G, M, HAS_MASK>), grid, dim3(kThreads), 0, s, p, (const G*)grad, m, v, (const M*)mask, begin, n, a, h, step_dev);
-  }
-  return check_launch("tf24_adamw_masked_decay");
+  if (blocks > 0x7fffffff) return fail(TF24_ERR_SHAPE, "%s: too many elements for one launch", fn);
+  hipLaunchKernelGGL((adamw_list<G, M>), dim3((unsigned)blocks), dim3(kThreads), 0, s, list, a, h);
+  return check_launch(fn);
 }
 
 template <typename G>
-int dispatch_mask(const void* mask, int mask_dtype, float* p, const void* grad, float* m, float* v, int64_t n, const AdamArgs& a,
-                  const AdamHyper& h, const int64_t* step_dev, hipStream_t s) {
-  if (!mask) return launch<G, uint8_t, false>(p, grad, m, v, nullptr, n, a, h, step_dev, s);
+int dispatch_mask(const char* fn, int mask_dtype, AdamList& list, const AdamArgs& a, const AdamHyper& h, hipStream_t s) {
   switch (mask_dtype) {
-    case TF24_U8: return launch<G, uint8_t, true>(p, grad, m, v, mask, n, a, h, step_dev, s);
-    case TF24_F32: return launch<G, float, true>(p, grad, m, v, mask, n, a, h, step_dev, s);
-    case TF24_F16: return launch<G, f16_t, true>(p, grad, m, v, mask, n, a, h, step_dev, s);
-    case TF24_BF16: return launch<G, bf16_t, true>(p, grad, m, v, mask, n, a, h, step_dev, s);
+    case TF24_U8: return launch<G, uint8_t>(fn, list, a, h, s);
+    case TF24_F32: return launch<G, float>(fn, list, a, h, s);
+    case TF24_F16: return launch<G, f16_t>(fn, list, a, h, s);
+    case TF24_BF16: return launch<G, bf16_t>(fn, list, a, h, s);
   }
-  return fail(TF24_ERR_DTYPE, "tf24_adamw_masked_decay: unsupported mask dtype %d", mask_dtype);
+  return fail(TF24_ERR_DTYPE, "%s: unsupported mask dtype %d", fn, mask_dtype);
 }
 
 }  // namespace
 }  // namespace tf24
 
-// step_host >= 1 with step_dev == nullptr, or step_dev (device memory) and step_host ignored
-static int adamw_masked_decay(const char* fn, float* p, const void* grad, int grad_dtype, float* exp_avg, float* exp_avg_sq,
-                              const void* mask, int mask_dtype, int64_t n, double lr, double beta1, double beta2, double eps,
-                              double weight_decay, double decay_alpha, int64_t step_host, const int64_t* step_dev, void* stream) {
+// Every tensor with its own step count in device memory (step_host 0), or all of them at step_host >= 1.
+static int adamw_masked_decay(const char* fn, const tf24_adamw_tensor* tensors, int count, int grad_dtype, int mask_dtype, double lr,
+                              double beta1, double beta2, double eps, double weight_decay, double decay_alpha, int64_t step_host,
+                              void* stream) {
   using namespace tf24;
-  if (n < 0) return fail(TF24_ERR_SHAPE, "%s: negative element count", fn);
-  if (n == 0) return TF24_OK;
-  if (!p || !grad || !exp_avg || !exp_avg_sq) return fail(TF24_ERR_ARG, "%s: null pointer", fn);
-  if (!step_dev && step_host < 1) return fail(TF24_ERR_ARG, "%s: step %lld must be >= 1", fn, (long long)step_host);
-  if (step_dev && (uintptr_t)step_dev % 8 != 0) return fail(TF24_ERR_STRIDE, "%s: the step count must be 8-byte aligned", fn);
+  if (count < 0 || (count > 0 && !tensors)) return fail(TF24_ERR_ARG, "%s: bad tensor list", fn);
   if (!(lr >= 0.0) || !(eps >= 0.0) || !(beta1 >= 0.0 && beta1 < 1.0) || !(beta2 >= 0.0 && beta2 < 1.0))
     return fail(TF24_ERR_ARG, "%s: invalid hyper-parameter (lr %g, eps %g, betas %g %g)", fn, lr, eps, beta1, beta2);
-  const AdamHyper h{lr, beta1, beta2, eps, weight_decay, decay_alpha};
-  const AdamArgs a = adam_args(h, step_dev ? 1 : step_host);
-  hipStream_t s = (hipStream_t)stream;
-  switch (grad_dtype) {
-    case TF24_F32: return dispatch_mask<float>(mask, mask_dtype, p, grad, exp_avg, exp_avg_sq, n, a, h, step_dev, s);
-    case TF24_F16: return dispatch_mask<f16_t>(mask, mask_dtype, p, grad, exp_avg, exp_avg_sq, n, a, h, step_dev, s);
-    case TF24_BF16: return dispatch_mask<bf16_t>(mask, mask_dtype, p, grad, exp_avg, exp_avg_sq, n, a, h, step_dev, s);
+  if (grad_dtype != TF24_F32 && grad_dtype != TF24_F16 && grad_dtype != TF24_BF16)
+    return fail(TF24_ERR_DTYPE, "%s: unsupported gradient dtype %d", fn, grad_dtype);
+  for (int i = 0; i < count; i++) {            // the whole list is checked before anything is launched
+    const tf24_adamw_tensor& t = tensors[i];
+    if (t.n < 0) return fail(TF24_ERR_SHAPE, "%s: negative element count", fn);
+    if (t.n == 0) continue;
+    if (!t.p || !t.grad || !t.exp_avg || !t.exp_avg_sq) return fail(TF24_ERR_ARG, "%s: null pointer", fn);
+    if (!t.step && step_host < 1) return fail(TF24_ERR_ARG, "%s: step %lld must be >= 1", fn, (long long)step_host);
+    if (t.step && (uintptr_t)t.step % 8 != 0) return fail(TF24_ERR_STRIDE, "%s: the step count must be 8-byte aligned", fn);
   }
-  return fail(TF24_ERR_DTYPE, "%s: unsupported gradient dtype %d", fn, grad_dtype);
+  const AdamHyper h{lr, beta1, beta2, eps, weight_decay, decay_alpha};
+  const AdamArgs a = adam_args(h, step_host < 1 ? 1 : step_host);
+  hipStream_t s = (hipStream_t)stream;
+  AdamList list;
+  for (int i = 0; i < count;) {
+    list.count = 0;
+    for (; i < count && list.count < kMaxTensors; i++) {
+      const tf24_adamw_tensor& t = tensors[i];
+      if (t.n > 0) list.t[list.count++] = AdamTensor{t.p, t.exp_avg, t.exp_avg_sq, t.grad, t.mask, t.step, t.n, 0, 0};
+    }
+    if (!list.count) break;
+    int rc;
+    switch (grad_dtype) {
+      case TF24_F32: rc = dispatch_mask<float>(fn, mask_dtype, list, a, h, s); break;
+      case TF24_F16: rc = dispatch_mask<f16_t>(fn, mask_dtype, list, a, h, s); break;
+      default: rc = dispatch_mask<bf16_t>(fn, mask_dtype, list, a, h, s); break;
+    }
+    if (rc) return rc;
+  }
+  return TF24_OK;
+}
+
+extern "C" int tf24_adamw_masked_decay_list(const tf24_adamw_tensor* tensors, int count, int grad_dtype, int mask_dtype, double lr,
+                                            double beta1, double beta2, double eps, double weight_decay, double decay_alpha,
+                                            int64_t step, void* stream) {
+  return adamw_masked_decay("tf24_adamw_masked_decay_list", tensors, count, grad_dtype, mask_dtype, lr, beta1, beta2, eps, weight_decay,
+                            decay_alpha, step, stream);
 }
 
 extern "C" int tf24_adamw_masked_decay(float* p, const void* grad, int grad_dtype, float* exp_avg, float* exp_avg_sq,
                                        const void* mask, int mask_dtype, int64_t n, double lr, double beta1, double beta2,
                                        double eps, double weight_decay, double decay_alpha, int64_t step, void* stream) {
-  return adamw_masked_decay("tf24_adamw_masked_decay", p, grad, grad_dtype, exp_avg, exp_avg_sq, mask, mask_dtype, n, lr, beta1, beta2,
-                            eps, weight_decay, decay_alpha, step, nullptr, stream);
+  if (n == 0) return TF24_OK;
+  const tf24_adamw_tensor t{p, grad, exp_avg, exp_avg_sq, mask, nullptr, n};
+  return adamw_masked_decay("tf24_adamw_masked_decay", &t, 1, grad_dtype, mask ? mask_dtype : TF24_U8, lr, beta1, beta2, eps,
+                            weight_decay, decay_alpha, step, stream);
 }
 
 extern "C" int tf24_adamw_masked_decay_device_step(float* p, const void* grad, int grad_dtype, float* exp_avg, float* exp_avg_sq,
@@ -167,6 +210,8 @@ extern "C" int tf24_adamw_masked_decay_device_step(float* p, const void* grad, i
                                                    double beta2, double eps, double weight_decay, double decay_alpha,
                                                    const int64_t* step, void* stream) {
   if (!step) return tf24::fail(TF24_ERR_ARG, "tf24_adamw_masked_decay_device_step: null step pointer");
-  return adamw_masked_decay("tf24_adamw_masked_decay_device_step", p, grad, grad_dtype, exp_avg, exp_avg_sq, mask, mask_dtype, n, lr,
-                            beta1, beta2, eps, weight_decay, decay_alpha, 0, step, stream);
+  if (n == 0) return TF24_OK;
+  const tf24_adamw_tensor t{p, grad, exp_avg, exp_avg_sq, mask, step, n};
+  return adamw_masked_decay("tf24_adamw_masked_decay_device_step", &t, 1, grad_dtype, mask ? mask_dtype : TF24_U8, lr, beta1, beta2, eps,
+                            weight_decay, decay_alpha, 0, stream);
 }

@@ -1,4 +1,5 @@
-"""AdamW with the masked decay of the 2:4 recipe folded into the update (one HIP kernel per tensor).
+"""AdamW with the masked decay of the 2:4 recipe folded into the update (one HIP launch for all
+tensors of a parameter group).
 
 The reference trains with its AdamW (sparse/adamw.py:9-115) after a loop that adds the decay term
 to the gradients of masked weights (README.md:205-213):
@@ -16,6 +17,8 @@ device operation), as torch's own optimizers do under that name: a step recorded
 replays with the count of the replay.  Hyper-parameters are read on the host at every call, so a
 recording holds the values of its time.
 """
+import struct
+
 import torch
 from torch.optim.optimizer import Optimizer
 
@@ -45,8 +48,8 @@ class MaskedDecayAdamW(Optimizer):
             raise RuntimeError("MaskedDecayAdamW: parameters must be dense in memory")
         state = self.state[p]
         state["step"] = torch.zeros((), dtype=torch.int64, device=p.device) if capturable else 0
-        state["exp_avg"] = torch.zeros_like(p, memory_format=torch.preserve_format)
-        state["exp_avg_sq"] = torch.zeros_like(p, memory_format=torch.preserve_format)
+        state["exp_avg"] = torch.empty_like(p, memory_format=torch.preserve_format)       # zeroed with the others of the
+        state["exp_avg_sq"] = torch.empty_like(p, memory_format=torch.preserve_format)    # group, in one launch (step)
         return state
 
     @torch.no_grad()
@@ -55,11 +58,12 @@ class MaskedDecayAdamW(Optimizer):
         if closure is not None:
             with torch.enable_grad():
                 loss = closure()
-        host_step, device_step = N.lib().tf24_adamw_masked_decay, N.lib().tf24_adamw_masked_decay_device_step
-        stream = N.stream_ptr()
         for group in self.param_groups:
             beta1, beta2 = group["betas"]
             lr, eps, wd, alpha = float(group["lr"]), float(group["eps"]), float(group["weight_decay"]), float(group["alpha"])
+            # Everything is looked at before anything is launched; the tensors of one launch share the types of
+            # gradient and mask and a host-side step count (device-side counts travel with their tensor)
+            entries, counts, launches, fresh = [], [], {}, []
             for p in group["params"]:
                 grad = p.grad
                 if grad is None:
@@ -67,19 +71,34 @@ class MaskedDecayAdamW(Optimizer):
                 state = self.state[p]
                 if not state:
                     state = self._check(p, group.get("capturable", False))
-                if grad.is_sparse or grad.stride() != p.stride():
+                    fresh += [state["exp_avg"], state["exp_avg_sq"]]
+                stride = p.stride()
+                if grad.is_sparse or grad.stride() != stride:
                     raise RuntimeError("MaskedDecayAdamW: the gradient must be dense with the parameter's strides")
-                state["step"] += 1
                 mask = getattr(p, "mask", None)
-                mask_ptr, mask_code = None, N.U8
-                if mask is not None and torch.is_tensor(mask) and getattr(p, "mode", "sparse") == "sparse":
-                    if mask.stride() != p.stride() or mask.device != p.device:
-                        raise RuntimeError("MaskedDecayAdamW: mask must have the parameter's strides and device")
-                    mask_ptr, mask_code = mask.data_ptr(), N.dtype_code(mask.dtype)
+                if mask is not None and not (torch.is_tensor(mask) and getattr(p, "mode", "sparse") == "sparse"):
+                    mask = None
+                if mask is not None and (mask.stride() != stride or mask.device != p.device):
+                    raise RuntimeError("MaskedDecayAdamW: mask must have the parameter's strides and device")
+                entries.append((p, grad, state, mask, N.dtype_code(grad.dtype), N.U8 if mask is None else N.dtype_code(mask.dtype)))
+                if torch.is_tensor(state["step"]):
+                    counts.append(state["step"])
+            if fresh:
+                torch._foreach_zero_(fresh)
+            if counts:
+                torch._foreach_add_(counts, 1)
+            for p, grad, state, mask, grad_code, mask_code in entries:
+                step = state["step"]
+                if torch.is_tensor(step):
+                    key, step_ptr = (grad_code, mask_code, 0), step.data_ptr()
+                else:
+                    step = state["step"] = step + 1
+                    key, step_ptr = (grad_code, mask_code, step), 0
+                if mask is not None:
                     p.cnt = 0
-                on_device = torch.is_tensor(state["step"])
-                N.check((device_step if on_device else host_step)(
-                    p.data_ptr(), grad.data_ptr(), N.dtype_code(grad.dtype), state["exp_avg"].data_ptr(),
-                    state["exp_avg_sq"].data_ptr(), mask_ptr, mask_code, p.numel(), lr, float(beta1), float(beta2),
-                    eps, wd, alpha, state["step"].data_ptr() if on_device else state["step"], stream))
+                launches.setdefault(key, []).extend((p.data_ptr(), grad.data_ptr(), state["exp_avg"].data_ptr(), state["exp_avg_sq"].data_ptr(),
+                                                     0 if mask is None else mask.data_ptr(), step_ptr, p.numel()))
+            for (grad_code, mask_code, step), words in launches.items():
+                N.check(N.lib().tf24_adamw_masked_decay_list(struct.pack("%dq" % len(words), *words), len(words) // 7, grad_code, mask_code,
+                                                             lr, float(beta1), float(beta2), eps, wd, alpha, step, N.stream_ptr()))
         return loss

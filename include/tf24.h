@@ -286,6 +286,23 @@ int tf24_adamw_masked_decay_device_step(float* p, const void* grad, int grad_dty
                                         const void* mask, int mask_dtype, int64_t n, double lr, double beta1,
                                         double beta2, double eps, double weight_decay, double decay_alpha,
                                         const int64_t* step, void* stream);
+/*
+ * The same update of a list of tensors that share the gradient and mask types and the hyper-parameters, in one launch
+ * per 56 tensors (the reference's optimizer walks its parameters one by one, sparse/adamw.py:56-113).  `step` of a
+ * tensor: its count in device memory (as above), or NULL: the argument `step` (>= 1).  mask NULL: no decay of that
+ * tensor.  `tensors` is host memory, read during the call.
+ */
+typedef struct {
+  float* p;
+  const void* grad;
+  float *exp_avg, *exp_avg_sq;
+  const void* mask;
+  const int64_t* step;
+  int64_t n;
+} tf24_adamw_tensor;
+int tf24_adamw_masked_decay_list(const tf24_adamw_tensor* tensors, int count, int grad_dtype, int mask_dtype, double lr,
+                                 double beta1, double beta2, double eps, double weight_decay, double decay_alpha,
+                                 int64_t step, void* stream);
 
 /*
  * The update of the STEP optimizer, one pass per tensor: replaces the body of AdamW_STEP.step

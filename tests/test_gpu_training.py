@@ -264,6 +264,44 @@ def test_masked_decay_adamw_kernel(cuda, gdt):
         assert torch.allclose(plain.detach(), ref_plain.detach(), rtol=1e-5, atol=1e-7)
 
 
+@pytest.mark.parametrize("gdt,mdt,device_step", [(torch.float32, torch.bool, False), (torch.float16, torch.float32, True)])
+def test_masked_decay_adamw_list_of_tensors(cuda, gdt, mdt, device_step):
+    """A group of more tensors than one launch takes (56), with the lengths around a block of 1024 elements, a tensor
+    whose storage starts off a 16-byte boundary, masked and unmasked ones mixed: two updates against the oracle
+    (float32; rtol 2e-6 as above).  A tensor of another step count goes with the others of its own."""
+    import sparse
+    g = torch.Generator().manual_seed(32)
+    hyp = dict(lr=3e-3, betas=(0.9, 0.95), eps=1e-8, weight_decay=0.1)
+    lengths = [1, 3, 4, 1020, 1023, 1024, 1025, 2048, 4096, 4099] * 6
+    params, refs = [], []
+    for i, n in enumerate(lengths):
+        flat = torch.randn(n + 1, generator=g).to(cuda)
+        p = torch.nn.Parameter(flat[1:] if i % 7 == 3 else flat[:-1])          # 4 bytes off a 16-byte boundary: single accesses
+        p.grad_dtype = None
+        mask = None
+        if i % 3:
+            mask = torch.rand(n, generator=g) > 0.5
+            p.mask, p.mode = mask.to(cuda).to(mdt), "sparse"
+        params.append(p)
+        refs.append([p.detach().cpu().clone(), torch.zeros(n), torch.zeros(n), mask, 0])
+    opt = sparse.MaskedDecayAdamW(params, alpha=2e-4, capturable=device_step, **hyp)
+    for update in range(2):
+        for i, (p, r) in enumerate(zip(params, refs)):
+            if update == 0 and i == 5:
+                p.grad = None                                                  # one update behind the others from here on
+                continue
+            grad = torch.randn(len(r[0]), generator=g).to(gdt)
+            p.grad = grad.to(cuda)
+            r[4] += 1
+            r[0], r[1], r[2] = oracle.adamw_masked_decay(r[0], grad, r[1], r[2], r[3], r[4], alpha=2e-4, **hyp)
+        opt.step()
+    for p, (want, m, v, _, step) in zip(params, refs):
+        assert torch.allclose(p.detach().cpu(), want, rtol=2e-6, atol=1e-8)
+        assert torch.allclose(opt.state[p]["exp_avg"].cpu(), m, rtol=2e-6, atol=1e-10)
+        assert torch.allclose(opt.state[p]["exp_avg_sq"].cpu(), v, rtol=2e-6, atol=1e-12)
+        assert int(opt.state[p]["step"]) == step
+
+
 @pytest.mark.parametrize("gdt", [torch.float32, torch.bfloat16])
 def test_masked_decay_adamw_step_count_on_the_device(cuda, gdt):
     """capturable=True: the step count is an int64 in device memory and the bias corrections 1 - beta^step are
