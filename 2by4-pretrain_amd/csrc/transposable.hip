@@ -107,62 +107,58 @@ __device__ __forceinline__ uint32_t search_block(const float (&a)[4][4]) {
   return mask;
 }
 
-// E = elements per row of a block = 4.  TRANS: the matrix is column-major (element (r,c) at c*ld + r),
+// Bound by memory (5 bytes per element of a 16-bit type, 9 of float32; the search is some 330 vector instructions per
+// block, half of the time of a 16-bit matrix).  With two adjacent blocks per lane a wave instruction over float32
+// touched half lines (32 bytes from lane to lane): 11008 x 4096 float32 83.6 us = 4.85 TB/s, with one block per lane
+// 67.5 us = 6.0 TB/s; bf16 40.1 and 38.5 us, 3072 x 768 float32 5.9 and 5.0, bf16 5.2 and 4.8.
+// TRANS: the matrix is column-major (element (r,c) at c*ld + r),
 // so the lane reads the block transposed and writes its results transposed.
 template <typename T, bool ABS, bool TRANS>
 __global__ void __launch_bounds__(kThreads)
-transposable_kernel(const T* __restrict__ dense, int64_t ld, int64_t nmajor4, int64_t nminor8,
+transposable_kernel(const T* __restrict__ dense, int64_t ld, int64_t nmajor4, int64_t nminor4,
                     T* __restrict__ sparse, uint8_t* __restrict__ mask_out) {
-  // "major" = the strided dimension in memory, "minor" = the contiguous one.  A lane owns two
-  // adjacent 4 x 4 blocks (8 contiguous elements of 4 lines): 16-byte loads and stores for 16-bit
-  // types, 8-byte mask stores.
+  // "major" = the strided dimension in memory, "minor" = the contiguous one.
   // blocks are numbered along the contiguous dimension first: blocks that run together read
   // neighbouring pieces of the same four lines
-  const uint32_t chunks = (uint32_t)((nminor8 + kThreads - 1) / kThreads);
+  const uint32_t chunks = (uint32_t)((nminor4 + kThreads - 1) / kThreads);
   const int64_t bmajor = blockIdx.x / chunks;
   const int64_t bminor = (int64_t)(blockIdx.x - (uint32_t)bmajor * chunks) * kThreads + threadIdx.x;
-  if (bminor >= nminor8) return;
-  const int64_t off = bmajor * 4 * ld + bminor * 8;
-  Pack<T, 8> in[4];
+  if (bminor >= nminor4) return;
+  const int64_t off = bmajor * 4 * ld + bminor * 4;
+  Pack<T, 4> in[4];
 #pragma unroll
   for (int p = 0; p < 4; p++) in[p].load_stream(dense + off + p * ld);
-  uint32_t mbits[2];
+  float a[4][4];
 #pragma unroll
-  for (int h = 0; h < 2; h++) {
-    float a[4][4];
+  for (int p = 0; p < 4; p++)
 #pragma unroll
-    for (int p = 0; p < 4; p++)
-#pragma unroll
-      for (int e = 0; e < 4; e++) {
-        float v = to_float(in[p].v[4 * h + e]);
-        if (ABS) v = __builtin_fabsf(v);
-        if (TRANS) a[e][p] = v; else a[p][e] = v;
-      }
-    mbits[h] = search_block(a);
-  }
+    for (int e = 0; e < 4; e++) {
+      float v = to_float(in[p].v[e]);
+      if (ABS) v = __builtin_fabsf(v);
+      if (TRANS) a[e][p] = v; else a[p][e] = v;
+    }
+  const uint32_t mbits = search_block(a);
 #pragma unroll
   for (int p = 0; p < 4; p++) {
-    uint32_t bytes[2] = {0, 0};
-    Pack<T, 8> out;
+    uint32_t bytes = 0;
+    Pack<T, 4> out;
 #pragma unroll
-    for (int h = 0; h < 2; h++)
-#pragma unroll
-      for (int e = 0; e < 4; e++) {
-        const int bit = TRANS ? (4 * e + p) : (4 * p + e);
-        const bool keep = (mbits[h] >> bit) & 1;
-        bytes[h] |= (uint32_t)keep << (8 * e);
-        out.v[4 * h + e] = keep ? in[p].v[4 * h + e] : T{};
-      }
-    *reinterpret_cast<uint2*>(mask_out + off + p * ld) = make_uint2(bytes[0], bytes[1]);   // streaming here costs 15 %
+    for (int e = 0; e < 4; e++) {
+      const int bit = TRANS ? (4 * e + p) : (4 * p + e);
+      const bool keep = (mbits >> bit) & 1;
+      bytes |= (uint32_t)keep << (8 * e);
+      out.v[e] = keep ? in[p].v[e] : T{};
+    }
+    *reinterpret_cast<uint32_t*>(mask_out + off + p * ld) = bytes;
     if (sparse) out.store_stream(sparse + off + p * ld);
   }
 }
 
 template <typename T, bool ABS, bool TRANS>
 int launch(const void* dense, int64_t ld, int64_t m, int64_t k, void* sparse, uint8_t* mask, hipStream_t s) {
-  const int64_t nmajor4 = (TRANS ? k : m) / 4, nminor8 = (TRANS ? m : k) / 8;     // both extents are multiples of 32
-  dim3 grid((unsigned)(nmajor4 * ((nminor8 + kThreads - 1) / kThreads)));
-  hipLaunchKernelGGL((transposable_kernel<T, ABS, TRANS>), grid, dim3(kThreads), 0, s, (const T*)dense, ld, nmajor4, nminor8,
+  const int64_t nmajor4 = (TRANS ? k : m) / 4, nminor4 = (TRANS ? m : k) / 4;     // both extents are multiples of 32
+  dim3 grid((unsigned)(nmajor4 * ((nminor4 + kThreads - 1) / kThreads)));
+  hipLaunchKernelGGL((transposable_kernel<T, ABS, TRANS>), grid, dim3(kThreads), 0, s, (const T*)dense, ld, nmajor4, nminor4,
                      (T*)sparse, mask);
   return check_launch("tf24_transposable_mask");
 }
