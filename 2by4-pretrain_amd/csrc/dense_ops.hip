@@ -10,18 +10,17 @@ constexpr int kThreads = 256;
 enum { OP_SOFT = 0, OP_SPARSE24 = 1, OP_MVUE = 2 };
 
 // One group: inputs x[4] (float32), outputs y[4] (value to store where kept) and mask bits.
-template <int OP>
+template <typename T, int OP>
 __device__ __forceinline__ uint32_t group_op(const float (&x)[4], float r0, float r1, float (&y)[4]) {
   if constexpr (OP == OP_MVUE) {
     // only the two kept values are rescaled; with fewer than two mask bits the kept element is
     // still one of the two encoded positions
-    const Mvue4 g = mvue4(x[0], x[1], x[2], x[3], r0, r1);
-    const uint32_t pa = g.keep.nibble() & 3;
-    const float ya = mvue_rescale(g.keep.first(x[0], x[1], x[2]), g.keep.first(g.p[0], g.p[1], g.p[2]), g.in_range);
-    const float yb = mvue_rescale(g.keep.second(x[1], x[2], x[3]), g.keep.second(g.p[1], g.p[2], g.p[3]), g.in_range);
+    bool finite;
+    const Mvue4 g = mvue4<T>(x, r0, r1, finite);
+    const uint32_t pa = g.nibble & 3;
 #pragma unroll
-    for (int i = 0; i < 4; i++) y[i] = (uint32_t)i == pa ? ya : yb;
-    return g.keep.bits();
+    for (int i = 0; i < 4; i++) y[i] = (uint32_t)i == pa ? g.first : g.second;
+    return g.bits;
   } else {
     uint32_t mb = magnitude_mask4(x[0], x[1], x[2], x[3]);
     if constexpr (OP == OP_SOFT) {
@@ -67,7 +66,7 @@ dense_op_row(const T* __restrict__ dense, int64_t ld, int64_t m, int64_t k, cons
     float x[4], y[4];
 #pragma unroll
     for (int i = 0; i < 4; i++) x[i] = to_float(in.v[4 * g + i]);
-    uint32_t mb = group_op<OP>(x, r[2 * g], r[2 * g + 1], y);
+    uint32_t mb = group_op<T, OP>(x, r[2 * g], r[2 * g + 1], y);
 #pragma unroll
     for (int i = 0; i < 4; i++) {
       bool keep = (mb >> i) & 1;
@@ -106,7 +105,7 @@ dense_op_col(const T* __restrict__ dense, int64_t ld, int64_t m, int64_t k, cons
     for (int c = 0; c < 4; c++) x[c] = to_float(in[c].v[i]);
     float u0 = 0.f, u1 = 0.f;
     if constexpr (OP == OP_MVUE) { u0 = rr[0].v[i]; u1 = rr[1].v[i]; }
-    uint32_t mb = group_op<OP>(x, u0, u1, y);
+    uint32_t mb = group_op<T, OP>(x, u0, u1, y);
 #pragma unroll
     for (int c = 0; c < 4; c++) {
       bool keep = (mb >> c) & 1;

@@ -3,8 +3,8 @@
 // Row-major input: one lane owns 8 consecutive elements (two groups): 128-bit loads for 16-bit
 // inputs, 4 kept values leave as one 64-bit (16-bit values) or 32-bit (fp8) store, and the lane's
 // metadata byte is merged across 4 lanes with wave shuffles into one 32-bit store.
-// Column-major input (W.T, dY.t() views): one lane owns a 4-column x R-row sub-tile (R groups that
-// live entirely in its registers), a 256-lane block covers 8R rows x 128 columns, and the
+// Column-major input (W.T, dY.t() views): one lane owns an 8-column x R-row sub-tile (2R groups that
+// live entirely in its registers), a 256-lane block covers 16R rows x 128 columns, and the
 // compressed tile is transposed through LDS so that values and metadata leave row-major with
 // full-line stores.
 #include <mutex>
@@ -21,28 +21,21 @@ constexpr int kThreads = 256;
 // uniforms) one unit per lane and four times the blocks is (MVUE24 82 against 85 us, mask 67 against 71).
 template <int MODE> constexpr int unroll_for() { return MODE == TF24_PRUNE_MAGNITUDE ? 4 : 1; }
 
-// The kept elements of one group; in MVUE mode also the inclusion probabilities the two kept
-// values are divided by.
-template <typename In, int MODE, typename MaskT>
-__device__ __forceinline__ Keep4 prune_group(const float (&x)[4], const MaskT* mk, float r0, float r1, Mvue4& g) {
-  if constexpr (MODE == TF24_PRUNE_MAGNITUDE) {
-    return magnitude_keep4(x[0], x[1], x[2], x[3]);
-  } else if constexpr (MODE == TF24_PRUNE_MASK) {
-    return Keep4{to_float(mk[0]) != 0.0f, to_float(mk[1]) != 0.0f, to_float(mk[2]) != 0.0f, to_float(mk[3]) != 0.0f};
-  } else {
-    g = mvue4(x[0], x[1], x[2], x[3], r0, r1);
-    return g.keep;
-  }
-}
-
-// The two values stored for a group: the kept elements in ascending position (MVUE: rescaled).
-template <int MODE>
-__device__ __forceinline__ void kept_values(const Keep4& keep, const float (&x)[4], const Mvue4& g, float& first, float& second) {
-  first = keep.first(x[0], x[1], x[2]);
-  second = keep.second(x[1], x[2], x[3]);
+// The nibble of one group and the two values stored for it, in ascending position (MVUE: rescaled).
+template <typename In, typename Out, int MODE, typename MaskT>
+__device__ __forceinline__ uint32_t prune_group(const float (&x)[4], const MaskT* mk, float r0, float r1, Pack<Out, 2>& kept) {
   if constexpr (MODE == TF24_PRUNE_MVUE) {
-    first = mvue_rescale(first, keep.first(g.p[0], g.p[1], g.p[2]), g.in_range);
-    second = mvue_rescale(second, keep.second(g.p[1], g.p[2], g.p[3]), g.in_range);
+    bool finite;
+    const Mvue4 g = mvue4<In>(x, r0, r1, finite);
+    kept = from_float2<Out>(g.first, g.second, finite);
+    return g.nibble;
+  } else {
+    Keep4 keep;
+    if constexpr (MODE == TF24_PRUNE_MAGNITUDE) keep = magnitude_keep4(x[0], x[1], x[2], x[3]);
+    else keep = Keep4{to_float(mk[0]) != 0.0f, to_float(mk[1]) != 0.0f, to_float(mk[2]) != 0.0f, to_float(mk[3]) != 0.0f};
+    kept.v[0] = from_float<Out>(keep.first(x[0], x[1], x[2]));
+    kept.v[1] = from_float<Out>(keep.second(x[1], x[2], x[3]));
+    return keep.nibble();
   }
 }
 
@@ -67,68 +60,68 @@ __device__ __forceinline__ void store_panel_meta_block(const uint32_t* s_words, 
 }
 
 // ------------------------------------------------------------------ row-major
-// panel = false: canonical output, values [m, k/2] and metadata [m, k/8 bytes] row-major; units
+// PANEL = false: canonical output, values [m, k/2] and metadata [m, k/8 bytes] row-major; units
 //   (8 dense elements) are walked along rows.
-// panel = true : panel output, [k/KP][m][64 bytes] values (KP = 128 / sizeof(Out) dense elements per
+// PANEL = true : panel output, [k/KP][m][64 bytes] values (KP = 128 / sizeof(Out) dense elements per
 //   panel) and [k/32][m][4 bytes] metadata.  A block covers 64 rows x 128 dense columns
 //   (32 x 256 when m is not a multiple of 64): 2^lpr_shift lanes read consecutive columns of one row,
 //   the other lanes of the wave take the next rows, so that every store instruction writes, per
 //   panel, the contiguous 64-byte pieces of 4 (2) adjacent rows.
-template <typename In, typename Out, int MODE, typename MaskT>
+// Rows and units of the panel form are 32-bit numbers (the grid bounds both), combined to 64-bit offsets by a
+// multiply-add: formed in 64 bits throughout, and for both forms of output in one kernel,
+// the addresses were a fifth of the MVUE24 conversion's vector instructions.
+template <typename In, typename Out, int MODE, typename MaskT, bool PANEL>
 __global__ void __launch_bounds__(kThreads)
 prune_compress_row(const In* __restrict__ dense, int64_t ld, int64_t m, int64_t k,
                    const MaskT* __restrict__ mask, int64_t mask_ld,
                    RandSrc rs,
-                   Out* __restrict__ values, uint8_t* __restrict__ meta, bool contiguous, bool panel, int lpr_shift) {
+                   Out* __restrict__ values, uint8_t* __restrict__ meta, bool contiguous, int lpr_shift) {
   constexpr int kUnroll = unroll_for<MODE>();
-  constexpr int UPP = (128 / (int)sizeof(Out)) / 8;      // units per panel row (8 or 16)
-  __shared__ __attribute__((aligned(16))) uint32_t s_words[kUnroll * kThreads / 4];
-  const int64_t upr = k >> 3;                             // 8-element units per row
-  const int64_t total = m * upr;
-  const int64_t base = (int64_t)blockIdx.x * (kThreads * kUnroll) + threadIdx.x;
+  constexpr uint32_t UPP = (128 / (uint32_t)sizeof(Out)) / 8;     // units per panel row (8 or 16)
+  __shared__ __attribute__((aligned(16))) uint32_t s_words[PANEL ? kUnroll * kThreads / 4 : 1];
+  const uint32_t upr = (uint32_t)(k >> 3);                // 8-element units per row
 #pragma unroll
   for (int it = 0; it < kUnroll; it++) {
-    const int64_t u = base + (int64_t)it * kThreads;
-    bool live = u < total;
-    uint32_t mbyte = 0;
+    bool live;
+    uint32_t mbyte = 0, row = 0;
+    std::conditional_t<PANEL, uint32_t, uint64_t> col8;
+    uint64_t ounit, ometa = 0;                             // unit index among the values, byte offset of its metadata byte
     Pack<Out, 4> out;
-    int64_t row = 0, col8 = 0, ounit = 0, ometa = 0;       // unit index among the values, byte offset of its metadata byte
-    if (panel) {
-      const int rpi = kThreads >> lpr_shift;                 // rows per iteration
+    if constexpr (PANEL) {
+      const uint32_t rpi = kThreads >> lpr_shift;          // rows per iteration
       // blocks that run together (consecutive blockIdx.x) read neighbouring column ranges of the same rows
-      row = (int64_t)blockIdx.y * (kUnroll * rpi) + it * rpi + (threadIdx.x >> lpr_shift);
-      col8 = ((int64_t)blockIdx.x << lpr_shift) + (threadIdx.x & ((1 << lpr_shift) - 1));
+      row = blockIdx.y * (kUnroll * rpi) + it * rpi + (threadIdx.x >> lpr_shift);
+      col8 = (blockIdx.x << lpr_shift) + (threadIdx.x & ((1u << lpr_shift) - 1u));
       live = col8 < upr;                                   // m is a multiple of 32
+      ounit = ((uint64_t)(col8 / UPP) * (uint32_t)m + row) * UPP + col8 % UPP;
+    } else {
+      const uint64_t u = (uint64_t)blockIdx.x * (kThreads * kUnroll) + it * kThreads + threadIdx.x;
+      live = u < (uint64_t)m * upr;
+      if (contiguous) {            // every leading dimension equals k: offsets are linear in u
+        col8 = u;
+      } else {
+        row = (uint32_t)u / upr;
+        col8 = (uint32_t)u - row * upr;       // (fewer than 2^32 units)
+      }
+      ounit = (uint64_t)row * upr + col8;
+      ometa = ounit;
     }
     if (live) {
-      if (panel) {
-        ounit = ((col8 / UPP) * m + row) * UPP + col8 % UPP;
-        ometa = panel_meta_offset(col8, row, m);
-      } else {
-        if (contiguous) {          // every leading dimension equals k: offsets are linear in u
-          col8 = u;
-        } else {
-          row = (int64_t)((uint32_t)u / (uint32_t)upr);
-          col8 = u - row * upr;
-        }
-        ounit = row * upr + col8;
-        ometa = ounit;
-      }
       Pack<In, 8> in;
-      in.load_stream(dense + row * ld + col8 * 8);
+      in.load_stream(dense + (uint64_t)row * ld + (uint64_t)col8 * 8);
       Pack<MaskT, 8> mk;
       float r[4] = {0.f, 0.f, 0.f, 0.f};
-      if constexpr (MODE == TF24_PRUNE_MASK) mk.load_stream(mask + row * mask_ld + col8 * 8);
+      if constexpr (MODE == TF24_PRUNE_MASK) mk.load_stream(mask + (uint64_t)row * mask_ld + (uint64_t)col8 * 8);
       if constexpr (MODE == TF24_PRUNE_MVUE) {
         if (rs.kind == RAND_SEEDED) {
-          const Philox4 c = philox4x32_10(rs.seed_now(), (uint64_t)(row * upr + col8), rs.offset_now());
+          const Philox4 c = philox4x32_10(rs.seed_now(), (uint64_t)row * upr + col8, rs.offset_now());
           r[0] = philox_uniform(c.x); r[1] = philox_uniform(c.y); r[2] = philox_uniform(c.z); r[3] = philox_uniform(c.w);
         } else if (rs.kind == RAND_PACKED) {                   // [m, k/2]: the unit's four uniforms are adjacent
           Pack<float, 4> r4;
-          r4.load_stream(rs.ptr + row * rs.ld + col8 * 4);
+          r4.load_stream(rs.ptr + (uint64_t)row * rs.ld + (uint64_t)col8 * 4);
           r[0] = r4.v[0]; r[1] = r4.v[1]; r[2] = r4.v[2]; r[3] = r4.v[3];
         } else {
-          const float* rp = rs.ptr + row * rs.ld + col8 * 8;
+          const float* rp = rs.ptr + (uint64_t)row * rs.ld + (uint64_t)col8 * 8;
           Pack<float, 2> ra, rb;                               // the group's two uniforms: the second load meets the first one's line in L1
           ra.load(rp);
           rb.load(rp + 4);
@@ -138,24 +131,19 @@ prune_compress_row(const In* __restrict__ dense, int64_t ld, int64_t m, int64_t 
 #pragma unroll
       for (int g = 0; g < 2; g++) {
         float x[4];
-        Mvue4 pr;
 #pragma unroll
         for (int i = 0; i < 4; i++) x[i] = to_float(in.v[4 * g + i]);
-        const Keep4 keep = prune_group<In, MODE, MaskT>(x, &mk.v[4 * g], r[2 * g], r[2 * g + 1], pr);
-        float v0, v1;
-        kept_values<MODE>(keep, x, pr, v0, v1);
-        out.v[2 * g] = from_float<Out>(v0);
-        out.v[2 * g + 1] = from_float<Out>(v1);
-        mbyte |= keep.nibble() << (4 * g);
+        Pack<Out, 2> kept;
+        const uint32_t nib = prune_group<In, Out, MODE, MaskT>(x, &mk.v[4 * g], r[2 * g], r[2 * g + 1], kept);
+        out.v[2 * g] = kept.v[0];
+        out.v[2 * g + 1] = kept.v[1];
+        mbyte |= nib << (4 * g);
       }
       out.store_stream(values + ounit * 4);
     }
     // 4 adjacent lanes (32 dense columns of one row) -> one metadata dword
-    uint32_t w = mbyte;
-    w |= __shfl_down(mbyte, 1) << 8;
-    w |= __shfl_down(mbyte, 2) << 16;
-    w |= __shfl_down(mbyte, 3) << 24;
-    if (panel) {
+    const uint32_t w = quad_bytes(mbyte);
+    if constexpr (PANEL) {
       const int rpi = kThreads >> lpr_shift;
       if ((threadIdx.x & 3) == 0)
         s_words[((threadIdx.x & ((1 << lpr_shift) - 1)) >> 2) * (kUnroll * rpi) + it * rpi + (threadIdx.x >> lpr_shift)] = w;
@@ -163,7 +151,7 @@ prune_compress_row(const In* __restrict__ dense, int64_t ld, int64_t m, int64_t 
       *reinterpret_cast<uint32_t*>(meta + ometa) = w;
     }
   }
-  if (panel) {
+  if constexpr (PANEL) {
     __syncthreads();
     const int rows = kUnroll * (kThreads >> lpr_shift);
     store_panel_meta_block(s_words, rows, 1 << (lpr_shift - 2), (int64_t)blockIdx.y * rows, (int64_t)blockIdx.x << lpr_shift, upr, m, meta);
@@ -240,10 +228,7 @@ prune_compress_row_mag16(const In* __restrict__ dense, int64_t ld, int64_t m, in
     if (live[it]) out.store_stream(values + ounit[it] * 4);
     // 4 adjacent lanes (32 dense columns of one row) -> one metadata dword
     const uint32_t mbyte = live[it] ? n0 | (n1 << 4) : 0u;
-    uint32_t w = mbyte;
-    w |= __shfl_down(mbyte, 1) << 8;
-    w |= __shfl_down(mbyte, 2) << 16;
-    w |= __shfl_down(mbyte, 3) << 24;
+    const uint32_t w = quad_bytes(mbyte);
     if (panel) {
       const int rpi = kThreads >> lpr_shift;
       if ((threadIdx.x & 3) == 0)
@@ -314,10 +299,7 @@ prune_compress_row_mag16_panel(const In* __restrict__ dense, int64_t ld, int64_t
     }
     s_x[wave][it * XROW + lane] = *reinterpret_cast<const piece_t*>(out.v);
     const uint32_t mbyte = live ? n0 | (n1 << 4) : 0u;
-    uint32_t w = mbyte;
-    w |= __shfl_down(mbyte, 1) << 8;
-    w |= __shfl_down(mbyte, 2) << 16;
-    w |= __shfl_down(mbyte, 3) << 24;
+    const uint32_t w = quad_bytes(mbyte);
     words[it] = w;
   }
   // lane l' of store instruction i takes row l'/16, unit 16 i + l'%16 (LDS accesses of one wave execute in order: no barrier)
@@ -334,7 +316,10 @@ prune_compress_row_mag16_panel(const In* __restrict__ dense, int64_t ld, int64_t
 }
 
 // ------------------------------------------------------------------ column-major
-// element (r,c) at c*ld + r.  R = rows per lane = 16 bytes / sizeof(In).
+// element (r,c) at c*ld + r.  A lane owns 8 columns x R rows, R = 8 bytes / sizeof(In): both groups that one generator
+// call serves and one metadata byte of a row are in one lane (with 4 columns x 2R rows per lane, 16-byte loads, the
+// lanes of two adjacent groups exchanged half of their uniforms and every nibble).  16 lanes read 128 contiguous bytes
+// of a column.
 template <typename In, typename Out, int MODE, typename MaskT>
 __global__ void __launch_bounds__(kThreads)
 prune_compress_col(const In* __restrict__ dense, int64_t ld, int64_t m, int64_t k,
@@ -342,97 +327,88 @@ prune_compress_col(const In* __restrict__ dense, int64_t ld, int64_t m, int64_t 
                    RandSrc rs,
                    Out* __restrict__ values, uint8_t* __restrict__ meta, bool panel,
                    float* __restrict__ rowsum_partial) {
-  constexpr int R = 16 / sizeof(In);
-  constexpr int TR = 8 * R;          // tile rows
-  constexpr int TC = 128;            // tile columns (32 groups)
-  constexpr int VPITCH = (TC / 2) * sizeof(Out) + 4;   // bytes per row of the value tile (+1 bank)
+  constexpr int R = 8 / sizeof(In);
+  constexpr int TR = 16 * R;         // tile rows
+  constexpr int TC = 128;            // tile columns (16 units of 8)
+  constexpr int VPITCH = (TC / 2) * sizeof(Out) + 4 * sizeof(Out);   // bytes per row of the value tile: the 16 row chunks of a write
+                                                                     // are 8 (4) dwords apart modulo the banks, the units fill the gaps
   constexpr int MPITCH = TC / 8 + 4;                   // bytes per row of the metadata tile
   __shared__ __attribute__((aligned(16))) uint8_t s_val[TR * VPITCH];
   __shared__ __attribute__((aligned(16))) uint8_t s_meta[TR * MPITCH];
-  // Row sums of the dense input (the bias gradient when the input is dY^T): a lane adds its 4
-  // columns, the 32 lanes that share a row meet in LDS, the block leaves one float per row in
+  // Row sums of the dense input (the bias gradient when the input is dY^T): a lane adds its 8
+  // columns, the 16 lanes that share a row meet in LDS, the block leaves one float per row in
   // rowsum_partial[column block][row]; a second kernel adds the column blocks.  Fixed order throughout.
-  constexpr int SPITCH = TC / 4 + 1;
+  constexpr int SPITCH = TC / 8 + 1;
   __shared__ float s_sum[TR * SPITCH];
 
   const int tid = threadIdx.x;
-  const int rchunk = tid & 7, grp = tid >> 3;           // 8 row chunks x 32 groups
+  const int rchunk = tid & 15, unit = tid >> 4;         // 16 row chunks x 16 units
   // consecutive blockIdx.x walk the contiguous (row) dimension of the column-major input
   const int64_t row0 = (int64_t)blockIdx.x * TR, col0 = (int64_t)blockIdx.y * TC;
-  const int64_t r0 = row0 + rchunk * R, c0 = col0 + grp * 4;
+  const int64_t r0 = row0 + rchunk * R, c0 = col0 + unit * 8;
   float psum[R];
 #pragma unroll
   for (int i = 0; i < R; i++) psum[i] = 0.0f;
-  // Seeded uniforms: one generator call serves the two groups of an 8-column unit, which two lanes
-  // 8 apart own (grp and grp ^ 1).  Each computes the calls of half of the R rows (the even group's
-  // lane the first half) and hands the other lane its two words; every lane of the wave takes part.
-  Pack<float, R> su[2];
-  if constexpr (MODE == TF24_PRUNE_MVUE) {
-    if (rs.kind == RAND_SEEDED) {
-      const int par = grp & 1;
-#pragma unroll
-      for (int j = 0; j < R / 2; j++) {
-        const int64_t row = r0 + j + par * (R / 2);
-        const Philox4 c = philox4x32_10(rs.seed_now(), (uint64_t)(row * (k >> 3) + (c0 >> 3)), rs.offset_now());
-        const float own0 = philox_uniform(par ? c.z : c.x), own1 = philox_uniform(par ? c.w : c.y);
-        const float snd0 = philox_uniform(par ? c.x : c.z), snd1 = philox_uniform(par ? c.y : c.w);
-        const float rcv0 = __shfl_xor(snd0, 8), rcv1 = __shfl_xor(snd1, 8);
-        su[0].v[j] = par ? rcv0 : own0;          su[1].v[j] = par ? rcv1 : own1;            // row j
-        su[0].v[j + R / 2] = par ? own0 : rcv0;  su[1].v[j + R / 2] = par ? own1 : rcv1;    // row j + R/2
-      }
-    }
-  }
   if (r0 < m && c0 < k) {
-    Pack<In, R> in[4];
-    Pack<MaskT, R> mk[4];
-    Pack<float, R> rr[2];
+    Pack<In, R> in[8];
+    Pack<MaskT, R> mk[8];
+    Pack<float, R> rr[4];              // group 0: rr[0], rr[1]; group 1: rr[2], rr[3]
 #pragma unroll
-    for (int c = 0; c < 4; c++) in[c].load_stream(dense + (c0 + c) * ld + r0);
+    for (int c = 0; c < 8; c++) in[c].load_stream(dense + (c0 + c) * ld + r0);
     if constexpr (MODE == TF24_PRUNE_MASK) {
 #pragma unroll
-      for (int c = 0; c < 4; c++) mk[c].load_stream(mask + (c0 + c) * mask_ld + r0);
+      for (int c = 0; c < 8; c++) mk[c].load_stream(mask + (c0 + c) * mask_ld + r0);
     }
     if constexpr (MODE == TF24_PRUNE_MVUE) {
       if (rs.kind == RAND_SEEDED) {
-        rr[0] = su[0]; rr[1] = su[1];
+        const uint64_t seed = rs.seed_now(), offset = rs.offset_now();
+        const uint64_t index = (uint64_t)r0 * (uint64_t)(k >> 3) + (uint64_t)(c0 >> 3);
+#pragma unroll
+        for (int i = 0; i < R; i++) {
+          const Philox4 c = philox4x32_10(seed, index + (uint64_t)i * (uint64_t)(k >> 3), offset);
+          rr[0].v[i] = philox_uniform(c.x); rr[1].v[i] = philox_uniform(c.y);
+          rr[2].v[i] = philox_uniform(c.z); rr[3].v[i] = philox_uniform(c.w);
+        }
       } else {
-        const int64_t rc = rs.kind == RAND_PACKED ? c0 >> 1 : c0;   // packed: columns 2g, 2g+1 of a [m, k/2] tensor
+        // packed: columns 2g, 2g+1 of a [m, k/2] tensor; full: columns 4g, 4g+1 of a [m, k] one
+        const int64_t rc = rs.kind == RAND_PACKED ? c0 >> 1 : c0, step = rs.kind == RAND_PACKED ? 2 : 4;
         rr[0].load_stream(rs.ptr + (rc + 0) * rs.ld + r0);
         rr[1].load_stream(rs.ptr + (rc + 1) * rs.ld + r0);
+        rr[2].load_stream(rs.ptr + (rc + step) * rs.ld + r0);
+        rr[3].load_stream(rs.ptr + (rc + step + 1) * rs.ld + r0);
       }
     }
 #pragma unroll
     for (int i = 0; i < R; i++) {
-      float x[4];
-      Mvue4 pr;
-      MaskT mrow[4];
-#pragma unroll
-      for (int c = 0; c < 4; c++) { x[c] = to_float(in[c].v[i]); if constexpr (MODE == TF24_PRUNE_MASK) mrow[c] = mk[c].v[i]; }
-      float u0 = 0.f, u1 = 0.f;
-      if constexpr (MODE == TF24_PRUNE_MVUE) { u0 = rr[0].v[i]; u1 = rr[1].v[i]; }
-      if (rowsum_partial) psum[i] = (x[0] + x[1]) + (x[2] + x[3]);
-      const Keep4 keep = prune_group<In, MODE, MaskT>(x, mrow, u0, u1, pr);
-      const uint32_t nib = keep.nibble();
-      float v0, v1;
-      kept_values<MODE>(keep, x, pr, v0, v1);
-      Pack<Out, 2> o;
-      o.v[0] = from_float<Out>(v0);
-      o.v[1] = from_float<Out>(v1);
       const int lr = rchunk * R + i;
-      o.store(reinterpret_cast<Out*>(s_val + lr * VPITCH) + grp * 2);
-      // two groups share a metadata byte: even group low nibble, odd group high nibble
-      uint32_t other = __shfl_xor(nib, 8);     // lane with grp^1 (same rchunk)
-      if ((grp & 1) == 0) s_meta[lr * MPITCH + (grp >> 1)] = (uint8_t)(nib | (other << 4));
+      Pack<Out, 4> out;
+      uint32_t mbyte = 0;
+#pragma unroll
+      for (int g = 0; g < 2; g++) {
+        float x[4];
+        MaskT mrow[4];
+#pragma unroll
+        for (int c = 0; c < 4; c++) { x[c] = to_float(in[4 * g + c].v[i]); if constexpr (MODE == TF24_PRUNE_MASK) mrow[c] = mk[4 * g + c].v[i]; }
+        float u0 = 0.f, u1 = 0.f;
+        if constexpr (MODE == TF24_PRUNE_MVUE) { u0 = rr[2 * g].v[i]; u1 = rr[2 * g + 1].v[i]; }
+        if (rowsum_partial) psum[i] += (x[0] + x[1]) + (x[2] + x[3]);
+        Pack<Out, 2> o;
+        mbyte |= prune_group<In, Out, MODE, MaskT>(x, mrow, u0, u1, o) << (4 * g);
+        out.v[2 * g] = o.v[0];
+        out.v[2 * g + 1] = o.v[1];
+      }
+      out.store(reinterpret_cast<Out*>(s_val + lr * VPITCH) + unit * 4);
+      s_meta[lr * MPITCH + unit] = (uint8_t)mbyte;
     }
   }
   if (rowsum_partial) {
 #pragma unroll
-    for (int i = 0; i < R; i++) s_sum[(rchunk * R + i) * SPITCH + grp] = psum[i];
+    for (int i = 0; i < R; i++) s_sum[(rchunk * R + i) * SPITCH + unit] = psum[i];
   }
   __syncthreads();
   if (rowsum_partial && tid < TR && row0 + tid < m) {
     float t = 0.0f;
-    for (int g = 0; g < TC / 4; g++) t += s_sum[tid * SPITCH + g];
+    for (int u = 0; u < TC / 8; u++) t += s_sum[tid * SPITCH + u];
     rowsum_partial[(int64_t)blockIdx.y * m + row0 + tid] = t;
   }
   // values: TR rows x (TC/2)*sizeof(Out) bytes, 16 bytes per lane.  Canonical output: row gr, byte
@@ -451,7 +427,7 @@ prune_compress_col(const In* __restrict__ dense, int64_t ld, int64_t m, int64_t 
     const int64_t gr = row0 + lr;
     const int64_t gbyte = (col0 >> 1) * sizeof(Out) + seg * 16;
     if (lr < TR && gr < m && gbyte < vpitch_out) {
-      // LDS rows are padded by 4 bytes, so read as four dwords
+      // LDS rows are padded by 8 (4) bytes, so read as four dwords
       const uint32_t* sp = reinterpret_cast<const uint32_t*>(s_val + lr * VPITCH + seg * 16);
       uint4 v = make_uint4(sp[0], sp[1], sp[2], sp[3]);
       int64_t dst = gr * vpitch_out + gbyte;
@@ -491,8 +467,16 @@ rowsum_finish(const float* __restrict__ partial, int nblocks, int64_t m, T* __re
   const int lr = threadIdx.x & 31, part = threadIdx.x >> 5;
   const int64_t r = (int64_t)blockIdx.x * 32 + lr;
   float t = 0.0f;
-  if (r < m)
-    for (int b = part; b < nblocks; b += 8) t += partial[(int64_t)b * m + r];
+  if (r < m) {
+    // eight loads in flight: waiting for each made this tail 5 us long on 96 column blocks
+    for (int b = part; b < nblocks; b += 64) {
+      float v[8];
+#pragma unroll
+      for (int u = 0; u < 8; u++) v[u] = b + 8 * u < nblocks ? partial[(int64_t)(b + 8 * u) * m + r] : 0.0f;
+#pragma unroll
+      for (int u = 0; u < 8; u++) t += v[u];
+    }
+  }
   s_part[part][lr] = t;
   __syncthreads();
   if (part == 0 && r < m) {
@@ -536,13 +520,15 @@ int launch(const void* dense, int layout, int64_t ld, int64_t m, int64_t k, cons
       hipLaunchKernelGGL((prune_compress_row_mag16<In, Out>), grid, dim3(kThreads), 0, stream,
                          (const In*)dense, ld, m, k, (Out*)values, (uint8_t*)meta, contiguous, panel, lpr_shift);
     } else {
-      hipLaunchKernelGGL((prune_compress_row<In, Out, MODE, MaskT>), grid, dim3(kThreads), 0, stream,
-                         (const In*)dense, ld, m, k, (const MaskT*)mask, mask_ld, rs, (Out*)values, (uint8_t*)meta,
-                         contiguous, panel, lpr_shift);
+      auto go = [&](auto to_panel) {
+        hipLaunchKernelGGL((prune_compress_row<In, Out, MODE, MaskT, decltype(to_panel)::value>), grid, dim3(kThreads), 0, stream,
+                           (const In*)dense, ld, m, k, (const MaskT*)mask, mask_ld, rs, (Out*)values, (uint8_t*)meta, contiguous, lpr_shift);
+      };
+      if (panel) go(std::true_type{}); else go(std::false_type{});
     }
   } else {
-    constexpr int R = 16 / sizeof(In);
-    dim3 grid((unsigned)((m + 8 * R - 1) / (8 * R)), (unsigned)((k + 127) / 128));
+    constexpr int TR = 128 / sizeof(In);       // rows of a block's tile
+    dim3 grid((unsigned)((m + TR - 1) / TR), (unsigned)((k + 127) / 128));
     hipLaunchKernelGGL((prune_compress_col<In, Out, MODE, MaskT>), grid, dim3(kThreads), 0, stream,
                        (const In*)dense, ld, m, k, (const MaskT*)mask, mask_ld, rs, (Out*)values, (uint8_t*)meta, panel,
                        rowsum_partial);

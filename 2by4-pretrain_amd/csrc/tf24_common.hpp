@@ -4,6 +4,7 @@
 #include <stdint.h>
 
 #include <initializer_list>
+#include <type_traits>
 
 #include "tf24.h"
 
@@ -218,6 +219,17 @@ struct Pack {
   }
 };
 
+// The bytes of 4 adjacent lanes as one word, lane 0's lowest (in every lane of the quad that matters, the first): data
+// parallel primitives move them between lanes without the LDS round trip of a shuffle.
+__device__ __forceinline__ uint32_t quad_bytes(uint32_t b) {
+  const uint32_t b1 = (uint32_t)__builtin_amdgcn_mov_dpp((int)b, 0x55, 0xf, 0xf, true);      // quad_perm [1,1,1,1]
+  const uint32_t b2 = (uint32_t)__builtin_amdgcn_mov_dpp((int)b, 0xaa, 0xf, 0xf, true);      // [2,2,2,2]
+  const uint32_t b3 = (uint32_t)__builtin_amdgcn_mov_dpp((int)b, 0xff, 0xf, 0xf, true);      // [3,3,3,3]
+  return b | (b1 << 8) | (b2 << 16) | (b3 << 24);
+}
+// the value of the lane 8 away inside its row of 16 (row_ror:8)
+__device__ __forceinline__ uint32_t xor8_lane(uint32_t v) { return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x128, 0xf, 0xf, true); }
+
 // ---------------------------------------------------------------- 2:4 group math
 // The kept elements of one group as four flags, and what the reference's 16-row table
 // (_semi_structured_conversions.py:46-82) makes of them: idx0 = 0 if m0, else 1 if m1, else 2;
@@ -228,8 +240,8 @@ struct Pack {
 // vector instructions.
 struct Keep4 {
   bool m0, m1, m2, m3;
-  __device__ __forceinline__ bool second_is_1() const { return m0 & m1 & !m2; }
-  __device__ __forceinline__ bool second_is_2() const { return m2 & (m0 | m1); }
+  __device__ __forceinline__ bool second_is_1() const { return m0 && m1 && !m2; }
+  __device__ __forceinline__ bool second_is_2() const { return m2 && (m0 || m1); }
   template <typename T> __device__ __forceinline__ T first(T v0, T v1, T v2) const { return m0 ? v0 : (m1 ? v1 : v2); }
   template <typename T> __device__ __forceinline__ T second(T v1, T v2, T v3) const { return second_is_1() ? v1 : (second_is_2() ? v2 : v3); }
   // pos0 | pos1 << 2
@@ -295,20 +307,25 @@ __device__ __forceinline__ T select4(uint32_t pos, T v0, T v1, T v2, T v3) {
   return (pos & 2) ? hi : lo;
 }
 
-// Float32 division for operands inside the normal range.  This is the arithmetic the compiler's
-// own division performs between its v_div_scale and v_div_fixup steps: one Newton step on
-// v_rcp_f32, then two residual corrections of the quotient.  It returns the correctly rounded
-// quotient whenever v_div_scale would leave both operands unscaled and v_div_fixup would pass the
-// result through: numerator and denominator finite, non-zero and normal, |numerator| > 2^-104,
-// denominator < 2^126, exponent difference below 96 and a normal quotient.  Callers establish those
-// bounds and use operator/ outside them.  A reciprocal can be shared between quotients.
+// Float32 division for operands inside the normal range, correctly rounded in five instructions (a reciprocal can be
+// shared by several quotients).
+//   refined_rcp: one Newton step on v_rcp_f32.  On gfx950 the result is RN(1/b) for every b from 2^-126 up to 2^126
+//     (all 2.1e9 bit patterns compared with 1/b in float64).
+//   div_in_range: q = RN(a r), then ONE residual correction.  With a, b in [1, 2) and r = RN(1/b), q is off by less
+//     than a/2 + 1/2 units in its last place when a < b and by less than 1 when a >= b.  A quotient of two 24-bit
+//     numbers is never closer than 2^-25 units to a midpoint between two floats (the distance is a non-zero multiple of
+//     1/(2B), B < 2^24 the integer of b), and beside a midpoint q is therefore off by half a unit (one and a half would
+//     take a = 2 - 2^-23 < b < 2).  There the residual is exact and the corrected sum, before its one rounding, is off by
+//     at most 2^-25 b/2 < 2^-25 units: it rounds as the quotient does.  (Compared with the float64 quotient on 1e11
+//     random and adversarial pairs; the general sequence takes a second correction because it does not assume r.)
+// Needed: numerator and denominator normal, |numerator| > 2^-104, denominator < 2^126, exponent difference below 96
+// and a normal quotient.  Callers establish those bounds and use operator/ outside them.
 __device__ __forceinline__ float refined_rcp(float b) {
   float r = __builtin_amdgcn_rcpf(b);
   return __builtin_fmaf(__builtin_fmaf(-b, r, 1.0f), r, r);
 }
 __device__ __forceinline__ float div_in_range(float a, float b, float r) {
-  float q = a * r;
-  q = __builtin_fmaf(__builtin_fmaf(-b, q, a), r, q);
+  const float q = a * r;
   return __builtin_fmaf(__builtin_fmaf(-b, q, a), r, q);
 }
 
@@ -345,29 +362,28 @@ struct RandSrc {
 };
 
 // MVUE24 of one group in float32, in the reference's operation order (no contraction): inclusion
-// probabilities p_i and the kept-mask bits.  The kept values are x_i / p_i (mvue_rescale); only
-// the two kept ones need the division.
-//
-// in_range: |x_i| + eps >= 2^-23 always, so with sum < 2^40 and every s_i = sum - a_i > 0 (then
-// s_i >= 2^-46) the quotients t_i = a_i/sum >= 2^-63 and k_i = t_i/s_i >= 2^-104 meet the bounds of
-// div_in_range; p_i >= t_i because k >= k_i for a rounded sum of non-negatives.
+// probabilities p_i, the kept elements, and the two kept values x_i / p_i in ascending position.  Only the two kept
+// values are divided.
 struct Mvue4 {
-  float p[4];
-  Keep4 keep;
-  bool in_range;
+  uint32_t nibble, bits;      // of the kept flags (as words: flags merged behind a branch would be rebuilt from registers)
+  float first, second;
 };
 
-__device__ __forceinline__ Mvue4 mvue4(float x0, float x1, float x2, float x3, float r0, float r1) {
+// FAST: every division through div_in_range, in straight-line code; `ok` says whether the bounds of div_in_range held
+// throughout (if not, the result is not to be used).  |x_i| + eps >= 2^-23 always, so with sum < 2^40 and every
+// s_i = sum - a_i > 0 (then s_i >= 2^-46) the quotients t_i = a_i/sum >= 2^-63 and k_i = t_i/s_i >= 2^-104 meet them;
+// p_i >= t_i because k >= k_i for a rounded sum of non-negatives, so p_i in [2^-63, 2] once it is at most 2, and
+// |x_i| <= sum p_i keeps the exponents within 96 of each other; |x_i| >= 2^-100 or x_i = 0 keeps the quotient normal or
+// zero.  (Half precision, WIDE = false, holds neither a sum of 2^40 nor a value below 2^-100.)
+template <bool FAST, bool WIDE>
+__device__ __forceinline__ Mvue4 mvue4_as(const float (&x)[4], float r0, float r1, bool& ok) {
   const float eps = 1.19209e-07f;
-  float a0 = __builtin_fabsf(x0) + eps, a1 = __builtin_fabsf(x1) + eps;
-  float a2 = __builtin_fabsf(x2) + eps, a3 = __builtin_fabsf(x3) + eps;
-  float sum = ((a0 + a1) + a2) + a3;
-  float s0 = sum - a0, s1 = sum - a1, s2 = sum - a2, s3 = sum - a3;
-  Mvue4 g;
-  // every s_i > 0  <=>  their minimum is (none of them is a NaN when sum < 2^40: all a_i are finite then)
-  g.in_range = (sum < 0x1p40f) && (__builtin_fminf(__builtin_fminf(s0, s1), __builtin_fminf(s2, s3)) > 0.0f);
+  const float a0 = __builtin_fabsf(x[0]) + eps, a1 = __builtin_fabsf(x[1]) + eps;
+  const float a2 = __builtin_fabsf(x[2]) + eps, a3 = __builtin_fabsf(x[3]) + eps;
+  const float sum = ((a0 + a1) + a2) + a3;
+  const float s0 = sum - a0, s1 = sum - a1, s2 = sum - a2, s3 = sum - a3;
   float t0, t1, t2, t3, k0, k1, k2, k3;
-  if (g.in_range) {
+  if constexpr (FAST) {
     const float rs = refined_rcp(sum);
     t0 = div_in_range(a0, sum, rs); t1 = div_in_range(a1, sum, rs);
     t2 = div_in_range(a2, sum, rs); t3 = div_in_range(a3, sum, rs);
@@ -377,34 +393,80 @@ __device__ __forceinline__ Mvue4 mvue4(float x0, float x1, float x2, float x3, f
     t0 = a0 / sum; t1 = a1 / sum; t2 = a2 / sum; t3 = a3 / sum;
     k0 = t0 / s0; k1 = t1 / s1; k2 = t2 / s2; k3 = t3 / s3;
   }
-  float k = ((k0 + k1) + k2) + k3;
-  g.p[0] = t0 + a0 * (k - k0); g.p[1] = t1 + a1 * (k - k1);
-  g.p[2] = t2 + a2 * (k - k2); g.p[3] = t3 + a3 * (k - k3);
-  bool m0 = r0 <= t0;
-  bool m1 = (r0 <= (t0 + t1)) & !m0;
-  bool m2 = (r0 <= ((t0 + t1) + t2)) & !m1 & !m0;
-  bool m3 = !m2 & !m1 & !m0;
-  float d0 = m0 ? 0.0f : a0, d1 = m1 ? 0.0f : a1, d2 = m2 ? 0.0f : a2, d3 = m3 ? 0.0f : a3;
-  float dsum = ((d0 + d1) + d2) + d3;
-  float t = r1 * dsum;
-  bool e0 = t <= d0;
-  bool e1 = (t <= (d0 + d1)) & !e0;
-  bool e2 = (t <= ((d0 + d1) + d2)) & !e1 & !e0;
-  bool e3 = !e2 & !e1 & !e0;
-  g.keep.m0 = m0 | e0; g.keep.m1 = m1 | e1; g.keep.m2 = m2 | e2; g.keep.m3 = m3 | e3;
+  const float k = ((k0 + k1) + k2) + k3;
+  const float p0 = t0 + a0 * (k - k0), p1 = t1 + a1 * (k - k1), p2 = t2 + a2 * (k - k2), p3 = t3 + a3 * (k - k3);
+  const bool m0 = r0 <= t0;
+  const bool m1 = r0 <= (t0 + t1) && !m0;
+  const bool m2 = r0 <= ((t0 + t1) + t2) && !m1 && !m0;
+  const bool m3 = !m2 && !m1 && !m0;
+  const float d0 = m0 ? 0.0f : a0, d1 = m1 ? 0.0f : a1, d2 = m2 ? 0.0f : a2, d3 = m3 ? 0.0f : a3;
+  const float dsum = ((d0 + d1) + d2) + d3;
+  const float t = r1 * dsum;
+  const bool e0 = t <= d0;
+  const bool e1 = t <= (d0 + d1) && !e0;
+  const bool e2 = t <= ((d0 + d1) + d2) && !e1 && !e0;
+  const bool e3 = !e2 && !e1 && !e0;
+  const Keep4 keep{m0 || e0, m1 || e1, m2 || e2, m3 || e3};
+  const float xa = keep.first(x[0], x[1], x[2]), xb = keep.second(x[1], x[2], x[3]);
+  const float pa = keep.first(p0, p1, p2), pb = keep.second(p1, p2, p3);
+  Mvue4 g;
+  g.nibble = keep.nibble();
+  g.bits = keep.bits();
+  if constexpr (FAST) {
+    // div_in_range with the residual's sign turned round, which keeps the sign of a zero numerator
+    const float ra = refined_rcp(pa), rb = refined_rcp(pb);
+    const float qa = xa * ra, qb = xb * rb;
+    g.first = __builtin_fmaf(-__builtin_fmaf(pa, qa, -xa), ra, qa);
+    g.second = __builtin_fmaf(-__builtin_fmaf(pb, qb, -xb), rb, qb);
+    // an s_i of zero (they are never negative) makes its reciprocal, k and with it every p a NaN: no test of its own
+    ok = pa <= 2.0f && pb <= 2.0f;
+    if constexpr (WIDE) {        // In can hold what half precision cannot: a sum of 2^40, values below 2^-100
+      ok = ok && sum < 0x1p40f;
+      // 0 or at least 2^-100 (0x0d800000), for both: one less than zero wraps round
+      const uint32_t ua = (__builtin_bit_cast(uint32_t, xa) & 0x7fffffffu) - 1u, ub = (__builtin_bit_cast(uint32_t, xb) & 0x7fffffffu) - 1u;
+      ok = ok && (ua < ub ? ua : ub) >= 0x0d800000u - 1u;
+    }
+  } else {
+    g.first = xa / pa;
+    g.second = xb / pb;
+    ok = true;
+  }
   return g;
 }
 
-// x / p for a value of a group whose probabilities came from mvue4.  In range: p in [2^-63, 2],
-// |x| <= sum * p (so the exponent difference stays below 96) and |x| >= 2^-100 keeps the quotient
-// normal; a zero numerator returns the signed zero the division would.
-__device__ __forceinline__ float mvue_rescale(float x, float p, bool in_range) {
-  const bool ok = in_range & (p <= 2.0f) & ((x == 0.0f) | (__builtin_fabsf(x) >= 0x1p-100f));
-  if (ok) {
-    float q = div_in_range(x, p, refined_rcp(p));
-    return x == 0.0f ? x : q;
+// What bounds the kernels that call this, when the uniforms are drawn in the kernel, is the vector ALU.  Rates measured
+// on gfx950, in lanes per clock of the chip: float32 add, multiply, fma and the bitwise operations 32768; compares,
+// selects, minima, shifts, conversions and 32-bit multiplies 16384; v_rcp_f32 8192.  In units of the middle rate a group
+// costs 80 (half precision) to 85, a generator call 50 for two groups.  One correction per division instead of two, no
+// branch and one test of the bounds per group (the slow path is laid out behind the kernel), flags as short-circuit
+// expressions (as integers they went through vector registers), kept values converted without a test for NaN, and leaner
+// addresses in the callers: 8192 x 8192 bf16 to e4m3 82 -> 64.5 us, to fp16 78.6 -> 64.5 (with a supplied tensor, where
+// its 268 MB are the bound, 77 -> 69), a column-major 3072 x 12288 half matrix with its row sums 54.5 -> 44 us.
+template <typename In>
+__device__ __forceinline__ Mvue4 mvue4(const float (&x)[4], float r0, float r1, bool& finite) {
+  bool ok;
+  Mvue4 g = mvue4_as<true, !std::is_same<In, f16_t>::value>(x, r0, r1, ok);
+  finite = ok;
+  if (__builtin_expect(!ok, 0)) g = mvue4_as<false, false>(x, r0, r1, ok);
+  return g;
+}
+
+// Two values next to each other as they are stored, `finite`: neither is a NaN (spares the 8-bit types the test).
+template <typename Out>
+__device__ __forceinline__ Pack<Out, 2> from_float2(float a, float b, bool finite) {
+  Pack<Out, 2> o;
+  if constexpr (std::is_same<Out, e4m3_t>::value || std::is_same<Out, e5m2_t>::value) {
+    uint32_t w;
+    if constexpr (std::is_same<Out, e4m3_t>::value) w = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(a, b, 0, false);
+    else w = (uint32_t)__builtin_amdgcn_cvt_pk_bf8_f32(a, b, 0, false);
+    if (__builtin_expect(!finite, 0)) w = (uint32_t)from_float<Out>(a).bits | ((uint32_t)from_float<Out>(b).bits << 8);
+    o.v[0].bits = (uint8_t)w;
+    o.v[1].bits = (uint8_t)(w >> 8);
+  } else {
+    o.v[0] = from_float<Out>(a);
+    o.v[1] = from_float<Out>(b);
   }
-  return x / p;
+  return o;
 }
 
 }  // namespace tf24
