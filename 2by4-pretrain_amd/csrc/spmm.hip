@@ -3,10 +3,11 @@
 // spmm_e5m2.hip, spmm_i8.hip), so that they compile side by side.
 #include "spmm_kernels.hpp"
 
-extern "C" int tf24_spmm_validate(int dtype, int64_t n_sparse, int64_t k, int b_layout, int64_t ldb, int64_t n_dense,
-                                  int out_dtype, int c_layout, int64_t ldc, int activation) {
-  using namespace tf24;
-  const char* fn = "tf24_spmm";
+namespace tf24 {
+namespace {
+// extent: what the number of dense columns must be a multiple of (0: the operand type's own)
+int validate(const char* fn, int dtype, int64_t n_sparse, int64_t k, int b_layout, int64_t ldb, int64_t n_dense, int64_t extent,
+             int out_dtype, int c_layout, int64_t ldc, int activation) {
   if (dtype != TF24_F16 && dtype != TF24_BF16 && !is_8bit(dtype)) return fail(TF24_ERR_DTYPE, "%s: unsupported operand dtype %d", fn, dtype);
   if (dtype == TF24_I8) {
     // integer product (.cu:594-637): int32 results, no or ReLU activation
@@ -19,7 +20,7 @@ extern "C" int tf24_spmm_validate(int dtype, int64_t n_sparse, int64_t k, int b_
   const int64_t kmult = eight ? 128 : 64, dmult = eight ? 16 : 8;
   if (n_sparse <= 0 || n_sparse % 32) return fail(TF24_ERR_SHAPE, "%s: sparse operand rows %lld must be a positive multiple of 32", fn, (long long)n_sparse);
   if (k <= 0 || k % kmult) return fail(TF24_ERR_SHAPE, "%s: inner dimension %lld must be a positive multiple of %lld", fn, (long long)k, (long long)kmult);
-  if (n_dense <= 0 || n_dense % dmult) return fail(TF24_ERR_SHAPE, "%s: dense operand extent %lld must be a positive multiple of %lld", fn, (long long)n_dense, (long long)dmult);
+  if (n_dense <= 0 || n_dense % (extent ? extent : dmult)) return fail(TF24_ERR_SHAPE, "%s: dense operand extent %lld must be a positive multiple of %lld", fn, (long long)n_dense, (long long)(extent ? extent : dmult));
   if (b_layout != TF24_ROW_MAJOR && b_layout != TF24_COL_MAJOR) return fail(TF24_ERR_ARG, "%s: bad b_layout %d", fn, b_layout);
   if (c_layout != TF24_ROW_MAJOR && c_layout != TF24_COL_MAJOR) return fail(TF24_ERR_ARG, "%s: bad c_layout %d", fn, c_layout);
   const int64_t bext = b_layout == TF24_ROW_MAJOR ? k : n_dense;
@@ -32,6 +33,13 @@ extern "C" int tf24_spmm_validate(int dtype, int64_t n_sparse, int64_t k, int b_
   if (ldc < cext || ldc % cmult) return fail(TF24_ERR_STRIDE, "%s: ldc %lld must be >= %lld and a multiple of %lld", fn, (long long)ldc, (long long)cext, (long long)cmult);
   if (activation < TF24_ACT_NONE || activation > TF24_ACT_GELU) return fail(TF24_ERR_ARG, "%s: bad activation %d", fn, activation);
   return TF24_OK;
+}
+}  // namespace
+}  // namespace tf24
+
+extern "C" int tf24_spmm_validate(int dtype, int64_t n_sparse, int64_t k, int b_layout, int64_t ldb, int64_t n_dense,
+                                  int out_dtype, int c_layout, int64_t ldc, int activation) {
+  return tf24::validate("tf24_spmm", dtype, n_sparse, k, b_layout, ldb, n_dense, 0, out_dtype, c_layout, ldc, activation);
 }
 
 namespace tf24 {
@@ -56,22 +64,22 @@ extern "C" int64_t tf24_spmm_workspace_bytes(int dtype, int64_t n_sparse, int64_
   return bytes;
 }
 
-extern "C" int tf24_spmm(const void* a_values, const void* a_meta, int a_layout, int dtype, int64_t n_sparse, int64_t k,
-                         const void* b, int b_layout, int64_t ldb, int64_t n_dense,
-                         void* c, int out_dtype, int c_layout, int64_t ldc,
-                         const void* bias, float scale, int activation, void* workspace, int64_t workspace_bytes, void* stream) {
-  using namespace tf24;
-  int rc = tf24_spmm_validate(dtype, n_sparse, k, b_layout, ldb, n_dense, out_dtype, c_layout, ldc, activation);
+namespace tf24 {
+namespace {
+int run_spmm(const char* fn, const void* a_values, const void* a_meta, int a_layout, int dtype, int64_t n_sparse, int64_t k,
+             const void* b, int b_layout, int64_t ldb, int64_t n_dense, int64_t extent, void* c, int out_dtype, int c_layout, int64_t ldc,
+             const void* bias, float scale, int activation, void* workspace, int64_t workspace_bytes, void* stream) {
+  int rc = validate(fn, dtype, n_sparse, k, b_layout, ldb, n_dense, extent, out_dtype, c_layout, ldc, activation);
   if (rc) return rc;
-  if (!a_values || !a_meta || !b || !c) return fail(TF24_ERR_ARG, "tf24_spmm: null pointer");
-  if ((rc = check_aligned("tf24_spmm", 16, {a_values, b, c, workspace}))) return rc;
+  if (!a_values || !a_meta || !b || !c) return fail(TF24_ERR_ARG, "%s: null pointer", fn);
+  if ((rc = check_aligned(fn, 16, {a_values, b, c, workspace}))) return rc;
   // panel metadata is copied 16 bytes per lane; canonical metadata is read in words of up to 4 bytes, row pitch k/8
-  if ((rc = check_aligned("tf24_spmm", a_layout == TF24_COMPRESSED_PANEL ? 16 : a_layout == TF24_COMPRESSED_CUTLASS ? 4 : 8, {a_meta}))) return rc;
-  if ((rc = check_aligned("tf24_spmm", dtype_size(out_dtype), {bias}))) return rc;
+  if ((rc = check_aligned(fn, a_layout == TF24_COMPRESSED_PANEL ? 16 : a_layout == TF24_COMPRESSED_CUTLASS ? 4 : 8, {a_meta}))) return rc;
+  if ((rc = check_aligned(fn, dtype_size(out_dtype), {bias}))) return rc;
   if (a_layout != TF24_COMPRESSED_CANONICAL && a_layout != TF24_COMPRESSED_PANEL && a_layout != TF24_COMPRESSED_CUTLASS)
-    return fail(TF24_ERR_ARG, "tf24_spmm: bad compressed layout %d", a_layout);
+    return fail(TF24_ERR_ARG, "%s: bad compressed layout %d", fn, a_layout);
   hipStream_t s = (hipStream_t)stream;
-  if (dtype == TF24_I8 && scale != 1.0f) return fail(TF24_ERR_ARG, "tf24_spmm: int8 products are exact, scale must be 1 (%g given)", (double)scale);
+  if (dtype == TF24_I8 && scale != 1.0f) return fail(TF24_ERR_ARG, "%s: int8 products are exact, scale must be 1 (%g given)", fn, (double)scale);
   switch (dtype) {
     case TF24_I8: return spmm_i8(out_dtype, a_values, a_meta, a_layout, n_sparse, k, b, b_layout, ldb, n_dense, c, c_layout, ldc, bias, scale, activation, workspace, workspace_bytes, s);
     case TF24_F16: return spmm_f16(out_dtype, a_values, a_meta, a_layout, n_sparse, k, b, b_layout, ldb, n_dense, c, c_layout, ldc, bias, scale, activation, workspace, workspace_bytes, s);
@@ -79,4 +87,26 @@ extern "C" int tf24_spmm(const void* a_values, const void* a_meta, int a_layout,
     case TF24_E5M2: return spmm_e5m2(out_dtype, a_values, a_meta, a_layout, n_sparse, k, b, b_layout, ldb, n_dense, c, c_layout, ldc, bias, scale, activation, workspace, workspace_bytes, s);
     default: return spmm_e4m3(out_dtype, a_values, a_meta, a_layout, n_sparse, k, b, b_layout, ldb, n_dense, c, c_layout, ldc, bias, scale, activation, workspace, workspace_bytes, s);
   }
+}
+}  // namespace
+}  // namespace tf24
+
+extern "C" int tf24_spmm(const void* a_values, const void* a_meta, int a_layout, int dtype, int64_t n_sparse, int64_t k,
+                         const void* b, int b_layout, int64_t ldb, int64_t n_dense,
+                         void* c, int out_dtype, int c_layout, int64_t ldc,
+                         const void* bias, float scale, int activation, void* workspace, int64_t workspace_bytes, void* stream) {
+  return tf24::run_spmm("tf24_spmm", a_values, a_meta, a_layout, dtype, n_sparse, k, b, b_layout, ldb, n_dense, 0, c, out_dtype, c_layout, ldc,
+                        bias, scale, activation, workspace, workspace_bytes, stream);
+}
+
+// Rows of x are the dense columns with k contiguous, rows of y the output stored j-major: in that orientation no kernel
+// loads or stores more than one row of either with one access, rows past the last are clamped on loads and skipped on
+// stores, so any number of rows goes (in the other orientations 16-byte accesses run along the dense columns).
+// A copy padded to a multiple of 8 rows costs what it moves: 3001 x 11008 bf16 36 us beside a product of 131 us, one row of
+// 4096 two launches of 3.5 us beside one of 13 us.
+extern "C" int tf24_linear(const void* a_values, const void* a_meta, int a_layout, int dtype, int64_t n_sparse, int64_t k,
+                           const void* x, int64_t ldx, int64_t rows, void* y, int out_dtype, int64_t ldy,
+                           const void* bias, float scale, int activation, void* workspace, int64_t workspace_bytes, void* stream) {
+  return tf24::run_spmm("tf24_linear", a_values, a_meta, a_layout, dtype, n_sparse, k, x, TF24_ROW_MAJOR, ldx, rows, 1, y, out_dtype,
+                        TF24_COL_MAJOR, ldy, bias, scale, activation, workspace, workspace_bytes, stream);
 }

@@ -229,6 +229,9 @@ def _spmm(sparse, dense, sparse_first, bias=None, out_dtype=None, scale=1.0, act
     else:
         dense = dense.contiguous()
         lay, ld = N.ROW_MAJOR, dense.stride(0)
+    if lay == N.COL_MAJOR and not sparse_first and d0 % 8:
+        dense = dense.contiguous()               # any number of rows, but only with k contiguous
+        lay, ld = N.ROW_MAJOR, dense.stride(0)
     # When k is the strided dimension of the dense operand (`S @ dense` with a row-major dense, e.g.
     # dW = MVUE(dY^T) @ x) the tiled kernel reads 16-bit operands as they are, transposing while it
     # loads fragments.  For 8-bit operands it wants k contiguous: one transposing copy of the dense
@@ -274,24 +277,28 @@ def _spmm(sparse, dense, sparse_first, bias=None, out_dtype=None, scale=1.0, act
     if ws_bytes is None:
         ws_bytes = _WORKSPACE_BYTES[ws_key] = lib.tf24_spmm_workspace_bytes(code, n, k, j)
     workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=device) if ws_bytes else None
-    N.check(lib.tf24_spmm(
-        values.data_ptr(), meta.data_ptr(), store_layout, code, n, k,
-        dense.data_ptr(), b_layout, ld, j, out.data_ptr(), N.operand_code(out_dtype), c_layout, out_shape[1],
-        None if bias is None else bias.data_ptr(), float(scale), activation,
-        None if workspace is None else workspace.data_ptr(), ws_bytes, N.stream_ptr()))
+    tail = (None if bias is None else bias.data_ptr(), float(scale), activation,
+            None if workspace is None else workspace.data_ptr(), ws_bytes, N.stream_ptr())
+    if not sparse_first and lay == N.ROW_MAJOR:
+        N.check(lib.tf24_linear(values.data_ptr(), meta.data_ptr(), store_layout, code, n, k, dense.data_ptr(), ld, j,
+                                out.data_ptr(), N.operand_code(out_dtype), n, *tail))
+    else:
+        N.check(lib.tf24_spmm(values.data_ptr(), meta.data_ptr(), store_layout, code, n, k, dense.data_ptr(), b_layout, ld, j,
+                              out.data_ptr(), N.operand_code(out_dtype), c_layout, out_shape[1], *tail))
     return out
 
 
 def _dense_times_sparse_t(dense2d, sparse, bias=None):
-    """dense2d @ S.t() (+ bias): what `torch.mm(x, S.t())` / `torch.addmm(bias, x, S.t())` dispatch to, without
-    building the transposed wrapper and without the dispatcher round trip (some 40 us of host time per
-    product, which a training step that is bound by its launch rate pays three times)."""
+    """dense2d @ S.t() (+ bias): what `torch.mm(x, S.t())` / `torch.addmm(bias, x, S.t())` dispatch to, and what the
+    training layer calls without building the transposed wrapper and without the dispatcher round trip (some 40 us
+    of host time per product, which a training step that is bound by its launch rate pays three times).  The rows of
+    the dense operand are taken as they are, whatever their number; only a column count that no compressed
+    operand has is padded as the reference does (semi_structured.py:351-368)."""
     rows, cols = dense2d.shape
-    cfg = _DTYPE_TO_SEMI_STRUCTURED_SPARSE_CONFIG[dense2d.dtype]
-    padded = dense2d if rows % cfg.dense_min_rows == 0 and cols % cfg.dense_min_cols == 0 else sparse._pad_tensor_for_matmul(dense2d)
-    out_dtype = sparse._FP8_OUT_DTYPE if sparse._store_values.dtype in _FLOAT8 else None
-    out = _spmm(sparse, padded, False, bias=bias, out_dtype=out_dtype)
-    return out if padded is dense2d else out[:rows, :]
+    if cols % _DTYPE_TO_SEMI_STRUCTURED_SPARSE_CONFIG[dense2d.dtype].dense_min_cols == 0:
+        return _spmm(sparse, dense2d, False, bias=bias, out_dtype=sparse._out_dtype())
+    padded = sparse._pad_tensor_for_matmul(dense2d)
+    return _spmm(sparse, padded, False, bias=bias, out_dtype=sparse._out_dtype())[:rows, :]
 
 
 class SparseSemiStructuredTensor(torch.Tensor):
@@ -485,9 +492,7 @@ class SparseSemiStructuredTensor(torch.Tensor):
             bias, input_A, input_B = args
             # F.linear(x) = addmm(bias, x, W.t()) = (W x' + b')'
             if isinstance(input_B, cls) and input_B.transposed:
-                row, _ = input_A.shape
-                padded = input_B._pad_tensor_for_matmul(input_A)
-                return _spmm(input_B, padded, False, bias=bias, out_dtype=input_B._out_dtype())[:row, :]
+                return _dense_times_sparse_t(input_A, input_B, bias)
 
         if func is torch.ops.aten.mm.default:
             input_A, input_B = args
@@ -496,20 +501,14 @@ class SparseSemiStructuredTensor(torch.Tensor):
                 padded = input_A._pad_tensor_for_matmul(input_B)
                 return _spmm(input_A, padded, True, out_dtype=input_A._out_dtype())[:, :col]
             if isinstance(input_B, cls) and input_B.transposed:              # second operand sparse
-                row, _ = input_A.shape
-                padded = input_B._pad_tensor_for_matmul(input_A)
-                return _spmm(input_B, padded, False, out_dtype=input_B._out_dtype())[:row, :]
+                return _dense_times_sparse_t(input_A, input_B)
 
         # inference mode does not decompose linear into t + addmm
         if func is torch.ops.aten.linear.default:
             input_tensor, weight, bias = args
             if isinstance(weight, cls):
                 shape = input_tensor.shape
-                x2d = input_tensor.reshape(-1, shape[-1])
-                row, _ = x2d.shape
-                padded = weight._pad_tensor_for_matmul(x2d)
-                res = _spmm(weight, padded, False, bias=bias, out_dtype=weight._out_dtype())
-                return res[:row, :].view(*shape[:-1], -1)
+                return _dense_times_sparse_t(input_tensor.reshape(-1, shape[-1]), weight, bias).view(*shape[:-1], -1)
 
         if func is torch.ops.aten.values.default:
             return args[0].sparse_tensor_cutlass.detach()

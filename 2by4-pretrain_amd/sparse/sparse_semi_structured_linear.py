@@ -73,7 +73,10 @@ def sparse_semi_structured_linear(input: torch.Tensor, weight, meta: Optional[to
     shape = input.shape
     x2d = input.reshape(-1, shape[-1])
     rows = x2d.shape[0]
-    padded = weight._pad_tensor_for_matmul(x2d)
+    if x2d.dtype == weight.dtype and x2d.shape[1] == weight._store_shape[1]:
+        padded = x2d                     # any number of rows
+    else:
+        padded = weight._pad_tensor_for_matmul(x2d)
     if out_dtype is None:
         out_dtype = weight._out_dtype()
     out = _spmm(weight, padded, False, bias=bias_opt, out_dtype=out_dtype, scale=scale, activation=_ACTIVATIONS[activation_opt],

@@ -366,6 +366,15 @@ int tf24_spmm(const void* a_values, const void* a_meta, int a_layout, int dtype,
               const void* b, int b_layout, int64_t ldb, int64_t n_dense,
               void* c, int out_dtype, int c_layout, int64_t ldc,
               const void* bias, float scale, int activation, void* workspace, int64_t workspace_bytes, void* stream);
+/*
+ * y = act(scale * x . S^T + bias), x [rows, k] and y [rows, n_sparse] row-major: tf24_spmm with b_layout TF24_ROW_MAJOR and
+ * c_layout TF24_COL_MAJOR for ANY number of rows >= 1 (the reference pads the activations to multiples of 8 or 16 rows and
+ * slices the result, sparse/semi_structured.py:351-368).  Everything else as tf24_spmm; workspace of
+ * tf24_spmm_workspace_bytes(dtype, n_sparse, k, rows).
+ */
+int tf24_linear(const void* a_values, const void* a_meta, int a_layout, int dtype, int64_t n_sparse, int64_t k,
+                const void* x, int64_t ldx, int64_t rows, void* y, int out_dtype, int64_t ldy,
+                const void* bias, float scale, int activation, void* workspace, int64_t workspace_bytes, void* stream);
 int64_t tf24_spmm_workspace_bytes(int dtype, int64_t n_sparse, int64_t k, int64_t n_dense);
 
 /*

@@ -1090,3 +1090,33 @@ def test_spmm_chained_tiles_32bit_output(cuda, dtype, k, act):
         want = torch.nn.functional.silu(pre)
         assert bool(((got - want).abs() <= 2e-6 + 2e-6 * want.abs()).all())
     assert run().equal(out)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float8_e4m3fn, torch.int8])
+@pytest.mark.parametrize("n,k,rows", [(64, 128, 1), (32, 128, 7), (8192, 256, 3), (10240, 128, 15), (512, 512, 17), (288, 384, 63), (544, 2048, 65),
+                                      (768, 256, 127), (256, 4096, 129), (4096, 1024, 255), (3072, 768, 1025), (2304, 4096, 2049), (1600, 6400, 4001)])
+def test_linear_any_number_of_rows(cuda, dtype, n, k, rows):
+    """tf24_linear against the float32 product on small integers (exact), row counts that are multiples of nothing and
+    reach every kernel and tile width; the rows behind the last stay as they were."""
+    import sparse
+    from sparse import _native as N
+    g = torch.Generator().manual_seed(rows)
+    w = torch.randint(-2, 3, (n, k), generator=g).float()
+    src = w.to(torch.int8) if dtype == torch.int8 else w
+    s = sparse.to_sparse_semi_structured(src.to(cuda), dtype=dtype)
+    x = torch.randint(-2, 3, (rows, k), generator=g).float().to(cuda)
+    out_dtype = torch.int32 if dtype == torch.int8 else torch.float32
+    want = (x @ s.to_dense().float().t()).to(out_dtype)
+    xs = x.to(dtype)
+    y = torch.full((rows + 5, n), 77, dtype=out_dtype, device=cuda)
+    code = N.operand_code(dtype)
+    ws_bytes = N.lib().tf24_spmm_workspace_bytes(code, n, k, rows)
+    ws = torch.empty(max(ws_bytes, 16), dtype=torch.uint8, device=cuda)
+    for ws_ptr, ws_len in ((ws.data_ptr(), ws_bytes), (None, 0)):
+        y[:rows] = 0
+        N.check(N.lib().tf24_linear(s._store_values.data_ptr(), s._store_meta.data_ptr(), N.COMPRESSED_PANEL, code, n, k, xs.data_ptr(), k, rows,
+                                    y.data_ptr(), N.operand_code(out_dtype), n, None, 1.0, N.ACT_NONE, ws_ptr, ws_len, N.stream_ptr()))
+        assert y[:rows].equal(want)
+        assert bool((y[rows:] == 77).all())
+    got = torch.mm(xs, s.t())
+    assert got.shape == (rows, n) and got.float().equal(want.to(got.dtype).float())
