@@ -47,7 +47,7 @@ namespace {
 template <typename C>
 int64_t split_bytes(int dtype, int64_t n_sparse, int64_t k, int64_t n_dense) {
   const int64_t big = (int64_t)1 << 40;
-  const int splits = is_8bit(dtype) ? choose_splits<e4m3_t, C>(n_sparse, k, n_dense, big) : choose_splits<f16_t, C>(n_sparse, k, n_dense, big);
+  const int splits = is_8bit(dtype) ? choose_splits<e4m3_t, C>(n_sparse, k, n_dense, big, true) : choose_splits<f16_t, C>(n_sparse, k, n_dense, big, true);
   if (splits < 2) return 0;
   const int64_t tiles = ((n_sparse + C::BI - 1) / C::BI) * ((n_dense + C::BJ - 1) / C::BJ);
   return splits * tiles * C::BI * C::BJ * 4;

@@ -1031,36 +1031,37 @@ spmm_reduce_splits(const float* __restrict__ partial, int splits, int tiles_i, i
   }
 }
 
-// k-splits for shapes whose tiles cannot fill the 256 CUs (k-heavy products such as dW): as many as
-// fit, each at least 4 stages long, if the caller's workspace holds the float32 partial tiles.
+// How many k pieces a product is cut into, for shapes whose tiles cannot fill the 256 compute units: the number for which
+//     stages of one piece x STAGE_US + (pieces > 1: SPLIT_US + MB of partial tiles, all pieces, x PARTIAL_US)
+// is least, among those whose blocks fit one round (two blocks of the narrowest tiles share a compute unit) and whose
+// float32 partial tiles fit the caller's workspace.  The constants are the least-squares fit, per tile configuration, to
+// 560 timings of 1 to 16 pieces over weights from 768 x 768 to 8192 x 8192 (12 to 192 stages) and 20 to 3000 dense
+// columns; the pieces chosen this way are within 1 % of the best ones on average (6 % at worst), where 192 / tiles pieces
+// were 14 % off: a piece of few stages saves less than its partial tiles cost.  us, before and after:
+// 3072 x 768 against 1024 columns 22.2 -> 9.0 (2 pieces -> 1), 768 x 3072 20.6 -> 16.5 (8 -> 3), 4096 x 4096 against 128
+// columns 19.0 -> 16.1 (12 -> 4); dW of 1024 tokens, 3072 x 768, 26.2 -> 16.4 (4 -> 1).  (The partial tiles of the
+// k-strided products count a fifth more than the fit says: inside a training step they leave the caches, and with dW of
+// 12288 tokens in six pieces instead of five the step took 1 % longer although the product alone takes the same 49 us.)
+// 256 x 256 tiles with a k-contiguous dense operand are never cut: where their tiles leave compute units idle, 256 x 128
+// tiles reach twice as many (and are taken, see dispatch_out).
+template <typename C> struct SplitCost;
+template <> struct SplitCost<SlimCfg> { static constexpr double STAGE_US = 0.33, SPLIT_US = 1.1, PARTIAL_US = 0.35; static constexpr int BLOCKS = 512; };
+template <> struct SplitCost<MidCfg> { static constexpr double STAGE_US = 0.31, SPLIT_US = 2.3, PARTIAL_US = 0.45; static constexpr int BLOCKS = 256; };
+template <> struct SplitCost<TiledCfg> { static constexpr double STAGE_US = 0.46, SPLIT_US = 1.2, PARTIAL_US = 0.35; static constexpr int BLOCKS = 256; };   // k-strided
 template <typename T, typename C>
-int choose_splits(int64_t n_sparse, int64_t k, int64_t n_dense, int64_t workspace_bytes) {
+int choose_splits(int64_t n_sparse, int64_t k, int64_t n_dense, int64_t workspace_bytes, bool k_strided) {
+  using S = SplitCost<C>;
+  if (std::is_same<C, TiledCfg>::value && !k_strided) return 1;
   const int64_t tiles = ((n_sparse + C::BI - 1) / C::BI) * ((n_dense + C::BJ - 1) / C::BJ);
   const int64_t nstages = k * (int64_t)sizeof(T) / C::KB;
-  if (tiles >= 160) return 1;
-  int64_t splits = 192 / tiles;              // measured: filling all 256 CUs costs more in partial tiles than it gains
-  if (splits > nstages / 4) splits = nstages / 4;
-  if (splits > 16) splits = 16;
-  while (splits > 1 && splits * tiles * C::BI * C::BJ * 4 > workspace_bytes) splits--;
-  return splits < 2 ? 1 : (int)splits;
-}
-
-// Time estimate of the tiled kernel on one tile configuration, to choose between 256 x 256 and
-// 256 x 128 tiles for operands of a few hundred dense columns: rounds of at most 256 blocks (one per
-// CU) x stages per block x the stage time measured for that configuration (0.95 us for 256 x 256
-// tiles, 0.55 us for 256 x 128), plus, with k pieces, the partial tiles written and read at
-// 4.5 TB/s and the second launch.  On W[11008, 4096], W[4096, 11008] and W[8192, 8192] with 256 to
-// 1536 dense columns it picks the faster configuration in every case measured (up to 30 % apart).
-struct TileCost { int64_t blocks; double us; };
-template <typename T, typename C>
-TileCost tile_cost(int64_t n_sparse, int64_t k, int64_t n_dense, int64_t workspace_bytes, double stage_us) {
-  const int64_t tiles = ((n_sparse + C::BI - 1) / C::BI) * ((n_dense + C::BJ - 1) / C::BJ);
-  const int64_t nstages = k * (int64_t)sizeof(T) / C::KB;
-  const int64_t splits = workspace_bytes > 0 ? choose_splits<T, C>(n_sparse, k, n_dense, workspace_bytes) : 1;
-  const int64_t blocks = tiles * splits, rounds = (blocks + 255) / 256;
-  double us = (double)rounds * (double)((nstages + splits - 1) / splits) * stage_us;
-  if (splits > 1) us += 2.0 * (double)(splits * tiles * C::BI * C::BJ * 4) / 4.5e6 + 3.0;
-  return {blocks, us};
+  const double tile_mb = C::BI * C::BJ * 4e-6;
+  int best = 1;
+  double least = (double)nstages * S::STAGE_US;
+  for (int64_t p = 2; p <= 16 && p <= nstages / 2 && p * tiles <= S::BLOCKS && p * tiles * C::BI * C::BJ * 4 <= workspace_bytes; p++) {
+    const double us = (double)((nstages + p - 1) / p) * S::STAGE_US + S::SPLIT_US + (double)(p * tiles) * tile_mb * S::PARTIAL_US;
+    if (us < least) { least = us; best = (int)p; }
+  }
+  return best;
 }
 
 // compute units of the current device (looked up once per device; the cache is a table of atomics: two threads
@@ -1083,7 +1084,7 @@ int launch_tiled(const void* av, const void* am, int64_t n_sparse, int64_t k, co
                  void* workspace, int64_t workspace_bytes, hipStream_t s) {
   int tiles_i = (int)((n_sparse + C::BI - 1) / C::BI);
   const int tiles_j = (int)((n_dense + C::BJ - 1) / C::BJ);
-  const int splits = workspace ? choose_splits<T, C>(n_sparse, k, n_dense, workspace_bytes) : 1;
+  const int splits = workspace ? choose_splits<T, C>(n_sparse, k, n_dense, workspace_bytes, b_layout == TF24_COL_MAJOR) : 1;
   const int cu_slots = compute_units() / 8;
   // A last round that fills less than half of the compute units: the tile rows that make up the full rounds stay
   // with the chained 256 x 256 tiles, the remaining rows go to a second launch on 256 x 128 tiles, which reach twice
@@ -1473,12 +1474,11 @@ int dispatch_out(int out_dtype, const void* av, const void* am, int a_layout, in
   const bool tiled = panel && (b_layout == TF24_ROW_MAJOR || sizeof(T) == 2) && n_sparse >= 64;
   // up to 64 dense columns: the tiled kernel on 256 x 64 tiles; up to 128: on 256 x 128 tiles
   const bool slim = tiled && b_layout == TF24_ROW_MAJOR && n_dense <= SlimCfg::BJ;
-  // wider operands that still fit one round of 256 x 128 tiles take those when the estimate below says so
-  const int64_t ws_bytes = workspace ? workspace_bytes : 0;
+  // wider operands whose 256 x 128 tiles fit one round of the 256 compute units take those: they reach twice as many
+  // compute units as 256 x 256 tiles (on the timings behind choose_splits they are the faster ones in every such case,
+  // 4096 x 4096 against 1000 columns 30.0 and 43.2 us, 1600 x 6400 against 3000 48.1 and 59.9)
   const bool mid = tiled && b_layout == TF24_ROW_MAJOR &&
-                   (n_dense <= MidCfg::BJ ||
-                    (tile_cost<T, MidCfg>(n_sparse, k, n_dense, ws_bytes, 0.55).blocks <= 256 &&
-                     tile_cost<T, MidCfg>(n_sparse, k, n_dense, ws_bytes, 0.55).us < tile_cost<T, TiledCfg>(n_sparse, k, n_dense, ws_bytes, 0.95).us));
+                   (n_dense <= MidCfg::BJ || ((n_sparse + MidCfg::BI - 1) / MidCfg::BI) * ((n_dense + MidCfg::BJ - 1) / MidCfg::BJ) <= 256);
   // at most 8 dense columns: one pass over the compressed operand; up to 16 when the sparse operand
   // has enough rows for the four-row-block form of that kernel (13.0 against 15.7 us on 11008 rows,
   // but 19.7 against 18.6 us on 8192), or when the tiled kernel cannot cut k into pieces (no
