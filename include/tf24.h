@@ -399,6 +399,20 @@ int tf24_gelu_glu_backward(const void* grad_out, int64_t ld_grad_out, const void
                            void* stream);
 
 /*
+ * Weight and bias gradient of a linear layer whose weight is dense:
+ *     dw[i, j] = sum_t g[t, i] * x[t, j],  db[i] = sum_t g[t, i]   (t < tokens, i < m, j < n)
+ * g [tokens, m] and x [tokens, n] row-major F16 or BF16 with leading dimensions ldg, ldx (multiples of 8, 16-byte aligned);
+ * dw [m, n] and db [m] (NULL: not wanted) contiguous, of the same type, each sum float32 rounded once.
+ * m and n multiples of 8, any number of tokens >= 1.  The reference leaves these products to torch
+ * (sparse/sparse_ops.py:36-43, README.md:245-266).
+ *   workspace  16-byte aligned scratch; with tf24_grad_weight_workspace_bytes(tokens, m, n) bytes the token axis is cut into
+ *              the number of pieces that suits the shape (0: one piece), with less or none into fewer.  Deterministic either way.
+ */
+int tf24_grad_weight(const void* g, int64_t ldg, const void* x, int64_t ldx, int dtype, int64_t tokens, int64_t m, int64_t n,
+                     void* dw, void* db, void* workspace, int64_t workspace_bytes, void* stream);
+int64_t tf24_grad_weight_workspace_bytes(int64_t tokens, int64_t m, int64_t n);
+
+/*
  * out[c, r] = in[r, c] for 2-byte (F16|BF16) and 1-byte (E4M3|E5M2|U8) elements; in [rows, cols] with
  * leading dimension ld_in, out [cols, rows] with ld_out.  No counterpart in the reference (CUTLASS
  * reads either operand layout): it feeds tf24_spmm's fast kernel, which wants an 8-bit dense operand

@@ -519,3 +519,69 @@ def test_entry_points_under_graph_capture(cuda):
         torch.cuda.synchronize()
         for name, a, b in zip(("x @ S.t", "S @ w.t", "masked decay"), captured, eager):
             assert torch.equal(a, b), (it, name)
+
+
+@pytest.mark.parametrize("tokens,m,n", [(1, 8, 8), (31, 264, 40), (32, 256, 256), (33, 512, 264), (65, 248, 1000), (96, 256, 8),
+                                        (128, 8, 256), (129, 768, 512), (161, 256, 256), (1000, 3072, 768), (4099, 768, 3072)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_grad_weight_kernel(cuda, tokens, m, n, dtype):
+    """dY^T x and sum(dY) of the dense layers' kernel, with as many pieces of the token axis as it likes, in one piece, with and
+    without the sums, and from rows with a pitch; columns and tokens that fill no tile or stage.
+    Bound: a float32 sum of `tokens` exact products in any order errs by at most tokens * 2^-23 times the sum of their
+    magnitudes, and is rounded once to 11 (8) bits."""
+    from sparse import _native as N
+    gen = torch.Generator(device=cuda).manual_seed(tokens * 7 + m + n)
+    g = torch.randn(tokens, m + 16, device=cuda, generator=gen).to(dtype)[:, 8:8 + m]
+    x = torch.randn(tokens, n, device=cuda, generator=gen).to(dtype)
+    lib = N.lib()
+    nbytes = lib.tf24_grad_weight_workspace_bytes(tokens, m, n)
+    gt, xd = g.double().t().contiguous(), x.double()
+    half_ulp = 2.0 ** (-11 if dtype == torch.float16 else -8)
+    for want, size, name in ((gt @ xd, gt.abs() @ xd.abs(), "dW"), (gt.sum(1), gt.abs().sum(1), "db")):
+        limit = want.abs() * half_ulp + size * tokens * 2.0 ** -23 + 1e-7
+        for bytes_given in {0, nbytes}:
+            for with_bias in (True, False):
+                ws = torch.empty(max(bytes_given, 16), dtype=torch.uint8, device=cuda)
+                dw = torch.full((m, n), float("nan"), dtype=dtype, device=cuda)
+                db = torch.full((m,), float("nan"), dtype=dtype, device=cuda)
+                N.check(lib.tf24_grad_weight(g.data_ptr(), g.stride(0), x.data_ptr(), x.stride(0), N.dtype_code(dtype), tokens, m, n, dw.data_ptr(),
+                                             db.data_ptr() if with_bias else None, ws.data_ptr(), bytes_given, N.stream_ptr()))
+                if name == "db" and not with_bias:
+                    assert db.isnan().all()
+                else:
+                    got = dw if name == "dW" else db
+                    assert ((got.double() - want).abs() <= limit).all(), (name, bytes_given, with_bias)
+
+
+@pytest.mark.parametrize("tokens,bias,dtype", [((300,), True, torch.bfloat16), ((5, 41), True, torch.float16), ((4100,), False, torch.bfloat16),
+                                               ((3, 200), False, torch.float16)])
+def test_soft_threshold_linear_under_autocast(cuda, tokens, bias, dtype):
+    """In mixed precision the module takes its own weight gradient (from a number of tokens on); the same as F.linear under
+    autocast, also where a graph of the gradients, a tangent of the input or a mode asks for torch's operators."""
+    import sparse
+    torch.manual_seed(8)
+    mod = sparse.SoftThresholdLinear(128, 264, bias=bias, device=cuda)
+    mod.init_scale()
+    params = list(mod.parameters())
+    x = torch.randn(*tokens, 128, device=cuda, requires_grad=True)
+    gy = torch.randn(*tokens, 264, device=cuda).to(dtype)
+
+    def grads(y, **kw):
+        return [y] + list(torch.autograd.grad(y, [x] + params, gy, **kw))
+
+    with torch.autocast("cuda", dtype=dtype):
+        y_ref = F.linear(x, mod.get_sparse_weights(), mod.bias)
+        y = mod(x)
+    assert "linear16" in type(y.grad_fn).__name__
+    want = grads(y_ref)
+    # one rounding to 16 bits each, of sums that differ in order: at most a unit in the last place where they straddle a boundary
+    tol = 2.0 ** (-10 if dtype == torch.float16 else -7)
+    for a, b in zip(grads(y, retain_graph=True), want):
+        assert a.dtype == b.dtype and torch.allclose(a.float(), b.float(), rtol=tol, atol=1e-4)
+    first = grads(y, create_graph=True)
+    assert first[1].grad_fn is not None
+    torch.autograd.grad(first[1].float().sum(), params[0])                          # reaches the weight through dX
+    with torch.autograd.forward_ad.dual_level(), torch.autocast("cuda", dtype=dtype):
+        dual = torch.autograd.forward_ad.make_dual(x.detach(), torch.ones_like(x))
+        tangent = torch.autograd.forward_ad.unpack_dual(mod(dual)).tangent
+    assert tangent is not None
