@@ -47,6 +47,7 @@ _SIGNATURES = {
     "tf24_transposable_mask": (_i, [_p, _i, _i, _i64, _i64, _i64, _i, _p, _p, _p]),
     "tf24_transposable_mask_validate": (_i, [_i, _i, _i64, _i64, _i64]),
     "tf24_soft_threshold24": (_i, [_p, _i, _i, _i64, _i64, _i64, _p, _p, _p]),
+    "tf24_soft_threshold24_scaled": (_i, [_p, _i64, _i64, _p, _f, _p, _i, _p]),
     "tf24_sparse24_dense": (_i, [_p, _i, _i, _i64, _i64, _i64, _p, _p, _p]),
     "tf24_mvue24_dense": (_i, [_p, _i, _i, _i64, _i64, _i64, _p, _i64, _p, _p]),
     "tf24_masked_add": (_i, [_p, _i, _p, _i, _p, _i, _i64, _f, _p]),

@@ -259,6 +259,13 @@ int tf24_transposable_mask_validate(int dtype, int layout, int64_t ld, int64_t m
  */
 int tf24_soft_threshold24(const void* dense, int dtype, int layout, int64_t ld, int64_t m, int64_t k,
                           void* sparse_out, void* mask_out, void* stream);
+/*
+ * out = scale * soft_threshold24(dense) rounded to out_dtype (F16|BF16): the weight that an S-STE layer in mixed precision
+ * multiplies by (README.md:233-266).  dense float32 and out contiguous [m, k], k % 4 == 0; scale is one float32 on
+ * the device, or NULL: scale_value.
+ */
+int tf24_soft_threshold24_scaled(const float* dense, int64_t m, int64_t k, const float* scale, float scale_value, void* out, int out_dtype,
+                                 void* stream);
 int tf24_sparse24_dense(const void* dense, int dtype, int layout, int64_t ld, int64_t m, int64_t k,
                         void* sparse_out, void* mask_out, void* stream);
 int tf24_mvue24_dense(const void* dense, int dtype, int layout, int64_t ld, int64_t m, int64_t k,

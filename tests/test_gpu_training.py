@@ -585,3 +585,20 @@ def test_soft_threshold_linear_under_autocast(cuda, tokens, bias, dtype):
         dual = torch.autograd.forward_ad.make_dual(x.detach(), torch.ones_like(x))
         tangent = torch.autograd.forward_ad.unpack_dual(mod(dual)).tangent
     assert tangent is not None
+
+
+@pytest.mark.parametrize("shape", [(1, 8), (64, 128), (37, 1000), (768, 3072)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_soft_threshold16_is_threshold_scale_and_cast(cuda, shape, dtype):
+    """Bit for bit, special values (and a negative scale, which makes dropped zeros negative) included."""
+    import sparse
+    from sparse.sparse_ops import _soft_threshold16
+    torch.manual_seed(1)
+    w = torch.randn(*shape, device=cuda) * torch.logspace(-9, 6, shape[1], device=cuda)
+    w.view(-1)[:8] = torch.tensor([0.0, -0.0, float("inf"), 1.0, 2.0, 2.0, -2.0, 1e-42], device=cuda)
+    for value, where in ((1.37, cuda), (-0.6, cuda), (-0.6, "cpu"), (1.37, "cpu")):      # (a layer made on the GPU keeps its scale on the host)
+        scale = torch.tensor(value, device=where)
+        want = (sparse.soft_threshold24(w)[0] * scale).to(dtype)
+        got = _soft_threshold16.apply(w, scale, dtype)
+        assert got.view(torch.int16).equal(want.view(torch.int16)) or (
+            got.isnan().equal(want.isnan()) and got[~got.isnan()].view(torch.int16).equal(want[~want.isnan()].view(torch.int16)))
