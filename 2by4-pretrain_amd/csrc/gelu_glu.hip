@@ -14,11 +14,16 @@ namespace {
 constexpr int kThreads = 256;
 constexpr float kBeta = 0.7978845608028654f;     // sqrt(2/pi)
 constexpr float kKappa = 0.044715f;
+constexpr float kExpLinear = (float)(-2.0 * 0.7978845608028654 * 1.4426950408889634);               // -2u as a power of two
+constexpr float kExpCubic = (float)(-2.0 * 0.7978845608028654 * 1.4426950408889634 * 0.044715);
 
 // 0.5 * (1 + tanh(u)) is the logistic function of 2u: one exponential and one reciprocal per
-// element (written with tanh, exp and a division, as the reference does, the forward kernel is
-// bound by the vector ALUs at 0.59 of the HBM peak instead of by memory).  exp of a large
-// argument gives +inf and the reciprocal 0, so no range split is needed.
+// element.  exp of a large argument gives +inf and the reciprocal 0, so no range split is needed.
+// The vector ALUs are busy for more than half of the memory time, so instructions count: with the
+// polynomials as multiply-adds (the factors of the exponent folded into their constants) an element
+// takes 8 and 14 of them instead of 11 and 22, and with loads that may stay in the caches 12288 x 8192
+// fp16 takes 45.5 + 77 instead of 48.4 + 81.7 us (forward + backward; streaming stores: 10 us less
+// than plain ones).  Error against float64 as before: that of the rounding to 16 bits.
 struct GluTerms {
   float gelu;      // gelu_tanh(gate) = gate * sig
   float dgelu;     // d gelu_tanh / d gate = sig + gate * sig * (1 - sig) * 2 * du/dgate
@@ -26,12 +31,11 @@ struct GluTerms {
 template <bool GRAD>
 __device__ __forceinline__ GluTerms glu_terms(float gate) {
   const float g2 = gate * gate;
-  const float u = kBeta * (gate + kKappa * g2 * gate);
-  const float sig = __builtin_amdgcn_rcpf(1.0f + __expf(-2.0f * u));
+  const float sig = __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(gate * __builtin_fmaf(g2, kExpCubic, kExpLinear)));
   GluTerms r;
   r.gelu = gate * sig;
   r.dgelu = 0.0f;
-  if constexpr (GRAD) r.dgelu = sig + gate * (sig * (1.0f - sig)) * ((2.0f * kBeta) * (1.0f + (3.0f * kKappa) * g2));
+  if constexpr (GRAD) r.dgelu = __builtin_fmaf(r.gelu * (1.0f - sig), __builtin_fmaf(g2, 6.0f * kBeta * kKappa, 2.0f * kBeta), sig);
   return r;
 }
 
@@ -45,8 +49,8 @@ gelu_glu_fwd(const T* __restrict__ in, int64_t ld_in, int64_t gate_off, int64_t 
   const int64_t j = ((int64_t)(blockIdx.x - (uint32_t)i * chunks) * kThreads + threadIdx.x) * V;
   if (j >= nj) return;
   Pack<T, V> x, g, o;
-  x.load_stream(in + i * ld_in + j);
-  g.load_stream(in + i * ld_in + j + gate_off);
+  x.load(in + i * ld_in + j);
+  g.load(in + i * ld_in + j + gate_off);
 #pragma unroll
   for (int e = 0; e < V; e++) o.v[e] = from_float<T>(glu_terms<false>(to_float(g.v[e])).gelu * to_float(x.v[e]));
   o.store_stream(out + i * ld_out + j);
@@ -61,9 +65,9 @@ gelu_glu_bwd(const T* __restrict__ grad_out, int64_t ld_go, const T* __restrict_
   const int64_t j = ((int64_t)(blockIdx.x - (uint32_t)i * chunks) * kThreads + threadIdx.x) * V;
   if (j >= nj) return;
   Pack<T, V> go, x, g, gx, gg;
-  go.load_stream(grad_out + i * ld_go + j);
-  x.load_stream(in + i * ld_in + j);
-  g.load_stream(in + i * ld_in + j + gate_off);
+  go.load(grad_out + i * ld_go + j);
+  x.load(in + i * ld_in + j);
+  g.load(in + i * ld_in + j + gate_off);
 #pragma unroll
   for (int e = 0; e < V; e++) {
     const GluTerms t = glu_terms<true>(to_float(g.v[e]));
