@@ -77,6 +77,8 @@ int launch(const void* values, const void* meta, int layout, int64_t m, int64_t 
 // 8 panels: a wave the values of 2 rows x 8 panels, 16 bytes per lane (canonical side: 512
 // contiguous bytes per row; panel side: the two rows' adjacent pieces, one cache line per panel);
 // the first wave also the 64 metadata pieces, lane = (row, panel) (64- or 128-byte runs on both sides).
+// Streaming accesses: 22 us for 8192 x 8192 either way, but conversion, export and decompression of a
+// weight in a row take 99.0 us with and 101.3 without (what they wrote is still draining into memory).
 template <int META_BYTES>
 __global__ void __launch_bounds__(kThreads)
 repack_kernel(const uint8_t* __restrict__ vin, const uint8_t* __restrict__ min_, int64_t m, int64_t panels, uint32_t chunks,
@@ -89,7 +91,9 @@ repack_kernel(const uint8_t* __restrict__ vin, const uint8_t* __restrict__ min_,
     if (p < panels && row < m) {
       const int64_t canon = row * panels + p, panel = p * m + row;
       const int64_t src = to_panel ? canon : panel, dst = to_panel ? panel : canon;
-      *reinterpret_cast<uint4*>(vout + dst * 64 + part * 16) = *reinterpret_cast<const uint4*>(vin + src * 64 + part * 16);
+      typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+      __builtin_nontemporal_store(__builtin_nontemporal_load(reinterpret_cast<const u32x4*>(vin + src * 64 + part * 16)),
+                                  reinterpret_cast<u32x4*>(vout + dst * 64 + part * 16));
     }
   }
   if (wave == 0 && mout) {
@@ -105,7 +109,31 @@ repack_kernel(const uint8_t* __restrict__ vin, const uint8_t* __restrict__ min_,
   }
 }
 
-// Metadata between any two storage forms, one lane per metadata word (WB bytes), lanes walking the
+// Metadata between the canonical and the panel form, as 4-byte words: [m][k/32] <-> [k/32][m], the transpose of a matrix
+// in[rows][cols].  A block moves 64 x 64 words through LDS, 256 contiguous bytes per wave and access on both sides (the
+// word-by-word kernel below scatters 2-byte words: 8192 x 8192 13.6 us, here 5.0).
+__global__ void __launch_bounds__(kThreads)
+transpose_words(const uint32_t* __restrict__ in, int64_t rows, int64_t cols, uint32_t tiles_c, uint32_t* __restrict__ out) {
+  __shared__ uint32_t s_tile[64][65];
+  const int64_t r0 = (int64_t)(blockIdx.x / tiles_c) * 64, c0 = (int64_t)(blockIdx.x % tiles_c) * 64;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  uint32_t w[16];
+#pragma unroll
+  for (int i = 0; i < 16; i++) {
+    const int64_t r = r0 + wave * 16 + i;
+    w[i] = r < rows && c0 + lane < cols ? __builtin_nontemporal_load(in + r * cols + c0 + lane) : 0u;
+  }
+#pragma unroll
+  for (int i = 0; i < 16; i++) s_tile[wave * 16 + i][lane] = w[i];
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < 16; i++) {
+    const int64_t c = c0 + wave * 16 + i;
+    if (c < cols && r0 + lane < rows) __builtin_nontemporal_store(s_tile[lane][wave * 16 + i], out + c * rows + r0 + lane);
+  }
+}
+
+// Metadata from or to the reordered form, one lane per metadata word (WB bytes), lanes walking the
 // words in the order of the reordered form ([word-column pair][row][2]: whole cache lines on that side,
 // and on the panel side up to a permutation of 32 adjacent rows).
 template <int WB>
@@ -168,6 +196,13 @@ extern "C" int tf24_repack_to(const void* values_in, const void* meta_in, int dt
   const int64_t panels = k / kp, chunks = (panels + 7) / 8, vblocks = chunks * ((m + 7) / 8);
   if (blocks > 0x7fffffffLL || vblocks > 0x7fffffffLL) return fail(TF24_ERR_SHAPE, "%s: matrix too large", fn);
   hipStream_t s = (hipStream_t)stream;
+  if (from_layout != TF24_COMPRESSED_CUTLASS && to_layout != TF24_COMPRESSED_CUTLASS) {        // (values_out is NULL here)
+    const int64_t rows = from_layout == TF24_COMPRESSED_PANEL ? k / 32 : m, cols = from_layout == TF24_COMPRESSED_PANEL ? m : k / 32;
+    const int64_t tiles_c = (cols + 63) / 64, tiles = tiles_c * ((rows + 63) / 64);
+    if (tiles > 0x7fffffffLL) return fail(TF24_ERR_SHAPE, "%s: matrix too large", fn);
+    hipLaunchKernelGGL(transpose_words, dim3((unsigned)tiles), dim3(kThreads), 0, s, (const uint32_t*)meta_in, rows, cols, (uint32_t)tiles_c, (uint32_t*)meta_out);
+    return check_launch(fn);
+  }
   if (is_8bit(dtype))
     hipLaunchKernelGGL(repack_meta_kernel<4>, dim3((unsigned)blocks), dim3(kThreads), 0, s, (const uint8_t*)meta_in, from_layout, to_layout, m, k, (uint8_t*)meta_out);
   else

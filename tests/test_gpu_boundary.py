@@ -318,3 +318,17 @@ def test_repack_to_one_part_only(cuda, dtype, m, k):
     N.check(N.lib().tf24_repack_to(None, got.data_ptr(), code, m, k, N.COMPRESSED_CUTLASS, N.COMPRESSED_PANEL, None, back.data_ptr(), N.stream_ptr()))
     assert bytes_of(back).equal(bytes_of(pm))
     assert N.lib().tf24_repack_to(None, None, code, m, k, N.COMPRESSED_PANEL, N.COMPRESSED_CANONICAL, None, None, N.stream_ptr()) != 0
+
+
+@pytest.mark.parametrize("m,k", [(32, 128), (96, 2176), (64, 2048), (1056, 192 * 32)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float8_e4m3fn])
+def test_metadata_words_move_alone(cuda, dtype, m, k):
+    """canonical <-> panel metadata without the values: the transpose of 4-byte words, at sizes that fill its 64 x 64 tiles and not."""
+    import sparse
+    N = sparse._native
+    words = torch.randint(-2 ** 31, 2 ** 31 - 1, (m, k // 32), device=cuda, dtype=torch.int32, generator=torch.Generator(device=cuda).manual_seed(m + k))
+    code, panel, back = N.operand_code(dtype), torch.zeros(k // 32, m, device=cuda, dtype=torch.int32), torch.zeros_like(words)
+    N.check(N.lib().tf24_repack_to(None, words.data_ptr(), code, m, k, N.COMPRESSED_CANONICAL, N.COMPRESSED_PANEL, None, panel.data_ptr(), N.stream_ptr()))
+    assert panel.equal(words.t())
+    N.check(N.lib().tf24_repack_to(None, panel.data_ptr(), code, m, k, N.COMPRESSED_PANEL, N.COMPRESSED_CANONICAL, None, back.data_ptr(), N.stream_ptr()))
+    assert back.equal(words)
