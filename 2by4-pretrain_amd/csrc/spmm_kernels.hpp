@@ -1042,8 +1042,12 @@ spmm_reduce_splits(const float* __restrict__ partial, int splits, int tiles_i, i
 // columns 19.0 -> 16.1 (12 -> 4); dW of 1024 tokens, 3072 x 768, 26.2 -> 16.4 (4 -> 1).  (The partial tiles of the
 // k-strided products count a fifth more than the fit says: inside a training step they leave the caches, and with dW of
 // 12288 tokens in six pieces instead of five the step took 1 % longer although the product alone takes the same 49 us.)
+// Narrow tiles whose one piece is short (ONE_PIECE_US: up to 27 stages) are not cut: the reduction takes 4 us of a call that
+// takes 8 to 13 without it, and its launch and workspace 4 us of host time, which bounds such calls one after the other
+// (linear of 37 tokens, 3072 x 768, 2304 x 768 and 1600 x 1600: 19.4 us in pieces, 15.4 in one; 768 x 3072 19.4 and 22).
 // 256 x 256 tiles with a k-contiguous dense operand are never cut: where their tiles leave compute units idle, 256 x 128
 // tiles reach twice as many (and are taken, see dispatch_out).
+constexpr double ONE_PIECE_US = 9.0;
 template <typename C> struct SplitCost;
 template <> struct SplitCost<SlimCfg> { static constexpr double STAGE_US = 0.33, SPLIT_US = 1.1, PARTIAL_US = 0.35; static constexpr int BLOCKS = 512; };
 template <> struct SplitCost<MidCfg> { static constexpr double STAGE_US = 0.31, SPLIT_US = 2.3, PARTIAL_US = 0.45; static constexpr int BLOCKS = 256; };
@@ -1057,6 +1061,7 @@ int choose_splits(int64_t n_sparse, int64_t k, int64_t n_dense, int64_t workspac
   const double tile_mb = C::BI * C::BJ * 4e-6;
   int best = 1;
   double least = (double)nstages * S::STAGE_US;
+  if (!std::is_same<C, TiledCfg>::value && least <= ONE_PIECE_US) return 1;
   for (int64_t p = 2; p <= 16 && p <= nstages / 2 && p * tiles <= S::BLOCKS && p * tiles * C::BI * C::BJ * 4 <= workspace_bytes; p++) {
     const double us = (double)((nstages + p - 1) / p) * S::STAGE_US + S::SPLIT_US + (double)(p * tiles) * tile_mb * S::PARTIAL_US;
     if (us < least) { least = us; best = (int)p; }
