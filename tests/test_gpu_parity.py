@@ -1120,3 +1120,35 @@ def test_linear_any_number_of_rows(cuda, dtype, n, k, rows):
         assert bool((y[rows:] == 77).all())
     got = torch.mm(xs, s.t())
     assert got.shape == (rows, n) and got.float().equal(want.to(got.dtype).float())
+
+
+@pytest.mark.parametrize("dtype,rows,k,view", [
+    (torch.float8_e4m3fn, 72, 128, "columns"), (torch.int8, 24, 256, "columns"), (torch.float16, 72, 128, "columns"), (torch.float16, 75, 128, "columns"),
+    (torch.float8_e4m3fn, 17, 128, "pitch"), (torch.int8, 88, 128, "pitch"), (torch.bfloat16, 17, 128, "pitch"),
+    (torch.float16, 3, 128, "far"), (torch.float8_e4m3fn, 3, 128, "far"), (torch.bfloat16, 1, 128, "far"),
+    (torch.bfloat16, 1, 128, "off"), (torch.float16, 17, 128, "off"), (torch.int8, 1, 128, "off"), (torch.float16, 1, 128, "odd"), (torch.float16, 9, 128, "odd")])
+@pytest.mark.parametrize("n", [32, 96])
+def test_linear_rows_in_views(cuda, dtype, rows, k, view, n):
+    """Row counts off the type's multiple in views that the kernels cannot address as they lie: k strided, a pitch of 8 one-byte
+    elements, rows more than 16 MiB apart, a start off a
+    16-byte boundary, an odd pitch.  Exact: small integers."""
+    import sparse
+    g = torch.Generator().manual_seed(rows + n)
+    w = torch.randint(-2, 3, (n, k), generator=g)
+    s = sparse.to_sparse_semi_structured((w if dtype == torch.int8 else w.float()).to(cuda).to(torch.int8 if dtype == torch.int8 else torch.float32), dtype=dtype)
+    x = torch.randint(-2, 3, (rows, k), generator=g).float().to(cuda).to(dtype)
+    if view == "columns":
+        base = torch.zeros(k, rows, dtype=dtype, device=cuda)
+        at = base.t()
+    elif view == "pitch":
+        at = torch.zeros(rows, k + 8, dtype=dtype, device=cuda)[:, :k]
+    elif view == "off":
+        at = torch.zeros(rows * k + 1, dtype=dtype, device=cuda)[1:].view(rows, k)
+    elif view == "odd":
+        at = torch.zeros(rows, k + 1, dtype=dtype, device=cuda)[:, :k]
+    else:
+        at = torch.zeros(rows, (1 << 24) // x.element_size() + 16, dtype=dtype, device=cuda)[:, :k]
+    at.copy_(x)
+    want = x.float() @ s.to_dense().float().t()
+    for got in (torch.mm(at, s.t()), sparse.sparse_semi_structured_linear(at, s)):
+        assert got.shape == (rows, n) and got.float().equal(want.to(got.dtype).float())
