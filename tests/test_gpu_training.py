@@ -578,6 +578,10 @@ def test_soft_threshold_linear_under_autocast(cuda, tokens, bias, dtype):
     tol = 2.0 ** (-10 if dtype == torch.float16 else -7)
     for a, b in zip(grads(y, retain_graph=True), want):
         assert a.dtype == b.dtype and torch.allclose(a.float(), b.float(), rtol=tol, atol=1e-4)
+    if dtype == torch.float16:                                                      # gradients that autograd maps over
+        mapped = torch.autograd.grad(y, params, torch.stack([gy, -2 * gy]), is_grads_batched=True, retain_graph=True)
+        for got, b in zip(mapped, want[2:]):
+            assert torch.allclose(got[0].float(), b.float(), rtol=tol, atol=1e-4) and torch.allclose(got[1].float(), -2 * b.float(), rtol=tol, atol=2e-4)
     first = grads(y, create_graph=True)
     assert first[1].grad_fn is not None
     torch.autograd.grad(first[1].float().sum(), params[0])                          # reaches the weight through dX
