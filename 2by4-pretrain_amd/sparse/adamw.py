@@ -46,11 +46,9 @@ class MaskedDecayAdamW(Optimizer):
             raise RuntimeError("MaskedDecayAdamW: parameters must be float32 GPU tensors")
         if not (p.is_contiguous() or (p.dim() == 2 and p.t().is_contiguous())):
             raise RuntimeError("MaskedDecayAdamW: parameters must be dense in memory")
-        state = self.state[p]
-        state["step"] = torch.zeros((), dtype=torch.int64, device=p.device) if capturable else 0
-        state["exp_avg"] = torch.empty_like(p, memory_format=torch.preserve_format)       # zeroed with the others of the
-        state["exp_avg_sq"] = torch.empty_like(p, memory_format=torch.preserve_format)    # group, in one launch (step)
-        return state
+        return {"step": torch.zeros((), dtype=torch.int64, device=p.device) if capturable else 0,
+                "exp_avg": torch.empty_like(p, memory_format=torch.preserve_format),       # zeroed with the others of the
+                "exp_avg_sq": torch.empty_like(p, memory_format=torch.preserve_format)}    # group, in one launch (step)
 
     @torch.no_grad()
     def step(self, closure=None):
@@ -71,7 +69,7 @@ class MaskedDecayAdamW(Optimizer):
                 state = self.state[p]
                 if not state:
                     state = self._check(p, group.get("capturable", False))
-                    fresh += [state["exp_avg"], state["exp_avg_sq"]]
+                    fresh.append((p, state))                       # the optimizer's own only once it holds zeros
                 stride = p.stride()
                 if grad.is_sparse or grad.stride() != stride:
                     raise RuntimeError("MaskedDecayAdamW: the gradient must be dense with the parameter's strides")
@@ -84,7 +82,9 @@ class MaskedDecayAdamW(Optimizer):
                 if torch.is_tensor(state["step"]):
                     counts.append(state["step"])
             if fresh:
-                torch._foreach_zero_(fresh)
+                torch._foreach_zero_([state[name] for _, state in fresh for name in ("exp_avg", "exp_avg_sq")])
+                for p, state in fresh:
+                    self.state[p] = state
             if counts:
                 torch._foreach_add_(counts, 1)
             for p, grad, state, mask, grad_code, mask_code in entries:

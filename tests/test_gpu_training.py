@@ -302,6 +302,26 @@ def test_masked_decay_adamw_list_of_tensors(cuda, gdt, mdt, device_step):
         assert int(opt.state[p]["step"]) == step
 
 
+def test_masked_decay_adamw_moments_after_a_refused_gradient(cuda):
+    """A first step that is refused because of a later tensor leaves nothing behind: the moments start from zero afterwards."""
+    import sparse
+    first = [torch.nn.Parameter(torch.ones(64, 32, device=cuda)) for _ in range(2)]
+    opt = sparse.MaskedDecayAdamW(first, lr=1e-2)
+    first[0].grad = torch.full_like(first[0], 0.5)
+    first[1].grad = torch.full((32, 64), 0.5, device=cuda).t()
+    junk = [torch.full((64, 32), float("nan"), device=cuda) for _ in range(8)]       # what fresh memory may hold
+    del junk
+    with pytest.raises(RuntimeError, match="strides"):
+        opt.step()
+    first[1].grad = first[0].grad.clone()
+    opt.step()
+    want, m, v = oracle.adamw_masked_decay(torch.ones(64, 32), torch.full((64, 32), 0.5), torch.zeros(64, 32), torch.zeros(64, 32), None, 1, alpha=0.0,
+                                           lr=1e-2, betas=opt.defaults["betas"], eps=opt.defaults["eps"], weight_decay=opt.defaults["weight_decay"])
+    for p in first:                                                                  # float32 arithmetic of a few operations
+        assert torch.allclose(p.detach().cpu(), want, rtol=2e-6, atol=1e-8)
+        assert torch.allclose(opt.state[p]["exp_avg"].cpu(), m, rtol=2e-6, atol=1e-10)
+
+
 @pytest.mark.parametrize("gdt", [torch.float32, torch.bfloat16])
 def test_masked_decay_adamw_step_count_on_the_device(cuda, gdt):
     """capturable=True: the step count is an int64 in device memory and the bias corrections 1 - beta^step are
