@@ -27,6 +27,19 @@ from . import _native as N
 __all__ = ["MaskedDecayAdamW"]
 
 
+def _rounds(params):
+    """`params` as lists in which no storage stands twice: the tensors of one launch are updated side by side, and a
+    parameter listed twice (torch warns of it), or two that share their memory, one after the other."""
+    rounds, times = [], {}
+    for p in params:
+        key = p.data_ptr() or id(p)                                # (tensors without elements all have the null pointer)
+        turn = times[key] = times.get(key, -1) + 1
+        if turn == len(rounds):
+            rounds.append([])
+        rounds[turn].append(p)
+    return rounds
+
+
 class MaskedDecayAdamW(Optimizer):
     def __init__(self, params, lr=1e-3, betas=(0.9, 0.999), eps=1e-8, weight_decay=1e-2, alpha=0.0, capturable=False):
         if not 0.0 <= lr:
@@ -56,13 +69,13 @@ class MaskedDecayAdamW(Optimizer):
         if closure is not None:
             with torch.enable_grad():
                 loss = closure()
-        for group in self.param_groups:
+        for group, params in ((group, params) for group in self.param_groups for params in _rounds(group["params"])):
             beta1, beta2 = group["betas"]
             lr, eps, wd, alpha = float(group["lr"]), float(group["eps"]), float(group["weight_decay"]), float(group["alpha"])
             # Everything is looked at before anything is launched; the tensors of one launch share the types of
             # gradient and mask and a host-side step count (device-side counts travel with their tensor)
             entries, counts, launches, fresh = [], [], {}, []
-            for p in group["params"]:
+            for p in params:
                 grad = p.grad
                 if grad is None:
                     continue

@@ -322,6 +322,28 @@ def test_masked_decay_adamw_moments_after_a_refused_gradient(cuda):
         assert torch.allclose(opt.state[p]["exp_avg"].cpu(), m, rtol=2e-6, atol=1e-10)
 
 
+@pytest.mark.parametrize("capturable", [False, True])
+def test_masked_decay_adamw_shared_storage(cuda, capturable):
+    """Two parameters on the same memory are updated one after the other, as by one launch each."""
+    import sparse
+    torch.manual_seed(3)
+    base = torch.randn(300, 512, device=cuda)
+    results = []
+    for grouped in (True, False):
+        data = base.clone()
+        params = [torch.nn.Parameter(data), torch.nn.Parameter(torch.ones(7, device=cuda)), torch.nn.Parameter(data)]
+        for i, p in enumerate(params):
+            p.grad = torch.full_like(p, 0.25 * (i + 1))
+        groups = [params] if grouped else [[p] for p in params]
+        opts = [sparse.MaskedDecayAdamW(g, lr=1e-2, weight_decay=0.1, capturable=capturable) for g in groups]
+        for _ in range(2):
+            for opt in opts:
+                opt.step()
+        results.append([p.detach().clone() for p in params])
+    for a, b in zip(*results):
+        assert a.equal(b)
+
+
 @pytest.mark.parametrize("gdt", [torch.float32, torch.bfloat16])
 def test_masked_decay_adamw_step_count_on_the_device(cuda, gdt):
     """capturable=True: the step count is an int64 in device memory and the bias corrections 1 - beta^step are
