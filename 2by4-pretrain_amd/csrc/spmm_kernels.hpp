@@ -1211,47 +1211,58 @@ int launch_tiled(const void* av, const void* am, int64_t n_sparse, int64_t k, co
 }
 
 // ------------------------------------------------------------------------------------------
-// Narrow kernels: at most 16 dense columns (decoding a few tokens against a large sparse weight).
+// Narrow kernels: at most 64 dense columns (decoding a few tokens against a large sparse weight, a batch of
+// sequences against a small one).
 // The product is bound by one pass over the compressed operand, so the sparse operand is not
 // staged: a wave streams the A fragments of 16 sparse rows straight into registers (in the panel
 // layout 1 KB of contiguous memory per panel, 16 bytes per lane, and their index words 128 (256)
 // contiguous bytes) and runs one V_SMFMAC_*_16X16 per panel.  Loads are issued a batch of panels at
 // a time into one of two register sets, the next batch while the current one is multiplied: left
 // to itself the compiler waits for each panel's loads before it issues the next.
-// Fewer than 512 row blocks (spmm_narrow): a block owns 16 rows, its up to four waves each take a
-// share of the k range, read their dense fragments from global memory (64 contiguous bytes from
-// each of the 16 dense rows, twice) and meet in LDS at the end (added in wave order).
+// Fewer than 512 row blocks, or more than 16 columns (spmm_narrow): a block owns 16 rows, its up to four waves each take a
+// share of the k range, read their dense fragments, NB of 16 columns, from global memory (64 contiguous bytes from
+// each of the 16 dense rows, twice) and meet in LDS at the end (added in wave order).  Bound by latency, a few loads deep, at
+// short k and by the requests of the dense fragments at long k: 3072 x 768 bf16 against 37 columns 8.9 us on 256 x 64 tiles,
+// of which there are 12, and 5.4 us here.  Eight waves a block were no faster (4096 x 11008, 1 column: 13.2 -> 16.9 us).
 // From 512 row blocks on (spmm_narrow_shared): see there.
 // ------------------------------------------------------------------------------------------
-constexpr int kNarrowMaxDense = 16;
 constexpr int kNarrowWaves = 4;
 constexpr int kNarrowSharedMin = 160;      // workgroups of four 16-row blocks below which two blocks per workgroup are faster
 
-template <typename T, typename OutT, bool C_JMAJOR>
+template <typename T, typename OutT, bool C_JMAJOR, int NB>
 __global__ void __launch_bounds__(64 * kNarrowWaves)
 spmm_narrow(const uint8_t* __restrict__ a_values, const uint8_t* __restrict__ a_meta, int64_t n_sparse, int64_t k,
             const uint8_t* __restrict__ b, int64_t ldb_bytes, int64_t n_dense,
             OutT* __restrict__ c, int64_t ldc, const OutT* __restrict__ bias, float scale, int act) {
   constexpr int KSTEP = mma16<T>::KSTEP;     // dense k per panel = per instruction
   constexpr int M_ROW = KSTEP / 8;           // metadata bytes per row per panel
-  constexpr int BATCH = 8;                   // panels per load batch; two batches are in flight
+  constexpr int BATCH = NB == 1 ? 8 : NB == 2 ? 4 : 2;          // panels per load batch; two batches are in flight
+  constexpr int CHAINS = NB == 1 ? 2 : 1;    // consecutive instructions do not wait on each other: two chains, or the fragments
   using acc_t = typename mma16<T>::acc_t;
-  __shared__ acc_t s_acc[kNarrowWaves - 1][64];
+  __shared__ acc_t s_acc[NB == 1 ? kNarrowWaves - 1 : kNarrowWaves][NB][64];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, li = lane & 15, lk = lane >> 4;
   const int64_t i0 = (int64_t)blockIdx.x * 16;
   const int64_t npanels = k / KSTEP;
   const int nwaves = blockDim.x >> 6;
   const int64_t p_begin = wave * npanels / nwaves, p_end = (wave + 1) * npanels / nwaves;
-  const int64_t col = li < n_dense ? li : n_dense - 1;          // clamp: the column is never stored
-  const uint8_t* bp = b + col * ldb_bytes + lk * 16;
+  const uint8_t* bp[NB];
+#pragma unroll
+  for (int f = 0; f < NB; f++) {
+    const int64_t col = f * 16 + li < n_dense ? f * 16 + li : n_dense - 1;      // clamp: the column is never stored
+    bp[f] = b + col * ldb_bytes + lk * 16;
+  }
   const uint8_t* av = a_values + (i0 + li) * 64 + lk * 16;
   const uint8_t* am = a_meta + panel_meta_offset(lk * (M_ROW / 4), i0 + li, n_sparse);   // (a panel's further words: n_sparse * 4 bytes apart)
   const int64_t a_step = n_sparse * 64, m_step = n_sparse * M_ROW;
-  acc_t acc[2];                              // two chains, so that consecutive instructions do not wait on each other
+  acc_t acc[NB][CHAINS];
 #pragma unroll
-  for (int r = 0; r < 4; r++) { acc[0][r] = 0; acc[1][r] = 0; }
+  for (int f = 0; f < NB; f++)
+#pragma unroll
+    for (int h = 0; h < CHAINS; h++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) acc[f][h][r] = 0;
   // two register sets: the loads of the next batch are in flight while the current one is multiplied
-  int4v af[2][BATCH], lo[2][BATCH], hi[2][BATCH];
+  int4v af[2][BATCH], lo[2][BATCH][NB], hi[2][BATCH][NB];
   int idx[2][BATCH];
   auto load_batch = [&](int set, int64_t p) {
 #pragma unroll
@@ -1260,16 +1271,23 @@ spmm_narrow(const uint8_t* __restrict__ a_values, const uint8_t* __restrict__ a_
       af[set][u] = __builtin_nontemporal_load(reinterpret_cast<const int4v*>(av + pp * a_step));
       if constexpr (sizeof(T) == 2) idx[set][u] = *reinterpret_cast<const uint16_t*>(am + pp * m_step);
       else idx[set][u] = *reinterpret_cast<const int*>(am + pp * m_step);
-      lo[set][u] = *reinterpret_cast<const int4v*>(bp + pp * 128);
-      hi[set][u] = *reinterpret_cast<const int4v*>(bp + pp * 128 + 64);
+#pragma unroll
+      for (int f = 0; f < NB; f++) {
+        lo[set][u][f] = *reinterpret_cast<const int4v*>(bp[f] + pp * 128);
+        hi[set][u][f] = *reinterpret_cast<const int4v*>(bp[f] + pp * 128 + 64);
+      }
     }
   };
   auto multiply_batch = [&](int set, int64_t p) {
 #pragma unroll
     for (int u = 0; u < BATCH; u++) {
       const int4v a = p + u < p_end ? af[set][u] : int4v{0, 0, 0, 0};
-      const int8v bfrag = {lo[set][u][0], lo[set][u][1], lo[set][u][2], lo[set][u][3], hi[set][u][0], hi[set][u][1], hi[set][u][2], hi[set][u][3]};
-      acc[u & 1] = mma16<T>::template run<0>(a, bfrag, acc[u & 1], idx[set][u]);
+#pragma unroll
+      for (int f = 0; f < NB; f++) {
+        const int4v l = lo[set][u][f], h = hi[set][u][f];
+        const int8v bfrag = {l[0], l[1], l[2], l[3], h[0], h[1], h[2], h[3]};
+        acc[f][u % CHAINS] = mma16<T>::template run<0>(a, bfrag, acc[f][u % CHAINS], idx[set][u]);
+      }
     }
   };
   if (p_begin < p_end) load_batch(0, p_begin);
@@ -1285,21 +1303,27 @@ spmm_narrow(const uint8_t* __restrict__ a_values, const uint8_t* __restrict__ a_
       __builtin_amdgcn_sched_barrier(0);
     }
   }
-  acc_t sum = acc[0] + acc[1];
-  if (wave > 0) s_acc[wave - 1][lane] = sum;
+  const acc_t own = CHAINS == 2 ? acc[0][0] + acc[0][CHAINS - 1] : acc[0][0];
+  if (wave > 0) s_acc[wave - 1][0][lane] = own;
+#pragma unroll
+  for (int f = 1; f < NB; f++) s_acc[wave][f][lane] = acc[f][0];
   __syncthreads();
-  if (wave > 0 || li >= n_dense) return;
+  for (int f = wave; f < NB; f += nwaves) {  // a wave finishes every nwaves-th fragment, its pieces added in wave order
+    const int64_t col = f * 16 + li;
+    if (col >= n_dense) continue;
+    acc_t sum = f == 0 ? own : s_acc[0][f][lane];
 #pragma unroll
-  for (int w = 0; w < nwaves - 1; w++) sum += s_acc[w][lane];
-  const int64_t row = i0 + lk * 4;           // D layout: column l%16, rows 4*(l/16) + r
-  OutT o[4];
+    for (int w = 1; w < nwaves; w++) sum += s_acc[f == 0 ? w - 1 : w][f][lane];
+    const int64_t row = i0 + lk * 4;         // D layout: column l%16, rows 4*(l/16) + r
+    OutT o[4];
 #pragma unroll
-  for (int r = 0; r < 4; r++) o[r] = to_out<OutT>(finish_value(sum[r], scale, bias, row + r, act));
-  if constexpr (C_JMAJOR) {
-    *reinterpret_cast<Pack<OutT, 4>*>(c + (int64_t)li * ldc + row) = *reinterpret_cast<Pack<OutT, 4>*>(o);
-  } else {
+    for (int r = 0; r < 4; r++) o[r] = to_out<OutT>(finish_value(sum[r], scale, bias, row + r, act));
+    if constexpr (C_JMAJOR) {
+      *reinterpret_cast<Pack<OutT, 4>*>(c + col * ldc + row) = *reinterpret_cast<Pack<OutT, 4>*>(o);
+    } else {
 #pragma unroll
-    for (int r = 0; r < 4; r++) c[(row + r) * ldc + li] = o[r];
+      for (int r = 0; r < 4; r++) c[(row + r) * ldc + col] = o[r];
+    }
   }
 }
 
@@ -1420,12 +1444,25 @@ spmm_narrow_shared(const uint8_t* __restrict__ a_values, const uint8_t* __restri
   }
 }
 
+// Up to how many dense columns the narrow kernels are the faster ones; us on float16 operands, tiled -> narrow:
+// from 512 row blocks on (spmm_narrow_shared) 16: 8192 x 8192 22.0 -> 20.2, 8192 x 1024 10.2 -> 4.8; below that the fragments of
+// more columns cost requests with every panel of every block, so it depends on the panels: 16 columns of 4096 x 4096 12.8 -> 8.7,
+// of 768 x 3072 8.8 -> 7.9, but of 1600 x 6400 12.4 -> 14.8; 32 of 4096 x 2048 10.3 -> 7.7; 64 of 4096 x 1536 13.5 -> 9.4, of
+// 2304 x 768 9.0 -> 6.5, but of 2304 x 2048 10.7 -> 11.2.  With two blocks to a compute unit (6144 rows): 48 of k = 768
+// 9.0 -> 8.0 and of 1536 13.7 -> 12.5, 64 of k = 768 9.1 -> 9.6.
+inline int64_t narrow_columns(int64_t n_sparse, int64_t npanels) {
+  const int64_t blocks = n_sparse / 16;
+  if (blocks <= 256) return npanels <= 24 ? 64 : npanels <= 32 ? 32 : npanels <= 64 ? 16 : 8;
+  if (blocks <= 512 && npanels <= 32) return npanels <= 24 ? 48 : 32;
+  return blocks >= 512 ? 16 : 8;
+}
+
 template <typename T, typename OutT>
 int launch_narrow(const void* av, const void* am, int64_t n_sparse, int64_t k, const void* b, int64_t ldb, int64_t n_dense,
                   void* c, int c_layout, int64_t ldc, const void* bias, float scale, int act, hipStream_t s) {
   dim3 grid((unsigned)(n_sparse / 16));
   const int64_t blocks = n_sparse / 16, npanels = k * (int64_t)sizeof(T) / 128;
-  if (blocks >= 512) {          // enough row blocks: several per workgroup, dense operand through LDS
+  if (blocks >= 512 && n_dense <= 16) {          // enough row blocks: several per workgroup, dense operand through LDS
     const bool jm = c_layout == TF24_COL_MAJOR;
     const int nw = blocks / 4 >= kNarrowSharedMin ? 4 : 2;      // four row blocks per workgroup only if that leaves enough workgroups
     dim3 sgrid((unsigned)((blocks + nw - 1) / nw));
@@ -1442,14 +1479,19 @@ int launch_narrow(const void* av, const void* am, int64_t n_sparse, int64_t k, c
     else { if (jm) go_nw(std::true_type{}, std::integral_constant<int, 16>{}); else go_nw(std::false_type{}, std::integral_constant<int, 16>{}); }
     return check_launch("tf24_spmm");
   }
-  int nwaves = kNarrowWaves;                 // few row blocks: the waves of a block split k
+  int nwaves = kNarrowWaves;                                    // few row blocks: the waves of a block split k
   while (nwaves > 1 && npanels / nwaves < 4) nwaves /= 2;
-  if (c_layout == TF24_COL_MAJOR)
-    hipLaunchKernelGGL((spmm_narrow<T, OutT, true>), grid, dim3(64 * nwaves), 0, s, (const uint8_t*)av, (const uint8_t*)am, n_sparse, k,
-                       (const uint8_t*)b, ldb * (int64_t)sizeof(T), n_dense, (OutT*)c, ldc, (const OutT*)bias, scale, act);
-  else
-    hipLaunchKernelGGL((spmm_narrow<T, OutT, false>), grid, dim3(64 * nwaves), 0, s, (const uint8_t*)av, (const uint8_t*)am, n_sparse, k,
-                       (const uint8_t*)b, ldb * (int64_t)sizeof(T), n_dense, (OutT*)c, ldc, (const OutT*)bias, scale, act);
+  auto go = [&](auto jmajor, auto nb) {
+    hipLaunchKernelGGL((spmm_narrow<T, OutT, decltype(jmajor)::value, decltype(nb)::value>), grid, dim3(64 * nwaves), 0, s, (const uint8_t*)av,
+                       (const uint8_t*)am, n_sparse, k, (const uint8_t*)b, ldb * (int64_t)sizeof(T), n_dense, (OutT*)c, ldc, (const OutT*)bias, scale, act);
+  };
+  auto go_nb = [&](auto jmajor) {
+    if (n_dense <= 16) go(jmajor, std::integral_constant<int, 1>{});
+    else if (n_dense <= 32) go(jmajor, std::integral_constant<int, 2>{});
+    else if (n_dense <= 48) go(jmajor, std::integral_constant<int, 3>{});
+    else go(jmajor, std::integral_constant<int, 4>{});
+  };
+  if (c_layout == TF24_COL_MAJOR) go_nb(std::true_type{}); else go_nb(std::false_type{});
   return check_launch("tf24_spmm");
 }
 
@@ -1484,12 +1526,10 @@ int dispatch_out(int out_dtype, const void* av, const void* am, int a_layout, in
   // 4096 x 4096 against 1000 columns 30.0 and 43.2 us, 1600 x 6400 against 3000 48.1 and 59.9)
   const bool mid = tiled && b_layout == TF24_ROW_MAJOR &&
                    (n_dense <= MidCfg::BJ || ((n_sparse + MidCfg::BI - 1) / MidCfg::BI) * ((n_dense + MidCfg::BJ - 1) / MidCfg::BJ) <= 256);
-  // at most 8 dense columns: one pass over the compressed operand; up to 16 when the sparse operand
-  // has enough rows for the four-row-block form of that kernel (13.0 against 15.7 us on 11008 rows,
-  // but 19.7 against 18.6 us on 8192), or when the tiled kernel cannot cut k into pieces (no
-  // workspace), which it needs to fill the chip
+  // few dense columns: one pass over the compressed operand (narrow_columns), also up to 16 when the tiled kernel cannot cut k
+  // into pieces (no workspace), which it needs to fill the chip
   const bool narrow = panel && b_layout == TF24_ROW_MAJOR &&
-                      (n_dense <= 8 || (n_dense <= kNarrowMaxDense && (n_sparse / 64 >= kNarrowSharedMin || !(slim && workspace))));
+                      (n_dense <= narrow_columns(n_sparse, k * (int64_t)sizeof(T) / 128) || (n_dense <= 16 && !(slim && workspace)));
   if constexpr (std::is_same<T, i8_t>::value) {        // integer product: int32 accumulators, results and bias
     if (narrow) return launch_narrow<T, int32_t>(av, am, n_sparse, k, b, ldb, n_dense, c, c_layout, ldc, bias, scale, act, s);
     if (slim) return launch_tiled<T, int32_t, SlimCfg>(av, am, n_sparse, k, b, b_layout, ldb, n_dense, c, c_layout, ldc, bias, scale, act, workspace, workspace_bytes, s);

@@ -1152,3 +1152,34 @@ def test_linear_rows_in_views(cuda, dtype, rows, k, view, n):
     want = x.float() @ s.to_dense().float().t()
     for got in (torch.mm(at, s.t()), sparse.sparse_semi_structured_linear(at, s)):
         assert got.shape == (rows, n) and got.float().equal(want.to(got.dtype).float())
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float8_e4m3fn, torch.int8])
+@pytest.mark.parametrize("n,panels", [(32, 1), (256, 5), (4096, 24), (4128, 24), (4096, 25), (768, 32), (4096, 33), (96, 64), (6144, 9), (8192, 17), (8224, 3)])
+def test_few_dense_columns(cuda, dtype, n, panels):
+    """Dense extents up to and past those that the narrow kernels take, both output orders; exact on small integers."""
+    import sparse
+    from sparse import _native as N
+    k = panels * 128 // torch.empty(0, dtype=dtype).element_size()
+    g = torch.Generator(device=cuda).manual_seed(n + panels)
+    w = torch.randint(-2, 3, (n, k), device=cuda, generator=g)
+    s = sparse.to_sparse_semi_structured(w.to(torch.int8) if dtype == torch.int8 else w.float(), dtype=dtype)
+    dense = s.to_dense().float()
+    out_dtype = torch.int32 if dtype == torch.int8 else torch.float32
+    code = N.operand_code(dtype)
+    bias = torch.randint(-5, 6, (n,), device=cuda, generator=g).to(out_dtype)
+    for rows in (8, 9, 16, 17, 31, 32, 33, 47, 48, 49, 63, 64, 65):
+        x = torch.randint(-2, 3, (rows, k), device=cuda, generator=g).to(dtype)
+        want = (x.float() @ dense.t() + bias.float()).to(out_dtype)
+        nbytes = N.lib().tf24_spmm_workspace_bytes(code, n, k, rows)
+        ws = torch.empty(max(nbytes, 16), dtype=torch.uint8, device=cuda)
+        y = torch.full((rows + 1, n), 77, dtype=out_dtype, device=cuda)
+        N.check(N.lib().tf24_linear(s._store_values.data_ptr(), s._store_meta.data_ptr(), N.COMPRESSED_PANEL, code, n, k, x.data_ptr(), k, rows, y.data_ptr(),
+                                    N.operand_code(out_dtype), n, bias.data_ptr(), 1.0, N.ACT_NONE, ws.data_ptr(), nbytes, N.stream_ptr()))
+        assert y[:rows].equal(want) and bool((y[rows:] == 77).all()), rows
+        if rows % 16 == 0:
+            yt = torch.full((n, rows), 77, dtype=out_dtype, device=cuda)
+            N.check(N.lib().tf24_spmm(s._store_values.data_ptr(), s._store_meta.data_ptr(), N.COMPRESSED_PANEL, code, n, k, x.data_ptr(), N.ROW_MAJOR, k, rows,
+                                      yt.data_ptr(), N.operand_code(out_dtype), N.ROW_MAJOR, rows, bias.data_ptr(), 1.0, N.ACT_NONE, ws.data_ptr(), nbytes,
+                                      N.stream_ptr()))
+            assert yt.equal(want.t()), rows
