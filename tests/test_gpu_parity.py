@@ -1183,3 +1183,28 @@ def test_few_dense_columns(cuda, dtype, n, panels):
                                       yt.data_ptr(), N.operand_code(out_dtype), N.ROW_MAJOR, rows, bias.data_ptr(), 1.0, N.ACT_NONE, ws.data_ptr(), nbytes,
                                       N.stream_ptr()))
             assert yt.equal(want.t()), rows
+
+
+@pytest.mark.parametrize("dtype,special", [(F16, float("inf")), (BF16, float("-inf")), (E5M2, float("inf")), (E4M3, float("nan"))])
+@pytest.mark.parametrize("n,panels", [(768, 12), (512, 11), (256, 5), (4096, 22), (1024, 37), (8192, 17), (8224, 3), (10240, 43)])
+def test_few_dense_columns_special_values(cuda, dtype, special, n, panels):
+    """An infinity or NaN among the activations reaches only the outputs whose weight keeps its position, as itself, also in
+    the last panel, where a batch of panels may end early.  All kept weights are non-zero integers: exact."""
+    import sparse
+    width = 128 // torch.empty(0, dtype=dtype).element_size()
+    k = panels * width
+    g = torch.Generator(device=cuda).manual_seed(n + panels)
+    w = torch.randint(1, 3, (n, k), device=cuda, generator=g).float() * (torch.randint(0, 2, (n, k), device=cuda, generator=g) * 2 - 1).float()
+    s = sparse.to_sparse_semi_structured(w, dtype=dtype)
+    dense = s.to_dense().float()
+    for rows in (1, 8, 13, 16, 29, 45, 64):
+        x = torch.randint(-2, 3, (rows, k), device=cuda, generator=g).float()
+        at = torch.tensor([(k - 3, k - width, 0, k - 9)[r % 4] for r in range(rows)], device=cuda)      # row r is special in column at[r]
+        line = torch.arange(rows, device=cuda)
+        x[line, at] = 0
+        want = x @ dense.t()
+        hit = dense.t()[at]                                                                           # [rows, n]: the weights it meets
+        want = torch.where(hit != 0, special * hit, want)
+        x[line, at] = special
+        got = torch.mm(x.to(dtype), s.t())
+        assert torch.allclose(got.float(), want.to(got.dtype).float(), rtol=0, atol=0, equal_nan=True), rows
