@@ -28,15 +28,19 @@ __all__ = ["MaskedDecayAdamW"]
 
 
 def _rounds(params):
-    """`params` as lists in which no storage stands twice: the tensors of one launch are updated side by side, and a
-    parameter listed twice (torch warns of it), or two that share their memory, one after the other."""
-    rounds, times = [], {}
-    for p in params:
-        key = p.data_ptr() or id(p)                                # (tensors without elements all have the null pointer)
-        turn = times[key] = times.get(key, -1) + 1
-        if turn == len(rounds):
+    """`params` as lists in which no memory stands twice: the tensors of one launch are updated side by side, and those
+    that overlap (a parameter listed twice, of which torch warns, or views of one buffer) one after the other, in the
+    order of the list."""
+    spans = [(p.data_ptr(), p.numel() * p.element_size()) for p in params]
+    in_memory = sorted(span for span in spans if span[1])
+    if all(start + size <= after for (start, size), (after, _) in zip(in_memory, in_memory[1:])):
+        return [params]
+    rounds, turns = [], []
+    for p, (start, size) in zip(params, spans):
+        turns.append(1 + max((turn for turn, (other, extent) in zip(turns, spans) if other < start + size and start < other + extent), default=-1))
+        if turns[-1] == len(rounds):
             rounds.append([])
-        rounds[turn].append(p)
+        rounds[turns[-1]].append(p)
     return rounds
 
 

@@ -344,6 +344,28 @@ def test_masked_decay_adamw_shared_storage(cuda, capturable):
         assert a.equal(b)
 
 
+@pytest.mark.parametrize("capturable", [False, True])
+@pytest.mark.parametrize("starts", [(0, 4), (513, 0), (0, 1024)])
+def test_masked_decay_adamw_overlapping_parameters(cuda, capturable, starts):
+    """Parameters that are overlapping parts of one buffer are updated one after the other, as by one optimizer each."""
+    import sparse
+    torch.manual_seed(4)
+    base = torch.randn(150000, device=cuda)
+    results = []
+    for grouped in (True, False):
+        data = base.clone()
+        params = [torch.nn.Parameter(data[start:]) for start in starts + starts[:1]]
+        for i, p in enumerate(params):
+            p.grad = torch.full_like(p, 0.25 * (i + 1))
+        groups = [params] if grouped else [[p] for p in params]
+        opts = [sparse.MaskedDecayAdamW(g, lr=1e-2, weight_decay=0.1, capturable=capturable) for g in groups]
+        for _ in range(2):
+            for opt in opts:
+                opt.step()
+        results.append(data)
+    assert results[0].equal(results[1])
+
+
 @pytest.mark.parametrize("gdt", [torch.float32, torch.bfloat16])
 def test_masked_decay_adamw_step_count_on_the_device(cuda, gdt):
     """capturable=True: the step count is an int64 in device memory and the bias corrections 1 - beta^step are

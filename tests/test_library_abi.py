@@ -196,3 +196,23 @@ def test_reference_api_names_present():
     assert sig.parameters["dtype"].default is torch.float16
     cls = sparse.SparseSemiStructuredTensor
     assert cls._FORCE_CUTLASS is True and cls._FUSE_TRANSPOSE is False
+
+
+def test_parameters_that_overlap_take_turns():
+    """The optimizer updates the tensors of a round side by side: none of them may share memory, wherever they start, and of
+    two that overlap the earlier one of the list goes first."""
+    from sparse.adamw import _rounds
+    base, other, empty = torch.zeros(100), torch.zeros(40), torch.zeros(0)
+
+    def check(params, expected):
+        rounds = _rounds(params)
+        assert [[next(i for i, q in enumerate(params) if q is p) for p in r] for r in rounds] == expected
+
+    check([base[:50], other, base[50:]], [[0, 1, 2]])
+    check([base, base[4:], other], [[0, 2], [1]])
+    check([base[4:], other, base], [[0, 1], [2]])
+    check([base[:60], base[40:], base[:40]], [[0], [1, 2]])
+    check([base, base[4:], base.view(10, 10), empty, torch.zeros(0)], [[0, 3, 4], [1], [2]])
+    check([base[:1], base, base[99:]], [[0], [1], [2]])
+    check([base.view(10, 10).t(), other.view(8, 5)], [[0, 1]])
+    assert not any(_rounds([]))
