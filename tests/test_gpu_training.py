@@ -655,6 +655,22 @@ def test_soft_threshold_linear_under_autocast(cuda, tokens, bias, dtype):
     assert tangent is not None
 
 
+@pytest.mark.parametrize("n,m", [(8, (1 << 20) + 8), ((1 << 20) + 8, 8), (8, 1 << 20)])
+def test_soft_threshold_linear_very_wide(cuda, n, m):
+    """More features on either side than the weight-gradient kernel takes, and as many: the gradients of F.linear.  Exact:
+    small integers, sums below 2^8 in magnitude."""
+    import sparse
+    mod = sparse.SoftThresholdLinear(n, m, device=cuda)
+    mod.init_scale()
+    g = torch.Generator(device=cuda).manual_seed(m)
+    x = torch.randint(-1, 2, (256, n), device=cuda, generator=g).float()
+    gy = (torch.randint(-1, 2, (256, m), device=cuda, generator=g) * (torch.rand(256, m, device=cuda, generator=g) < 0.3)).bfloat16()
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        y = mod(x)
+    grads = torch.autograd.grad(y, [mod.weight, mod.bias], gy)
+    assert grads[0].equal(gy.float().t() @ x) and grads[1].equal(gy.float().sum(0))
+
+
 @pytest.mark.parametrize("shape", [(1, 8), (64, 128), (37, 1000), (768, 3072)])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_soft_threshold16_is_threshold_scale_and_cast(cuda, shape, dtype):
