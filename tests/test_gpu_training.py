@@ -655,6 +655,41 @@ def test_soft_threshold_linear_under_autocast(cuda, tokens, bias, dtype):
     assert tangent is not None
 
 
+@pytest.mark.parametrize("tokens,bias", [(300, True), (4100, False)])
+def test_soft_threshold_linear_backward_under_tangents_and_modes(cuda, tokens, bias):
+    """A tangent of the output's gradient reaches the weight's and the bias's, and a dispatch mode around the backward pass sees
+    the products, also where the forward pass ran without either."""
+    import sparse
+    from torch.autograd import forward_ad
+    from torch.utils._python_dispatch import TorchDispatchMode
+    torch.manual_seed(9)
+    mod = sparse.SoftThresholdLinear(128, 264, bias=bias, device=cuda)
+    mod.init_scale()
+    params = list(mod.parameters())
+    x = torch.randn(tokens, 128, device=cuda)
+    gy, tangent = (torch.randn(tokens, 264, device=cuda).bfloat16() for _ in range(2))
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        y = mod(x)
+    assert "linear16" in type(y.grad_fn).__name__
+    want, want_tangent = ([gy_.float().t() @ x.bfloat16().float()] + ([gy_.float().sum(0)] if bias else []) for gy_ in (gy, tangent))
+    with forward_ad.dual_level():
+        got = [forward_ad.unpack_dual(t) for t in torch.autograd.grad(y, params, forward_ad.make_dual(gy, tangent), retain_graph=True)]
+        for t, a, b in zip(got, want, want_tangent):                      # one rounding to bfloat16 each, of sums in another order
+            assert torch.allclose(t.primal, a, rtol=2 ** -7, atol=1e-2)
+            assert t.tangent is not None and torch.allclose(t.tangent, b, rtol=2 ** -7, atol=1e-2)
+
+    class Seen(TorchDispatchMode):
+        names = []
+
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            self.names.append(func.__name__)
+            return func(*args, **(kwargs or {}))
+
+    with Seen() as seen:
+        torch.autograd.grad(y, params, gy)
+    assert seen.names.count("mm.default") == 1                            # dW (x needs no gradient)
+
+
 @pytest.mark.parametrize("n,m", [(8, (1 << 20) + 8), ((1 << 20) + 8, 8), (8, 1 << 20)])
 def test_soft_threshold_linear_very_wide(cuda, n, m):
     """More features on either side than the weight-gradient kernel takes, and as many: the gradients of F.linear.  Exact:
