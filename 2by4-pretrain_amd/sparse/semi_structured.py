@@ -218,27 +218,25 @@ def _spmm(sparse, dense, sparse_first, bias=None, out_dtype=None, scale=1.0, act
     vdtype = values.dtype
     if dense.dtype != vdtype:
         raise RuntimeError(f"dense operand dtype {dense.dtype} does not match the sparse operand's {vdtype}")
-    # (layout, leading dimension) of the dense operand as it lies, or of a contiguous copy when the kernels cannot
-    # address it (N.as_matrix + N.layout_of, written out: this function is on the training step's host path)
+    # (layout, leading dimension) of the dense operand as it lies (written out: this function is on the training step's host
+    # path), or of a contiguous copy where the kernels cannot address it: a start or a pitch off the 16-byte boundaries, a
+    # pitch of more than 16 MiB (the last token of long sequences: hidden[:, -1]), both strides above 1 -- and, since
+    # only rows with k contiguous go in any number, a count off the type's multiple with k strided.  clone: a tensor that
+    # starts off such a boundary counts as contiguous.
+    multiple = _DTYPE_TO_SEMI_STRUCTURED_SPARSE_CONFIG[vdtype].dense_min_rows        # elements of 16 bytes
     d0, d1 = dense.shape
     s0, s1 = dense.stride()
     if d0 == 1 and s1 == 1:
         s0 = d1                                  # (the pitch of a single row means nothing)
-    if s1 == 1 and s0 >= d1 and s0 % 8 == 0 and dense.data_ptr() % 16 == 0:
+    if s1 == 1 and s0 >= d1:
         lay, ld = N.ROW_MAJOR, s0
-    elif s0 == 1 and s1 >= d0 and s1 % 8 == 0 and dense.data_ptr() % 16 == 0:
+    elif s0 == 1 and s1 >= d0 and (sparse_first or d0 % multiple == 0):
         lay, ld = N.COL_MAJOR, s1
     else:
-        dense = dense.contiguous()
-        lay, ld = N.ROW_MAJOR, dense.stride(0)
-    if not sparse_first:
-        # any number of rows goes, but off the type's multiple only as rows that the kernels can address: k contiguous, 16-byte
-        # alignment and pitch, at most 16 MiB of it (the last token of long sequences: hidden[:, -1]).  clone, since a
-        # tensor that starts off such a boundary, or a single row of any pitch, counts as contiguous.
-        multiple = _DTYPE_TO_SEMI_STRUCTURED_SPARSE_CONFIG[vdtype].dense_min_rows
-        if d0 % multiple and (lay == N.COL_MAJOR or ld % multiple or ld * dense.element_size() > 1 << 24 or dense.data_ptr() % 16):
-            dense = dense.clone(memory_format=torch.contiguous_format)
-            lay, ld = N.ROW_MAJOR, d1
+        lay, ld = None, 0
+    if lay is None or ld % multiple or ld * vdtype.itemsize > 1 << 24 or dense.data_ptr() % 16:
+        dense = dense.clone(memory_format=torch.contiguous_format)
+        lay, ld = N.ROW_MAJOR, d1
     # When k is the strided dimension of the dense operand (`S @ dense` with a row-major dense, e.g.
     # dW = MVUE(dY^T) @ x) the tiled kernel reads 16-bit operands as they are, transposing while it
     # loads fragments.  For 8-bit operands it wants k contiguous: one transposing copy of the dense

@@ -1208,3 +1208,28 @@ def test_few_dense_columns_special_values(cuda, dtype, special, n, panels):
         x[line, at] = special
         got = torch.mm(x.to(dtype), s.t())
         assert torch.allclose(got.float(), want.to(got.dtype).float(), rtol=0, atol=0, equal_nan=True), rows
+
+
+@pytest.mark.parametrize("dtype,pitch", [(F16, 0), (BF16, 0), (E4M3, 0), (E4M3, 8), (torch.int8, 8)])
+@pytest.mark.parametrize("rows", [8, 16, 48])
+@pytest.mark.parametrize("view", ["far", "off"])
+def test_products_of_views_at_full_multiples(cuda, dtype, pitch, rows, view):
+    """Row counts that are multiples of everything, in views that start off a 16-byte boundary, whose rows are more than 16 MiB
+    apart or have a pitch of 8 one-byte elements: the rows of x @ S.t() and of S @ x.t(), where an odd count works too.
+    Exact: small integers."""
+    import sparse
+    k = 128
+    g = torch.Generator().manual_seed(rows)
+    w = torch.randint(-2, 3, (64, k), generator=g)
+    s = sparse.to_sparse_semi_structured((w.to(torch.int8) if dtype == torch.int8 else w.float()).to(cuda), dtype=dtype)
+    x = torch.randint(-2, 3, (rows, k), generator=g).float().to(cuda).to(dtype)
+    if view == "off":
+        at = torch.zeros(rows * (k + pitch) + 1, dtype=dtype, device=cuda)[1:].view(rows, k + pitch)[:, :k]
+    elif pitch:
+        at = torch.zeros(rows, k + pitch, dtype=dtype, device=cuda)[:, :k]
+    else:
+        at = torch.zeros(rows, (1 << 24) // x.element_size() + 16, dtype=dtype, device=cuda)[:, :k]
+    at.copy_(x)
+    want = x.float() @ s.to_dense().float().t()
+    for got in (torch.mm(at, s.t()), sparse.sparse_semi_structured_linear(at, s), torch.mm(s, at.t()).t()):
+        assert got.shape == (rows, 64) and got.float().equal(want.to(got.dtype).float())
