@@ -57,6 +57,12 @@ class MaskedDecayAdamW(Optimizer):
         super().__init__(params, dict(lr=lr, betas=betas, eps=eps, weight_decay=weight_decay, alpha=alpha,
                                       capturable=bool(capturable)))
 
+    def __setstate__(self, state):
+        super().__setstate__(state)
+        for of_p in self.state.values():         # (load_state_dict makes float32 of a capturable optimizer's step counts)
+            if torch.is_tensor(of_p.get("step")):
+                of_p["step"] = of_p["step"].to(torch.int64)
+
     def _check(self, p, capturable=False):
         """Once per parameter: what the kernel assumes about it (flat float32 storage shared by the moments)."""
         if p.dtype != torch.float32 or not p.is_cuda:

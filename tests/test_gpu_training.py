@@ -417,6 +417,37 @@ def test_masked_decay_adamw_step_count_on_the_device(cuda, gdt):
         same(step)
 
 
+@pytest.mark.parametrize("capturable", [False, True])
+def test_masked_decay_adamw_resumes_from_a_state_dict(cuda, capturable):
+    """Three updates, the state through a checkpoint on the host, two more: the bits of five updates in a row."""
+    import io
+    import sparse
+    grads = torch.randn(5, 1003, generator=torch.Generator().manual_seed(5)).to(cuda)
+
+    def updates(p, opt, which):
+        for i in which:
+            p.grad = grads[i].clone()
+            opt.step()
+
+    def fresh(data):
+        p = torch.nn.Parameter(data.clone())
+        return p, sparse.MaskedDecayAdamW([p], lr=1e-2, weight_decay=0.1, capturable=capturable)
+
+    start = torch.ones(1003, device=cuda)
+    whole, opt = fresh(start)
+    updates(whole, opt, range(5))
+    first, opt_first = fresh(start)
+    updates(first, opt_first, range(3))
+    blob = io.BytesIO()
+    torch.save(opt_first.state_dict(), blob)
+    blob.seek(0)
+    second, opt_second = fresh(first.detach())
+    opt_second.load_state_dict(torch.load(blob, map_location="cpu", weights_only=True))
+    updates(second, opt_second, range(3, 5))
+    assert second.equal(whole)
+    assert int(opt_second.state[second]["step"]) == 5 and opt_second.state[second]["exp_avg_sq"].equal(opt.state[whole]["exp_avg_sq"])
+
+
 @pytest.mark.parametrize("dtype,tol", [(torch.float32, 2e-6), (torch.float16, 1e-3), (torch.bfloat16, 8e-3)])
 @pytest.mark.parametrize("shape", [(4, 32, 256), (3, 5, 24), (2, 7, 10), (1, 1, 2)])
 @pytest.mark.parametrize("transposed", [False, True])
