@@ -44,24 +44,28 @@ extern "C" int tf24_spmm_validate(int dtype, int64_t n_sparse, int64_t k, int b_
 
 namespace tf24 {
 namespace {
-template <typename C>
-int64_t split_bytes(int dtype, int64_t n_sparse, int64_t k, int64_t n_dense) {
-  const int64_t big = (int64_t)1 << 40;
-  const int splits = is_8bit(dtype) ? choose_splits<e4m3_t, C>(n_sparse, k, n_dense, big, true) : choose_splits<f16_t, C>(n_sparse, k, n_dense, big, true);
-  if (splits < 2) return 0;
-  const int64_t tiles = ((n_sparse + C::BI - 1) / C::BI) * ((n_dense + C::BJ - 1) / C::BJ);
-  return splits * tiles * C::BI * C::BJ * 4;
+// the float32 partial tiles of the pieces chosen with any workspace
+template <typename T, typename C>
+int64_t piece_bytes(int64_t n_sparse, int64_t k, int64_t n_dense, bool k_strided) {
+  const int pieces = choose_pieces<T, C>(n_sparse, k, n_dense, (int64_t)1 << 40, k_strided).count;
+  if (pieces < 2) return 0;
+  return pieces * ((n_sparse + C::BI - 1) / C::BI) * ((n_dense + C::BJ - 1) / C::BJ) * C::BI * C::BJ * 4;
+}
+// for either orientation of the dense operand that the kernels of this operand size take (dispatch_out)
+template <typename T>
+int64_t workspace_bytes(int64_t n_sparse, int64_t k, int64_t n_dense) {
+  const int64_t strided = sizeof(T) == 2 && n_dense % 8 == 0 ? piece_bytes<T, TiledCfg>(n_sparse, k, n_dense, true) : 0;
+  if (n_dense <= narrow_columns(n_sparse, k * (int64_t)sizeof(T) / 128)) return strided;
+  return std::max(strided, n_dense <= SlimCfg::BJ ? piece_bytes<T, SlimCfg>(n_sparse, k, n_dense, false)
+                           : takes_mid<T>(n_sparse, k, n_dense, (int64_t)1 << 40) ? piece_bytes<T, MidCfg>(n_sparse, k, n_dense, false)
+                                                                                  : piece_bytes<T, TiledCfg>(n_sparse, k, n_dense, false));
 }
 }  // namespace
 }  // namespace tf24
 
-// the float32 partial tiles of the k pieces, for whichever tile configuration the shape selects
 extern "C" int64_t tf24_spmm_workspace_bytes(int dtype, int64_t n_sparse, int64_t k, int64_t n_dense) {
   using namespace tf24;
-  int64_t bytes = split_bytes<TiledCfg>(dtype, n_sparse, k, n_dense);
-  bytes = std::max(bytes, split_bytes<MidCfg>(dtype, n_sparse, k, n_dense));
-  if (n_dense <= SlimCfg::BJ) bytes = std::max(bytes, split_bytes<SlimCfg>(dtype, n_sparse, k, n_dense));
-  return bytes;
+  return is_8bit(dtype) ? workspace_bytes<e4m3_t>(n_sparse, k, n_dense) : workspace_bytes<f16_t>(n_sparse, k, n_dense);
 }
 
 namespace tf24 {

@@ -1032,41 +1032,60 @@ spmm_reduce_splits(const float* __restrict__ partial, int splits, int tiles_i, i
 }
 
 // How many k pieces a product is cut into, for shapes whose tiles cannot fill the 256 compute units: the number for which
-//     stages of one piece x STAGE_US + (pieces > 1: SPLIT_US + MB of partial tiles, all pieces, x PARTIAL_US)
-// is least, among those whose blocks fit one round (two blocks of the narrowest tiles share a compute unit) and whose
-// float32 partial tiles fit the caller's workspace.  The constants are the least-squares fit, per tile configuration, to
-// 560 timings of 1 to 16 pieces over weights from 768 x 768 to 8192 x 8192 (12 to 192 stages) and 20 to 3000 dense
-// columns; the pieces chosen this way are within 1 % of the best ones on average (6 % at worst), where 192 / tiles pieces
-// were 14 % off: a piece of few stages saves less than its partial tiles cost.  us, before and after:
-// 3072 x 768 against 1024 columns 22.2 -> 9.0 (2 pieces -> 1), 768 x 3072 20.6 -> 16.5 (8 -> 3), 4096 x 4096 against 128
-// columns 19.0 -> 16.1 (12 -> 4); dW of 1024 tokens, 3072 x 768, 26.2 -> 16.4 (4 -> 1).  (The partial tiles of the
-// k-strided products count a fifth more than the fit says: inside a training step they leave the caches, and with dW of
-// 12288 tokens in six pieces instead of five the step took 1 % longer although the product alone takes the same 49 us.)
-// Narrow tiles whose one piece is short (ONE_PIECE_US: up to 27 stages) are not cut: the reduction takes 4 us of a call that
-// takes 8 to 13 without it, and its launch and workspace 4 us of host time, which bounds such calls one after the other
-// (linear of 37 tokens, 3072 x 768, 2304 x 768 and 1600 x 1600: 19.4 us in pieces, 15.4 in one; 768 x 3072 19.4 and 22).
-// 256 x 256 tiles with a k-contiguous dense operand are never cut: where their tiles leave compute units idle, 256 x 128
-// tiles reach twice as many (and are taken, see dispatch_out).
-constexpr double ONE_PIECE_US = 9.0;
-template <typename C> struct SplitCost;
-template <> struct SplitCost<SlimCfg> { static constexpr double STAGE_US = 0.33, SPLIT_US = 1.1, PARTIAL_US = 0.35; static constexpr int BLOCKS = 512; };
-template <> struct SplitCost<MidCfg> { static constexpr double STAGE_US = 0.31, SPLIT_US = 2.3, PARTIAL_US = 0.45; static constexpr int BLOCKS = 256; };
-template <> struct SplitCost<TiledCfg> { static constexpr double STAGE_US = 0.46, SPLIT_US = 1.2, PARTIAL_US = 0.35; static constexpr int BLOCKS = 256; };   // k-strided
+//     CALL_US + max(stages of one piece x STAGE_US, MB of the compressed operand x OPERAND_US)
+//             + (pieces > 1: SPLIT_US + MB of partial sums, all pieces, x PARTIAL_US)
+// is least, among those whose blocks fit one round of the compute units and whose float32 partial tiles fit the caller's
+// workspace.  (Two of the narrowest tiles fit on one compute unit, but a few blocks more than there are units make the
+// whole product wait for the shared ones: fp8 11008 x 11008 against 48 columns 19.3 us in 5 pieces = 215 blocks, 26.4 in 6 = 258.)
+// Only the 32-column slabs that the dense operand reaches are written and read back, so only they count: k-strided
+// 6144 x 1536 against 16 columns 20.5 us in one piece, 12.4 in five.  Below some pieces the narrowest tiles are bound by the
+// one pass over the compressed operand (OPERAND_US: 8.8 TB/s, it stays in the last cache over repeated products).
+// The constants are least-squares fits, per tile configuration, to 25 000 timings of 1 to 16 pieces over fp16 and fp8 weights from
+// 256 x 768 to 20480 x 11008 (6 to 512 stages) and 16 to 3072 dense columns.  The pieces chosen this way are within 1 % of
+// the best ones on average and within 5 % for 19 in 20 (a fixed 192 / tiles of them: 5, 18 and 9 % off for the three
+// configurations below, and twice the time at worst; a fit to the range of 768 x 768 to 8192 x 8192 alone that counted whole tiles
+// 7, 2 and 5 %, half again the time at worst).  us, with 192 / tiles pieces and now: 3072 x 768 against 1024 columns
+// 22.2 -> 9.0 (2 pieces -> 1), 4096 x 4096 against 128 19.0 -> 16.1 (12 -> 5); dW of 1024 tokens, 3072 x 768, 26.2 -> 16.4 (4 -> 1).
+// A k-contiguous product of at most kShortStages stages is not cut: the reduction's launch and workspace are 4 us of host time,
+// which bounds such calls one after the other (linear of 96 rows with 256 x 1536: 14.6 us a call in one piece, 18.5 in
+// eight; alone 33.0 and 30.3 us, on the GPU 12.9 and 8.6).
+struct PieceCost { double call_us, stage_us, split_us, partial_us, operand_us; };
+template <typename C>
+constexpr PieceCost piece_cost(bool k_strided) {
+  return std::is_same<C, SlimCfg>::value ? PieceCost{5.1, 0.37, 1.8, 0.48, 0.113}
+         : std::is_same<C, MidCfg>::value ? PieceCost{5.6, 0.33, 2.1, 0.45, 0.0}
+         : k_strided ? PieceCost{7.1, 0.55, 1.15, 0.42, 0.0} : PieceCost{6.9, 0.50, 3.3, 0.385, 0.0};
+}
+constexpr int64_t kShortStages = 28;
+struct Pieces { int count; double us; };
 template <typename T, typename C>
-int choose_splits(int64_t n_sparse, int64_t k, int64_t n_dense, int64_t workspace_bytes, bool k_strided) {
-  using S = SplitCost<C>;
-  if (std::is_same<C, TiledCfg>::value && !k_strided) return 1;
-  const int64_t tiles = ((n_sparse + C::BI - 1) / C::BI) * ((n_dense + C::BJ - 1) / C::BJ);
-  const int64_t nstages = k * (int64_t)sizeof(T) / C::KB;
-  const double tile_mb = C::BI * C::BJ * 4e-6;
-  int best = 1;
-  double least = (double)nstages * S::STAGE_US;
-  if (!std::is_same<C, TiledCfg>::value && least <= ONE_PIECE_US) return 1;
-  for (int64_t p = 2; p <= 16 && p <= nstages / 2 && p * tiles <= S::BLOCKS && p * tiles * C::BI * C::BJ * 4 <= workspace_bytes; p++) {
-    const double us = (double)((nstages + p - 1) / p) * S::STAGE_US + S::SPLIT_US + (double)(p * tiles) * tile_mb * S::PARTIAL_US;
-    if (us < least) { least = us; best = (int)p; }
-  }
+Pieces choose_pieces(int64_t n_sparse, int64_t k, int64_t n_dense, int64_t workspace_bytes, bool k_strided) {
+  const PieceCost cost = piece_cost<C>(k_strided);
+  const int64_t tiles_i = (n_sparse + C::BI - 1) / C::BI, tiles = tiles_i * ((n_dense + C::BJ - 1) / C::BJ);
+  const int64_t stages = k * (int64_t)sizeof(T) / C::KB;
+  const double operand_us = (double)(n_sparse * k * (int64_t)sizeof(T)) * (9.0 / 16.0) * 1e-6 * cost.operand_us;
+  const double partial_us = (double)(tiles_i * C::BI * ((n_dense + 31) / 32 * 32)) * 4e-6 * cost.partial_us;     // of one piece
+  auto us = [&](int64_t p) {
+    return cost.call_us + std::max((double)((stages + p - 1) / p) * cost.stage_us, operand_us) + (p > 1 ? cost.split_us + (double)p * partial_us : 0.0);
+  };
+  Pieces best{1, us(1)};
+  if (!k_strided && stages <= kShortStages) return best;
+  for (int64_t p = 2; p <= 16 && p <= stages / 2 && p * tiles <= 256 && p * tiles * C::BI * C::BJ * 4 <= workspace_bytes; p++)
+    if (us(p) < best.us) best = {(int)p, us(p)};
   return best;
+}
+
+// A k-contiguous dense operand of more than 64 columns takes 256 x 128 tiles up to 128 columns, and beyond that where they fit one
+// round of the 256 compute units: they reach twice as many of them as 256 x 256 tiles, which are then the faster ones only with
+// k pieces under a long k (of 671 products timed with the pieces chosen above: 4096 x 4096 against 1000 columns
+// 30.0 and 43.2 us, 1600 x 6400 against 3000 48.1 and 59.9, but 6144 x 32768 against 512 159 and 118; with this
+// comparison of the estimates no product is more than 2 % off the better of the two, without it 4 are, by up to 35 %).
+template <typename T>
+bool takes_mid(int64_t n_sparse, int64_t k, int64_t n_dense, int64_t workspace_bytes) {
+  if (n_dense <= MidCfg::BJ) return true;
+  if (((n_sparse + MidCfg::BI - 1) / MidCfg::BI) * ((n_dense + MidCfg::BJ - 1) / MidCfg::BJ) > 256) return false;
+  return n_dense < TiledCfg::BJ || choose_pieces<T, TiledCfg>(n_sparse, k, n_dense, workspace_bytes, false).us >=
+                                       0.95 * choose_pieces<T, MidCfg>(n_sparse, k, n_dense, workspace_bytes, false).us;
 }
 
 // compute units of the current device (looked up once per device; the cache is a table of atomics: two threads
@@ -1089,7 +1108,7 @@ int launch_tiled(const void* av, const void* am, int64_t n_sparse, int64_t k, co
                  void* workspace, int64_t workspace_bytes, hipStream_t s) {
   int tiles_i = (int)((n_sparse + C::BI - 1) / C::BI);
   const int tiles_j = (int)((n_dense + C::BJ - 1) / C::BJ);
-  const int splits = workspace ? choose_splits<T, C>(n_sparse, k, n_dense, workspace_bytes, b_layout == TF24_COL_MAJOR) : 1;
+  const int splits = workspace ? choose_pieces<T, C>(n_sparse, k, n_dense, workspace_bytes, b_layout == TF24_COL_MAJOR).count : 1;
   const int cu_slots = compute_units() / 8;
   // A last round that fills less than half of the compute units: the tile rows that make up the full rounds stay
   // with the chained 256 x 256 tiles, the remaining rows go to a second launch on 256 x 128 tiles, which reach twice
@@ -1470,12 +1489,13 @@ spmm_narrow_shared(const uint8_t* __restrict__ a_values, const uint8_t* __restri
 // more columns cost requests with every panel of every block, so it depends on the panels: 16 columns of 4096 x 4096 12.8 -> 8.7,
 // of 768 x 3072 8.8 -> 7.9, but of 1600 x 6400 12.4 -> 14.8; 32 of 4096 x 2048 10.3 -> 7.7; 64 of 4096 x 1536 13.5 -> 9.4, of
 // 2304 x 768 9.0 -> 6.5, but of 2304 x 2048 10.7 -> 11.2.  With two blocks to a compute unit (6144 rows): 48 of k = 768
-// 9.0 -> 8.0 and of 1536 13.7 -> 12.5, 64 of k = 768 9.1 -> 9.6.
+// 9.0 -> 8.0 and of 1536 13.7 -> 12.5, 64 of k = 768 9.1 -> 9.6.  Past 128 panels the few workgroups of the shared form fall behind
+// k pieces (16 columns of 8192 x 8192 18.6 -> 19.5, of 8192 x 16384 28.3 -> 34.8, of 11008 x 16384 35.7 -> 49.5).
 inline int64_t narrow_columns(int64_t n_sparse, int64_t npanels) {
   const int64_t blocks = n_sparse / 16;
   if (blocks <= 256) return npanels <= 24 ? 64 : npanels <= 32 ? 32 : npanels <= 64 ? 16 : 8;
   if (blocks <= 512 && npanels <= 32) return npanels <= 24 ? 48 : 32;
-  return blocks >= 512 ? 16 : 8;
+  return blocks >= 512 && npanels <= 128 ? 16 : 8;
 }
 
 template <typename T, typename OutT>
@@ -1540,13 +1560,9 @@ int dispatch_out(int out_dtype, const void* av, const void* am, int a_layout, in
   // the tiled kernel reads a k-strided dense operand through transposing LDS reads (16-bit types only)
   // (also for a narrow dense operand: with its k pieces the tiled kernel beats the general one from 8 columns on)
   const bool tiled = panel && (b_layout == TF24_ROW_MAJOR || sizeof(T) == 2) && n_sparse >= 64;
-  // up to 64 dense columns: the tiled kernel on 256 x 64 tiles; up to 128: on 256 x 128 tiles
+  // up to 64 dense columns: the tiled kernel on 256 x 64 tiles; more: 256 x 128 or 256 x 256 tiles (takes_mid)
   const bool slim = tiled && b_layout == TF24_ROW_MAJOR && n_dense <= SlimCfg::BJ;
-  // wider operands whose 256 x 128 tiles fit one round of the 256 compute units take those: they reach twice as many
-  // compute units as 256 x 256 tiles (on the timings behind choose_splits they are the faster ones in every such case,
-  // 4096 x 4096 against 1000 columns 30.0 and 43.2 us, 1600 x 6400 against 3000 48.1 and 59.9)
-  const bool mid = tiled && b_layout == TF24_ROW_MAJOR &&
-                   (n_dense <= MidCfg::BJ || ((n_sparse + MidCfg::BI - 1) / MidCfg::BI) * ((n_dense + MidCfg::BJ - 1) / MidCfg::BJ) <= 256);
+  const bool mid = tiled && b_layout == TF24_ROW_MAJOR && takes_mid<T>(n_sparse, k, n_dense, workspace ? workspace_bytes : 0);
   // few dense columns: one pass over the compressed operand (narrow_columns), also up to 16 when the tiled kernel cannot cut k
   // into pieces (no workspace), which it needs to fill the chip
   const bool narrow = panel && b_layout == TF24_ROW_MAJOR &&

@@ -216,3 +216,19 @@ def test_parameters_that_overlap_take_turns():
     check([base[:1], base, base[99:]], [[0], [1], [2]])
     check([base.view(10, 10).t(), other.view(8, 5)], [[0, 1]])
     assert not any(_rounds([]))
+
+
+def test_pieces_of_products_with_few_columns():
+    """Pieces of k, read off the scratch that a product asks for (float32 partial tiles of 256 x 64, k-strided 256 x 256): their
+    blocks fit one round of 256 compute units, partial tiles count for the columns that the dense operand
+    reaches, and one pass over the weight asks for none."""
+    from sparse import _native as N
+    scratch = N.lib().tf24_spmm_workspace_bytes
+    for code, n, k, columns in ((N.E4M3, 11008, 11008, 48), (N.E4M3, 5120, 32768, 32), (N.E4M3, 20480, 8192, 64), (N.F16, 12288, 8192, 64)):
+        tile = 256 * (64 if code == N.E4M3 else 256) * 4                       # (16-bit types: k-strided, the larger tile)
+        blocks = scratch(code, n, k, columns) // tile
+        assert 0 < blocks <= 256 and blocks % ((n + 255) // 256) == 0, (n, k)
+    for n, k in ((6144, 1536), (5120, 1024), (11008, 2048)):
+        assert scratch(N.F16, n, k, 16) > 0
+    for n, k in ((11008, 4096), (3072, 768), (8192, 8192)):
+        assert scratch(N.F16, n, k, 1) == scratch(N.E4M3, n, k, 1) == scratch(N.E4M3, n, k, 8) == 0
