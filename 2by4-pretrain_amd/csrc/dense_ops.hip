@@ -60,6 +60,9 @@ dense_op_row(const T* __restrict__ dense, int64_t ld, int64_t m, int64_t k, cons
     ra.load_stream(rp);
     rb.load_stream(rp + 4);
     r[0] = ra.v[0]; r[1] = ra.v[1]; r[2] = rb.v[0]; r[3] = rb.v[1];
+    // the two loads share their lines: converting the first operand in between, the half-precision kernel fetched them
+    // twice (8192 x 8192 108 us, 85 side by side)
+    __builtin_amdgcn_sched_barrier(0);
   }
 #pragma unroll
   for (int g = 0; g < 2; g++) {
