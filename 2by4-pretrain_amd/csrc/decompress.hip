@@ -196,10 +196,14 @@ extern "C" int tf24_repack_to(const void* values_in, const void* meta_in, int dt
   const int64_t panels = k / kp, chunks = (panels + 7) / 8, vblocks = chunks * ((m + 7) / 8);
   if (blocks > 0x7fffffffLL || vblocks > 0x7fffffffLL) return fail(TF24_ERR_SHAPE, "%s: matrix too large", fn);
   hipStream_t s = (hipStream_t)stream;
-  if (from_layout != TF24_COMPRESSED_CUTLASS && to_layout != TF24_COMPRESSED_CUTLASS) {        // (values_out is NULL here)
-    const int64_t rows = from_layout == TF24_COMPRESSED_PANEL ? k / 32 : m, cols = from_layout == TF24_COMPRESSED_PANEL ? m : k / 32;
-    const int64_t tiles_c = (cols + 63) / 64, tiles = tiles_c * ((rows + 63) / 64);
-    if (tiles > 0x7fffffffLL) return fail(TF24_ERR_SHAPE, "%s: matrix too large", fn);
+  const int64_t rows = from_layout == TF24_COMPRESSED_PANEL ? k / 32 : m, cols = from_layout == TF24_COMPRESSED_PANEL ? m : k / 32;
+  const int64_t tiles_c = (cols + 63) / 64, tiles = tiles_c * ((rows + 63) / 64);
+  if (tiles > 0x7fffffffLL) return fail(TF24_ERR_SHAPE, "%s: matrix too large", fn);
+  // metadata alone between the canonical and the panel form (values_out is NULL then): by transposition from the number of
+  // 64 x 64 tiles on that occupies the chip.  us, word by word -> transposed: 16-bit types 3072 x 768 (48 tiles) 2.5 -> 3.4, 1600 x 6400
+  // (100) 3.5 to 5.4 -> 3.5 to 4.0, 4096 x 4096 (128) 4.3 -> 3.6; 8-bit types, whose words are twice as wide, 4096 x 4096 3.3 -> 3.9,
+  // 3072 x 12288 (288) 6.7 -> 4.7.
+  if (from_layout != TF24_COMPRESSED_CUTLASS && to_layout != TF24_COMPRESSED_CUTLASS && tiles >= (is_8bit(dtype) ? 192 : 96)) {
     hipLaunchKernelGGL(transpose_words, dim3((unsigned)tiles), dim3(kThreads), 0, s, (const uint32_t*)meta_in, rows, cols, (uint32_t)tiles_c, (uint32_t*)meta_out);
     return check_launch(fn);
   }
