@@ -242,7 +242,9 @@ def test_product_from_reference_ordered_metadata(cuda, dtype, n, k, j):
     (torch.float16, 96, 256, 8, False),            # one-pass kernel for a few dense columns
     (torch.float16, 352, 640, 48, False),          # 256 x 64 tiles
     (torch.bfloat16, 352, 640, 120, False),        # 256 x 128 tiles
-    (torch.float16, 352, 640, 296, False),         # 256 x 256 tiles, one workgroup per tile
+    (torch.float16, 352, 640, 296, False),         # 256 x 128 tiles, several columns of them
+    (torch.float16, 768, 320, 12288, False),       # 256 x 256 tiles, one workgroup per tile
+    (torch.float8_e4m3fn, 768, 640, 12288, False),
     (torch.float16, 352, 640, 296, True),          # i-major output, k strided dense operand
     (torch.float16, 256, 4096, 264, False),        # k pieces through the workspace
     (torch.bfloat16, 4128, 320, 4112, False),      # chained tiles, 8 waves
@@ -320,10 +322,11 @@ def test_repack_to_one_part_only(cuda, dtype, m, k):
     assert N.lib().tf24_repack_to(None, None, code, m, k, N.COMPRESSED_PANEL, N.COMPRESSED_CANONICAL, None, None, N.stream_ptr()) != 0
 
 
-@pytest.mark.parametrize("m,k", [(32, 128), (96, 2176), (64, 2048), (1056, 192 * 32)])
+@pytest.mark.parametrize("m,k", [(32, 128), (96, 2176), (64, 2048), (1056, 192 * 32), (2016, 192 * 32), (2048, 192 * 32), (4096, 192 * 32), (4128, 200 * 32)])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.float8_e4m3fn])
 def test_metadata_words_move_alone(cuda, dtype, m, k):
-    """canonical <-> panel metadata without the values: the transpose of 4-byte words, at sizes that fill its 64 x 64 tiles and not."""
+    """canonical <-> panel metadata without the values: word by word below 96 tiles of 64 x 64 words (8-bit types 192), from there
+    on transposed tile by tile, with tiles that are full and not."""
     import sparse
     N = sparse._native
     words = torch.randint(-2 ** 31, 2 ** 31 - 1, (m, k // 32), device=cuda, dtype=torch.int32, generator=torch.Generator(device=cuda).manual_seed(m + k))

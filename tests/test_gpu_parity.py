@@ -1096,8 +1096,8 @@ def test_spmm_chained_tiles_32bit_output(cuda, dtype, k, act):
 @pytest.mark.parametrize("n,k,rows", [(64, 128, 1), (32, 128, 7), (8192, 256, 3), (10240, 128, 15), (512, 512, 17), (288, 384, 63), (544, 2048, 65),
                                       (768, 256, 127), (256, 4096, 129), (4096, 1024, 255), (3072, 768, 1025), (2304, 4096, 2049), (1600, 6400, 4001)])
 def test_linear_any_number_of_rows(cuda, dtype, n, k, rows):
-    """tf24_linear against the float32 product on small integers (exact), row counts that are multiples of nothing and
-    reach every kernel and tile width; the rows behind the last stay as they were."""
+    """tf24_linear against the float32 product on small integers (exact), row counts that are multiples of nothing, on the
+    narrow kernels and the 64- and 128-wide tiles; the rows behind the last stay as they were."""
     import sparse
     from sparse import _native as N
     g = torch.Generator().manual_seed(rows)
@@ -1120,6 +1120,42 @@ def test_linear_any_number_of_rows(cuda, dtype, n, k, rows):
         assert bool((y[rows:] == 77).all())
     got = torch.mm(xs, s.t())
     assert got.shape == (rows, n) and got.float().equal(want.to(got.dtype).float())
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float8_e4m3fn, torch.int8])
+@pytest.mark.parametrize("n,stages,rows", [
+    (768, 12, 12285),          # 256 x 256 tiles, a workgroup each
+    (6144, 192, 757),          # 256 x 256 tiles in three pieces of k
+    (4128, 4, 4111),           # 289 tiles on 256 workgroups, chained, eight waves
+    (4128, 33, 4111),          # the same, four waves; 256 x 192 tiles with 16-bit results
+    (1760, 33, 12271),         # two rounds of 256 x 192 tiles with 16-bit results
+    (800, 33, 12271),          # one round of them
+    (4128, 33, 8175)])         # full rounds of 256 x 256 tiles, the last tile row in a second launch
+def test_linear_ragged_rows_on_wide_tiles(cuda, dtype, n, stages, rows):
+    """Row counts that fill no tile on each kernel of more than 256 tiles of 256 x 128, with 32- and 16-bit results; the rows behind
+    the last stay as they were.  Exact on small integers.  S @ x.t(), whose results lie the other way round, with the
+    rows that are whole multiples of 16."""
+    import sparse
+    from sparse import _native as N
+    k = stages * 128 // torch.empty(0, dtype=dtype).element_size()
+    g = torch.Generator(device=cuda).manual_seed(rows + stages)
+    w = torch.randint(-2, 3, (n, k), device=cuda, generator=g)
+    s = sparse.to_sparse_semi_structured(w.to(torch.int8) if dtype == torch.int8 else w.float(), dtype=dtype)
+    x = torch.randint(-2, 3, (rows, k), device=cuda, generator=g).to(dtype)
+    want = x.float() @ s.to_dense().float().t()
+    code, lib = N.operand_code(dtype), N.lib()
+    nbytes = lib.tf24_spmm_workspace_bytes(code, n, k, rows)
+    ws = torch.empty(max(nbytes, 16), dtype=torch.uint8, device=cuda)
+    a = (s._store_values.data_ptr(), s._store_meta.data_ptr(), N.COMPRESSED_PANEL, code, n, k, x.data_ptr())
+    tail = (None, 1.0, N.ACT_NONE, ws.data_ptr(), nbytes, N.stream_ptr())
+    for out_dtype in ((torch.int32,) if dtype == torch.int8 else (torch.float32, torch.float16, torch.bfloat16)):
+        y = torch.full((rows + 3, n), 77, dtype=out_dtype, device=cuda)
+        N.check(lib.tf24_linear(*a, k, rows, y.data_ptr(), N.operand_code(out_dtype), n, *tail))
+        assert y[:rows].equal(want.to(out_dtype)) and bool((y[rows:] == 77).all()), out_dtype
+        whole = rows // 16 * 16
+        yt = torch.full((n + 1, whole), 77, dtype=out_dtype, device=cuda)
+        N.check(lib.tf24_spmm(*a, N.ROW_MAJOR, k, whole, yt.data_ptr(), N.operand_code(out_dtype), N.ROW_MAJOR, whole, *tail))
+        assert yt[:n].equal(want[:whole].t().to(out_dtype)) and bool((yt[n] == 77).all()), out_dtype
 
 
 @pytest.mark.parametrize("dtype,rows,k,view", [

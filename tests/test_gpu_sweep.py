@@ -53,8 +53,8 @@ def _store(x, col_major, pad, dev):
 
 @pytest.mark.parametrize("seed,large", [(1, False), (2, False), (3, True)])
 def test_spmm_sweep(cuda, seed, large):
-    """Every kernel of the matmul (one-pass, 64-, 128- and 256-wide tiles with and without k pieces,
-    general) is reached by some of these shapes; all five operand dtypes, all operand positions."""
+    """The matmul's one-pass and general kernels, its 64- and 128-wide tiles and, with a k-strided dense operand, its 256-wide ones,
+    with and without k pieces, are reached by some of these shapes; all five operand dtypes, all operand positions."""
     import sparse
     rng = random.Random(seed)
     failures = []

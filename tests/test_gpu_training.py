@@ -648,6 +648,41 @@ def test_grad_weight_kernel(cuda, tokens, m, n, dtype):
                     assert ((got.double() - want).abs() <= limit).all(), (name, bytes_given, with_bias)
 
 
+@pytest.mark.parametrize("tokens,m,n", [(1, 8, 8), (31, 264, 40), (65, 248, 1000), (129, 768, 512), (1000, 3072, 768), (4099, 768, 3072), (12287, 520, 264)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_grad_weight_kernel_is_exact_and_deterministic(cuda, tokens, m, n, dtype):
+    """Small integers, whose sums float32 holds exactly in any order: dW and db are those sums rounded once, whatever the number
+    of pieces (partial sums of 16 bits would not be).  Random operands: the same bits again, and an error of about
+    sqrt(tokens) roundings of sums of that size (8 standard deviations of them) beside the one to 16 bits."""
+    from sparse import _native as N
+    gen = torch.Generator(device=cuda).manual_seed(tokens + m + n)
+    lib = N.lib()
+    nbytes = lib.tf24_grad_weight_workspace_bytes(tokens, m, n)
+    ws = torch.empty(max(nbytes, 16), dtype=torch.uint8, device=cuda)
+
+    def run(g, x, bytes_given):
+        dw, db = torch.empty((m, n), dtype=dtype, device=cuda), torch.empty((m,), dtype=dtype, device=cuda)
+        N.check(lib.tf24_grad_weight(g.data_ptr(), m, x.data_ptr(), n, N.dtype_code(dtype), tokens, m, n, dw.data_ptr(), db.data_ptr(),
+                                     ws.data_ptr(), bytes_given, N.stream_ptr()))
+        return dw, db
+
+    g, x = (torch.randint(-8, 9, (tokens, c), device=cuda, generator=gen).to(dtype) for c in (m, n))
+    want = (g.double().t().contiguous() @ x.double()).to(dtype), g.double().sum(0).to(dtype)
+    for bytes_given in {0, nbytes}:
+        for got, exact in zip(run(g, x, bytes_given), want):
+            assert got.equal(exact), bytes_given
+    g, x = (torch.randn(tokens, c, device=cuda, generator=gen).to(dtype) for c in (m, n))
+    exact = g.double().t().contiguous() @ x.double(), g.double().sum(0)
+    half_ulp = 2.0 ** (-11 if dtype == torch.float16 else -8)
+    for bytes_given in {0, nbytes}:
+        first = run(g, x, bytes_given)
+        for got, again, ref in zip(first, run(g, x, bytes_given), exact):
+            assert got.equal(again), bytes_given
+            # each of the `tokens` additions rounds a partial sum of at most about 4 sqrt(tokens) by half of 2^-23 of it
+            limit = ref.abs() * half_ulp + 8 * tokens ** 0.5 * (4 * tokens ** 0.5) * 2.0 ** -24 + 2.0 ** -25
+            assert bool(((got.double() - ref).abs() <= limit).all()), bytes_given
+
+
 @pytest.mark.parametrize("tokens,bias,dtype", [((300,), True, torch.bfloat16), ((5, 41), True, torch.float16), ((4100,), False, torch.bfloat16),
                                                ((3, 200), False, torch.float16)])
 def test_soft_threshold_linear_under_autocast(cuda, tokens, bias, dtype):
