@@ -18,22 +18,14 @@
 // one of the 64 banks once (with a swizzle that only spreads 16 lanes, half of the LDS cycles are conflicts).
 // Few tiles and a long token axis: the axis is cut into pieces (choose_pieces); their float32 partial tiles are added in
 // piece order by a second kernel, which rounds once.
-#include "tf24_common.hpp"
+#include "lds_copies.hpp"
 #include <algorithm>
 #include <type_traits>
 
 namespace tf24 {
 namespace {
 
-typedef _Float16 half8 __attribute__((ext_vector_type(8)));
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float float4v __attribute__((ext_vector_type(4)));
-typedef float float16v __attribute__((ext_vector_type(16)));
-typedef short short4v __attribute__((ext_vector_type(4)));
 typedef short short8v __attribute__((ext_vector_type(8)));
-typedef int int4v __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(3))) void* lds_ptr_t;
-typedef __attribute__((address_space(3))) short4v* lds_short4_ptr;
 
 constexpr int kTile = 256, kStageTokens = 32, kRing = 5;
 constexpr int kRowBytes = kTile * 2, kOperand = kStageTokens * kRowBytes, kStage = 2 * kOperand;
@@ -53,15 +45,6 @@ __device__ __forceinline__ float16v mma(bf16_t, short8v a, short8v b, float16v c
 __device__ __forceinline__ float widen(f16_t, short h) { return to_float(f16_t{(uint16_t)h}); }
 __device__ __forceinline__ float widen(bf16_t, short h) { return to_float(bf16_t{(uint16_t)h}); }
 
-// 16 bytes per lane straight into LDS (lane l at base + 16 * l), invisible to the compiler's wait counts: it would drain
-// every copy before each fragment read.  Waits are written out below.
-__device__ __forceinline__ void copy16(const uint8_t* base, uint32_t lane_offset, uint32_t lds_base) {
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(lane_offset), "s"(base), "s"(lds_base) : "memory", "m0");
-}
-template <int N>
-__device__ __forceinline__ void wait_copies_and_barrier() {
-  asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(N) : "memory");
-}
 __device__ __forceinline__ uint32_t swizzle(uint32_t token) { return ((token & 3) << 2) | (((token >> 3) & 1) << 1); }
 
 // Rows of fragment ti of a wave: the four waves that share 128 rows hold their fragments rotated, so that fragment 0 of
@@ -114,18 +97,18 @@ grad_weight_pipe(const uint8_t* __restrict__ g, int64_t ldg, const uint8_t* __re
     og[q] = offset_of(q, i0, m, ldg, kStageTokens);
     ox[q] = offset_of(q, j0, n, ldx, kStageTokens);
   }
-  const uint32_t smem_at = (uint32_t)(uintptr_t)(lds_ptr_t)smem;
+  const uint32_t smem_at = lds_offset(smem);
   auto copy_one = [&](int q, int st, uint32_t buf) {             // q: the wave's copies of G, then those of X
     const uint32_t dst = smem_at + buf + (uint32_t)(wave * kCopies + (q % kCopies)) * 1024;
-    if (q < kCopies) copy16(g_at + (int64_t)st * g_step, og[q], dst);
-    else copy16(x_at + (int64_t)st * x_step, ox[q - kCopies], dst + kOperand);
+    if (q < kCopies) g2l16(g_at + (int64_t)st * g_step, og[q], dst);
+    else g2l16(x_at + (int64_t)st * x_step, ox[q - kCopies], dst + kOperand);
   };
   auto copy_ragged = [&](int st, uint32_t buf) {                 // tokens past the last one re-read it (and are zeroed on arrival)
 #pragma unroll
     for (int q = 0; q < kCopies; q++) {
       const uint32_t dst = smem_at + buf + (uint32_t)(wave * kCopies + q) * 1024;
-      copy16(g_at + (int64_t)st * g_step, offset_of(q, i0, m, ldg, ragged), dst);
-      copy16(x_at + (int64_t)st * x_step, offset_of(q, j0, n, ldx, ragged), dst + kOperand);
+      g2l16(g_at + (int64_t)st * g_step, offset_of(q, i0, m, ldg, ragged), dst);
+      g2l16(x_at + (int64_t)st * x_step, offset_of(q, j0, n, ldx, ragged), dst + kOperand);
     }
   };
   auto copy_stage = [&](int st, uint32_t buf) {
@@ -138,9 +121,9 @@ grad_weight_pipe(const uint8_t* __restrict__ g, int64_t ldg, const uint8_t* __re
   // stage st has arrived when this wave's copies of the (at most two) stages behind it are all that is in flight
   auto arrive = [&](int st, uint32_t buf) {
     const int behind = nstages - 1 - st;
-    if (behind >= 2) wait_copies_and_barrier<4 * kCopies>();
-    else if (behind == 1) wait_copies_and_barrier<2 * kCopies>();
-    else wait_copies_and_barrier<0>();
+    if (behind >= 2) wait_copies_and_barrier<4 * kCopies, false>();
+    else if (behind == 1) wait_copies_and_barrier<2 * kCopies, false>();
+    else wait_copies_and_barrier<0, false>();
     if (st == ragged_stage) {
       for (int c = tid; c < (kStageTokens - ragged) * (kRowBytes / 16); c += kThreads) {
         *reinterpret_cast<int4v*>(smem + buf + ragged * kRowBytes + c * 16) = int4v{0, 0, 0, 0};
@@ -185,7 +168,7 @@ grad_weight_pipe(const uint8_t* __restrict__ g, int64_t ldg, const uint8_t* __re
   // Column sums of G: one element behind each matrix instruction (two vector instructions under 32 cycles of it), by the
   // blocks of every tile column: a branch here would make the compiler wait for all reads in flight.
   float colsum[kSums] = {};
-  // The 16 instructions of a step from one register set; behind each of them one read of the next step into the other set
+  // The instructions of a step from one register set; behind each of them one read of the next step into the other set
   // and, over the two steps of a stage, the copies of stage cst.
   auto mma_step = [&](int set, bool reads, uint32_t src, int rstep, int half, bool copies, int cst, uint32_t dst) {
     __builtin_amdgcn_sched_barrier(0);
@@ -223,7 +206,7 @@ grad_weight_pipe(const uint8_t* __restrict__ g, int64_t ldg, const uint8_t* __re
   int st = 1;
   for (; st + 3 < whole; st++) {
     cur = next_buf(cur); far = next_buf(far);
-    wait_copies_and_barrier<4 * kCopies>();
+    wait_copies_and_barrier<4 * kCopies, false>();
     mma_step(1, true, cur, 0, 0, true, st + 3, far);             // the last step of stage st - 1
     mma_step(0, true, cur, 1, 1, true, st + 3, far);
   }

@@ -15,7 +15,7 @@
 //      range shifted by K/2
 //   D: 16x16: column l%16, rows 4*(l/16)+r;  32x32: column l%32, rows 8*(r/4) + 4*(l/32) + r%4
 #pragma once
-#include "tf24_common.hpp"
+#include "lds_copies.hpp"
 #include <algorithm>
 #include <atomic>
 #include <type_traits>
@@ -23,13 +23,8 @@
 namespace tf24 {
 namespace {
 
-typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef _Float16 half16 __attribute__((ext_vector_type(16)));
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x16 __attribute__((ext_vector_type(16)));
-typedef float float4v __attribute__((ext_vector_type(4)));
-typedef float float16v __attribute__((ext_vector_type(16)));
-typedef int int4v __attribute__((ext_vector_type(4)));
 typedef int int8v __attribute__((ext_vector_type(8)));
 typedef int int16v __attribute__((ext_vector_type(16)));
 
@@ -350,32 +345,6 @@ using SlimCfg = TileCfgT<1, 2>;
 // 256 x 128 tiles, four waves: dense operands of 65 to 128 columns
 using MidCfg = TileCfgT<2, 2>;
 
-typedef __attribute__((address_space(3))) void* lds_ptr_t;
-
-// The copies are issued from inline assembly so that the compiler's wait-count insertion does not
-// see them: it would otherwise drain all outstanding copies (vmcnt(0)) before every LDS read, because
-// it cannot tell the three stage buffers apart.  Ordering is enforced by hand with s_waitcnt vmcnt(N)
-// before the stage barrier.  M0 carries the wave-uniform LDS base of the copy.
-__device__ __forceinline__ uint32_t lds_offset(const void* p) {
-  return (uint32_t)(uintptr_t)(lds_ptr_t)p;
-}
-// The source address is a wave-uniform 64-bit base in scalar registers plus a 32-bit offset per lane: with a
-// 64-bit address per lane the same copies hold up the matrix instructions issued around them (on an
-// instruction mix like the main loop's, 25 % more cycles than the matrix instructions alone against 3 %).
-// same with one dword per lane: lane l writes LDS[base + 4*l]
-__device__ __forceinline__ void g2l4(const uint8_t* base, uint32_t lane_offset, uint32_t lds_base) {
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" ::"v"(lane_offset), "s"(base), "s"(lds_base) : "memory", "m0");
-}
-__device__ __forceinline__ void g2l16(const uint8_t* base, uint32_t lane_offset, uint32_t lds_base) {
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(lane_offset), "s"(base), "s"(lds_base) : "memory", "m0");
-}
-// s_waitcnt vmcnt(N) + s_barrier with a compile-time N (a bare s_barrier: __syncthreads() would add
-// a fence that drains every outstanding copy)
-template <int N>
-__device__ __forceinline__ void wait_copies_and_barrier() {
-  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
-}
-
 // workgroup barrier behind this wave's LDS reads only: copies stay in flight
 __device__ __forceinline__ void wait_reads_and_barrier() {
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
@@ -583,8 +552,6 @@ spmm_pipe(const uint8_t* __restrict__ a_values, const uint8_t* __restrict__ a_me
   int4v af[2][C::TI];
   int idx[2][C::TI];
   int4v bf[2][C::TJ][2];                         // the two 16-byte halves of a dense fragment
-  typedef short short4v __attribute__((ext_vector_type(4)));
-  typedef __attribute__((address_space(3))) short4v* lds_short4_ptr;
   short4v bq[2][C::TJ][4];                       // k-strided B: the four 8-byte quarters
   // The reads of a step, in the order the next step's instructions need them: its first row of
   // instructions takes every dense fragment and sparse fragment 0, row r then only needs sparse
@@ -682,9 +649,9 @@ spmm_pipe(const uint8_t* __restrict__ a_values, const uint8_t* __restrict__ a_me
   static_assert(C::STEPS == 2, "the pipeline below is written for two instruction steps per stage");
   static_assert(!PERSIST || C_JMAJOR, "chained tiles rely on the wait inside the j-major output passes");
   auto stage_barrier = [&](bool more) {          // B(st+1): only this wave's copies of stage st+2 may still fly
-    if (!more) wait_copies_and_barrier<0>();
-    else if (MWAVES == C::NW || has_meta) wait_copies_and_barrier<NCOPY>();
-    else wait_copies_and_barrier<NCOPY - MW>();
+    if (!more) wait_copies_and_barrier<0, true>();
+    else if (MWAVES == C::NW || has_meta) wait_copies_and_barrier<NCOPY, true>();
+    else wait_copies_and_barrier<NCOPY - MW, true>();
   };
 
   issue(0, smem_at);
