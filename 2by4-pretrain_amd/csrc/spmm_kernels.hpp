@@ -1456,13 +1456,15 @@ spmm_narrow_shared(const uint8_t* __restrict__ a_values, const uint8_t* __restri
 // more columns cost requests with every panel of every block, so it depends on the panels: 16 columns of 4096 x 4096 12.8 -> 8.7,
 // of 768 x 3072 8.8 -> 7.9, but of 1600 x 6400 12.4 -> 14.8; 32 of 4096 x 2048 10.3 -> 7.7; 64 of 4096 x 1536 13.5 -> 9.4, of
 // 2304 x 768 9.0 -> 6.5, but of 2304 x 2048 10.7 -> 11.2.  With two blocks to a compute unit (6144 rows): 48 of k = 768
-// 9.0 -> 8.0 and of 1536 13.7 -> 12.5, 64 of k = 768 9.1 -> 9.6.  Past 128 panels the few workgroups of the shared form fall behind
+// 9.0 -> 8.0 and of 1536 13.7 -> 12.5, 64 of k = 768 9.1 -> 9.6; 9 and 16 columns of 64 panels 12.2 -> 10.5
+// and 12.4 -> 12.8, of 96 14.0 -> 14.3 and 18.0.  With three (12288 rows) 17 and 32 columns of 16 panels 10.4 -> 8.1 and 10.0, 32 of
+// 24 panels 13.5 -> 14.1; with four (16384 rows) 32 of 16 panels 10.5 -> 12.1.  Past 128 panels the few workgroups of the shared form fall behind
 // k pieces (16 columns of 8192 x 8192 18.6 -> 19.5, of 8192 x 16384 28.3 -> 34.8, of 11008 x 16384 35.7 -> 49.5).
 inline int64_t narrow_columns(int64_t n_sparse, int64_t npanels) {
   const int64_t blocks = n_sparse / 16;
-  if (blocks <= 256) return npanels <= 24 ? 64 : npanels <= 32 ? 32 : npanels <= 64 ? 16 : 8;
-  if (blocks <= 512 && npanels <= 32) return npanels <= 24 ? 48 : 32;
-  return blocks >= 512 && npanels <= 128 ? 16 : 8;
+  if (blocks <= 512 && npanels <= 32) return npanels > 24 ? 32 : blocks <= 256 ? 64 : 48;
+  if (blocks <= 768 && npanels <= 16) return 32;
+  return npanels <= (blocks >= 512 ? 128 : 64) ? 16 : 8;
 }
 
 template <typename T, typename OutT>

@@ -1191,7 +1191,8 @@ def test_linear_rows_in_views(cuda, dtype, rows, k, view, n):
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float8_e4m3fn, torch.int8])
-@pytest.mark.parametrize("n,panels", [(32, 1), (256, 5), (4096, 24), (4128, 24), (4096, 25), (768, 32), (4096, 33), (96, 64), (6144, 9), (8192, 17), (8224, 3)])
+@pytest.mark.parametrize("n,panels", [(32, 1), (256, 5), (4096, 24), (4128, 24), (4096, 25), (768, 32), (4096, 33), (96, 64), (6144, 9), (8192, 17), (8224, 3), (4128, 33), (7168, 64),
+                                      (4128, 65), (8192, 33), (12288, 16), (12320, 5), (10240, 17)])
 def test_few_dense_columns(cuda, dtype, n, panels):
     """Dense extents up to and past those that the narrow kernels take, both output orders; exact on small integers."""
     import sparse
