@@ -111,7 +111,7 @@ repack_kernel(const uint8_t* __restrict__ vin, const uint8_t* __restrict__ min_,
 
 // Metadata between the canonical and the panel form, as 4-byte words: [m][k/32] <-> [k/32][m], the transpose of a matrix
 // in[rows][cols].  A block moves 64 x 64 words through LDS, 256 contiguous bytes per wave and access on both sides (the
-// word-by-word kernel below scatters 2-byte words: 8192 x 8192 13.6 us, here 5.0).
+// word-by-word kernel below scatters 2-byte words: 8192 x 8192 13.6 us, here 5.0; with few tiles it is the faster one).
 __global__ void __launch_bounds__(kThreads)
 transpose_words(const uint32_t* __restrict__ in, int64_t rows, int64_t cols, uint32_t tiles_c, uint32_t* __restrict__ out) {
   __shared__ uint32_t s_tile[64][65];
@@ -133,7 +133,7 @@ transpose_words(const uint32_t* __restrict__ in, int64_t rows, int64_t cols, uin
   }
 }
 
-// Metadata from or to the reordered form, one lane per metadata word (WB bytes), lanes walking the
+// Metadata between any two forms, one lane per metadata word (WB bytes), lanes walking the
 // words in the order of the reordered form ([word-column pair][row][2]: whole cache lines on that side,
 // and on the panel side up to a permutation of 32 adjacent rows).
 template <int WB>
@@ -186,7 +186,7 @@ extern "C" int tf24_repack_to(const void* values_in, const void* meta_in, int dt
   }
   if (m <= 0 || m % 32 || k <= 0 || k % kp)
     return fail(TF24_ERR_SHAPE, "%s: shape (%lld, %lld): m must be a positive multiple of 32 and k of %lld", fn, (long long)m, (long long)k, (long long)kp);
-  // from here on the metadata moves through the word-by-word kernel: any pair with the reordered form, or metadata alone
+  // from here on: any pair with the reordered form, or metadata alone
   const bool panel_side = from_layout == TF24_COMPRESSED_PANEL || to_layout == TF24_COMPRESSED_PANEL;
   if (!meta_in || !meta_out || (values_out && !values_in)) return fail(TF24_ERR_ARG, "%s: null pointer", fn);
   if (meta_in == meta_out || (values_out && values_in == values_out)) return fail(TF24_ERR_ARG, "%s: in-place conversion is not supported", fn);

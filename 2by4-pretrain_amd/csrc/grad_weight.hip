@@ -289,7 +289,8 @@ int64_t piece_bytes(int64_t tiles_i, int64_t tiles_j) { return (tiles_i * tiles_
 
 // The number of pieces with the least  stages of one piece x 0.6 us + (more than one: 3 us + 0.32 us per MB of partial tiles),
 // all in one round of the compute units.  The constants are fitted to timings of 1 to 16 pieces over 500 to 16384 tokens
-// and 2048 x 512 to 6400 x 1600 outputs; the choice is within 4 % of the best on all of them.  36 tiles, us:
+// and 2048 x 512 to 6400 x 1600 outputs; the choice is within 4 % of the best on all of them.  More than 128 tiles stay in one
+// piece, since two would need a second round of the compute units (against the library's product see _linear16).  36 tiles, us:
 // 12288 tokens 209 in one piece, 82 in three, 72 in seven; 1024 tokens 24 in one, 31 in seven.
 int choose_pieces(int64_t tokens, int64_t tiles_i, int64_t tiles_j, int64_t workspace_bytes) {
   const int64_t stages = (tokens + kStageTokens - 1) / kStageTokens, tiles = tiles_i * tiles_j;

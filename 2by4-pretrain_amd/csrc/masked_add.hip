@@ -4,7 +4,7 @@
 // Bound by memory.  At 8 float32 elements per lane (two 16-byte accesses, 32 bytes from lane to lane) every wave
 // instruction touched half lines: 8192 x 8192 float32 with a byte mask 147 us = 5.9 TB/s, streaming accesses of the
 // gradient 154 us.  With one 16-byte access per lane and streaming accesses of everything, the gradient included:
-// 127 us = 6.9 TB/s (11008 x 4096: 101 -> 88 us, 3072 x 768: 7.0 -> 6.2 us).
+// 134.7 us = 6.5 TB/s (11008 x 4096: 101 -> 88 us, 3072 x 768: 7.0 -> 6.2 us).
 #include "tf24_common.hpp"
 
 namespace tf24 {

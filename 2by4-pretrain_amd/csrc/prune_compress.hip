@@ -542,7 +542,7 @@ int dispatch_mask(const void* dense, int layout, int64_t ld, int64_t m, int64_t 
   if constexpr (MODE != TF24_PRUNE_MASK) {
     return launch<In, Out, MODE, uint8_t>(dense, layout, ld, m, k, nullptr, 0, rs, values, meta, panel, rowsum_partial, s);
   } else if constexpr (std::is_same<In, i8_t>::value) {
-    // int8 matrices take byte masks only (the column kernel reads 16 rows per lane: 16-byte mask loads)
+    // int8 matrices take byte masks only (the column kernel reads 8 rows per lane and column: 8-byte mask loads)
     if (mask_dtype != TF24_U8) return fail(TF24_ERR_DTYPE, "tf24_prune_compress: int8 input takes a byte mask (dtype %d given)", mask_dtype);
     return launch<In, Out, MODE, uint8_t>(dense, layout, ld, m, k, mask, mask_ld, rs, values, meta, panel, rowsum_partial, s);
   } else {

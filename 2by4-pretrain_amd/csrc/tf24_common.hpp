@@ -189,8 +189,8 @@ struct Pack {
     *reinterpret_cast<V*>(p) = *reinterpret_cast<const V*>(v);
   }
   // Streaming variants for data touched once per kernel (non-temporal: the lines are not kept in
-  // L2).  On the one-pass conversion kernels they are worth 5-20 %; not for read-modify-write
-  // operands, whose loads got slower.
+  // L2).  On the one-pass conversion kernels they are worth 5-20 %.  Operands that
+  // are updated in place gain only where both the load and the store are of this form.
   __device__ __forceinline__ void load_stream(const T* p) {
     constexpr int B = sizeof(T) * N;
     if constexpr (B % 16 == 0) {
@@ -440,8 +440,8 @@ __device__ __forceinline__ Mvue4 mvue4_as(const float (&x)[4], float r0, float r
 // costs 80 (half precision) to 85, a generator call 50 for two groups.  One correction per division instead of two, no
 // branch and one test of the bounds per group (the slow path is laid out behind the kernel), flags as short-circuit
 // expressions (as integers they went through vector registers), kept values converted without a test for NaN, and leaner
-// addresses in the callers: 8192 x 8192 bf16 to e4m3 82 -> 64.5 us, to fp16 78.6 -> 64.5 (with a supplied tensor, where
-// its 268 MB are the bound, 77 -> 69), a column-major 3072 x 12288 half matrix with its row sums 54.5 -> 44 us.
+// addresses in the callers: 8192 x 8192 bf16 to e4m3 82 -> 64.5 us, to fp16 78.6 -> 64.5 (with a supplied tensor its
+// 268 MB are the bound: 80 us before and after), a column-major 3072 x 12288 half matrix with its row sums 54.5 -> 44 us.
 template <typename In>
 __device__ __forceinline__ Mvue4 mvue4(const float (&x)[4], float r0, float r1, bool& finite) {
   bool ok;
