@@ -1000,28 +1000,33 @@ spmm_reduce_splits(const float* __restrict__ partial, int splits, int tiles_i, i
 
 // How many k pieces a product is cut into, for shapes whose tiles cannot fill the 256 compute units: the number for which
 //     CALL_US + max(stages of one piece x STAGE_US, MB of the compressed operand x OPERAND_US)
-//             + (pieces > 1: SPLIT_US + MB of partial sums, all pieces, x PARTIAL_US)
+//             + (pieces > 1: SPLIT_US + pieces x PIECE_US + MB of partial sums, all pieces, x PARTIAL_US) + (pieces > 8: 0.5),
+// and 2 % more with over 208 blocks,
 // is least, among those whose blocks fit one round of the compute units and whose float32 partial tiles fit the caller's
 // workspace.  (Two of the narrowest tiles fit on one compute unit, but a few blocks more than there are units make the
 // whole product wait for the shared ones: fp8 11008 x 11008 against 48 columns 19.3 us in 5 pieces = 215 blocks, 26.4 in 6 = 258.)
 // Only the 32-column slabs that the dense operand reaches are written and read back, so only they count: k-strided
 // 6144 x 1536 against 16 columns 20.5 us in one piece, 12.4 in five.  Below some pieces the narrowest tiles are bound by the
 // one pass over the compressed operand (OPERAND_US: 8.8 TB/s, it stays in the last cache over repeated products).
+// From nine pieces on the reduction, which loads eight at a time, goes round twice: 768 x 3072 against 86 columns 10.0 us in
+// eight pieces, 10.5 in nine and more; 480 x 2816 against 321 11.7 in five, 13.2 in nine.
+// Rounds of more than 208 blocks scatter: 4096 x 11008 against 257 to 305 columns 29.4 to 34.6 us in five pieces = 240 blocks,
+// 29.8 to 30.8 in four.
 // The constants are least-squares fits, per tile configuration, to 25 000 timings of 1 to 16 pieces over fp16 and fp8 weights from
 // 256 x 768 to 20480 x 11008 (6 to 512 stages) and 16 to 3072 dense columns.  The pieces chosen this way are within 1 % of
-// the best ones on average and within 5 % for 19 in 20 (a fixed 192 / tiles of them: 5, 18 and 9 % off for the three
+// the best ones on average and within 4 to 6 % for 19 in 20 (a fixed 192 / tiles of them: 5, 18 and 9 % off for the three
 // configurations below, and twice the time at worst; a fit to the range of 768 x 768 to 8192 x 8192 alone that counted whole tiles
 // 7, 2 and 5 %, half again the time at worst).  us, with 192 / tiles pieces and now: 3072 x 768 against 1024 columns
 // 22.2 -> 9.0 (2 pieces -> 1), 4096 x 4096 against 128 19.0 -> 16.1 (12 -> 5); dW of 1024 tokens, 3072 x 768, 26.2 -> 16.4 (4 -> 1).
 // A k-contiguous product of at most kShortStages stages is not cut: the reduction's launch and workspace are 4 us of host time,
 // which bounds such calls one after the other (linear of 96 rows with 256 x 1536: 14.6 us a call in one piece, 18.5 in
 // eight; alone 33.0 and 30.3 us, on the GPU 12.9 and 8.6).
-struct PieceCost { double call_us, stage_us, split_us, partial_us, operand_us; };
+struct PieceCost { double call_us, stage_us, split_us, piece_us, partial_us, operand_us; };
 template <typename C>
 constexpr PieceCost piece_cost(bool k_strided) {
-  return std::is_same<C, SlimCfg>::value ? PieceCost{5.1, 0.37, 1.8, 0.48, 0.113}
-         : std::is_same<C, MidCfg>::value ? PieceCost{5.6, 0.33, 2.1, 0.45, 0.0}
-         : k_strided ? PieceCost{7.1, 0.55, 1.15, 0.42, 0.0} : PieceCost{6.9, 0.50, 3.3, 0.385, 0.0};
+  return std::is_same<C, SlimCfg>::value ? PieceCost{5.1, 0.37, 1.8, 0.0, 0.48, 0.113}
+         : std::is_same<C, MidCfg>::value ? PieceCost{5.6, 0.33, 2.1, 0.1, 0.45, 0.0}
+         : k_strided ? PieceCost{7.1, 0.55, 1.15, 0.0, 0.42, 0.0} : PieceCost{6.9, 0.50, 3.3, 0.0, 0.385, 0.0};
 }
 constexpr int64_t kShortStages = 28;
 struct Pieces { int count; double us; };
@@ -1033,7 +1038,9 @@ Pieces choose_pieces(int64_t n_sparse, int64_t k, int64_t n_dense, int64_t works
   const double operand_us = (double)(n_sparse * k * (int64_t)sizeof(T)) * (9.0 / 16.0) * 1e-6 * cost.operand_us;
   const double partial_us = (double)(tiles_i * C::BI * ((n_dense + 31) / 32 * 32)) * 4e-6 * cost.partial_us;     // of one piece
   auto us = [&](int64_t p) {
-    return cost.call_us + std::max((double)((stages + p - 1) / p) * cost.stage_us, operand_us) + (p > 1 ? cost.split_us + (double)p * partial_us : 0.0);
+    const double one = cost.call_us + std::max((double)((stages + p - 1) / p) * cost.stage_us, operand_us);
+    if (p == 1) return one;
+    return (one + cost.split_us + (double)p * (cost.piece_us + partial_us) + (p > 8 ? 0.5 : 0.0)) * (p * tiles > 208 ? 1.02 : 1.0);
   };
   Pieces best{1, us(1)};
   if (!k_strided && stages <= kShortStages) return best;
