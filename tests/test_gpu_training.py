@@ -721,6 +721,25 @@ def test_soft_threshold_linear_under_autocast(cuda, tokens, bias, dtype):
     assert tangent is not None
 
 
+@pytest.mark.parametrize("tokens,bias", [(40, True), (300, True), (300, False), (4100, False)])
+def test_soft_threshold_linear_backward_inside_autocast(cuda, tokens, bias):
+    """The backward pass gives the same bits outside autocast, inside it, and inside it with another type."""
+    import sparse
+    torch.manual_seed(9)
+    mod = sparse.SoftThresholdLinear(128, 264, bias=bias, device=cuda)
+    mod.init_scale()
+    x = torch.randn(tokens, 128, device=cuda, requires_grad=True)
+    gy = torch.randn(tokens, 264, device=cuda).bfloat16()
+    wanted = [x] + list(mod.parameters())
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        y = mod(x)
+        inside = torch.autograd.grad(y, wanted, gy, retain_graph=True)
+    with torch.autocast("cuda", dtype=torch.float16):
+        other = torch.autograd.grad(y, wanted, gy, retain_graph=True)
+    for a, b, c in zip(torch.autograd.grad(y, wanted, gy), inside, other):
+        assert a.dtype == torch.float32 and a.equal(b) and a.equal(c)
+
+
 @pytest.mark.parametrize("tokens,bias", [(300, True), (4100, False)])
 def test_soft_threshold_linear_backward_under_tangents_and_modes(cuda, tokens, bias):
     """A tangent of the output's gradient reaches the weight's and the bias's, and a dispatch mode around the backward pass sees
