@@ -339,6 +339,7 @@ using Wave4Cfg = TileCfgT<2, 4>;
 // W[11008, 4096] against 2048 tokens alike).  Long chained tiles only, like the 4-wave form itself.
 using Wave4Cfg192 = TileCfgT<2, 3>;
 constexpr int kWave4MinStages = 32;
+constexpr int kRotateMinStages = 64;       // (at least 24: the first three stages of a tile are copied before the order wraps)
 // 256 x 64 tiles, two waves: for dense operands of at most 64 columns (a few dozen tokens), where a
 // 256-wide tile would copy and multiply clamped columns.  26 KB per stage, two blocks per CU.
 using SlimCfg = TileCfgT<1, 2>;
@@ -433,6 +434,17 @@ spmm_pipe(const uint8_t* __restrict__ a_values, const uint8_t* __restrict__ a_me
   const int nstages_total = (int)((k * ES) / C::KB);
   const int st_begin = (int)((int64_t)split * nstages_total / splits);
   const int nstages = (int)((int64_t)(split + 1) * nstages_total / splits) - st_begin;
+  // The tiles of XCD x take their stages from the x-th eighth of k on and wrap round (4-wave form, kRotateMinStages or more
+  // stages).  A stage of the dense operand is 128 bytes from each of 256 rows, whose pitch is often a multiple of some
+  // 4 KB: with all XCDs at the same stage the whole chip reads the same few memory channels at a time, and the copies, two
+  // stages ahead, arrive late wherever the operand comes from memory and not from the last cache.  us on operands that
+  // change from product to product, without and with: e4m3 16384 x 8192 x 8192 537 -> 515 (on the same operands 494 and
+  // 494), bf16 3001 x 11008 x 4096 143 -> 132, f16 8192 x 8192 x 8192 515 -> 498, bf16 9000 x 4096 x 3072 125 -> 122,
+  // f16 8192 x 4096 x 11008 362 -> 362 to 364.  By halves or quarters of k instead of eighths 134 and 133 for the
+  // second, three stages apart 138; 24 and 48 stages: no difference that repeats.
+  constexpr bool ROTATE = PERSIST && C::NW == 4;
+  const int rot = ROTATE && nstages >= kRotateMinStages ? (bid & 7) * nstages >> 3 : 0;
+  const int st_first = st_begin + rot;
 
   // ---- per-lane global sources of the copies (first stage of this unit); LDS destinations are wave-uniform.
   // B: copy q of a wave brings 8 rows x 128 bytes; lane -> (row, swizzled chunk).
@@ -454,10 +466,10 @@ spmm_pipe(const uint8_t* __restrict__ a_values, const uint8_t* __restrict__ a_me
     int lane = threadIdx.x & 63;
     if constexpr (PERSIST) asm volatile("" : "+v"(lane));
     const int64_t last_j = n_dense - 1 - tj0, last_i = n_sparse - 1 - ti0;       // >= 0: tile origins lie inside
-    if constexpr (B_KSTRIDED) tile_b = b + (int64_t)st_begin * B_STAGE_ADVANCE_ROWS * ldb_bytes;   // columns stay absolute: the clamp may step left of the tile
-    else tile_b = b + tj0 * ldb_bytes + (int64_t)st_begin * C::B_ROW;
-    tile_a = a_values + (ti0 + (int64_t)st_begin * n_sparse) * 64;
-    tile_m = a_meta + (ti0 + (int64_t)st_begin * STAGE_KB * n_sparse) * 4;
+    if constexpr (B_KSTRIDED) tile_b = b + (int64_t)st_first * B_STAGE_ADVANCE_ROWS * ldb_bytes;   // columns stay absolute: the clamp may step left of the tile
+    else tile_b = b + tj0 * ldb_bytes + (int64_t)st_first * C::B_ROW;
+    tile_a = a_values + (ti0 + (int64_t)st_first * n_sparse) * 64;
+    tile_m = a_meta + (ti0 + (int64_t)st_first * STAGE_KB * n_sparse) * 4;
 #pragma unroll
     for (int q = 0; q < C::NB; q++) {
       if constexpr (B_KSTRIDED) {
@@ -491,15 +503,18 @@ spmm_pipe(const uint8_t* __restrict__ a_values, const uint8_t* __restrict__ a_me
 
   // copy q of this wave for stage st into the stage buffer at LDS byte address `dst`
   const uint32_t smem_at = lds_offset(smem);
-  auto issue_one = [&](int q, int st, uint32_t dst) {
-    if (q < C::NB) g2l16(tile_b + (int64_t)st * b_stage_stride, ob[q], dst + B_AT + (wave * C::NB + q) * 1024);
-    else if (q < C::NB + C::NA) g2l16(tile_a + (int64_t)st * a_stage_stride, oa[q - C::NB], dst + (wave * C::NA + q - C::NB) * 1024);
-    else if constexpr (M_DWORD) g2l4(tile_m + (int64_t)st * m_stage_stride, om[q - C::NB - C::NA], dst + M_AT + ((wave - (C::NW - MWAVES)) * MW + q - C::NB - C::NA) * 256);
-    else if (has_meta) g2l16(tile_m + (int64_t)st * m_stage_stride, om[q - C::NB - C::NA], dst + M_AT + ((wave - (C::NW - MWAVES)) * MW + q - C::NB - C::NA) * 1024);
+  auto issue_one = [&](int q, uint32_t dst) {
+    if (q < C::NB) g2l16(tile_b, ob[q], dst + B_AT + (wave * C::NB + q) * 1024);
+    else if (q < C::NB + C::NA) g2l16(tile_a, oa[q - C::NB], dst + (wave * C::NA + q - C::NB) * 1024);
+    else if constexpr (M_DWORD) g2l4(tile_m, om[q - C::NB - C::NA], dst + M_AT + ((wave - (C::NW - MWAVES)) * MW + q - C::NB - C::NA) * 256);
+    else if (has_meta) g2l16(tile_m, om[q - C::NB - C::NA], dst + M_AT + ((wave - (C::NW - MWAVES)) * MW + q - C::NB - C::NA) * 1024);
   };
-  auto issue = [&](int st, uint32_t dst) {
+  // the sources advance a stage behind each stage's copies (formed from a stage number they cost four more scalar instructions)
+  auto next_stage = [&]() { tile_b += b_stage_stride; tile_a += a_stage_stride; tile_m += m_stage_stride; };
+  auto issue = [&](uint32_t dst) {
 #pragma unroll
-    for (int q = 0; q < NCOPY; q++) issue_one(q, st, dst);
+    for (int q = 0; q < NCOPY; q++) issue_one(q, dst);
+    next_stage();
   };
 
   typename mma32<T>::acc_t acc[C::TI][C::TJ];
@@ -585,7 +600,7 @@ spmm_pipe(const uint8_t* __restrict__ a_values, const uint8_t* __restrict__ a_me
   constexpr int PER_SLOT = (NCOPY + 2 * C::TI - 1) / (2 * C::TI);
   // copies of a stage issued during the first of its two steps (the rest during the second)
   constexpr int FIRST_HALF_COPIES = C::NW == 4 ? (NCOPY + 1) / 2 : (C::TI * PER_SLOT < NCOPY ? C::TI * PER_SLOT : NCOPY);
-  auto mma_step = [&](int set, int half, bool copies, int pst, uint32_t dst, bool reads, uint32_t src, int rstep) {
+  auto mma_step = [&](int set, int half, bool copies, uint32_t dst, bool reads, uint32_t src, int rstep) {
     __builtin_amdgcn_sched_barrier(0);
     if constexpr (C::NW == 4) {
       // One wave per SIMD: no other wave fills the matrix pipe while this one issues reads and copies, so they go
@@ -610,7 +625,7 @@ spmm_pipe(const uint8_t* __restrict__ a_values, const uint8_t* __restrict__ a_me
           }
 #pragma unroll
           for (int q = 0; q < NCOPY; q++)
-            if ((q * 2 * SLOTS) / NCOPY == half * SLOTS + n && copies) issue_one(q, pst, dst);
+            if ((q * 2 * SLOTS) / NCOPY == half * SLOTS + n && copies) issue_one(q, dst);
           __builtin_amdgcn_sched_barrier(0);
         }
       }
@@ -641,7 +656,7 @@ spmm_pipe(const uint8_t* __restrict__ a_values, const uint8_t* __restrict__ a_me
 #pragma unroll
       for (int u = 0; u < PER_SLOT; u++) {
         const int q = (half * C::TI + ti) * PER_SLOT + u;
-        if (q < NCOPY && copies) issue_one(q, pst, dst);
+        if (q < NCOPY && copies) issue_one(q, dst);
       }
       __builtin_amdgcn_sched_barrier(0);
     }
@@ -654,8 +669,8 @@ spmm_pipe(const uint8_t* __restrict__ a_values, const uint8_t* __restrict__ a_me
     else wait_copies_and_barrier<NCOPY - MW, true>();
   };
 
-  issue(0, smem_at);
-  if (nstages > 1) issue(1, smem_at + STAGE_BYTES);
+  issue(smem_at);
+  if (nstages > 1) issue(smem_at + STAGE_BYTES);
   uint32_t cur = 0, nxt = STAGE_BYTES, fre = 2 * STAGE_BYTES;   // buffers of stage st, st+1, st+2 (= st-1)
   // PERSIST (nstages >= 4, no k pieces): the workgroup walks its tiles in one pipeline.  The copies of
   // the next tile's first two stages are issued during the last two stages of the current one, into
@@ -682,19 +697,27 @@ spmm_pipe(const uint8_t* __restrict__ a_values, const uint8_t* __restrict__ a_me
     for (int n = 0; n < N_READS; n++) read_one(0, n, cur, 0);
     if (more) {
 #pragma unroll
-      for (int q = 0; q < FIRST_HALF_COPIES; q++) issue_one(q, 2, smem_at + fre);
+      for (int q = 0; q < FIRST_HALF_COPIES; q++) issue_one(q, smem_at + fre);
     }
-    mma_step(0, 1, more, 2, smem_at + fre, true, cur, 1);
+    mma_step(0, 1, more, smem_at + fre, true, cur, 1);
+    if (more) next_stage();
     if (PERSIST && chained) wait_reads_and_barrier();
     else stage_barrier(more);
   }
   // stage st: behind B(st), register set 1 holds the last step of stage st-1
   int st = 1;
-  for (; st + 2 < nstages; st++) {
-    const uint32_t t = cur; cur = nxt; nxt = fre; fre = t;
-    mma_step(1, 0, true, st + 2, smem_at + fre, true, cur, 0);
-    mma_step(0, 1, true, st + 2, smem_at + fre, true, cur, 1);
-    stage_barrier(true);
+  for (int lim = nstages - 2 - rot;; lim = nstages - 2) {          // up to the wrap of the stage order, then the rest
+    for (; st < lim; st++) {
+      const uint32_t t = cur; cur = nxt; nxt = fre; fre = t;
+      mma_step(1, 0, true, smem_at + fre, true, cur, 0);
+      mma_step(0, 1, true, smem_at + fre, true, cur, 1);
+      next_stage();
+      stage_barrier(true);
+    }
+    if (!ROTATE || st >= nstages - 2) break;         // (lim >= 1: the wrap is behind the copies of stage 2)
+    tile_b -= nstages * b_stage_stride;
+    tile_a -= nstages * a_stage_stride;
+    tile_m -= nstages * m_stage_stride;
   }
   if constexpr (PERSIST) {
     next_unit = unit + slots;
@@ -706,9 +729,9 @@ spmm_pipe(const uint8_t* __restrict__ a_values, const uint8_t* __restrict__ a_me
   }
   for (; st < nstages; st++) {                    // the last two stages: nothing left to copy for this tile
     const uint32_t t = cur; cur = nxt; nxt = fre; fre = t;
-    const int pst = st - (nstages - 2);           // stage 0, then 1 of the next tile
-    mma_step(1, 0, has_next, pst, smem_at + fre, true, cur, 0);
-    mma_step(0, 1, has_next, pst, smem_at + fre, true, cur, 1);
+    mma_step(1, 0, has_next, smem_at + fre, true, cur, 0);   // (copies: the first two stages of the next tile)
+    mma_step(0, 1, has_next, smem_at + fre, true, cur, 1);
+    next_stage();
     // behind the last barrier of a tile no wave reads the stage buffers any more; the next tile's
     // copies are not waited for here
     if (st + 1 < nstages) stage_barrier(has_next);
@@ -732,7 +755,7 @@ spmm_pipe(const uint8_t* __restrict__ a_values, const uint8_t* __restrict__ a_me
       bias_w[q] = bias_bits(bias[row < n_sparse ? row : n_sparse - 1]);
     }
   }
-  mma_step(1, 0, false, 0, 0, false, 0, 0);       // the last step
+  mma_step(1, 0, false, 0, false, 0, 0);       // the last step
   if (splits == 1 && bias != nullptr) {
 #pragma unroll
     for (int q = 0; q < C::WI / 64; q++) asm volatile("" : "+v"(bias_w[q]));

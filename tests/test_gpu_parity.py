@@ -1270,3 +1270,26 @@ def test_products_of_views_at_full_multiples(cuda, dtype, pitch, rows, view):
     want = x.float() @ s.to_dense().float().t()
     for got in (torch.mm(at, s.t()), sparse.sparse_semi_structured_linear(at, s), torch.mm(s, at.t()).t()):
         assert got.shape == (rows, 64) and got.float().equal(want.to(got.dtype).float())
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float8_e4m3fn, torch.int8])
+@pytest.mark.parametrize("n,stages,rows", [
+    (4128, 63, 4111),          # four waves, every XCD from the first stage on
+    (4128, 64, 4111),          # from here on each from its own eighth of k: chained tiles of either width
+    (4128, 71, 4111),          # eighths of unequal length
+    (800, 66, 12271),          # one round of 256 x 192 tiles with 16-bit results
+    (4128, 65, 8175)])         # full rounds of 256 x 256 tiles, the last tile row in a second launch
+def test_linear_stage_order_by_xcd(cuda, dtype, n, stages, rows):
+    """Long tiles whose stages start at another eighth of k on each XCD and wrap round: exact on small integers, with
+    32- and 16-bit results (256 x 256 and 256 x 192 tiles), and the same again on a second call."""
+    import sparse
+    k = stages * 128 // torch.empty(0, dtype=dtype).element_size()
+    g = torch.Generator(device=cuda).manual_seed(rows + stages)
+    w = torch.randint(-2, 3, (n, k), device=cuda, generator=g)
+    s = sparse.to_sparse_semi_structured(w.to(torch.int8) if dtype == torch.int8 else w.float(), dtype=dtype)
+    x = torch.randint(-2, 3, (rows, k), device=cuda, generator=g).to(dtype)
+    want = x.float() @ s.to_dense().float().t()
+    for out_dtype in {torch.int8: (torch.int32,), torch.float16: (torch.float16,)}.get(dtype, (torch.float32, torch.bfloat16)):
+        got = sparse.sparse_semi_structured_linear(x, s, out_dtype=out_dtype)
+        assert got.equal(want.to(out_dtype))
+        assert sparse.sparse_semi_structured_linear(x, s, out_dtype=out_dtype).equal(got)
