@@ -54,7 +54,8 @@ int64_t piece_bytes(int64_t n_sparse, int64_t k, int64_t n_dense, bool k_strided
 // for either orientation of the dense operand that the kernels of this operand size take (dispatch_out)
 template <typename T>
 int64_t workspace_bytes(int64_t n_sparse, int64_t k, int64_t n_dense) {
-  const int64_t strided = sizeof(T) == 2 && n_dense % 8 == 0 ? piece_bytes<T, TiledCfg>(n_sparse, k, n_dense, true) : 0;
+  const int64_t strided = sizeof(T) == 2 && n_dense % 8 == 0 ? std::max(piece_bytes<T, TiledCfg>(n_sparse, k, n_dense, true),
+                                                                       piece_bytes<T, SquareCfg>(n_sparse, k, n_dense, true)) : 0;
   if (n_dense <= narrow_columns(n_sparse, k * (int64_t)sizeof(T) / 128)) return strided;
   return std::max(strided, n_dense <= SlimCfg::BJ ? piece_bytes<T, SlimCfg>(n_sparse, k, n_dense, false)
                            : takes_mid<T>(n_sparse, k, n_dense, (int64_t)1 << 40) ? piece_bytes<T, MidCfg>(n_sparse, k, n_dense, false)

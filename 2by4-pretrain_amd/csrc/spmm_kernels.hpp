@@ -244,7 +244,7 @@ spmm_general(const uint8_t* __restrict__ a_values, const uint8_t* __restrict__ a
 // ------------------------------------------------------------------------------------------
 // Tiled kernel: A in the panel layout, B with k contiguous.
 //
-// A block computes a 256(i) x 256(j) tile with V_SMFMAC_F32_32X32X32_{F16,BF16} / 32X32X64_FP8:
+// A block computes a 256(i) x 256(j) tile (or one of the other TileCfgT shapes) with V_SMFMAC_F32_32X32X32_{F16,BF16} / 32X32X64_FP8:
 // 8 waves (2 along i x 4 along j), wave tile 128 x 64 = 4 x 2 instructions, 2 waves per SIMD.
 // (4 waves with 128 x 128 wave tiles and 256 accumulators read less LDS per instruction but were
 // measured slower: with one wave per SIMD nothing covers a wave's own stalls.)
@@ -305,15 +305,16 @@ template <> struct mma32<i8_t> {
   }
 };
 
-template <int WAVES_J_, int TJ_>
+template <int WAVES_J_, int TJ_, int TI_ = 4>
 struct TileCfgT {
   static constexpr int WAVES_I = 2, WAVES_J = WAVES_J_;
   static constexpr int NW = WAVES_I * WAVES_J;
   static constexpr int THREADS = 64 * NW;
-  static constexpr int TI = 4, TJ = TJ_;         // 32x32 instructions per wave
+  static constexpr int TI = TI_, TJ = TJ_;       // 32x32 instructions per wave
   static constexpr int WI = 32 * TI, WJ = 32 * TJ;
   static constexpr int BI = WI * WAVES_I, BJ = WJ * WAVES_J;
-  static_assert(BI == 256 && (BJ == 256 || BJ == 192 || BJ == 128 || BJ == 64), "stage buffers are sized for 256-row tiles of 256, 192, 128 or 64 columns");
+  static_assert((BI == 256 && (BJ == 256 || BJ == 192 || BJ == 128 || BJ == 64)) || (BI == 192 && BJ == 192),
+                "stage buffers are sized for 256-row tiles of 256, 192, 128 or 64 columns and for 192 x 192 tiles");
   static constexpr int KB = 128;                 // bytes of dense k per row per stage
   static constexpr int STEPS = KB / 64;          // instruction steps per stage
   static constexpr int A_ROW = KB / 2;           // LDS bytes per row per stage: compressed values
@@ -338,6 +339,17 @@ using Wave4Cfg = TileCfgT<2, 4>;
 // (W[1600, 6400] against 12288 tokens: 336 wide tiles or 448 narrow ones, two rounds either way, 147 against 165 us;
 // W[11008, 4096] against 2048 tokens alike).  Long chained tiles only, like the 4-wave form itself.
 using Wave4Cfg192 = TileCfgT<2, 3>;
+// 192 x 192 tiles in the 4-wave form (wave tile 96 x 96, 144 accumulators): a stage takes 0.53 us against 0.93 of a
+// 256 x 256 one for 0.5625 of its work, so that they cost next to nothing in rate and rounds of the compute units fill
+// better -- 3072 and 768 rows against 12288 columns are 1024 and 256 of them, four rounds and one.  With a quarter of the
+// accumulators free they also hold the transposing fragment reads of a k-strided dense operand, which the other two
+// 4-wave tiles spill.  us, 256 rows a tile and now, fp16: 3072 x 768 against 12288 columns 51.2 -> 43.8, 6400 x 1600 against 2800
+// 53.3 -> 38.5, 768 x 3072 against 12288 44.3 -> 41.8 (bound by the 75 MB of its dense operand: 34 where they come from the last
+// cache); e4m3 5760 x 2688 against 6023 75.5 -> 62.1; k-strided 3072 x 12288 against 768 columns 50.8 -> 44.2, 768 x 12288 against
+// 3072 57.4 -> 51.4, 3072 x 1024 against 768 16.6 -> 13.1 (40 products of 8 to 253 stages: 14 % less on average).
+// Two stage buffers and two workgroups to a compute unit (76 KB and 256 registers each) instead of three buffers and
+// chained tiles: 39.5 and 40.6 us for the first, 52.0 and 41.8 for the third, 36.2 and 35.9 for the second.
+using SquareCfg = TileCfgT<2, 3, 3>;
 constexpr int kWave4MinStages = 32;
 constexpr int kRotateMinStages = 64;       // (at least 24: the first three stages of a tile are copied before the order wraps)
 // 256 x 64 tiles, two waves: for dense operands of at most 64 columns (a few dozen tokens), where a
@@ -372,12 +384,16 @@ spmm_pipe(const uint8_t* __restrict__ a_values, const uint8_t* __restrict__ a_me
   // workgroup (copied a dword per lane, 16 instructions per stage, the same bytes took a fifth of the fp8
   // kernel's copy time).  With 16-bit values and more waves than runs every wave brings a quarter run (or more)
   // with dword copies instead, so that all waves run the same code: a branch in the loop body makes the compiler
-  // re-mask the 16-bit index words behind it, and that wait for all of a step's reads costs 5 %.
+  // re-mask the 16-bit index words behind it, and that wait for all of a step's reads costs 5 %.  (Runs of 192 rows
+  // are three quarters; where those do not divide among the waves, the last ones are copied twice, with the same bytes.)
   constexpr int STAGE_KB = M_ROW / 4;                        // 1 KB metadata runs per stage
-  constexpr bool M_DWORD = ES == 2 && C::NW > STAGE_KB;      // quarter runs, every wave
+  constexpr bool M_DWORD = (ES == 2 && C::NW > STAGE_KB) || C::BI != 256;   // quarter runs, every wave
   constexpr int MWAVES = M_DWORD ? C::NW : (STAGE_KB < C::NW ? STAGE_KB : C::NW);   // waves that copy metadata
-  constexpr int MW = (M_DWORD ? STAGE_KB * 4 : STAGE_KB) / MWAVES;                  // copies per such wave
-  static_assert(MW * MWAVES == (M_DWORD ? STAGE_KB * 4 : STAGE_KB) && C::BI * 4 == 1024, "metadata copies must divide among the waves");
+  constexpr int QUARTERS = C::BI / 64;                       // of a run
+  constexpr int MCOPIES = M_DWORD ? STAGE_KB * QUARTERS : STAGE_KB;
+  constexpr int MW = (MCOPIES + MWAVES - 1) / MWAVES;        // copies per such wave
+  static_assert(MW * MWAVES == MCOPIES || C::BI != 256, "metadata copies must divide among the waves");
+  static_assert(M_DWORD || C::BI == 256, "full runs are 256 rows");
   constexpr bool M_HALF_MAJOR = ES == 1;
   // one stage buffer = [A values | B | A metadata]; three of them rotate
   constexpr int A_STAGE = C::BI * C::A_ROW, B_STAGE = C::BJ * C::B_ROW, M_STAGE = C::BI * M_ROW;
@@ -452,11 +468,20 @@ spmm_pipe(const uint8_t* __restrict__ a_values, const uint8_t* __restrict__ a_me
   //    (and 256*M_ROW metadata bytes): copy q brings 16 rows x 64 bytes.
   // Every source is (tile base, uniform, advanced by whole stages) + (lane offset inside the tile's first stage).
   uint32_t ob[C::NB], oa[C::NA], om[MW];
+  auto m_copy = [&](int q) {                     // which of the stage's metadata copies is the q-th of this wave
+    const int c = (wave - (C::NW - MWAVES)) * MW + q;
+    return MW * MWAVES == MCOPIES ? c : min(c, MCOPIES - 1);
+  };
   const uint8_t *tile_b, *tile_a, *tile_m;
-  // B with k strided (element (k,j) at k*ldb + j, 16-bit types): the stage is kept as [64 k][256 j]
-  // in LDS, copy q brings 2 k-rows x 512 bytes; 16-byte chunks are XOR-swizzled with
+  // B with k strided (element (k,j) at k*ldb + j, 16-bit types): the stage is kept as [64 k][BJ j]
+  // in LDS, copy q brings 1 KB of it (2 k-rows of 256 columns); 16-byte chunks are XOR-swizzled with
   // ((k & 3) << 1) | ((k >> 3 & 1) << 3) so that the transposing fragment reads below (four k-rows x
-  // 32 bytes per 16 lanes) touch every bank once.  Columns past n_dense re-read the last chunk.
+  // 32 bytes per 16 lanes) touch every bank once.  Rows of 192 columns start half of the banks apart by
+  // themselves, and their 24 chunks go with ((k >> 1 & 1) << 2) | ((k >> 3 & 1) << 1).
+  // Columns past n_dense re-read the last chunk.
+  auto kstrided_swizzle = [](int krow) {
+    return C::BJ == 256 ? ((krow & 3) << 1) | (((krow >> 3) & 1) << 3) : (((krow >> 1) & 1) << 2) | (((krow >> 3) & 1) << 1);
+  };
   constexpr int64_t B_STAGE_ADVANCE_ROWS = B_KSTRIDED ? C::KB / ES : 0;
   const int64_t b_stage_stride = B_KSTRIDED ? B_STAGE_ADVANCE_ROWS * ldb_bytes : (int64_t)C::B_ROW;
   auto point_at = [&](int64_t ti0, int64_t tj0) {              // sources of the first stage of the tile at (ti0, tj0)
@@ -473,8 +498,9 @@ spmm_pipe(const uint8_t* __restrict__ a_values, const uint8_t* __restrict__ a_me
 #pragma unroll
     for (int q = 0; q < C::NB; q++) {
       if constexpr (B_KSTRIDED) {
-        const int krow = (wave * C::NB + q) * 2 + (lane >> 5);
-        const int ch = (lane & 31) ^ (((krow & 3) << 1) | (((krow >> 3) & 1) << 3));
+        constexpr int CHUNKS = C::BJ / 8;        // of a k-row
+        const int piece = (wave * C::NB + q) * 64 + lane, krow = piece / CHUNKS;
+        const int ch = (piece % CHUNKS) ^ kstrided_swizzle(krow);
         const int64_t col = min(tj0 + ch * 8, n_dense - 8);
         ob[q] = (uint32_t)(krow * ldb_bytes + col * ES);
       } else {
@@ -491,8 +517,8 @@ spmm_pipe(const uint8_t* __restrict__ a_values, const uint8_t* __restrict__ a_me
     }
 #pragma unroll
     for (int q = 0; q < MW; q++) {
-      const int c = (wave - (C::NW - MWAVES)) * MW + q;        // quarter run (a lane brings one row's word) or run (4 rows' words)
-      om[q] = M_DWORD ? (uint32_t)(((c >> 2) * n_sparse + min((int64_t)((c & 3) * 64 + lane), last_i)) * 4)
+      const int c = m_copy(q);                                 // quarter run (a lane brings one row's word) or run (4 rows' words)
+      om[q] = M_DWORD ? (uint32_t)(((c / QUARTERS) * n_sparse + min((int64_t)((c % QUARTERS) * 64 + lane), last_i)) * 4)
                       : (uint32_t)((c * n_sparse + min((int64_t)lane * 4, last_i - 3)) * 4);
     }
   };
@@ -506,8 +532,8 @@ spmm_pipe(const uint8_t* __restrict__ a_values, const uint8_t* __restrict__ a_me
   auto issue_one = [&](int q, uint32_t dst) {
     if (q < C::NB) g2l16(tile_b, ob[q], dst + B_AT + (wave * C::NB + q) * 1024);
     else if (q < C::NB + C::NA) g2l16(tile_a, oa[q - C::NB], dst + (wave * C::NA + q - C::NB) * 1024);
-    else if constexpr (M_DWORD) g2l4(tile_m, om[q - C::NB - C::NA], dst + M_AT + ((wave - (C::NW - MWAVES)) * MW + q - C::NB - C::NA) * 256);
-    else if (has_meta) g2l16(tile_m, om[q - C::NB - C::NA], dst + M_AT + ((wave - (C::NW - MWAVES)) * MW + q - C::NB - C::NA) * 1024);
+    else if constexpr (M_DWORD) g2l4(tile_m, om[q - C::NB - C::NA], dst + M_AT + m_copy(q - C::NB - C::NA) * 256);
+    else if (has_meta) g2l16(tile_m, om[q - C::NB - C::NA], dst + M_AT + m_copy(q - C::NB - C::NA) * 1024);
   };
   // the sources advance a stage behind each stage's copies (formed from a stage number they cost four more scalar instructions)
   auto next_stage = [&]() { tile_b += b_stage_stride; tile_a += a_stage_stride; tile_m += m_stage_stride; };
@@ -545,11 +571,11 @@ spmm_pipe(const uint8_t* __restrict__ a_values, const uint8_t* __restrict__ a_me
   if constexpr (B_KSTRIDED) {
     const int g16 = lane >> 4, s16 = lane & 15;
     const int kb = g16 >> 1, jbase = (g16 & 1) * 16;
-    const int swz = ((s16 >> 2) << 1) | (kb << 3);                // (k & 3) << 1 | (k >> 3 & 1) << 3 of the rows read
+    const int swz = kstrided_swizzle(kb * 8 + (s16 >> 2));        // the same for all four rows read
 #pragma unroll
     for (int tj = 0; tj < C::TJ; tj++) {
       const int col = wj * C::WJ + tj * 32 + jbase + (s16 & 3) * 4;  // halfword column in the tile
-      bt_off[tj] = (kb * 8 + (s16 >> 2)) * 512 + (((col >> 3) ^ swz) * 16) + ((col >> 2) & 1) * 8;
+      bt_off[tj] = (kb * 8 + (s16 >> 2)) * (C::BJ * 2) + (((col >> 3) ^ swz) * 16) + ((col >> 2) & 1) * 8;
     }
   }
 
@@ -582,7 +608,7 @@ spmm_pipe(const uint8_t* __restrict__ a_values, const uint8_t* __restrict__ a_me
     if (n < B_READS) {
       if constexpr (B_KSTRIDED) {
         const int tj = n >> 2, quarter = n & 3;                  // quarter: k0 = 8*kb + {0, 4, 16, 20}
-        const uint8_t* src_q = base + B_AT + bt_off[tj] + step * (32 * 512) + ((quarter & 1) * 4 + (quarter >> 1) * 16) * 512;
+        const uint8_t* src_q = base + B_AT + bt_off[tj] + step * (32 * C::BJ * 2) + ((quarter & 1) * 4 + (quarter >> 1) * 16) * (C::BJ * 2);
         bq[set][tj][quarter] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4_ptr)(lds_ptr_t)src_q);
       } else {
         bf[set][n >> 1][n & 1] = *reinterpret_cast<const int4v*>(base + B_AT + b_off[step][n & 1] + (n >> 1) * 32 * C::B_ROW);
@@ -600,6 +626,17 @@ spmm_pipe(const uint8_t* __restrict__ a_values, const uint8_t* __restrict__ a_me
   constexpr int PER_SLOT = (NCOPY + 2 * C::TI - 1) / (2 * C::TI);
   // copies of a stage issued during the first of its two steps (the rest during the second)
   constexpr int FIRST_HALF_COPIES = C::NW == 4 ? (NCOPY + 1) / 2 : (C::TI * PER_SLOT < NCOPY ? C::TI * PER_SLOT : NCOPY);
+  auto dense_fragment = [&](int set, int tj) {
+    if constexpr (B_KSTRIDED) {
+      typedef int int2v __attribute__((ext_vector_type(2)));
+      const int2v q0 = __builtin_bit_cast(int2v, bq[set][tj][0]), q1 = __builtin_bit_cast(int2v, bq[set][tj][1]);
+      const int2v q2 = __builtin_bit_cast(int2v, bq[set][tj][2]), q3 = __builtin_bit_cast(int2v, bq[set][tj][3]);
+      return int8v{q0[0], q0[1], q1[0], q1[1], q2[0], q2[1], q3[0], q3[1]};
+    } else {
+      const int4v lo = bf[set][tj][0], hi = bf[set][tj][1];
+      return int8v{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+    }
+  };
   auto mma_step = [&](int set, int half, bool copies, uint32_t dst, bool reads, uint32_t src, int rstep) {
     __builtin_amdgcn_sched_barrier(0);
     if constexpr (C::NW == 4) {
@@ -608,14 +645,12 @@ spmm_pipe(const uint8_t* __restrict__ a_values, const uint8_t* __restrict__ a_me
       // than the 8-wave form instead of faster).  Ending the reads a few instructions before the step does, so
       // that the stage barrier finds them landed, changes nothing measurable.
       constexpr int SLOTS = C::TI * C::TJ;
-      static_assert(!B_KSTRIDED, "the 4-wave form is built for a k-contiguous dense operand (with the transposing reads it spills)");
+      static_assert(!B_KSTRIDED || C::TI * C::TJ <= 9, "with the transposing reads of a k-strided dense operand wave tiles of 128 x 128 spill");
 #pragma unroll
       for (int ti = 0; ti < C::TI; ti++) {
 #pragma unroll
         for (int tj = 0; tj < C::TJ; tj++) {
-          const int4v lo = bf[set][tj][0], hi = bf[set][tj][1];
-          const int8v bfrag = int8v{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-          acc[ti][tj] = mma32<T>::run(af[set][ti], bfrag, acc[ti][tj], idx[set][ti]);
+          acc[ti][tj] = mma32<T>::run(af[set][ti], dense_fragment(set, tj), acc[ti][tj], idx[set][ti]);
           __builtin_amdgcn_sched_barrier(0);
           const int n = ti * C::TJ + tj;
           if (reads) {
@@ -635,17 +670,7 @@ spmm_pipe(const uint8_t* __restrict__ a_values, const uint8_t* __restrict__ a_me
     for (int ti = 0; ti < C::TI; ti++) {
 #pragma unroll
       for (int tj = 0; tj < C::TJ; tj++) {
-        int8v bfrag;
-        if constexpr (B_KSTRIDED) {
-          typedef int int2v __attribute__((ext_vector_type(2)));
-          const int2v q0 = __builtin_bit_cast(int2v, bq[set][tj][0]), q1 = __builtin_bit_cast(int2v, bq[set][tj][1]);
-          const int2v q2 = __builtin_bit_cast(int2v, bq[set][tj][2]), q3 = __builtin_bit_cast(int2v, bq[set][tj][3]);
-          bfrag = int8v{q0[0], q0[1], q1[0], q1[1], q2[0], q2[1], q3[0], q3[1]};
-        } else {
-          const int4v lo = bf[set][tj][0], hi = bf[set][tj][1];
-          bfrag = int8v{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-        }
-        acc[ti][tj] = mma32<T>::run(af[set][ti], bfrag, acc[ti][tj], idx[set][ti]);
+        acc[ti][tj] = mma32<T>::run(af[set][ti], dense_fragment(set, tj), acc[ti][tj], idx[set][ti]);
       }
       __builtin_amdgcn_sched_barrier(0);
       if (reads) {
@@ -745,12 +770,13 @@ spmm_pipe(const uint8_t* __restrict__ a_values, const uint8_t* __restrict__ a_me
   // The loaded bits are first touched behind that step (the empty asm statements): converted right away, the compiler
   // waits for each load -- and with it for every copy in flight -- before the step's matrix instructions.
   using accs_t = std::remove_reference_t<decltype(acc[0][0][0])>;
-  uint32_t bias_w[C::WI / 64];
+  constexpr int BIAS_Q = (C::WI + 63) / 64;
+  uint32_t bias_w[BIAS_Q];
 #pragma unroll
-  for (int q = 0; q < C::WI / 64; q++) bias_w[q] = 0;
+  for (int q = 0; q < BIAS_Q; q++) bias_w[q] = 0;
   if (splits == 1 && bias != nullptr) {
 #pragma unroll
-    for (int q = 0; q < C::WI / 64; q++) {
+    for (int q = 0; q < BIAS_Q; q++) {
       const int64_t row = i0 + wi * C::WI + q * 64 + (int)(threadIdx.x & 63);
       bias_w[q] = bias_bits(bias[row < n_sparse ? row : n_sparse - 1]);
     }
@@ -758,7 +784,7 @@ spmm_pipe(const uint8_t* __restrict__ a_values, const uint8_t* __restrict__ a_me
   mma_step(1, 0, false, 0, false, 0, 0);       // the last step
   if (splits == 1 && bias != nullptr) {
 #pragma unroll
-    for (int q = 0; q < C::WI / 64; q++) asm volatile("" : "+v"(bias_w[q]));
+    for (int q = 0; q < BIAS_Q; q++) asm volatile("" : "+v"(bias_w[q]));
   }
 
   // ---- split-K: park the 32-bit accumulators in the workspace, in register order (every group of
@@ -780,6 +806,12 @@ spmm_pipe(const uint8_t* __restrict__ a_values, const uint8_t* __restrict__ a_me
     return;
   }
 
+  // 16-bit j-major outputs leave in pieces of 32(j) x 32*PASS_TI(i): 64 i, or the whole 96 of a wave tile of three fragments
+  // (rows of 192 bytes, 208 apart in LDS: 16 rows' chunks of one position lie on different banks)
+  constexpr int PASS_TI = C::TI % 2 == 0 ? 2 : C::TI;
+  constexpr int PITCH = PASS_TI == 2 ? 128 : PASS_TI * 64 + 16;
+  constexpr int SLICE = 32 * PITCH;              // of the staging buffer, per wave
+  static_assert(C::NW * (SLICE + BIAS_Q * 256) <= STAGE_BYTES, "the output pass stages through one stage buffer");
   auto output_pass = [&](auto mode_c) {
     constexpr int MODE = decltype(mode_c)::value;
     int lane = threadIdx.x & 63;
@@ -787,10 +819,10 @@ spmm_pipe(const uint8_t* __restrict__ a_values, const uint8_t* __restrict__ a_me
     const int l32 = lane & 31, lh = lane >> 5;
     // the bias of this wave's WI rows, behind the staging slices of all waves; the wave reads back what its own lanes
     // wrote (LDS accesses of one wave execute in order: no barrier)
-    accs_t* bias_lds = reinterpret_cast<accs_t*>(smem + cur + C::NW * 4096 + wave * (C::WI * 4));
+    accs_t* bias_lds = reinterpret_cast<accs_t*>(smem + cur + C::NW * SLICE + wave * (BIAS_Q * 256));
     if constexpr (MODE != EPI_PLAIN) {
 #pragma unroll
-      for (int q = 0; q < C::WI / 64; q++) {
+      for (int q = 0; q < BIAS_Q; q++) {
         const accs_t v = bias_as(accs_t(0), bias_from_bits<OutT>(bias_w[q]));
         bias_lds[q * 64 + lane] = i0 + wi * C::WI + q * 64 + lane < n_sparse ? v : accs_t(0);
       }
@@ -817,36 +849,36 @@ spmm_pipe(const uint8_t* __restrict__ a_values, const uint8_t* __restrict__ a_me
     // displace operand lines in L2).  LDS accesses of one wave execute in order, so the passes need
     // no barrier between them.
     if constexpr (C_JMAJOR && sizeof(OutT) == 2) {
-      uint8_t* stage = smem + cur + wave * 4096;
-      const int rr = lane >> 3, chr = lane & 7;
+      uint8_t* stage = smem + cur + wave * SLICE;
+      constexpr int CHUNKS = PASS_TI * 4;                       // 16-byte chunks of a row of the piece
+      auto chunk_at = [](int row, int ch) { return row * PITCH + (PASS_TI == 2 ? ch ^ (row & 7) : ch) * 16; };
   #pragma unroll
       for (int tj = 0; tj < C::TJ; tj++) {
   #pragma unroll
-        for (int ip = 0; ip < C::TI / 2; ip++) {                // 64 sparse rows (i) per pass
-          bias4_t bq[2][4];
-          bias_quads(ip * 2, bq[0]);
-          bias_quads(ip * 2 + 1, bq[1]);
+        for (int ip = 0; ip < C::TI / PASS_TI; ip++) {          // 32 * PASS_TI sparse rows (i) per pass
+          bias4_t bq[PASS_TI][4];
   #pragma unroll
-          for (int t2 = 0; t2 < 2; t2++) {
-            const int ti = ip * 2 + t2;
+          for (int t2 = 0; t2 < PASS_TI; t2++) bias_quads(ip * PASS_TI + t2, bq[t2]);
+  #pragma unroll
+          for (int t2 = 0; t2 < PASS_TI; t2++) {
+            const int ti = ip * PASS_TI + t2;
   #pragma unroll
             for (int g = 0; g < 4; g++) {
               OutT o[4];
   #pragma unroll
               for (int r = 0; r < 4; r++) o[r] = to_out<OutT>(finish_element<MODE>(acc[ti][tj][g * 4 + r], scale, bq[t2][g][r]));
-              const int ch = t2 * 4 + g;
-              *reinterpret_cast<Pack<OutT, 4>*>(stage + l32 * 128 + ((ch ^ (l32 & 7)) * 16) + lh * 8) = *reinterpret_cast<Pack<OutT, 4>*>(o);
+              *reinterpret_cast<Pack<OutT, 4>*>(stage + chunk_at(l32, t2 * 4 + g) + lh * 8) = *reinterpret_cast<Pack<OutT, 4>*>(o);
             }
           }
-          const int64_t icol = i0 + wi * C::WI + ip * 64 + chr * 8;
           // the next tile's first two stages (issued one and two stages ago) have to be in LDS before this
           // wave's first store joins the outstanding operations
           if (PERSIST && tj == 0 && ip == 0 && has_next) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   #pragma unroll
-          for (int it = 0; it < 4; it++) {
-            const int jl = it * 8 + rr;
+          for (int it = 0; it < CHUNKS / 2; it++) {
+            const int piece = it * 64 + lane, jl = piece / CHUNKS, ch = piece % CHUNKS;
+            const int64_t icol = i0 + wi * C::WI + ip * (32 * PASS_TI) + ch * 8;
             const int64_t jrow = j0 + wj * C::WJ + tj * 32 + jl;
-            const int4v v = *reinterpret_cast<const int4v*>(stage + jl * 128 + ((chr ^ (jl & 7)) * 16));
+            const int4v v = *reinterpret_cast<const int4v*>(stage + chunk_at(jl, ch));
             if (jrow < n_dense && icol < n_sparse) __builtin_nontemporal_store(v, reinterpret_cast<int4v*>(c + jrow * ldc + icol));
           }
         }
@@ -855,7 +887,7 @@ spmm_pipe(const uint8_t* __restrict__ a_values, const uint8_t* __restrict__ a_me
       // j-major 32-bit output (float32 from 8-bit operands, int32 from int8: the reference's output types for
       // them): the same staging with 32(j) x 32(i) pieces -- a lane's four consecutive i are one 16-byte chunk of
       // a 128-byte row -- so that the stores are full 128-byte row segments instead of 32-byte ones.
-      uint8_t* stage = smem + cur + wave * 4096;
+      uint8_t* stage = smem + cur + wave * SLICE;
       const int rr = lane >> 3, chr = lane & 7;
   #pragma unroll
       for (int tj = 0; tj < C::TJ; tj++) {
@@ -884,11 +916,11 @@ spmm_pipe(const uint8_t* __restrict__ a_values, const uint8_t* __restrict__ a_me
           }
         }
       }
-    } else if constexpr (!C_JMAJOR && sizeof(OutT) == 2) {
+    } else if constexpr (!C_JMAJOR && sizeof(OutT) == 2 && C::TJ % 2 == 0) {
       // i-major 16-bit output (the W.B of `S @ dense`): a lane owns single elements of 64+ different
       // rows.  Stage 32(i) x 64(j) pieces as [i][64 j] (128-byte rows, chunks XOR-swizzled with the
       // row) and stream them out as eight full 128-byte rows per instruction.
-      uint8_t* stage = smem + cur + wave * 4096;
+      uint8_t* stage = smem + cur + wave * SLICE;
       const int rr = lane >> 3, chr = lane & 7;
   #pragma unroll
       for (int half = 0; half < C::TJ / 2; half++) {            // 64 output columns (j) per pass
@@ -1049,6 +1081,7 @@ template <typename C>
 constexpr PieceCost piece_cost(bool k_strided) {
   return std::is_same<C, SlimCfg>::value ? PieceCost{5.1, 0.37, 1.8, 0.0, 0.48, 0.113}
          : std::is_same<C, MidCfg>::value ? PieceCost{5.6, 0.33, 2.1, 0.1, 0.45, 0.0}
+         : std::is_same<C, SquareCfg>::value ? PieceCost{7.3, 0.40, 1.15, 0.0, 0.40, 0.0}
          : k_strided ? PieceCost{7.1, 0.55, 1.15, 0.0, 0.42, 0.0} : PieceCost{6.9, 0.50, 3.3, 0.0, 0.385, 0.0};
 }
 constexpr int64_t kShortStages = 28;
@@ -1085,6 +1118,47 @@ bool takes_mid(int64_t n_sparse, int64_t k, int64_t n_dense, int64_t workspace_b
                                        0.95 * choose_pieces<T, MidCfg>(n_sparse, k, n_dense, workspace_bytes, false).us;
 }
 
+// Rounds of the compute units that so many tiles take (each XCD has an eighth of both).
+inline int64_t tile_rounds(int64_t tiles, int64_t cu_slots) { return ((tiles + 7) / 8 + cu_slots - 1) / cu_slots; }
+
+// Whether a product with 16-bit j-major results and k contiguous, in one piece, takes 192 x 192 tiles: rounds x (us of a tile's
+// stages + its prologue and output pass) against the same of what it would take otherwise -- 256 x 256 tiles (chained, with
+// their last rows on half tiles: tiles_i and tail_rows), or from kWave4MinStages stages on 256 x 192 ones.  The constants are
+// read off timings of 8 to 172 stages and 1 to 4 rounds; of 74 products drawn from 512 x 320 to 11008 x 8704 and 500
+// to 16000 columns (fp16 and e4m3) the choice is 0.4 % off the better one on average and 3 to 7 % for six of them.
+inline int square_stagger_ticks(int64_t rounds, int stages) { return rounds > 1 && stages <= 32 ? 300 : 0; }
+inline bool takes_square(int64_t n_sparse, int64_t n_dense, int stages, int tiles_i, int tail_rows, int cu_slots) {
+  const int64_t tiles_j = (n_dense + TiledCfg::BJ - 1) / TiledCfg::BJ;
+  const int64_t square = ((n_sparse + SquareCfg::BI - 1) / SquareCfg::BI) * ((n_dense + SquareCfg::BJ - 1) / SquareCfg::BJ);
+  const int64_t rounds = tile_rounds(square, cu_slots);
+  const bool four_waves = stages >= kWave4MinStages;
+  double others = (double)tile_rounds(tiles_i * tiles_j, cu_slots) * (four_waves ? 0.93 * stages + 2.5 : 0.88 * stages + 3.8);
+  if (tail_rows) others += 0.5 * stages + 5.0;
+  if (four_waves) {
+    const int64_t narrow = (tiles_i + tail_rows) * ((n_dense + Wave4Cfg192::BJ - 1) / Wave4Cfg192::BJ);
+    others = std::min(others, (double)tile_rounds(narrow, cu_slots) * (0.69 * stages + 2.0));
+  }
+  return (double)rounds * (0.53 * stages + 1.6) + 0.01 * square_stagger_ticks(rounds, stages) < 0.97 * others;
+}
+
+// Whether a product with k strided does: the pieces that either tile would be cut into, estimated as choose_pieces does and
+// with further rounds counted by their stages.  (Few products are not: 6400 x 2816 against 1600 columns, 306 tiles instead of 175,
+// 39.8 us and 45.  Uncut 16-bit results stored i-major would leave in 2-byte stores: the staged pass takes 64 columns.)
+template <typename T, typename OutT>
+bool strided_takes_square(int64_t n_sparse, int64_t k, int64_t n_dense, int64_t workspace_bytes, bool c_jmajor, int cu_slots) {
+  if (cu_slots <= 0) return false;
+  const int64_t stages = k * (int64_t)sizeof(T) / TiledCfg::KB;
+  auto us = [&](auto cfg, Pieces p) {
+    using C = decltype(cfg);
+    const int64_t tiles = ((n_sparse + C::BI - 1) / C::BI) * ((n_dense + C::BJ - 1) / C::BJ);
+    return p.us + (double)((tile_rounds(tiles * p.count, cu_slots) - 1) * ((stages + p.count - 1) / p.count)) * piece_cost<C>(true).stage_us;
+  };
+  const Pieces wide = choose_pieces<T, TiledCfg>(n_sparse, k, n_dense, workspace_bytes, true);
+  const Pieces square = choose_pieces<T, SquareCfg>(n_sparse, k, n_dense, workspace_bytes, true);
+  if (sizeof(OutT) == 2 && !c_jmajor && square.count == 1) return false;
+  return us(SquareCfg{}, square) < 0.97 * us(TiledCfg{}, wide);
+}
+
 // compute units of the current device (looked up once per device; the cache is a table of atomics: two threads
 // that meet on an empty entry both look the value up and store the same number)
 inline int compute_units() {
@@ -1103,10 +1177,17 @@ template <typename T, typename OutT, typename C>
 int launch_tiled(const void* av, const void* am, int64_t n_sparse, int64_t k, const void* b, int b_layout, int64_t ldb,
                  int64_t n_dense, void* c, int c_layout, int64_t ldc, const void* bias, float scale, int act,
                  void* workspace, int64_t workspace_bytes, hipStream_t s) {
+  constexpr bool SQUARE = std::is_same<C, SquareCfg>::value;       // (this way for a k-strided dense operand only)
+  const int cu_slots = compute_units() / 8;
+  if constexpr (std::is_same<C, TiledCfg>::value && sizeof(T) == 2) {
+    if (b_layout == TF24_COL_MAJOR &&
+        strided_takes_square<T, OutT>(n_sparse, k, n_dense, workspace ? workspace_bytes : 0, c_layout == TF24_COL_MAJOR, cu_slots))
+      return launch_tiled<T, OutT, SquareCfg>(av, am, n_sparse, k, b, b_layout, ldb, n_dense, c, c_layout, ldc, bias, scale, act, workspace,
+                                              workspace_bytes, s);
+  }
   int tiles_i = (int)((n_sparse + C::BI - 1) / C::BI);
   const int tiles_j = (int)((n_dense + C::BJ - 1) / C::BJ);
   const int splits = workspace ? choose_pieces<T, C>(n_sparse, k, n_dense, workspace_bytes, b_layout == TF24_COL_MAJOR).count : 1;
-  const int cu_slots = compute_units() / 8;
   // A last round that fills less than half of the compute units: the tile rows that make up the full rounds stay
   // with the chained 256 x 256 tiles, the remaining rows go to a second launch on 256 x 128 tiles, which reach twice
   // as many compute units for half the time each (W[11008, 4096] against 8192 tokens: 1376 tiles = 5 rounds of 256
@@ -1159,6 +1240,19 @@ int launch_tiled(const void* av, const void* am, int64_t n_sparse, int64_t k, co
   if constexpr (std::is_same<C, TiledCfg>::value && sizeof(OutT) == 2) {
     const int tiles_j192 = (int)((n_dense + Wave4Cfg192::BJ - 1) / Wave4Cfg192::BJ);
     const int per_xcd192 = (tiles_i * tiles_j192 + 7) / 8;
+    if (jm && b_layout == TF24_ROW_MAJOR && splits == 1 && k * (int64_t)sizeof(T) / C::KB >= 4 && cu_slots > 0 &&
+        takes_square(n_sparse, n_dense, (int)(k * (int64_t)sizeof(T) / C::KB), tiles_i, tail_rows, cu_slots)) {
+      const int square_i = (int)((n_sparse + SquareCfg::BI - 1) / SquareCfg::BI), square_j = (int)((n_dense + SquareCfg::BJ - 1) / SquareCfg::BJ);
+      const int square_stagger = square_stagger_ticks(tile_rounds((int64_t)square_i * square_j, cu_slots), (int)(k * (int64_t)sizeof(T) / C::KB));
+      auto square = [&](auto acts) {
+        hipLaunchKernelGGL((spmm_pipe<T, OutT, true, SquareCfg, false, true, decltype(acts)::value>), dim3((unsigned)(cu_slots * 8)),
+                           dim3(SquareCfg::THREADS), 0, s, (const uint8_t*)av, (const uint8_t*)am, n_sparse, k, (const uint8_t*)b,
+                           ldb * (int64_t)sizeof(T), n_dense, (OutT*)c, ldc, (const OutT*)bias, scale, act, square_i, square_j, 1,
+                           (float*)nullptr, square_stagger);
+      };
+      if (act == TF24_ACT_NONE) square(std::false_type{}); else square(std::true_type{});
+      return check_launch("tf24_spmm");
+    }
     // Also where both widths fit one round and the narrow tiles spread over more compute units (W[768, 3072] against
     // 12288 tokens: 144 wide tiles or 192 narrow ones, 36.1 -> 34.1 us; W[1024, 4096]: 192 or 256 tiles, 56.2 -> 53.9 us).
     const bool one_round192 = C::BJ == 256 && c_layout == TF24_COL_MAJOR && splits == 1 && b_layout == TF24_ROW_MAJOR &&
@@ -1202,14 +1296,14 @@ int launch_tiled(const void* av, const void* am, int64_t n_sparse, int64_t k, co
     if (act == TF24_ACT_NONE || splits > 1) launch_epi(c_jmajor, b_kstrided, std::false_type{});
     else launch_epi(c_jmajor, b_kstrided, std::true_type{});
   };
-  bool kstrided = false;
+  bool kstrided = SQUARE;
   if constexpr (sizeof(T) == 2 && C::BJ == 256) kstrided = b_layout == TF24_COL_MAJOR;
   if (kstrided) {
-    if constexpr (sizeof(T) == 2 && C::BJ == 256) {
+    if constexpr (sizeof(T) == 2 && (C::BJ == 256 || SQUARE)) {
       if (jm) launch(std::true_type{}, std::true_type{});
       else launch(std::false_type{}, std::true_type{});
     }
-  } else {
+  } else if constexpr (!SQUARE) {
     if (jm) launch(std::true_type{}, std::false_type{});
     else launch(std::false_type{}, std::false_type{});
   }

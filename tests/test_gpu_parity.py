@@ -1293,3 +1293,45 @@ def test_linear_stage_order_by_xcd(cuda, dtype, n, stages, rows):
         got = sparse.sparse_semi_structured_linear(x, s, out_dtype=out_dtype)
         assert got.equal(want.to(out_dtype))
         assert sparse.sparse_semi_structured_linear(x, s, out_dtype=out_dtype).equal(got)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float8_e4m3fn])
+@pytest.mark.parametrize("n,stages,rows", [
+    (736, 4, 12271),           # one round, the shortest tiles; partial ones on either edge
+    (768, 5, 12288),           # 256 full tiles
+    (3040, 5, 6130),           # two rounds, every second workgroup starts late
+    (3040, 33, 6130),          # the same, together
+    (3040, 67, 6130)])         # from another eighth of k on each XCD
+@pytest.mark.parametrize("activation", [None, "relu"])
+def test_linear_square_tiles(cuda, dtype, n, stages, rows, activation):
+    """Products on 192 x 192 tiles, with and without bias: exact on small integers."""
+    import sparse
+    k = stages * 128 // torch.empty(0, dtype=dtype).element_size()
+    g = torch.Generator(device=cuda).manual_seed(rows + stages)
+    s = sparse.to_sparse_semi_structured(torch.randint(-1, 2, (n, k), device=cuda, generator=g).float(), dtype=dtype)
+    x = torch.randint(-1, 2, (rows, k), device=cuda, generator=g).to(dtype)
+    out_dtype = torch.bfloat16 if dtype == torch.float8_e4m3fn else dtype
+    bias = torch.randint(-3, 4, (n,), device=cuda, generator=g).to(out_dtype)
+    want = x.float() @ s.to_dense().float().t()
+    act = torch.relu if activation else (lambda t: t)
+    assert sparse.sparse_semi_structured_linear(x, s, out_dtype=out_dtype, activation=activation).equal(act(want).to(out_dtype))
+    assert sparse.sparse_semi_structured_linear(x, s, bias=bias, out_dtype=out_dtype, activation=activation).equal(act(want + bias.float()).to(out_dtype))
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("n,stages,cols", [
+    (64, 4, 72), (224, 5, 200), (192, 9, 192), (352, 25, 2376), (416, 8, 160),       # one piece, tiles past either edge
+    (992, 40, 392), (544, 117, 120), (3072, 48, 768), (3424, 202, 80)])              # pieces of k
+def test_spmm_square_tiles_k_strided(cuda, dtype, n, stages, cols):
+    """Products with a k-strided dense operand on 192 x 192 tiles, in one and in several pieces: exact on small integers, with
+    float32 and 16-bit results of either order."""
+    import sparse
+    from sparse.semi_structured import _spmm
+    k = stages * 64
+    g = torch.Generator(device=cuda).manual_seed(n + stages)
+    s = sparse.to_sparse_semi_structured(torch.randint(-1, 2, (n, k), device=cuda, generator=g).float(), dtype=dtype)
+    x = torch.randint(-1, 2, (k, cols), device=cuda, generator=g).to(dtype)
+    want = s.to_dense().float() @ x.float()
+    assert _spmm(s, x, True, out_dtype=torch.float32).equal(want)
+    assert torch.mm(s, x).equal(want.to(dtype))
+    assert torch.mm(x.t(), s.t()).equal(want.t().to(dtype))
