@@ -127,6 +127,25 @@ def stream_ptr():
     return torch.cuda.current_stream().cuda_stream
 
 
+def plain_eager():
+    """No transform, mode or tracer stands between a call and its kernels."""
+    return not (torch._C._are_functorch_transforms_active() or torch.autograd.forward_ad._current_level >= 0 or torch.compiler.is_compiling()
+                or torch.jit.is_tracing() or torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack())
+
+
+_PLAIN_KEYS = set()
+
+
+def is_plain(t):
+    """An ordinary strided GPU tensor: what torch dispatches on says that nothing is left to be done to it (a negation or
+    conjugation, names, a batch or a tangent) before a kernel reads its storage."""
+    if not _PLAIN_KEYS:
+        for inference in (False, True):
+            with torch.inference_mode(inference):
+                _PLAIN_KEYS.add(torch._C._dispatch_keys(torch.empty(0, device="cuda")).raw_repr())
+    return type(t) in (torch.Tensor, torch.nn.Parameter) and torch._C._dispatch_keys(t).raw_repr() in _PLAIN_KEYS
+
+
 def layout_of(t):
     """(layout, ld) of a 2-d tensor that is dense in one of its two dimensions, else None."""
     m, k = t.shape

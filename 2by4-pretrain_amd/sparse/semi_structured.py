@@ -26,6 +26,8 @@ import torch
 
 from . import _native as N
 
+_F_LINEAR = torch.nn.functional.linear
+
 __all__ = ["SparseSemiStructuredTensor", "to_sparse_semi_structured", "to_sparse_semi_structured_pair",
            "to_sparse_semi_structured_with_row_sums", "mvue_device_state"]
 
@@ -42,6 +44,7 @@ _DTYPE_TO_SEMI_STRUCTURED_SPARSE_CONFIG = {
 
 
 _FLOAT8 = (torch.float8_e4m3fn, torch.float8_e5m2)
+_SIXTEEN_BIT = (torch.float16, torch.bfloat16)
 _EIGHT_BIT = _FLOAT8 + (torch.int8,)          # 128 dense columns per panel, int32 metadata words
 
 
@@ -306,6 +309,40 @@ def _dense_times_sparse_t(dense2d, sparse, bias=None):
     return _spmm(sparse, padded, False, bias=bias, out_dtype=sparse._out_dtype())[:rows, :]
 
 
+def _linear_no_grad(x, weight, bias):
+    """torch.nn.functional.linear(x, weight, bias) of ordinary tensors where the kernels read x as it lies and the result has its
+    dtype, without the views, the general checks and the layouts of _spmm; None for any other call."""
+    values, meta = weight._store_values, weight._store_meta
+    n, k = weight._store_shape
+    shape, dtype, src = x.shape, x.dtype, x.data_ptr()
+    if (dtype not in _SIXTEEN_BIT or dtype is not values.dtype or dtype is not weight._dtype or weight._store_layout != N.COMPRESSED_PANEL or shape[-1:] != (k,)
+            or 2 * k > 1 << 24 or src % 16 or torch.is_autocast_enabled("cuda")):
+        return None
+    # contiguous by the letter: strides of dimensions of size 1 decide in torch's own route which operators it takes
+    if len(shape) == 3:
+        if x.stride() != (shape[1] * k, k, 1):
+            return None
+    elif len(shape) != 2 or x.stride() != (k, 1):
+        return None
+    rows = x.numel() // k
+    if not rows or (bias is not None and (bias.dtype is not dtype or bias.dim() != 1 or bias.shape[0] != n or not bias.is_contiguous())):
+        return None
+    lib = N.lib()
+    out = torch.empty((*shape[:-1], n), dtype=dtype, device=x.device)
+    code = N.F16 if dtype is torch.float16 else N.BF16
+    ws_key = (dtype, n, k, rows)
+    ws_bytes = _WORKSPACE_BYTES.get(ws_key)
+    if ws_bytes is None:
+        ws_bytes = _WORKSPACE_BYTES[ws_key] = lib.tf24_spmm_workspace_bytes(code, n, k, rows)
+    workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=x.device) if ws_bytes else None
+    rc = lib.tf24_linear(values.data_ptr(), meta.data_ptr(), N.COMPRESSED_PANEL, code, n, k, src, k, rows, out.data_ptr(), code, n,
+                         None if bias is None else bias.data_ptr(), 1.0, N.ACT_NONE, None if workspace is None else workspace.data_ptr(),
+                         ws_bytes, N.stream_ptr())
+    if rc:
+        N.check(rc)
+    return out
+
+
 class SparseSemiStructuredTensor(torch.Tensor):
     """2:4 semi-structured sparse matrix as a wrapper tensor subclass: logically the dense
     [m, k] matrix, physically `sparse_tensor_cutlass` (kept values [m, k/2]) and
@@ -344,9 +381,10 @@ class SparseSemiStructuredTensor(torch.Tensor):
             previous = sparse_tensor_cutlass
         else:
             raise ValueError("All of the tensor arguments are None!")
-        return torch.Tensor._make_wrapper_subclass(
-            cls, original_shape, device=previous.device, dtype=previous.dtype if dtype is None else dtype,
-            layout=previous.layout, requires_grad=False)
+        dtype = previous.dtype if dtype is None else dtype
+        out = torch.Tensor._make_wrapper_subclass(cls, original_shape, device=previous.device, dtype=dtype, layout=previous.layout, requires_grad=False)
+        out._dtype = dtype                           # (as an attribute of the object: `dtype` itself goes by __torch_function__)
+        return out
 
     def __init__(self, original_tensor: Optional[torch.Tensor], original_shape: Optional[torch.Size] = None,
                  compressed_tensor_cusparselt: Optional[torch.Tensor] = None,
@@ -451,6 +489,7 @@ class SparseSemiStructuredTensor(torch.Tensor):
         cls._warn_once()
         out = torch.Tensor._make_wrapper_subclass(cls, shape, device=values.device, dtype=values.dtype, layout=values.layout,
                                                   requires_grad=False)
+        out._dtype = values.dtype
         out._store_values, out._store_meta = values, meta
         out._store_shape, out._store_layout = store_shape, store_layout
         out.original_tensor = None
@@ -463,7 +502,20 @@ class SparseSemiStructuredTensor(torch.Tensor):
         return (f"SparseSemiStructuredTensor(shape={self.shape}, transposed={self.transposed}"
                 f"values={self.values()}metadata={self.indices()})")
 
-    __torch_function__ = torch._C._disabled_torch_function_impl
+    @classmethod
+    def __torch_function__(cls, func, types, args=(), kwargs=None):
+        """torch.nn.functional.linear without gradients goes to the kernels from here.  Through the dispatcher it is two
+        calls of __torch_dispatch__, one of which builds the transposed wrapper: 15.4 us of host time a call, which bounds the
+        products of few tokens (3072 x 768 against 37: 5.7 us on the GPU); from here 10.9, 4.3 of them the launch itself.
+        Everything that torch does on the way (autocast, transforms, modes, tracing) and every other function takes torch's
+        own route."""
+        if func is _F_LINEAR and not kwargs and not torch.is_grad_enabled():
+            x, weight, bias = args if len(args) == 3 else (*args, None)
+            if type(weight) is cls and not weight.transposed and N.plain_eager() and N.is_plain(x) and (bias is None or N.is_plain(bias)):
+                out = _linear_no_grad(x, weight, bias)
+                if out is not None:
+                    return out
+        return torch._C._disabled_torch_function_impl(func, types, args, kwargs or {})
 
     def _clone_view(self, shape, transposed):
         return SparseSemiStructuredTensor._from_storage(
@@ -481,7 +533,7 @@ class SparseSemiStructuredTensor(torch.Tensor):
         return original_tensor
 
     def _out_dtype(self):
-        return self._FP8_OUT_DTYPE if self.dtype in _FLOAT8 else None
+        return self._FP8_OUT_DTYPE if self._dtype in _FLOAT8 else None
 
     @classmethod
     def __torch_dispatch__(cls, func, types, args, kwargs) -> Any:

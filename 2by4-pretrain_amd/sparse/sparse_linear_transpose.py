@@ -37,7 +37,7 @@ class sparse_linear_transpose(autograd.Function):
 
     @staticmethod
     def forward(ctx, input, weight, weight_sparse, weight_sparse_T, bias):
-        compute = weight_sparse.dtype
+        compute = weight_sparse._dtype
         if input.dtype != compute:
             input = input.to(compute)
         if bias is not None and bias.dtype != compute:

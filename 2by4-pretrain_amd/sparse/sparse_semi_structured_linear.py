@@ -73,7 +73,7 @@ def sparse_semi_structured_linear(input: torch.Tensor, weight, meta: Optional[to
     shape = input.shape
     x2d = input.reshape(-1, shape[-1])
     rows = x2d.shape[0]
-    if x2d.dtype == weight.dtype and x2d.shape[1] == weight._store_shape[1]:
+    if x2d.dtype == weight._dtype and x2d.shape[1] == weight._store_shape[1]:
         padded = x2d                     # any number of rows
     else:
         padded = weight._pad_tensor_for_matmul(x2d)

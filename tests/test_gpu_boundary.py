@@ -335,3 +335,49 @@ def test_metadata_words_move_alone(cuda, dtype, m, k):
     assert panel.equal(words.t())
     N.check(N.lib().tf24_repack_to(None, panel.data_ptr(), code, m, k, N.COMPRESSED_PANEL, N.COMPRESSED_CANONICAL, None, back.data_ptr(), N.stream_ptr()))
     assert back.equal(words)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_linear_without_gradients_is_the_dispatched_one(cuda, dtype):
+    """torch.nn.functional.linear under no_grad and inference_mode against the same call through the dispatcher: the same bits
+    for every form of its arguments that either takes, the same refusals."""
+    import sparse
+    g = torch.Generator(device=cuda).manual_seed(0)
+    s = sparse.to_sparse_semi_structured(torch.randn(96, 128, device=cuda, generator=g), dtype=dtype)
+    pieces = sparse.SparseSemiStructuredTensor(None, s.shape, sparse_tensor_cutlass=s.values(), meta_tensor_cutlass=s.indices(), dtype=dtype)
+    x = torch.randn(4, 6, 128, device=cuda, generator=g).to(dtype)
+    b = torch.randn(96, device=cuda, generator=g).to(dtype)
+    flat = torch.randn(6 * 128 + 8, device=cuda, generator=g).to(dtype)
+    inputs = {"2d": x[0], "3d": x, "4d": x.view(2, 2, 6, 128), "one": x[:1, :1], "rows apart": x[:, ::2], "last": x[:, -1], "transposed": x.transpose(0, 1),
+              "expanded": x[:1].expand(3, 6, 128), "column-major": x[0].t().contiguous().t(), "off 16 bytes": flat[4:772].view(6, 128),
+              "negated view": torch._neg_view(x[0]), "none": x[0, :0], "vector": x[0, 0], "parameter": torch.nn.Parameter(x.clone(), requires_grad=False),
+              "float32": x.float(), "wrong k": x[..., :64].contiguous()}
+    biases = {"": None, "bias": b, "parameter": torch.nn.Parameter(b.clone(), requires_grad=False), "float32": b.float(), "strided": b.repeat_interleave(2)[::2],
+              "short": b[:8]}
+    weights = {"": s, "parameter": torch.nn.Parameter(s, requires_grad=False), "pieces": pieces, "transposed": s.t()}
+
+    def outcome(weight, inp, bias):
+        try:
+            return torch.nn.functional.linear(inp, weight, bias)
+        except Exception as e:                       # noqa: BLE001 -- the kind of refusal is what is compared
+            return type(e)
+
+    for wn, weight in weights.items():
+        for xn, inp in inputs.items():
+            for bn, bias in biases.items():
+                with torch.no_grad():
+                    got = outcome(weight, inp, bias)
+                    with torch._C.DisableTorchFunctionSubclass():
+                        want = outcome(weight, inp, bias)
+                if isinstance(want, type):
+                    assert got is want, (wn, xn, bn, got, want)
+                else:
+                    assert got.dtype == want.dtype and got.shape == want.shape and got.equal(want), (wn, xn, bn)
+    with torch.inference_mode():
+        assert torch.nn.functional.linear(x, s, b).equal(torch.nn.functional.linear(x.clone(), s, b))
+    with torch.no_grad(), torch.autocast("cuda", dtype=dtype):
+        got = torch.nn.functional.linear(x.float(), s, b)
+        with torch._C.DisableTorchFunctionSubclass():
+            assert got.equal(torch.nn.functional.linear(x.float(), s, b))
+    with torch.no_grad():
+        assert torch.vmap(lambda v: torch.nn.functional.linear(v, s))(x).equal(torch.nn.functional.linear(x, s))
