@@ -617,11 +617,12 @@ def test_entry_points_under_graph_capture(cuda):
 
 
 @pytest.mark.parametrize("tokens,m,n", [(1, 8, 8), (31, 264, 40), (32, 256, 256), (33, 512, 264), (65, 248, 1000), (96, 256, 8),
-                                        (128, 8, 256), (129, 768, 512), (161, 256, 256), (1000, 3072, 768), (4099, 768, 3072)])
+                                        (128, 8, 256), (129, 768, 512), (161, 256, 256), (1000, 3072, 768), (4099, 768, 3072),
+                                        (33, 192, 192), (65, 200, 384), (65, 4104, 3080), (2308, 240, 456), (3189, 256, 208)])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_grad_weight_kernel(cuda, tokens, m, n, dtype):
     """dY^T x and sum(dY) of the dense layers' kernel, with as many pieces of the token axis as it likes, in one piece, with and
-    without the sums, and from rows with a pitch; columns and tokens that fill no tile or stage.
+    without the sums, and from rows with a pitch; columns and tokens that fill no tile or stage; the last three are products for 256 x 256 tiles, the others for 192 x 192 ones.
     Bound: a float32 sum of `tokens` exact products in any order errs by at most tokens * 2^-23 times the sum of their
     magnitudes, and is rounded once to 11 (8) bits."""
     from sparse import _native as N
