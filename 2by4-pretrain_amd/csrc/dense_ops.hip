@@ -125,11 +125,13 @@ dense_op_col(const T* __restrict__ dense, int64_t ld, int64_t m, int64_t k, cons
 
 // scale * soft threshold of a contiguous float32 matrix, rounded to 16 bits: what a layer in mixed precision multiplies by.
 // One group per lane (16 bytes in, 8 out).  One pass of 6 bytes per element where threshold, product and conversion as
-// three operators move 26: 3072 x 768 19 -> 5.8 us.  The float32 product is formed for dropped elements too (0 * scale).
+// three operators move 26: 3072 x 768 19 -> 5.8 us.  The layer's bias, rounded on the way, spares a launch of 3 to 4 us.  The float32 product is formed for dropped elements too (0 * scale).
 template <typename T>
 __global__ void __launch_bounds__(kThreads)
-soft_threshold_scaled(const float* __restrict__ dense, int64_t groups, const float* __restrict__ scale, float scale_value, T* __restrict__ out) {
+soft_threshold_scaled(const float* __restrict__ dense, int64_t groups, const float* __restrict__ scale, float scale_value, T* __restrict__ out,
+                      const float* __restrict__ bias, int64_t nbias, T* __restrict__ bias_out) {
   const int64_t g = (int64_t)blockIdx.x * kThreads + threadIdx.x;
+  if (g < nbias) bias_out[g] = from_float<T>(bias[g]);           // (no more than there are groups)
   if (g >= groups) return;
   const float s = scale ? *scale : scale_value;
   Pack<float, 4> in;
@@ -188,23 +190,40 @@ extern "C" int tf24_soft_threshold24(const void* dense, int dtype, int layout, i
   return tf24::run<tf24::OP_SOFT>("tf24_soft_threshold24", dense, dtype, layout, ld, m, k, nullptr, 0, sparse_out, mask_out, stream);
 }
 
-extern "C" int tf24_soft_threshold24_scaled(const float* dense, int64_t m, int64_t k, const float* scale, float scale_value, void* out, int out_dtype,
-                                            void* stream) {
-  using namespace tf24;
-  const char* fn = "tf24_soft_threshold24_scaled";
+namespace tf24 {
+namespace {
+int run_scaled(const char* fn, const float* dense, int64_t m, int64_t k, const float* scale, float scale_value, void* out, const float* bias,
+               void* bias_out, int out_dtype, void* stream) {
   if (m <= 0 || k <= 0 || k % 4 || m > 0x7fffffffLL || k > 0x7fffffffLL || m * (k / 4) > (int64_t)0x7fffffff * kThreads)
     return fail(TF24_ERR_SHAPE, "%s: bad shape %lld x %lld (k must be a multiple of 4)", fn, (long long)m, (long long)k);
   if (out_dtype != TF24_F16 && out_dtype != TF24_BF16) return fail(TF24_ERR_DTYPE, "%s: unsupported output dtype %d", fn, out_dtype);
   if (!dense || !out) return fail(TF24_ERR_ARG, "%s: null pointer", fn);
   if (int rc = check_aligned(fn, 16, {dense, out})) return rc;
-  if (int rc = check_aligned(fn, 4, {scale})) return rc;
-  const int64_t groups = m * (k / 4);
-  const dim3 grid((unsigned)((groups + kThreads - 1) / kThreads));
-  if (out_dtype == TF24_F16)
-    hipLaunchKernelGGL(soft_threshold_scaled<f16_t>, grid, dim3(kThreads), 0, (hipStream_t)stream, dense, groups, scale, scale_value, (f16_t*)out);
-  else
-    hipLaunchKernelGGL(soft_threshold_scaled<bf16_t>, grid, dim3(kThreads), 0, (hipStream_t)stream, dense, groups, scale, scale_value, (bf16_t*)out);
+  if (int rc = check_aligned(fn, 4, {scale, bias})) return rc;
+  if (int rc = check_aligned(fn, 2, {bias_out})) return rc;
+  const int64_t groups = m * (k / 4), nbias = bias ? m : 0;
+  auto go = [&](auto t) {
+    using T = decltype(t);
+    hipLaunchKernelGGL(soft_threshold_scaled<T>, dim3((unsigned)((groups + kThreads - 1) / kThreads)), dim3(kThreads), 0, (hipStream_t)stream, dense, groups,
+                       scale, scale_value, (T*)out, bias, nbias, (T*)bias_out);
+  };
+  if (out_dtype == TF24_F16) go(f16_t{}); else go(bf16_t{});
   return check_launch(fn);
+}
+}  // namespace
+}  // namespace tf24
+
+extern "C" int tf24_soft_threshold24_scaled(const float* dense, int64_t m, int64_t k, const float* scale, float scale_value, void* out, int out_dtype,
+                                            void* stream) {
+  return tf24::run_scaled("tf24_soft_threshold24_scaled", dense, m, k, scale, scale_value, out, nullptr, nullptr, out_dtype, stream);
+}
+
+extern "C" int tf24_soft_threshold24_scaled_bias(const float* dense, int64_t m, int64_t k, const float* scale, float scale_value, void* out,
+                                                 const float* bias, void* bias_out, int out_dtype, void* stream) {
+  using namespace tf24;
+  const char* fn = "tf24_soft_threshold24_scaled_bias";
+  if (!bias || !bias_out) return fail(TF24_ERR_ARG, "%s: null pointer", fn);
+  return run_scaled(fn, dense, m, k, scale, scale_value, out, bias, bias_out, out_dtype, stream);
 }
 
 extern "C" int tf24_sparse24_dense(const void* dense, int dtype, int layout, int64_t ld, int64_t m, int64_t k,

@@ -63,6 +63,14 @@ __device__ __forceinline__ float16v mma(bf16_t, short8v a, short8v b, float16v c
 __device__ __forceinline__ float widen(f16_t, short h) { return to_float(f16_t{(uint16_t)h}); }
 __device__ __forceinline__ float widen(bf16_t, short h) { return to_float(bf16_t{(uint16_t)h}); }
 
+// a sum rounded to the operands' type, as it is stored (float32 results hold the same values: a pass of its own that widens
+// them, and one for db, are 5 us each)
+template <typename T, typename OutT>
+__device__ __forceinline__ OutT rounded(float v) {
+  if constexpr (std::is_same<OutT, float>::value) return to_float(from_float<T>(v));
+  else return from_float<T>(v);
+}
+
 struct Piece { int tile_i, tile_j, split; };
 // units are (piece, tile), piece-major, the tiles of a piece column by column; see the kernel for the XCD order
 __device__ __forceinline__ Piece locate(int unit, int tiles_i, int tiles_j) {
@@ -70,11 +78,11 @@ __device__ __forceinline__ Piece locate(int unit, int tiles_i, int tiles_j) {
   return {tile / tiles_j, tile % tiles_j, split};
 }
 
-template <typename T, typename C, bool SUMS>
+template <typename T, typename OutT, typename C, bool SUMS>
 __global__ void __launch_bounds__(C::THREADS)
 grad_weight_pipe(const uint8_t* __restrict__ g, int64_t ldg, const uint8_t* __restrict__ x, int64_t ldx, int64_t tokens,
                  int64_t m, int64_t n, int tiles_i, int tiles_j, int splits, float* __restrict__ partial, float* __restrict__ sums,
-                 T* __restrict__ dw, T* __restrict__ db) {
+                 OutT* __restrict__ dw, OutT* __restrict__ db) {
   __shared__ __attribute__((aligned(1024))) uint8_t smem[kRing * C::STAGE];
   // workgroup ids are dealt to the 8 XCDs round-robin: each XCD takes a run of units, which share operand columns in its L2
   const int nunits = tiles_i * tiles_j * splits, per_xcd = (nunits + 7) / 8;
@@ -242,7 +250,7 @@ grad_weight_pipe(const uint8_t* __restrict__ g, int64_t ldg, const uint8_t* __re
       const int64_t row = i0 + C::fragment_row(wave, h) + l32;
       if (lh == 0) {
         if (splits > 1) sums[(int64_t)at.split * tiles_i * C::TILE + row] = v;
-        else if (row < m) db[row] = from_float<T>(v);
+        else if (row < m) db[row] = rounded<T, OutT>(v);
       }
     }
   }
@@ -261,23 +269,23 @@ grad_weight_pipe(const uint8_t* __restrict__ g, int64_t ldg, const uint8_t* __re
     const int64_t row = i0 + C::fragment_row(wave, s / (4 * C::TJ)) + (s & 3) * 8 + lh * 4, col = j0 + (wj * C::TJ + (s >> 2) % C::TJ) * 32 + l32;
     if (row < m && col < n) {
 #pragma unroll
-      for (int r = 0; r < 4; r++) dw[(row + r) * n + col] = from_float<T>(acc[s / (4 * C::TJ)][(s >> 2) % C::TJ][(s & 3) * 4 + r]);
+      for (int r = 0; r < 4; r++) dw[(row + r) * n + col] = rounded<T, OutT>(acc[s / (4 * C::TJ)][(s >> 2) % C::TJ][(s & 3) * 4 + r]);
     }
     __builtin_amdgcn_sched_barrier(0);
   }
 }
 
 // dW and db from the pieces: block (tile, slab), and with blockIdx.x one past the tiles the sums of the columns
-template <typename T, typename C>
+template <typename T, typename OutT, typename C>
 __global__ void __launch_bounds__(C::THREADS)
 grad_weight_reduce(const float* __restrict__ partial, const float* __restrict__ sums, int splits, int64_t m, int64_t n, int tiles_i, int tiles_j,
-                   T* __restrict__ dw, T* __restrict__ db) {
+                   OutT* __restrict__ dw, OutT* __restrict__ db) {
   const int ntiles = tiles_i * tiles_j, tid = threadIdx.x;
   if ((int)blockIdx.x == ntiles) {
     for (int64_t i = (int64_t)blockIdx.y * C::THREADS + tid; i < m; i += (int64_t)gridDim.y * C::THREADS) {
       float v = 0.0f;
       for (int p = 0; p < splits; p++) v += sums[(int64_t)p * tiles_i * C::TILE + i];
-      db[i] = from_float<T>(v);
+      db[i] = rounded<T, OutT>(v);
     }
     return;
   }
@@ -298,7 +306,7 @@ grad_weight_reduce(const float* __restrict__ partial, const float* __restrict__ 
       if (p0 + u < splits) v += part[u];
   }
 #pragma unroll
-  for (int r = 0; r < 4; r++) dw[(row + r) * n + col] = from_float<T>(v[r]);
+  for (int r = 0; r < 4; r++) dw[(row + r) * n + col] = rounded<T, OutT>(v[r]);
 }
 
 template <typename C>
@@ -331,7 +339,7 @@ bool takes_square(int64_t tokens, int64_t m, int64_t n, int64_t workspace_bytes)
   return choose_pieces<Square>(tokens, m, n, workspace_bytes).us < 0.97 * choose_pieces<Wide>(tokens, m, n, workspace_bytes).us;
 }
 
-template <typename T, typename C>
+template <typename T, typename OutT, typename C>
 int launch(const void* g, int64_t ldg, const void* x, int64_t ldx, int64_t tokens, int64_t m, int64_t n, void* dw, void* db,
            void* workspace, int64_t workspace_bytes, hipStream_t s) {
   const int tiles_i = (int)((m + C::TILE - 1) / C::TILE), tiles_j = (int)((n + C::TILE - 1) / C::TILE);
@@ -340,20 +348,20 @@ int launch(const void* g, int64_t ldg, const void* x, int64_t ldx, int64_t token
   float* sums = pieces > 1 ? partial + (int64_t)pieces * tiles_i * tiles_j * C::TILE * C::TILE : nullptr;     // behind the partial tiles
   const int per_xcd = (tiles_i * tiles_j * pieces + 7) / 8;
   auto pipe = [&](auto with_sums) {
-    hipLaunchKernelGGL((grad_weight_pipe<T, C, decltype(with_sums)::value>), dim3((unsigned)(per_xcd * 8)), dim3(C::THREADS), 0, s, (const uint8_t*)g, ldg * 2,
-                       (const uint8_t*)x, ldx * 2, tokens, m, n, tiles_i, tiles_j, pieces, partial, sums, (T*)dw, (T*)db);
+    hipLaunchKernelGGL((grad_weight_pipe<T, OutT, C, decltype(with_sums)::value>), dim3((unsigned)(per_xcd * 8)), dim3(C::THREADS), 0, s, (const uint8_t*)g, ldg * 2,
+                       (const uint8_t*)x, ldx * 2, tokens, m, n, tiles_i, tiles_j, pieces, partial, sums, (OutT*)dw, (OutT*)db);
   };
   if (db) pipe(std::true_type{}); else pipe(std::false_type{});
   if (pieces > 1)
-    hipLaunchKernelGGL((grad_weight_reduce<T, C>), dim3((unsigned)(tiles_i * tiles_j + (db ? 1 : 0)), C::SLABS), dim3(C::THREADS), 0, s, partial, sums, pieces, m, n,
-                       tiles_i, tiles_j, (T*)dw, (T*)db);
+    hipLaunchKernelGGL((grad_weight_reduce<T, OutT, C>), dim3((unsigned)(tiles_i * tiles_j + (db ? 1 : 0)), C::SLABS), dim3(C::THREADS), 0, s, partial, sums, pieces, m, n,
+                       tiles_i, tiles_j, (OutT*)dw, (OutT*)db);
   return check_launch("tf24_grad_weight");
 }
 
-template <typename T>
+template <typename T, typename OutT>
 int launch_either(const void* g, int64_t ldg, const void* x, int64_t ldx, int64_t tokens, int64_t m, int64_t n, void* dw, void* db,
                   void* workspace, int64_t workspace_bytes, hipStream_t s) {
-  auto* go = takes_square(tokens, m, n, workspace ? workspace_bytes : 0) ? launch<T, Square> : launch<T, Wide>;
+  auto* go = takes_square(tokens, m, n, workspace ? workspace_bytes : 0) ? launch<T, OutT, Square> : launch<T, OutT, Wide>;
   return go(g, ldg, x, ldx, tokens, m, n, dw, db, workspace, workspace_bytes, s);
 }
 
@@ -372,10 +380,10 @@ extern "C" int64_t tf24_grad_weight_workspace_bytes(int64_t tokens, int64_t m, i
   return takes_square(tokens, m, n, (int64_t)1 << 40) ? bytes_wanted<Square>(tokens, m, n) : bytes_wanted<Wide>(tokens, m, n);
 }
 
-extern "C" int tf24_grad_weight(const void* g, int64_t ldg, const void* x, int64_t ldx, int dtype, int64_t tokens, int64_t m, int64_t n,
-                                void* dw, void* db, void* workspace, int64_t workspace_bytes, void* stream) {
-  using namespace tf24;
-  const char* fn = "tf24_grad_weight";
+namespace tf24 {
+namespace {
+int run(const char* fn, bool f32, const void* g, int64_t ldg, const void* x, int64_t ldx, int dtype, int64_t tokens, int64_t m, int64_t n,
+        void* dw, void* db, void* workspace, int64_t workspace_bytes, void* stream) {
   if (dtype != TF24_F16 && dtype != TF24_BF16) return fail(TF24_ERR_DTYPE, "%s: unsupported dtype %d", fn, dtype);
   if (tokens <= 0 || tokens > 0x7fffffffLL) return fail(TF24_ERR_SHAPE, "%s: bad number of tokens %lld", fn, (long long)tokens);
   if (m <= 0 || m % 8 || n <= 0 || n % 8 || m > (1 << 20) || n > (1 << 20))
@@ -386,8 +394,21 @@ extern "C" int tf24_grad_weight(const void* g, int64_t ldg, const void* x, int64
   if (!g || !x || !dw) return fail(TF24_ERR_ARG, "%s: null pointer", fn);
   if (workspace_bytes < 0) return fail(TF24_ERR_ARG, "%s: negative workspace size", fn);
   if (int rc = check_aligned(fn, 16, {g, x, workspace})) return rc;
-  if (int rc = check_aligned(fn, 2, {dw, db})) return rc;
+  if (int rc = check_aligned(fn, f32 ? 4 : 2, {dw, db})) return rc;
   hipStream_t s = (hipStream_t)stream;
-  if (dtype == TF24_F16) return launch_either<f16_t>(g, ldg, x, ldx, tokens, m, n, dw, db, workspace, workspace_bytes, s);
-  return launch_either<bf16_t>(g, ldg, x, ldx, tokens, m, n, dw, db, workspace, workspace_bytes, s);
+  auto* go = dtype == TF24_F16 ? (f32 ? launch_either<f16_t, float> : launch_either<f16_t, f16_t>)
+                               : (f32 ? launch_either<bf16_t, float> : launch_either<bf16_t, bf16_t>);
+  return go(g, ldg, x, ldx, tokens, m, n, dw, db, workspace, workspace_bytes, s);
+}
+}  // namespace
+}  // namespace tf24
+
+extern "C" int tf24_grad_weight(const void* g, int64_t ldg, const void* x, int64_t ldx, int dtype, int64_t tokens, int64_t m, int64_t n,
+                                void* dw, void* db, void* workspace, int64_t workspace_bytes, void* stream) {
+  return tf24::run("tf24_grad_weight", false, g, ldg, x, ldx, dtype, tokens, m, n, dw, db, workspace, workspace_bytes, stream);
+}
+
+extern "C" int tf24_grad_weight_f32(const void* g, int64_t ldg, const void* x, int64_t ldx, int dtype, int64_t tokens, int64_t m, int64_t n,
+                                    float* dw, float* db, void* workspace, int64_t workspace_bytes, void* stream) {
+  return tf24::run("tf24_grad_weight_f32", true, g, ldg, x, ldx, dtype, tokens, m, n, dw, db, workspace, workspace_bytes, stream);
 }

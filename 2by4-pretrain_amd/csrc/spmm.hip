@@ -74,13 +74,15 @@ namespace {
 int run_spmm(const char* fn, const void* a_values, const void* a_meta, int a_layout, int dtype, int64_t n_sparse, int64_t k,
              const void* b, int b_layout, int64_t ldb, int64_t n_dense, int64_t extent, void* c, int out_dtype, int c_layout, int64_t ldc,
              const void* bias, float scale, int activation, void* workspace, int64_t workspace_bytes, void* stream) {
-  int rc = validate(fn, dtype, n_sparse, k, b_layout, ldb, n_dense, extent, out_dtype, c_layout, ldc, activation);
+  const int bias_f32 = activation & TF24_BIAS_F32;
+  int rc = validate(fn, dtype, n_sparse, k, b_layout, ldb, n_dense, extent, out_dtype, c_layout, ldc, activation & ~TF24_BIAS_F32);
   if (rc) return rc;
+  if (bias_f32 && out_dtype == TF24_I32) return fail(TF24_ERR_ARG, "%s: integer results take an integer bias", fn);
   if (!a_values || !a_meta || !b || !c) return fail(TF24_ERR_ARG, "%s: null pointer", fn);
   if ((rc = check_aligned(fn, 16, {a_values, b, c, workspace}))) return rc;
   // panel metadata is copied 16 bytes per lane; canonical metadata is read in words of up to 4 bytes, row pitch k/8
   if ((rc = check_aligned(fn, a_layout == TF24_COMPRESSED_PANEL ? 16 : a_layout == TF24_COMPRESSED_CUTLASS ? 4 : 8, {a_meta}))) return rc;
-  if ((rc = check_aligned(fn, dtype_size(out_dtype), {bias}))) return rc;
+  if ((rc = check_aligned(fn, bias_f32 ? 4 : dtype_size(out_dtype), {bias}))) return rc;
   if (a_layout != TF24_COMPRESSED_CANONICAL && a_layout != TF24_COMPRESSED_PANEL && a_layout != TF24_COMPRESSED_CUTLASS)
     return fail(TF24_ERR_ARG, "%s: bad compressed layout %d", fn, a_layout);
   hipStream_t s = (hipStream_t)stream;

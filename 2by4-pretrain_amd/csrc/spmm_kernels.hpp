@@ -93,6 +93,7 @@ __device__ __forceinline__ float gelu_erf(float v) {
 }
 
 __device__ __forceinline__ float apply_act(float v, int act) {
+  act &= ~TF24_BIAS_F32;
   if (act == TF24_ACT_RELU) return v > 0.0f ? v : 0.0f;
   if (act == TF24_ACT_SILU) return v / (1.0f + __expf(-v));
   if (act == TF24_ACT_GELU) return gelu_erf(v);
@@ -106,7 +107,10 @@ template <typename OutT> __device__ __forceinline__ OutT to_out(int v) { return 
 template <typename OutT>
 __device__ __forceinline__ float finish_value(float accv, float scale, const OutT* bias, int64_t row, int act) {
   float v = accv * scale;
-  if (bias) v += to_float(bias[row]);
+  if (bias) {
+    if (sizeof(OutT) == 2 && (act & TF24_BIAS_F32)) v += to_float(from_float<OutT>(reinterpret_cast<const float*>(bias)[row]));
+    else v += to_float(bias[row]);
+  }
   return apply_act(v, act);
 }
 template <typename OutT>
@@ -771,6 +775,7 @@ spmm_pipe(const uint8_t* __restrict__ a_values, const uint8_t* __restrict__ a_me
   // waits for each load -- and with it for every copy in flight -- before the step's matrix instructions.
   using accs_t = std::remove_reference_t<decltype(acc[0][0][0])>;
   constexpr int BIAS_Q = (C::WI + 63) / 64;
+  const bool bias_f32 = sizeof(OutT) == 2 && (act & TF24_BIAS_F32);
   uint32_t bias_w[BIAS_Q];
 #pragma unroll
   for (int q = 0; q < BIAS_Q; q++) bias_w[q] = 0;
@@ -778,7 +783,9 @@ spmm_pipe(const uint8_t* __restrict__ a_values, const uint8_t* __restrict__ a_me
 #pragma unroll
     for (int q = 0; q < BIAS_Q; q++) {
       const int64_t row = i0 + wi * C::WI + q * 64 + (int)(threadIdx.x & 63);
-      bias_w[q] = bias_bits(bias[row < n_sparse ? row : n_sparse - 1]);
+      const int64_t at = row < n_sparse ? row : n_sparse - 1;
+      if (bias_f32) bias_w[q] = reinterpret_cast<const uint32_t*>(bias)[at];      // (rounded where it is unpacked)
+      else bias_w[q] = bias_bits(bias[at]);
     }
   }
   mma_step(1, 0, false, 0, false, 0, 0);       // the last step
@@ -823,7 +830,10 @@ spmm_pipe(const uint8_t* __restrict__ a_values, const uint8_t* __restrict__ a_me
     if constexpr (MODE != EPI_PLAIN) {
 #pragma unroll
       for (int q = 0; q < BIAS_Q; q++) {
-        const accs_t v = bias_as(accs_t(0), bias_from_bits<OutT>(bias_w[q]));
+        uint32_t w = bias_w[q];
+        if constexpr (sizeof(OutT) == 2)
+          if (bias_f32) w = bias_bits(from_float<OutT>(__builtin_bit_cast(float, w)));
+        const accs_t v = bias_as(accs_t(0), bias_from_bits<OutT>(w));
         bias_lds[q * 64 + lane] = i0 + wi * C::WI + q * 64 + lane < n_sparse ? v : accs_t(0);
       }
     }
@@ -983,11 +993,11 @@ spmm_pipe(const uint8_t* __restrict__ a_values, const uint8_t* __restrict__ a_me
     if (!bias) output_pass(std::integral_constant<int, EPI_PLAIN>{});
     else output_pass(std::integral_constant<int, EPI_BIAS>{});
   } else if constexpr (INT_ACC) {
-    if (act == TF24_ACT_RELU) output_pass(std::integral_constant<int, EPI_RELU>{});
+    if ((act & ~TF24_BIAS_F32) == TF24_ACT_RELU) output_pass(std::integral_constant<int, EPI_RELU>{});
     else output_pass(std::integral_constant<int, EPI_BIAS>{});
   } else {
-    if (act == TF24_ACT_RELU) output_pass(std::integral_constant<int, EPI_RELU>{});
-    else if (act == TF24_ACT_SILU) output_pass(std::integral_constant<int, EPI_SILU>{});
+    if ((act & ~TF24_BIAS_F32) == TF24_ACT_RELU) output_pass(std::integral_constant<int, EPI_RELU>{});
+    else if ((act & ~TF24_BIAS_F32) == TF24_ACT_SILU) output_pass(std::integral_constant<int, EPI_SILU>{});
     else output_pass(std::integral_constant<int, EPI_GELU>{});
   }
   if (!has_next) break;
@@ -1233,7 +1243,7 @@ int launch_tiled(const void* av, const void* am, int64_t n_sparse, int64_t k, co
                              (const uint8_t*)av, (const uint8_t*)am, n_sparse, k, (const uint8_t*)b, ldb * (int64_t)sizeof(T), n_dense,
                              (OutT*)c, ldc, (const OutT*)bias, scale, act, tail_rows, tj, 1, (float*)nullptr, tiles_i);
         };
-        if (act == TF24_ACT_NONE) tail(std::false_type{}); else tail(std::true_type{});
+        if ((act & ~TF24_BIAS_F32) == TF24_ACT_NONE) tail(std::false_type{}); else tail(std::true_type{});
       }
     }
   };
@@ -1250,7 +1260,7 @@ int launch_tiled(const void* av, const void* am, int64_t n_sparse, int64_t k, co
                            ldb * (int64_t)sizeof(T), n_dense, (OutT*)c, ldc, (const OutT*)bias, scale, act, square_i, square_j, 1,
                            (float*)nullptr, square_stagger);
       };
-      if (act == TF24_ACT_NONE) square(std::false_type{}); else square(std::true_type{});
+      if ((act & ~TF24_BIAS_F32) == TF24_ACT_NONE) square(std::false_type{}); else square(std::true_type{});
       return check_launch("tf24_spmm");
     }
     // Also where both widths fit one round and the narrow tiles spread over more compute units (W[768, 3072] against
@@ -1264,7 +1274,7 @@ int launch_tiled(const void* av, const void* am, int64_t n_sparse, int64_t k, co
                            (const uint8_t*)av, (const uint8_t*)am, n_sparse, k, (const uint8_t*)b, ldb * (int64_t)sizeof(T), n_dense,
                            (OutT*)c, ldc, (const OutT*)bias, scale, act, tiles_i, tiles_j192, splits, (float*)workspace, stagger);
       };
-      if (act == TF24_ACT_NONE) narrow(std::false_type{}); else narrow(std::true_type{});
+      if ((act & ~TF24_BIAS_F32) == TF24_ACT_NONE) narrow(std::false_type{}); else narrow(std::true_type{});
       launch_tail();
       return check_launch("tf24_spmm");
     }
@@ -1293,7 +1303,7 @@ int launch_tiled(const void* av, const void* am, int64_t n_sparse, int64_t k, co
   };
   auto launch = [&](auto c_jmajor, auto b_kstrided) {
     // with k pieces the reduction kernel applies bias and activation, not this one
-    if (act == TF24_ACT_NONE || splits > 1) launch_epi(c_jmajor, b_kstrided, std::false_type{});
+    if ((act & ~TF24_BIAS_F32) == TF24_ACT_NONE || splits > 1) launch_epi(c_jmajor, b_kstrided, std::false_type{});
     else launch_epi(c_jmajor, b_kstrided, std::true_type{});
   };
   bool kstrided = SQUARE;

@@ -16,6 +16,7 @@ F32, F16, BF16, E4M3, U8, E5M2, I8, I32 = 0, 1, 2, 3, 4, 5, 6, 7
 ROW_MAJOR, COL_MAJOR = 0, 1
 PRUNE_MAGNITUDE, PRUNE_MASK, PRUNE_MVUE, PRUNE_MVUE_PACKED, PRUNE_MVUE_SEEDED, PRUNE_MVUE_SEEDED_DEVICE = 0, 1, 2, 3, 4, 5
 ACT_NONE, ACT_RELU, ACT_SILU, ACT_GELU = 0, 1, 2, 3
+BIAS_F32 = 0x100                                   # or-ed to the activation of a product
 COMPRESSED_CANONICAL, COMPRESSED_PANEL, COMPRESSED_CUTLASS = 0, 1, 2
 
 _DTYPES = {
@@ -48,6 +49,7 @@ _SIGNATURES = {
     "tf24_transposable_mask_validate": (_i, [_i, _i, _i64, _i64, _i64]),
     "tf24_soft_threshold24": (_i, [_p, _i, _i, _i64, _i64, _i64, _p, _p, _p]),
     "tf24_soft_threshold24_scaled": (_i, [_p, _i64, _i64, _p, _f, _p, _i, _p]),
+    "tf24_soft_threshold24_scaled_bias": (_i, [_p, _i64, _i64, _p, _f, _p, _p, _p, _i, _p]),
     "tf24_sparse24_dense": (_i, [_p, _i, _i, _i64, _i64, _i64, _p, _p, _p]),
     "tf24_mvue24_dense": (_i, [_p, _i, _i, _i64, _i64, _i64, _p, _i64, _p, _p]),
     "tf24_masked_add": (_i, [_p, _i, _p, _i, _p, _i, _i64, _f, _p]),
@@ -62,6 +64,7 @@ _SIGNATURES = {
     "tf24_linear": (_i, [_p, _p, _i, _i, _i64, _i64, _p, _i64, _i64, _p, _i, _i64, _p, _f, _i, _p, _i64, _p]),
     "tf24_spmm_workspace_bytes": (_i64, [_i, _i64, _i64, _i64]),
     "tf24_grad_weight": (_i, [_p, _i64, _p, _i64, _i, _i64, _i64, _i64, _p, _p, _p, _i64, _p]),
+    "tf24_grad_weight_f32": (_i, [_p, _i64, _p, _i64, _i, _i64, _i64, _i64, _p, _p, _p, _i64, _p]),
     "tf24_grad_weight_workspace_bytes": (_i64, [_i64, _i64, _i64]),
     "tf24_transpose": (_i, [_p, _i, _i64, _i64, _i64, _p, _i64, _p]),
     "tf24_spmm_validate": (_i, [_i, _i64, _i64, _i, _i64, _i64, _i, _i, _i64, _i]),

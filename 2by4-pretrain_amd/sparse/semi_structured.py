@@ -130,7 +130,7 @@ def _next_philox_state(device):
 def _compress(original, dtype, MVUE24, mask, rand, panel, row_sums=False):
     """One allocation of numel*cf/16 elements: values first, metadata in the tail
     (reference :215-243); then the HIP prune+compress kernel.  Returns flat storage views; with
-    `row_sums` (column-major input only) also original.sum(1), taken from the same read."""
+    `row_sums` (column-major input only; True, or the dtype wanted) also original.sum(1), taken from the same read."""
     m, n = original.shape
     cfg = _DTYPE_TO_SEMI_STRUCTURED_SPARSE_CONFIG[dtype]
     buf = torch.empty((original.nelement() * cfg.compression_factor // 16,), dtype=dtype, device=original.device)
@@ -180,7 +180,7 @@ def _compress(original, dtype, MVUE24, mask, rand, panel, row_sums=False):
             rand_t = N.as_matrix(rand.float(), like=dense)
             rand_ld = N.layout_of(rand_t)[1]
     if row_sums:
-        sums = torch.empty((m,), dtype=dense.dtype, device=dense.device)
+        sums = torch.empty((m,), dtype=dense.dtype if row_sums is True else row_sums, device=dense.device)
         ws_bytes = N.lib().tf24_prune_compress_rowsum_workspace_bytes(m, n)
         workspace = torch.empty((ws_bytes // 4,), dtype=torch.float32, device=dense.device)
         N.check(N.lib().tf24_prune_compress_rowsum(
@@ -274,7 +274,9 @@ def _spmm(sparse, dense, sparse_first, bias=None, out_dtype=None, scale=1.0, act
     device = dense.device
     out = torch.empty(out_shape, dtype=out_dtype, device=device)
     if bias is not None:
-        if bias.dtype != out_dtype or not bias.is_contiguous():
+        if bias.dtype is torch.float32 and out_dtype in _SIXTEEN_BIT and bias.is_contiguous():
+            activation |= N.BIAS_F32                 # rounded where it is read
+        elif bias.dtype != out_dtype or not bias.is_contiguous():
             bias = bias.to(out_dtype).contiguous()
         if bias.numel() != n:
             raise RuntimeError(f"bias must have {n} elements, got {bias.numel()}")
@@ -657,13 +659,13 @@ def to_sparse_semi_structured_pair(original_tensor: torch.Tensor, mask: torch.Te
 
 def to_sparse_semi_structured_with_row_sums(original_tensor: torch.Tensor, MVUE24: bool = False,
                                             mask: Optional[torch.Tensor] = None, dtype: torch.dtype = torch.float16,
-                                            rand: Optional[torch.Tensor] = None):
+                                            rand: Optional[torch.Tensor] = None, sums_dtype: Optional[torch.dtype] = None):
     """(to_sparse_semi_structured(t, MVUE24=..., mask=..., dtype=..., rand=...), t.sum(1)).
 
     For a column-major `t` (the `grad_output.t()` of the training layer's backward, README.md:190-197,
     where the row sums are the bias gradient `grad_output.sum(0)`) both results come from one pass over
-    `t`; the sums are added in float32 and rounded once to t's dtype.  Any other input runs the
-    conversion and torch's sum separately."""
+    `t`; the sums are added in float32 and rounded once to t's dtype (`sums_dtype` float32: not at all).  Any
+    other input runs the conversion and torch's sum separately."""
     t = original_tensor
     cfg = _DTYPE_TO_SEMI_STRUCTURED_SPARSE_CONFIG.get(dtype)
     fusable = (t.is_cuda and t.dim() == 2 and cfg is not None and t.dtype in (torch.float32, torch.float16, torch.bfloat16)
@@ -675,6 +677,6 @@ def to_sparse_semi_structured_with_row_sums(original_tensor: torch.Tensor, MVUE2
                    and n % cfg.sparse_min_cols == 0 and lay is not None and lay[0] == N.COL_MAJOR and lay[1] % 8 == 0
                    and t.data_ptr() % 16 == 0 and t.stride(0) == 1)
     if not fusable:
-        return (to_sparse_semi_structured(t, MVUE24=MVUE24, mask=mask, dtype=dtype, rand=rand), t.sum(1))
-    values, meta, sums = _compress(t, dtype, MVUE24, mask, rand, True, row_sums=True)
+        return (to_sparse_semi_structured(t, MVUE24=MVUE24, mask=mask, dtype=dtype, rand=rand), t.sum(1, dtype=sums_dtype))
+    values, meta, sums = _compress(t, dtype, MVUE24, mask, rand, True, row_sums=sums_dtype or True)
     return SparseSemiStructuredTensor._from_storage(values, meta, (m, n), N.COMPRESSED_PANEL, torch.Size((m, n)), False), sums

@@ -40,9 +40,12 @@ class sparse_linear_transpose(autograd.Function):
         compute = weight_sparse._dtype
         if input.dtype != compute:
             input = input.to(compute)
-        if bias is not None and bias.dtype != compute:
+        # a float32 bias goes to the product as it is, which rounds it to `compute` where it reads it, and gets a float32 gradient
+        # (a cast either way is a launch of 3 to 5 us)
+        ctx.bias_dtype = None if bias is None else bias.dtype
+        if bias is not None and bias.dtype != compute and bias.dtype != torch.float32:
             bias = bias.to(compute)
-        ctx.save_for_backward(input, weight_sparse_T, bias)
+        ctx.save_for_backward(input, weight_sparse_T, bias if ctx.bias_dtype != torch.float32 else None)
         shape = ctx.shape = input.shape
         ctx.weight_dtype = weight.dtype
         if len(shape) != 2:
@@ -79,7 +82,8 @@ class sparse_linear_transpose(autograd.Function):
                 input = input.view(-1, input.shape[-1])
             if needs[4]:
                 # MVUE24(dY^T) and grad_bias = dY.sum(0) (README.md:193-197) from one read of dY
-                grad_sparse, grad_bias = to_sparse_semi_structured_with_row_sums(grad_output.t(), MVUE24=True, dtype=grad_output.dtype)
+                grad_sparse, grad_bias = to_sparse_semi_structured_with_row_sums(
+                    grad_output.t(), MVUE24=True, dtype=grad_output.dtype, sums_dtype=torch.float32 if ctx.bias_dtype == torch.float32 else None)
             else:
                 grad_sparse = to_sparse_semi_structured(grad_output.t(), MVUE24=True, dtype=grad_output.dtype)
             grad_weight = _spmm(grad_sparse, input, True, out_dtype=ctx.weight_dtype)

@@ -69,6 +69,9 @@ typedef enum {
 
 /* GELU is the exact (erf) form, torch.nn.functional.gelu's default; the reference's epilogues stop at SILU */
 typedef enum { TF24_ACT_NONE = 0, TF24_ACT_RELU = 1, TF24_ACT_SILU = 2, TF24_ACT_GELU = 3 } tf24_activation;
+/* or-ed to the activation of tf24_spmm / tf24_linear: the bias is float32 whatever out_dtype is, and is rounded to it before it is added
+ * (what a layer with a float32 bias in mixed precision does with a cast of its own).  Not for integer results. */
+#define TF24_BIAS_F32 0x100
 
 /*
  * Storage of a compressed [m,k] matrix (values + metadata).
@@ -266,6 +269,9 @@ int tf24_soft_threshold24(const void* dense, int dtype, int layout, int64_t ld, 
  */
 int tf24_soft_threshold24_scaled(const float* dense, int64_t m, int64_t k, const float* scale, float scale_value, void* out, int out_dtype,
                                  void* stream);
+/* the same, and bias_out[0..m) = bias[0..m) rounded to out_dtype: both operands of the layer's product from one launch */
+int tf24_soft_threshold24_scaled_bias(const float* dense, int64_t m, int64_t k, const float* scale, float scale_value, void* out,
+                                      const float* bias, void* bias_out, int out_dtype, void* stream);
 int tf24_sparse24_dense(const void* dense, int dtype, int layout, int64_t ld, int64_t m, int64_t k,
                         void* sparse_out, void* mask_out, void* stream);
 int tf24_mvue24_dense(const void* dense, int dtype, int layout, int64_t ld, int64_t m, int64_t k,
@@ -357,7 +363,7 @@ int tf24_masked_add(void* grad, int grad_dtype, const void* p, int p_dtype, cons
  *              TF24_COL_MAJOR means stored [k, n_dense] (element (k,j) at k*ldb + j)
  *   c          output; c_layout TF24_ROW_MAJOR stores C[i,j] at i*ldc + j ([n_sparse,n_dense]);
  *              TF24_COL_MAJOR stores it at j*ldc + i ([n_dense,n_sparse]: the Y of X.W^T)
- *   bias       NULL or [n_sparse] of out_dtype's float family (added per sparse row i)
+ *   bias       NULL or [n_sparse] of out_dtype's float family, or float32 with TF24_BIAS_F32 (added per sparse row i)
  *   scale      multiplies the accumulator before bias (1.0 for 16-bit; scale_a*scale_b for fp8)
  *   workspace  NULL, or scratch of workspace_bytes for k-split partial tiles: products whose output
  *              tiles cannot fill the GPU (k-heavy shapes such as dW) are split along k and reduced in
@@ -417,6 +423,9 @@ int tf24_gelu_glu_backward(const void* grad_out, int64_t ld_grad_out, const void
  */
 int tf24_grad_weight(const void* g, int64_t ldg, const void* x, int64_t ldx, int dtype, int64_t tokens, int64_t m, int64_t n,
                      void* dw, void* db, void* workspace, int64_t workspace_bytes, void* stream);
+/* the same with dw and db float32: the values tf24_grad_weight gives, widened (gradients of float32 parameters) */
+int tf24_grad_weight_f32(const void* g, int64_t ldg, const void* x, int64_t ldx, int dtype, int64_t tokens, int64_t m, int64_t n,
+                         float* dw, float* db, void* workspace, int64_t workspace_bytes, void* stream);
 int64_t tf24_grad_weight_workspace_bytes(int64_t tokens, int64_t m, int64_t n);
 
 /*

@@ -1335,3 +1335,32 @@ def test_spmm_square_tiles_k_strided(cuda, dtype, n, stages, cols):
     assert _spmm(s, x, True, out_dtype=torch.float32).equal(want)
     assert torch.mm(s, x).equal(want.to(dtype))
     assert torch.mm(x.t(), s.t()).equal(want.t().to(dtype))
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("n,k,rows", [(32, 64, 5), (256, 256, 3), (8192, 128, 7), (4096, 4096, 40), (1024, 4096, 100),      # general, narrow, slim, half tiles
+                                      (6144, 192 * 64, 757), (4128, 192, 4111), (4128, 2112, 4111), (3040, 320, 6130)])     # pieces, 256 x 256, 192 x 192
+@pytest.mark.parametrize("activation", [None, "relu"])
+def test_linear_float32_bias_is_rounded(cuda, dtype, n, k, rows, activation):
+    """A float32 bias with 16-bit results: the same bits as the bias rounded by the caller, in every kernel."""
+    import sparse
+    g = torch.Generator(device=cuda).manual_seed(n + rows)
+    s = sparse.to_sparse_semi_structured(torch.randn(n, k, device=cuda, generator=g), dtype=dtype)
+    x = torch.randn(rows, k, device=cuda, generator=g).to(dtype)
+    bias = 3 * torch.randn(n, device=cuda, generator=g)
+    bias[::7] *= 1e-6                                              # (subnormal in half precision)
+    call = lambda b: sparse.sparse_semi_structured_linear(x, s, bias=b, activation=activation)
+    assert call(bias).equal(call(bias.to(dtype)))
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("m,k", [(1, 4), (8, 8), (300, 1028)])
+def test_soft_threshold_scaled_with_bias(cuda, dtype, m, k):
+    from sparse import _native as N
+    g = torch.Generator(device=cuda).manual_seed(m)
+    w, b = torch.randn(m, k, device=cuda, generator=g), torch.randn(m, device=cuda, generator=g)
+    want, out, rounded = (torch.empty(shape, dtype=dtype, device=cuda) for shape in ((m, k), (m, k), (m,)))
+    code = N.dtype_code(dtype)
+    N.check(N.lib().tf24_soft_threshold24_scaled(w.data_ptr(), m, k, None, 1.25, want.data_ptr(), code, N.stream_ptr()))
+    N.check(N.lib().tf24_soft_threshold24_scaled_bias(w.data_ptr(), m, k, None, 1.25, out.data_ptr(), b.data_ptr(), rounded.data_ptr(), code, N.stream_ptr()))
+    assert out.equal(want) and rounded.equal(b.to(dtype))

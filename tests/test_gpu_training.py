@@ -677,6 +677,10 @@ def test_grad_weight_kernel_is_exact_and_deterministic(cuda, tokens, m, n, dtype
     half_ulp = 2.0 ** (-11 if dtype == torch.float16 else -8)
     for bytes_given in {0, nbytes}:
         first = run(g, x, bytes_given)
+        wide = torch.empty((m, n), device=cuda), torch.empty((m,), device=cuda)          # the float32 form: the same values
+        N.check(lib.tf24_grad_weight_f32(g.data_ptr(), m, x.data_ptr(), n, N.dtype_code(dtype), tokens, m, n, wide[0].data_ptr(), wide[1].data_ptr(),
+                                         ws.data_ptr(), bytes_given, N.stream_ptr()))
+        assert all(a.equal(b.float()) for a, b in zip(wide, first))
         for got, again, ref in zip(first, run(g, x, bytes_given), exact):
             assert got.equal(again), bytes_given
             # each of the `tokens` additions rounds a partial sum of at most about 4 sqrt(tokens) by half of 2^-23 of it
