@@ -20,6 +20,7 @@ behaviour.  Differences, all deliberate:
 import ctypes
 import warnings
 from collections import namedtuple
+from functools import cached_property
 from typing import Any, Optional
 
 import torch
@@ -385,7 +386,7 @@ class SparseSemiStructuredTensor(torch.Tensor):
             raise ValueError("All of the tensor arguments are None!")
         dtype = previous.dtype if dtype is None else dtype
         out = torch.Tensor._make_wrapper_subclass(cls, original_shape, device=previous.device, dtype=dtype, layout=previous.layout, requires_grad=False)
-        out._dtype = dtype                           # (as an attribute of the object: `dtype` itself goes by __torch_function__)
+        out._dtype = dtype
         return out
 
     def __init__(self, original_tensor: Optional[torch.Tensor], original_shape: Optional[torch.Size] = None,
@@ -533,6 +534,12 @@ class SparseSemiStructuredTensor(torch.Tensor):
         if to_pad_m or to_pad_n:
             return torch.nn.functional.pad(original_tensor, (0, to_pad_n, 0, to_pad_m))
         return original_tensor
+
+    @cached_property
+    def _dtype(self):
+        """`dtype` as an attribute of the object, without __torch_function__.  Set where the object is made; looked up here for one
+        that was saved before there was such an attribute."""
+        return self.dtype
 
     def _out_dtype(self):
         return self._FP8_OUT_DTYPE if self._dtype in _FLOAT8 else None

@@ -232,3 +232,17 @@ def test_pieces_of_products_with_few_columns():
         assert scratch(N.F16, n, k, 16) > 0
     for n, k in ((11008, 4096), (3072, 768), (8192, 8192)):
         assert scratch(N.F16, n, k, 1) == scratch(N.E4M3, n, k, 1) == scratch(N.E4M3, n, k, 8) == 0
+
+
+def test_weights_saved_without_their_dtype_attribute(tmp_path):
+    """A compressed weight that was saved before its objects carried the dtype loads and answers as a new one does."""
+    from sparse import SparseSemiStructuredTensor
+    new = SparseSemiStructuredTensor(None, torch.Size((32, 64)), sparse_tensor_cutlass=torch.ones(32, 32).half(),
+                                     meta_tensor_cutlass=torch.zeros(32, 4, dtype=torch.int16))
+    old = new.detach()
+    del old.__dict__["_dtype"]
+    for i, weight in enumerate((new, old)):
+        torch.save(weight, tmp_path / f"{i}.pt")
+        loaded = torch.load(tmp_path / f"{i}.pt", weights_only=False)
+        for w in (loaded, loaded.detach(), loaded.t()):
+            assert w._dtype is w.dtype is torch.float16 and w._out_dtype() is None
