@@ -275,6 +275,8 @@ def _spmm(sparse, dense, sparse_first, bias=None, out_dtype=None, scale=1.0, act
     device = dense.device
     out = torch.empty(out_shape, dtype=out_dtype, device=device)
     if bias is not None:
+        if bias.is_neg():
+            bias = bias.resolve_neg()                # (the kernels read its storage)
         if bias.dtype is torch.float32 and out_dtype in _SIXTEEN_BIT and bias.is_contiguous():
             activation |= N.BIAS_F32                 # rounded where it is read
         elif bias.dtype != out_dtype or not bias.is_contiguous():

@@ -1351,6 +1351,8 @@ def test_linear_float32_bias_is_rounded(cuda, dtype, n, k, rows, activation):
     bias[::7] *= 1e-6                                              # (subnormal in half precision)
     call = lambda b: sparse.sparse_semi_structured_linear(x, s, bias=b, activation=activation)
     assert call(bias).equal(call(bias.to(dtype)))
+    for b in (bias, bias.to(dtype)):
+        assert call(torch._neg_view(b)).equal(call(-b))
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
