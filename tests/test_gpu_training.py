@@ -796,6 +796,18 @@ def test_soft_threshold_linear_very_wide(cuda, n, m):
     assert grads[0].equal(gy.float().t() @ x) and grads[1].equal(gy.float().sum(0))
 
 
+def test_soft_threshold_linear_negated_bias(cuda):
+    """A bias whose sign is still to be applied is not read as it lies.  Bit for bit the result of the bias with its sign."""
+    import sparse
+    torch.manual_seed(3)
+    mod = sparse.SoftThresholdLinear(128, 264, device=cuda)
+    mod.init_scale()
+    x, bias = torch.randn(300, 128, device=cuda), torch.randn(264, device=cuda)
+    call = lambda b: torch.func.functional_call(mod, {"bias": b}, (x,))
+    with torch.no_grad(), torch.autocast("cuda", dtype=torch.bfloat16):
+        assert call(torch._neg_view(bias)).equal(call(-bias))
+
+
 @pytest.mark.parametrize("shape", [(1, 8), (64, 128), (37, 1000), (768, 3072)])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_soft_threshold16_is_threshold_scale_and_cast(cuda, shape, dtype):
