@@ -355,7 +355,7 @@ using Wave4Cfg192 = TileCfgT<2, 3>;
 // chained tiles: 39.5 and 40.6 us for the first, 52.0 and 41.8 for the third, 36.2 and 35.9 for the second.
 using SquareCfg = TileCfgT<2, 3, 3>;
 constexpr int kWave4MinStages = 32;
-constexpr int kRotateMinStages = 64;       // (at least 24: the first three stages of a tile are copied before the order wraps)
+constexpr int kRotateMinK = 8192;          // (at least 24 stages: the first three of a tile are copied before the order wraps)
 // 256 x 64 tiles, two waves: for dense operands of at most 64 columns (a few dozen tokens), where a
 // 256-wide tile would copy and multiply clamped columns.  26 KB per stage, two blocks per CU.
 using SlimCfg = TileCfgT<1, 2>;
@@ -454,16 +454,16 @@ spmm_pipe(const uint8_t* __restrict__ a_values, const uint8_t* __restrict__ a_me
   const int nstages_total = (int)((k * ES) / C::KB);
   const int st_begin = (int)((int64_t)split * nstages_total / splits);
   const int nstages = (int)((int64_t)(split + 1) * nstages_total / splits) - st_begin;
-  // The tiles of XCD x take their stages from the x-th eighth of k on and wrap round (4-wave form, kRotateMinStages or more
-  // stages).  A stage of the dense operand is 128 bytes from each of 256 rows, whose pitch is often a multiple of some
+  // The tiles of XCD x take their stages from the x-th eighth of k on and wrap round (4-wave form, k of kRotateMinK or
+  // more).  A stage of the dense operand is 128 bytes from each of 256 rows, whose pitch is often a multiple of some
   // 4 KB: with all XCDs at the same stage the whole chip reads the same few memory channels at a time, and the copies, two
   // stages ahead, arrive late wherever the operand comes from memory and not from the last cache.  us on operands that
   // change from product to product, without and with: e4m3 16384 x 8192 x 8192 537 -> 515 (on the same operands 494 and
-  // 494), bf16 3001 x 11008 x 4096 143 -> 132, f16 8192 x 8192 x 8192 515 -> 498, bf16 9000 x 4096 x 3072 125 -> 122,
-  // f16 8192 x 4096 x 11008 362 -> 362 to 364.  By halves or quarters of k instead of eighths 134 and 133 for the
-  // second, three stages apart 138; 24 and 48 stages: no difference that repeats.
+  // 494), bf16 3001 x 11008 x 4096 143 -> 132, f16 8192 x 8192 x 8192 515 -> 498.  By halves or quarters of k instead of
+  // eighths 134 and 133 for the second, three stages apart 138.  Below kRotateMinK it is no gain: f16 8192 x 4096 x 11008
+  // 362 -> 362 to 364, 8192 x 5120 x 8192 330 -> 334, 8192 x 6144 x 8192 387 -> 392; bf16 9000 x 4096 x 3072 125 -> 122.
   constexpr bool ROTATE = PERSIST && C::NW == 4;
-  const int rot = ROTATE && nstages >= kRotateMinStages ? (bid & 7) * nstages >> 3 : 0;
+  const int rot = ROTATE && k >= kRotateMinK ? (bid & 7) * nstages >> 3 : 0;
   const int st_first = st_begin + rot;
 
   // ---- per-lane global sources of the copies (first stage of this unit); LDS destinations are wave-uniform.
@@ -1134,7 +1134,10 @@ inline int64_t tile_rounds(int64_t tiles, int64_t cu_slots) { return ((tiles + 7
 // Whether a product with 16-bit j-major results and k contiguous, in one piece, takes 192 x 192 tiles: rounds x (us of a tile's
 // stages + its prologue and output pass) against the same of what it would take otherwise -- 256 x 256 tiles (chained, with
 // their last rows on half tiles: tiles_i and tail_rows), or from kWave4MinStages stages on 256 x 192 ones.  The constants are
-// read off timings of 8 to 172 stages and 1 to 4 rounds; of 74 products drawn from 512 x 320 to 11008 x 8704 and 500
+// read off timings of 8 to 172 stages and 1 to 4 rounds; where full rounds follow each other the matrix cores are held to the clock
+// that their power allows, and no tile takes less than its share of the chip at that clock: 0.64 us a stage of 256 square tiles,
+// 0.75 and 1.0 of the others, whose fragments serve more instructions (W[11008, 4096] against 4096 columns, five full rounds of
+// square tiles: 205 us, on 256 x 192 ones 184).  Without that limit, of 74 products drawn from 512 x 320 to 11008 x 8704 and 500
 // to 16000 columns (fp16 and e4m3) the choice is 0.4 % off the better one on average and 3 to 7 % for six of them.
 inline int square_stagger_ticks(int64_t rounds, int stages) { return rounds > 1 && stages <= 32 ? 300 : 0; }
 inline bool takes_square(int64_t n_sparse, int64_t n_dense, int stages, int tiles_i, int tail_rows, int cu_slots) {
@@ -1142,13 +1145,16 @@ inline bool takes_square(int64_t n_sparse, int64_t n_dense, int stages, int tile
   const int64_t square = ((n_sparse + SquareCfg::BI - 1) / SquareCfg::BI) * ((n_dense + SquareCfg::BJ - 1) / SquareCfg::BJ);
   const int64_t rounds = tile_rounds(square, cu_slots);
   const bool four_waves = stages >= kWave4MinStages;
-  double others = (double)tile_rounds(tiles_i * tiles_j, cu_slots) * (four_waves ? 0.93 * stages + 2.5 : 0.88 * stages + 3.8);
+  auto us = [&](int64_t tiles, double of_round, double sustained) {
+    return std::max((double)tile_rounds(tiles, cu_slots) * of_round, (double)tiles / (8 * cu_slots) * sustained * stages);
+  };
+  double others = us(tiles_i * tiles_j, four_waves ? 0.93 * stages + 2.5 : 0.88 * stages + 3.8, 1.0);
   if (tail_rows) others += 0.5 * stages + 5.0;
   if (four_waves) {
     const int64_t narrow = (tiles_i + tail_rows) * ((n_dense + Wave4Cfg192::BJ - 1) / Wave4Cfg192::BJ);
-    others = std::min(others, (double)tile_rounds(narrow, cu_slots) * (0.69 * stages + 2.0));
+    others = std::min(others, us(narrow, 0.69 * stages + 2.0, 0.75));
   }
-  return (double)rounds * (0.53 * stages + 1.6) + 0.01 * square_stagger_ticks(rounds, stages) < 0.97 * others;
+  return us(square, 0.53 * stages + 1.6, 0.64) + 0.01 * square_stagger_ticks(rounds, stages) < 0.97 * others;
 }
 
 // Whether a product with k strided does: the pieces that either tile would be cut into, estimated as choose_pieces does and
