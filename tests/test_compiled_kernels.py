@@ -1,0 +1,62 @@
+"""Properties of the tiled 2:4 kernels that a result cannot show, read from the assembly that hipcc makes of this
+repository's sources: whether the copies of a stage may stay in flight over the stage barrier."""
+import importlib.util
+import os
+import re
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+
+def _assembly(tmp_path, kernels):
+    """{kernel symbol: its lines} of spmm_pipe instantiated for each of `kernels` (template arguments)"""
+    spec = importlib.util.spec_from_file_location("tf24_build", os.path.join(ROOT, "2by4-pretrain_amd", "build.py"))
+    build = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(build)
+    if not os.path.exists(build.HIPCC):
+        pytest.skip("no hipcc")
+    src, out = tmp_path / "kernels.hip", tmp_path / "kernels.s"
+    src.write_text('#include "spmm_kernels.hpp"\nnamespace tf24 { const void* kernels[] = {'
+                   + ", ".join(f"(const void*)spmm_pipe<{k}>" for k in kernels) + "}; }\n")
+    subprocess.run([build.HIPCC, *build.FLAGS, "--cuda-device-only", "-S", str(src), "-o", str(out)], check=True, capture_output=True)
+    found, lines = {}, None
+    for line in out.read_text().splitlines():
+        start = re.match(r"(_Z\w*spmm_pipe\w*):\s*; @", line)
+        if start:
+            lines = found[start.group(1)] = []
+        elif line.startswith(".Lfunc_end"):
+            lines = None
+        elif lines is not None:
+            lines.append(line)
+    assert len(found) == len(kernels)
+    return found
+
+
+def _stage_loop(lines):
+    """The first innermost loop with matrix instructions."""
+    labels, loops = {}, []
+    for i, line in enumerate(lines):
+        label = re.match(r"(\.LBB\w+):", line)
+        if label:
+            labels[label.group(1)] = i
+        branch = re.search(r"s_c?branch\w*\s+(\.LBB\w+)", line)
+        if branch and branch.group(1) in labels:
+            loops.append((labels[branch.group(1)], i))
+    loops = [(a, b) for a, b in loops if any("smfmac" in line for line in lines[a:b])]
+    a, b = min((a, b) for a, b in loops if not any((c, d) != (a, b) and a <= c and d <= b for c, d in loops))
+    return lines[a:b]
+
+
+def test_chained_tiles_wait_only_at_the_stage_barrier(tmp_path):
+    """The loop over the stages waits for memory once, at its barrier, with the next stage's copies left in flight."""
+    kernels = [f"{t}, {out}, true, {tile}, {strided}, true, {acts}"
+               for t, out, tile, strided, acts in (
+                   ("f16_t", "f16_t", "TiledCfg", "false", "false"), ("f16_t", "f16_t", "TiledCfg", "true", "false"),
+                   ("bf16_t", "bf16_t", "TiledCfg", "false", "false"), ("f16_t", "float", "TiledCfg", "false", "false"),
+                   ("f16_t", "float", "TiledCfg", "true", "true"), ("f16_t", "f16_t", "SquareCfg", "false", "false"),
+                   ("f16_t", "f16_t", "Wave4Cfg", "false", "false"), ("f16_t", "f16_t", "Wave4Cfg192", "false", "false"))]
+    for name, lines in _assembly(tmp_path, kernels).items():
+        waits = [int(n) for line in _stage_loop(lines) for n in re.findall(r"vmcnt\((\d+)\)", line)]
+        assert len(waits) == 1 and waits[0] > 0, (name, waits)
