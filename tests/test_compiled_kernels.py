@@ -1,5 +1,5 @@
 """Properties of the tiled 2:4 kernels that a result cannot show, read from the assembly that hipcc makes of this
-repository's sources: whether the copies of a stage may stay in flight over the stage barrier."""
+repository's sources: whether the copies of a stage may stay in flight over the stage barrier, and what is spilled."""
 import importlib.util
 import os
 import re
@@ -60,3 +60,13 @@ def test_chained_tiles_wait_only_at_the_stage_barrier(tmp_path):
     for name, lines in _assembly(tmp_path, kernels).items():
         waits = [int(n) for line in _stage_loop(lines) for n in re.findall(r"vmcnt\((\d+)\)", line)]
         assert len(waits) == 1 and waits[0] > 0, (name, waits)
+
+
+def test_activation_forms_spill_nothing(tmp_path):
+    """The 8-wave kernels with an activation, the ones nearest to their 256 registers, keep everything in them."""
+    kernels = [f"{t}, {out}, true, TiledCfg, {strided}, {chained}, true"
+               for t, out, strided, chained in (
+                   ("f16_t", "f16_t", "false", "true"), ("f16_t", "f16_t", "true", "true"), ("f16_t", "f16_t", "true", "false"),
+                   ("bf16_t", "bf16_t", "false", "true"), ("e4m3_t", "bf16_t", "false", "true"), ("e4m3_t", "f16_t", "false", "true"))]
+    for name, lines in _assembly(tmp_path, kernels).items():
+        assert not any("scratch_" in line for line in lines), name
