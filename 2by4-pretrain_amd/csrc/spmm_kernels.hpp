@@ -343,16 +343,15 @@ using Wave4Cfg = TileCfgT<2, 4>;
 // (W[1600, 6400] against 12288 tokens: 336 wide tiles or 448 narrow ones, two rounds either way, 147 against 165 us;
 // W[11008, 4096] against 2048 tokens alike).  Long chained tiles only, like the 4-wave form itself.
 using Wave4Cfg192 = TileCfgT<2, 3>;
-// 192 x 192 tiles in the 4-wave form (wave tile 96 x 96, 144 accumulators): a stage takes 0.53 us against 0.93 of a
-// 256 x 256 one for 0.5625 of its work, so that they cost next to nothing in rate and rounds of the compute units fill
-// better -- 3072 and 768 rows against 12288 columns are 1024 and 256 of them, four rounds and one.  With a quarter of the
-// accumulators free they also hold the transposing fragment reads of a k-strided dense operand, which the other two
-// 4-wave tiles spill.  us, 256 rows a tile and now, fp16: 3072 x 768 against 12288 columns 51.2 -> 43.8, 6400 x 1600 against 2800
-// 53.3 -> 38.5, 768 x 3072 against 12288 44.3 -> 41.8 (bound by the 75 MB of its dense operand: 34 where they come from the last
-// cache); e4m3 5760 x 2688 against 6023 75.5 -> 62.1; k-strided 3072 x 12288 against 768 columns 50.8 -> 44.2, 768 x 12288 against
-// 3072 57.4 -> 51.4, 3072 x 1024 against 768 16.6 -> 13.1 (40 products of 8 to 253 stages: 14 % less on average).
+// 192 x 192 tiles in the 4-wave form (wave tile 96 x 96, 144 accumulators): where rounds of the compute units fill better with
+// them (takes_square).  A stage takes 0.53 us against 0.93 of a 256 x 256 one for 0.5625 of its work, but 0.67 against 1.0 at the
+// clock that full rounds sustain.  With a quarter of the accumulators free they also hold the transposing fragment reads of a
+// k-strided dense operand, which the other two 4-wave tiles spill.  us, 256 rows a tile and now, fp16: 6400 x 1600 against 2800
+// columns 53.3 -> 38.5, 768 x 3072 against 12288 43.5 -> 42.0 (bound by the 75 MB of its dense operand: 34 where they come from the
+// last cache); e4m3 5760 x 2688 against 6023 75.5 -> 62.1; k-strided 3072 x 12288 against 768 columns 50.8 -> 44.2, 768 x 12288
+// against 3072 57.4 -> 51.4, 3072 x 1024 against 768 16.6 -> 13.1 (40 products of 8 to 253 stages: 14 % less on average).
 // Two stage buffers and two workgroups to a compute unit (76 KB and 256 registers each) instead of three buffers and
-// chained tiles: 39.5 and 40.6 us for the first, 52.0 and 41.8 for the third, 36.2 and 35.9 for the second.
+// chained tiles: 36.2 and 35.9 us for the first, 52.0 and 41.8 for the second.
 using SquareCfg = TileCfgT<2, 3, 3>;
 constexpr int kWave4MinStages = 32;
 constexpr int kRotateMinK = 8192;          // (at least 24 stages: the first three of a tile are copied before the order wraps)
@@ -1136,30 +1135,45 @@ bool takes_mid(int64_t n_sparse, int64_t k, int64_t n_dense, int64_t workspace_b
 // Rounds of the compute units that so many tiles take (each XCD has an eighth of both).
 inline int64_t tile_rounds(int64_t tiles, int64_t cu_slots) { return ((tiles + 7) / 8 + cu_slots - 1) / cu_slots; }
 
+// A last round that fills less than half of the compute units: the tile rows that make up the full rounds stay
+// with the chained 256 x 256 tiles, the remaining rows go to a second launch on 256 x 128 tiles, which reach twice
+// as many compute units for half the time each (W[11008, 4096] against 8192 tokens: 1376 tiles = 5 rounds of 256
+// + 96; 40 tile rows chained, 3 rows as 192 half tiles: 351.6 -> 341.6 us).  Long tiles only: what a short
+// tile's round costs is mostly its prologue and output pass, which the second launch pays again.
+struct TileRows { int tiles_i, tail_rows; };
+inline TileRows full_rounds(int64_t n_sparse, int64_t n_dense, int stages, int cu_slots) {
+  const int tiles_i = (int)((n_sparse + TiledCfg::BI - 1) / TiledCfg::BI), tiles_j = (int)((n_dense + TiledCfg::BJ - 1) / TiledCfg::BJ);
+  const int cus = cu_slots * 8, tiles = tiles_i * tiles_j;
+  if (cus <= 0 || tiles % cus == 0 || stages < kWave4MinStages) return {tiles_i, 0};
+  const int rows = tiles / cus * cus / tiles_j, left = tiles_i - rows;                       // tile rows of the full rounds
+  const int64_t half_tiles = (int64_t)left * ((n_dense + MidCfg::BJ - 1) / MidCfg::BJ);
+  return rows * tiles_j > cus && left > 0 && half_tiles <= cus ? TileRows{rows, left} : TileRows{tiles_i, 0};
+}
+
 // Whether a product with 16-bit j-major results and k contiguous, in one piece, takes 192 x 192 tiles: rounds x (us of a tile's
 // stages + its prologue and output pass) against the same of what it would take otherwise -- 256 x 256 tiles (chained, with
-// their last rows on half tiles: tiles_i and tail_rows), or from kWave4MinStages stages on 256 x 192 ones.  The constants are
-// read off timings of 8 to 172 stages and 1 to 4 rounds; where full rounds follow each other the matrix cores are held to the clock
-// that their power allows, and no tile takes less than its share of the chip at that clock: 0.64 us a stage of 256 square tiles,
-// 0.75 and 1.0 of the others, whose fragments serve more instructions (W[11008, 4096] against 4096 columns, five full rounds of
-// square tiles: 205 us, on 256 x 192 ones 184).  Without that limit, of 74 products drawn from 512 x 320 to 11008 x 8704 and 500
-// to 16000 columns (fp16 and e4m3) the choice is 0.4 % off the better one on average and 3 to 7 % for six of them.
-inline int square_stagger_ticks(int64_t rounds, int stages) { return rounds > 1 && stages <= 32 ? 300 : 0; }
-inline bool takes_square(int64_t n_sparse, int64_t n_dense, int stages, int tiles_i, int tail_rows, int cu_slots) {
+// their last rows on half tiles: full_rounds), or from kWave4MinStages stages on 256 x 192 ones.  Where full rounds follow each
+// other the matrix cores are held to the clock that their power allows, and no tile takes less than its share of the chip at that
+// clock: 0.67 us a stage of 256 square tiles, 0.75 and 1.0 of the others, whose fragments serve more instructions.  Of 258
+// products of 5 to 172 stages drawn from 512 to 11008 rows and 500 to 16000 columns (fp16, bf16 and e4m3, operands that change
+// from product to product) the choice is 0.04 % off the better one on average, 3.6 % at worst; of 90 others that the constants
+// were not fitted to, a third of them on the same operands, 0.01 and 0.6 %.  (With 0.53 and 1.6 for square tiles and 0.88 and 3.8
+// for the 8-wave ones, which were read off few products, 2.2 and 18 % below 32 stages: 3072 x 768 against 12288 columns 44.2 us
+// on wide tiles and 48.3 on square ones, 2048 x 512 23.9 and 27.9, 6656 x 704 against 12879 86 and 101.)
+inline bool takes_square(int64_t n_sparse, int64_t n_dense, int stages, TileRows wide, int cu_slots) {
   const int64_t tiles_j = (n_dense + TiledCfg::BJ - 1) / TiledCfg::BJ;
   const int64_t square = ((n_sparse + SquareCfg::BI - 1) / SquareCfg::BI) * ((n_dense + SquareCfg::BJ - 1) / SquareCfg::BJ);
-  const int64_t rounds = tile_rounds(square, cu_slots);
   const bool four_waves = stages >= kWave4MinStages;
   auto us = [&](int64_t tiles, double of_round, double sustained) {
     return std::max((double)tile_rounds(tiles, cu_slots) * of_round, (double)tiles / (8 * cu_slots) * sustained * stages);
   };
-  double others = us(tiles_i * tiles_j, four_waves ? 0.93 * stages + 2.5 : 0.88 * stages + 3.8, 1.0);
-  if (tail_rows) others += 0.5 * stages + 5.0;
+  double others = us(wide.tiles_i * tiles_j, four_waves ? 0.93 * stages + 2.5 : 0.84 * stages + 5.5, 1.0);
+  if (wide.tail_rows) others += 0.5 * stages + 5.0;
   if (four_waves) {
-    const int64_t narrow = (tiles_i + tail_rows) * ((n_dense + Wave4Cfg192::BJ - 1) / Wave4Cfg192::BJ);
+    const int64_t narrow = (wide.tiles_i + wide.tail_rows) * ((n_dense + Wave4Cfg192::BJ - 1) / Wave4Cfg192::BJ);
     others = std::min(others, us(narrow, 0.69 * stages + 2.0, 0.75));
   }
-  return us(square, 0.53 * stages + 1.6, 0.64) + 0.01 * square_stagger_ticks(rounds, stages) < 0.97 * others;
+  return us(square, 0.53 * stages + 5.0, 0.67) < 0.95 * others;
 }
 
 // Whether a product with k strided does: the pieces that either tile would be cut into, estimated as choose_pieces does and
@@ -1209,20 +1223,13 @@ int launch_tiled(const void* av, const void* am, int64_t n_sparse, int64_t k, co
   int tiles_i = (int)((n_sparse + C::BI - 1) / C::BI);
   const int tiles_j = (int)((n_dense + C::BJ - 1) / C::BJ);
   const int splits = workspace ? choose_pieces<T, C>(n_sparse, k, n_dense, workspace_bytes, b_layout == TF24_COL_MAJOR).count : 1;
-  // A last round that fills less than half of the compute units: the tile rows that make up the full rounds stay
-  // with the chained 256 x 256 tiles, the remaining rows go to a second launch on 256 x 128 tiles, which reach twice
-  // as many compute units for half the time each (W[11008, 4096] against 8192 tokens: 1376 tiles = 5 rounds of 256
-  // + 96; 40 tile rows chained, 3 rows as 192 half tiles: 351.6 -> 341.6 us).  Long tiles only: what a short
-  // tile's round costs is mostly its prologue and output pass, which the second launch pays again.
+  const int stages = (int)(k * (int64_t)sizeof(T) / C::KB);
   int tail_rows = 0;
   if constexpr (std::is_same<C, TiledCfg>::value) {
-    const int cus = cu_slots * 8, tiles = tiles_i * tiles_j;
-    if (cus > 0 && c_layout == TF24_COL_MAJOR && b_layout == TF24_ROW_MAJOR && splits == 1 && tiles % cus != 0 &&
-        k * (int64_t)sizeof(T) / C::KB >= kWave4MinStages) {
-      const int rows = tiles / cus * cus / tiles_j;            // tile rows of the full rounds
-      const int left = tiles_i - rows;
-      const int64_t half_tiles = (int64_t)left * ((n_dense + MidCfg::BJ - 1) / MidCfg::BJ);
-      if (rows * tiles_j > cus && left > 0 && half_tiles <= cus) { tiles_i = rows; tail_rows = left; }
+    if (c_layout == TF24_COL_MAJOR && b_layout == TF24_ROW_MAJOR && splits == 1) {
+      const TileRows rows = full_rounds(n_sparse, n_dense, stages, cu_slots);
+      tiles_i = rows.tiles_i;
+      tail_rows = rows.tail_rows;
     }
   }
   const int per_xcd = (tiles_i * tiles_j * splits + 7) / 8;
@@ -1261,10 +1268,10 @@ int launch_tiled(const void* av, const void* am, int64_t n_sparse, int64_t k, co
   if constexpr (std::is_same<C, TiledCfg>::value && sizeof(OutT) == 2) {
     const int tiles_j192 = (int)((n_dense + Wave4Cfg192::BJ - 1) / Wave4Cfg192::BJ);
     const int per_xcd192 = (tiles_i * tiles_j192 + 7) / 8;
-    if (jm && b_layout == TF24_ROW_MAJOR && splits == 1 && k * (int64_t)sizeof(T) / C::KB >= 4 && cu_slots > 0 &&
-        takes_square(n_sparse, n_dense, (int)(k * (int64_t)sizeof(T) / C::KB), tiles_i, tail_rows, cu_slots)) {
+    if (jm && b_layout == TF24_ROW_MAJOR && splits == 1 && stages >= 4 && cu_slots > 0 &&
+        takes_square(n_sparse, n_dense, stages, {tiles_i, tail_rows}, cu_slots)) {
       const int square_i = (int)((n_sparse + SquareCfg::BI - 1) / SquareCfg::BI), square_j = (int)((n_dense + SquareCfg::BJ - 1) / SquareCfg::BJ);
-      const int square_stagger = square_stagger_ticks(tile_rounds((int64_t)square_i * square_j, cu_slots), (int)(k * (int64_t)sizeof(T) / C::KB));
+      const int square_stagger = tile_rounds((int64_t)square_i * square_j, cu_slots) > 1 && stages <= 32 ? 300 : 0;
       auto square = [&](auto acts) {
         hipLaunchKernelGGL((spmm_pipe<T, OutT, true, SquareCfg, false, true, decltype(acts)::value>), dim3((unsigned)(cu_slots * 8)),
                            dim3(SquareCfg::THREADS), 0, s, (const uint8_t*)av, (const uint8_t*)am, n_sparse, k, (const uint8_t*)b,
