@@ -354,7 +354,8 @@ using Wave4Cfg192 = TileCfgT<2, 3>;
 // chained tiles: 36.2 and 35.9 us for the first, 52.0 and 41.8 for the second.
 using SquareCfg = TileCfgT<2, 3, 3>;
 constexpr int kWave4MinStages = 32;
-constexpr int kRotateMinK = 8192;          // (at least 24 stages: the first three of a tile are copied before the order wraps)
+constexpr int kRotateMinStages = 56;
+static_assert(kRotateMinStages - 2 - (7 * kRotateMinStages >> 3) >= 1, "the first three stages of a tile are copied before the order wraps");
 // 256 x 64 tiles, two waves: for dense operands of at most 64 columns (a few dozen tokens), where a
 // 256-wide tile would copy and multiply clamped columns.  26 KB per stage, two blocks per CU.
 using SlimCfg = TileCfgT<1, 2>;
@@ -453,16 +454,20 @@ spmm_pipe(const uint8_t* __restrict__ a_values, const uint8_t* __restrict__ a_me
   const int nstages_total = (int)((k * ES) / C::KB);
   const int st_begin = (int)((int64_t)split * nstages_total / splits);
   const int nstages = (int)((int64_t)(split + 1) * nstages_total / splits) - st_begin;
-  // The tiles of XCD x take their stages from the x-th eighth of k on and wrap round (4-wave form, k of kRotateMinK or
-  // more).  A stage of the dense operand is 128 bytes from each of 256 rows, whose pitch is often a multiple of some
+  // The tiles of XCD x take their stages from the x-th eighth of k on and wrap round (4-wave form, kRotateMinStages or more).
+  // A stage of the dense operand is 128 bytes from each of 256 rows, whose pitch is often a multiple of some
   // 4 KB: with all XCDs at the same stage the whole chip reads the same few memory channels at a time, and the copies, two
-  // stages ahead, arrive late wherever the operand comes from memory and not from the last cache.  us on operands that
-  // change from product to product, without and with: e4m3 16384 x 8192 x 8192 537 -> 515 (on the same operands 494 and
-  // 494), bf16 3001 x 11008 x 4096 143 -> 132, f16 8192 x 8192 x 8192 515 -> 498.  By halves or quarters of k instead of
-  // eighths 134 and 133 for the second, three stages apart 138.  Below kRotateMinK it is no gain: f16 8192 x 4096 x 11008
-  // 362 -> 362 to 364, 8192 x 5120 x 8192 330 -> 334, 8192 x 6144 x 8192 387 -> 392; bf16 9000 x 4096 x 3072 125 -> 122.
+  // stages ahead, arrive late wherever the operand comes from memory and not from the last cache.  What counts is stages and
+  // not elements.  us on operands that change from product to product, without and with: 24 to 32 stages alike; 40 and 48
+  // within 0.7 % but for some products on square tiles (e4m3 3040 x 5120 against 6130 columns 69.7 -> 61.9); 56 e4m3 8192 x 7168
+  // against 8192 233 -> 227, 3040 x 7168 against 6130 84.4 -> 80.7, fp16 5120 x 3584 against 5000 112.2 -> 112.7; 64 fp16
+  // 4096 x 4096 against 3001 56.5 -> 53.8, 11008 x 4096 against 8192 358.1 -> 358.4, e4m3 8192 x 8192 against 16384 541.9 -> 513.7;
+  // 128 fp16 8192 x 8192 against 8192 530 -> 504; 172 bf16 4096 x 11008 against 3001 144.1 -> 132.9.  On the same operands 60 products
+  // of 40 to 128 stages are within 0.4 %.  By halves or quarters of k instead of eighths 134 and 133 for the last, three stages
+  // apart 138.  (So two equal rows of the dense operand may differ in the last bits of their sums where their tiles are on two XCDs;
+  // the same call gives the same bits.)
   constexpr bool ROTATE = PERSIST && C::NW == 4;
-  const int rot = ROTATE && k >= kRotateMinK ? (bid & 7) * nstages >> 3 : 0;
+  const int rot = ROTATE && nstages >= kRotateMinStages ? (bid & 7) * nstages >> 3 : 0;
   const int st_first = st_begin + rot;
 
   // ---- per-lane global sources of the copies (first stage of this unit); LDS destinations are wave-uniform.
@@ -1176,6 +1181,21 @@ inline bool takes_square(int64_t n_sparse, int64_t n_dense, int stages, TileRows
   return us(square, 0.53 * stages + 5.0, 0.67) < 0.95 * others;
 }
 
+// The tiles of a product with j-major results and k contiguous, in one piece: 256 x 256 ones on eight waves, or 4-wave forms --
+// those, where there are more of them than compute units (chained), 256 x 192 or 192 x 192 ones (16-bit results).
+// 256 x 192 also where both widths fit one round and the narrow tiles spread over more compute units (W[768, 3072] against
+// 12288 tokens: 144 wide tiles or 192 narrow ones, 36.1 -> 34.1 us; W[1024, 4096]: 192 or 256 tiles, 56.2 -> 53.9 us).
+enum class Tiles { WIDE8, WIDE4, NARROW4, SQUARE4 };
+inline Tiles choose_tiles(int64_t n_sparse, int64_t n_dense, int stages, TileRows wide, bool results16, int cu_slots) {
+  if (cu_slots <= 0 || stages < 4) return Tiles::WIDE8;
+  if (results16 && takes_square(n_sparse, n_dense, stages, wide, cu_slots)) return Tiles::SQUARE4;
+  if (stages < kWave4MinStages) return Tiles::WIDE8;
+  const int64_t tiles = wide.tiles_i * ((n_dense + TiledCfg::BJ - 1) / TiledCfg::BJ), narrow = wide.tiles_i * ((n_dense + Wave4Cfg192::BJ - 1) / Wave4Cfg192::BJ);
+  const int64_t rounds = tile_rounds(tiles, cu_slots), narrow_rounds = tile_rounds(narrow, cu_slots);
+  if (results16 && narrow_rounds <= rounds && (narrow_rounds > 1 || (narrow + 7) / 8 > (tiles + 7) / 8)) return Tiles::NARROW4;
+  return rounds > 1 ? Tiles::WIDE4 : Tiles::WIDE8;
+}
+
 // Whether a product with k strided does: the pieces that either tile would be cut into, estimated as choose_pieces does and
 // with further rounds counted by their stages.  (Few products are not: 6400 x 2816 against 1600 columns, 306 tiles instead of 175,
 // 39.8 us and 45.  Uncut 16-bit results stored i-major would leave in 2-byte stores: the staged pass takes 64 columns.)
@@ -1248,9 +1268,8 @@ int launch_tiled(const void* av, const void* am, int64_t n_sparse, int64_t k, co
   const int stagger_rounds = persist ? (per_xcd + cu_slots - 1) / cu_slots : 0;
   const int stagger = !persist ? 0 : k * (int64_t)sizeof(T) / C::KB <= 32 ? (sizeof(OutT) == 2 ? 300 : 600)
                                : (sizeof(OutT) == 4 && stagger_rounds >= 3) ? 600 : 0;
-  // long chained tiles of a k-contiguous dense operand take the 4-wave form
-  const bool wave4 = persist && std::is_same<C, TiledCfg>::value && b_layout == TF24_ROW_MAJOR &&
-                     k * (int64_t)sizeof(T) / C::KB >= kWave4MinStages;
+  const Tiles form = std::is_same<C, TiledCfg>::value && jm && b_layout == TF24_ROW_MAJOR && splits == 1
+                         ? choose_tiles(n_sparse, n_dense, stages, {tiles_i, tail_rows}, sizeof(OutT) == 2, cu_slots) : Tiles::WIDE8;
   auto launch_tail = [&]() {                       // the rows behind the full rounds, on 256 x 128 tiles
     if constexpr (std::is_same<C, TiledCfg>::value) {
       if (tail_rows > 0) {
@@ -1266,33 +1285,23 @@ int launch_tiled(const void* av, const void* am, int64_t n_sparse, int64_t k, co
     }
   };
   if constexpr (std::is_same<C, TiledCfg>::value && sizeof(OutT) == 2) {
-    const int tiles_j192 = (int)((n_dense + Wave4Cfg192::BJ - 1) / Wave4Cfg192::BJ);
-    const int per_xcd192 = (tiles_i * tiles_j192 + 7) / 8;
-    if (jm && b_layout == TF24_ROW_MAJOR && splits == 1 && stages >= 4 && cu_slots > 0 &&
-        takes_square(n_sparse, n_dense, stages, {tiles_i, tail_rows}, cu_slots)) {
-      const int square_i = (int)((n_sparse + SquareCfg::BI - 1) / SquareCfg::BI), square_j = (int)((n_dense + SquareCfg::BJ - 1) / SquareCfg::BJ);
-      const int square_stagger = tile_rounds((int64_t)square_i * square_j, cu_slots) > 1 && stages <= 32 ? 300 : 0;
-      auto square = [&](auto acts) {
-        hipLaunchKernelGGL((spmm_pipe<T, OutT, true, SquareCfg, false, true, decltype(acts)::value>), dim3((unsigned)(cu_slots * 8)),
-                           dim3(SquareCfg::THREADS), 0, s, (const uint8_t*)av, (const uint8_t*)am, n_sparse, k, (const uint8_t*)b,
-                           ldb * (int64_t)sizeof(T), n_dense, (OutT*)c, ldc, (const OutT*)bias, scale, act, square_i, square_j, 1,
-                           (float*)nullptr, square_stagger);
-      };
-      if ((act & ~TF24_BIAS_F32) == TF24_ACT_NONE) square(std::false_type{}); else square(std::true_type{});
+    auto chained = [&](auto cfg, auto acts, int ti, int tj, int start_stagger) {
+      using Cfg = decltype(cfg);
+      hipLaunchKernelGGL((spmm_pipe<T, OutT, true, Cfg, false, true, decltype(acts)::value>), dim3((unsigned)(cu_slots * 8)), dim3(Cfg::THREADS), 0, s,
+                         (const uint8_t*)av, (const uint8_t*)am, n_sparse, k, (const uint8_t*)b, ldb * (int64_t)sizeof(T), n_dense,
+                         (OutT*)c, ldc, (const OutT*)bias, scale, act, ti, tj, 1, (float*)nullptr, start_stagger);
+    };
+    auto either = [&](auto cfg, int ti, int tj, int start_stagger) {
+      if ((act & ~TF24_BIAS_F32) == TF24_ACT_NONE) chained(cfg, std::false_type{}, ti, tj, start_stagger);
+      else chained(cfg, std::true_type{}, ti, tj, start_stagger);
+    };
+    if (form == Tiles::SQUARE4) {
+      const int ti = (int)((n_sparse + SquareCfg::BI - 1) / SquareCfg::BI), tj = (int)((n_dense + SquareCfg::BJ - 1) / SquareCfg::BJ);
+      either(SquareCfg{}, ti, tj, tile_rounds((int64_t)ti * tj, cu_slots) > 1 && stages <= 32 ? 300 : 0);
       return check_launch("tf24_spmm");
     }
-    // Also where both widths fit one round and the narrow tiles spread over more compute units (W[768, 3072] against
-    // 12288 tokens: 144 wide tiles or 192 narrow ones, 36.1 -> 34.1 us; W[1024, 4096]: 192 or 256 tiles, 56.2 -> 53.9 us).
-    const bool one_round192 = C::BJ == 256 && c_layout == TF24_COL_MAJOR && splits == 1 && b_layout == TF24_ROW_MAJOR &&
-                              k * (int64_t)sizeof(T) / C::KB >= kWave4MinStages && cu_slots > 0 && per_xcd192 <= cu_slots && per_xcd192 > per_xcd;
-    if (one_round192 || (wave4 && per_xcd192 > cu_slots && (per_xcd192 + cu_slots - 1) / cu_slots <= (per_xcd + cu_slots - 1) / cu_slots)) {
-      if (one_round192) grid = dim3((unsigned)(cu_slots * 8));    // the chained-tile kernel with one tile per workgroup
-      auto narrow = [&](auto acts) {
-        hipLaunchKernelGGL((spmm_pipe<T, OutT, true, Wave4Cfg192, false, true, decltype(acts)::value>), grid, dim3(Wave4Cfg192::THREADS), 0, s,
-                           (const uint8_t*)av, (const uint8_t*)am, n_sparse, k, (const uint8_t*)b, ldb * (int64_t)sizeof(T), n_dense,
-                           (OutT*)c, ldc, (const OutT*)bias, scale, act, tiles_i, tiles_j192, splits, (float*)workspace, stagger);
-      };
-      if ((act & ~TF24_BIAS_F32) == TF24_ACT_NONE) narrow(std::false_type{}); else narrow(std::true_type{});
+    if (form == Tiles::NARROW4) {
+      either(Wave4Cfg192{}, tiles_i, (int)((n_dense + Wave4Cfg192::BJ - 1) / Wave4Cfg192::BJ), stagger);
       launch_tail();
       return check_launch("tf24_spmm");
     }
@@ -1301,7 +1310,7 @@ int launch_tiled(const void* av, const void* am, int64_t n_sparse, int64_t k, co
     constexpr bool ACTS = decltype(acts)::value;
     if constexpr (C::BJ == 256 && decltype(c_jmajor)::value) {
       if constexpr (std::is_same<C, TiledCfg>::value && !decltype(b_kstrided)::value) {
-        if (wave4) {
+        if (form == Tiles::WIDE4) {
           hipLaunchKernelGGL((spmm_pipe<T, OutT, true, Wave4Cfg, false, true, ACTS>), grid, dim3(Wave4Cfg::THREADS), 0, s,
                              (const uint8_t*)av, (const uint8_t*)am, n_sparse, k, (const uint8_t*)b, ldb * (int64_t)sizeof(T), n_dense,
                              (OutT*)c, ldc, (const OutT*)bias, scale, act, tiles_i, tiles_j, splits, (float*)workspace, stagger);

@@ -368,7 +368,9 @@ int tf24_masked_add(void* grad, int grad_dtype, const void* p, int p_dtype, cons
  *   workspace  NULL, or scratch of workspace_bytes for k-split partial tiles: products whose output
  *              tiles cannot fill the GPU (k-heavy shapes such as dW) are split along k and reduced in
  *              a second launch.  tf24_spmm_workspace_bytes() gives the size that enables every split
- *              the heuristic would take (0 = the shape is never split).  Deterministic either way.
+ *              the heuristic would take (0 = the shape is never split).  Deterministic either way: the same
+ *              call gives the same bits.  Where a sum over k starts depends on the tile under long k (7168 bytes
+ *              of a dense row or more), so two equal dense columns may differ in the last bits of a float result.
  * Shape rules (.cu:101-109): n_sparse % 32 == 0, k % 64 == 0 (16-bit) / 128 (8-bit),
  * n_dense % 8 == 0 (16-bit) / 16 (8-bit).  Leading dimensions: ldb a multiple of 8 (16-bit) / 16 (8-bit)
  * elements and at most 16 MiB per row (a tile's rows are addressed by 32-bit offsets), ldc a multiple of 8 for

@@ -1272,16 +1272,24 @@ def test_products_of_views_at_full_multiples(cuda, dtype, pitch, rows, view):
         assert got.shape == (rows, 64) and got.float().equal(want.to(got.dtype).float())
 
 
-@pytest.mark.parametrize("dtype", [torch.float16, torch.float8_e4m3fn, torch.int8])
-@pytest.mark.parametrize("n,stages,rows", [
-    (4128, 63, 4111),          # four waves, every XCD from the first stage on
-    (4128, 64, 4111),          # from here on each from its own eighth of k: chained tiles of either width
-    (4128, 71, 4111),          # eighths of unequal length
-    (800, 66, 12271),          # one round of 256 x 192 tiles with 16-bit results
-    (4128, 65, 8175)])         # full rounds of 256 x 256 tiles, the last tile row in a second launch
+# rows of the weight, stages of 128 bytes of k, dense rows; the tiles that products with 16-bit results take, and whether their
+# stages start at another eighth of k on each XCD (test_tile_rules.py holds both against the rules)
+STAGE_ORDER = [
+    (4384, 55, 5766, "wide", False),                # every XCD from the first stage on
+    (4384, 56, 5766, "wide", True),                 # from here on each from its own eighth of k
+    (4384, 59, 5766, "wide", True),                 # eighths of unequal length
+    (4960, 59, 6428, "wide, two launches", True),   # full rounds of 256 x 256 tiles, the last tile row on others
+    (800, 59, 12271, "narrow", True),               # one round of 256 x 192 tiles
+    (1568, 66, 10814, "narrow", True),              # two of them
+    (4128, 59, 4111, "square", True),               # 192 x 192 tiles, partial ones on either edge
+    (3040, 56, 6130, "square", True)]
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float8_e4m3fn, torch.int8])
+@pytest.mark.parametrize("n,stages,rows", [case[:3] for case in STAGE_ORDER])
 def test_linear_stage_order_by_xcd(cuda, dtype, n, stages, rows):
     """Long tiles whose stages start at another eighth of k on each XCD and wrap round: exact on small integers, with
-    32- and 16-bit results (256 x 256 and 256 x 192 tiles), and the same again on a second call."""
+    32- and 16-bit results (256 x 256, 256 x 192 and 192 x 192 tiles), and the same again on a second call."""
     import sparse
     k = stages * 128 // torch.empty(0, dtype=dtype).element_size()
     g = torch.Generator(device=cuda).manual_seed(rows + stages)
@@ -1289,19 +1297,22 @@ def test_linear_stage_order_by_xcd(cuda, dtype, n, stages, rows):
     s = sparse.to_sparse_semi_structured(w.to(torch.int8) if dtype == torch.int8 else w.float(), dtype=dtype)
     x = torch.randint(-2, 3, (rows, k), device=cuda, generator=g).to(dtype)
     want = x.float() @ s.to_dense().float().t()
-    for out_dtype in {torch.int8: (torch.int32,), torch.float16: (torch.float16,)}.get(dtype, (torch.float32, torch.bfloat16)):
+    for out_dtype in {torch.int8: (torch.int32,)}.get(dtype, (torch.float32, dtype if dtype.itemsize == 2 else torch.bfloat16)):
         got = sparse.sparse_semi_structured_linear(x, s, out_dtype=out_dtype)
         assert got.equal(want.to(out_dtype))
         assert sparse.sparse_semi_structured_linear(x, s, out_dtype=out_dtype).equal(got)
 
 
+SQUARE = [
+    (736, 4, 12271, False),         # one round, the shortest tiles; partial ones on either edge
+    (768, 5, 12288, False),         # 256 full tiles
+    (3040, 5, 6130, False),         # two rounds, every second workgroup starts late
+    (3040, 33, 6130, False),        # the same, together
+    (3040, 67, 6130, True)]         # from another eighth of k on each XCD
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float8_e4m3fn])
-@pytest.mark.parametrize("n,stages,rows", [
-    (736, 4, 12271),           # one round, the shortest tiles; partial ones on either edge
-    (768, 5, 12288),           # 256 full tiles
-    (3040, 5, 6130),           # two rounds, every second workgroup starts late
-    (3040, 33, 6130),          # the same, together
-    (3040, 67, 6130)])         # from another eighth of k on each XCD
+@pytest.mark.parametrize("n,stages,rows", [case[:3] for case in SQUARE])
 @pytest.mark.parametrize("activation", [None, "relu"])
 def test_linear_square_tiles(cuda, dtype, n, stages, rows, activation):
     """Products on 192 x 192 tiles, with and without bias: exact on small integers."""

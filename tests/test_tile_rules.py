@@ -6,6 +6,8 @@ import subprocess
 
 import pytest
 
+from test_gpu_parity import SQUARE, STAGE_ORDER
+
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 CU_SLOTS = 32                      # compute units of an XCD
 
@@ -24,10 +26,16 @@ def rules(tmp_path_factory):
 extern "C" int square(int64_t n_sparse, int64_t n_dense, int stages, int cu_slots) {
   return tf24::takes_square(n_sparse, n_dense, stages, tf24::full_rounds(n_sparse, n_dense, stages, cu_slots), cu_slots);
 }
+extern "C" int tiles(int64_t n_sparse, int64_t n_dense, int stages, int results16, int cu_slots) {
+  const tf24::TileRows rows = tf24::full_rounds(n_sparse, n_dense, stages, cu_slots);
+  return (int)tf24::choose_tiles(n_sparse, n_dense, stages, rows, results16, cu_slots) + (rows.tail_rows ? 100 : 0);
+}
+extern "C" int rotate_from() { return tf24::kRotateMinStages; }
 """)
     subprocess.run([build.HIPCC, *build.FLAGS, "--offload-host-only", "-shared", str(src), "-o", str(lib)], check=True, capture_output=True)
     handle = ctypes.CDLL(str(lib))
     handle.square.argtypes = [ctypes.c_int64, ctypes.c_int64, ctypes.c_int, ctypes.c_int]
+    handle.tiles.argtypes = [ctypes.c_int64, ctypes.c_int64, ctypes.c_int, ctypes.c_int, ctypes.c_int]
     return handle
 
 
@@ -39,3 +47,12 @@ extern "C" int square(int64_t n_sparse, int64_t n_dense, int stages, int cu_slot
     (4096, 15, 4145, 1), (4320, 25, 7701, 1)])                                # 31.9 26.4, 75.1 70.6
 def test_square_tiles_where_they_are_the_faster_ones(rules, n, stages, columns, square):
     assert rules.square(n, columns, stages, CU_SLOTS) == square
+
+
+@pytest.mark.parametrize("n,stages,rows,tiles,rotates", STAGE_ORDER + [case[:3] + ("square",) + case[3:] for case in SQUARE])
+def test_products_tested_on_the_gpu_take_the_tiles_they_are_for(rules, n, stages, rows, tiles, rotates):
+    code = rules.tiles(n, rows, stages, 1, CU_SLOTS)
+    assert code == {"wide": 1, "wide, two launches": 101, "narrow": 2, "square": 3}[tiles]
+    assert rotates == (stages >= rules.rotate_from())
+    # more than one round of half tiles, which would be taken first, and no room for pieces of k
+    assert -(-n // 256) * -(-rows // 128) > 256 and -(-n // 256) * -(-rows // 256) > 128
