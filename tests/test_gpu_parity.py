@@ -1329,10 +1329,13 @@ def test_linear_square_tiles(cuda, dtype, n, stages, rows, activation):
     assert sparse.sparse_semi_structured_linear(x, s, bias=bias, out_dtype=out_dtype, activation=activation).equal(act(want + bias.float()).to(out_dtype))
 
 
+SQUARE_STRIDED = [                  # and in how many pieces of k (test_tile_rules.py)
+    (64, 4, 72, 1), (224, 5, 200, 1), (192, 9, 192, 3), (352, 25, 2376, 3), (416, 8, 560, 1),         # tiles past either edge
+    (992, 40, 392, 5), (544, 117, 120, 15), (3072, 48, 768, 2), (3424, 202, 80, 11)]
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
-@pytest.mark.parametrize("n,stages,cols", [
-    (64, 4, 72), (224, 5, 200), (192, 9, 192), (352, 25, 2376), (416, 8, 160),       # one piece, tiles past either edge
-    (992, 40, 392), (544, 117, 120), (3072, 48, 768), (3424, 202, 80)])              # pieces of k
+@pytest.mark.parametrize("n,stages,cols", [case[:3] for case in SQUARE_STRIDED])
 def test_spmm_square_tiles_k_strided(cuda, dtype, n, stages, cols):
     """Products with a k-strided dense operand on 192 x 192 tiles, in one and in several pieces: exact on small integers, with
     float32 and 16-bit results of either order."""

@@ -6,7 +6,7 @@ import subprocess
 
 import pytest
 
-from test_gpu_parity import SQUARE, STAGE_ORDER
+from test_gpu_parity import SQUARE, SQUARE_STRIDED, STAGE_ORDER
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 CU_SLOTS = 32                      # compute units of an XCD
@@ -30,12 +30,21 @@ extern "C" int tiles(int64_t n_sparse, int64_t n_dense, int stages, int results1
   const tf24::TileRows rows = tf24::full_rounds(n_sparse, n_dense, stages, cu_slots);
   return (int)tf24::choose_tiles(n_sparse, n_dense, stages, rows, results16, cu_slots) + (rows.tail_rows ? 100 : 0);
 }
+extern "C" int strided(int64_t n_sparse, int64_t n_dense, int stages, int results16, int jmajor, int cu_slots) {
+  auto* rule = results16 ? tf24::strided_takes_square<tf24::f16_t, tf24::f16_t> : tf24::strided_takes_square<tf24::f16_t, float>;
+  return rule(n_sparse, (int64_t)stages * 64, n_dense, (int64_t)1 << 40, jmajor, cu_slots);
+}
+extern "C" int strided_pieces(int64_t n_sparse, int64_t n_dense, int stages) {
+  return tf24::choose_pieces<tf24::f16_t, tf24::SquareCfg>(n_sparse, (int64_t)stages * 64, n_dense, (int64_t)1 << 40, true).count;
+}
 extern "C" int rotate_from() { return tf24::kRotateMinStages; }
 """)
     subprocess.run([build.HIPCC, *build.FLAGS, "--offload-host-only", "-shared", str(src), "-o", str(lib)], check=True, capture_output=True)
     handle = ctypes.CDLL(str(lib))
     handle.square.argtypes = [ctypes.c_int64, ctypes.c_int64, ctypes.c_int, ctypes.c_int]
     handle.tiles.argtypes = [ctypes.c_int64, ctypes.c_int64, ctypes.c_int, ctypes.c_int, ctypes.c_int]
+    handle.strided.argtypes = [ctypes.c_int64, ctypes.c_int64, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int]
+    handle.strided_pieces.argtypes = [ctypes.c_int64, ctypes.c_int64, ctypes.c_int]
     return handle
 
 
@@ -56,3 +65,11 @@ def test_products_tested_on_the_gpu_take_the_tiles_they_are_for(rules, n, stages
     assert rotates == (stages >= rules.rotate_from())
     # more than one round of half tiles, which would be taken first, and no room for pieces of k
     assert -(-n // 256) * -(-rows // 128) > 256 and -(-n // 256) * -(-rows // 256) > 128
+
+
+@pytest.mark.parametrize("n,stages,columns,pieces", SQUARE_STRIDED)
+def test_k_strided_products_tested_on_the_gpu_take_square_tiles(rules, n, stages, columns, pieces):
+    assert rules.strided_pieces(n, columns, stages) == pieces
+    # with float32 results and with 16-bit ones stored j-major; i-major ones only where a reduction writes them
+    forms = [rules.strided(n, columns, stages, results16, jmajor, CU_SLOTS) for results16, jmajor in ((0, 0), (1, 1), (1, 0))]
+    assert forms == [1, 1, int(pieces > 1)]
