@@ -338,10 +338,19 @@ def test_metadata_words_move_alone(cuda, dtype, m, k):
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
-def test_linear_without_gradients_is_the_dispatched_one(cuda, dtype):
+def test_linear_without_gradients_is_the_dispatched_one(cuda, dtype, monkeypatch):
     """torch.nn.functional.linear under no_grad and inference_mode against the same call through the dispatcher: the same bits
-    for every form of its arguments that either takes, the same refusals."""
+    for every form of its arguments that either takes, the same refusals.  Counted: contiguous 2-d and 3-d inputs with a bias of
+    their type or none go to the kernels in one call, the other forms through the dispatcher."""
     import sparse
+    from sparse import semi_structured
+    direct, in_one_call = semi_structured._linear_no_grad, []
+
+    def counted(*args):
+        out = direct(*args)
+        in_one_call.append(out is not None)
+        return out
+    monkeypatch.setattr(semi_structured, "_linear_no_grad", counted)
     g = torch.Generator(device=cuda).manual_seed(0)
     s = sparse.to_sparse_semi_structured(torch.randn(96, 128, device=cuda, generator=g), dtype=dtype)
     pieces = sparse.SparseSemiStructuredTensor(None, s.shape, sparse_tensor_cutlass=s.values(), meta_tensor_cutlass=s.indices(), dtype=dtype)
@@ -366,17 +375,31 @@ def test_linear_without_gradients_is_the_dispatched_one(cuda, dtype):
         for xn, inp in inputs.items():
             for bn, bias in biases.items():
                 with torch.no_grad():
+                    in_one_call.clear()
                     got = outcome(weight, inp, bias)
+                    if wn != "pieces":               # (in panel form after its first product)
+                        plain = wn in ("", "parameter") and xn in ("2d", "3d", "parameter") and bn in ("", "bias", "parameter")
+                        assert any(in_one_call) == plain, (wn, xn, bn)
+                    in_one_call.clear()
                     with torch._C.DisableTorchFunctionSubclass():
                         want = outcome(weight, inp, bias)
+                    assert not in_one_call
                 if isinstance(want, type):
                     assert got is want, (wn, xn, bn, got, want)
                 else:
                     assert got.dtype == want.dtype and got.shape == want.shape and got.equal(want), (wn, xn, bn)
     with torch.inference_mode():
-        assert torch.nn.functional.linear(x, s, b).equal(torch.nn.functional.linear(x.clone(), s, b))
+        for inp in (x, x.clone(), x[0]):
+            in_one_call.clear()
+            got = torch.nn.functional.linear(inp, s, b)
+            assert in_one_call == [True]
+            with torch._C.DisableTorchFunctionSubclass():
+                assert got.equal(torch.nn.functional.linear(inp, s, b))
+            assert in_one_call == [True]
+    in_one_call.clear()
     with torch.no_grad(), torch.autocast("cuda", dtype=dtype):
         got = torch.nn.functional.linear(x.float(), s, b)
+        assert torch.nn.functional.linear(x, s, b).equal(got) and not any(in_one_call)
         with torch._C.DisableTorchFunctionSubclass():
             assert got.equal(torch.nn.functional.linear(x.float(), s, b))
     with torch.no_grad():
