@@ -142,11 +142,13 @@ _PLAIN_KEYS = set()
 def is_plain(t):
     """An ordinary strided GPU tensor: what torch dispatches on says that nothing is left to be done to it (a negation or
     conjugation, names, a batch or a tangent) before a kernel reads its storage."""
+    if type(t) not in (torch.Tensor, torch.nn.Parameter) or not t.is_cuda:
+        return False
     if not _PLAIN_KEYS:
         for inference in (False, True):
             with torch.inference_mode(inference):
                 _PLAIN_KEYS.add(torch._C._dispatch_keys(torch.empty(0, device="cuda")).raw_repr())
-    return type(t) in (torch.Tensor, torch.nn.Parameter) and torch._C._dispatch_keys(t).raw_repr() in _PLAIN_KEYS
+    return torch._C._dispatch_keys(t).raw_repr() in _PLAIN_KEYS
 
 
 def layout_of(t):

@@ -524,7 +524,14 @@ class SparseSemiStructuredTensor(torch.Tensor):
                 out = _linear_no_grad(x, weight, bias)
                 if out is not None:
                     return out
-        return _torch_route(func, types, args, kwargs or {})
+        # other classes with a __torch_function__ decide among themselves, as they do where this class has none (torch's default for
+        # a tensor subclass declines whatever is not a subclass of its own)
+        others = tuple(t for t in types if not issubclass(t, SparseSemiStructuredTensor))
+        for other in others:
+            result = other.__torch_function__(func, others, args, kwargs or {})
+            if result is not NotImplemented:
+                return result
+        return NotImplemented if others else _torch_route(func, types, args, kwargs or {})
 
     # Torch's own route for the methods, without the way through __torch_function__, which is 1.2 us of host time: converting a
     # weight of 768 x 768 and reading its values, metadata and dense form 37.0 us that way, 33.1 this way.

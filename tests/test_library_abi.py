@@ -246,3 +246,39 @@ def test_weights_saved_without_their_dtype_attribute(tmp_path):
         loaded = torch.load(tmp_path / f"{i}.pt", weights_only=False)
         for w in (loaded, loaded.detach(), loaded.t()):
             assert w._dtype is w.dtype is torch.float16 and w._out_dtype() is None
+
+
+def test_other_tensor_classes_meet_a_compressed_weight(monkeypatch):
+    """A 2:4 weight takes no part in what other classes do with torch's functions: a plain subclass of Tensor keeps its class, one
+    whose handler declines classes that it does not know is asked without this one, as beside a dense weight."""
+    import torch.nn.functional as F
+    from sparse import SparseSemiStructuredTensor, semi_structured
+    monkeypatch.setattr(semi_structured, "_spmm", lambda s, x, first, **kw: torch.full((x.shape[0], 32), 2.0, dtype=x.dtype))
+    weight = SparseSemiStructuredTensor(None, torch.Size((32, 64)), sparse_tensor_cutlass=torch.ones(32, 32).half(),
+                                        meta_tensor_cutlass=torch.zeros(32, 4, dtype=torch.int16))
+
+    class Plain(torch.Tensor):
+        pass
+
+    class Handler(torch.Tensor):
+        @classmethod
+        def __torch_function__(cls, func, types, args=(), kwargs=None):
+            return types if all(issubclass(t, Handler) for t in types) else NotImplemented
+
+    class Declines(torch.Tensor):
+        @classmethod
+        def __torch_function__(cls, func, types, args=(), kwargs=None):
+            return NotImplemented
+
+    x = torch.ones(8, 64).half()
+    for grad in (False, True):
+        with torch.set_grad_enabled(grad):
+            for call in (lambda x: F.linear(x, weight), lambda x: torch.mm(x, weight.t())):
+                for cls in (torch.Tensor, Plain):
+                    out = call(x.as_subclass(cls))
+                    assert type(out) is cls and out.shape == (8, 32)
+                assert call(x.as_subclass(Handler)) == (Handler,)
+                with pytest.raises(TypeError):
+                    call(x.as_subclass(Declines))
+            assert torch.mm(weight, x.t().as_subclass(Handler)) == (Handler,)
+            assert F.linear(x, weight, torch.ones(32).as_subclass(Handler)) == (Handler,)
