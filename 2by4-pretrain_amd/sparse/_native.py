@@ -162,9 +162,16 @@ def layout_of(t):
     return None
 
 
+def resolved(t):
+    """t, with its sign applied where it is a negated view (torch._neg_view, the imaginary part of a conjugate): the kernels
+    read storage."""
+    return t.resolve_neg() if t.is_neg() else t
+
+
 def as_matrix(t, like=None):
     """t itself when the kernels can address it (row- or column-major, 16-byte aligned, leading
     dimension a multiple of 8), otherwise a copy; with `like`, a copy laid out like that tensor."""
+    t = resolved(t)
     if like is not None:
         lay = layout_of(like)
         mine = layout_of(t)

@@ -84,7 +84,7 @@ class MaskedDecayAdamW(Optimizer):
             lr, eps, wd, alpha = float(group["lr"]), float(group["eps"]), float(group["weight_decay"]), float(group["alpha"])
             # Everything is looked at before anything is launched; the tensors of one launch share the types of
             # gradient and mask and a host-side step count (device-side counts travel with their tensor)
-            entries, counts, launches, fresh = [], [], {}, []
+            entries, counts, launches, fresh, negated = [], [], {}, [], []
             for p in params:
                 grad = p.grad
                 if grad is None:
@@ -101,7 +101,7 @@ class MaskedDecayAdamW(Optimizer):
                     mask = None
                 if mask is not None and (mask.stride() != stride or mask.device != p.device):
                     raise RuntimeError("MaskedDecayAdamW: mask must have the parameter's strides and device")
-                entries.append((p, grad, state, mask, N.dtype_code(grad.dtype), N.U8 if mask is None else N.dtype_code(mask.dtype)))
+                entries.append((p, N.resolved(grad), state, mask, N.dtype_code(grad.dtype), N.U8 if mask is None else N.dtype_code(mask.dtype)))
                 if torch.is_tensor(state["step"]):
                     counts.append(state["step"])
             if fresh:
@@ -119,9 +119,14 @@ class MaskedDecayAdamW(Optimizer):
                     key, step_ptr = (grad_code, mask_code, step), 0
                 if mask is not None:
                     p.cnt = 0
-                launches.setdefault(key, []).extend((p.data_ptr(), grad.data_ptr(), state["exp_avg"].data_ptr(), state["exp_avg_sq"].data_ptr(),
+                values = N.resolved(p)
+                if values is not p:
+                    negated.append((p, values))
+                launches.setdefault(key, []).extend((values.data_ptr(), grad.data_ptr(), state["exp_avg"].data_ptr(), state["exp_avg_sq"].data_ptr(),
                                                      0 if mask is None else mask.data_ptr(), step_ptr, p.numel()))
             for (grad_code, mask_code, step), words in launches.items():
                 N.check(N.lib().tf24_adamw_masked_decay_list(struct.pack("%dq" % len(words), *words), len(words) // 7, grad_code, mask_code,
                                                              lr, float(beta1), float(beta2), eps, wd, alpha, step, N.stream_ptr()))
+            for p, values in negated:
+                p.copy_(values)
         return loss

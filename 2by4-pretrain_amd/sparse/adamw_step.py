@@ -89,6 +89,7 @@ class AdamW_STEP(Optimizer):
                 if grad.stride() != p.stride():
                     raise RuntimeError("AdamW_STEP: the gradient must have the parameter's strides")
                 state['step'] += 1
+                values, grad = N.resolved(p), N.resolved(grad)
                 tracked = hasattr(p, 'mask')
                 z_ptr, z_option, precond = None, 0, None
                 if tracked and watching:
@@ -101,9 +102,11 @@ class AdamW_STEP(Optimizer):
                     assert p.mask == 'sparse'
                     precond = state['preconditioned_variance'].data_ptr()
                 N.check(lib.tf24_adamw_step(
-                    p.data_ptr(), grad.data_ptr(), N.dtype_code(grad.dtype), state['exp_avg'].data_ptr(),
+                    values.data_ptr(), grad.data_ptr(), N.dtype_code(grad.dtype), state['exp_avg'].data_ptr(),
                     state['exp_avg_sq'].data_ptr(), state['max_exp_avg_sq'].data_ptr() if amsgrad else None, precond,
                     p.numel(), lr, float(beta1), float(beta2), eps, wd, state['step'], z_ptr, z_option, stream))
+                if values is not p:
+                    p.copy_(values)
         if watching:
             self._watch_variance(partials, tracked_elements)
         return loss

@@ -21,5 +21,8 @@ def masked_add_(grad: torch.Tensor, p_data: torch.Tensor, p_mask: torch.Tensor, 
     dense_in_memory = grad.is_contiguous() or (grad.dim() == 2 and grad.t().is_contiguous())
     if not dense_in_memory:
         raise RuntimeError("masked_add_: tensors must be dense in memory (contiguous in some dimension order)")
-    N.check(N.lib().tf24_masked_add(grad.data_ptr(), N.dtype_code(grad.dtype), p_data.data_ptr(), N.dtype_code(p_data.dtype),
+    target, p_data = N.resolved(grad), N.resolved(p_data)
+    N.check(N.lib().tf24_masked_add(target.data_ptr(), N.dtype_code(grad.dtype), p_data.data_ptr(), N.dtype_code(p_data.dtype),
                                     p_mask.data_ptr(), N.dtype_code(p_mask.dtype), n, float(alpha), N.stream_ptr()))
+    if target is not grad:
+        grad.copy_(target)

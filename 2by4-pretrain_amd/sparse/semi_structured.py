@@ -232,6 +232,7 @@ def _spmm(sparse, dense, sparse_first, bias=None, out_dtype=None, scale=1.0, act
     # only rows with k contiguous go in any number, a count off the type's multiple with k strided.  clone: a tensor that
     # starts off such a boundary counts as contiguous.
     multiple = _DTYPE_TO_SEMI_STRUCTURED_SPARSE_CONFIG[vdtype].dense_min_rows        # elements of 16 bytes
+    dense = N.resolved(dense)
     d0, d1 = dense.shape
     s0, s1 = dense.stride()
     if d0 == 1 and s1 == 1:
@@ -279,8 +280,7 @@ def _spmm(sparse, dense, sparse_first, bias=None, out_dtype=None, scale=1.0, act
     device = dense.device
     out = torch.empty(out_shape, dtype=out_dtype, device=device)
     if bias is not None:
-        if bias.is_neg():
-            bias = bias.resolve_neg()                # (the kernels read its storage)
+        bias = N.resolved(bias)
         if bias.dtype is torch.float32 and out_dtype in _SIXTEEN_BIT and bias.is_contiguous():
             activation |= N.BIAS_F32                 # rounded where it is read
         elif bias.dtype != out_dtype or not bias.is_contiguous():
@@ -426,7 +426,7 @@ class SparseSemiStructuredTensor(torch.Tensor):
             # built from pieces: values [m, k/2] row-major and metadata, canonical nibble stream or (class
             # flag) the reference's reordered words
             mm, half = sparse_tensor_cutlass.shape
-            self._set_storage(sparse_tensor_cutlass.contiguous().view(-1), meta_tensor_cutlass.contiguous().view(-1),
+            self._set_storage(N.resolved(sparse_tensor_cutlass).contiguous().view(-1), meta_tensor_cutlass.contiguous().view(-1),
                               (mm, 2 * half), N.COMPRESSED_CUTLASS if self._CUTLASS_METADATA else N.COMPRESSED_CANONICAL)
         else:
             self._set_storage(None, None, None, N.COMPRESSED_CANONICAL)
@@ -658,7 +658,7 @@ def to_sparse_semi_structured_pair(original_tensor: torch.Tensor, mask: torch.Te
     rebuilds every optimizer step (README.md:165-166).  Both results are bit-identical to the
     separate calls.  w [m, k] row-major, both dimensions a multiple of 64 (128 for float8); with
     any other input the two separate conversions run instead."""
-    w = original_tensor
+    w = N.resolved(original_tensor)
     if not w.is_cuda or w.dim() != 2 or dtype not in _DTYPE_TO_SEMI_STRUCTURED_SPARSE_CONFIG or mask is None:
         return (to_sparse_semi_structured(w, mask=mask, dtype=dtype), to_sparse_semi_structured(w.T, mask=mask.T, dtype=dtype))
     m, k = w.shape
@@ -697,7 +697,7 @@ def to_sparse_semi_structured_with_row_sums(original_tensor: torch.Tensor, MVUE2
     where the row sums are the bias gradient `grad_output.sum(0)`) both results come from one pass over
     `t`; the sums are added in float32 and rounded once to t's dtype (`sums_dtype` float32: not at all).  Any
     other input runs the conversion and torch's sum separately."""
-    t = original_tensor
+    t = N.resolved(original_tensor)
     cfg = _DTYPE_TO_SEMI_STRUCTURED_SPARSE_CONFIG.get(dtype)
     fusable = (t.is_cuda and t.dim() == 2 and cfg is not None and t.dtype in (torch.float32, torch.float16, torch.bfloat16)
                and dtype != torch.int8 and not (mask is not None and MVUE24) and SparseSemiStructuredTensor._PANEL_LAYOUT)

@@ -36,6 +36,7 @@ def _borrowed_wrapper(values, meta, meta_layout):
         layout = _META_LAYOUTS[meta_layout]
     else:
         raise RuntimeError(f"meta_layout {meta_layout!r} is not supported (canonical, cutlass)")
+    values = N.resolved(values)
     m, half = values.shape
     wrapper = SparseSemiStructuredTensor(None, original_shape=torch.Size([m, 2 * half]), sparse_tensor_cutlass=values,
                                          meta_tensor_cutlass=meta, dtype=values.dtype)

@@ -65,6 +65,8 @@ def transposable_mask_(dense: Tensor, mask: Tensor, abs: bool = True) -> Tensor:
         raise RuntimeError("transposable_mask_: mask must be a bool tensor with the shape, strides and device of a dense "
                            "row- or column-major matrix (16-byte aligned, leading dimension a multiple of 8)")
     m, k = dense.shape
+    if dense.is_neg():                               # (the kernel reads storage, with the mask's pitch)
+        dense = torch.empty_strided(dense.shape, dense.stride(), dtype=dense.dtype, device=dense.device).copy_(dense)
     layout, ld = N.layout_of(dense)
     N.check(N.lib().tf24_transposable_mask(dense.data_ptr(), N.dtype_code(dense.dtype), layout, ld, m, k, int(bool(abs)),
                                            None, mask.data_ptr(), N.stream_ptr()))

@@ -404,3 +404,83 @@ def test_linear_without_gradients_is_the_dispatched_one(cuda, dtype, monkeypatch
             assert got.equal(torch.nn.functional.linear(x.float(), s, b))
     with torch.no_grad():
         assert torch.vmap(lambda v: torch.nn.functional.linear(v, s))(x).equal(torch.nn.functional.linear(x, s))
+
+
+def _negated(t):
+    """A view of -t whose storage holds t."""
+    return torch._neg_view(t)
+
+
+def test_negated_views_are_read_with_their_sign(cuda):
+    """Every entry point on views whose sign is still to be applied: bit for bit the results of the tensors with their sign."""
+    import sparse
+    from sparse.sparse_linear_transpose import sparse_linear_transpose
+    from sparse.transposable_semi_structured import transposable_mask_
+    g = torch.Generator(device=cuda).manual_seed(7)
+    w = torch.randn(128, 256, device=cuda, generator=g)
+    x = torch.randn(64, 256, device=cuda, generator=g).half()
+    gy = torch.randn(64, 128, device=cuda, generator=g).half()
+    rand = torch.rand(128, 256, device=cuda, generator=g)
+    mask = sparse.sparse24(w)[1] != 0
+    s = sparse.to_sparse_semi_structured(w)
+    values, meta = s.values().clone(), s.indices().clone()
+    both = lambda c: (c.values(), c.indices())
+
+    def transpose_layer(x, gy):
+        x = x.detach().requires_grad_()
+        weight, bias = torch.nn.Parameter(w.clone()), torch.nn.Parameter(w[:, 0].clone())
+        pair = sparse.to_sparse_semi_structured_pair(w, torch.ones_like(mask) & mask, dtype=torch.float16)
+        torch.manual_seed(1)
+        y = sparse_linear_transpose.apply(x, weight, *pair, bias)
+        return (y.detach(), *torch.autograd.grad(y, (x, weight, bias), gy))
+
+    def s_ste_layer(x, weight, gy):
+        mod = sparse.SoftThresholdLinear(256, 128, device=cuda)
+        mod.scale.fill_(1.25)
+        x, weight = x.detach().requires_grad_(), weight.detach().requires_grad_()
+        with torch.autocast("cuda", dtype=torch.float16):
+            y = torch.func.functional_call(mod, {"weight": weight, "bias": w[:, 1].clone()}, (x,))
+        return (y.detach(), *torch.autograd.grad(y, (x, weight), gy))
+
+    def gated(x, gy):
+        x = x.view(4, 16, 256).detach().requires_grad_()
+        y = sparse.GELUglu()(x)
+        return y.detach(), torch.autograd.grad(y, x, gy.view(4, 16, 128))[0]
+
+    def masked_decay(grad, p):
+        grad = grad.clone() if not grad.is_neg() else _negated(grad.neg())
+        sparse.masked_add_(grad, p, mask, alpha=0.5)
+        return grad.resolve_neg()
+
+    def step(make, p, grad):
+        p = torch.nn.Parameter(p.clone() if not p.is_neg() else _negated(p.neg()))
+        p.grad, p.mask = grad, mask if make is sparse.MaskedDecayAdamW else "dense"
+        make([p], lr=0.1).step()
+        return p.detach().resolve_neg()
+
+    linear = sparse.sparse_semi_structured_linear
+    calls = {
+        "compress": (lambda w: both(sparse.to_sparse_semi_structured(w)), w),
+        "compress by mask": (lambda w: both(sparse.to_sparse_semi_structured(w, mask=mask)), w),
+        "compress MVUE24": (lambda w, r: both(sparse.to_sparse_semi_structured(w, MVUE24=True, rand=r)), w, rand),
+        "compress column-major": (lambda w: both(sparse.to_sparse_semi_structured(w.t())), w),
+        "compress a pitched view": (lambda w: both(sparse.to_sparse_semi_structured(w[:, :128])), w),
+        "pair": (lambda w: sum((both(c) for c in sparse.to_sparse_semi_structured_pair(w, mask)), ()), w),
+        "row sums": (lambda w: (lambda c, sums: (*both(c), sums))(*sparse.to_sparse_semi_structured_with_row_sums(w.t())), w),
+        "row sums of a pitched view": (lambda w: (lambda c, sums: (*both(c), sums))(*sparse.to_sparse_semi_structured_with_row_sums(w[:, :128].t())), w),
+        "soft threshold": (sparse.soft_threshold24, w), "sparse24": (sparse.sparse24, w), "MVUE24": (sparse.MVUE24_approx, w, rand),
+        "search": (lambda w: sparse.TransposableSparse(abs=False)(w), w),
+        "search in place": (lambda w: transposable_mask_(w, torch.empty_like(w, dtype=torch.bool), abs=False), w),
+        "search in place, pitched": (lambda w: transposable_mask_(w[:, :128], torch.zeros(128, 256, dtype=torch.bool, device=cuda)[:, :128], abs=False), w),
+        "product": (lambda x: linear(x, s), x), "product of raw operands": (lambda x, v: linear(x, v, meta), x, values),
+        "product of pieces": (lambda v: torch.mm(x, sparse.SparseSemiStructuredTensor(None, s.shape, sparse_tensor_cutlass=v, meta_tensor_cutlass=meta).t()), values),
+        "bias": (lambda b: linear(x, s, bias=b), w[:, 2].contiguous()), "S @ dense": (lambda x: torch.mm(s, x.t()), x),
+        "transpose layer": (transpose_layer, x, gy), "s-ste layer": (s_ste_layer, x, w, gy), "gated": (gated, x, gy),
+        "masked decay": (masked_decay, w, w.flip(0)),
+        "AdamW": (lambda p, d: step(sparse.MaskedDecayAdamW, p, d), w, w.flip(0)), "AdamW_STEP": (lambda p, d: step(sparse.AdamW_STEP, p, d), w, w.flip(0))}
+    for name, (call, *args) in calls.items():
+        want = call(*[-a for a in args])
+        for which in range(len(args)):
+            got = call(*[_negated(a) if i == which else -a for i, a in enumerate(args)])
+            pairs = zip(want, got) if isinstance(want, tuple) else [(want, got)]
+            assert all(a.resolve_neg().equal(b.resolve_neg()) for a, b in pairs), (name, which)
