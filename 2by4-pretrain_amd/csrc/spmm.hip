@@ -8,6 +8,8 @@ namespace {
 // extent: what the number of dense columns must be a multiple of (0: the operand type's own)
 int validate(const char* fn, int dtype, int64_t n_sparse, int64_t k, int b_layout, int64_t ldb, int64_t n_dense, int64_t extent,
              int out_dtype, int c_layout, int64_t ldc, int activation) {
+  const bool bias_f32 = activation & TF24_BIAS_F32;
+  activation &= ~TF24_BIAS_F32;
   if (dtype != TF24_F16 && dtype != TF24_BF16 && !is_8bit(dtype)) return fail(TF24_ERR_DTYPE, "%s: unsupported operand dtype %d", fn, dtype);
   if (dtype == TF24_I8) {
     // integer product (.cu:594-637): int32 results, no or ReLU activation
@@ -32,6 +34,7 @@ int validate(const char* fn, int dtype, int64_t n_sparse, int64_t k, int b_layou
   const int64_t cmult = (out_dtype == TF24_F16 || out_dtype == TF24_BF16) ? 8 : 4;
   if (ldc < cext || ldc % cmult) return fail(TF24_ERR_STRIDE, "%s: ldc %lld must be >= %lld and a multiple of %lld", fn, (long long)ldc, (long long)cext, (long long)cmult);
   if (activation < TF24_ACT_NONE || activation > TF24_ACT_GELU) return fail(TF24_ERR_ARG, "%s: bad activation %d", fn, activation);
+  if (bias_f32 && out_dtype == TF24_I32) return fail(TF24_ERR_ARG, "%s: integer results take an integer bias", fn);
   return TF24_OK;
 }
 }  // namespace
@@ -75,9 +78,8 @@ int run_spmm(const char* fn, const void* a_values, const void* a_meta, int a_lay
              const void* b, int b_layout, int64_t ldb, int64_t n_dense, int64_t extent, void* c, int out_dtype, int c_layout, int64_t ldc,
              const void* bias, float scale, int activation, void* workspace, int64_t workspace_bytes, void* stream) {
   const int bias_f32 = activation & TF24_BIAS_F32;
-  int rc = validate(fn, dtype, n_sparse, k, b_layout, ldb, n_dense, extent, out_dtype, c_layout, ldc, activation & ~TF24_BIAS_F32);
+  int rc = validate(fn, dtype, n_sparse, k, b_layout, ldb, n_dense, extent, out_dtype, c_layout, ldc, activation);
   if (rc) return rc;
-  if (bias_f32 && out_dtype == TF24_I32) return fail(TF24_ERR_ARG, "%s: integer results take an integer bias", fn);
   if (!a_values || !a_meta || !b || !c) return fail(TF24_ERR_ARG, "%s: null pointer", fn);
   if ((rc = check_aligned(fn, 16, {a_values, b, c, workspace}))) return rc;
   // panel metadata is copied 16 bytes per lane; canonical metadata is read in words of up to 4 bytes, row pitch k/8

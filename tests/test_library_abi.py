@@ -97,6 +97,9 @@ def test_transposable_and_spmm_validators(native):
     assert sp(N.F16, 32, 64, 8, ldb=1 << 23) == 0 and sp(N.F16, 32, 64, 8, ldb=(1 << 23) + 8) == -3     # rows of the dense operand: at most 16 MiB
     assert sp(N.E4M3, 32, 128, 16, ldb=1 << 24) == 0 and sp(N.E4M3, 32, 128, 16, ldb=(1 << 24) + 16) == -3
     assert sp(N.F16, 32, 64, 8, act=5) == -5 and sp(N.F16, 32, 64, 8, bl=3) == -5
+    # a float32 bias, whatever the results are but integers
+    assert sp(N.F16, 32, 64, 8, act=N.BIAS_F32) == 0 and sp(N.E4M3, 32, 128, 16, out=N.F32, act=N.BIAS_F32 | N.ACT_GELU) == 0
+    assert sp(N.F16, 32, 64, 8, act=N.BIAS_F32 | 5) == -5 and sp(N.I8, 32, 128, 16, out=N.I32, act=N.BIAS_F32) == -5
 
 
 def test_misaligned_pointers_are_refused_before_any_launch(native):
