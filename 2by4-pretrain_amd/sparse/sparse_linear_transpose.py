@@ -45,7 +45,7 @@ class sparse_linear_transpose(autograd.Function):
         ctx.bias_dtype = None if bias is None else bias.dtype
         if bias is not None and bias.dtype != compute and bias.dtype != torch.float32:
             bias = bias.to(compute)
-        ctx.save_for_backward(input, weight_sparse_T, bias if ctx.bias_dtype != torch.float32 else None)
+        ctx.save_for_backward(input, weight_sparse_T)
         shape = ctx.shape = input.shape
         ctx.weight_dtype = weight.dtype
         if len(shape) != 2:
@@ -57,7 +57,7 @@ class sparse_linear_transpose(autograd.Function):
 
     @staticmethod
     def backward(ctx, grad_output):
-        input, weight_T, bias = ctx.saved_tensors
+        input, weight_T = ctx.saved_tensors
         grad_input = grad_weight = grad_bias = None
         # An expanded scalar gradient (all strides 0: the layer's output fed straight into .sum()) is
         # materialised with its values.  The reference replaces a 3-d one by ones (README.md:186-187), which

@@ -823,3 +823,19 @@ def test_soft_threshold16_is_threshold_scale_and_cast(cuda, shape, dtype):
         got = _soft_threshold16.apply(w, scale, dtype)
         assert got.view(torch.int16).equal(want.view(torch.int16)) or (
             got.isnan().equal(want.isnan()) and got[~got.isnan()].view(torch.int16).equal(want[~want.isnan()].view(torch.int16)))
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+def test_sparse_linear_transpose_bias_may_change_before_the_backward_pass(cuda, dtype):
+    """No gradient depends on the bias: one that has been updated in place since the forward pass, in either type, is no error."""
+    import sparse
+    torch.manual_seed(0)
+    mod = sparse.SparseLinearTranspose(128, 64, device=cuda)
+    bias = torch.nn.Parameter(torch.randn(64, device=cuda, dtype=dtype))
+    mod.bias = bias
+    x, gy = torch.randn(64, 128, device=cuda, dtype=torch.float16), torch.randn(64, 64, device=cuda, dtype=torch.float16)
+    y = mod(x)
+    with torch.no_grad():
+        bias += 1
+    y.backward(gy)
+    assert bias.grad.dtype == dtype and torch.allclose(bias.grad.float(), gy.float().sum(0), rtol=1e-3, atol=1e-2)
