@@ -839,3 +839,38 @@ def test_sparse_linear_transpose_bias_may_change_before_the_backward_pass(cuda, 
         bias += 1
     y.backward(gy)
     assert bias.grad.dtype == dtype and torch.allclose(bias.grad.float(), gy.float().sum(0), rtol=1e-3, atol=1e-2)
+
+
+@pytest.mark.parametrize("leaf", [True, False])
+def test_soft_threshold_linear_lets_go_of_its_weight(cuda, leaf):
+    """The layer's graph does not keep a float32 weight that is the result of something, and leads to it, or to a parameter, all
+    the same: d(sum of dX) / dW is the straight-through sum of dY over the tokens, also where the weight changes in between."""
+    import gc
+    import weakref
+    import sparse
+    torch.manual_seed(11)
+    mod = sparse.SoftThresholdLinear(128, 264, device=cuda)
+    mod.init_scale()
+    base = mod.weight
+    x, gy = torch.randn(300, 128, device=cuda, requires_grad=True), torch.randn(300, 264, device=cuda).bfloat16()
+
+    def forward():
+        weight = base if leaf else base * 1.0
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            return torch.func.functional_call(mod, {"weight": weight}, (x,)), None if leaf else weakref.ref(weight)
+
+    y, freed = forward()
+    gc.collect()
+    assert leaf or freed() is None
+    with torch.no_grad():
+        base.add_(1.0)
+    dx, = torch.autograd.grad(y, x, gy, create_graph=True)
+    second, = torch.autograd.grad(dx.float().sum(), base)
+    want = gy.float().sum(0)[:, None].expand(264, 128)
+    # (dX and its gradient are 16-bit products: 2^-8 of each sum of 300 terms of about 1)
+    assert second.dtype == torch.float32 and torch.allclose(second, want, rtol=2.0 ** -7, atol=0.1)
+    y, _ = forward()
+    first = torch.autograd.grad(y, (x, base, mod.bias), gy, retain_graph=True)
+    with torch.autograd.graph.save_on_cpu():
+        y, _ = forward()
+    assert all(a.equal(b) for a, b in zip(first, torch.autograd.grad(y, (x, base, mod.bias), gy)))
