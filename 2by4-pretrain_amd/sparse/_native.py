@@ -142,9 +142,11 @@ _PLAIN_KEYS = set()
 def is_plain(t):
     """An ordinary strided GPU tensor: what torch dispatches on says that nothing is left to be done to it (a negation or
     conjugation, names, a batch or a tangent) before a kernel reads its storage."""
-    if type(t) not in (torch.Tensor, torch.nn.Parameter) or not t.is_cuda:
+    if type(t) not in (torch.Tensor, torch.nn.Parameter):
         return False
     if not _PLAIN_KEYS:
+        if not t.is_cuda:                            # (nothing here needs a GPU before there is a tensor on it)
+            return False
         for inference in (False, True):
             with torch.inference_mode(inference):
                 _PLAIN_KEYS.add(torch._C._dispatch_keys(torch.empty(0, device="cuda")).raw_repr())
