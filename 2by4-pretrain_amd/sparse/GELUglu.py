@@ -16,7 +16,7 @@ __all__ = ["GELUglu", "gelu_glu"]
 def _as_2d(t):
     """(2-d view [rows, cols], layout, ld) the kernels can address, copying when neither
     dimension of the flattened tensor is contiguous."""
-    t2 = N.resolved(t).reshape(-1, t.shape[-1])
+    t2 = (t.resolve_neg() if t.is_neg() else t).reshape(-1, t.shape[-1])
     lay = N.layout_of(t2)
     if lay is None:
         t2 = t2.contiguous()
@@ -57,7 +57,7 @@ class gelu_glu(autograd.Function):
         (x2,) = ctx.saved_tensors
         layout = ctx.layout
         rows, cols = x2.shape
-        go = N.resolved(grad_output).reshape(rows, cols // 2).to(x2.dtype)
+        go = (grad_output.resolve_neg() if grad_output.is_neg() else grad_output).reshape(rows, cols // 2).to(x2.dtype)
         want = _empty_like_layout(rows, cols // 2, layout, x2)
         if go.stride() != want.stride():          # bring the gradient to the layout of the forward output
             want.copy_(go)

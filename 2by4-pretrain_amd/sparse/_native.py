@@ -97,11 +97,16 @@ def version():
     return lib().tf24_version().decode()
 
 
+class _Codes(dict):
+    def __missing__(self, dtype):
+        raise RuntimeError(f"dtype {dtype} is not supported by the gfx950 2:4 library")
+
+
+dtype_codes = _Codes(_DTYPES)
+
+
 def dtype_code(dtype):
-    try:
-        return _DTYPES[dtype]
-    except KeyError:
-        raise RuntimeError(f"dtype {dtype} is not supported by the gfx950 2:4 library") from None
+    return dtype_codes[dtype]
 
 
 def operand_code(dtype):
@@ -166,14 +171,20 @@ def layout_of(t):
 
 def resolved(t):
     """t, with its sign applied where it is a negated view (torch._neg_view, the imaginary part of a conjugate): the kernels
-    read storage."""
-    return t.resolve_neg() if t.is_neg() else t
+    read storage.  A column-major matrix stays one.  (is_neg alone is 0.2 us: entry points ask once per tensor, hot ones without
+    the call of this function.)"""
+    if not t.is_neg():
+        return t
+    if t.dim() == 2 and t.stride(0) == 1 and t.stride(1) > 1:
+        return t.t().resolve_neg().t()
+    return t.resolve_neg()
 
 
 def as_matrix(t, like=None):
     """t itself when the kernels can address it (row- or column-major, 16-byte aligned, leading
     dimension a multiple of 8), otherwise a copy; with `like`, a copy laid out like that tensor."""
-    t = resolved(t)
+    if t.is_neg():
+        t = resolved(t)
     if like is not None:
         lay = layout_of(like)
         mine = layout_of(t)

@@ -69,7 +69,8 @@ class MaskedDecayAdamW(Optimizer):
             raise RuntimeError("MaskedDecayAdamW: parameters must be float32 GPU tensors")
         if not (p.is_contiguous() or (p.dim() == 2 and p.t().is_contiguous())):
             raise RuntimeError("MaskedDecayAdamW: parameters must be dense in memory")
-        return {"step": torch.zeros((), dtype=torch.int64, device=p.device) if capturable else 0,
+        return {**({"negated": True} if p.is_neg() else {}),       # (updated beside, and written back through the view)
+                "step": torch.zeros((), dtype=torch.int64, device=p.device) if capturable else 0,
                 "exp_avg": torch.empty_like(p, memory_format=torch.preserve_format),       # zeroed with the others of the
                 "exp_avg_sq": torch.empty_like(p, memory_format=torch.preserve_format)}    # group, in one launch (step)
 
@@ -84,7 +85,7 @@ class MaskedDecayAdamW(Optimizer):
             lr, eps, wd, alpha = float(group["lr"]), float(group["eps"]), float(group["weight_decay"]), float(group["alpha"])
             # Everything is looked at before anything is launched; the tensors of one launch share the types of
             # gradient and mask and a host-side step count (device-side counts travel with their tensor)
-            entries, counts, launches, fresh, negated = [], [], {}, [], []
+            entries, counts, launches, fresh, negated, codes = [], [], {}, [], [], N.dtype_codes
             for p in params:
                 grad = p.grad
                 if grad is None:
@@ -101,26 +102,30 @@ class MaskedDecayAdamW(Optimizer):
                     mask = None
                 if mask is not None and (mask.stride() != stride or mask.device != p.device):
                     raise RuntimeError("MaskedDecayAdamW: mask must have the parameter's strides and device")
-                entries.append((p, N.resolved(grad), state, mask, N.dtype_code(grad.dtype), N.U8 if mask is None else N.dtype_code(mask.dtype)))
-                if torch.is_tensor(state["step"]):
-                    counts.append(state["step"])
+                if grad.is_neg():                                  # (the kernel reads and writes storage)
+                    grad = grad.resolve_neg()
+                step = state["step"]
+                on_device = type(step) is not int and torch.is_tensor(step)
+                if on_device:
+                    counts.append(step)
+                entries.append((p, grad, state, mask, codes[grad.dtype], N.U8 if mask is None else codes[mask.dtype], on_device))
             if fresh:
                 torch._foreach_zero_([state[name] for _, state in fresh for name in ("exp_avg", "exp_avg_sq")])
                 for p, state in fresh:
                     self.state[p] = state
             if counts:
                 torch._foreach_add_(counts, 1)
-            for p, grad, state, mask, grad_code, mask_code in entries:
-                step = state["step"]
-                if torch.is_tensor(step):
-                    key, step_ptr = (grad_code, mask_code, 0), step.data_ptr()
+            for p, grad, state, mask, grad_code, mask_code, on_device in entries:
+                if on_device:
+                    key, step_ptr = (grad_code, mask_code, 0), state["step"].data_ptr()
                 else:
-                    step = state["step"] = step + 1
+                    step = state["step"] = state["step"] + 1
                     key, step_ptr = (grad_code, mask_code, step), 0
                 if mask is not None:
                     p.cnt = 0
-                values = N.resolved(p)
-                if values is not p:
+                values = p
+                if "negated" in state:
+                    values = p.resolve_neg()
                     negated.append((p, values))
                 launches.setdefault(key, []).extend((values.data_ptr(), grad.data_ptr(), state["exp_avg"].data_ptr(), state["exp_avg_sq"].data_ptr(),
                                                      0 if mask is None else mask.data_ptr(), step_ptr, p.numel()))

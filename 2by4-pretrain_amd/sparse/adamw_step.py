@@ -89,7 +89,7 @@ class AdamW_STEP(Optimizer):
                 if grad.stride() != p.stride():
                     raise RuntimeError("AdamW_STEP: the gradient must have the parameter's strides")
                 state['step'] += 1
-                values, grad = N.resolved(p), N.resolved(grad)
+                values, grad = N.resolved(p), N.resolved(grad)     # (the kernel reads and writes storage)
                 tracked = hasattr(p, 'mask')
                 z_ptr, z_option, precond = None, 0, None
                 if tracked and watching:

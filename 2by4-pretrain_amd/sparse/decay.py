@@ -21,8 +21,13 @@ def masked_add_(grad: torch.Tensor, p_data: torch.Tensor, p_mask: torch.Tensor, 
     dense_in_memory = grad.is_contiguous() or (grad.dim() == 2 and grad.t().is_contiguous())
     if not dense_in_memory:
         raise RuntimeError("masked_add_: tensors must be dense in memory (contiguous in some dimension order)")
-    target, p_data = N.resolved(grad), N.resolved(p_data)
-    N.check(N.lib().tf24_masked_add(target.data_ptr(), N.dtype_code(grad.dtype), p_data.data_ptr(), N.dtype_code(p_data.dtype),
-                                    p_mask.data_ptr(), N.dtype_code(p_mask.dtype), n, float(alpha), N.stream_ptr()))
-    if target is not grad:
+    if grad.is_neg():                                # (the kernel reads and writes storage)
+        target = grad.resolve_neg()
+        masked_add_(target, p_data, p_mask, alpha)
         grad.copy_(target)
+        return
+    if p_data.is_neg():
+        p_data = p_data.resolve_neg()
+    codes = N.dtype_codes
+    N.check(N.lib().tf24_masked_add(grad.data_ptr(), codes[grad.dtype], p_data.data_ptr(), codes[p_data.dtype],
+                                    p_mask.data_ptr(), codes[p_mask.dtype], n, float(alpha), N.stream_ptr()))

@@ -209,6 +209,7 @@ _WORKSPACE_BYTES = {}      # (dtype, n, k, j) -> tf24_spmm_workspace_bytes, a pu
 def _spmm(sparse, dense, sparse_first, bias=None, out_dtype=None, scale=1.0, activation=N.ACT_NONE, keep_panel=True):
     """sparse_first: out = S @ dense  (S [n,k], dense [k,j])  -> [n, j]
        otherwise   : out = dense @ S^T (dense [j,k])          -> [j, n]
+    dense is no negated view: the dispatcher has resolved it, other callers have to.
     keep_panel: an operand that arrives in canonical or CUTLASS form is repacked to the panel form; keep
     that copy in the wrapper (the wrapper owns its tensors) or drop it after the product (the wrapper
     only borrows tensors its caller may rewrite)."""
@@ -232,7 +233,6 @@ def _spmm(sparse, dense, sparse_first, bias=None, out_dtype=None, scale=1.0, act
     # only rows with k contiguous go in any number, a count off the type's multiple with k strided.  clone: a tensor that
     # starts off such a boundary counts as contiguous.
     multiple = _DTYPE_TO_SEMI_STRUCTURED_SPARSE_CONFIG[vdtype].dense_min_rows        # elements of 16 bytes
-    dense = N.resolved(dense)
     d0, d1 = dense.shape
     s0, s1 = dense.stride()
     if d0 == 1 and s1 == 1:
@@ -280,7 +280,8 @@ def _spmm(sparse, dense, sparse_first, bias=None, out_dtype=None, scale=1.0, act
     device = dense.device
     out = torch.empty(out_shape, dtype=out_dtype, device=device)
     if bias is not None:
-        bias = N.resolved(bias)
+        if bias.is_neg():
+            bias = bias.resolve_neg()
         if bias.dtype is torch.float32 and out_dtype in _SIXTEEN_BIT and bias.is_contiguous():
             activation |= N.BIAS_F32                 # rounded where it is read
         elif bias.dtype != out_dtype or not bias.is_contiguous():
@@ -658,7 +659,9 @@ def to_sparse_semi_structured_pair(original_tensor: torch.Tensor, mask: torch.Te
     rebuilds every optimizer step (README.md:165-166).  Both results are bit-identical to the
     separate calls.  w [m, k] row-major, both dimensions a multiple of 64 (128 for float8); with
     any other input the two separate conversions run instead."""
-    w = N.resolved(original_tensor)
+    w = original_tensor
+    if w.is_neg():
+        w = N.resolved(w)
     if not w.is_cuda or w.dim() != 2 or dtype not in _DTYPE_TO_SEMI_STRUCTURED_SPARSE_CONFIG or mask is None:
         return (to_sparse_semi_structured(w, mask=mask, dtype=dtype), to_sparse_semi_structured(w.T, mask=mask.T, dtype=dtype))
     m, k = w.shape
@@ -697,7 +700,7 @@ def to_sparse_semi_structured_with_row_sums(original_tensor: torch.Tensor, MVUE2
     where the row sums are the bias gradient `grad_output.sum(0)`) both results come from one pass over
     `t`; the sums are added in float32 and rounded once to t's dtype (`sums_dtype` float32: not at all).  Any
     other input runs the conversion and torch's sum separately."""
-    t = N.resolved(original_tensor)
+    t = original_tensor
     cfg = _DTYPE_TO_SEMI_STRUCTURED_SPARSE_CONFIG.get(dtype)
     fusable = (t.is_cuda and t.dim() == 2 and cfg is not None and t.dtype in (torch.float32, torch.float16, torch.bfloat16)
                and dtype != torch.int8 and not (mask is not None and MVUE24) and SparseSemiStructuredTensor._PANEL_LAYOUT)

@@ -40,6 +40,8 @@ class sparse_linear_transpose(autograd.Function):
         compute = weight_sparse._dtype
         if input.dtype != compute:
             input = input.to(compute)
+        if input.is_neg():                           # (the kernels read storage)
+            input = input.resolve_neg()
         # a float32 bias goes to the product as it is, which rounds it to `compute` where it reads it, and gets a float32 gradient
         # (a cast either way is a launch of 3 to 5 us)
         ctx.bias_dtype = None if bias is None else bias.dtype
@@ -68,6 +70,8 @@ class sparse_linear_transpose(autograd.Function):
             grad_output = torch.ones_like(grad_output, memory_format=torch.contiguous_format)
         if grad_output.dim() != 2:
             grad_output = grad_output.reshape(-1, grad_output.shape[-1])
+        if grad_output.is_neg():
+            grad_output = grad_output.resolve_neg()
         if grad_output.stride(-1) != 1 or grad_output.stride(0) < grad_output.shape[-1]:
             grad_output = grad_output.contiguous()
         if grad_output.dtype != input.dtype:

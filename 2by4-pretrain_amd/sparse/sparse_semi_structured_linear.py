@@ -72,7 +72,7 @@ def sparse_semi_structured_linear(input: torch.Tensor, weight, meta: Optional[to
         weight = _borrowed_wrapper(weight, meta, meta_layout)
         borrowed = True
     shape = input.shape
-    x2d = input.reshape(-1, shape[-1])
+    x2d = N.resolved(input).reshape(-1, shape[-1])
     rows = x2d.shape[0]
     if x2d.dtype == weight._dtype and x2d.shape[1] == weight._store_shape[1]:
         padded = x2d                     # any number of rows
