@@ -5,7 +5,7 @@
 // G [tokens, m] and X [tokens, n] are read as they lie: the summed axis is the slow one of both.
 //
 // Bound by the matrix cores, and at this size by the power that they may draw: 12288 tokens, 3072 x 768 bf16 take 67
-// us with db (0.87 PFLOP/s; on 256 x 256 tiles 70, of zeros 54), where the library's product takes 125 to 140 us and its row sum 29.
+// us with db (0.87 PFLOP/s; on 256 x 256 tiles 70, of zeros 54), where the library's product takes 110 to 140 us and its row sum 20 to 29.
 //
 // A block multiplies a 256(i) x 256(j) tile over a piece of the token axis: eight waves (2 along i x 4 along j), two per
 // SIMD, wave tile 128 x 64 = 4 x 2 V_MFMA_F32_32X32X16.  (Four waves of 128 x 128 read a third less LDS, but nothing covers
