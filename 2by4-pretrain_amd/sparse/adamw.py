@@ -69,8 +69,7 @@ class MaskedDecayAdamW(Optimizer):
             raise RuntimeError("MaskedDecayAdamW: parameters must be float32 GPU tensors")
         if not (p.is_contiguous() or (p.dim() == 2 and p.t().is_contiguous())):
             raise RuntimeError("MaskedDecayAdamW: parameters must be dense in memory")
-        return {**({"negated": True} if p.is_neg() else {}),       # (updated beside, and written back through the view)
-                "step": torch.zeros((), dtype=torch.int64, device=p.device) if capturable else 0,
+        return {"step": torch.zeros((), dtype=torch.int64, device=p.device) if capturable else 0,
                 "exp_avg": torch.empty_like(p, memory_format=torch.preserve_format),       # zeroed with the others of the
                 "exp_avg_sq": torch.empty_like(p, memory_format=torch.preserve_format)}    # group, in one launch (step)
 
@@ -124,7 +123,7 @@ class MaskedDecayAdamW(Optimizer):
                 if mask is not None:
                     p.cnt = 0
                 values = p
-                if "negated" in state:
+                if p.is_neg():                                     # (updated beside, and written back through the view)
                     values = p.resolve_neg()
                     negated.append((p, values))
                 launches.setdefault(key, []).extend((values.data_ptr(), grad.data_ptr(), state["exp_avg"].data_ptr(), state["exp_avg_sq"].data_ptr(),
