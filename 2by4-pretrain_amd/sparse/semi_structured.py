@@ -535,15 +535,16 @@ class SparseSemiStructuredTensor(torch.Tensor):
         return NotImplemented if others else _torch_route(func, types, args, kwargs or {})
 
     # Torch's own route for the methods, without the way through __torch_function__, which is 1.2 us of host time: converting a
-    # weight of 768 x 768 and reading its values, metadata and dense form 37.0 us that way, 33.1 this way.
+    # weight of 768 x 768 and reading its values, metadata and dense form 37.0 us that way, 33.1 this way.  (A class derived from
+    # this one may have a handler of its own.)
     def t(self):
-        return _torch_route(torch.Tensor.t, (type(self),), (self,), {})
+        return _torch_route(torch.Tensor.t, (type(self),), (self,), {}) if type(self) is SparseSemiStructuredTensor else super().t()
 
     def values(self):
-        return _torch_route(torch.Tensor.values, (type(self),), (self,), {})
+        return _torch_route(torch.Tensor.values, (type(self),), (self,), {}) if type(self) is SparseSemiStructuredTensor else super().values()
 
     def indices(self):
-        return _torch_route(torch.Tensor.indices, (type(self),), (self,), {})
+        return _torch_route(torch.Tensor.indices, (type(self),), (self,), {}) if type(self) is SparseSemiStructuredTensor else super().indices()
 
     def _clone_view(self, shape, transposed):
         return SparseSemiStructuredTensor._from_storage(

@@ -285,3 +285,26 @@ def test_other_tensor_classes_meet_a_compressed_weight(monkeypatch):
                     call(x.as_subclass(Declines))
             assert torch.mm(weight, x.t().as_subclass(Handler)) == (Handler,)
             assert F.linear(x, weight, torch.ones(32).as_subclass(Handler)) == (Handler,)
+
+
+def test_derived_weights_handle_their_own_methods():
+    """A class derived from the 2:4 weights with a __torch_function__ of its own sees t, values and indices; one without has the
+    weight's."""
+    from sparse import SparseSemiStructuredTensor
+
+    class Derived(SparseSemiStructuredTensor):
+        pass
+
+    class Handles(SparseSemiStructuredTensor):
+        @classmethod
+        def __torch_function__(cls, func, types, args=(), kwargs=None):
+            return func.__name__
+
+    make = lambda cls: cls(None, torch.Size((32, 64)), sparse_tensor_cutlass=torch.ones(32, 32).half(),
+                           meta_tensor_cutlass=torch.zeros(32, 4, dtype=torch.int16))
+    handles = make(Handles)
+    assert (handles.t(), handles.values(), handles.indices()) == ("t", "values", "indices")
+    for cls in (Derived, SparseSemiStructuredTensor):
+        weight = make(cls)
+        assert weight.t().shape == (64, 32) and weight.t().transposed
+        assert weight.values().shape == (32, 32) and weight.indices().shape == (32, 4)
