@@ -67,6 +67,10 @@ __device__ __forceinline__ void store_panel_meta_block(const uint32_t* s_words, 
 //   (32 x 256 when m is not a multiple of 64): 2^lpr_shift lanes read consecutive columns of one row,
 //   the other lanes of the wave take the next rows, so that every store instruction writes, per
 //   panel, the contiguous 64-byte pieces of 4 (2) adjacent rows.
+// The magnitude rule reads and writes with ordinary accesses: a weight that it compresses is multiplied by, or taken apart
+// (values, dense form), next, and what it wrote is then still in the last cache.  float32 8192 x 8192 to fp16, compressed and
+// both taken 123.7 -> 118.0 us, 8192 x 4096 to bf16 75.9 -> 70.0; compressed alone, over and over, 59.0 and 59.1.  The other modes
+// stream: mask-driven fp32 8192 x 8192 66.1 us and 71.7 with ordinary accesses, bf16 42.0 and 45.0.
 // Rows and units of the panel form are 32-bit numbers (the grid bounds both), combined to 64-bit offsets by a
 // multiply-add: formed in 64 bits throughout, and for both forms of output in one kernel,
 // the addresses were a fifth of the MVUE24 conversion's vector instructions.
@@ -108,7 +112,8 @@ prune_compress_row(const In* __restrict__ dense, int64_t ld, int64_t m, int64_t 
     }
     if (live) {
       Pack<In, 8> in;
-      in.load_stream(dense + (uint64_t)row * ld + (uint64_t)col8 * 8);
+      if constexpr (MODE == TF24_PRUNE_MAGNITUDE) in.load(dense + (uint64_t)row * ld + (uint64_t)col8 * 8);
+      else in.load_stream(dense + (uint64_t)row * ld + (uint64_t)col8 * 8);
       Pack<MaskT, 8> mk;
       float r[4] = {0.f, 0.f, 0.f, 0.f};
       if constexpr (MODE == TF24_PRUNE_MASK) mk.load_stream(mask + (uint64_t)row * mask_ld + (uint64_t)col8 * 8);
@@ -139,7 +144,8 @@ prune_compress_row(const In* __restrict__ dense, int64_t ld, int64_t m, int64_t 
         out.v[2 * g + 1] = kept.v[1];
         mbyte |= nib << (4 * g);
       }
-      out.store_stream(values + ounit * 4);
+      if constexpr (MODE == TF24_PRUNE_MAGNITUDE) out.store(values + ounit * 4);
+      else out.store_stream(values + ounit * 4);
     }
     // 4 adjacent lanes (32 dense columns of one row) -> one metadata dword
     const uint32_t w = quad_bytes(mbyte);
@@ -249,6 +255,8 @@ prune_compress_row_mag16(const In* __restrict__ dense, int64_t ld, int64_t m, in
 // words of its quad for the 4 rows are one 16-byte piece of the [k/32][m] word matrix, stored by the quad leader
 // as it is.  (64 rows x 128 columns per block with 256-byte reads per row: 37.0 us at 8192 x 8192 bf16 -> fp16;
 // this kernel 35.5; the same without the exchange of the values, 64-byte pieces per store: 41.4.)
+// Ordinary accesses on both sides (see prune_compress_row): 35.2 -> 34.9 us, 11008 x 4096 24.8 -> 23.9; compressed and its values,
+// metadata and dense form taken 100.6 -> 95.9.
 template <typename In, typename Out>
 __global__ void __launch_bounds__(kThreads)
 prune_compress_row_mag16_panel(const In* __restrict__ dense, int64_t ld, int64_t m, int64_t k,
@@ -265,7 +273,7 @@ prune_compress_row_mag16_panel(const In* __restrict__ dense, int64_t ld, int64_t
 #pragma unroll
   for (int it = 0; it < 4; it++) {
     in[it] = u32x4{0, 0, 0, 0};
-    if (live) in[it] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(dense + (row0 + it) * ld + col8 * 8));
+    if (live) in[it] = *reinterpret_cast<const u32x4*>(dense + (row0 + it) * ld + col8 * 8);
   }
   // values: a lane's four 8-byte pieces are 64 bytes apart in the panel layout; the wave exchanges them through
   // a private LDS slice (rows padded by 128 bytes: both halves of a 64-lane read fall on all banks) so that a
@@ -309,7 +317,7 @@ prune_compress_row_mag16_panel(const In* __restrict__ dense, int64_t ld, int64_t
     Pack<Out, 4> v;
     *reinterpret_cast<piece_t*>(v.v) = s_x[wave][r * XROW + u];
     const int64_t c8 = (int64_t)blockIdx.x * 64 + u;
-    if (c8 < upr) v.store_stream(values + (((c8 / UPP) * m + row0 + r) * UPP + c8 % UPP) * 4);
+    if (c8 < upr) v.store(values + (((c8 / UPP) * m + row0 + r) * UPP + c8 % UPP) * 4);
   }
   if (live && (lane & 3) == 0)
     *reinterpret_cast<uint4*>(meta + panel_meta_offset(col8, row0, m)) = make_uint4(words[0], words[1], words[2], words[3]);
