@@ -317,13 +317,13 @@ struct TileCfgT {
   static constexpr int TI = TI_, TJ = TJ_;       // 32x32 instructions per wave
   static constexpr int WI = 32 * TI, WJ = 32 * TJ;
   static constexpr int BI = WI * WAVES_I, BJ = WJ * WAVES_J;
-  static_assert((BI == 256 && (BJ == 256 || BJ == 192 || BJ == 128 || BJ == 64)) || (BI == 192 && BJ == 192),
-                "stage buffers are sized for 256-row tiles of 256, 192, 128 or 64 columns and for 192 x 192 tiles");
+  static_assert((BI == 256 && (BJ == 256 || BJ == 192 || BJ == 128 || BJ == 64)) || (BJ == 192 && (BI == 192 || BI == 384)),
+                "stage buffers are sized for 256-row tiles of 256, 192, 128 or 64 columns and for 192-column tiles of 192 or 384 rows");
   static constexpr int KB = 128;                 // bytes of dense k per row per stage
   static constexpr int STEPS = KB / 64;          // instruction steps per stage
   static constexpr int A_ROW = KB / 2;           // LDS bytes per row per stage: compressed values
   static constexpr int B_ROW = KB;               //                              dense operand
-  static constexpr int GH = 8;                   // raster group height in tiles along i
+  static constexpr int GH = BI == 384 ? 6 : 8;   // raster group height in tiles along i
   static constexpr int NB = BJ * B_ROW / 1024 / NW;   // 1 KB copies per wave per stage: B
   static constexpr int NA = BI * A_ROW / 1024 / NW;   //                                 A values
 };
@@ -353,6 +353,14 @@ using Wave4Cfg192 = TileCfgT<2, 3>;
 // Two stage buffers and two workgroups to a compute unit (76 KB and 256 registers each) instead of three buffers and
 // chained tiles: 36.2 and 35.9 us for the first, 52.0 and 41.8 for the second.
 using SquareCfg = TileCfgT<2, 3, 3>;
+// 384 x 192 tiles in the 4-wave form (wave tile 192 x 96, 288 accumulators; 16-bit operands: the stage buffers of 8-bit ones do
+// not fit): 1.125 of the work of a 256 x 256 tile, for products whose tiles of the other sizes leave much of their last round of the
+// compute units empty (takes_tall).  At equally full rounds it takes what 256 x 256 tiles take (8192 x 8192 against 8192 columns,
+// four rounds of either, 518 and 497 us).  us on the other tiles and on these, fp16: 11008 x 4096 against 8192 columns 358 -> 346
+// (5.4 rounds -> 4.9), 6144 x 12288 against 3000 251 -> 205 (three rounds of 192 x 192 tiles -> one), 6144 x 8192 against 6144
+// 320 -> 280, 6144 x 3072 against 3000 64.9 -> 57.0, 1536 x 4096 against 12288 98 -> 77.  Raster groups of 5, 6 and 8 tiles: 346, 348
+// and 349 us for the first product, 342, 342 and 346 for 10752 x 4096 against 8192.
+using TallCfg = TileCfgT<2, 3, 6>;
 constexpr int kWave4MinStages = 32;
 constexpr int kRotateMinStages = 56;
 static_assert(kRotateMinStages - 2 - (7 * kRotateMinStages >> 3) >= 1, "the first three stages of a tile are copied before the order wraps");
@@ -1185,15 +1193,42 @@ inline bool takes_square(int64_t n_sparse, int64_t n_dense, int stages, TileRows
 // those, where there are more of them than compute units (chained), 256 x 192 or 192 x 192 ones (16-bit results).
 // 256 x 192 also where both widths fit one round and the narrow tiles spread over more compute units (W[768, 3072] against
 // 12288 tokens: 144 wide tiles or 192 narrow ones, 36.1 -> 34.1 us; W[1024, 4096]: 192 or 256 tiles, 56.2 -> 53.9 us).
-enum class Tiles { WIDE8, WIDE4, NARROW4, SQUARE4 };
-inline Tiles choose_tiles(int64_t n_sparse, int64_t n_dense, int stages, TileRows wide, bool results16, int cu_slots) {
-  if (cu_slots <= 0 || stages < 4) return Tiles::WIDE8;
+enum class Tiles { WIDE8, WIDE4, NARROW4, SQUARE4, TALL4 };
+inline Tiles choose_without_tall(int64_t n_sparse, int64_t n_dense, int stages, TileRows wide, bool results16, int cu_slots) {
   if (results16 && takes_square(n_sparse, n_dense, stages, wide, cu_slots)) return Tiles::SQUARE4;
   if (stages < kWave4MinStages) return Tiles::WIDE8;
   const int64_t tiles = wide.tiles_i * ((n_dense + TiledCfg::BJ - 1) / TiledCfg::BJ), narrow = wide.tiles_i * ((n_dense + Wave4Cfg192::BJ - 1) / Wave4Cfg192::BJ);
   const int64_t rounds = tile_rounds(tiles, cu_slots), narrow_rounds = tile_rounds(narrow, cu_slots);
   if (results16 && narrow_rounds <= rounds && (narrow_rounds > 1 || (narrow + 7) / 8 > (tiles + 7) / 8)) return Tiles::NARROW4;
   return rounds > 1 ? Tiles::WIDE4 : Tiles::WIDE8;
+}
+
+// Whether it takes 384 x 192 tiles instead of the form chosen among the others: the same estimate of both (0.98 us a stage and 5 us
+// for a round of these tiles, 1.12 a stage at the sustained clock), from kTallMinStages stages on.  Of 110 fp16 products of 10 to 168
+// stages, 960 to 12224 rows and 1237 to 15757 columns on operands that change from product to product, 13 take them, all 2 to 28 %
+// faster that way (1120 x 2816 against 14480 columns 69.9 -> 54.8, 2912 x 5824 against 12074 244 -> 200, 10624 x 3264 against 3385
+// 132 -> 117); of the others none would be more than 5 % faster.  Of 70 others, a third with bias, half of them bf16, 12
+// take them, 1 to 25 % faster.  With fewer stages a tile's prologue and output pass are what a
+// round costs and two waves a SIMD hide them better (5280 x 768 against 8114 46.8 on 256 x 256 tiles, 59.5).
+constexpr int kTallMinStages = 24;
+inline bool takes_tall(int64_t n_sparse, int64_t n_dense, int stages, TileRows wide, Tiles form, int cu_slots) {
+  if (stages < kTallMinStages) return false;
+  auto us = [&](int64_t tiles, double of_round, double sustained) {
+    return std::max((double)tile_rounds(tiles, cu_slots) * of_round, (double)tiles / (8 * cu_slots) * sustained * stages);
+  };
+  auto columns = [&](int64_t width) { return (n_dense + width - 1) / width; };
+  auto rows = [&](int64_t height) { return (n_sparse + height - 1) / height; };
+  double other;
+  if (form == Tiles::SQUARE4) other = us(rows(SquareCfg::BI) * columns(SquareCfg::BJ), 0.53 * stages + 5.0, 0.67);
+  else if (form == Tiles::NARROW4) other = us(rows(Wave4Cfg192::BI) * columns(Wave4Cfg192::BJ), 0.69 * stages + 2.0, 0.75);
+  else other = us(wide.tiles_i * columns(TiledCfg::BJ), stages >= kWave4MinStages ? 0.93 * stages + 2.5 : 0.84 * stages + 5.5, 1.0) +
+               (wide.tail_rows ? 0.5 * stages + 5.0 : 0.0);
+  return us(rows(TallCfg::BI) * columns(TallCfg::BJ), 0.98 * stages + 5.0, 1.12) < 0.98 * other;
+}
+inline Tiles choose_tiles(int64_t n_sparse, int64_t n_dense, int stages, TileRows wide, bool results16, int cu_slots, bool operands16 = false) {
+  if (cu_slots <= 0 || stages < 4) return Tiles::WIDE8;
+  const Tiles form = choose_without_tall(n_sparse, n_dense, stages, wide, results16, cu_slots);
+  return results16 && operands16 && takes_tall(n_sparse, n_dense, stages, wide, form, cu_slots) ? Tiles::TALL4 : form;
 }
 
 // Whether a product with k strided does: the pieces that either tile would be cut into, estimated as choose_pieces does and
@@ -1269,7 +1304,7 @@ int launch_tiled(const void* av, const void* am, int64_t n_sparse, int64_t k, co
   const int stagger = !persist ? 0 : k * (int64_t)sizeof(T) / C::KB <= 32 ? (sizeof(OutT) == 2 ? 300 : 600)
                                : (sizeof(OutT) == 4 && stagger_rounds >= 3) ? 600 : 0;
   const Tiles form = std::is_same<C, TiledCfg>::value && jm && b_layout == TF24_ROW_MAJOR && splits == 1
-                         ? choose_tiles(n_sparse, n_dense, stages, {tiles_i, tail_rows}, sizeof(OutT) == 2, cu_slots) : Tiles::WIDE8;
+                         ? choose_tiles(n_sparse, n_dense, stages, {tiles_i, tail_rows}, sizeof(OutT) == 2, cu_slots, sizeof(T) == 2) : Tiles::WIDE8;
   auto launch_tail = [&]() {                       // the rows behind the full rounds, on 256 x 128 tiles
     if constexpr (std::is_same<C, TiledCfg>::value) {
       if (tail_rows > 0) {
@@ -1299,6 +1334,12 @@ int launch_tiled(const void* av, const void* am, int64_t n_sparse, int64_t k, co
       const int ti = (int)((n_sparse + SquareCfg::BI - 1) / SquareCfg::BI), tj = (int)((n_dense + SquareCfg::BJ - 1) / SquareCfg::BJ);
       either(SquareCfg{}, ti, tj, tile_rounds((int64_t)ti * tj, cu_slots) > 1 && stages <= 32 ? 300 : 0);
       return check_launch("tf24_spmm");
+    }
+    if constexpr (sizeof(T) == 2) {
+      if (form == Tiles::TALL4) {
+        either(TallCfg{}, (int)((n_sparse + TallCfg::BI - 1) / TallCfg::BI), (int)((n_dense + TallCfg::BJ - 1) / TallCfg::BJ), 0);
+        return check_launch("tf24_spmm");
+      }
     }
     if (form == Tiles::NARROW4) {
       either(Wave4Cfg192{}, tiles_i, (int)((n_dense + Wave4Cfg192::BJ - 1) / Wave4Cfg192::BJ), stagger);

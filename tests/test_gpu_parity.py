@@ -1329,6 +1329,23 @@ def test_linear_square_tiles(cuda, dtype, n, stages, rows, activation):
     assert sparse.sparse_semi_structured_linear(x, s, bias=bias, out_dtype=out_dtype, activation=activation).equal(act(want + bias.float()).to(out_dtype))
 
 
+TALL = [
+    (1504, 24, 11707, False),       # one round, the fewest stages; partial tiles on either edge
+    (1120, 44, 14480, False),       # the last of three tile rows reaches 32 rows past its first wave
+    (3872, 45, 8535, False),        # two rounds
+    (2912, 58, 12074, True)]        # from another eighth of k on each XCD
+NOT_TALL = [                        # on the tiles of the cases above that 16-bit operands leave for tall ones
+    (1568, 33, 9867, "square"), (1568, 66, 9867, "square"), (3104, 59, 10790, "wide, two launches")]
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("n,stages,rows", [case[:3] for case in TALL + NOT_TALL])
+@pytest.mark.parametrize("activation", [None, "relu"])
+def test_linear_tall_tiles(cuda, dtype, n, stages, rows, activation):
+    """Products on 384 x 192 tiles, with and without bias: exact on small integers."""
+    test_linear_square_tiles(cuda, dtype, n, stages, rows, activation)
+
+
 SQUARE_STRIDED = [                  # and in how many pieces of k (test_tile_rules.py)
     (64, 4, 72, 1), (224, 5, 200, 1), (192, 9, 192, 3), (352, 25, 2376, 3), (416, 8, 560, 1),         # tiles past either edge
     (992, 40, 392, 5), (544, 117, 120, 15), (3072, 48, 768, 2), (3424, 202, 80, 11)]

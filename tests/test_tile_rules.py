@@ -6,7 +6,7 @@ import subprocess
 
 import pytest
 
-from test_gpu_parity import SQUARE, SQUARE_STRIDED, STAGE_ORDER
+from test_gpu_parity import NOT_TALL, SQUARE, SQUARE_STRIDED, STAGE_ORDER, TALL
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 CU_SLOTS = 32                      # compute units of an XCD
@@ -37,12 +37,17 @@ extern "C" int strided(int64_t n_sparse, int64_t n_dense, int stages, int result
 extern "C" int strided_pieces(int64_t n_sparse, int64_t n_dense, int stages) {
   return tf24::choose_pieces<tf24::f16_t, tf24::SquareCfg>(n_sparse, (int64_t)stages * 64, n_dense, (int64_t)1 << 40, true).count;
 }
+extern "C" int tiles_of_16_bits(int64_t n_sparse, int64_t n_dense, int stages, int cu_slots) {
+  const tf24::TileRows rows = tf24::full_rounds(n_sparse, n_dense, stages, cu_slots);
+  return (int)tf24::choose_tiles(n_sparse, n_dense, stages, rows, true, cu_slots, true) + (rows.tail_rows ? 100 : 0);
+}
 extern "C" int rotate_from() { return tf24::kRotateMinStages; }
 """)
     subprocess.run([build.HIPCC, *build.FLAGS, "--offload-host-only", "-shared", str(src), "-o", str(lib)], check=True, capture_output=True)
     handle = ctypes.CDLL(str(lib))
     handle.square.argtypes = [ctypes.c_int64, ctypes.c_int64, ctypes.c_int, ctypes.c_int]
     handle.tiles.argtypes = [ctypes.c_int64, ctypes.c_int64, ctypes.c_int, ctypes.c_int, ctypes.c_int]
+    handle.tiles_of_16_bits.argtypes = [ctypes.c_int64, ctypes.c_int64, ctypes.c_int, ctypes.c_int]
     handle.strided.argtypes = [ctypes.c_int64, ctypes.c_int64, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int]
     handle.strided_pieces.argtypes = [ctypes.c_int64, ctypes.c_int64, ctypes.c_int]
     return handle
@@ -73,3 +78,17 @@ def test_k_strided_products_tested_on_the_gpu_take_square_tiles(rules, n, stages
     # with float32 results and with 16-bit ones stored j-major; i-major ones only where a reduction writes them
     forms = [rules.strided(n, columns, stages, results16, jmajor, CU_SLOTS) for results16, jmajor in ((0, 0), (1, 1), (1, 0))]
     assert forms == [1, 1, int(pieces > 1)]
+
+
+@pytest.mark.parametrize("n,stages,columns,tall", [
+    # measured apart (us on the other tiles, on 384 x 192 ones)
+    (1120, 44, 14480, 1), (1504, 30, 11707, 1), (2912, 91, 12074, 1), (11008, 64, 8192, 1),            # 69.9 54.8, 53.1 42.3, 244 200, 358 346
+    (8192, 128, 8192, 0), (5280, 12, 8114, 0), (1312, 161, 13869, 0), (11776, 35, 1599, 0)]            # 497 518, 46.8 59.5, 231 288, 54.3 70.4
+    + [(n, stages, rows, 1) for n, stages, rows, _ in TALL])
+def test_tall_tiles_where_they_are_the_faster_ones(rules, n, stages, columns, tall):
+    assert (rules.tiles_of_16_bits(n, columns, stages, CU_SLOTS) % 100 == 4) == tall
+
+
+@pytest.mark.parametrize("n,stages,rows,tiles", NOT_TALL)
+def test_other_tiles_are_tested_with_16_bits_too(rules, n, stages, rows, tiles):
+    assert rules.tiles_of_16_bits(n, rows, stages, CU_SLOTS) == {"wide, two launches": 101, "square": 3}[tiles]
