@@ -119,8 +119,9 @@ prune_compress_row(const In* __restrict__ dense, int64_t ld, int64_t m, int64_t 
       if constexpr (MODE == TF24_PRUNE_MASK) mk.load_stream(mask + (uint64_t)row * mask_ld + (uint64_t)col8 * 8);
       if constexpr (MODE == TF24_PRUNE_MVUE) {
         if (rs.kind == RAND_SEEDED) {
-          const Philox4 c = philox4x32_10(rs.seed_now(), (uint64_t)row * upr + col8, rs.offset_now());
-          r[0] = philox_uniform(c.x); r[1] = philox_uniform(c.y); r[2] = philox_uniform(c.z); r[3] = philox_uniform(c.w);
+          Philox4 c[1];
+          philox4x32_10_calls(rs.seed_now(), (uint64_t)row * upr + col8, 0, rs.offset_now(), c);
+          r[0] = philox_uniform(c[0].x); r[1] = philox_uniform(c[0].y); r[2] = philox_uniform(c[0].z); r[3] = philox_uniform(c[0].w);
         } else if (rs.kind == RAND_PACKED) {                   // [m, k/2]: the unit's four uniforms are adjacent
           Pack<float, 4> r4;
           r4.load_stream(rs.ptr + (uint64_t)row * rs.ld + (uint64_t)col8 * 4);
@@ -162,6 +163,61 @@ prune_compress_row(const In* __restrict__ dense, int64_t ld, int64_t m, int64_t 
     const int rows = kUnroll * (kThreads >> lpr_shift);
     store_panel_meta_block(s_words, rows, 1 << (lpr_shift - 2), (int64_t)blockIdx.y * rows, (int64_t)blockIdx.x << lpr_shift, upr, m, meta);
   }
+}
+
+// MVUE24 into the PANEL layout: the work assignment of prune_compress_row, one unit per lane.  Bound by the vector instructions of a
+// unit (377 in prune_compress_row, 340 here, about 2.6 cycles each with eight waves on a SIMD, whatever their kind): rows
+// and units are counted inside the block, whose corner is formed in scalar registers, and the quad leaders store their metadata words themselves,
+// which in the other modes, bound by memory, costs more than the way through LDS (see store_panel_meta_block).
+template <typename In, typename Out>
+__global__ void __launch_bounds__(kThreads)
+prune_compress_row_mvue_panel(const In* __restrict__ dense, int64_t ld, int64_t m, int64_t k, RandSrc rs,
+                              Out* __restrict__ values, uint8_t* __restrict__ meta, int lpr_shift) {
+  constexpr uint32_t UPP = (128 / (uint32_t)sizeof(Out)) / 8;     // units per panel row (8 or 16)
+  const uint32_t upr = (uint32_t)(k >> 3), rows = kThreads >> lpr_shift;
+  const uint32_t row0 = blockIdx.y * rows, unit0 = blockIdx.x << lpr_shift;
+  const uint32_t row = threadIdx.x >> lpr_shift, unit = threadIdx.x & ((1u << lpr_shift) - 1u);        // in the block
+  if (unit >= upr - unit0) return;               // (whole quads: upr is a multiple of 8)
+  // the place of (row, unit) where a row of the matrix is `pitch` long and a unit of it `per_unit`: for the lane one multiply-add with
+  // the low word of the pitch (the high word, which only absurdly wide matrices have, in a branch)
+  auto place = [&](uint64_t pitch, uint32_t per_unit) {
+    uint64_t at = (uint64_t)row * (uint32_t)pitch + unit * per_unit;
+    if (pitch >> 32) at += (uint64_t)(row * (uint32_t)(pitch >> 32)) << 32;
+    return (uint64_t)row0 * pitch + (uint64_t)unit0 * per_unit + at;
+  };
+  Pack<In, 8> in;
+  in.load_stream(dense + place((uint64_t)ld, 8));
+  float r[4];
+  if (rs.kind == RAND_SEEDED) {
+    Philox4 c[1];
+    philox4x32_10_calls(rs.seed_now(), place(upr, 1), 0, rs.offset_now(), c);
+    r[0] = philox_uniform(c[0].x); r[1] = philox_uniform(c[0].y); r[2] = philox_uniform(c[0].z); r[3] = philox_uniform(c[0].w);
+  } else if (rs.kind == RAND_PACKED) {           // [m, k/2]: the unit's four uniforms are adjacent
+    Pack<float, 4> r4;
+    r4.load_stream(rs.ptr + place((uint64_t)rs.ld, 4));
+    r[0] = r4.v[0]; r[1] = r4.v[1]; r[2] = r4.v[2]; r[3] = r4.v[3];
+  } else {
+    const float* rp = rs.ptr + place((uint64_t)rs.ld, 8);
+    Pack<float, 2> ra, rb;                       // the group's two uniforms: the second load meets the first one's line in L1
+    ra.load(rp);
+    rb.load(rp + 4);
+    r[0] = ra.v[0]; r[1] = ra.v[1]; r[2] = rb.v[0]; r[3] = rb.v[1];
+  }
+  Mvue4 g[2];
+  bool finite[2];
+#pragma unroll
+  for (int i = 0; i < 2; i++) {
+    float x[4];
+#pragma unroll
+    for (int e = 0; e < 4; e++) x[e] = to_float(in.v[4 * i + e]);
+    g[i] = mvue4<In>(x, r[2 * i], r[2 * i + 1], finite[i]);
+  }
+  // (offsets inside the block fit 32 bits: the grid bounds the rows to two million)
+  Out* to = values + ((uint64_t)(unit0 / UPP) * (uint64_t)m + row0) * (UPP * 4) + ((unit / UPP) * ((uint32_t)m * (UPP * 4)) + row * (UPP * 4) + unit % UPP * 4);
+  from_float4<Out>(g[0].first, g[0].second, finite[0], g[1].first, g[1].second, finite[1]).store_stream(to);
+  const uint32_t w = quad_bytes(g[0].nibble | (g[1].nibble << 4));
+  if ((threadIdx.x & 3) == 0)
+    *reinterpret_cast<uint32_t*>(meta + ((uint64_t)(unit0 >> 2) * (uint64_t)m + row0) * 4 + ((unit >> 2) * ((uint32_t)m * 4) + row * 4)) = w;
 }
 
 // Magnitude mode on 16-bit floats (the weight conversions of the configs): same work assignment and
@@ -371,11 +427,12 @@ prune_compress_col(const In* __restrict__ dense, int64_t ld, int64_t m, int64_t 
       if (rs.kind == RAND_SEEDED) {
         const uint64_t seed = rs.seed_now(), offset = rs.offset_now();
         const uint64_t index = (uint64_t)r0 * (uint64_t)(k >> 3) + (uint64_t)(c0 >> 3);
+        Philox4 c[R];
+        philox4x32_10_calls(seed, index, (uint64_t)(k >> 3), offset, c);
 #pragma unroll
         for (int i = 0; i < R; i++) {
-          const Philox4 c = philox4x32_10(seed, index + (uint64_t)i * (uint64_t)(k >> 3), offset);
-          rr[0].v[i] = philox_uniform(c.x); rr[1].v[i] = philox_uniform(c.y);
-          rr[2].v[i] = philox_uniform(c.z); rr[3].v[i] = philox_uniform(c.w);
+          rr[0].v[i] = philox_uniform(c[i].x); rr[1].v[i] = philox_uniform(c[i].y);
+          rr[2].v[i] = philox_uniform(c[i].z); rr[3].v[i] = philox_uniform(c[i].w);
         }
       } else {
         // packed: columns 2g, 2g+1 of a [m, k/2] tensor; full: columns 4g, 4g+1 of a [m, k] one
@@ -527,12 +584,17 @@ int launch(const void* dense, int layout, int64_t ld, int64_t m, int64_t k, cons
       }
       hipLaunchKernelGGL((prune_compress_row_mag16<In, Out>), grid, dim3(kThreads), 0, stream,
                          (const In*)dense, ld, m, k, (Out*)values, (uint8_t*)meta, contiguous, panel, lpr_shift);
+    } else if (MODE == TF24_PRUNE_MVUE && panel) {
+      if constexpr (MODE == TF24_PRUNE_MVUE)
+        hipLaunchKernelGGL((prune_compress_row_mvue_panel<In, Out>), grid, dim3(kThreads), 0, stream, (const In*)dense, ld, m, k, rs, (Out*)values, (uint8_t*)meta, lpr_shift);
     } else {
       auto go = [&](auto to_panel) {
         hipLaunchKernelGGL((prune_compress_row<In, Out, MODE, MaskT, decltype(to_panel)::value>), grid, dim3(kThreads), 0, stream,
                            (const In*)dense, ld, m, k, (const MaskT*)mask, mask_ld, rs, (Out*)values, (uint8_t*)meta, contiguous, lpr_shift);
       };
-      if (panel) go(std::true_type{}); else go(std::false_type{});
+      if constexpr (MODE == TF24_PRUNE_MVUE) go(std::false_type{});
+      else if (panel) go(std::true_type{});
+      else go(std::false_type{});
     }
   } else {
     constexpr int TR = 128 / sizeof(In);       // rows of a block's tile

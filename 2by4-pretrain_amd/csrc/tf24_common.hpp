@@ -219,13 +219,13 @@ struct Pack {
   }
 };
 
-// The bytes of 4 adjacent lanes as one word, lane 0's lowest (in every lane of the quad that matters, the first): data
-// parallel primitives move them between lanes without the LDS round trip of a shuffle.
+// The bytes of 4 adjacent lanes (of a one-dimensional block) as one word, lane 0's lowest, in each of them: data parallel primitives
+// move them between lanes without the LDS round trip of a shuffle.
 __device__ __forceinline__ uint32_t quad_bytes(uint32_t b) {
-  const uint32_t b1 = (uint32_t)__builtin_amdgcn_mov_dpp((int)b, 0x55, 0xf, 0xf, true);      // quad_perm [1,1,1,1]
-  const uint32_t b2 = (uint32_t)__builtin_amdgcn_mov_dpp((int)b, 0xaa, 0xf, 0xf, true);      // [2,2,2,2]
-  const uint32_t b3 = (uint32_t)__builtin_amdgcn_mov_dpp((int)b, 0xff, 0xf, 0xf, true);      // [3,3,3,3]
-  return b | (b1 << 8) | (b2 << 16) | (b3 << 24);
+  uint32_t w = b << (8 * (threadIdx.x & 3));
+  w |= (uint32_t)__builtin_amdgcn_mov_dpp((int)w, 0xb1, 0xf, 0xf, true);      // quad_perm [1,0,3,2]
+  w |= (uint32_t)__builtin_amdgcn_mov_dpp((int)w, 0x4e, 0xf, 0xf, true);      // [2,3,0,1]
+  return w;
 }
 // the value of the lane 8 away inside its row of 16 (row_ror:8)
 __device__ __forceinline__ uint32_t xor8_lane(uint32_t v) { return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x128, 0xf, 0xf, true); }
@@ -346,6 +346,29 @@ __host__ __device__ inline Philox4 philox4x32_10(uint64_t seed, uint64_t index, 
   }
   return Philox4{c0, c1, c2, c3};
 }
+// The calls for the counters index, index + stride, ... of one lane, with three-input exclusive ors (v_bitop3_b32): 40 + 2
+// vector instructions a call instead of 58, which is what kernels that sample are bound by (see mvue4).
+template <int N>
+__device__ __forceinline__ void philox4x32_10_calls(uint64_t seed, uint64_t index, uint64_t stride, uint64_t offset, Philox4 (&out)[N]) {
+  uint32_t k0 = (uint32_t)seed, k1 = (uint32_t)(seed >> 32);
+#pragma unroll
+  for (int i = 0; i < N; i++) {
+    const uint64_t at = index + (uint64_t)i * stride;
+    out[i] = Philox4{(uint32_t)at, (uint32_t)(at >> 32), (uint32_t)offset, (uint32_t)(offset >> 32)};
+  }
+#pragma unroll
+  for (int round = 0; round < 10; round++) {
+#pragma unroll
+    for (int i = 0; i < N; i++) {
+      const uint64_t p0 = (uint64_t)0xD2511F53u * out[i].x, p1 = (uint64_t)0xCD9E8D57u * out[i].z;
+      const uint32_t h0 = (uint32_t)(p0 >> 32), h1 = (uint32_t)(p1 >> 32);
+      if (round == 0) out[i] = Philox4{out[i].y ^ (h1 ^ k0), (uint32_t)p1, h0 ^ (out[i].w ^ k1), (uint32_t)p0};   // (the offset's words are the same in all lanes)
+      else out[i] = Philox4{(uint32_t)__builtin_amdgcn_bitop3_b32(h1, out[i].y, k0, 0x96), (uint32_t)p1,
+                            (uint32_t)__builtin_amdgcn_bitop3_b32(h0, out[i].w, k1, 0x96), (uint32_t)p0};
+    }
+    k0 += 0x9E3779B9u; k1 += 0xBB67AE85u;
+  }
+}
 // 24 random bits -> [0, 1), exact in float32
 __host__ __device__ inline float philox_uniform(uint32_t bits) { return (float)(bits & 0xffffffu) * 5.9604644775390625e-8f; }
 
@@ -372,7 +395,7 @@ struct Mvue4 {
 // FAST: every division through div_in_range, in straight-line code; `ok` says whether the bounds of div_in_range held
 // throughout (if not, the result is not to be used).  |x_i| + eps >= 2^-23 always, so with sum < 2^40 and every
 // s_i = sum - a_i > 0 (then s_i >= 2^-46) the quotients t_i = a_i/sum >= 2^-63 and k_i = t_i/s_i >= 2^-104 meet them;
-// p_i >= t_i because k >= k_i for a rounded sum of non-negatives, so p_i in [2^-63, 2] once it is at most 2, and
+// p_i >= t_i because k >= k_i for a rounded sum of non-negatives, so p_i in [2^-63, 4] once two of them add up to at most 4, and
 // |x_i| <= sum p_i keeps the exponents within 96 of each other; |x_i| >= 2^-100 or x_i = 0 keeps the quotient normal or
 // zero.  (Half precision, WIDE = false, holds neither a sum of 2^40 nor a value below 2^-100.)
 template <bool FAST, bool WIDE>
@@ -395,17 +418,20 @@ __device__ __forceinline__ Mvue4 mvue4_as(const float (&x)[4], float r0, float r
   }
   const float k = ((k0 + k1) + k2) + k3;
   const float p0 = t0 + a0 * (k - k0), p1 = t1 + a1 * (k - k1), p2 = t2 + a2 * (k - k2), p3 = t3 + a3 * (k - k3);
-  const bool m0 = r0 <= t0;
-  const bool m1 = r0 <= (t0 + t1) && !m0;
-  const bool m2 = r0 <= ((t0 + t1) + t2) && !m1 && !m0;
-  const bool m3 = !m2 && !m1 && !m0;
-  const float d0 = m0 ? 0.0f : a0, d1 = m1 ? 0.0f : a1, d2 = m2 ? 0.0f : a2, d3 = m3 ? 0.0f : a3;
+  // (FAST: no term is negative, nor a NaN unless `ok` fails, so each compare implies the next one, and "this and none before" is
+  // where two neighbours differ; a condition that is used negated as well costs a second compare)
+  const bool m0 = r0 <= t0, upto1 = r0 <= (t0 + t1), upto2 = r0 <= ((t0 + t1) + t2);
+  const bool m1 = FAST ? upto1 != m0 : upto1 && !m0;
+  const bool m2 = FAST ? upto2 != upto1 : upto2 && !m1 && !m0;
+  const bool m3 = FAST ? !upto2 : !m2 && !m1 && !m0;
+  const float d0 = m0 ? 0.0f : a0, d1 = m1 ? 0.0f : a1, d2 = m2 ? 0.0f : a2;
+  const float d3 = FAST ? (upto2 ? a3 : 0.0f) : (m3 ? 0.0f : a3);
   const float dsum = ((d0 + d1) + d2) + d3;
   const float t = r1 * dsum;
-  const bool e0 = t <= d0;
-  const bool e1 = t <= (d0 + d1) && !e0;
-  const bool e2 = t <= ((d0 + d1) + d2) && !e1 && !e0;
-  const bool e3 = !e2 && !e1 && !e0;
+  const bool e0 = t <= d0, to1 = t <= (d0 + d1), to2 = t <= ((d0 + d1) + d2);
+  const bool e1 = FAST ? to1 != e0 : to1 && !e0;
+  const bool e2 = FAST ? to2 != to1 : to2 && !e1 && !e0;
+  const bool e3 = FAST ? !to2 : !e2 && !e1 && !e0;
   const Keep4 keep{m0 || e0, m1 || e1, m2 || e2, m3 || e3};
   const float xa = keep.first(x[0], x[1], x[2]), xb = keep.second(x[1], x[2], x[3]);
   const float pa = keep.first(p0, p1, p2), pb = keep.second(p1, p2, p3);
@@ -419,12 +445,12 @@ __device__ __forceinline__ Mvue4 mvue4_as(const float (&x)[4], float r0, float r
     g.first = __builtin_fmaf(-__builtin_fmaf(pa, qa, -xa), ra, qa);
     g.second = __builtin_fmaf(-__builtin_fmaf(pb, qb, -xb), rb, qb);
     // an s_i of zero (they are never negative) makes its reciprocal, k and with it every p a NaN: no test of its own
-    ok = pa <= 2.0f && pb <= 2.0f;
+    ok = pa + pb <= 4.0f;
     if constexpr (WIDE) {        // In can hold what half precision cannot: a sum of 2^40, values below 2^-100
       ok = ok && sum < 0x1p40f;
-      // 0 or at least 2^-100 (0x0d800000), for both: one less than zero wraps round
-      const uint32_t ua = (__builtin_bit_cast(uint32_t, xa) & 0x7fffffffu) - 1u, ub = (__builtin_bit_cast(uint32_t, xb) & 0x7fffffffu) - 1u;
-      ok = ok && (ua < ub ? ua : ub) >= 0x0d800000u - 1u;
+      // 0 or at least 2^-100 (0x0d800000), for both, twice without the sign: one less than zero wraps round
+      const uint32_t ua = (__builtin_bit_cast(uint32_t, xa) << 1) - 1u, ub = (__builtin_bit_cast(uint32_t, xb) << 1) - 1u;
+      ok = ok && (ua < ub ? ua : ub) >= 2u * 0x0d800000u - 1u;
     }
   } else {
     g.first = xa / pa;
@@ -434,14 +460,17 @@ __device__ __forceinline__ Mvue4 mvue4_as(const float (&x)[4], float r0, float r
   return g;
 }
 
-// What bounds the kernels that call this, when the uniforms are drawn in the kernel, is the vector ALU.  Rates measured
-// on gfx950, in lanes per clock of the chip: float32 add, multiply, fma and the bitwise operations 32768; compares,
-// selects, minima, shifts, conversions and 32-bit multiplies 16384; v_rcp_f32 8192.  In units of the middle rate a group
-// costs 80 (half precision) to 85, a generator call 50 for two groups.  One correction per division instead of two, no
+// What bounds the kernels that call this, when the uniforms are drawn in the kernel, is the number of their vector instructions:
+// with eight waves on a SIMD one issues every 2.6 cycles on average (counters of an 8192 x 8192 conversion), and although by
+// themselves float32 arithmetic and bitwise operations issue at up to twice the rate of compares, selects, minima and conversions, and
+// at half of it with an operand in a scalar register, a mixture follows the count (keys and constants moved to vector registers
+// for the faster rate, one instruction more each: no gain).  A group costs 116 of them, a generator call 42 for two groups.  One correction per division instead of two, no
 // branch and one test of the bounds per group (the slow path is laid out behind the kernel), flags as short-circuit
 // expressions (as integers they went through vector registers), kept values converted without a test for NaN, and leaner
 // addresses in the callers: 8192 x 8192 bf16 to e4m3 82 -> 64.5 us, to fp16 78.6 -> 64.5 (with a supplied tensor its
 // 268 MB are the bound: 80 us before and after), a column-major 3072 x 12288 half matrix with its row sums 54.5 -> 44 us.
+// Three-input exclusive ors, six compares instead of nine and a kernel of its own for panel output, on another card: 60.5 -> 54.9,
+// 61.5 -> 57.0 and 37.1 -> 36.1.
 template <typename In>
 __device__ __forceinline__ Mvue4 mvue4(const float (&x)[4], float r0, float r1, bool& finite) {
   bool ok;
@@ -465,6 +494,25 @@ __device__ __forceinline__ Pack<Out, 2> from_float2(float a, float b, bool finit
   } else {
     o.v[0] = from_float<Out>(a);
     o.v[1] = from_float<Out>(b);
+  }
+  return o;
+}
+
+// Four values, two of either group; 8-bit types in one word, the second pair converted into its upper half.
+template <typename Out>
+__device__ __forceinline__ Pack<Out, 4> from_float4(float a0, float b0, bool finite0, float a1, float b1, bool finite1) {
+  Pack<Out, 4> o;
+  if constexpr (std::is_same<Out, e4m3_t>::value || std::is_same<Out, e5m2_t>::value) {
+    int w;
+    asm("" : "=v"(w));                           // (what the conversions leave alone is written by the other one)
+    if constexpr (std::is_same<Out, e4m3_t>::value) w = __builtin_amdgcn_cvt_pk_fp8_f32(a1, b1, __builtin_amdgcn_cvt_pk_fp8_f32(a0, b0, w, false), true);
+    else w = __builtin_amdgcn_cvt_pk_bf8_f32(a1, b1, __builtin_amdgcn_cvt_pk_bf8_f32(a0, b0, w, false), true);
+    if (__builtin_expect(!(finite0 && finite1), 0))
+      w = (int)((uint32_t)from_float<Out>(a0).bits | ((uint32_t)from_float<Out>(b0).bits << 8) | ((uint32_t)from_float<Out>(a1).bits << 16) | ((uint32_t)from_float<Out>(b1).bits << 24));
+    __builtin_memcpy(o.v, &w, 4);
+  } else {
+    o.v[0] = from_float<Out>(a0); o.v[1] = from_float<Out>(b0);
+    o.v[2] = from_float<Out>(a1); o.v[3] = from_float<Out>(b1);
   }
   return o;
 }

@@ -351,6 +351,27 @@ def test_mvue_default_sampling_follows_torch_seed(cuda):
     assert err < 0.12, err
 
 
+@pytest.mark.parametrize("out_dtype", [F16, BF16, E4M3, E5M2])
+@pytest.mark.parametrize("in_dtype,shape,extra", [(BF16, (64, 128), 0), (F16, (96, 384), 8), (F32, (32, 2176), 64), (F32, (1056, 256), 0), (BF16, (160, 640), 24)])
+def test_mvue_panel_conversion(cuda, in_dtype, out_dtype, shape, extra):
+    """The kernel for row-major input and panel output: 16 or 8 rows to a block, rows of the matrix longer than its columns, partial
+    blocks on the right, uniforms from every source, groups whose largest element outweighs the others by up to 2^26 -- the bits of the oracle."""
+    import sparse
+    m, k = shape
+    g = torch.Generator().manual_seed(m + k)
+    wide = (torch.randn((m, k + extra), generator=g) * torch.exp2(torch.randint(-12, 15 if in_dtype != F16 else 4, (m, k + extra), generator=g).float())).to(in_dtype)
+    w = wide[:, :k]
+    seed, offset = 0xfedcba9876543210, (1 << 33) + 12
+    packed = oracle.mvue_uniforms(seed, offset, m, k)
+    full = torch.zeros(shape)
+    full[:, 0::4], full[:, 1::4] = packed[:, 0::2], packed[:, 1::2]
+    want_v, want_m, _ = oracle.mvue24(w, full, out_dtype=out_dtype)
+    for rand in ((seed, offset), packed.to(cuda), full.to(cuda)):
+        s = sparse.to_sparse_semi_structured(wide.to(cuda)[:, :k], MVUE24=True, dtype=out_dtype, rand=rand)
+        assert_same(s.indices(), want_m, "meta")
+        assert_same(torch.nan_to_num(s.values().float().cpu(), 1.5), torch.nan_to_num(want_v.float(), 1.5), "values")
+
+
 def _wide_range(shape, seed):
     """float32 values whose exponents span denormals to 2^60, with zeros, negative zeros and groups
     dominated by one element (sum - a_i rounds to zero): operands the in-range division must hand
