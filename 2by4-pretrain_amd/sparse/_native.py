@@ -66,6 +66,8 @@ _SIGNATURES = {
     "tf24_grad_weight": (_i, [_p, _i64, _p, _i64, _i, _i64, _i64, _i64, _p, _p, _p, _i64, _p]),
     "tf24_grad_weight_f32": (_i, [_p, _i64, _p, _i64, _i, _i64, _i64, _i64, _p, _p, _p, _i64, _p]),
     "tf24_grad_weight_workspace_bytes": (_i64, [_i64, _i64, _i64]),
+    "tf24_linear16_suits": (_i, [_i64, _i64, _i64]),
+    "tf24_linear16": (_i, [_p, _i64, _i, _p, _i64, _i, _i64, _i64, _i64, _p, _i64, _p, _p]),
     "tf24_transpose": (_i, [_p, _i, _i64, _i64, _i64, _p, _i64, _p]),
     "tf24_spmm_validate": (_i, [_i, _i64, _i64, _i, _i64, _i64, _i, _i, _i64, _i]),
 }

@@ -431,6 +431,20 @@ int tf24_grad_weight_f32(const void* g, int64_t ldg, const void* x, int64_t ldx,
 int64_t tf24_grad_weight_workspace_bytes(int64_t tokens, int64_t m, int64_t n);
 
 /*
+ * A linear layer's product with a dense weight:
+ *     y[t, i] = sum_k x[t, k] * W(i, k) + bias[i]      (t < tokens, i < rows)
+ * x [tokens, k], y [tokens, rows] row-major F16 or BF16 with leading dimensions ldx, ldy; W(i, k) at w[i * ldw + k], or with w_strided at
+ * w[k * ldw + i] (the gradient of the input: w [k, rows] is the weight, k its outputs); bias [rows] of the same type or NULL.
+ * Sums in float32, bias added, rounded once.  rows a multiple of 8, k one of 64 and at least 256, any number of tokens; leading dimensions
+ * multiples of 8, those of w and x at most 2^22; w, x and y 16-byte aligned.  The reference leaves these products to torch
+ * (sparse/sparse_ops.py:20-43).
+ */
+int tf24_linear16(const void* w, int64_t ldw, int w_strided, const void* x, int64_t ldx, int dtype, int64_t rows, int64_t k, int64_t tokens,
+                  void* y, int64_t ldy, const void* bias, void* stream);
+/* 1: a product of these sizes is one that tf24_linear16 takes and that its tiles fill the compute units with; 0: leave it to the library */
+int tf24_linear16_suits(int64_t rows, int64_t k, int64_t tokens);
+
+/*
  * out[c, r] = in[r, c] for 2-byte (F16|BF16) and 1-byte (E4M3|E5M2|U8) elements; in [rows, cols] with
  * leading dimension ld_in, out [cols, rows] with ld_out.  No counterpart in the reference (CUTLASS
  * reads either operand layout): it feeds tf24_spmm's fast kernel, which wants an 8-bit dense operand

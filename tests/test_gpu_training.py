@@ -874,3 +874,85 @@ def test_soft_threshold_linear_lets_go_of_its_weight(cuda, leaf):
     with torch.autograd.graph.save_on_cpu():
         y, _ = forward()
     assert all(a.equal(b) for a, b in zip(first, torch.autograd.grad(y, (x, base, mod.bias), gy)))
+
+
+@pytest.mark.parametrize("rows,k,tokens", [(8, 256, 1), (192, 256, 192), (200, 320, 193), (184, 1536, 191), (768, 3072, 400), (2056, 512, 4100), (520, 6400, 777)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("strided", [False, True])
+def test_dense_linear_kernel(cuda, rows, k, tokens, dtype, strided):
+    """The S-STE layer's product with its weight and with its transpose: rows and tokens that fill no tile, the fewest stages, stages
+    in another order per XCD (24 and more), tiles behind each other in one workgroup (2056 x 4100), operands and results with a pitch.
+    Small integers, whose sums float32 holds exactly: rounded once.  Random operands: a float32 sum of k exact products and the bias in any
+    order errs by at most (k + 1) * 2^-23 times the sum of their magnitudes, and is rounded once to 11 (8) bits."""
+    from sparse import _native as N
+    gen = torch.Generator(device=cuda).manual_seed(rows + k + tokens)
+    shape = (k, rows + 8) if strided else (rows, k + 8)
+
+    def run(w, x, bias):
+        y = torch.full((tokens, rows + 8), float("nan"), dtype=dtype, device=cuda)
+        N.check(N.lib().tf24_linear16(w.data_ptr(), w.stride(0), strided, x.data_ptr(), x.stride(0), N.dtype_code(dtype), rows, k, tokens, y.data_ptr(),
+                                      y.stride(0), N.ptr(bias), N.stream_ptr()))
+        assert y[:, rows:].isnan().all()
+        return y[:, :rows]
+
+    for ints in (True, False):
+        draw = (lambda *s: torch.randint(-4, 5, s, device=cuda, generator=gen).to(dtype)) if ints else (lambda *s: torch.randn(*s, device=cuda, generator=gen).to(dtype))
+        w, x, bias = draw(*shape), draw(tokens, k + 16)[:, 8:8 + k], draw(rows)
+        wk = (w[:, :rows].t() if strided else w[:, :k]).double().contiguous()
+        for b in (None, bias):
+            want = x.double() @ wk.t().contiguous() + (0 if b is None else b.double())
+            got = run(w, x, b)
+            if ints:
+                assert got.equal(want.to(dtype))
+            else:
+                size = x.double().abs() @ wk.abs().t().contiguous() + (0 if b is None else b.double().abs())
+                limit = want.abs() * 2.0 ** (-11 if dtype == torch.float16 else -8) + size * (k + 1) * 2.0 ** -23 + 1e-7
+                assert ((got.double() - want).abs() <= limit).all()
+                assert got.equal(run(w, x, b))
+
+
+@pytest.mark.parametrize("rows,k,tokens", [(3072, 768, 800), (768, 3072, 800), (2048, 512, 1500)])
+def test_soft_threshold_layer_products_take_the_kernel(cuda, rows, k, tokens, monkeypatch):
+    """One round of tiles or part of one: an S-STE layer's product and input gradient are the same where the kernel takes them as in the
+    library (two float32 sums of n terms, rounded to 8 bits), infinite activations included; gradients with another order take it too."""
+    from sparse import _native as N, SoftThresholdLinear
+    import torch.nn.functional as F
+    gen = torch.Generator(device=cuda).manual_seed(rows)
+    layer = SoftThresholdLinear(k, rows, device=cuda)
+    layer.init_scale()
+    x = torch.randn(2, tokens // 2, k, device=cuda, generator=gen).requires_grad_()
+    dy = torch.randn(2, tokens // 2, rows, device=cuda, generator=gen).bfloat16()
+    x.data[1, 3, 5] = float("inf")
+    calls, lib = [], N.lib()
+    spy = type("Spy", (), {"__getattr__": lambda self, name: (calls.append(name), getattr(lib, name))[1]})()
+    outs = []
+    for suits in (1, 0):
+        x.grad = None
+        calls.clear()
+        spy.__dict__["tf24_linear16_suits"] = lambda *a, suits=suits: suits
+        monkeypatch.setattr(N, "lib", lambda: spy)
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            y = layer(x)
+        y.backward(dy.transpose(0, 1).contiguous().transpose(0, 1) if suits else dy)
+        monkeypatch.undo()
+        assert calls.count("tf24_linear16") == (2 if suits else 0)
+        outs.append((y.detach().double(), x.grad.double()))
+    weight = layer.get_sparse_weights().detach().bfloat16().double().abs()
+    for got, want, size, terms in ((outs[0][0], outs[1][0], x.detach().bfloat16().double().abs() @ weight.t().contiguous() + layer.bias.detach().double().abs(), k + 1),
+                                   (outs[0][1], outs[1][1], dy.double().abs() @ weight, rows)):
+        assert got.isnan().equal(want.isnan()) and got.isinf().equal(want.isinf())
+        ok = want.isfinite()
+        limit = want.abs() * 2.0 ** -7 + 2 * size * terms * 2.0 ** -23 + 1e-7
+        assert ((got - want).abs() <= limit)[ok].all()
+
+
+def test_dense_linear_refuses_what_it_does_not_take(cuda):
+    from sparse import _native as N
+    t = torch.zeros(512, 512, dtype=torch.float16, device=cuda)
+    lib, p = N.lib(), t.data_ptr()
+    good = dict(w=p, ldw=512, strided=0, x=p, ldx=512, dtype=N.dtype_code(torch.float16), rows=256, k=256, tokens=64, y=p, ldy=512, bias=None)
+    for bad in (dict(dtype=N.dtype_code(torch.float32)), dict(rows=252), dict(rows=0), dict(k=192), dict(k=288), dict(tokens=0), dict(ldw=248), dict(ldx=252),
+                dict(ldx=516), dict(ldy=248), dict(ldw=(1 << 22) + 8), dict(strided=1, ldw=248), dict(w=None), dict(x=p + 2), dict(y=p + 8), dict(bias=p + 1)):
+        assert lib.tf24_linear16(*{**good, **bad}.values(), N.stream_ptr()) != 0, bad
+    for shape in ((252, 256, 64), (256, 192, 64), (256, 256, 0), (0, 256, 64)):
+        assert lib.tf24_linear16_suits(*shape) == 0
