@@ -3,13 +3,14 @@
     python 2by4-pretrain_amd/build.py [-j N] [--force]
 
 Objects go to 2by4-pretrain_amd/build/, the library next to the Python package that loads it
-(2by4-pretrain_amd/sparse/lib2by4_gfx950.so).
+(2by4-pretrain_amd/sparse/lib2by4_gfx950.so), beside it _fastcall.so, through which Python makes the frequent calls.
 """
 import argparse
 import concurrent.futures
 import os
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
@@ -17,6 +18,8 @@ CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(HERE, "build")
 LIB = os.path.join(HERE, "sparse", "lib2by4_gfx950.so")
 
+FASTCALL = os.path.join(HERE, "sparse", "_fastcall.so")
+CXX = os.environ.get("CXX", "g++")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC",
@@ -58,6 +61,13 @@ def build_library(jobs=8, force=True, verbose=False):
     res = subprocess.run(cmd, capture_output=True, text=True)
     if res.returncode:
         raise RuntimeError(f"link failed:\n{res.stdout}\n{res.stderr}")
+    # the CPython module over the library (found next to it at run time)
+    cmd = [CXX, "-O2", "-std=c++17", "-shared", "-fPIC", "-I", os.path.join(ROOT, "include"), "-I", sysconfig.get_paths()["include"],
+           os.path.join(CSRC, "fastcall.cpp"), "-o", FASTCALL, "-L", os.path.dirname(LIB), "-l:" + os.path.basename(LIB), "-Wl,-rpath,$ORIGIN",
+           "-Wl,--allow-shlib-undefined"]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode:
+        raise RuntimeError(f"building the CPython module failed:\n{res.stdout}\n{res.stderr}")
     return LIB
 
 

@@ -1,4 +1,5 @@
-"""ctypes binding of lib2by4_gfx950.so (C ABI declared in include/tf24.h).
+"""Binding of lib2by4_gfx950.so (C ABI declared in include/tf24.h): ctypes, and for the frequent calls the CPython module
+_fastcall.so over the same library (csrc/fastcall.cpp), which takes the same arguments.
 
 There is no fallback: if the library is missing or a call fails, a RuntimeError is raised.
 Every wrapper enqueues on torch's current HIP stream and passes raw device pointers.
@@ -91,6 +92,10 @@ def lib():
             fn = getattr(handle, name)          # AttributeError if the library lacks a declared symbol
             fn.restype = res
             fn.argtypes = args
+        from . import _fastcall                 # (ImportError if it has not been built)
+        for name in _SIGNATURES:
+            if hasattr(_fastcall, name):
+                setattr(handle, name, getattr(_fastcall, name))
         _lib = handle
     return _lib
 

@@ -516,7 +516,7 @@ class SparseSemiStructuredTensor(torch.Tensor):
     def __torch_function__(cls, func, types, args=(), kwargs=None):
         """torch.nn.functional.linear without gradients goes to the kernels from here.  Through the dispatcher it is two
         calls of __torch_dispatch__, one of which builds the transposed wrapper: 15.4 us of host time a call, which bounds the
-        products of few tokens (3072 x 768 against 37: 5.7 us on the GPU); from here 10.9, 4.3 of them the launch itself.
+        products of few tokens (3072 x 768 against 37: 5.7 us on the GPU); from here 9.8, 4.3 of them the launch itself (10.9 when the call was made through ctypes).
         Everything that torch does on the way (autocast, transforms, modes, tracing) and every other function takes torch's
         own route."""
         if func is _F_LINEAR and not kwargs and not torch.is_grad_enabled():

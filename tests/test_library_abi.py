@@ -308,3 +308,30 @@ def test_derived_weights_handle_their_own_methods():
         weight = make(cls)
         assert weight.t().shape == (64, 32) and weight.t().transposed
         assert weight.values().shape == (32, 32) and weight.indices().shape == (32, 4)
+
+
+def test_fast_calls_take_what_ctypes_takes():
+    """The CPython module's functions over the same library: the same results and the same refusals as through ctypes."""
+    import ctypes
+
+    import pytest
+    from sparse import _fastcall, _native as N
+    fast = N.lib()
+    slow = ctypes.CDLL(N.library_path())
+    names = [n for n in N._SIGNATURES if hasattr(_fastcall, n)]
+    assert "tf24_spmm" in names and "tf24_linear" in names and all(getattr(fast, n) is getattr(_fastcall, n) for n in names)
+    for name in names:
+        res, types = N._SIGNATURES[name]
+        fn = getattr(slow, name)
+        fn.restype, fn.argtypes = res, types
+        # null pointers and empty shapes: every entry point answers these on the host
+        args = [None if t is ctypes.c_void_p else 0 if t in (ctypes.c_int, ctypes.c_int64) else 0.0 for t in types]
+        assert getattr(fast, name)(*args) == fn(*args), name
+        for bad in (args[:-1], [*args[:-1], "x"], [1.5 if t in (ctypes.c_int, ctypes.c_int64) else a for t, a in zip(types, args)] if ctypes.c_int64 in types else args[:-1]):
+            with pytest.raises(TypeError):
+                getattr(fast, name)(*bad)
+    for shape in ((3072, 768, 12288), (4096, 11008, 37), (8, 64, 1), (True, 64, 64)):
+        for code in (N.F16, N.E4M3, N.I8):
+            assert fast.tf24_spmm_workspace_bytes(code, *shape) == slow.tf24_spmm_workspace_bytes(code, *shape)
+    assert fast.tf24_linear16_suits(2 ** 64 + 3072, 768, 12288) == slow.tf24_linear16_suits(2 ** 64 + 3072, 768, 12288) == 1      # modulo 2^64, as ctypes does
+    assert fast.tf24_adamw_masked_decay_list(b"", 0, 0, 0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0, None) == slow.tf24_adamw_masked_decay_list(b"", 0, 0, 0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0, None)
