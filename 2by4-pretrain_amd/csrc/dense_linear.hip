@@ -5,7 +5,7 @@
 // X [tokens, k] row-major.  W(i, k) lies at i * ldw + k (the forward product) or, STRIDED, at k * ldw + i (the gradient of the
 // input, whose summed axis is the slow one of the weight).
 //
-// A block of four waves (2 x 2, one per SIMD) computes 192(i) x 192(t) tiles, wave tile 96 x 96 = 3 x 3 V_MFMA_F32_32X32X16 with 144
+// A block of four waves (2 x 2, one per SIMD) computes 192(i) x 192(t) tiles, wave tile 96 x 96 = 6 x 6 V_MFMA_F32_16X16X32 with 144
 // accumulators.  64 elements of k of both operands are one stage of 48 KB, three of which rotate through the LDS: while stage s is
 // multiplied, the copies of s + 1 and s + 2 are in flight (global -> LDS directly).  The fragments of a step of 32 elements of k are
 // read behind the matrix instructions of the step before, one read behind each.  One workgroup per compute unit walks the tiles of its
@@ -13,8 +13,10 @@
 // output pass stages through the buffer that is free.
 //
 // Bound by the power that the matrix cores may draw: a stage takes 0.53 us on operands of zeros (0.48 by matrix instructions alone) and 0.87
-// on random ones, and a launch 8 us beside its stages.  12288 tokens, bf16, here and in the library (GPU time): 3072 x 768 with bias 57.5 and
-// 62.8 us, 768 x 3072 50 and 63, their input gradients 51.5 and 61, 59.5 and 72.  The reads of a step spread over its instructions or over the
+// on random ones, and a launch 8 us beside its stages.  Hence the 16 x 16 instructions: alone, on random operands in registers, they sustain
+// 1.9 PFLOP/s where the 32 x 32 ones do 1.65 (2.46 and 2.48 on zeros), and the products below took 1 to 5 % longer with the latter.
+// 12288 tokens, bf16, here and in the library (GPU time): 3072 x 768 with bias 57.9 and 62.8 us, 768 x 3072 49 and 63, their input
+// gradients 49.5 and 61, 58.8 and 72.  The reads of a step spread over its instructions or over the
 // first two thirds of them: alike.  Ordinary instead of streaming stores: 67 us for 61 (3072 x 768).
 #include "lds_copies.hpp"
 #include <algorithm>
@@ -26,7 +28,7 @@ namespace {
 
 typedef short short8v __attribute__((ext_vector_type(8)));
 
-constexpr int kTile = 192, kThreads = 256, kWaves = 4, kFrags = 3;          // fragments of 32 rows (and of 32 columns) per wave
+constexpr int kTile = 192, kThreads = 256, kWaves = 4, kFrags = 6;          // fragments of 16 rows (and of 16 columns) per wave
 constexpr int kStageK = 64, kRowBytes = kStageK * 2, kStridedRowBytes = kTile * 2;
 constexpr int kOperand = kTile * kRowBytes, kStage = 2 * kOperand;          // [W | X]
 constexpr int kCopies = kOperand / 1024 / kWaves;                           // 1 KB copies per wave and operand of a stage
@@ -37,11 +39,11 @@ constexpr int kRotateMinStages = 24;
 static_assert(kRotateMinStages - 2 - (7 * kRotateMinStages >> 3) >= 1, "the first three stages of a tile are copied before the order wraps");
 constexpr int kRaster = 8;                                                  // tiles along i of a group
 
-__device__ __forceinline__ float16v mma(f16_t, int4v a, int4v b, float16v c) {
-  return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8, a), __builtin_bit_cast(half8, b), c, 0, 0, 0);
+__device__ __forceinline__ float4v mma(f16_t, int4v a, int4v b, float4v c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, a), __builtin_bit_cast(half8, b), c, 0, 0, 0);
 }
-__device__ __forceinline__ float16v mma(bf16_t, int4v a, int4v b, float16v c) {
-  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+__device__ __forceinline__ float4v mma(bf16_t, int4v a, int4v b, float4v c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
 }
 
 template <typename T, bool STRIDED>
@@ -69,7 +71,7 @@ dense_linear(const uint8_t* __restrict__ w, int64_t ldw, const uint8_t* __restri
     for (int spin = 0; spin < 1024 && __builtin_amdgcn_s_memrealtime() - t0 < (uint64_t)stagger_ticks; spin++) __builtin_amdgcn_s_sleep(4);
   }
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int wi = wave >> 1, wj = wave & 1, l32 = lane & 31, lh = lane >> 5;
+  const int wi = wave >> 1, wj = wave & 1, l16 = lane & 15, lq = lane >> 4;
   const int nstages = (int)(k / kStageK);                        // (at least 4)
   const int64_t w_step = STRIDED ? kStageK * ldw : kRowBytes;
   const int first_stage = nstages >= kRotateMinStages ? xcd * nstages >> 3 : 0;
@@ -110,66 +112,61 @@ dense_linear(const uint8_t* __restrict__ w, int64_t ldw, const uint8_t* __restri
     next_stage();
   };
 
-  float16v acc[kFrags][kFrags];
+  float4v acc[kFrags][kFrags];
   auto clear = [&]() {
 #pragma unroll
     for (int ti = 0; ti < kFrags; ti++)
 #pragma unroll
-      for (int tj = 0; tj < kFrags; tj++)
-#pragma unroll
-        for (int r = 0; r < 16; r++) acc[ti][tj][r] = 0.0f;
+      for (int tj = 0; tj < kFrags; tj++) acc[ti][tj] = float4v{0, 0, 0, 0};
   };
   clear();
 
-  // ---- fragments of a step (32 elements of k): of either half, lane l takes row l % 32, elements 8 * (l / 32) .. + 7.  STRIDED: in a
-  // group of 16 lanes, lane i receives the halfwords i % 4 of the source lanes 4e + i / 4 (e = 0..3), so source lane s addresses
-  // k-row s / 4 (of four), columns 4 * (s % 4).. of the group's 16; two such reads make eight elements of k.
-  const int swizzle = (l32 >> 1) & 7;
-  uint32_t a_off[2][2], b_off[2][2], t_off[kFrags];
+  // ---- fragments of a step (32 elements of k): lane l takes row l % 16, elements 8 * (l / 16) .. + 7.  STRIDED: in a group of 16 lanes,
+  // lane i receives the halfwords i % 4 of the source lanes 4e + i / 4 (e = 0..3), so source lane s addresses k-row s / 4 (of
+  // four), columns 4 * (s % 4).. of the group's 16; two such reads make eight elements of k.
+  const int swizzle = (l16 >> 1) & 7;
+  uint32_t a_off[2], b_off[2], t_off[kFrags];
 #pragma unroll
-  for (int step = 0; step < 2; step++)
-#pragma unroll
-    for (int h = 0; h < 2; h++) {
-      const uint32_t chunk = (uint32_t)((step * 4 + h * 2 + lh) ^ swizzle) * 16;
-      a_off[step][h] = (uint32_t)(wi * 96 + l32) * kRowBytes + chunk;
-      b_off[step][h] = kOperand + (uint32_t)(wj * 96 + l32) * kRowBytes + chunk;
-    }
+  for (int step = 0; step < 2; step++) {
+    const uint32_t chunk = (uint32_t)((step * 4 + lq) ^ swizzle) * 16;
+    a_off[step] = (uint32_t)(wi * 96 + l16) * kRowBytes + chunk;
+    b_off[step] = kOperand + (uint32_t)(wj * 96 + l16) * kRowBytes + chunk;
+  }
   if constexpr (STRIDED) {
-    const uint32_t s16 = lane & 15, krow = lh * 8 + (s16 >> 2);
+    const uint32_t krow = lq * 8 + (l16 >> 2);
 #pragma unroll
     for (int f = 0; f < kFrags; f++) {
-      const uint32_t col = (uint32_t)(wi * 96 + f * 32 + ((lane >> 4) & 1) * 16) + (s16 & 3) * 4;
+      const uint32_t col = (uint32_t)(wi * 96 + f * 16) + (l16 & 3) * 4;
       t_off[f] = krow * kStridedRowBytes + (((col >> 3) ^ strided_swizzle(krow)) * 16) + ((col >> 2) & 1) * 8;
     }
   }
-  int4v af[2][2][kFrags], bf[2][2][kFrags];                      // [register set][half][fragment]
-  short4v aq[2][2][kFrags][2];                                   // STRIDED: the quarters of a fragment
-  constexpr int A_READS = STRIDED ? 2 * kFrags : kFrags, READS = 2 * (A_READS + kFrags), MMAS = 2 * kFrags * kFrags;
-  // the reads of a step, half by half: X's fragments, then W's
+  int4v af[2][kFrags], bf[2][kFrags];                            // [register set][fragment]
+  short4v aq[2][kFrags][2];                                      // STRIDED: the halves of a fragment
+  constexpr int A_READS = STRIDED ? 2 * kFrags : kFrags, READS = A_READS + kFrags, MMAS = kFrags * kFrags;
+  // the reads of a step in the order the next step's instructions need them: W's first fragment, X's, W's others
+  auto read_w = [&](int set, int q, uint32_t buf, int step) {
+    if constexpr (STRIDED)
+      aq[set][q >> 1][q & 1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+          (lds_short4_ptr)(lds_ptr_t)(smem + buf + t_off[q >> 1] + (step * 32 + (q & 1) * 4) * kStridedRowBytes));
+    else af[set][q] = *reinterpret_cast<const int4v*>(smem + buf + a_off[step] + q * 16 * kRowBytes);
+  };
   auto read_one = [&](int set, int n, uint32_t buf, int step) {
-    const int h = n / (A_READS + kFrags), q = n % (A_READS + kFrags);
-    const uint8_t* base = smem + buf;
-    if (q < kFrags) bf[set][h][q] = *reinterpret_cast<const int4v*>(base + b_off[step][h] + q * 32 * kRowBytes);
-    else if constexpr (STRIDED) {
-      const int f = (q - kFrags) >> 1, quarter = (q - kFrags) & 1;
-      aq[set][h][f][quarter] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-          (lds_short4_ptr)(lds_ptr_t)(base + t_off[f] + (step * 32 + h * 16 + quarter * 4) * kStridedRowBytes));
-    } else {
-      af[set][h][q - kFrags] = *reinterpret_cast<const int4v*>(base + a_off[step][h] + (q - kFrags) * 32 * kRowBytes);
-    }
+    constexpr int FIRST = A_READS / kFrags;
+    if (n >= FIRST && n < FIRST + kFrags) bf[set][n - FIRST] = *reinterpret_cast<const int4v*>(smem + buf + b_off[step] + (n - FIRST) * 16 * kRowBytes);
+    else read_w(set, n < FIRST ? n : n - kFrags, buf, step);
   };
-  auto w_fragment = [&](int set, int h, int f) {
-    if constexpr (STRIDED) return __builtin_bit_cast(int4v, __builtin_shufflevector(aq[set][h][f][0], aq[set][h][f][1], 0, 1, 2, 3, 4, 5, 6, 7));
-    else return af[set][h][f];
+  auto w_fragment = [&](int set, int f) {
+    if constexpr (STRIDED) return __builtin_bit_cast(int4v, __builtin_shufflevector(aq[set][f][0], aq[set][f][1], 0, 1, 2, 3, 4, 5, 6, 7));
+    else return af[set][f];
   };
-  // The instructions of a step from one register set; behind each of them the next step's reads into the other set and the copies
+  // The instructions of a step from one register set; behind them, one by one, the next step's reads into the other set and the copies
   // of half a stage.
   auto mma_step = [&](int set, int half, bool copies, uint32_t dst, bool reads, uint32_t src, int rstep) {
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int n = 0; n < MMAS; n++) {
-      const int h = n / (kFrags * kFrags), ti = n / kFrags % kFrags, tj = n % kFrags;
-      acc[ti][tj] = mma(T{}, w_fragment(set, h, ti), bf[set][h][tj], acc[ti][tj]);
+      const int ti = n / kFrags, tj = n % kFrags;
+      acc[ti][tj] = mma(T{}, w_fragment(set, ti), bf[set][tj], acc[ti][tj]);
       __builtin_amdgcn_sched_barrier(0);
       if (reads) {
 #pragma unroll
@@ -246,7 +243,7 @@ dense_linear(const uint8_t* __restrict__ w, int64_t ldw, const uint8_t* __restri
 #pragma unroll
     for (int q = 0; q < 2; q++) asm volatile("" : "+v"(bias_w[q]));
 
-    // ---- output pass: a lane holds column l % 32 and rows 8 * (r / 4) + 4 * (l / 32) + r % 4 of a fragment.  Each wave stages 32(t) x 96(i)
+    // ---- output pass: a lane holds column l % 16 and rows 4 * (l / 16) + r of a fragment.  Each wave stages 32(t) x 96(i)
     // pieces in a slice of the last stage's buffer (rows of 192 bytes, chunks XOR-swizzled with the row) and stores whole rows of them.
     constexpr int SLICE = 32 * 192;
     float* bias_lds = reinterpret_cast<float*>(smem + cur + kWaves * SLICE + wave * 384);
@@ -256,26 +253,24 @@ dense_linear(const uint8_t* __restrict__ w, int64_t ldw, const uint8_t* __restri
     uint8_t* stage = smem + cur + wave * SLICE;
     auto chunk_at = [](int row, int ch) { return row * 192 + (ch ^ ((row >> 2) & 3)) * 16; };
 #pragma unroll
-    for (int tj = 0; tj < kFrags; tj++) {
+    for (int tp = 0; tp < kFrags / 2; tp++) {                    // 32 columns (t)
 #pragma unroll
       for (int ti = 0; ti < kFrags; ti++) {
-        float4v add[4];
+        const float4v add = *reinterpret_cast<const float4v*>(bias_lds + ti * 16 + lq * 4);
 #pragma unroll
-        for (int g = 0; g < 4; g++) add[g] = *reinterpret_cast<const float4v*>(bias_lds + ti * 32 + g * 8 + lh * 4);
-#pragma unroll
-        for (int g = 0; g < 4; g++) {
+        for (int t2 = 0; t2 < 2; t2++) {
           T o[4];
 #pragma unroll
-          for (int r = 0; r < 4; r++) o[r] = from_float<T>(acc[ti][tj][g * 4 + r] + add[g][r]);
-          *reinterpret_cast<Pack<T, 4>*>(stage + chunk_at(l32, ti * 4 + g) + lh * 8) = *reinterpret_cast<Pack<T, 4>*>(o);
+          for (int r = 0; r < 4; r++) o[r] = from_float<T>(acc[ti][tp * 2 + t2][r] + add[r]);
+          *reinterpret_cast<Pack<T, 4>*>(stage + chunk_at(t2 * 16 + l16, ti * 2 + (lq >> 1)) + (lq & 1) * 8) = *reinterpret_cast<Pack<T, 4>*>(o);
         }
       }
-      if (tj == 0 && has_next) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");     // the next tile's first two stages
+      if (tp == 0 && has_next) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");     // the next tile's first two stages
 #pragma unroll
       for (int it = 0; it < 6; it++) {
         const uint32_t piece = it * 64 + lane;
         const int jl = piece / 12, ch = piece % 12;
-        const int64_t icol = i0 + wi * 96 + ch * 8, jrow = j0 + wj * 96 + tj * 32 + jl;
+        const int64_t icol = i0 + wi * 96 + ch * 8, jrow = j0 + wj * 96 + tp * 32 + jl;
         const int4v v = *reinterpret_cast<const int4v*>(stage + chunk_at(jl, ch));
         if (jrow < tokens && icol < rows) __builtin_nontemporal_store(v, reinterpret_cast<int4v*>(y + jrow * ldy + icol));
       }
