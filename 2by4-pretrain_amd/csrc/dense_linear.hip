@@ -309,17 +309,17 @@ int launch_linear(const void* w, int64_t ldw, bool strided, const void* x, int64
 }
 
 // Where the kernel is the faster one, against the library's product (hipBLASLt through torch, GPU time): tiles that fill the rounds of
-// the compute units.  `fill` is the share of the rounds' results that the product has.  Of 200 products of S-STE layers (512 to 1600
-// wide and four times that, 510 to 16384 tokens, both directions, operands that change from call to call) the rule takes 54: 16 % less
-// time than the library over them, 40 % at best, and 3 % more at worst.  fill, library and here, us: 3072 x 768 against 12288
-// tokens 1.00 62.8 57.5, its input gradient (768 rows, k 3072, STRIDED) 61.2 51.5; 2560 x 640 against 3286 0.89 25.0 15.1, 5120 x 1280
-// against 1080 0.59 23.1 19.5.  Left to the library: several rounds below 0.84 (6400 x 1600 against 1992 0.68 37.7 47.6, 4096 x 1024
-// against 4913 0.71 44.8 50.0), one round of long tiles below 0.75 (1600 x 6400 against 2831 0.48 64.4 77.2), where its smaller tiles and its
-// pieces of k reach more compute units, and one round of short ones below 0.55 (3072 x 768 against 555 0.18 9.5 12.5).
+// the compute units.  `fill` is the share of the rounds' results that the product has.  Of 480 products of S-STE layers (512 to 1600
+// wide and four times that, 500 to 16384 tokens, both directions, operands that change from call to call) the rule takes 86: 15 % less
+// time than the library over them, 40 % at best, and 2 % more at worst.  fill, library and here, us: 3072 x 768 against 12288
+// tokens 1.00 60.1 56.3, its input gradient (768 rows, k 3072, STRIDED) 59.7 48.0; 2560 x 640 against 13317 0.90 58.6 44.8, 5120 x 1280
+// against 1074 0.58 22.9 20.2.  Left to the library: several rounds below 0.89 (4096 x 1024 against 4053 0.88 29.0 35.3, 6400 x 1600
+// against 2525 0.86 40.2 51.9), one round of long tiles below 0.72 (1600 x 6400 against 2831 0.48 62.5 77.5), where its smaller tiles and its
+// pieces of k reach more compute units, and one round of short ones below 0.55 (4096 x 1024 against 1256 0.545 15.2 16.4).
 bool suits(int64_t rows, int64_t k, int64_t tokens, int cus) {
   const int64_t tiles = (rows + kTile - 1) / kTile * ((tokens + kTile - 1) / kTile), rounds = (tiles + cus - 1) / cus;
   const double fill = (double)rows * (double)tokens / ((double)(rounds * cus) * kTile * kTile);
-  return fill >= (rounds > 1 ? 0.84 : k / kStageK <= 25 ? 0.55 : 0.75);
+  return fill >= (rounds > 1 ? 0.89 : k / kStageK <= 25 ? 0.55 : 0.72);
 }
 
 bool shapes_fit(int64_t rows, int64_t k, int64_t tokens) {
