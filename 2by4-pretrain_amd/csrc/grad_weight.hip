@@ -5,7 +5,7 @@
 // G [tokens, m] and X [tokens, n] are read as they lie: the summed axis is the slow one of both.
 //
 // Bound by the matrix cores, and at this size by the power that they may draw: 12288 tokens, 3072 x 768 bf16 take 67
-// us with db (0.87 PFLOP/s; on 256 x 256 tiles 70, of zeros 54), where the library's product takes 110 to 140 us and its row sum 20 to 29.
+// us with db (0.87 PFLOP/s; on 32 x 32 instructions 71, on 256 x 256 tiles 70, of zeros 54), where the library's product takes 110 to 140 us and its row sum 20 to 29.
 //
 // A block multiplies a 256(i) x 256(j) tile over a piece of the token axis: eight waves (2 along i x 4 along j), two per
 // SIMD, wave tile 128 x 64 = 4 x 2 V_MFMA_F32_32X32X16.  (Four waves of 128 x 128 read a third less LDS, but nothing covers
@@ -14,6 +14,8 @@
 // stage of 32 KB (24); five stages rotate through the LDS.  At the start of stage s the copies of s+1 and s+2 are in
 // flight and those of s+3 go into the buffer of stage s-2, whose fragments every wave has used up before the barrier of
 // stage s: no wave waits for its own reads there.
+// Where takes_long says so, the 192 x 192 tiles take V_MFMA_F32_16X16X32 in stages of 64 tokens, three of which rotate: the copies of s+2 go
+// into the buffer of stage s-1, so the barrier of stage s waits for the reads as well.
 // Both operands need eight consecutive tokens of one column per lane: transposing reads (DS_READ_B64_TR_B16) of rows of
 // 256 (192) columns.  16-byte chunks are XOR-swizzled by token so that the four tokens x 64 bytes that 32 lanes read touch every
 // one of the 64 banks once (rows of 192 columns start half of the banks apart by themselves; with a swizzle that only spreads 16 lanes, half of the LDS cycles are conflicts).
@@ -28,37 +30,51 @@ namespace {
 
 typedef short short8v __attribute__((ext_vector_type(8)));
 
-constexpr int kStageTokens = 32, kRing = 5;
 constexpr int kMaxPieces = 16;
 
-template <int TILE_, int WAVES_J_>
+// FR: rows and columns of the matrix instruction, 32 (16 tokens each) or 16 (32 tokens); a stage is two steps of that many tokens
+template <int TILE_, int WAVES_J_, int FR_, int RING_>
 struct TileT {
   static constexpr int TILE = TILE_, WAVES_J = WAVES_J_, WAVES = 2 * WAVES_J, THREADS = 64 * WAVES;
-  static constexpr int ROW_BYTES = TILE * 2, OPERAND = kStageTokens * ROW_BYTES, STAGE = 2 * OPERAND;
+  static constexpr int FR = FR_, STEP_TOKENS = 512 / FR, STAGE_TOKENS = 2 * STEP_TOKENS, RING = RING_, AHEAD = RING == 5 ? 3 : 2;
+  static constexpr int ROW_BYTES = TILE * 2, OPERAND = STAGE_TOKENS * ROW_BYTES, STAGE = 2 * OPERAND;
   static constexpr int CHUNKS = TILE / 8;                               // 16-byte chunks of a token's columns
-  static constexpr int TI = TILE / 64, TJ = TILE / 32 / WAVES_J;        // fragments of 32 rows and of 32 columns per wave
+  static constexpr int TI = TILE / 2 / FR, TJ = TILE / FR / WAVES_J;    // fragments of FR rows and of FR columns per wave
   static constexpr int SUMS = (TI + WAVES_J - 1) / WAVES_J;             // row fragments whose column sums a wave forms
   static constexpr int COPIES = OPERAND / 1024 / WAVES;                 // 1 KB copies per wave and operand of a stage
-  static constexpr int MMA = TI * TJ, READS = 2 * (TI + TJ), SLABS = 4 * MMA;      // per step of 16 tokens; quarters of a wave's fragments
-  static_assert(COPIES * 1024 * WAVES == OPERAND && MMA % COPIES == 0 && kRing * STAGE <= 160 * 1024, "a stage's copies divide among the waves");
+  static constexpr int MMA = TI * TJ, READS = 2 * (TI + TJ);                         // per step
+  static constexpr int QUADS = FR * FR / 256, SLABS = QUADS * MMA;      // a lane's quads of four rows in a fragment and in all of a wave's
+  static_assert(COPIES * 1024 * WAVES == OPERAND && MMA % COPIES == 0 && RING * STAGE <= 160 * 1024 && (RING == 5 || RING == 3), "a stage's copies divide among the waves");
   static __device__ __forceinline__ uint32_t swizzle(uint32_t token) {
     return TILE == 256 ? ((token & 3) << 2) | (((token >> 3) & 1) << 1) : (((token >> 1) & 1) << 2) | (((token >> 3) & 1) << 1);
   }
   // Rows of fragment ti of a wave: the waves that share rows hold their fragments rotated, so that the first SUMS of each are
-  // (all but the last wave's, others: the same sums may be formed twice) another 32 of them: those are the rows whose column
+  // (all but the last wave's, others: the same sums may be formed twice) another FR of them: those are the rows whose column
   // sums the wave forms.
   static __device__ __forceinline__ int fragment_row(int wave, int ti) {
-    return (wave / WAVES_J) * (32 * TI) + ((ti + (wave % WAVES_J) * SUMS) % TI) * 32;
+    return (wave / WAVES_J) * (FR * TI) + ((ti + (wave % WAVES_J) * SUMS) % TI) * FR;
   }
+  // where slab s of a wave's accumulators lies in the tile: four rows of one column per lane
+  static __device__ __forceinline__ int slab_row(int wave, int lane, int s) {
+    return fragment_row(wave, s / (QUADS * TJ)) + (s % QUADS) * 8 + (lane / FR) * 4;
+  }
+  static __device__ __forceinline__ int slab_col(int wave, int lane, int s) { return ((wave % WAVES_J) * TJ + (s / QUADS) % TJ) * FR + lane % FR; }
 };
-using Wide = TileT<256, 4>;
-using Square = TileT<192, 2>;
+using Wide = TileT<256, 4, 32, 5>;
+using Square = TileT<192, 2, 32, 5>;
+using SquareLong = TileT<192, 2, 16, 3>;
 
 __device__ __forceinline__ float16v mma(f16_t, short8v a, short8v b, float16v c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8, a), __builtin_bit_cast(half8, b), c, 0, 0, 0);
 }
 __device__ __forceinline__ float16v mma(bf16_t, short8v a, short8v b, float16v c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+}
+__device__ __forceinline__ float4v mma(f16_t, short8v a, short8v b, float4v c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, a), __builtin_bit_cast(half8, b), c, 0, 0, 0);
+}
+__device__ __forceinline__ float4v mma(bf16_t, short8v a, short8v b, float4v c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
 }
 __device__ __forceinline__ float widen(f16_t, short h) { return to_float(f16_t{(uint16_t)h}); }
 __device__ __forceinline__ float widen(bf16_t, short h) { return to_float(bf16_t{(uint16_t)h}); }
@@ -83,7 +99,7 @@ __global__ void __launch_bounds__(C::THREADS)
 grad_weight_pipe(const uint8_t* __restrict__ g, int64_t ldg, const uint8_t* __restrict__ x, int64_t ldx, int64_t tokens,
                  int64_t m, int64_t n, int tiles_i, int tiles_j, int splits, float* __restrict__ partial, float* __restrict__ sums,
                  OutT* __restrict__ dw, OutT* __restrict__ db) {
-  __shared__ __attribute__((aligned(1024))) uint8_t smem[kRing * C::STAGE];
+  __shared__ __attribute__((aligned(1024))) uint8_t smem[C::RING * C::STAGE];
   // workgroup ids are dealt to the 8 XCDs round-robin: each XCD takes a run of units, which share operand columns in its L2
   const int nunits = tiles_i * tiles_j * splits, per_xcd = (nunits + 7) / 8;
   const int unit = (int)(blockIdx.x & 7) * per_xcd + (int)(blockIdx.x >> 3);
@@ -94,18 +110,18 @@ grad_weight_pipe(const uint8_t* __restrict__ g, int64_t ldg, const uint8_t* __re
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wj = wave % C::WAVES_J;
-  const int l32 = lane & 31, lh = lane >> 5;
-  const int stages_all = (int)((tokens + kStageTokens - 1) / kStageTokens);
+  const int lrow = lane % C::FR, lblock = lane / C::FR;            // row or column of a fragment, block of eight tokens
+  const int stages_all = (int)((tokens + C::STAGE_TOKENS - 1) / C::STAGE_TOKENS);
   const int st_begin = (int)((int64_t)at.split * stages_all / splits);
   const int nstages = (int)((int64_t)(at.split + 1) * stages_all / splits) - st_begin;
   // tokens of the last stage of the whole axis, if it is not a full one, and which stage of this piece that is (-1: none)
-  const int ragged = (int)(tokens % kStageTokens);
+  const int ragged = (int)(tokens % C::STAGE_TOKENS);
   const int ragged_stage = ragged && st_begin + nstages == stages_all ? nstages - 1 : -1;
 
   // ---- copies: number q of a wave brings 1 KB of a stage (2 tokens of 256 columns); columns past the matrix re-read its last chunk
-  const uint8_t* g_at = g + (int64_t)st_begin * kStageTokens * ldg;
-  const uint8_t* x_at = x + (int64_t)st_begin * kStageTokens * ldx;
-  const int64_t g_step = (int64_t)kStageTokens * ldg, x_step = (int64_t)kStageTokens * ldx;
+  const uint8_t* g_at = g + (int64_t)st_begin * C::STAGE_TOKENS * ldg;
+  const uint8_t* x_at = x + (int64_t)st_begin * C::STAGE_TOKENS * ldx;
+  const int64_t g_step = (int64_t)C::STAGE_TOKENS * ldg, x_step = (int64_t)C::STAGE_TOKENS * ldx;
   auto offset_of = [&](int q, int64_t c0, int64_t cols, int64_t ld, int rows) {
     const uint32_t chunk = (uint32_t)((wave * C::COPIES + q) * 64 + lane), token = chunk / C::CHUNKS;
     const int64_t col = min(c0 + (int64_t)((chunk % C::CHUNKS) ^ C::swizzle(token)) * 8, cols - 8);
@@ -114,8 +130,8 @@ grad_weight_pipe(const uint8_t* __restrict__ g, int64_t ldg, const uint8_t* __re
   uint32_t og[C::COPIES], ox[C::COPIES];
 #pragma unroll
   for (int q = 0; q < C::COPIES; q++) {
-    og[q] = offset_of(q, i0, m, ldg, kStageTokens);
-    ox[q] = offset_of(q, j0, n, ldx, kStageTokens);
+    og[q] = offset_of(q, i0, m, ldg, C::STAGE_TOKENS);
+    ox[q] = offset_of(q, j0, n, ldx, C::STAGE_TOKENS);
   }
   const uint32_t smem_at = lds_offset(smem);
   auto copy_one = [&](int q, int st, uint32_t buf) {             // q: the wave's copies of G, then those of X
@@ -138,14 +154,16 @@ grad_weight_pipe(const uint8_t* __restrict__ g, int64_t ldg, const uint8_t* __re
       for (int q = 0; q < 2 * C::COPIES; q++) copy_one(q, st, buf);
     }
   };
-  // stage st has arrived when this wave's copies of the (at most two) stages behind it are all that is in flight
+  // stage st has arrived when this wave's copies of the (at most AHEAD - 1) stages behind it are all that is in flight; with three
+  // buffers the next copies go into the stage just read, so the wave's reads of it are waited for as well
+  constexpr bool READS_TOO = C::RING == 3;
   auto arrive = [&](int st, uint32_t buf) {
-    const int behind = nstages - 1 - st;
-    if (behind >= 2) wait_copies_and_barrier<4 * C::COPIES, false>();
-    else if (behind == 1) wait_copies_and_barrier<2 * C::COPIES, false>();
-    else wait_copies_and_barrier<0, false>();
+    const int behind = min(nstages - 1 - st, C::AHEAD - 1);
+    if (behind >= 2) wait_copies_and_barrier<4 * C::COPIES, READS_TOO>();
+    else if (behind == 1) wait_copies_and_barrier<2 * C::COPIES, READS_TOO>();
+    else wait_copies_and_barrier<0, READS_TOO>();
     if (st == ragged_stage) {
-      for (int c = tid; c < (kStageTokens - ragged) * (C::ROW_BYTES / 16); c += C::THREADS) {
+      for (int c = tid; c < (C::STAGE_TOKENS - ragged) * (C::ROW_BYTES / 16); c += C::THREADS) {
         *reinterpret_cast<int4v*>(smem + buf + ragged * C::ROW_BYTES + c * 16) = int4v{0, 0, 0, 0};
         *reinterpret_cast<int4v*>(smem + buf + C::OPERAND + ragged * C::ROW_BYTES + c * 16) = int4v{0, 0, 0, 0};
       }
@@ -153,19 +171,19 @@ grad_weight_pipe(const uint8_t* __restrict__ g, int64_t ldg, const uint8_t* __re
     }
   };
 
-  float16v acc[C::TI][C::TJ];
+  std::conditional_t<C::FR == 32, float16v, float4v> acc[C::TI][C::TJ];
 #pragma unroll
   for (int ti = 0; ti < C::TI; ti++)
 #pragma unroll
     for (int tj = 0; tj < C::TJ; tj++)
 #pragma unroll
-      for (int r = 0; r < 16; r++) acc[ti][tj][r] = 0.0f;
+      for (int r = 0; r < 4 * C::QUADS; r++) acc[ti][tj][r] = 0.0f;
 
   // ---- fragments: in a group of 16 lanes, lane i receives the halfwords i % 4 of the source lanes 4e + i / 4 (e = 0..3).
   // Source lane s addresses token t0 + s / 4, columns 4 * (s % 4).. of the group's 16, so lane i gets tokens t0..t0+3 of
-  // column i; lanes 0..31 take tokens 0..7 of an instruction's 16 (t0 = 0, 4), lanes 32..63 tokens 8..15.
-  const int s16 = lane & 15, jbase = ((lane >> 4) & 1) * 16;
-  const uint32_t token0 = (uint32_t)(lh * 8 + (s16 >> 2));
+  // column i; the lanes of block b of FR lanes take tokens 8b .. 8b + 7 of an instruction's (t0 = 8b, 8b + 4).
+  const int s16 = lane & 15, jbase = C::FR == 32 ? ((lane >> 4) & 1) * 16 : 0;
+  const uint32_t token0 = (uint32_t)(lblock * 8 + (s16 >> 2));
   uint32_t a_off[C::TI], b_off[C::TJ];
 #pragma unroll
   for (int f = 0; f < C::TI; f++) {
@@ -174,13 +192,13 @@ grad_weight_pipe(const uint8_t* __restrict__ g, int64_t ldg, const uint8_t* __re
   }
 #pragma unroll
   for (int f = 0; f < C::TJ; f++) {
-    const uint32_t c = (uint32_t)((wj * C::TJ + f) * 32 + jbase + (s16 & 3) * 4);
+    const uint32_t c = (uint32_t)((wj * C::TJ + f) * C::FR + jbase + (s16 & 3) * 4);
     b_off[f] = C::OPERAND + token0 * C::ROW_BYTES + (((c >> 3) ^ C::swizzle(token0)) * 16) + ((c >> 2) & 1) * 8;
   }
   // the reads of a step in the order in which the next step's instructions need them: G's fragment 0, X's, G's others
   short4v af[2][C::TI][2], bf[2][C::TJ][2];
   auto read_one = [&](int set, int q, uint32_t buf, int step) {
-    const uint8_t* base = smem + buf + step * (16 * C::ROW_BYTES) + (q & 1) * (4 * C::ROW_BYTES);
+    const uint8_t* base = smem + buf + step * (C::STEP_TOKENS * C::ROW_BYTES) + (q & 1) * (4 * C::ROW_BYTES);
     const int f = q >> 1;
     if (f >= 1 && f <= C::TJ) bf[set][f - 1][q & 1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4_ptr)(lds_ptr_t)(base + b_off[f - 1]));
     else af[set][f ? f - C::TJ : 0][q & 1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4_ptr)(lds_ptr_t)(base + a_off[f ? f - C::TJ : 0]));
@@ -215,29 +233,29 @@ grad_weight_pipe(const uint8_t* __restrict__ g, int64_t ldg, const uint8_t* __re
       __builtin_amdgcn_sched_barrier(0);
     }
   };
-  auto next_buf = [](uint32_t b) { return b + C::STAGE == kRing * C::STAGE ? 0u : b + C::STAGE; };
+  auto next_buf = [](uint32_t b) { return b + C::STAGE == C::RING * C::STAGE ? 0u : b + C::STAGE; };
 
   copy_stage(0, 0);
   if (nstages > 1) copy_stage(1, C::STAGE);
-  if (nstages > 2) copy_stage(2, 2 * C::STAGE);
+  if (C::AHEAD > 2 && nstages > 2) copy_stage(2, 2 * C::STAGE);
   arrive(0, 0);
 #pragma unroll
   for (int q = 0; q < C::READS; q++) read_one(0, q, 0, 0);
-  uint32_t cur = 0, far = 3 * C::STAGE;                            // buffers of stage st and of stage st + 3
-  if (nstages > 3) copy_stage(3, far);
+  uint32_t cur = 0, far = C::AHEAD * C::STAGE;                     // buffers of stage st and of stage st + AHEAD
+  if (nstages > C::AHEAD) copy_stage(C::AHEAD, far);
   mma_step(0, true, cur, 1, 0, false, 0, 0);
   const int whole = ragged_stage < 0 ? nstages : nstages - 1;    // stages whose copies take the common form
   int st = 1;
-  for (; st + 3 < whole; st++) {
+  for (; st + C::AHEAD < whole; st++) {
     cur = next_buf(cur); far = next_buf(far);
-    wait_copies_and_barrier<4 * C::COPIES, false>();
-    mma_step(1, true, cur, 0, 0, true, st + 3, far);             // the last step of stage st - 1
-    mma_step(0, true, cur, 1, 1, true, st + 3, far);
+    wait_copies_and_barrier<(C::AHEAD - 1) * 2 * C::COPIES, READS_TOO>();
+    mma_step(1, true, cur, 0, 0, true, st + C::AHEAD, far);      // the last step of stage st - 1
+    mma_step(0, true, cur, 1, 1, true, st + C::AHEAD, far);
   }
   for (; st < nstages; st++) {
     cur = next_buf(cur); far = next_buf(far);
     arrive(st, cur);
-    if (st + 3 < nstages) copy_ragged(st + 3, far);
+    if (st + C::AHEAD < nstages) copy_ragged(st + C::AHEAD, far);
     mma_step(1, true, cur, 0, 0, false, 0, 0);
     mma_step(0, true, cur, 1, 0, false, 0, 0);
   }
@@ -246,9 +264,11 @@ grad_weight_pipe(const uint8_t* __restrict__ g, int64_t ldg, const uint8_t* __re
   if (SUMS && at.tile_j == 0) {
 #pragma unroll
     for (int h = 0; h < C::SUMS; h++) {
-      const float v = colsum[h] + __shfl_xor(colsum[h], 32);
-      const int64_t row = i0 + C::fragment_row(wave, h) + l32;
-      if (lh == 0) {
+      float v = colsum[h];
+      if (C::FR == 16) v += __shfl_xor(v, 16);
+      v += __shfl_xor(v, 32);
+      const int64_t row = i0 + C::fragment_row(wave, h) + lrow;
+      if (lblock == 0) {
         if (splits > 1) sums[(int64_t)at.split * tiles_i * C::TILE + row] = v;
         else if (row < m) db[row] = rounded<T, OutT>(v);
       }
@@ -258,18 +278,18 @@ grad_weight_pipe(const uint8_t* __restrict__ g, int64_t ldg, const uint8_t* __re
     float* out = partial + (int64_t)unit * (C::TILE * C::TILE) + tid * 4;
 #pragma unroll
     for (int s = 0; s < C::SLABS; s++) {
-      const float16v& v = acc[s / (4 * C::TJ)][(s >> 2) % C::TJ];
-      const int r = (s & 3) * 4;
+      const auto& v = acc[s / (C::QUADS * C::TJ)][s / C::QUADS % C::TJ];
+      const int r = s % C::QUADS * 4;
       *reinterpret_cast<float4v*>(out + s * (C::THREADS * 4)) = float4v{v[r], v[r + 1], v[r + 2], v[r + 3]};
     }
     return;
   }
 #pragma unroll
   for (int s = 0; s < C::SLABS; s++) {
-    const int64_t row = i0 + C::fragment_row(wave, s / (4 * C::TJ)) + (s & 3) * 8 + lh * 4, col = j0 + (wj * C::TJ + (s >> 2) % C::TJ) * 32 + l32;
+    const int64_t row = i0 + C::slab_row(wave, lane, s), col = j0 + C::slab_col(wave, lane, s);
     if (row < m && col < n) {
 #pragma unroll
-      for (int r = 0; r < 4; r++) dw[(row + r) * n + col] = rounded<T, OutT>(acc[s / (4 * C::TJ)][(s >> 2) % C::TJ][(s & 3) * 4 + r]);
+      for (int r = 0; r < 4; r++) dw[(row + r) * n + col] = rounded<T, OutT>(acc[s / (C::QUADS * C::TJ)][s / C::QUADS % C::TJ][s % C::QUADS * 4 + r]);
     }
     __builtin_amdgcn_sched_barrier(0);
   }
@@ -291,8 +311,7 @@ grad_weight_reduce(const float* __restrict__ partial, const float* __restrict__ 
   }
   const Piece at = locate((int)blockIdx.x, tiles_i, tiles_j);
   const int lane = tid & 63, wave = tid >> 6, s = (int)blockIdx.y;
-  const int64_t row = (int64_t)at.tile_i * C::TILE + C::fragment_row(wave, s / (4 * C::TJ)) + (s & 3) * 8 + (lane >> 5) * 4;
-  const int64_t col = (int64_t)at.tile_j * C::TILE + ((wave % C::WAVES_J) * C::TJ + (s >> 2) % C::TJ) * 32 + (lane & 31);
+  const int64_t row = (int64_t)at.tile_i * C::TILE + C::slab_row(wave, lane, s), col = (int64_t)at.tile_j * C::TILE + C::slab_col(wave, lane, s);
   if (row >= m || col >= n) return;
   const float* first = partial + (int64_t)blockIdx.x * (C::TILE * C::TILE) + s * (C::THREADS * 4) + tid * 4;
   const int64_t piece = (int64_t)ntiles * (C::TILE * C::TILE);
@@ -325,9 +344,9 @@ int64_t piece_bytes(int64_t tiles_i, int64_t tiles_j) { return (tiles_i * tiles_
 struct Pieces { int count; double us; };
 template <typename C>
 Pieces choose_pieces(int64_t tokens, int64_t m, int64_t n, int64_t workspace_bytes) {
-  constexpr double STAGE_US = std::is_same<C, Wide>::value ? 0.6 : 0.36;
+  constexpr double STAGE_US = std::is_same<C, Wide>::value ? 0.6 : 0.36;               // of 32 tokens
   const int64_t tiles_i = (m + C::TILE - 1) / C::TILE, tiles_j = (n + C::TILE - 1) / C::TILE;
-  const int64_t stages = (tokens + kStageTokens - 1) / kStageTokens, tiles = tiles_i * tiles_j;
+  const int64_t stages = (tokens + 31) / 32, tiles = tiles_i * tiles_j;
   Pieces best{1, (double)(stages * ((tiles + 255) / 256)) * STAGE_US};
   for (int64_t p = 2; p <= kMaxPieces && p <= stages / 4 && p * tiles <= 256 && p * piece_bytes<C>(tiles_i, tiles_j) <= workspace_bytes; p++) {
     const double us = (double)((stages + p - 1) / p) * STAGE_US + 3.0 + (double)(p * tiles) * (C::TILE * C::TILE * 4e-6 * 0.32);
@@ -337,6 +356,18 @@ Pieces choose_pieces(int64_t tokens, int64_t m, int64_t n, int64_t workspace_byt
 }
 bool takes_square(int64_t tokens, int64_t m, int64_t n, int64_t workspace_bytes) {
   return choose_pieces<Square>(tokens, m, n, workspace_bytes).us < 0.97 * choose_pieces<Wide>(tokens, m, n, workspace_bytes).us;
+}
+
+// 192 x 192 tiles of at least kLongTokens tokens on at least kLongBlocks compute units are bound by power, and take 16 x 16 instructions: alone, on
+// random operands in registers, those sustain 1.9 PFLOP/s where the 32 x 32 ones do 1.65.  Their stages are of 64 tokens, three buffers of
+// 48 KB.  us on 32 x 32 instructions and on these: 3072 x 768 over 12288 tokens (256 blocks of 3072) 72.3 and 69.6, 768 x 3072 70.9 and 67.8,
+// 2048 x 512 over 16384 (231 of 2340) 54.2 and 52.4, 5120 x 1280 over 4423 (189 of 4423) 72.0 and 67.8; fewer blocks or tokens, where the longer
+// first stage shows: 1024 x 4096 over 2000 (132 of 2000) 33.5 and 34.5, 3072 x 768 over 745 17.2 and 17.8, 512 x 2048 over 5000 25.7 and 26.7.
+constexpr int64_t kLongTokens = 1024, kLongBlocks = 160;
+bool takes_long(int64_t tokens, int64_t m, int64_t n, int64_t workspace_bytes) {
+  const int64_t pieces = choose_pieces<Square>(tokens, m, n, workspace_bytes).count;
+  const int64_t tiles = (m + Square::TILE - 1) / Square::TILE * ((n + Square::TILE - 1) / Square::TILE);
+  return tiles * pieces >= kLongBlocks && tokens >= kLongTokens * pieces;
 }
 
 template <typename T, typename OutT, typename C>
@@ -361,7 +392,8 @@ int launch(const void* g, int64_t ldg, const void* x, int64_t ldx, int64_t token
 template <typename T, typename OutT>
 int launch_either(const void* g, int64_t ldg, const void* x, int64_t ldx, int64_t tokens, int64_t m, int64_t n, void* dw, void* db,
                   void* workspace, int64_t workspace_bytes, hipStream_t s) {
-  auto* go = takes_square(tokens, m, n, workspace ? workspace_bytes : 0) ? launch<T, OutT, Square> : launch<T, OutT, Wide>;
+  const int64_t bytes = workspace ? workspace_bytes : 0;
+  auto* go = !takes_square(tokens, m, n, bytes) ? launch<T, OutT, Wide> : takes_long(tokens, m, n, bytes) ? launch<T, OutT, SquareLong> : launch<T, OutT, Square>;
   return go(g, ldg, x, ldx, tokens, m, n, dw, db, workspace, workspace_bytes, s);
 }
 
