@@ -18,6 +18,8 @@ class Library:
     def __getattr__(self, name):
         if name == "tf24_linear16_suits":
             return lambda rows, k, tokens: int(tokens > 0 and rows % 8 == 0 and k % 64 == 0 and k >= 256)
+        if name == "tf24_grad_weight_workspace_bytes":
+            return lambda *sizes: 0
         return lambda *args: (self.calls.append(name), 0)[1]
 
 
@@ -92,3 +94,18 @@ def test_weights_that_a_hook_unpacks_otherwise_are_left_to_torch(library, weight
             with pytest.raises(RuntimeError):
                 torch.mm(dy, weight)
     assert library.calls == []
+
+
+@pytest.mark.parametrize("x,taken", [
+    (draw(512, 256), True), (draw(512, 256, device="meta"), False), (draw(384, 256), False), (draw(512, 256).as_subclass(Derived), False)])
+def test_activations_that_a_hook_unpacks_otherwise_are_left_to_torch(library, x, taken):
+    """dW = dY^T x: an activation with fewer rows than the gradient would be read past its end."""
+    from sparse.sparse_ops import _linear16_backward
+    dy = draw(512, 384)
+    with torch.no_grad():
+        if not taken and x.shape[0] != 512:
+            with pytest.raises(RuntimeError):
+                _linear16_backward(dy, x, None, False, True, True)
+        else:
+            assert _linear16_backward(dy, x, None, False, True, True)[1].shape == (384, 256)
+    assert library.calls.count("tf24_grad_weight") == int(taken)
