@@ -3,7 +3,7 @@
     python 2by4-pretrain_amd/build.py [-j N] [--force]
 
 Objects go to 2by4-pretrain_amd/build/, the library next to the Python package that loads it
-(2by4-pretrain_amd/sparse/lib2by4_gfx950.so), beside it _fastcall.so, through which Python makes the frequent calls.
+(2by4-pretrain_amd/sparse/lib2by4_gfx950.so), beside it _fastcall.abi3.so, through which Python makes the frequent calls.
 """
 import argparse
 import concurrent.futures
@@ -18,7 +18,7 @@ CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(HERE, "build")
 LIB = os.path.join(HERE, "sparse", "lib2by4_gfx950.so")
 
-FASTCALL = os.path.join(HERE, "sparse", "_fastcall.so")
+FASTCALL = os.path.join(HERE, "sparse", "_fastcall.abi3.so")
 CXX = os.environ.get("CXX", "g++")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [
@@ -48,6 +48,23 @@ def _compile(src, force):
     return obj, res.stderr
 
 
+def build_fastcall():
+    """The CPython module over the library, of the stable ABI.  It finds the library beside itself, whatever LD_LIBRARY_PATH holds (hence
+    no new dtags).  Without Python's headers it is left out: ctypes makes its calls."""
+    stale = os.path.join(os.path.dirname(FASTCALL), "_fastcall.so")
+    if os.path.exists(stale):                                       # (built for one version of Python, without saying so in its name)
+        os.remove(stale)
+    include = sysconfig.get_paths()["include"]
+    if not os.path.exists(os.path.join(include, "Python.h")):
+        print(f"no Python.h under {include}: frequent calls will go through ctypes", file=sys.stderr)
+        return
+    cmd = [CXX, "-O2", "-std=c++17", "-shared", "-fPIC", "-I", os.path.join(ROOT, "include"), "-I", include, os.path.join(CSRC, "fastcall.cpp"), "-o", FASTCALL,
+           "-L", os.path.dirname(LIB), "-l:" + os.path.basename(LIB), "-Wl,--disable-new-dtags,-rpath,$ORIGIN", "-Wl,--allow-shlib-undefined"]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode:
+        raise RuntimeError(f"building the CPython module failed:\n{res.stdout}\n{res.stderr}")
+
+
 def build_library(jobs=8, force=True, verbose=False):
     os.makedirs(OBJ, exist_ok=True)
     with concurrent.futures.ThreadPoolExecutor(max_workers=max(1, jobs)) as pool:
@@ -61,13 +78,7 @@ def build_library(jobs=8, force=True, verbose=False):
     res = subprocess.run(cmd, capture_output=True, text=True)
     if res.returncode:
         raise RuntimeError(f"link failed:\n{res.stdout}\n{res.stderr}")
-    # the CPython module over the library (found next to it at run time)
-    cmd = [CXX, "-O2", "-std=c++17", "-shared", "-fPIC", "-I", os.path.join(ROOT, "include"), "-I", sysconfig.get_paths()["include"],
-           os.path.join(CSRC, "fastcall.cpp"), "-o", FASTCALL, "-L", os.path.dirname(LIB), "-l:" + os.path.basename(LIB), "-Wl,-rpath,$ORIGIN",
-           "-Wl,--allow-shlib-undefined"]
-    res = subprocess.run(cmd, capture_output=True, text=True)
-    if res.returncode:
-        raise RuntimeError(f"building the CPython module failed:\n{res.stdout}\n{res.stderr}")
+    build_fastcall()
     return LIB
 
 

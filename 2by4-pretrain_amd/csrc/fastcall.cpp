@@ -2,9 +2,10 @@
 //
 // ctypes converts each argument through a Python object of its own: 1.5 us for 10 arguments, 2.4 for the 20 of tf24_spmm, of the 11 us that
 // torch.nn.functional.linear with a 2:4 weight takes.  Here the argument types come from the declarations in tf24.h, and a call takes what
-// its conversions do.  As with ctypes a pointer is an address, bytes or None, an integer is taken modulo the size of its type, and other
-// Python threads run while the call does.
+// its conversions do.  As with ctypes a pointer is an address, bytes, None or an object of ctypes, an integer is taken modulo the size of its type,
+// and other Python threads run while the call does.  Only the stable ABI is used: one binary for every CPython from 3.10 on.
 #define PY_SSIZE_T_CLEAN
+#define Py_LIMITED_API 0x030a0000
 #include <Python.h>
 #include <cstdint>
 #include <tuple>
@@ -14,21 +15,49 @@
 
 namespace {
 
+// address that an object of ctypes (a pointer, an array, byref(..)) stands for
+bool ctypes_address(PyObject* o, void*& out) {
+  PyObject *ctypes = nullptr, *type = nullptr, *cast = nullptr, *value = nullptr;
+  if (!PyUnicode_Check(o) && (ctypes = PyImport_ImportModule("ctypes")) && (type = PyObject_GetAttrString(ctypes, "c_void_p")) &&
+      (cast = PyObject_CallMethod(ctypes, "cast", "OO", o, type)))
+    value = PyObject_GetAttrString(cast, "value");
+  const bool ok = value && (value == Py_None || PyLong_Check(value));
+  if (ok) out = value == Py_None ? nullptr : (void*)(uintptr_t)PyLong_AsUnsignedLongLongMask(value);
+  Py_XDECREF(value); Py_XDECREF(cast); Py_XDECREF(type); Py_XDECREF(ctypes);
+  if (!ok) PyErr_SetString(PyExc_TypeError, "a pointer is given as an address, bytes, None or an object of ctypes");
+  return ok;
+}
+
+template <typename T>
+bool number(PyObject* o, T& out) {
+  if constexpr (std::is_floating_point_v<T>) out = (T)PyFloat_AsDouble(o);
+  else out = (T)PyLong_AsUnsignedLongLongMask(o);                // (a float has no __index__: TypeError)
+  return out != (T)-1 || !PyErr_Occurred();                      // (either returns -1 with an error)
+}
+
 template <typename T>
 bool from_object(PyObject* o, T& out) {
   if constexpr (std::is_pointer_v<T>) {
-    out = nullptr;
-    if (o == Py_None) return true;
-    if (PyBytes_Check(o)) { out = (T)PyBytes_AS_STRING(o); return true; }       // (held by the caller's arguments)
-    if (!PyLong_Check(o)) { PyErr_SetString(PyExc_TypeError, "a pointer is given as an address, bytes or None"); return false; }
-    out = (T)(uintptr_t)PyLong_AsUnsignedLongLongMask(o);
-  } else if constexpr (std::is_floating_point_v<T>) {
-    out = (T)PyFloat_AsDouble(o);
+    void* at = nullptr;
+    if (o == Py_None) at = nullptr;
+    else if (PyLong_Check(o)) at = (void*)(uintptr_t)PyLong_AsUnsignedLongLongMask(o);
+    else if (PyBytes_Check(o)) at = PyBytes_AsString(o);         // (held by the caller's arguments)
+    else if (!ctypes_address(o, at)) return false;
+    out = (T)at;
+    return true;
   } else {
-    static_assert(std::is_integral_v<T>, "tf24.h passes pointers, floating-point numbers and integers");
-    out = (T)PyLong_AsUnsignedLongLongMask(o);                   // (a float has no __index__: TypeError)
+    static_assert(std::is_floating_point_v<T> || std::is_integral_v<T>, "tf24.h passes pointers, floating-point numbers and integers");
+    if (number(o, out)) return true;
+    PyObject *type, *error, *trace;                              // a number of ctypes holds it as its `value`
+    PyErr_Fetch(&type, &error, &trace);
+    PyObject* value = PyObject_HasAttrString(o, "_type_") ? PyObject_GetAttrString(o, "value") : nullptr;
+    PyErr_Clear();
+    const bool ok = value && number(value, out);
+    Py_XDECREF(value);
+    if (ok || PyErr_Occurred()) { Py_XDECREF(type); Py_XDECREF(error); Py_XDECREF(trace); }
+    else PyErr_Restore(type, error, trace);
+    return ok;
   }
-  return !PyErr_Occurred();
 }
 
 template <auto FN, typename R, typename... A, size_t... I>

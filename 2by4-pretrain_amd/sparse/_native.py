@@ -1,5 +1,6 @@
 """Binding of lib2by4_gfx950.so (C ABI declared in include/tf24.h): ctypes, and for the frequent calls the CPython module
-_fastcall.so over the same library (csrc/fastcall.cpp), which takes the same arguments.
+_fastcall.abi3.so over the same library (csrc/fastcall.cpp), which takes the same arguments.  Where that module is missing or does not load,
+ctypes makes its calls too, some 2 us slower each.
 
 There is no fallback: if the library is missing or a call fails, a RuntimeError is raised.
 Every wrapper enqueues on torch's current HIP stream and passes raw device pointers.
@@ -92,7 +93,10 @@ def lib():
             fn = getattr(handle, name)          # AttributeError if the library lacks a declared symbol
             fn.restype = res
             fn.argtypes = args
-        from . import _fastcall                 # (ImportError if it has not been built)
+        try:
+            from . import _fastcall
+        except ImportError:                     # not built, or not for this Python
+            _fastcall = None
         for name in _SIGNATURES:
             if hasattr(_fastcall, name):
                 setattr(handle, name, getattr(_fastcall, name))

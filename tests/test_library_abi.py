@@ -335,3 +335,58 @@ def test_fast_calls_take_what_ctypes_takes():
             assert fast.tf24_spmm_workspace_bytes(code, *shape) == slow.tf24_spmm_workspace_bytes(code, *shape)
     assert fast.tf24_linear16_suits(2 ** 64 + 3072, 768, 12288) == slow.tf24_linear16_suits(2 ** 64 + 3072, 768, 12288) == 1      # modulo 2^64, as ctypes does
     assert fast.tf24_adamw_masked_decay_list(b"", 0, 0, 0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0, None) == slow.tf24_adamw_masked_decay_list(b"", 0, 0, 0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0, None)
+
+
+def test_fast_calls_take_numbers_and_objects_of_ctypes():
+    """Floating-point arguments arrive as they are (the refusal of hyper-parameters names them), and what ctypes takes besides plain numbers is taken."""
+    from sparse import _native as N
+    fast = N.lib()
+    slow = ctypes.CDLL(N.library_path())
+    slow.tf24_last_error.restype = ctypes.c_char_p
+    slow.tf24_adamw_masked_decay_list.argtypes = N._SIGNATURES["tf24_adamw_masked_decay_list"][1]
+    slow.tf24_decompress.argtypes = N._SIGNATURES["tf24_decompress"][1]
+    outcomes = []
+    for numbers in ((1e-3, 1.25, 0.999, 1e-8, 0.0, 0.0), (2, -0.5, 0.875, 3e-7, 1, 0), tuple(map(ctypes.c_double, (1e-3, 1.25, 0.999, 1e-8, 0.0, 0.0)))):
+        for lib in (fast, slow):
+            assert lib.tf24_adamw_masked_decay_list(None, 0, 0, 0, *numbers, 1, None) != 0
+            outcomes.append(lib.tf24_last_error())
+        assert outcomes[-1] == outcomes[-2]
+    assert outcomes[0] == outcomes[4] and b"lr 0.001, eps 1e-08, betas 1.25 0.999" in outcomes[0] and b"lr 2, eps 3e-07, betas -0.5 0.875" in outcomes[2]
+    # pointers: a misaligned one is refused before anything is read from it
+    buffer = (ctypes.c_char * 80)()
+    at = ctypes.addressof(buffer) | 1
+    odd = (ctypes.c_char * 8).from_address(at)
+    for lib in (fast, slow):
+        for values in (at, ctypes.c_void_p(at), odd, ctypes.byref(odd), ctypes.pointer(odd)):
+            assert lib.tf24_decompress(values, N.F16, ctypes.c_void_p(64), ctypes.c_int(0), ctypes.c_int64(32), 64, 64, None) != 0
+            assert b"aligned" in lib.tf24_last_error(), lib.tf24_last_error()
+        with pytest.raises((TypeError, ctypes.ArgumentError)):
+            lib.tf24_decompress(1.5, N.F16, 64, 0, 32, 64, 64, None)
+
+
+@pytest.mark.parametrize("missing", [True, False])
+def test_library_loads_without_the_cpython_module(missing, monkeypatch):
+    """Not built, or built for another interpreter: ctypes makes the calls.  Only a missing library is an error, and says how to build it."""
+    import sys
+
+    import sparse
+    from sparse import _native as N
+    N.lib()
+    monkeypatch.setattr(N, "_lib", None)
+    monkeypatch.delattr(sparse, "_fastcall", raising=False)
+    if missing:
+        monkeypatch.setitem(sys.modules, "sparse._fastcall", None)           # (its import raises ImportError)
+        lib = N.lib()
+        assert isinstance(lib.tf24_spmm, ctypes._CFuncPtr) and lib.tf24_linear16_suits(3072, 768, 12288) == 1
+    else:
+        monkeypatch.setattr(N, "library_path", lambda: os.path.join(ROOT, "nowhere", "lib2by4_gfx950.so"))
+        with pytest.raises(RuntimeError, match="build.py"):
+            N.lib()
+
+
+def test_cpython_module_says_which_interpreters_it_fits():
+    import importlib.machinery
+
+    from sparse import _fastcall
+    suffix = os.path.basename(_fastcall.__file__)[len("_fastcall"):]
+    assert suffix == ".abi3.so" and suffix in importlib.machinery.EXTENSION_SUFFIXES
