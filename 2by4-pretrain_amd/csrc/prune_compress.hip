@@ -67,10 +67,13 @@ __device__ __forceinline__ void store_panel_meta_block(const uint32_t* s_words, 
 //   (32 x 256 when m is not a multiple of 64): 2^lpr_shift lanes read consecutive columns of one row,
 //   the other lanes of the wave take the next rows, so that every store instruction writes, per
 //   panel, the contiguous 64-byte pieces of 4 (2) adjacent rows.
-// The magnitude rule reads and writes with ordinary accesses: a weight that it compresses is multiplied by, or taken apart
-// (values, dense form), next, and what it wrote is then still in the last cache.  float32 8192 x 8192 to fp16, compressed and
-// both taken 123.7 -> 118.0 us, 8192 x 4096 to bf16 75.9 -> 70.0; compressed alone, over and over, 59.0 and 59.1.  The other modes
-// stream: mask-driven fp32 8192 x 8192 66.1 us and 71.7 with ordinary accesses, bf16 42.0 and 45.0.
+// The magnitude rule streams what it reads and stores ordinarily: a weight that it compresses is multiplied by, or taken apart
+// (values, dense form), next, and what it wrote is then still in the last cache; the dense weight is not read again.  On weights that change
+// from call to call, us: everything streamed, ordinary stores, ordinary loads as well.  float32 8192 x 8192 to fp16 with its values,
+// metadata and dense form 122.9, 118.9, 118.1, with a product of 128 rows 91.5, 86.8, 95.0, by itself 59.2, 63.5, 60.8; 8192 x 4096 to bf16
+// taken apart 75.1, 71.1, 69.8, by itself 36.4, 37.3, 36.7.  By itself a compression is slower for its stores' later write-back; with the
+// use of its result it is the faster one, or, before a product of thousands of rows, even (bf16 8192 x 8192, 2048 rows 168.4, 168.9, 167.1).
+// The other modes stream both ways: mask-driven fp32 8192 x 8192 66.1 us and 71.7 with ordinary accesses, bf16 42.0 and 45.0.
 // Rows and units of the panel form are 32-bit numbers (the grid bounds both), combined to 64-bit offsets by a
 // multiply-add: formed in 64 bits throughout, and for both forms of output in one kernel,
 // the addresses were a fifth of the MVUE24 conversion's vector instructions.
@@ -112,8 +115,7 @@ prune_compress_row(const In* __restrict__ dense, int64_t ld, int64_t m, int64_t 
     }
     if (live) {
       Pack<In, 8> in;
-      if constexpr (MODE == TF24_PRUNE_MAGNITUDE) in.load(dense + (uint64_t)row * ld + (uint64_t)col8 * 8);
-      else in.load_stream(dense + (uint64_t)row * ld + (uint64_t)col8 * 8);
+      in.load_stream(dense + (uint64_t)row * ld + (uint64_t)col8 * 8);
       Pack<MaskT, 8> mk;
       float r[4] = {0.f, 0.f, 0.f, 0.f};
       if constexpr (MODE == TF24_PRUNE_MASK) mk.load_stream(mask + (uint64_t)row * mask_ld + (uint64_t)col8 * 8);
@@ -225,7 +227,7 @@ prune_compress_row_mvue_panel(const In* __restrict__ dense, int64_t ld, int64_t 
 // a third of the instructions of the float compares) and the four dense loads of a lane issued
 // before the first is used: with one load in flight per wave the kernel is bound by memory latency,
 // a wave alternating between waiting for its load and computing.  A unit that holds a NaN is handed
-// to the float compares, whose answer for NaN the integer order does not give.
+// to the float compares, whose answer for NaN the integer order does not give.  Streams both ways.
 template <typename In, typename Out>
 __global__ void __launch_bounds__(kThreads)
 prune_compress_row_mag16(const In* __restrict__ dense, int64_t ld, int64_t m, int64_t k,
@@ -311,8 +313,9 @@ prune_compress_row_mag16(const In* __restrict__ dense, int64_t ld, int64_t m, in
 // words of its quad for the 4 rows are one 16-byte piece of the [k/32][m] word matrix, stored by the quad leader
 // as it is.  (64 rows x 128 columns per block with 256-byte reads per row: 37.0 us at 8192 x 8192 bf16 -> fp16;
 // this kernel 35.5; the same without the exchange of the values, 64-byte pieces per store: 41.4.)
-// Ordinary accesses on both sides (see prune_compress_row): 35.2 -> 34.9 us, 11008 x 4096 24.8 -> 23.9; compressed and its values,
-// metadata and dense form taken 100.6 -> 95.9.
+// Streaming loads and ordinary stores (see prune_compress_row).  bf16 to fp16 on weights that change from call to call, us: everything streamed,
+// ordinary stores, ordinary loads as well.  8192 x 8192 with its values, metadata and dense form 99.1, 96.3, 95.7, with a product of 128 rows
+// 67.7, 62.2, 70.1, by itself 35.2, 38.0, 39.4; 11008 x 4096 71.2, 68.1, 67.8, then 51.9, 48.6, 48.5, then 25.0, 26.3, 27.4.
 template <typename In, typename Out>
 __global__ void __launch_bounds__(kThreads)
 prune_compress_row_mag16_panel(const In* __restrict__ dense, int64_t ld, int64_t m, int64_t k,
@@ -329,7 +332,7 @@ prune_compress_row_mag16_panel(const In* __restrict__ dense, int64_t ld, int64_t
 #pragma unroll
   for (int it = 0; it < 4; it++) {
     in[it] = u32x4{0, 0, 0, 0};
-    if (live) in[it] = *reinterpret_cast<const u32x4*>(dense + (row0 + it) * ld + col8 * 8);
+    if (live) in[it] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(dense + (row0 + it) * ld + col8 * 8));
   }
   // values: a lane's four 8-byte pieces are 64 bytes apart in the panel layout; the wave exchanges them through
   // a private LDS slice (rows padded by 128 bytes: both halves of a 64-lane read fall on all banks) so that a

@@ -70,3 +70,21 @@ def test_activation_forms_spill_nothing(tmp_path):
                    ("bf16_t", "bf16_t", "false", "true"), ("e4m3_t", "bf16_t", "false", "true"), ("e4m3_t", "f16_t", "false", "true"))]
     for name, lines in _assembly(tmp_path, kernels).items():
         assert not any("scratch_" in line for line in lines), name
+
+
+def test_compression_by_magnitude_streams_its_loads_only(tmp_path):
+    """What it reads leaves the caches to what it wrote, which is used next: streaming loads, ordinary stores."""
+    spec = importlib.util.spec_from_file_location("tf24_build", os.path.join(ROOT, "2by4-pretrain_amd", "build.py"))
+    build = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(build)
+    if not os.path.exists(build.HIPCC):
+        pytest.skip("no hipcc")
+    out = tmp_path / "prune_compress.s"
+    subprocess.run([build.HIPCC, *build.FLAGS, "--cuda-device-only", "-S", os.path.join(build.CSRC, "prune_compress.hip"), "-o", str(out)],
+                   check=True, capture_output=True)
+    text = out.read_text()
+    for kernel in ("prune_compress_row_mag16_panelINS_6bf16_tENS_5f16_tE", "prune_compress_rowIfNS_5f16_tELi0EhLb1E"):
+        (body,) = re.findall(rf"^_Z\w*{kernel}\w*:.*?^\.Lfunc_end", text, flags=re.S | re.M)
+        loads, stores = re.findall(r"global_load_dwordx4.*", body), re.findall(r"global_store_dwordx2.*", body)
+        assert loads and all(line.endswith(" nt") for line in loads), (kernel, loads)
+        assert stores and not any(line.endswith(" nt") for line in stores), (kernel, stores)
