@@ -167,18 +167,20 @@ prune_compress_row(const In* __restrict__ dense, int64_t ld, int64_t m, int64_t 
   }
 }
 
-// MVUE24 into the PANEL layout: the work assignment of prune_compress_row, one unit per lane.  Bound by the vector instructions of a
-// unit (377 in prune_compress_row, 340 here, about 2.6 cycles each with eight waves on a SIMD, whatever their kind): rows
-// and units are counted inside the block, whose corner is formed in scalar registers, and the quad leaders store their metadata words themselves,
-// which in the other modes, bound by memory, costs more than the way through LDS (see store_panel_meta_block).
+// MVUE24 into the PANEL layout: the work assignment of prune_compress_row, one unit per lane, 16 rows x 16 units to a block (a matrix
+// that is compressed has a multiple of 32 rows).  Bound by the vector instructions of a unit (377 in prune_compress_row, 340 here, about
+// 2.6 cycles each with eight waves on a SIMD, whatever their kind): rows and units are counted inside the block, whose corner is
+// formed in scalar registers, and the quad leaders store their metadata words themselves, which in the other modes, bound by memory,
+// costs more than the way through LDS (see store_panel_meta_block).
+constexpr uint32_t kMvueUnits = 16, kMvueRows = kThreads / kMvueUnits;
 template <typename In, typename Out>
 __global__ void __launch_bounds__(kThreads)
 prune_compress_row_mvue_panel(const In* __restrict__ dense, int64_t ld, int64_t m, int64_t k, RandSrc rs,
-                              Out* __restrict__ values, uint8_t* __restrict__ meta, int lpr_shift) {
+                              Out* __restrict__ values, uint8_t* __restrict__ meta) {
   constexpr uint32_t UPP = (128 / (uint32_t)sizeof(Out)) / 8;     // units per panel row (8 or 16)
-  const uint32_t upr = (uint32_t)(k >> 3), rows = kThreads >> lpr_shift;
-  const uint32_t row0 = blockIdx.y * rows, unit0 = blockIdx.x << lpr_shift;
-  const uint32_t row = threadIdx.x >> lpr_shift, unit = threadIdx.x & ((1u << lpr_shift) - 1u);        // in the block
+  const uint32_t upr = (uint32_t)(k >> 3);
+  const uint32_t row0 = blockIdx.y * kMvueRows, unit0 = blockIdx.x * kMvueUnits;
+  const uint32_t row = threadIdx.x / kMvueUnits, unit = threadIdx.x % kMvueUnits;        // in the block
   if (unit >= upr - unit0) return;               // (whole quads: upr is a multiple of 8)
   // the place of (row, unit) where a row of the matrix is `pitch` long and a unit of it `per_unit`: for the lane one multiply-add with
   // the low word of the pitch (the high word, which only absurdly wide matrices have, in a branch)
@@ -214,7 +216,7 @@ prune_compress_row_mvue_panel(const In* __restrict__ dense, int64_t ld, int64_t 
     for (int e = 0; e < 4; e++) x[e] = to_float(in.v[4 * i + e]);
     g[i] = mvue4<In>(x, r[2 * i], r[2 * i + 1], finite[i]);
   }
-  // (offsets inside the block fit 32 bits: the grid bounds the rows to two million)
+  // (offsets inside the block fit 32 bits: the grid bounds the rows to 65535 x 16)
   Out* to = values + ((uint64_t)(unit0 / UPP) * (uint64_t)m + row0) * (UPP * 4) + ((unit / UPP) * ((uint32_t)m * (UPP * 4)) + row * (UPP * 4) + unit % UPP * 4);
   from_float4<Out>(g[0].first, g[0].second, finite[0], g[1].first, g[1].second, finite[1]).store_stream(to);
   const uint32_t w = quad_bytes(g[0].nibble | (g[1].nibble << 4));
@@ -565,7 +567,7 @@ int launch(const void* dense, int layout, int64_t ld, int64_t m, int64_t k, cons
            RandSrc rs, void* values, void* meta, bool panel, float* rowsum_partial, hipStream_t stream) {
   if (layout == TF24_ROW_MAJOR) {
     constexpr int kUnroll = unroll_for<MODE>();
-    const int64_t per_block = kThreads * kUnroll;
+    constexpr int64_t per_block = kThreads * kUnroll;
     const bool contiguous = ld == k && (MODE != TF24_PRUNE_MASK || mask_ld == k) && (MODE != TF24_PRUNE_MVUE || rs.kind == RAND_SEEDED || rs.ld == (rs.kind == RAND_PACKED ? k / 2 : k));
     const int64_t total = m * (k >> 3);
     dim3 grid((unsigned)((total + per_block - 1) / per_block));
@@ -588,8 +590,9 @@ int launch(const void* dense, int layout, int64_t ld, int64_t m, int64_t k, cons
       hipLaunchKernelGGL((prune_compress_row_mag16<In, Out>), grid, dim3(kThreads), 0, stream,
                          (const In*)dense, ld, m, k, (Out*)values, (uint8_t*)meta, contiguous, panel, lpr_shift);
     } else if (MODE == TF24_PRUNE_MVUE && panel) {
+      static_assert(MODE != TF24_PRUNE_MVUE || per_block == kMvueRows * kMvueUnits, "one unit per lane");     // lpr_shift is 4: 16 divides m
       if constexpr (MODE == TF24_PRUNE_MVUE)
-        hipLaunchKernelGGL((prune_compress_row_mvue_panel<In, Out>), grid, dim3(kThreads), 0, stream, (const In*)dense, ld, m, k, rs, (Out*)values, (uint8_t*)meta, lpr_shift);
+        hipLaunchKernelGGL((prune_compress_row_mvue_panel<In, Out>), grid, dim3(kThreads), 0, stream, (const In*)dense, ld, m, k, rs, (Out*)values, (uint8_t*)meta);
     } else {
       auto go = [&](auto to_panel) {
         hipLaunchKernelGGL((prune_compress_row<In, Out, MODE, MaskT, decltype(to_panel)::value>), grid, dim3(kThreads), 0, stream,

@@ -354,8 +354,8 @@ def test_mvue_default_sampling_follows_torch_seed(cuda):
 @pytest.mark.parametrize("out_dtype", [F16, BF16, E4M3, E5M2])
 @pytest.mark.parametrize("in_dtype,shape,extra", [(BF16, (64, 128), 0), (F16, (96, 384), 8), (F32, (32, 2176), 64), (F32, (1056, 256), 0), (BF16, (160, 640), 24)])
 def test_mvue_panel_conversion(cuda, in_dtype, out_dtype, shape, extra):
-    """The kernel for row-major input and panel output: 16 or 8 rows to a block, rows of the matrix longer than its columns, partial
-    blocks on the right, uniforms from every source, groups whose largest element outweighs the others by up to 2^26 -- the bits of the oracle."""
+    """The kernel for row-major input and panel output: 16 rows x 128 columns to a block, rows of the matrix longer than its columns,
+    uniforms from every source, groups whose largest element outweighs the others by up to 2^26 -- the bits of the oracle."""
     import sparse
     m, k = shape
     g = torch.Generator().manual_seed(m + k)
@@ -370,6 +370,13 @@ def test_mvue_panel_conversion(cuda, in_dtype, out_dtype, shape, extra):
         s = sparse.to_sparse_semi_structured(wide.to(cuda)[:, :k], MVUE24=True, dtype=out_dtype, rand=rand)
         assert_same(s.indices(), want_m, "meta")
         assert_same(torch.nan_to_num(s.values().float().cpu(), 1.5), torch.nan_to_num(want_v.float(), 1.5), "values")
+
+
+@pytest.mark.parametrize("out_dtype", [F16, BF16])
+@pytest.mark.parametrize("in_dtype,shape,extra", [(F16, (64, 192), 0), (F32, (32, 64), 0), (BF16, (96, 1088), 8)])
+def test_mvue_panel_conversion_with_partial_blocks(cuda, in_dtype, out_dtype, shape, extra):
+    """Half a block on the right: an odd multiple of 64 columns, which only 16-bit values take."""
+    test_mvue_panel_conversion(cuda, in_dtype, out_dtype, shape, extra)
 
 
 def _wide_range(shape, seed):
