@@ -172,16 +172,21 @@ prune_compress_row(const In* __restrict__ dense, int64_t ld, int64_t m, int64_t 
 // 2.6 cycles each with eight waves on a SIMD, whatever their kind): rows and units are counted inside the block, whose corner is
 // formed in scalar registers, and the quad leaders store their metadata words themselves, which in the other modes, bound by memory,
 // costs more than the way through LDS (see store_panel_meta_block).
+// SEEDED: uniforms drawn here.  Otherwise they are of a [m, k] tensor, for 16-bit matrices only: a conversion that reads its uniforms is
+// bound by memory.  us in prune_compress_row and here: bf16 8192 x 8192 to fp16, seeded 59.6 and 57.7, [m, k] 79.1 and 77.1, [m, k/2]
+// 59.0 and 60.9; 11008 x 4096 40.3 and 39.9, 55.1 and 53.4, 40.3 and 42.6; float32 8192 x 8192 66.8 and 66.1, 99.0 and 99.9, 76.7 and 78.5.
+// Lanes past the matrix compute on its first unit of the block and store nothing: with an early return the arguments are fetched in two
+// turns, the second waiting for the first (3072 x 768 4.6 -> 4.5 us).
 constexpr uint32_t kMvueUnits = 16, kMvueRows = kThreads / kMvueUnits;
-template <typename In, typename Out>
+template <typename In, typename Out, bool SEEDED>
 __global__ void __launch_bounds__(kThreads)
 prune_compress_row_mvue_panel(const In* __restrict__ dense, int64_t ld, int64_t m, int64_t k, RandSrc rs,
                               Out* __restrict__ values, uint8_t* __restrict__ meta) {
   constexpr uint32_t UPP = (128 / (uint32_t)sizeof(Out)) / 8;     // units per panel row (8 or 16)
   const uint32_t upr = (uint32_t)(k >> 3);
   const uint32_t row0 = blockIdx.y * kMvueRows, unit0 = blockIdx.x * kMvueUnits;
-  const uint32_t row = threadIdx.x / kMvueUnits, unit = threadIdx.x % kMvueUnits;        // in the block
-  if (unit >= upr - unit0) return;               // (whole quads: upr is a multiple of 8)
+  const bool live = threadIdx.x % kMvueUnits < upr - unit0;       // (whole quads: upr is a multiple of 8)
+  const uint32_t row = threadIdx.x / kMvueUnits, unit = live ? threadIdx.x % kMvueUnits : 0;        // in the block
   // the place of (row, unit) where a row of the matrix is `pitch` long and a unit of it `per_unit`: for the lane one multiply-add with
   // the low word of the pitch (the high word, which only absurdly wide matrices have, in a branch)
   auto place = [&](uint64_t pitch, uint32_t per_unit) {
@@ -192,21 +197,20 @@ prune_compress_row_mvue_panel(const In* __restrict__ dense, int64_t ld, int64_t 
   Pack<In, 8> in;
   in.load_stream(dense + place((uint64_t)ld, 8));
   float r[4];
-  if (rs.kind == RAND_SEEDED) {
+  if constexpr (SEEDED) {
     Philox4 c[1];
     philox4x32_10_calls(rs.seed_now(), place(upr, 1), 0, rs.offset_now(), c);
     r[0] = philox_uniform(c[0].x); r[1] = philox_uniform(c[0].y); r[2] = philox_uniform(c[0].z); r[3] = philox_uniform(c[0].w);
-  } else if (rs.kind == RAND_PACKED) {           // [m, k/2]: the unit's four uniforms are adjacent
-    Pack<float, 4> r4;
-    r4.load_stream(rs.ptr + place((uint64_t)rs.ld, 4));
-    r[0] = r4.v[0]; r[1] = r4.v[1]; r[2] = r4.v[2]; r[3] = r4.v[3];
   } else {
     const float* rp = rs.ptr + place((uint64_t)rs.ld, 8);
     Pack<float, 2> ra, rb;                       // the group's two uniforms: the second load meets the first one's line in L1
     ra.load(rp);
     rb.load(rp + 4);
+    __builtin_amdgcn_sched_barrier(0);           // (the compiler sinks the second load below the wait for the matrix: 76 -> 80.5 us)
     r[0] = ra.v[0]; r[1] = ra.v[1]; r[2] = rb.v[0]; r[3] = rb.v[1];
   }
+  // (every argument is fetched by here, behind the wait for the matrix: one fetched where a store needs it is waited for there)
+  asm volatile("" ::"s"(values), "s"(meta), "s"(m));
   Mvue4 g[2];
   bool finite[2];
 #pragma unroll
@@ -218,9 +222,10 @@ prune_compress_row_mvue_panel(const In* __restrict__ dense, int64_t ld, int64_t 
   }
   // (offsets inside the block fit 32 bits: the grid bounds the rows to 65535 x 16)
   Out* to = values + ((uint64_t)(unit0 / UPP) * (uint64_t)m + row0) * (UPP * 4) + ((unit / UPP) * ((uint32_t)m * (UPP * 4)) + row * (UPP * 4) + unit % UPP * 4);
-  from_float4<Out>(g[0].first, g[0].second, finite[0], g[1].first, g[1].second, finite[1]).store_stream(to);
+  const Pack<Out, 4> kept = from_float4<Out>(g[0].first, g[0].second, finite[0], g[1].first, g[1].second, finite[1]);
+  if (live) kept.store_stream(to);
   const uint32_t w = quad_bytes(g[0].nibble | (g[1].nibble << 4));
-  if ((threadIdx.x & 3) == 0)
+  if (live && (threadIdx.x & 3) == 0)
     *reinterpret_cast<uint32_t*>(meta + ((uint64_t)(unit0 >> 2) * (uint64_t)m + row0) * 4 + ((unit >> 2) * ((uint32_t)m * 4) + row * 4)) = w;
 }
 
@@ -589,18 +594,22 @@ int launch(const void* dense, int layout, int64_t ld, int64_t m, int64_t k, cons
       }
       hipLaunchKernelGGL((prune_compress_row_mag16<In, Out>), grid, dim3(kThreads), 0, stream,
                          (const In*)dense, ld, m, k, (Out*)values, (uint8_t*)meta, contiguous, panel, lpr_shift);
-    } else if (MODE == TF24_PRUNE_MVUE && panel) {
+    } else if (MODE == TF24_PRUNE_MVUE && panel && (rs.kind == RAND_SEEDED || (rs.kind == RAND_FULL && sizeof(In) == 2))) {
       static_assert(MODE != TF24_PRUNE_MVUE || per_block == kMvueRows * kMvueUnits, "one unit per lane");     // lpr_shift is 4: 16 divides m
-      if constexpr (MODE == TF24_PRUNE_MVUE)
-        hipLaunchKernelGGL((prune_compress_row_mvue_panel<In, Out>), grid, dim3(kThreads), 0, stream, (const In*)dense, ld, m, k, rs, (Out*)values, (uint8_t*)meta);
+      auto go = [&](auto seeded) {
+        hipLaunchKernelGGL((prune_compress_row_mvue_panel<In, Out, decltype(seeded)::value>), grid, dim3(kThreads), 0, stream,
+                           (const In*)dense, ld, m, k, rs, (Out*)values, (uint8_t*)meta);
+      };
+      if constexpr (MODE == TF24_PRUNE_MVUE) {
+        if (rs.kind == RAND_SEEDED) go(std::true_type{});
+        else if constexpr (sizeof(In) == 2) go(std::false_type{});
+      }
     } else {
       auto go = [&](auto to_panel) {
         hipLaunchKernelGGL((prune_compress_row<In, Out, MODE, MaskT, decltype(to_panel)::value>), grid, dim3(kThreads), 0, stream,
                            (const In*)dense, ld, m, k, (const MaskT*)mask, mask_ld, rs, (Out*)values, (uint8_t*)meta, contiguous, lpr_shift);
       };
-      if constexpr (MODE == TF24_PRUNE_MVUE) go(std::false_type{});
-      else if (panel) go(std::true_type{});
-      else go(std::false_type{});
+      if (panel) go(std::true_type{}); else go(std::false_type{});
     }
   } else {
     constexpr int TR = 128 / sizeof(In);       // rows of a block's tile
