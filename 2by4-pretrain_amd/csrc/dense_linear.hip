@@ -20,7 +20,6 @@
 // first two thirds of them: alike.  Ordinary instead of streaming stores: 67 us for 61 (3072 x 768).
 #include "lds_copies.hpp"
 #include <algorithm>
-#include <atomic>
 #include <type_traits>
 
 namespace tf24 {
@@ -185,7 +184,6 @@ dense_linear(const uint8_t* __restrict__ w, int64_t ldw, const uint8_t* __restri
     if (more) wait_copies_and_barrier<2 * kCopies, true>();
     else wait_copies_and_barrier<0, true>();
   };
-  auto wait_reads_and_barrier = []() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
 
   copy_stage(0);
   copy_stage(kStage);
@@ -280,18 +278,6 @@ dense_linear(const uint8_t* __restrict__ w, int64_t ldw, const uint8_t* __restri
     rotate();
     clear();
   }
-}
-
-inline int compute_units() {
-  static std::atomic<int> cached[64];
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-  int n = cached[dev].load(std::memory_order_relaxed);
-  if (!n) {
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
-    cached[dev].store(n, std::memory_order_relaxed);
-  }
-  return n;
 }
 
 template <typename T>

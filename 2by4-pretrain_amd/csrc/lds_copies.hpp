@@ -1,7 +1,8 @@
 // What the kernels that stream operands through LDS into matrix instructions share: vector types, copies from memory straight
-// into LDS, and the waits that go with them.
+// into LDS, the waits that go with them, and the number of compute units that tiles are dealt to.
 #pragma once
 #include "tf24_common.hpp"
+#include <atomic>
 
 namespace tf24 {
 namespace {
@@ -39,6 +40,24 @@ template <int N, bool READS>
 __device__ __forceinline__ void wait_copies_and_barrier() {
   if constexpr (READS) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
   else asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(N) : "memory");
+}
+// workgroup barrier behind this wave's LDS reads only: copies stay in flight
+__device__ __forceinline__ void wait_reads_and_barrier() {
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
+// compute units of the current device (looked up once per device; the cache is a table of atomics: two threads
+// that meet on an empty entry both look the value up and store the same number)
+inline int compute_units() {
+  static std::atomic<int> cached[64];
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
+  int n = cached[dev].load(std::memory_order_relaxed);
+  if (!n) {
+    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
+    cached[dev].store(n, std::memory_order_relaxed);
+  }
+  return n;
 }
 
 }  // namespace

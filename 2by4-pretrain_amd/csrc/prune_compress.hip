@@ -831,8 +831,9 @@ mvue_uniforms_kernel(uint64_t seed, uint64_t offset, int64_t m, int64_t upr, boo
   const int64_t u = (int64_t)blockIdx.x * kThreads + threadIdx.x;
   if (u >= m * upr) return;
   const int64_t row = u / upr, unit = u - row * upr;
-  const Philox4 c = philox4x32_10(seed, (uint64_t)u, offset);
-  const float v[4] = {philox_uniform(c.x), philox_uniform(c.y), philox_uniform(c.z), philox_uniform(c.w)};
+  Philox4 c[1];
+  philox4x32_10_calls(seed, (uint64_t)u, 0, offset, c);
+  const float v[4] = {philox_uniform(c[0].x), philox_uniform(c[0].y), philox_uniform(c[0].z), philox_uniform(c[0].w)};
   if (col_major) {
 #pragma unroll
     for (int i = 0; i < 4; i++) out[(unit * 4 + i) * ld + row] = v[i];

@@ -17,7 +17,6 @@
 #pragma once
 #include "lds_copies.hpp"
 #include <algorithm>
-#include <atomic>
 #include <type_traits>
 
 namespace tf24 {
@@ -369,11 +368,6 @@ static_assert(kRotateMinStages - 2 - (7 * kRotateMinStages >> 3) >= 1, "the firs
 using SlimCfg = TileCfgT<1, 2>;
 // 256 x 128 tiles, four waves: dense operands of 65 to 128 columns
 using MidCfg = TileCfgT<2, 2>;
-
-// workgroup barrier behind this wave's LDS reads only: copies stay in flight
-__device__ __forceinline__ void wait_reads_and_barrier() {
-  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-}
 
 // ACTS: the kernel is built twice, for launches without an activation (output pass: plain or bias only) and with one
 // (bias or zeros, then ReLU, SiLU or GELU); with all five passes in one kernel the compiler no longer keeps the
@@ -1247,20 +1241,6 @@ bool strided_takes_square(int64_t n_sparse, int64_t k, int64_t n_dense, int64_t 
   const Pieces square = choose_pieces<T, SquareCfg>(n_sparse, k, n_dense, workspace_bytes, true);
   if (sizeof(OutT) == 2 && !c_jmajor && square.count == 1) return false;
   return us(SquareCfg{}, square) < 0.97 * us(TiledCfg{}, wide);
-}
-
-// compute units of the current device (looked up once per device; the cache is a table of atomics: two threads
-// that meet on an empty entry both look the value up and store the same number)
-inline int compute_units() {
-  static std::atomic<int> cached[64];
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-  int n = cached[dev].load(std::memory_order_relaxed);
-  if (!n) {
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
-    cached[dev].store(n, std::memory_order_relaxed);
-  }
-  return n;
 }
 
 template <typename T, typename OutT, typename C>

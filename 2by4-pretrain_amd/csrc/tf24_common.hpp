@@ -334,20 +334,10 @@ __device__ __forceinline__ float div_in_range(float a, float b, float r) {
 // the four uniforms of two adjacent groups: `index` = row * (k / 8) + (8-column unit of the row),
 // words 0,1 for the even group of the unit and 2,3 for the odd one.
 struct Philox4 { uint32_t x, y, z, w; };
-__host__ __device__ inline Philox4 philox4x32_10(uint64_t seed, uint64_t index, uint64_t offset) {
-  uint32_t c0 = (uint32_t)index, c1 = (uint32_t)(index >> 32), c2 = (uint32_t)offset, c3 = (uint32_t)(offset >> 32);
-  uint32_t k0 = (uint32_t)seed, k1 = (uint32_t)(seed >> 32);
-#pragma unroll
-  for (int round = 0; round < 10; round++) {
-    const uint64_t p0 = (uint64_t)0xD2511F53u * c0, p1 = (uint64_t)0xCD9E8D57u * c2;
-    const uint32_t n0 = (uint32_t)(p1 >> 32) ^ c1 ^ k0, n2 = (uint32_t)(p0 >> 32) ^ c3 ^ k1;
-    c0 = n0; c1 = (uint32_t)p1; c2 = n2; c3 = (uint32_t)p0;
-    k0 += 0x9E3779B9u; k1 += 0xBB67AE85u;
-  }
-  return Philox4{c0, c1, c2, c3};
-}
-// The calls for the counters index, index + stride, ... of one lane, with three-input exclusive ors (v_bitop3_b32): 40 + 2
-// vector instructions a call instead of 58, which is what kernels that sample are bound by (see mvue4).
+// The calls for the counters index, index + stride, ... of one lane.  The only generator here: uniforms that are written out are those that a
+// conversion draws, and saved seeds have to give the same bits as ever (the oracle has its own, pinned by known answers).  With
+// three-input exclusive ors (v_bitop3_b32) a call takes 40 + 2 vector instructions instead of 58, which is what kernels that sample are bound
+// by (see mvue4).
 template <int N>
 __device__ __forceinline__ void philox4x32_10_calls(uint64_t seed, uint64_t index, uint64_t stride, uint64_t offset, Philox4 (&out)[N]) {
   uint32_t k0 = (uint32_t)seed, k1 = (uint32_t)(seed >> 32);
