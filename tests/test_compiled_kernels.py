@@ -56,7 +56,8 @@ def test_chained_tiles_wait_only_at_the_stage_barrier(tmp_path):
                    ("f16_t", "f16_t", "TiledCfg", "false", "false"), ("f16_t", "f16_t", "TiledCfg", "true", "false"),
                    ("bf16_t", "bf16_t", "TiledCfg", "false", "false"), ("f16_t", "float", "TiledCfg", "false", "false"),
                    ("f16_t", "float", "TiledCfg", "true", "true"), ("f16_t", "f16_t", "SquareCfg", "false", "false"),
-                   ("f16_t", "f16_t", "Wave4Cfg", "false", "false"), ("f16_t", "f16_t", "Wave4Cfg192", "false", "false"))]
+                   ("f16_t", "f16_t", "Wave4Cfg", "false", "false"), ("f16_t", "f16_t", "Wave4Cfg192", "false", "false"),
+                   ("f16_t", "f16_t", "TallCfg", "false", "false"), ("bf16_t", "bf16_t", "TallCfg", "false", "true"))]
     for name, lines in _assembly(tmp_path, kernels).items():
         waits = [int(n) for line in _stage_loop(lines) for n in re.findall(r"vmcnt\((\d+)\)", line)]
         assert len(waits) == 1 and waits[0] > 0, (name, waits)
@@ -70,6 +71,14 @@ def test_activation_forms_spill_nothing(tmp_path):
                    ("bf16_t", "bf16_t", "false", "true"), ("e4m3_t", "bf16_t", "false", "true"), ("e4m3_t", "f16_t", "false", "true"))]
     for name, lines in _assembly(tmp_path, kernels).items():
         assert not any("scratch_" in line for line in lines), name
+
+
+def test_four_wave_forms_spill_outside_the_stage_loop_only(tmp_path):
+    """Tiles of the 4-wave forms keep every vector register, and what they put aside of the scalar ones stays aside while stages are multiplied."""
+    kernels = [f"f16_t, f16_t, true, {tile}, false, true, {acts}" for tile in ("TallCfg", "Wave4Cfg", "Wave4Cfg192", "SquareCfg") for acts in ("false", "true")]
+    for name, lines in _assembly(tmp_path, kernels).items():
+        assert not any("scratch_" in line for line in lines), name
+        assert not any("v_writelane" in line or "v_readlane" in line for line in _stage_loop(lines)), name
 
 
 def test_compression_by_magnitude_streams_its_loads_only(tmp_path):

@@ -958,7 +958,10 @@ def test_dense_linear_refuses_what_it_does_not_take(cuda):
         assert lib.tf24_linear16_suits(*shape) == 0
 
 
-@pytest.mark.parametrize("tokens,m,n", [(12289, 3072, 768), (1024, 3072, 2304), (1087, 3080, 2000), (2100, 1992, 3072)])
+MANY_LONG = [(12289, 3072, 768), (1024, 3072, 2304), (1087, 3080, 2000), (2100, 1992, 3072)]          # (test_tile_rules.py)
+
+
+@pytest.mark.parametrize("tokens,m,n", MANY_LONG)
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_grad_weight_kernel_on_many_long_tiles(cuda, tokens, m, n, dtype):
     """The products whose 192 x 192 tiles take stages of 64 tokens: last stages of 1, 64, 63 and 52 tokens, in four pieces and in one.  Bounds

@@ -7,6 +7,7 @@ import subprocess
 import pytest
 
 from test_gpu_parity import NOT_TALL, SQUARE, SQUARE_STRIDED, STAGE_ORDER, TALL
+from test_gpu_training import MANY_LONG
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 CU_SLOTS = 32                      # compute units of an XCD
@@ -92,3 +93,50 @@ def test_tall_tiles_where_they_are_the_faster_ones(rules, n, stages, columns, ta
 @pytest.mark.parametrize("n,stages,rows,tiles", NOT_TALL)
 def test_other_tiles_are_tested_with_16_bits_too(rules, n, stages, rows, tiles):
     assert rules.tiles_of_16_bits(n, rows, stages, CU_SLOTS) == {"wide, two launches": 101, "square": 3}[tiles]
+
+
+@pytest.fixture(scope="module")
+def dense_rules(tmp_path_factory):
+    spec = importlib.util.spec_from_file_location("tf24_build", os.path.join(ROOT, "2by4-pretrain_amd", "build.py"))
+    build = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(build)
+    if not os.path.exists(build.HIPCC):
+        pytest.skip("no hipcc")
+    folder = tmp_path_factory.mktemp("dense_rules")
+    handles = []
+    for source, rule in (
+            ("dense_linear.hip", "linear(int64_t rows, int64_t k, int64_t tokens) { return tf24::shapes_fit(rows, k, tokens) && tf24::suits(rows, k, tokens, 256); }"),
+            ("grad_weight.hip", "gradient(int64_t tokens, int64_t m, int64_t n) {\n"
+                                "  const int64_t any = (int64_t)1 << 40;\n"
+                                "  return !tf24::takes_square(tokens, m, n, any) ? 0 : tf24::takes_long(tokens, m, n, any) ? 2 : 1;\n}")):
+        src, lib = folder / ("rules_" + source), folder / (source + ".so")
+        # (the rules alone: no kernel is instantiated, and what the source shares with the rest of the library stays undefined)
+        src.write_text('#include "lds_copies.hpp"\n#undef hipLaunchKernelGGL\n#define hipLaunchKernelGGL(...) (void)0\n'
+                       f'#include "{source}"\nextern "C" int {rule}\n')
+        subprocess.run([build.HIPCC, *build.FLAGS, "--offload-host-only", "-shared", "-Wl,--unresolved-symbols=ignore-all", str(src), "-o", str(lib)],
+                       check=True, capture_output=True)
+        handles.append(ctypes.CDLL(str(lib), mode=os.RTLD_LAZY))
+    for handle, name in zip(handles, ("linear", "gradient")):
+        getattr(handle, name).argtypes = [ctypes.c_int64] * 3
+    return handles
+
+
+@pytest.mark.parametrize("rows,k,tokens,taken", [
+    # measured (us in the library, in the kernel): several rounds of tiles, filled to 0.89 and more or not
+    (3072, 768, 12288, 1), (768, 3072, 12288, 1), (2560, 640, 13317, 1),             # 60.1 56.3, 59.7 48.0, 58.6 44.8
+    (4096, 1024, 4053, 0), (6400, 1600, 2525, 0),                                    # 29.0 35.3, 40.2 51.9
+    # one round of long tiles (0.72) and of short ones (0.55)
+    (1600, 6400, 2831, 0), (640, 2560, 10655, 1), (5120, 1280, 1074, 1), (4096, 1024, 1256, 0),          # 62.5 77.5, 46.0 37.2, 22.9 20.2, 15.2 16.4
+    # what the kernel does not take at all
+    (3076, 768, 12288, 0), (3072, 800, 12288, 0), (3072, 192, 12288, 0), (3072, 768, 0, 0), (0, 768, 12288, 0)])
+def test_dense_products_are_taken_where_the_kernel_is_the_faster_one(dense_rules, rows, k, tokens, taken):
+    assert dense_rules[0].linear(rows, k, tokens) == taken
+
+
+@pytest.mark.parametrize("tokens,m,n,form", [
+    # measured (us on 32 x 32 instructions, on 16 x 16 ones): at least 160 blocks of at least 1024 tokens, or less
+    (12288, 3072, 768, 2), (12288, 768, 3072, 2), (16384, 2048, 512, 2), (4423, 5120, 1280, 2),          # 72.3 69.6, 70.9 67.8, 54.2 52.4, 72.0 67.8
+    (2000, 1024, 4096, 1), (745, 3072, 768, 1), (5000, 512, 2048, 1)]                                    # 33.5 34.5, 17.2 17.8, 25.7 26.7
+    + [(*sizes, 2) for sizes in MANY_LONG])
+def test_weight_gradients_take_long_tiles_where_they_are_the_faster_ones(dense_rules, tokens, m, n, form):
+    assert dense_rules[1].gradient(tokens, m, n) == form
