@@ -4,8 +4,9 @@
 //
 // G [tokens, m] and X [tokens, n] are read as they lie: the summed axis is the slow one of both.
 //
-// Bound by the matrix cores, and at this size by the power that they may draw: 12288 tokens, 3072 x 768 bf16 take 67
-// us with db (0.87 PFLOP/s; on 32 x 32 instructions 71, on 256 x 256 tiles 70, of zeros 54), where the library's product takes 110 to 140 us and its row sum 20 to 29.
+// Bound by the matrix cores, and at this size by the power that they may draw: 12288 tokens, 3072 x 768 bf16 take 62
+// us with db on one card (0.94 PFLOP/s; on 32 x 32 instructions 65, on 256 x 256 tiles 69, of zeros 55 on any; another card took 69.6 and
+// 72.3 for the first two), where the library's product takes 110 to 140 us and its row sum 20 to 29.
 //
 // A block multiplies a 256(i) x 256(j) tile over a piece of the token axis: eight waves (2 along i x 4 along j), two per
 // SIMD, wave tile 128 x 64 = 4 x 2 V_MFMA_F32_32X32X16.  (Four waves of 128 x 128 read a third less LDS, but nothing covers
@@ -360,9 +361,9 @@ bool takes_square(int64_t tokens, int64_t m, int64_t n, int64_t workspace_bytes)
 
 // 192 x 192 tiles of at least kLongTokens tokens on at least kLongBlocks compute units are bound by power, and take 16 x 16 instructions: alone, on
 // random operands in registers, those sustain 1.9 PFLOP/s where the 32 x 32 ones do 1.65.  Their stages are of 64 tokens, three buffers of
-// 48 KB.  us on 32 x 32 instructions and on these: 3072 x 768 over 12288 tokens (256 blocks of 3072) 72.3 and 69.6, 768 x 3072 70.9 and 67.8,
-// 2048 x 512 over 16384 (231 of 2340) 54.2 and 52.4, 5120 x 1280 over 4423 (189 of 4423) 72.0 and 67.8; fewer blocks or tokens, where the longer
-// first stage shows: 1024 x 4096 over 2000 (132 of 2000) 33.5 and 34.5, 3072 x 768 over 745 17.2 and 17.8, 512 x 2048 over 5000 25.7 and 26.7.
+// 48 KB.  us on 32 x 32 instructions and on these: 3072 x 768 over 12288 tokens (256 blocks of 3072) 65.2 and 62.5, 768 x 3072 65.5 and 63.7,
+// 2048 x 512 over 16384 (231 of 2340) 48.9 and 47.5, 5120 x 1280 over 4423 (189 of 4423) 65.8 and 63.9; fewer blocks or tokens, where the longer
+// first stage shows: 1024 x 4096 over 2000 (132 of 2000) 32.8 and 33.7, 3072 x 768 over 745 16.9 and 17.4, 512 x 2048 over 5000 24.6 and 25.2.
 constexpr int64_t kLongTokens = 1024, kLongBlocks = 160;
 bool takes_long(int64_t tokens, int64_t m, int64_t n, int64_t workspace_bytes) {
   const int64_t pieces = choose_pieces<Square>(tokens, m, n, workspace_bytes).count;
@@ -420,7 +421,7 @@ int run(const char* fn, bool f32, const void* g, int64_t ldg, const void* x, int
   if (tokens <= 0 || tokens > 0x7fffffffLL) return fail(TF24_ERR_SHAPE, "%s: bad number of tokens %lld", fn, (long long)tokens);
   if (m <= 0 || m % 8 || n <= 0 || n % 8 || m > (1 << 20) || n > (1 << 20))
     return fail(TF24_ERR_SHAPE, "%s: %lld x %lld must be positive multiples of 8, at most %d", fn, (long long)m, (long long)n, 1 << 20);
-  // 32 tokens are addressed by 32-bit lane offsets
+  // a stage's tokens, 32 or 64, are addressed by 32-bit lane offsets
   if (ldg < m || ldg % 8 || ldg > (1 << 23) || ldx < n || ldx % 8 || ldx > (1 << 23))
     return fail(TF24_ERR_STRIDE, "%s: leading dimensions %lld, %lld must cover the rows, be multiples of 8 and at most %d", fn, (long long)ldg, (long long)ldx, 1 << 23);
   if (!g || !x || !dw) return fail(TF24_ERR_ARG, "%s: null pointer", fn);

@@ -358,7 +358,8 @@ using SquareCfg = TileCfgT<2, 3, 3>;
 // four rounds of either, 518 and 497 us).  us on the other tiles and on these, fp16: 11008 x 4096 against 8192 columns 358 -> 346
 // (5.4 rounds -> 4.9), 6144 x 12288 against 3000 251 -> 205 (three rounds of 192 x 192 tiles -> one), 6144 x 8192 against 6144
 // 320 -> 280, 6144 x 3072 against 3000 64.9 -> 57.0, 1536 x 4096 against 12288 98 -> 77.  Raster groups of 5, 6 and 8 tiles: 346, 348
-// and 349 us for the first product, 342, 342 and 346 for 10752 x 4096 against 8192.
+// and 349 us for the first product, 342, 342 and 346 for 10752 x 4096 against 8192.  All vector registers are kept; 51 to 60 scalar ones
+// are spilled (35 to 46 in the other 4-wave forms), none of them inside the stage loop.
 using TallCfg = TileCfgT<2, 3, 6>;
 constexpr int kWave4MinStages = 32;
 constexpr int kRotateMinStages = 56;

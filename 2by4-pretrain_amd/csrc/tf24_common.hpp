@@ -460,7 +460,9 @@ __device__ __forceinline__ Mvue4 mvue4_as(const float (&x)[4], float r0, float r
 // addresses in the callers: 8192 x 8192 bf16 to e4m3 82 -> 64.5 us, to fp16 78.6 -> 64.5 (with a supplied tensor its
 // 268 MB are the bound: 80 us before and after), a column-major 3072 x 12288 half matrix with its row sums 54.5 -> 44 us.
 // Three-input exclusive ors, six compares instead of nine and a kernel of its own for panel output, on another card: 60.5 -> 54.9,
-// 61.5 -> 57.0 and 37.1 -> 36.1.
+// 61.5 -> 57.0 and 37.1 -> 36.1.  Each taken back by itself, 8192 x 8192 bf16 to fp16, to e4m3, float32 to fp16 (58.7, 56.9, 65.6 with
+// all): the exclusive ors 60.7, 60.2, 67.9, the compares 60.5, 59.7, 66.9, the kernel 61.1, 61.1, 67.7; the shorter range tests 58.8, 59.4, 65.3
+// (one median of three beyond the spread), the bytes of a quad in two steps instead of three 58.3, 57.7, 65.9 (none, nor in the modes bound by memory).
 template <typename In>
 __device__ __forceinline__ Mvue4 mvue4(const float (&x)[4], float r0, float r1, bool& finite) {
   bool ok;

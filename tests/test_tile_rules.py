@@ -135,8 +135,8 @@ def test_dense_products_are_taken_where_the_kernel_is_the_faster_one(dense_rules
 
 @pytest.mark.parametrize("tokens,m,n,form", [
     # measured (us on 32 x 32 instructions, on 16 x 16 ones): at least 160 blocks of at least 1024 tokens, or less
-    (12288, 3072, 768, 2), (12288, 768, 3072, 2), (16384, 2048, 512, 2), (4423, 5120, 1280, 2),          # 72.3 69.6, 70.9 67.8, 54.2 52.4, 72.0 67.8
-    (2000, 1024, 4096, 1), (745, 3072, 768, 1), (5000, 512, 2048, 1)]                                    # 33.5 34.5, 17.2 17.8, 25.7 26.7
+    (12288, 3072, 768, 2), (12288, 768, 3072, 2), (16384, 2048, 512, 2), (4423, 5120, 1280, 2),          # 65.2 62.5, 65.5 63.7, 48.9 47.5, 65.8 63.9
+    (2000, 1024, 4096, 1), (745, 3072, 768, 1), (5000, 512, 2048, 1)]                                    # 32.8 33.7, 16.9 17.4, 24.6 25.2
     + [(*sizes, 2) for sizes in MANY_LONG])
 def test_weight_gradients_take_long_tiles_where_they_are_the_faster_ones(dense_rules, tokens, m, n, form):
     assert dense_rules[1].gradient(tokens, m, n) == form
