@@ -1145,9 +1145,10 @@ inline int64_t tile_rounds(int64_t tiles, int64_t cu_slots) { return ((tiles + 7
 
 // A last round that fills less than half of the compute units: the tile rows that make up the full rounds stay
 // with the chained 256 x 256 tiles, the remaining rows go to a second launch on 256 x 128 tiles, which reach twice
-// as many compute units for half the time each (W[11008, 4096] against 8192 tokens: 1376 tiles = 5 rounds of 256
-// + 96; 40 tile rows chained, 3 rows as 192 half tiles: 351.6 -> 341.6 us).  Long tiles only: what a short
-// tile's round costs is mostly its prologue and output pass, which the second launch pays again.
+// as many compute units for half the time each (fp16, W[11008, 4096] against 8192 tokens, before 384 x 192 tiles took that
+// product (takes_tall): 1376 tiles = 5 rounds of 256 + 96; 40 tile rows chained, 3 rows as 192 half tiles: 351.6 -> 341.6 us;
+// e4m3, W[8448, 8192] against 8192: 291 -> 277).  Long tiles only: what a short tile's round costs is mostly its prologue and
+// output pass, which the second launch pays again.
 struct TileRows { int tiles_i, tail_rows; };
 inline TileRows full_rounds(int64_t n_sparse, int64_t n_dense, int stages, int cu_slots) {
   const int tiles_i = (int)((n_sparse + TiledCfg::BI - 1) / TiledCfg::BI), tiles_j = (int)((n_dense + TiledCfg::BJ - 1) / TiledCfg::BJ);
