@@ -425,18 +425,26 @@ spmm_pipe(const uint8_t* __restrict__ a_values, const uint8_t* __restrict__ a_me
   // (a launch may cover the tile rows [aux, aux + tiles_i) of the product; n_sparse stays the row count of the whole operand)
   const int stagger_ticks = PERSIST ? aux : 0;
   const int tile_row0 = PERSIST ? 0 : aux;
-  int split = 0;
   int64_t i0 = 0, j0 = 0;
-  auto locate = [&](int u, int64_t& ti0, int64_t& tj0) {       // unit -> k piece and tile origin
-    split = u / ntiles;
-    const int tile = u - split * ntiles;
-    const int group = tile / (GH * tiles_j);
+  const int split = PERSIST ? 0 : __builtin_amdgcn_readfirstlane(unit / ntiles);                // k piece
+  int group = __builtin_amdgcn_readfirstlane((unit - split * ntiles) / (GH * tiles_j)), in_group = unit - split * ntiles - group * (GH * tiles_j);
+  // origin of the tile number in_group of the group: the divisor is GH but for the last group (a division by a number that is not
+  // known to the compiler is some 40 instructions, which nothing covers where one wave has a SIMD)
+  auto locate = [&](int64_t& ti0, int64_t& tj0) {
     const int gh = min(GH, tiles_i - group * GH);
-    const int in_group = tile - group * GH * tiles_j;
-    ti0 = (int64_t)(tile_row0 + group * GH + in_group % gh) * C::BI;
-    tj0 = (int64_t)(in_group / gh) * C::BJ;
+    int col = (unsigned)in_group / GH;
+    if (gh != GH) col = __builtin_amdgcn_readfirstlane((unsigned)in_group / (unsigned)gh);
+    ti0 = (int64_t)(tile_row0 + group * GH + (in_group - col * gh)) * C::BI;
+    tj0 = (int64_t)col * C::BJ;
   };
-  locate(unit, i0, j0);
+  auto advance = [&]() {                                       // to the workgroup's next tile
+    in_group += slots;
+    for (int size = min(GH, tiles_i - group * GH) * tiles_j; in_group >= size; size = min(GH, tiles_i - group * GH) * tiles_j) {
+      in_group -= size;
+      group++;
+    }
+  };
+  locate(i0, j0);
   // Chained tiles: every second workgroup of an XCD starts `stagger_ticks` (10 ns each) late.  All compute units
   // otherwise finish their tiles at the same moment and write them out together, at the HBM rate, while no matrix
   // instruction issues (a wave's stores share the counter its copies are waited on, so the next tile stalls until
@@ -495,6 +503,7 @@ spmm_pipe(const uint8_t* __restrict__ a_values, const uint8_t* __restrict__ a_me
   };
   constexpr int64_t B_STAGE_ADVANCE_ROWS = B_KSTRIDED ? C::KB / ES : 0;
   const int64_t b_stage_stride = B_KSTRIDED ? B_STAGE_ADVANCE_ROWS * ldb_bytes : (int64_t)C::B_ROW;
+  bool lanes_whole = false;
   auto point_at = [&](int64_t ti0, int64_t tj0) {              // sources of the first stage of the tile at (ti0, tj0)
     // (PERSIST: the lane id is made opaque here and in the output pass, so that the per-lane terms of the
     // addresses are formed again for every tile instead of living in registers through the main loop,
@@ -506,6 +515,10 @@ spmm_pipe(const uint8_t* __restrict__ a_values, const uint8_t* __restrict__ a_me
     else tile_b = b + tj0 * ldb_bytes + (int64_t)st_first * C::B_ROW;
     tile_a = a_values + (ti0 + (int64_t)st_first * n_sparse) * 64;
     tile_m = a_meta + (ti0 + (int64_t)st_first * STAGE_KB * n_sparse) * 4;
+    // the lanes' offsets are those of any other tile unless rows of one of the two are clamped
+    const bool whole = !B_KSTRIDED && last_j >= C::BJ - 1 && last_i >= C::BI - 1;
+    if (whole && lanes_whole) return;
+    lanes_whole = whole;
 #pragma unroll
     for (int q = 0; q < C::NB; q++) {
       if constexpr (B_KSTRIDED) {
@@ -712,7 +725,6 @@ spmm_pipe(const uint8_t* __restrict__ a_values, const uint8_t* __restrict__ a_me
   // the next tile's first two stages are issued during the last two stages of the current one, into
   // the two buffers those stages leave free; the output pass then stages through the third (the last
   // stage's) while they fly, and the next tile starts with its operands already in LDS.
-  int next_unit = unit;
   int64_t next_i0 = 0, next_j0 = 0;
   bool has_next = false;
   bool chained = false;                          // this tile's first two stages were copied under the previous tile
@@ -728,7 +740,7 @@ spmm_pipe(const uint8_t* __restrict__ a_values, const uint8_t* __restrict__ a_me
   else stage_barrier(nstages > 1);
   // stage 0: nothing to multiply yet
   {
-    const bool more = 2 < nstages;
+    const bool more = PERSIST || 2 < nstages;      // (chained tiles have four stages at least)
 #pragma unroll
     for (int n = 0; n < N_READS; n++) read_one(0, n, cur, 0);
     if (more) {
@@ -742,7 +754,13 @@ spmm_pipe(const uint8_t* __restrict__ a_values, const uint8_t* __restrict__ a_me
   }
   // stage st: behind B(st), register set 1 holds the last step of stage st-1
   int st = 1;
-  for (int lim = nstages - 2 - rot;; lim = nstages - 2) {          // up to the wrap of the stage order, then the rest
+  // Up to the wrap of the stage order, to the last two stages, and, where a tile follows, through those: what they copy are its first two.
+  // (Of one loop, and the next tile found with few instructions: nothing covers what a workgroup does between tiles, on four waves least
+  // of all.  With two stages of their own, in which every copy stood behind a branch, and new lane offsets and four divisions for each
+  // tile, us on operands that change, then and now: fp16 3072 x 768 against 12288 columns 44.8 and 43.0 on 8-wave tiles, 55 and 40 on
+  // 256 x 192 ones; 2048 x 512 24.3 and 22.7; 6400 x 1600 against 6000 77.4 and 76.1; 11008 x 4096 against 8192 352.5 and 350.9.)
+  has_next = false;
+  for (int lim = nstages - 2 - rot;;) {
     for (; st < lim; st++) {
       const uint32_t t = cur; cur = nxt; nxt = fre; fre = t;
       mma_step(1, 0, true, smem_at + fre, true, cur, 0);
@@ -750,29 +768,26 @@ spmm_pipe(const uint8_t* __restrict__ a_values, const uint8_t* __restrict__ a_me
       next_stage();
       stage_barrier(true);
     }
-    if (!ROTATE || st >= nstages - 2) break;         // (lim >= 1: the wrap is behind the copies of stage 2)
-    tile_b -= nstages * b_stage_stride;
-    tile_a -= nstages * a_stage_stride;
-    tile_m -= nstages * m_stage_stride;
-  }
-  if constexpr (PERSIST) {
-    next_unit = unit + slots;
-    has_next = next_unit < xcd_end;
-    if (has_next) {                                 // every copy of this tile has been issued: aim at the next one
-      locate(next_unit, next_i0, next_j0);
-      point_at(next_i0, next_j0);
+    if (ROTATE && st < nstages - 2) {                // (lim >= 1: the wrap is behind the copies of stage 2)
+      tile_b -= nstages * b_stage_stride;
+      tile_a -= nstages * a_stage_stride;
+      tile_m -= nstages * m_stage_stride;
+      lim = nstages - 2;
+      continue;
     }
+    if (!PERSIST || st >= nstages || unit + slots >= xcd_end) break;
+    unit += slots;                                   // every copy of this tile has been issued: aim at the next one
+    has_next = true;
+    advance();
+    locate(next_i0, next_j0);
+    point_at(next_i0, next_j0);
+    lim = nstages;
   }
-  for (; st < nstages; st++) {                    // the last two stages: nothing left to copy for this tile
+  for (; st < nstages; st++) {                       // the last two stages of the last tile
     const uint32_t t = cur; cur = nxt; nxt = fre; fre = t;
-    mma_step(1, 0, has_next, smem_at + fre, true, cur, 0);   // (copies: the first two stages of the next tile)
-    mma_step(0, 1, has_next, smem_at + fre, true, cur, 1);
-    next_stage();
-    // behind the last barrier of a tile no wave reads the stage buffers any more; the next tile's
-    // copies are not waited for here
-    if (st + 1 < nstages) stage_barrier(has_next);
-    else if (has_next) wait_reads_and_barrier();
-    else stage_barrier(false);
+    mma_step(1, 0, false, 0, true, cur, 0);
+    mma_step(0, 1, false, 0, true, cur, 1);
+    stage_barrier(false);
   }
   // ---- bias: every lane fetches the bias of WI/64 of its wave's rows here, one instruction step ahead of the
   // output pass, which hands them round the wave through LDS.  (Fetched per element inside the pass -- 128 two-byte
@@ -1014,7 +1029,7 @@ spmm_pipe(const uint8_t* __restrict__ a_values, const uint8_t* __restrict__ a_me
   }
   if (!has_next) break;
   // ---- the next tile: its first two stages are (about to be) in the buffers nxt and fre
-  unit = next_unit; i0 = next_i0; j0 = next_j0; chained = true;
+  i0 = next_i0; j0 = next_j0; chained = true;
   { const uint32_t t = cur; cur = nxt; nxt = fre; fre = t; }
 #pragma unroll
   for (int ti = 0; ti < C::TI; ti++)
