@@ -1215,15 +1215,12 @@ inline Tiles choose_without_tall(int64_t n_sparse, int64_t n_dense, int stages, 
 }
 
 // Whether it takes 384 x 192 tiles instead of the form chosen among the others: the same estimate of both (0.98 us a stage and 5 us
-// for a round of these tiles, 1.12 a stage at the sustained clock), from kTallMinStages stages on.  Of 110 fp16 products of 10 to 168
+// for a round of these tiles, 1.12 a stage at the sustained clock), from kWave4MinStages stages on (choose_short: fewer).  Of 110 fp16 products of 10 to 168
 // stages, 960 to 12224 rows and 1237 to 15757 columns on operands that change from product to product, 13 take them, all 2 to 28 %
 // faster that way (1120 x 2816 against 14480 columns 69.9 -> 54.8, 2912 x 5824 against 12074 244 -> 200, 10624 x 3264 against 3385
 // 132 -> 117); of the others none would be more than 5 % faster.  Of 70 others, a third with bias, half of them bf16, 12
-// take them, 1 to 25 % faster.  With fewer stages a tile's prologue and output pass are what a
-// round costs and two waves a SIMD hide them better (5280 x 768 against 8114 46.8 on 256 x 256 tiles, 59.5).
-constexpr int kTallMinStages = 24;
+// take them, 1 to 25 % faster.
 inline bool takes_tall(int64_t n_sparse, int64_t n_dense, int stages, TileRows wide, Tiles form, int cu_slots) {
-  if (stages < kTallMinStages) return false;
   auto us = [&](int64_t tiles, double of_round, double sustained) {
     return std::max((double)tile_rounds(tiles, cu_slots) * of_round, (double)tiles / (8 * cu_slots) * sustained * stages);
   };
@@ -1232,13 +1229,39 @@ inline bool takes_tall(int64_t n_sparse, int64_t n_dense, int stages, TileRows w
   double other;
   if (form == Tiles::SQUARE4) other = us(rows(SquareCfg::BI) * columns(SquareCfg::BJ), 0.53 * stages + 5.0, 0.67);
   else if (form == Tiles::NARROW4) other = us(rows(Wave4Cfg192::BI) * columns(Wave4Cfg192::BJ), 0.69 * stages + 2.0, 0.75);
-  else other = us(wide.tiles_i * columns(TiledCfg::BJ), stages >= kWave4MinStages ? 0.93 * stages + 2.5 : 0.84 * stages + 5.5, 1.0) +
+  else other = us(wide.tiles_i * columns(TiledCfg::BJ), 0.93 * stages + 2.5, 1.0) +
                (wide.tail_rows ? 0.5 * stages + 5.0 : 0.0);
   return us(rows(TallCfg::BI) * columns(TallCfg::BJ), 0.98 * stages + 5.0, 1.12) < 0.98 * other;
+}
+
+// Whether a product of fewer than kWave4MinStages stages takes 256 x 192 or (16-bit operands, kShortTallMinStages stages or more) 384 x 192 tiles
+// instead of the form chosen among the others.  Rounds and filled rounds (tiles / compute units) each cost something by the stage and by the tile;
+// fitted to the times of every form on 230 products of 5 to 31 stages (fp16, bf16 and e4m3, 640 to 11000 rows, 900 to 16000 columns,
+// operands that change from product to product), within 5 % of them (root mean square).  97 of those products take the two forms, 6 % faster on
+// average, 17 % at best and 9 % slower at worst; over all of them the choice is 0.6 % off the best form.  us on the others and now: fp16
+// 3072 x 768 against 12288 columns (three full rounds of 256 x 192 tiles) 41.8 and 39.0, 5120 x 1280 against 4096 40.0 and 36.2, 4800 x 1600
+// against 4096 47.0 and 41.9, 4096 x 960 against 4145 26.1 and 23.3 (384 x 192).  One round of wide tiles and of narrow ones, up to 11 stages:
+// no better (2048 x 512 against 6144 13.1 and 13.6, e4m3 4224 x 1024 against 2384 12.1 and 14.6; with 12 stages 2304 x 768 against 4096 14.3 and 13.7).
+constexpr int kShortTallMinStages = 8, kShortOneRoundStages = 12;
+inline Tiles choose_short(int64_t n_sparse, int64_t n_dense, int stages, Tiles form, bool operands16, int cu_slots) {
+  struct Cost { int rows, columns; double round_stage, stage, round, tile, call; };
+  auto rounds_of = [&](int rows, int columns) { return tile_rounds(((n_sparse + rows - 1) / rows) * ((n_dense + columns - 1) / columns), cu_slots); };
+  auto us = [&](Cost c) {
+    const double filled = (double)(((n_sparse + c.rows - 1) / c.rows) * ((n_dense + c.columns - 1) / c.columns)) / (8 * cu_slots);
+    return (double)rounds_of(c.rows, c.columns) * (c.round_stage * stages + c.round) + filled * (c.stage * stages + c.tile) + c.call;
+  };
+  const Cost wide{TiledCfg::BI, TiledCfg::BJ, 0.37, 0.56, 2.49, 1.85, 2.81}, square{SquareCfg::BI, SquareCfg::BJ, 0.34, 0.23, 2.9, 0.0, 3.52};
+  const Cost present = form == Tiles::SQUARE4 ? square : wide;
+  const double other = us(present), narrow = us({Wave4Cfg192::BI, Wave4Cfg192::BJ, 0.33, 0.37, 4.3, 0.0, 2.31});
+  const double tall = us({TallCfg::BI, TallCfg::BJ, 0.52, 0.40, 4.48, 4.37, 1.3});
+  if (operands16 && stages >= kShortTallMinStages && tall < 0.96 * narrow) return tall < 0.98 * other ? Tiles::TALL4 : form;
+  if (stages < kShortOneRoundStages && rounds_of(present.rows, present.columns) == 1) return form;
+  return narrow < 0.98 * other ? Tiles::NARROW4 : form;
 }
 inline Tiles choose_tiles(int64_t n_sparse, int64_t n_dense, int stages, TileRows wide, bool results16, int cu_slots, bool operands16 = false) {
   if (cu_slots <= 0 || stages < 4) return Tiles::WIDE8;
   const Tiles form = choose_without_tall(n_sparse, n_dense, stages, wide, results16, cu_slots);
+  if (results16 && stages < kWave4MinStages) return choose_short(n_sparse, n_dense, stages, form, operands16, cu_slots);
   return results16 && operands16 && takes_tall(n_sparse, n_dense, stages, wide, form, cu_slots) ? Tiles::TALL4 : form;
 }
 

@@ -1374,6 +1374,23 @@ def test_linear_tall_tiles(cuda, dtype, n, stages, rows, activation):
     test_linear_square_tiles(cuda, dtype, n, stages, rows, activation)
 
 
+SHORT = [                           # fewer stages than chained 256 x 256 tiles take on four waves: (form on 16-bit operands, on 8-bit ones)
+    (2080, 4, 10541, "narrow", "narrow"),               # the fewest stages; two rounds, partial tiles on either edge
+    (3072, 12, 12288, "narrow", "narrow"),              # three full rounds
+    (800, 12, 10188, "narrow", "narrow"),               # one round, the fewest stages for that
+    (640, 31, 12472, "narrow", "narrow"),               # the most stages
+    (1312, 8, 11029, "tall", "square"),                 # the fewest stages of tall tiles
+    (3456, 12, 10590, "tall", "wide"), (1120, 31, 12811, "tall", "square")]
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float8_e4m3fn])
+@pytest.mark.parametrize("n,stages,rows", [case[:3] for case in SHORT])
+@pytest.mark.parametrize("activation", [None, "relu"])
+def test_linear_narrow_and_tall_tiles_of_few_stages(cuda, dtype, n, stages, rows, activation):
+    """Products on chained 256 x 192 and 384 x 192 tiles of few stages, with and without bias: exact on small integers."""
+    test_linear_square_tiles(cuda, dtype, n, stages, rows, activation)
+
+
 SQUARE_STRIDED = [                  # and in how many pieces of k (test_tile_rules.py)
     (64, 4, 72, 1), (224, 5, 200, 1), (192, 9, 192, 3), (352, 25, 2376, 3), (416, 8, 560, 1),         # tiles past either edge
     (992, 40, 392, 5), (544, 117, 120, 15), (3072, 48, 768, 2), (3424, 202, 80, 11)]

@@ -6,7 +6,7 @@ import subprocess
 
 import pytest
 
-from test_gpu_parity import NOT_TALL, SQUARE, SQUARE_STRIDED, STAGE_ORDER, TALL
+from test_gpu_parity import NOT_TALL, SHORT, SQUARE, SQUARE_STRIDED, STAGE_ORDER, TALL
 from test_gpu_training import MANY_LONG
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -93,6 +93,23 @@ def test_tall_tiles_where_they_are_the_faster_ones(rules, n, stages, columns, ta
 @pytest.mark.parametrize("n,stages,rows,tiles", NOT_TALL)
 def test_other_tiles_are_tested_with_16_bits_too(rules, n, stages, rows, tiles):
     assert rules.tiles_of_16_bits(n, rows, stages, CU_SLOTS) == {"wide, two launches": 101, "square": 3}[tiles]
+
+
+@pytest.mark.parametrize("n,stages,rows,form16,form8", SHORT)
+def test_products_of_few_stages_tested_on_the_gpu_take_the_tiles_they_are_for(rules, n, stages, rows, form16, form8):
+    codes = {"wide": 0, "narrow": 2, "square": 3, "tall": 4}
+    assert (rules.tiles_of_16_bits(n, rows, stages, CU_SLOTS), rules.tiles(n, rows, stages, 1, CU_SLOTS)) == (codes[form16], codes[form8])
+    assert rules.tiles(n, rows, stages, 0, CU_SLOTS) == 0                     # 32-bit results stay on 256 x 256 tiles
+    assert -(-n // 256) * -(-rows // 128) > 256
+
+
+@pytest.mark.parametrize("n,stages,columns,form", [
+    # measured (us on the other tiles, on the form taken): rounds that other widths fill better, or do not
+    (3072, 12, 12288, 2), (5120, 20, 4096, 2), (4800, 25, 4096, 2), (4096, 15, 4145, 4),              # 41.8 39.0, 40.0 36.2, 47.0 41.9, 26.1 23.3
+    (4096, 16, 8192, 0), (6400, 25, 6144, 0), (5280, 12, 8114, 0),                                    # 40.5 46.3, 75.8 81.2, 46.8 53
+    (2048, 8, 6144, 0), (2304, 12, 4096, 2)])                                                         # 13.1 13.6, 14.3 13.7
+def test_tiles_of_products_of_few_stages(rules, n, stages, columns, form):
+    assert rules.tiles_of_16_bits(n, columns, stages, CU_SLOTS) == form
 
 
 @pytest.fixture(scope="module")
