@@ -1380,7 +1380,7 @@ SHORT = [                           # fewer stages than chained 256 x 256 tiles 
     (800, 12, 10188, "narrow", "narrow"),               # one round, the fewest stages for that
     (640, 31, 12472, "narrow", "narrow"),               # the most stages
     (1312, 8, 11029, "tall", "square"),                 # the fewest stages of tall tiles
-    (3456, 12, 10590, "tall", "wide"), (1120, 31, 12811, "tall", "square")]
+    (3456, 12, 10590, "tall", "wide"), (1120, 31, 12811, "tall", "wide")]
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float8_e4m3fn])
