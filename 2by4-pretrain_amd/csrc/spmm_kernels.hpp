@@ -1430,17 +1430,14 @@ int launch_tiled(const void* av, const void* am, int64_t n_sparse, int64_t k, co
 // A batch that reaches past the last panel re-reads it and leaves it out of the product: multiplied by zeros it would
 // make NaN of an infinite activation.  The full batches are straight-line code and only the last one tests its panels,
 // which is also the faster form (with a test of zeros in every panel 1600 x 6400 fp16 against one column takes 8.5 us, with
-// a choice of the two forms in every batch 9.3, this way 7.8; 8192 x 8192 with the shared form 18.3 -> 17.0).
-// Fewer than 512 row blocks, or more than 16 columns (spmm_narrow): a block owns 16 rows, its up to four waves each take a
+// a choice of the two forms in every batch 9.3, this way 7.8).
+// Up to 16 columns: spmm_few.  17 to 64 (spmm_narrow): a block owns 16 rows, its up to four waves each take a
 // share of the k range, read their dense fragments, NB of 16 columns, from global memory (64 contiguous bytes from
 // each of the 16 dense rows, twice) and meet in LDS at the end (added in wave order).  Bound by latency, a few loads deep, at
 // short k and by the requests of the dense fragments at long k: 3072 x 768 bf16 against 37 columns 8.9 us on 256 x 64 tiles,
-// of which there are 12, and 5.4 us here.  Eight waves a block were no faster (4096 x 11008, 1 column: 13.2 -> 16.9 us).
-// From 512 row blocks on (spmm_narrow_shared): see there.
+// of which there are 12, and 5.4 us here.
 // ------------------------------------------------------------------------------------------
 constexpr int kNarrowWaves = 4;
-constexpr int kNarrowSharedMin = 160;      // workgroups of four 16-row blocks below which two blocks per workgroup are faster
-
 template <typename T, typename OutT, bool C_JMAJOR, int NB>
 __global__ void __launch_bounds__(64 * kNarrowWaves)
 spmm_narrow(const uint8_t* __restrict__ a_values, const uint8_t* __restrict__ a_meta, int64_t n_sparse, int64_t k,
@@ -1448,10 +1445,9 @@ spmm_narrow(const uint8_t* __restrict__ a_values, const uint8_t* __restrict__ a_
             OutT* __restrict__ c, int64_t ldc, const OutT* __restrict__ bias, float scale, int act) {
   constexpr int KSTEP = mma16<T>::KSTEP;     // dense k per panel = per instruction
   constexpr int M_ROW = KSTEP / 8;           // metadata bytes per row per panel
-  constexpr int BATCH = NB == 1 ? 8 : NB == 2 ? 4 : 2;          // panels per load batch; two batches are in flight
-  constexpr int CHAINS = NB == 1 ? 2 : 1;    // consecutive instructions do not wait on each other: two chains, or the fragments
+  constexpr int BATCH = NB == 2 ? 4 : 2;     // panels per load batch; two batches are in flight
   using acc_t = typename mma16<T>::acc_t;
-  __shared__ acc_t s_acc[NB == 1 ? kNarrowWaves - 1 : kNarrowWaves][NB][64];
+  __shared__ acc_t s_acc[kNarrowWaves][NB][64];
   const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);      // (its panels are counted in scalar registers)
   const int64_t i0 = (int64_t)blockIdx.x * 16;
@@ -1467,13 +1463,11 @@ spmm_narrow(const uint8_t* __restrict__ a_values, const uint8_t* __restrict__ a_
   const uint8_t* av = a_values + (i0 + li) * 64 + lk * 16;
   const uint8_t* am = a_meta + panel_meta_offset(lk * (M_ROW / 4), i0 + li, n_sparse);   // (a panel's further words: n_sparse * 4 bytes apart)
   const int64_t a_step = n_sparse * 64, m_step = n_sparse * M_ROW;
-  acc_t acc[NB][CHAINS];
+  acc_t acc[NB];                             // (of consecutive instructions, so that none waits for the one before)
 #pragma unroll
   for (int f = 0; f < NB; f++)
 #pragma unroll
-    for (int h = 0; h < CHAINS; h++)
-#pragma unroll
-      for (int r = 0; r < 4; r++) acc[f][h][r] = 0;
+    for (int r = 0; r < 4; r++) acc[f][r] = 0;
   // two register sets: the loads of the next batch are in flight while the current one is multiplied
   int4v af[2][BATCH], lo[2][BATCH][NB], hi[2][BATCH][NB];
   int idx[2][BATCH];
@@ -1496,7 +1490,7 @@ spmm_narrow(const uint8_t* __restrict__ a_values, const uint8_t* __restrict__ a_
     for (int f = 0; f < NB; f++) {
       const int4v l = lo[set][u][f], h = hi[set][u][f];
       const int8v bfrag = {l[0], l[1], l[2], l[3], h[0], h[1], h[2], h[3]};
-      acc[f][u % CHAINS] = mma16<T>::template run<0>(af[set][u], bfrag, acc[f][u % CHAINS], idx[set][u]);
+      acc[f] = mma16<T>::template run<0>(af[set][u], bfrag, acc[f], idx[set][u]);
     }
   };
   // (the scheduling barriers keep the loads ahead of the instructions that wait for the previous batch)
@@ -1526,17 +1520,15 @@ spmm_narrow(const uint8_t* __restrict__ a_values, const uint8_t* __restrict__ a_
   } else if (p < p_end) {
     multiply_last(0, p);
   }
-  const acc_t own = CHAINS == 2 ? acc[0][0] + acc[0][CHAINS - 1] : acc[0][0];
-  if (wave > 0) s_acc[wave - 1][0][lane] = own;
 #pragma unroll
-  for (int f = 1; f < NB; f++) s_acc[wave][f][lane] = acc[f][0];
+  for (int f = 0; f < NB; f++) s_acc[wave][f][lane] = acc[f];
   __syncthreads();
   for (int f = wave; f < NB; f += nwaves) {  // a wave finishes every nwaves-th fragment, its pieces added in wave order
     const int64_t col = f * 16 + li;
     if (col >= n_dense) continue;
-    acc_t sum = f == 0 ? own : s_acc[0][f][lane];
+    acc_t sum = s_acc[0][f][lane];
 #pragma unroll
-    for (int w = 1; w < nwaves; w++) sum += s_acc[f == 0 ? w - 1 : w][f][lane];
+    for (int w = 1; w < nwaves; w++) sum += s_acc[w][f][lane];
     const int64_t row = i0 + lk * 4;         // D layout: column l%16, rows 4*(l/16) + r
     OutT o[4];
 #pragma unroll
@@ -1550,117 +1542,120 @@ spmm_narrow(const uint8_t* __restrict__ a_values, const uint8_t* __restrict__ a_
   }
 }
 
-// Narrow kernel for many sparse rows: the NW (2 or 4) waves of a block own adjacent 16-row blocks and
-// share the dense operand through LDS, 16 panels (a chunk) at a time in two buffers, so that the
-// only loads of the main loop are the sparse operand's: the one-wave form above sends every wave's
-// dense fragments through L1 (twice the requests of its share of the sparse operand), and the
-// kernel is bound by the number of requests in flight, not by bytes.  LDS holds
-// [panel][column][128 bytes] with the 16-byte pieces of a column XOR-swizzled by column / 2, so the
-// 16 lanes that read one piece position of 16 columns hit 16 different bank groups.
-// NC = dense columns kept in LDS (8 or 16).
+// Up to 16 dense columns (NC = 8 or 16): a block owns 16 sparse rows, its NW waves each take a share of the k range and meet in LDS at the
+// end (added in wave order).  Bound by the one pass over the compressed operand (50.7 MB of fp16 11008 x 4096, 7.9 us at the rate of a copy) and
+// what a launch, its first loads and its last store take beside it (768 x 768: 2.8 us).  A wave keeps two chunks of 8 panels in flight, in
+// registers; nothing it loads comes from the dense operand but each of the columns there are once, 1 KB a chunk, handed to the fragments
+// through LDS of its own (no barrier: the LDS accesses of a wave execute in order).  Read as fragments from memory the dense operand costs
+// twice the sparse one's requests, and a compute unit takes 64 bytes of them a clock; shared by the waves of a block, 16 panels between two
+// barriers, it leaves a third of the compute units without a block.  The metadata of two panels are one load of a word per lane,
+// brought to their lanes by swaps of rows.  Adjacent row blocks, which share the lines of their metadata, are dealt to the same XCD.
+// us before and now, fp16, operands from memory, one column: 11008 x 4096 12.5 and 10.6, 8192 x 8192 17.7 and 14.0, 4096 x 11008 12.8 and 11.3,
+// 4096 x 4096 6.6 and 5.7, 768 x 3072 5.3 and 4.0; eight: 12.8 and 11.7, 17.8 and 15.8, 14.5 and 12.8, 7.0 and 6.1.  Chunks of
+// 16 panels 11008 x 4096 13.6, 8192 x 8192 15.1; two row blocks a wave 12.2 and 15.1 (against 16 columns 14.6 and 16.5, here 14.1 and 19.1).
 template <typename T, typename OutT, bool C_JMAJOR, int NC, int NW>
 __global__ void __launch_bounds__(64 * NW)
-spmm_narrow_shared(const uint8_t* __restrict__ a_values, const uint8_t* __restrict__ a_meta, int64_t n_sparse, int64_t k,
-                   const uint8_t* __restrict__ b, int64_t ldb_bytes, int64_t n_dense,
-                   OutT* __restrict__ c, int64_t ldc, const OutT* __restrict__ bias, float scale, int act) {
+spmm_few(const uint8_t* __restrict__ a_values, const uint8_t* __restrict__ a_meta, int64_t n_sparse, int64_t k,
+         const uint8_t* __restrict__ b, int64_t ldb_bytes, int64_t n_dense,
+         OutT* __restrict__ c, int64_t ldc, const OutT* __restrict__ bias, float scale, int act) {
   constexpr int KSTEP = mma16<T>::KSTEP;
-  constexpr int M_ROW = KSTEP / 8;
-  constexpr int CH = 16;                              // panels per chunk
-  constexpr int THREADS = 64 * NW;
-  constexpr int PIECES = NC * CH * 8 / THREADS;       // 16-byte pieces of the dense chunk per thread (4 to 16)
+  constexpr int CH = 8;                               // panels per chunk: a lane brings one 16-byte piece of each dense column
+  constexpr bool PAIR = sizeof(T) == 2;               // two words of metadata per row and panel (8-bit values: four, one for each lane of a row)
   using acc_t = typename mma16<T>::acc_t;
-  __shared__ __attribute__((aligned(16))) uint8_t s_b[2][CH * NC * 128];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, li = lane & 15, lk = lane >> 4;
-  const int64_t blocks16 = n_sparse / 16;
-  const int64_t rb = (int64_t)blockIdx.x * NW + wave;
-  const bool active = rb < blocks16;
-  const int64_t i0 = (active ? rb : blocks16 - 1) * 16;
-  const int64_t npanels = k / KSTEP;
-  const int nchunks = (int)((npanels + CH - 1) / CH);
+  __shared__ __attribute__((aligned(16))) uint8_t s_b[NW][CH * NC * 128];
+  __shared__ acc_t s_acc[NW - 1][64];
+  const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int64_t blocks16 = n_sparse / 16, per_xcd = (blocks16 + 7) / 8;           // (workgroup ids are dealt to the XCDs round-robin)
+  const int64_t rb = (int64_t)(blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+  if ((int64_t)(blockIdx.x >> 3) >= per_xcd || rb >= blocks16) return;
+  const int64_t i0 = rb * 16, npanels = k / KSTEP;
+  const int p_begin = (int)(wave * npanels / NW), p_end = (int)((wave + 1) * npanels / NW);
   const uint8_t* av = a_values + (i0 + li) * 64 + lk * 16;
-  const uint8_t* am = a_meta + panel_meta_offset(lk * (M_ROW / 4), i0 + li, n_sparse);   // (a panel's further words: n_sparse * 4 bytes apart)
-  const int64_t a_step = n_sparse * 64, m_step = n_sparse * M_ROW;
-  // dense chunk: thread's piece q = tid + THREADS j -> column q / (CH * 8), piece q % (CH * 8) of the column's 2 KB
-  const uint8_t* bsrc[PIECES];
-  int bdst[PIECES], bwithin[PIECES];
-#pragma unroll
-  for (int j = 0; j < PIECES; j++) {
-    const int q = tid + THREADS * j, col = q / (CH * 8), within = q % (CH * 8);
-    const int64_t gcol = col < n_dense ? col : n_dense - 1;
-    bsrc[j] = b + gcol * ldb_bytes + within * 16;
-    bwithin[j] = within;
-    bdst[j] = ((within >> 3) * NC + col) * 128 + (((within & 7) ^ ((col >> 1) & 7)) * 16);
-  }
-  const int64_t row_bytes = npanels * 128;             // bytes of one dense row
+  const uint8_t* am = a_meta + (i0 + li) * 4;
+  const int64_t a_step = n_sparse * 64, word_step = n_sparse * 4;
+  // the wave's chunk of the dense operand: [panel][column][128 bytes], the 16-byte pieces of a column XOR-swizzled by column / 2, so that
+  // the 16 lanes that read one piece position of 16 columns hit different banks
+  uint8_t* const sb = s_b[wave];
   const int colr = li < n_dense ? li : (int)n_dense - 1;
   const int rd_lo = colr * 128 + ((lk ^ ((colr >> 1) & 7)) * 16), rd_hi = colr * 128 + (((lk + 4) ^ ((colr >> 1) & 7)) * 16);
   acc_t acc[2];
 #pragma unroll
   for (int r = 0; r < 4; r++) { acc[0][r] = 0; acc[1][r] = 0; }
-  int4v af[2][CH], breg[PIECES];
-  int idx[2][CH];
-  auto load_a = [&](int set, int chunk) {
+  int4v af[2][CH], breg[NC];
+  uint32_t words[2][PAIR ? CH / 2 : CH];
+  auto load_a = [&](int set, int p) __attribute__((always_inline)) {
 #pragma unroll
     for (int u = 0; u < CH; u++) {
-      const int64_t p = (int64_t)chunk * CH + u;
-      const int64_t pp = p < npanels ? p : npanels - 1;          // past the end: re-read the last panel, do not multiply it
+      const int pp = min(p + u, p_end - 1);           // past the end: re-read the last panel, do not multiply it
       af[set][u] = __builtin_nontemporal_load(reinterpret_cast<const int4v*>(av + pp * a_step));
-      if constexpr (sizeof(T) == 2) idx[set][u] = *reinterpret_cast<const uint16_t*>(am + pp * m_step);
-      else idx[set][u] = *reinterpret_cast<const int*>(am + pp * m_step);
+      if constexpr (!PAIR) words[set][u] = *reinterpret_cast<const uint32_t*>(am + (pp * 4 + lk) * word_step);
+      else if (u % 2 == 0) words[set][u / 2] = *reinterpret_cast<const uint32_t*>(am + min((p + u) * 2 + lk, p_end * 2 - 1) * word_step);
     }
   };
-  auto load_b = [&](int chunk) {
+  auto load_b = [&](int p) __attribute__((always_inline)) {
+    const int64_t at = (int64_t)min(p + (lane >> 3), p_end - 1) * 128 + (lane & 7) * 16;
 #pragma unroll
-    for (int j = 0; j < PIECES; j++) {
-      int64_t off = (int64_t)chunk * (CH * 128) + bwithin[j] * 16;
-      if (off > row_bytes - 16) off = row_bytes - 16;             // pieces past k are never multiplied
-      breg[j] = *reinterpret_cast<const int4v*>(bsrc[j] - bwithin[j] * 16 + off);
+    for (int j = 0; j < NC; j++)
+      if (j < n_dense) breg[j] = *reinterpret_cast<const int4v*>(b + j * ldb_bytes + at);
+  };
+  auto store_b = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < NC; j++)
+      if (j < n_dense) *reinterpret_cast<int4v*>(sb + ((lane >> 3) * NC + j) * 128 + (((lane & 7) ^ ((j >> 1) & 7)) * 16)) = breg[j];
+  };
+  auto index_of = [&](int set, int u) __attribute__((always_inline)) {
+    if constexpr (PAIR) {
+      // row r of 16 lanes holds word r of the pair of panels; it needs the half r % 2 of word r / 2 of its panel
+      typedef uint32_t uint2v __attribute__((ext_vector_type(2)));
+      const uint2v panels = __builtin_amdgcn_permlane32_swap(words[set][u / 2], words[set][u / 2], false, false);      // words 0 1 0 1, and 2 3 2 3
+      const uint2v both = __builtin_amdgcn_permlane16_swap(panels[u % 2], panels[u % 2], false, false);                // of it 0 0 0 0, and 1 1 1 1
+      return (int)((lk < 2 ? both[0] : both[1]) >> ((lk & 1) * 16));
+    } else {
+      return (int)words[set][u];
     }
   };
-  auto multiply_panel = [&](int set, int u) {
-    const uint8_t* sb = s_b[set];
+  auto multiply_panel = [&](int set, int u) __attribute__((always_inline)) {
     const int4v lo = *reinterpret_cast<const int4v*>(sb + u * NC * 128 + rd_lo);
     const int4v hi = *reinterpret_cast<const int4v*>(sb + u * NC * 128 + rd_hi);
     const int8v bfrag = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-    acc[u & 1] = mma16<T>::template run<0>(af[set][u], bfrag, acc[u & 1], idx[set][u]);
+    acc[u & 1] = mma16<T>::template run<0>(af[set][u], bfrag, acc[u & 1], index_of(set, u));
   };
-  auto multiply = [&](int set, int chunk) {
-    if ((int64_t)(chunk + 1) * CH <= npanels) {
+  auto multiply = [&](int set, int p) __attribute__((always_inline)) {
+    if (p + CH <= p_end) {
 #pragma unroll
       for (int u = 0; u < CH; u++) multiply_panel(set, u);
     } else {
 #pragma unroll
       for (int u = 0; u < CH; u++)
-        if ((int64_t)chunk * CH + u < npanels) multiply_panel(set, u);
+        if (p + u < p_end) multiply_panel(set, u);
     }
   };
-  auto store_b = [&](int set) {
-#pragma unroll
-    for (int j = 0; j < PIECES; j++) *reinterpret_cast<int4v*>(s_b[set] + bdst[j]) = breg[j];
-  };
-  load_b(0);
-  load_a(0, 0);
-  __builtin_amdgcn_sched_barrier(0);
-  // one barrier per chunk: a buffer is rewritten two iterations after it was read, and every wave
-  // passes the barrier in between only after that read
-  for (int ch = 0; ch < nchunks; ch += 2) {
-    store_b(0);
-    if (ch + 1 < nchunks) { load_b(ch + 1); load_a(1, ch + 1); }
-    __builtin_amdgcn_sched_barrier(0);
-    __syncthreads();
-    multiply(0, ch);
-    __builtin_amdgcn_sched_barrier(0);
-    if (ch + 1 < nchunks) {
-      store_b(1);
-      if (ch + 2 < nchunks) { load_b(ch + 2); load_a(0, ch + 2); }
+  if (p_begin < p_end) {
+    load_b(p_begin);
+    load_a(0, p_begin);
+    __builtin_amdgcn_sched_barrier(0);                // (the scheduling barriers keep a chunk's loads ahead of the instructions that wait for the one before)
+    for (int p = p_begin; p < p_end; p += 2 * CH) {
+      store_b();
+      if (p + CH < p_end) { load_b(p + CH); load_a(1, p + CH); }
       __builtin_amdgcn_sched_barrier(0);
-      __syncthreads();
-      multiply(1, ch + 1);
+      multiply(0, p);
       __builtin_amdgcn_sched_barrier(0);
+      if (p + CH < p_end) {
+        store_b();
+        if (p + 2 * CH < p_end) { load_b(p + 2 * CH); load_a(0, p + 2 * CH); }
+        __builtin_amdgcn_sched_barrier(0);
+        multiply(1, p + CH);
+        __builtin_amdgcn_sched_barrier(0);
+      }
     }
   }
-  if (!active || li >= n_dense) return;
-  const acc_t sum = acc[0] + acc[1];
+  acc_t sum = acc[0] + acc[1];
+  if (wave > 0) s_acc[wave - 1][lane] = sum;
+  __syncthreads();
+  if (wave > 0 || li >= n_dense) return;
+#pragma unroll
+  for (int w = 1; w < NW; w++) sum += s_acc[w - 1][lane];
   const int64_t row = i0 + lk * 4;           // D layout: column l%16, rows 4*(l/16) + r
   OutT o[4];
 #pragma unroll
@@ -1673,20 +1668,31 @@ spmm_narrow_shared(const uint8_t* __restrict__ a_values, const uint8_t* __restri
   }
 }
 
+// Waves that share a row block: some 1400 to 2000 waves in all, and six panels for each of them, or two.  us with 2, 4 and 8, fp16, one column:
+// 11008 x 4096 (688 row blocks) 10.6, 11.0 and 12.7; 8192 x 8192 (512) 14.0, 14.3 and 15.8; 6144 x 4096 (384) 7.9, 7.8 and 8.6;
+// 4096 x 11008 (256) 13.9, 11.4 and 11.3; 768 x 3072 (48) 4.7, 4.3 and 4.0; 3072 x 768 (192, 12 panels) 2.96, 3.03 and 3.6.
+inline int few_waves(int64_t blocks, int64_t npanels) {
+  int waves = blocks <= 256 ? 8 : blocks < 512 ? 4 : 2;
+  while (waves > 2 && npanels < 6 * waves) waves /= 2;
+  return waves;
+}
+
 // Up to how many dense columns the narrow kernels are the faster ones; us on float16 operands, tiled -> narrow:
-// from 512 row blocks on (spmm_narrow_shared) 16: 8192 x 8192 22.0 -> 20.2, 8192 x 1024 10.2 -> 4.8; below that the fragments of
-// more columns cost requests with every panel of every block, so it depends on the panels: 16 columns of 4096 x 4096 12.8 -> 8.7,
-// of 768 x 3072 8.8 -> 7.9, but of 1600 x 6400 12.4 -> 14.8; 32 of 4096 x 2048 10.3 -> 7.7; 64 of 4096 x 1536 13.5 -> 9.4, of
+// 16 on spmm_few up to 128 panels (9 and 16 columns of 4096 x 8192 14.9 -> 9.9 and 15.0 -> 11.0, of 6144 x 6144 15.0 -> 12.2 and 14.1, of 1600 x 6400
+// 12.3 -> 7.8 and 11.5 -> 9.2) and some further where there are rows for k pieces of the tiled kernel to be small, but not many (of
+// 4096 x 11008 17.3 -> 13.0 and 17.4 -> 14.7, of 2048 x 11008 14.3 -> 13.0 with 16); beyond, nine or ten from 512 row blocks on (9 and 16 of 8192 x 16384
+// 31.3 -> 30.3 and 31.2 -> 34.7, of 11008 x 16384 42.4 -> 40.3 and 42.7 -> 48.4, but 16 of 768 x 11008 11.8 -> 12.5 and of 512 x 16384 13.4 -> 15.7).
+// More on spmm_narrow, whose fragments cost requests with every panel of every block, so it depends on the panels: 32 columns of 4096 x 2048
+// 10.3 -> 7.7; 64 of 4096 x 1536 13.5 -> 9.4, of
 // 2304 x 768 9.0 -> 6.5, but of 2304 x 2048 10.7 -> 11.2.  With two blocks to a compute unit (6144 rows): 48 of k = 768
-// 9.0 -> 8.0 and of 1536 13.7 -> 12.5, 64 of k = 768 9.1 -> 9.6; 9 and 16 columns of 64 panels 12.2 -> 10.5
-// and 12.4 -> 12.8, of 96 14.0 -> 14.3 and 18.0.  With three (12288 rows) 17 and 32 columns of 16 panels 10.4 -> 8.1 and 10.0, 32 of
-// 24 panels 13.5 -> 14.1; with four (16384 rows) 32 of 16 panels 10.5 -> 12.1.  Past 128 panels the few workgroups of the shared form fall behind
-// k pieces (16 columns of 8192 x 8192 18.6 -> 19.5, of 8192 x 16384 28.3 -> 34.8, of 11008 x 16384 35.7 -> 49.5).
+// 9.0 -> 8.0 and of 1536 13.7 -> 12.5, 64 of k = 768 9.1 -> 9.6.  With three (12288 rows) 17 and 32 columns of 16 panels 10.4 -> 8.1 and 10.0, 32 of
+// 24 panels 13.5 -> 14.1; with four (16384 rows) 32 of 16 panels 10.5 -> 12.1.
 inline int64_t narrow_columns(int64_t n_sparse, int64_t npanels) {
   const int64_t blocks = n_sparse / 16;
   if (blocks <= 512 && npanels <= 32) return npanels > 24 ? 32 : blocks <= 256 ? 64 : 48;
   if (blocks <= 768 && npanels <= 16) return 32;
-  return npanels <= (blocks >= 512 ? 128 : 64) ? 16 : 8;
+  if (npanels <= 128 || (blocks >= 96 && blocks <= 256 && npanels <= 192)) return 16;
+  return blocks >= 512 ? 10 : 8;
 }
 
 template <typename T, typename OutT>
@@ -1694,21 +1700,23 @@ int launch_narrow(const void* av, const void* am, int64_t n_sparse, int64_t k, c
                   void* c, int c_layout, int64_t ldc, const void* bias, float scale, int act, hipStream_t s) {
   dim3 grid((unsigned)(n_sparse / 16));
   const int64_t blocks = n_sparse / 16, npanels = k * (int64_t)sizeof(T) / 128;
-  if (blocks >= 512 && n_dense <= 16) {          // enough row blocks: several per workgroup, dense operand through LDS
-    const bool jm = c_layout == TF24_COL_MAJOR;
-    const int nw = blocks / 4 >= kNarrowSharedMin ? 4 : 2;      // four row blocks per workgroup only if that leaves enough workgroups
-    dim3 sgrid((unsigned)((blocks + nw - 1) / nw));
+  if (n_dense <= 16) {
+    const int nw = few_waves(blocks, npanels);
     auto go = [&](auto jmajor, auto nc, auto nwc) {
-      hipLaunchKernelGGL((spmm_narrow_shared<T, OutT, decltype(jmajor)::value, decltype(nc)::value, decltype(nwc)::value>), sgrid,
+      hipLaunchKernelGGL((spmm_few<T, OutT, decltype(jmajor)::value, decltype(nc)::value, decltype(nwc)::value>), dim3((unsigned)((blocks + 7) / 8 * 8)),
                          dim3(64 * decltype(nwc)::value), 0, s,
                          (const uint8_t*)av, (const uint8_t*)am, n_sparse, k, (const uint8_t*)b, ldb * (int64_t)sizeof(T), n_dense,
                          (OutT*)c, ldc, (const OutT*)bias, scale, act);
     };
     auto go_nw = [&](auto jmajor, auto nc) {
-      if (nw == 4) go(jmajor, nc, std::integral_constant<int, 4>{}); else go(jmajor, nc, std::integral_constant<int, 2>{});
+      if (nw == 8) go(jmajor, nc, std::integral_constant<int, 8>{});
+      else if (nw == 4) go(jmajor, nc, std::integral_constant<int, 4>{});
+      else go(jmajor, nc, std::integral_constant<int, 2>{});
     };
-    if (n_dense <= 8) { if (jm) go_nw(std::true_type{}, std::integral_constant<int, 8>{}); else go_nw(std::false_type{}, std::integral_constant<int, 8>{}); }
-    else { if (jm) go_nw(std::true_type{}, std::integral_constant<int, 16>{}); else go_nw(std::false_type{}, std::integral_constant<int, 16>{}); }
+    auto go_nc = [&](auto jmajor) {
+      if (n_dense <= 8) go_nw(jmajor, std::integral_constant<int, 8>{}); else go_nw(jmajor, std::integral_constant<int, 16>{});
+    };
+    if (c_layout == TF24_COL_MAJOR) go_nc(std::true_type{}); else go_nc(std::false_type{});
     return check_launch("tf24_spmm");
   }
   int nwaves = kNarrowWaves;                                    // few row blocks: the waves of a block split k
@@ -1718,8 +1726,7 @@ int launch_narrow(const void* av, const void* am, int64_t n_sparse, int64_t k, c
                        (const uint8_t*)am, n_sparse, k, (const uint8_t*)b, ldb * (int64_t)sizeof(T), n_dense, (OutT*)c, ldc, (const OutT*)bias, scale, act);
   };
   auto go_nb = [&](auto jmajor) {
-    if (n_dense <= 16) go(jmajor, std::integral_constant<int, 1>{});
-    else if (n_dense <= 32) go(jmajor, std::integral_constant<int, 2>{});
+    if (n_dense <= 32) go(jmajor, std::integral_constant<int, 2>{});
     else if (n_dense <= 48) go(jmajor, std::integral_constant<int, 3>{});
     else go(jmajor, std::integral_constant<int, 4>{});
   };

@@ -1250,6 +1250,28 @@ def test_few_dense_columns(cuda, dtype, n, panels):
             assert yt.equal(want.t()), rows
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float8_e4m3fn])
+@pytest.mark.parametrize("n,panels", [(96, 11), (416, 12), (4096, 23), (4128, 23),            # two waves a row block, a share of five panels and more
+                                      (1056, 25), (6144, 49), (8160, 31),                     # four
+                                      (32, 48), (1568, 49), (4096, 131), (1536, 191),         # eight, shares of one chunk and of several, odd ones
+                                      (8192, 129), (10272, 18)])                              # two again
+def test_one_to_sixteen_rows(cuda, dtype, n, panels):
+    """Few rows against a weight whose row blocks are shared by two, four and eight waves, in whole and partial chunks of panels: exact
+    on small integers, the row behind the last stays as it was."""
+    import sparse
+    from sparse import _native as N
+    k = panels * 128 // torch.empty(0, dtype=dtype).element_size()
+    g = torch.Generator(device=cuda).manual_seed(n + panels)
+    s = sparse.to_sparse_semi_structured(torch.randint(-2, 3, (n, k), device=cuda, generator=g).float(), dtype=dtype)
+    dense = s.to_dense().float()
+    for rows in (1, 2, 3, 7, 8, 9, 10, 15, 16):
+        x = torch.randint(-2, 3, (rows, k), device=cuda, generator=g).to(dtype)
+        y = torch.full((rows + 1, n), 77, dtype=torch.float32, device=cuda)
+        N.check(N.lib().tf24_linear(s._store_values.data_ptr(), s._store_meta.data_ptr(), N.COMPRESSED_PANEL, N.operand_code(dtype), n, k, x.data_ptr(), k, rows,
+                                    y.data_ptr(), N.F32, n, None, 1.0, N.ACT_NONE, None, 0, N.stream_ptr()))
+        assert y[:rows].equal(x.float() @ dense.t()) and bool((y[rows:] == 77).all()), rows
+
+
 @pytest.mark.parametrize("dtype,special", [(F16, float("inf")), (BF16, float("-inf")), (E5M2, float("inf")), (E4M3, float("nan"))])
 @pytest.mark.parametrize("n,panels", [(768, 12), (512, 11), (256, 5), (4096, 22), (1024, 37), (8192, 17), (8224, 3), (10240, 43)])
 def test_few_dense_columns_special_values(cuda, dtype, special, n, panels):
