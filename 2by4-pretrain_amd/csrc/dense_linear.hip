@@ -56,13 +56,23 @@ dense_linear(const uint8_t* __restrict__ w, int64_t ldw, const uint8_t* __restri
   const int xcd = (int)(blockIdx.x & 7), slot = (int)(blockIdx.x >> 3), xcd_end = min((xcd + 1) * per_xcd, ntiles);
   int tile = xcd * per_xcd + slot;
   if (tile >= xcd_end) return;
-  auto locate = [&](int t, int64_t& ti0, int64_t& tj0) {
-    const int group = t / (kRaster * tiles_j), gh = min(kRaster, tiles_i - group * kRaster), in_group = t - group * kRaster * tiles_j;
-    ti0 = (int64_t)(group * kRaster + in_group % gh) * kTile;
-    tj0 = (int64_t)(in_group / gh) * kTile;
+  int group = __builtin_amdgcn_readfirstlane(tile / (kRaster * tiles_j)), in_group = tile - group * (kRaster * tiles_j);
+  auto locate = [&](int64_t& ti0, int64_t& tj0) {                // origin of the tile number in_group of the group
+    const int gh = min(kRaster, tiles_i - group * kRaster);
+    int col = (unsigned)in_group / kRaster;
+    if (gh != kRaster) col = __builtin_amdgcn_readfirstlane((unsigned)in_group / (unsigned)gh);
+    ti0 = (int64_t)(group * kRaster + (in_group - col * gh)) * kTile;
+    tj0 = (int64_t)col * kTile;
+  };
+  auto advance = [&]() {                                         // to the workgroup's next tile
+    in_group += slots;
+    for (int size = min(kRaster, tiles_i - group * kRaster) * tiles_j; in_group >= size; size = min(kRaster, tiles_i - group * kRaster) * tiles_j) {
+      in_group -= size;
+      group++;
+    }
   };
   int64_t i0, j0;
-  locate(tile, i0, j0);
+  locate(i0, j0);
   // every second workgroup of an XCD starts 3 us late, so that not all of them write their tiles out at the same moment (bounded, also
   // in iterations): 4096 x 1024 against 6912 tokens 69.9 -> 64.2 us, 3072 x 768 against 12288 61.4 -> 60.9; 6 us late 66.6, 61.8
   if (stagger_ticks > 0 && (slot & 1)) {
@@ -81,18 +91,24 @@ dense_linear(const uint8_t* __restrict__ w, int64_t ldw, const uint8_t* __restri
   auto strided_swizzle = [](uint32_t krow) { return (((krow >> 1) & 1) << 2) | (((krow >> 3) & 1) << 1); };
   uint32_t ow[kCopies], ox[kCopies];
   const uint8_t *w_at, *x_at;
+  bool lanes_whole = false;
   auto point_at = [&](int64_t ti0, int64_t tj0) {                // sources of the first stage of the tile at (ti0, tj0)
     const int64_t last_i = rows - 1 - ti0, last_j = tokens - 1 - tj0;
     w_at = (STRIDED ? w : w + ti0 * ldw) + first_stage * w_step;
     x_at = x + tj0 * ldx + first_stage * kRowBytes;
+    if constexpr (STRIDED) w_at += ti0 * 2;
+    // the lanes' offsets are those of any other tile unless rows of one of the two are clamped
+    const bool whole = last_i >= kTile - 1 && last_j >= kTile - 1;
+    if (whole && lanes_whole) return;
+    lanes_whole = whole;
 #pragma unroll
     for (int q = 0; q < kCopies; q++) {
       const int row = (wave * kCopies + q) * 8 + (lane >> 3), chunk = (lane & 7) ^ ((row >> 1) & 7);
       ox[q] = (uint32_t)(min((int64_t)row, last_j) * ldx + chunk * 16);
       if constexpr (STRIDED) {
         const uint32_t piece = (uint32_t)((wave * kCopies + q) * 64 + lane), krow = piece / (kTile / 8);
-        const int64_t col = min(ti0 + (int64_t)((piece % (kTile / 8)) ^ strided_swizzle(krow)) * 8, rows - 8);
-        ow[q] = (uint32_t)(krow * ldw + col * 2);
+        const int64_t col = min((int64_t)((piece % (kTile / 8)) ^ strided_swizzle(krow)) * 8, rows - 8 - ti0);
+        ow[q] = (uint32_t)(krow * ldw + col * 2);                // (a tile's columns begin before the last eight: rows is a multiple of 8)
       } else {
         ow[q] = (uint32_t)(min((int64_t)row, last_i) * ldw + chunk * 16);
       }
@@ -203,8 +219,14 @@ dense_linear(const uint8_t* __restrict__ w, int64_t ldw, const uint8_t* __restri
     next_stage();
     if (chained) wait_reads_and_barrier();
     else stage_barrier(true);
+    // Up to the wrap of the stage order, to the last two stages, and, where a tile follows, through those, whose copies are its first two.
+    // (One loop, and few instructions between tiles, which nothing covers: us with stages of their own, in which every copy
+    // stood behind a branch, and new offsets and divisions for every tile, and now: 2048 x 512 against 16384 tokens 43.7 and 42.5, 4096 x 1024 against
+    // 6912 66.0 and 64.3, 5120 x 1280 against 4416 62.0 and 60.3, 3072 x 768 against 12288 59.7 and 58.9.)
     int st = 1;
-    for (int lim = nstages - 2 - first_stage;; lim = nstages - 2) {
+    bool has_next = false;
+    int64_t next_i0 = i0, next_j0 = j0;
+    for (int lim = nstages - 2 - first_stage;;) {
       for (; st < lim; st++) {
         rotate();
         mma_step(1, 0, true, fre, true, cur, 0);                 // the last step of stage st - 1
@@ -212,24 +234,25 @@ dense_linear(const uint8_t* __restrict__ w, int64_t ldw, const uint8_t* __restri
         next_stage();
         stage_barrier(true);
       }
-      if (st >= nstages - 2) break;
-      w_at -= nstages * w_step;                                  // the stage order wraps
-      x_at -= nstages * kRowBytes;
-    }
-    const int next_tile = tile + slots;
-    const bool has_next = next_tile < xcd_end;
-    int64_t next_i0 = i0, next_j0 = j0;
-    if (has_next) {
-      locate(next_tile, next_i0, next_j0);
+      if (st < nstages - 2) {
+        w_at -= nstages * w_step;                                // the stage order wraps
+        x_at -= nstages * kRowBytes;
+        lim = nstages - 2;
+        continue;
+      }
+      if (st >= nstages || tile + slots >= xcd_end) break;
+      tile += slots;
+      has_next = true;
+      advance();
+      locate(next_i0, next_j0);
       point_at(next_i0, next_j0);
+      lim = nstages;
     }
-    for (; st < nstages; st++) {                                 // the last two stages: the copies are the next tile's first two
+    for (; st < nstages; st++) {                                 // the last two stages of the last tile
       rotate();
-      mma_step(1, 0, has_next, fre, true, cur, 0);
-      mma_step(0, 1, has_next, fre, true, cur, 1);
-      next_stage();
-      if (st + 1 < nstages) stage_barrier(has_next);
-      else wait_reads_and_barrier();
+      mma_step(1, 0, false, 0, true, cur, 0);
+      mma_step(0, 1, false, 0, true, cur, 1);
+      stage_barrier(false);
     }
     // the bias of the wave's 96 rows, fetched ahead of the last step
     uint32_t bias_w[2] = {0, 0};
@@ -274,7 +297,7 @@ dense_linear(const uint8_t* __restrict__ w, int64_t ldw, const uint8_t* __restri
       }
     }
     if (!has_next) break;
-    tile = next_tile; i0 = next_i0; j0 = next_j0; chained = true;
+    i0 = next_i0; j0 = next_j0; chained = true;
     rotate();
     clear();
   }
