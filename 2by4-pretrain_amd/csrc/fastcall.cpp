@@ -87,6 +87,7 @@ PyMethodDef methods[] = {
     TF24_METHOD(tf24_masked_add), TF24_METHOD(tf24_adamw_masked_decay_list), TF24_METHOD(tf24_gelu_glu_forward), TF24_METHOD(tf24_gelu_glu_backward),
     TF24_METHOD(tf24_spmm), TF24_METHOD(tf24_linear), TF24_METHOD(tf24_spmm_workspace_bytes), TF24_METHOD(tf24_grad_weight), TF24_METHOD(tf24_grad_weight_f32),
     TF24_METHOD(tf24_grad_weight_workspace_bytes), TF24_METHOD(tf24_linear16), TF24_METHOD(tf24_linear16_suits), TF24_METHOD(tf24_transpose),
+    TF24_METHOD(tf24_mvue_weight_grad), TF24_METHOD(tf24_mvue_weight_grad_workspace_bytes),
     {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_fastcall", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 

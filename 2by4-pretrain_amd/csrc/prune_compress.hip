@@ -532,35 +532,9 @@ prune_compress_col(const In* __restrict__ dense, int64_t ld, int64_t m, int64_t 
   }
 }
 
-// rowsum[r] = sum over column blocks of partial[b][r], one rounding to T.  A block takes 32 rows;
-// its 8 groups of 32 lanes each add every 8th column block (coalesced 128-byte reads), then the 8
-// group sums of a row are added in group order.
-template <typename T>
+// a block for every 32 rows (row_sums_of_block)
 __global__ void __launch_bounds__(kThreads)
-rowsum_finish(const float* __restrict__ partial, int nblocks, int64_t m, T* __restrict__ out) {
-  __shared__ float s_part[8][32];
-  const int lr = threadIdx.x & 31, part = threadIdx.x >> 5;
-  const int64_t r = (int64_t)blockIdx.x * 32 + lr;
-  float t = 0.0f;
-  if (r < m) {
-    // eight loads in flight: waiting for each made this tail 5 us long on 96 column blocks
-    for (int b = part; b < nblocks; b += 64) {
-      float v[8];
-#pragma unroll
-      for (int u = 0; u < 8; u++) v[u] = b + 8 * u < nblocks ? partial[(int64_t)(b + 8 * u) * m + r] : 0.0f;
-#pragma unroll
-      for (int u = 0; u < 8; u++) t += v[u];
-    }
-  }
-  s_part[part][lr] = t;
-  __syncthreads();
-  if (part == 0 && r < m) {
-    float sum = 0.0f;
-#pragma unroll
-    for (int q = 0; q < 8; q++) sum += s_part[q][lr];
-    out[r] = from_float<T>(sum);
-  }
-}
+rowsum_finish(RowSums sums) { row_sums_of_block(sums, blockIdx.x); }
 
 // {seed, offset} in device memory: offset += by (vector store from one lane)
 __global__ void advance_philox_offset(uint64_t* state, uint64_t by) {
@@ -727,6 +701,17 @@ extern "C" int tf24_prune_compress(const void* dense, int in_dtype, int layout, 
                                   values, out_dtype, meta, out_layout, nullptr, stream);
 }
 
+int tf24::compress_with_partial_sums(const char* fn, const void* dense, int dtype, int64_t ld, int64_t m, int64_t k, int mode, const void* rnd, void* values,
+                                     void* meta, float* partial, hipStream_t stream) {
+  return run_prune_compress(fn, dense, dtype, TF24_COL_MAJOR, ld, m, k, mode, nullptr, TF24_U8, 0, (const float*)rnd, 0, values, dtype, meta, TF24_COMPRESSED_PANEL,
+                            partial, stream);
+}
+
+int tf24::finish_row_sums(const char* fn, const RowSums& sums, hipStream_t stream) {
+  hipLaunchKernelGGL(rowsum_finish, dim3((unsigned)sums.blocks()), dim3(kThreads), 0, stream, sums);
+  return check_launch(fn);
+}
+
 extern "C" int64_t tf24_prune_compress_rowsum_workspace_bytes(int64_t m, int64_t k) {
   return m > 0 && k > 0 ? ((k + 127) / 128) * m * (int64_t)sizeof(float) : 0;
 }
@@ -753,15 +738,7 @@ extern "C" int tf24_prune_compress_rowsum(const void* dense, int in_dtype, int l
   rc = run_prune_compress(fn, dense, in_dtype, layout, ld, m, k, mode, mask, mask_dtype, mask_ld, rnd, rand_ld, values, out_dtype, meta,
                           out_layout, (float*)workspace, stream);
   if (rc) return rc;
-  const int nblocks = (int)((k + 127) / 128);
-  dim3 grid((unsigned)((m + 31) / 32));
-  hipStream_t s = (hipStream_t)stream;
-  switch (rowsum_dtype) {
-    case TF24_F32: hipLaunchKernelGGL((rowsum_finish<float>), grid, dim3(kThreads), 0, s, (const float*)workspace, nblocks, m, (float*)rowsum); break;
-    case TF24_F16: hipLaunchKernelGGL((rowsum_finish<f16_t>), grid, dim3(kThreads), 0, s, (const float*)workspace, nblocks, m, (f16_t*)rowsum); break;
-    default: hipLaunchKernelGGL((rowsum_finish<bf16_t>), grid, dim3(kThreads), 0, s, (const float*)workspace, nblocks, m, (bf16_t*)rowsum); break;
-  }
-  return check_launch(fn);
+  return finish_row_sums(fn, RowSums{(const float*)workspace, (int)((k + 127) / 128), m, rowsum, rowsum_dtype}, (hipStream_t)stream);
 }
 
 // ------------------------------------------------------------------------------------------

@@ -76,7 +76,7 @@ namespace tf24 {
 namespace {
 int run_spmm(const char* fn, const void* a_values, const void* a_meta, int a_layout, int dtype, int64_t n_sparse, int64_t k,
              const void* b, int b_layout, int64_t ldb, int64_t n_dense, int64_t extent, void* c, int out_dtype, int c_layout, int64_t ldc,
-             const void* bias, float scale, int activation, void* workspace, int64_t workspace_bytes, void* stream) {
+             const void* bias, float scale, int activation, void* workspace, int64_t workspace_bytes, void* stream, RowSums* sums = nullptr) {
   const int bias_f32 = activation & TF24_BIAS_F32;
   int rc = validate(fn, dtype, n_sparse, k, b_layout, ldb, n_dense, extent, out_dtype, c_layout, ldc, activation);
   if (rc) return rc;
@@ -90,11 +90,11 @@ int run_spmm(const char* fn, const void* a_values, const void* a_meta, int a_lay
   hipStream_t s = (hipStream_t)stream;
   if (dtype == TF24_I8 && scale != 1.0f) return fail(TF24_ERR_ARG, "%s: int8 products are exact, scale must be 1 (%g given)", fn, (double)scale);
   switch (dtype) {
-    case TF24_I8: return spmm_i8(out_dtype, a_values, a_meta, a_layout, n_sparse, k, b, b_layout, ldb, n_dense, c, c_layout, ldc, bias, scale, activation, workspace, workspace_bytes, s);
-    case TF24_F16: return spmm_f16(out_dtype, a_values, a_meta, a_layout, n_sparse, k, b, b_layout, ldb, n_dense, c, c_layout, ldc, bias, scale, activation, workspace, workspace_bytes, s);
-    case TF24_BF16: return spmm_bf16(out_dtype, a_values, a_meta, a_layout, n_sparse, k, b, b_layout, ldb, n_dense, c, c_layout, ldc, bias, scale, activation, workspace, workspace_bytes, s);
-    case TF24_E5M2: return spmm_e5m2(out_dtype, a_values, a_meta, a_layout, n_sparse, k, b, b_layout, ldb, n_dense, c, c_layout, ldc, bias, scale, activation, workspace, workspace_bytes, s);
-    default: return spmm_e4m3(out_dtype, a_values, a_meta, a_layout, n_sparse, k, b, b_layout, ldb, n_dense, c, c_layout, ldc, bias, scale, activation, workspace, workspace_bytes, s);
+    case TF24_I8: return spmm_i8(out_dtype, a_values, a_meta, a_layout, n_sparse, k, b, b_layout, ldb, n_dense, c, c_layout, ldc, bias, scale, activation, workspace, workspace_bytes, s, sums);
+    case TF24_F16: return spmm_f16(out_dtype, a_values, a_meta, a_layout, n_sparse, k, b, b_layout, ldb, n_dense, c, c_layout, ldc, bias, scale, activation, workspace, workspace_bytes, s, sums);
+    case TF24_BF16: return spmm_bf16(out_dtype, a_values, a_meta, a_layout, n_sparse, k, b, b_layout, ldb, n_dense, c, c_layout, ldc, bias, scale, activation, workspace, workspace_bytes, s, sums);
+    case TF24_E5M2: return spmm_e5m2(out_dtype, a_values, a_meta, a_layout, n_sparse, k, b, b_layout, ldb, n_dense, c, c_layout, ldc, bias, scale, activation, workspace, workspace_bytes, s, sums);
+    default: return spmm_e4m3(out_dtype, a_values, a_meta, a_layout, n_sparse, k, b, b_layout, ldb, n_dense, c, c_layout, ldc, bias, scale, activation, workspace, workspace_bytes, s, sums);
   }
 }
 }  // namespace
@@ -118,4 +118,51 @@ extern "C" int tf24_linear(const void* a_values, const void* a_meta, int a_layou
                            const void* bias, float scale, int activation, void* workspace, int64_t workspace_bytes, void* stream) {
   return tf24::run_spmm("tf24_linear", a_values, a_meta, a_layout, dtype, n_sparse, k, x, TF24_ROW_MAJOR, ldx, rows, 1, y, out_dtype,
                         TF24_COL_MAJOR, ldy, bias, scale, activation, workspace, workspace_bytes, stream);
+}
+
+// ---- the weight gradient of the transposable layer: MVUE24(dY^T) . X and the row sums of dY^T, three launches (conversion, product in pieces
+// of the token axis, their sum with the row sums) and one workspace.
+namespace tf24 {
+namespace {
+struct GradSpace { int64_t meta, partial, pieces, pieces_bytes, total; };          // offsets behind the compressed values
+GradSpace grad_space(int64_t m, int64_t n, int64_t tokens) {
+  auto up = [](int64_t b) { return (b + 255) / 256 * 256; };
+  GradSpace g;
+  g.meta = up(m * tokens);                                                          // (two bytes for every other element)
+  g.partial = g.meta + up(m * tokens / 8);
+  g.pieces = g.partial + up(tf24_prune_compress_rowsum_workspace_bytes(m, tokens));
+  g.pieces_bytes = tf24_spmm_workspace_bytes(TF24_F16, m, tokens, n);
+  g.total = g.pieces + g.pieces_bytes;
+  return g;
+}
+}  // namespace
+}  // namespace tf24
+
+extern "C" int64_t tf24_mvue_weight_grad_workspace_bytes(int64_t m, int64_t n, int64_t tokens) {
+  return m > 0 && n > 0 && tokens > 0 ? tf24::grad_space(m, n, tokens).total : 0;
+}
+
+extern "C" int tf24_mvue_weight_grad(const void* grad, int64_t ldg, const void* x, int64_t ldx, int dtype, int64_t m, int64_t n, int64_t tokens, int mode,
+                                     const void* rnd, void* dw, int dw_dtype, void* db, int db_dtype, void* workspace, int64_t workspace_bytes, void* stream) {
+  using namespace tf24;
+  const char* fn = "tf24_mvue_weight_grad";
+  if (dtype != TF24_F16 && dtype != TF24_BF16) return fail(TF24_ERR_DTYPE, "%s: unsupported operand dtype %d", fn, dtype);
+  if (db_dtype != TF24_F32 && db_dtype != TF24_F16 && db_dtype != TF24_BF16) return fail(TF24_ERR_DTYPE, "%s: unsupported row-sum dtype %d", fn, db_dtype);
+  if (mode != TF24_PRUNE_MVUE_SEEDED && mode != TF24_PRUNE_MVUE_SEEDED_DEVICE) return fail(TF24_ERR_ARG, "%s: mode %d does not draw its uniforms", fn, mode);
+  // (everything that the product will ask for, before the conversion is launched)
+  int rc = validate(fn, dtype, m, tokens, TF24_COL_MAJOR, ldx, n, 0, dw_dtype, TF24_ROW_MAJOR, n, TF24_ACT_NONE);
+  if (rc) return rc;
+  if (!grad || !x || !dw || !db || !workspace) return fail(TF24_ERR_ARG, "%s: null pointer", fn);
+  const GradSpace at = grad_space(m, n, tokens);
+  if (workspace_bytes < at.total)
+    return fail(TF24_ERR_ARG, "%s: workspace of %lld bytes is too small (%lld needed)", fn, (long long)workspace_bytes, (long long)at.total);
+  if ((rc = check_aligned(fn, 16, {x, dw, workspace}))) return rc;
+  if ((rc = check_aligned(fn, dtype_size(db_dtype), {db}))) return rc;
+  uint8_t* const ws = (uint8_t*)workspace;
+  float* const partial = (float*)(ws + at.partial);
+  if ((rc = compress_with_partial_sums(fn, grad, dtype, ldg, m, tokens, mode, rnd, ws, ws + at.meta, partial, (hipStream_t)stream))) return rc;
+  RowSums sums{partial, (int)((tokens + 127) / 128), m, db, db_dtype};
+  rc = run_spmm(fn, ws, ws + at.meta, TF24_COMPRESSED_PANEL, dtype, m, tokens, x, TF24_COL_MAJOR, ldx, n, 0, dw, dw_dtype, TF24_ROW_MAJOR, n, nullptr, 1.0f, TF24_ACT_NONE,
+                at.pieces_bytes ? ws + at.pieces : nullptr, at.pieces_bytes, stream, &sums);
+  return rc || !sums.partial ? rc : finish_row_sums(fn, sums, (hipStream_t)stream);
 }

@@ -1042,13 +1042,20 @@ spmm_pipe(const uint8_t* __restrict__ a_values, const uint8_t* __restrict__ a_me
 
 // Second pass of a split-K product: a block handles one eighth of a tile (the accumulator groups
 // `slab` of one ti), same lane -> element mapping as spmm_pipe; sums the `splits` partial tiles
-// (float32, or int32 for int8 operands) and applies scale / bias / activation / conversion.
+// (float32, or int32 for int8 operands) and applies scale / bias / activation / conversion.  Blocks past the tiles finish the row
+// sums that a weight gradient's conversion left (`sums`; a launch of their own takes 4 to 5 us).
 template <typename Acc4, typename OutT, bool C_JMAJOR, typename C>
 __global__ void __launch_bounds__(C::THREADS)
 spmm_reduce_splits(const float* __restrict__ partial, int splits, int tiles_i, int tiles_j, int64_t n_sparse, int64_t n_dense,
-                   OutT* __restrict__ c, int64_t ldc, const OutT* __restrict__ bias, float scale, int act) {
+                   OutT* __restrict__ c, int64_t ldc, const OutT* __restrict__ bias, float scale, int act, RowSums sums) {
   const int ntiles = tiles_i * tiles_j;
   const int tile = blockIdx.x;
+  if constexpr (C::THREADS >= 256) {
+    if (tile >= ntiles) {
+      row_sums_of_block(sums, (int64_t)(tile - ntiles) * gridDim.y + blockIdx.y);       // (past the last row: none)
+      return;
+    }
+  }
   constexpr int GH = C::GH;
   const int group = tile / (GH * tiles_j);
   const int gh = min(GH, tiles_i - group * GH);
@@ -1286,14 +1293,14 @@ bool strided_takes_square(int64_t n_sparse, int64_t k, int64_t n_dense, int64_t 
 template <typename T, typename OutT, typename C>
 int launch_tiled(const void* av, const void* am, int64_t n_sparse, int64_t k, const void* b, int b_layout, int64_t ldb,
                  int64_t n_dense, void* c, int c_layout, int64_t ldc, const void* bias, float scale, int act,
-                 void* workspace, int64_t workspace_bytes, hipStream_t s) {
+                 void* workspace, int64_t workspace_bytes, hipStream_t s, RowSums* sums = nullptr) {
   constexpr bool SQUARE = std::is_same<C, SquareCfg>::value;       // (this way for a k-strided dense operand only)
   const int cu_slots = compute_units() / 8;
   if constexpr (std::is_same<C, TiledCfg>::value && sizeof(T) == 2) {
     if (b_layout == TF24_COL_MAJOR &&
         strided_takes_square<T, OutT>(n_sparse, k, n_dense, workspace ? workspace_bytes : 0, c_layout == TF24_COL_MAJOR, cu_slots))
       return launch_tiled<T, OutT, SquareCfg>(av, am, n_sparse, k, b, b_layout, ldb, n_dense, c, c_layout, ldc, bias, scale, act, workspace,
-                                              workspace_bytes, s);
+                                              workspace_bytes, s, sums);
   }
   int tiles_i = (int)((n_sparse + C::BI - 1) / C::BI);
   const int tiles_j = (int)((n_dense + C::BJ - 1) / C::BJ);
@@ -1407,13 +1414,16 @@ int launch_tiled(const void* av, const void* am, int64_t n_sparse, int64_t k, co
   }
   launch_tail();
   if (splits > 1) {
-    dim3 rgrid((unsigned)(tiles_i * tiles_j), C::TI * C::TJ * 4);      // one accumulator group of the tile per block
+    constexpr int GROUPS = C::TI * C::TJ * 4;                                      // one accumulator group of the tile per block
+    RowSums rows{};
+    if (C::THREADS >= 256 && sums) { rows = *sums; sums->partial = nullptr; }      // (finished here)
+    dim3 rgrid((unsigned)(tiles_i * tiles_j + (rows.blocks() + GROUPS - 1) / GROUPS), GROUPS);
     if (jm)
       hipLaunchKernelGGL((spmm_reduce_splits<typename mma32<T>::acc4_t, OutT, true, C>), rgrid, dim3(C::THREADS), 0, s, (const float*)workspace, splits, tiles_i, tiles_j,
-                         n_sparse, n_dense, (OutT*)c, ldc, (const OutT*)bias, scale, act);
+                         n_sparse, n_dense, (OutT*)c, ldc, (const OutT*)bias, scale, act, rows);
     else
       hipLaunchKernelGGL((spmm_reduce_splits<typename mma32<T>::acc4_t, OutT, false, C>), rgrid, dim3(C::THREADS), 0, s, (const float*)workspace, splits, tiles_i, tiles_j,
-                         n_sparse, n_dense, (OutT*)c, ldc, (const OutT*)bias, scale, act);
+                         n_sparse, n_dense, (OutT*)c, ldc, (const OutT*)bias, scale, act, rows);
   }
   return check_launch("tf24_spmm");
 }
@@ -1753,7 +1763,7 @@ int launch_general(const void* av, const void* am, int a_layout, int64_t n_spars
 template <typename T>
 int dispatch_out(int out_dtype, const void* av, const void* am, int a_layout, int64_t n_sparse, int64_t k, const void* b, int b_layout,
                  int64_t ldb, int64_t n_dense, void* c, int c_layout, int64_t ldc, const void* bias, float scale, int act,
-                 void* workspace, int64_t workspace_bytes, hipStream_t s) {
+                 void* workspace, int64_t workspace_bytes, hipStream_t s, RowSums* sums) {
   const bool panel = a_layout == TF24_COMPRESSED_PANEL;
   // the tiled kernel reads a k-strided dense operand through transposing LDS reads (16-bit types only)
   // (also for a narrow dense operand: with its k pieces the tiled kernel beats the general one from 8 columns on)
@@ -1795,9 +1805,9 @@ int dispatch_out(int out_dtype, const void* av, const void* am, int a_layout, in
   }
   if (tiled) {
     switch (out_dtype) {
-      case TF24_F16: return launch_tiled<T, f16_t, TiledCfg>(av, am, n_sparse, k, b, b_layout, ldb, n_dense, c, c_layout, ldc, bias, scale, act, workspace, workspace_bytes, s);
-      case TF24_BF16: return launch_tiled<T, bf16_t, TiledCfg>(av, am, n_sparse, k, b, b_layout, ldb, n_dense, c, c_layout, ldc, bias, scale, act, workspace, workspace_bytes, s);
-      case TF24_F32: return launch_tiled<T, float, TiledCfg>(av, am, n_sparse, k, b, b_layout, ldb, n_dense, c, c_layout, ldc, bias, scale, act, workspace, workspace_bytes, s);
+      case TF24_F16: return launch_tiled<T, f16_t, TiledCfg>(av, am, n_sparse, k, b, b_layout, ldb, n_dense, c, c_layout, ldc, bias, scale, act, workspace, workspace_bytes, s, sums);
+      case TF24_BF16: return launch_tiled<T, bf16_t, TiledCfg>(av, am, n_sparse, k, b, b_layout, ldb, n_dense, c, c_layout, ldc, bias, scale, act, workspace, workspace_bytes, s, sums);
+      case TF24_F32: return launch_tiled<T, float, TiledCfg>(av, am, n_sparse, k, b, b_layout, ldb, n_dense, c, c_layout, ldc, bias, scale, act, workspace, workspace_bytes, s, sums);
     }
   }
   switch (out_dtype) {
@@ -1812,11 +1822,12 @@ int dispatch_out(int out_dtype, const void* av, const void* am, int a_layout, in
 }  // namespace
 
 // One translation unit per operand type instantiates the kernels of that type (spmm_<type>.hip) behind
-// one of these functions; tf24_spmm (spmm.hip) validates and dispatches on the type.
+// one of these functions; tf24_spmm (spmm.hip) validates and dispatches on the type.  `sums`: row sums that the product's last launch may
+// finish as well; it clears their `partial` if it does.
 #define TF24_SPMM_ENTRY_ARGS int out_dtype, const void* av, const void* am, int a_layout, int64_t n_sparse, int64_t k, const void* b, int b_layout, \
                  int64_t ldb, int64_t n_dense, void* c, int c_layout, int64_t ldc, const void* bias, float scale, int act, \
-                 void* workspace, int64_t workspace_bytes, hipStream_t s
-#define TF24_SPMM_ENTRY_PASS out_dtype, av, am, a_layout, n_sparse, k, b, b_layout, ldb, n_dense, c, c_layout, ldc, bias, scale, act, workspace, workspace_bytes, s
+                 void* workspace, int64_t workspace_bytes, hipStream_t s, RowSums* sums
+#define TF24_SPMM_ENTRY_PASS out_dtype, av, am, a_layout, n_sparse, k, b, b_layout, ldb, n_dense, c, c_layout, ldc, bias, scale, act, workspace, workspace_bytes, s, sums
 int spmm_f16(TF24_SPMM_ENTRY_ARGS);
 int spmm_bf16(TF24_SPMM_ENTRY_ARGS);
 int spmm_e4m3(TF24_SPMM_ENTRY_ARGS);

@@ -509,4 +509,49 @@ __device__ __forceinline__ Pack<Out, 4> from_float4(float a0, float b0, bool fin
   return o;
 }
 
+// ---------------------------------------------------------------- row sums
+// out[r] = sum over column blocks of partial[b * m + r], one rounding to out's type (F32 | F16 | BF16): what is left to do behind a
+// conversion that also adds the rows of its matrix, 128 columns at a time.
+struct RowSums {
+  const float* partial;
+  int nblocks;
+  int64_t m;
+  void* out;
+  int dtype;
+  int64_t blocks() const { return (m + 31) / 32; }
+};
+// Rows 32 `block` .. + 31, by the first 256 lanes of a workgroup (all of which enter).  8 groups of 32 lanes each add every 8th column
+// block (coalesced 128-byte reads), then the 8 group sums of a row are added in group order.
+__device__ __forceinline__ void row_sums_of_block(const RowSums& s, int64_t block) {
+  __shared__ float s_part[8][32];
+  const int lr = threadIdx.x & 31, part = threadIdx.x >> 5;
+  const int64_t r = block * 32 + lr;
+  float t = 0.0f;
+  if (r < s.m && part < 8) {
+    // eight loads in flight: waiting for each made this tail 5 us long on 96 column blocks
+    for (int b = part; b < s.nblocks; b += 64) {
+      float v[8];
+#pragma unroll
+      for (int u = 0; u < 8; u++) v[u] = b + 8 * u < s.nblocks ? s.partial[(int64_t)(b + 8 * u) * s.m + r] : 0.0f;
+#pragma unroll
+      for (int u = 0; u < 8; u++) t += v[u];
+    }
+  }
+  if (part < 8) s_part[part][lr] = t;
+  __syncthreads();
+  if (part == 0 && r < s.m) {
+    float sum = 0.0f;
+#pragma unroll
+    for (int q = 0; q < 8; q++) sum += s_part[q][lr];
+    if (s.dtype == TF24_F32) reinterpret_cast<float*>(s.out)[r] = sum;
+    else if (s.dtype == TF24_F16) reinterpret_cast<f16_t*>(s.out)[r] = from_float<f16_t>(sum);
+    else reinterpret_cast<bf16_t*>(s.out)[r] = from_float<bf16_t>(sum);
+  }
+}
+// The conversion of a column-major matrix by an MVUE mode that draws its uniforms, to panel form of the same 16-bit type, its partial
+// sums left in `partial`; and the launch that finishes them.
+int compress_with_partial_sums(const char* fn, const void* dense, int dtype, int64_t ld, int64_t m, int64_t k, int mode, const void* rnd, void* values, void* meta,
+                               float* partial, hipStream_t stream);
+int finish_row_sums(const char* fn, const RowSums& sums, hipStream_t stream);
+
 }  // namespace tf24

@@ -65,6 +65,8 @@ _SIGNATURES = {
     "tf24_spmm": (_i, [_p, _p, _i, _i, _i64, _i64, _p, _i, _i64, _i64, _p, _i, _i, _i64, _p, _f, _i, _p, _i64, _p]),
     "tf24_linear": (_i, [_p, _p, _i, _i, _i64, _i64, _p, _i64, _i64, _p, _i, _i64, _p, _f, _i, _p, _i64, _p]),
     "tf24_spmm_workspace_bytes": (_i64, [_i, _i64, _i64, _i64]),
+    "tf24_mvue_weight_grad": (_i, [_p, _i64, _p, _i64, _i, _i64, _i64, _i64, _i, _p, _p, _i, _p, _i, _p, _i64, _p]),
+    "tf24_mvue_weight_grad_workspace_bytes": (_i64, [_i64, _i64, _i64]),
     "tf24_grad_weight": (_i, [_p, _i64, _p, _i64, _i, _i64, _i64, _i64, _p, _p, _p, _i64, _p]),
     "tf24_grad_weight_f32": (_i, [_p, _i64, _p, _i64, _i, _i64, _i64, _i64, _p, _p, _p, _i64, _p]),
     "tf24_grad_weight_workspace_bytes": (_i64, [_i64, _i64, _i64]),

@@ -715,3 +715,41 @@ def to_sparse_semi_structured_with_row_sums(original_tensor: torch.Tensor, MVUE2
         return (to_sparse_semi_structured(t, MVUE24=MVUE24, mask=mask, dtype=dtype, rand=rand), t.sum(1, dtype=sums_dtype))
     values, meta, sums = _compress(t, dtype, MVUE24, mask, rand, True, row_sums=sums_dtype or True)
     return SparseSemiStructuredTensor._from_storage(values, meta, (m, n), N.COMPRESSED_PANEL, torch.Size((m, n)), False), sums
+
+
+_GRAD_SPACE = {}           # (m, n, tokens) -> tf24_mvue_weight_grad_workspace_bytes, a pure function of the shape
+
+
+def _mvue_weight_gradient(grad, x, weight_dtype, sums_dtype):
+    """(MVUE24(grad.T) @ x, grad.sum(0)), the gradients of a layer's weight and bias, in one call of the library: the bits of
+    to_sparse_semi_structured_with_row_sums and the product with its result, with one allocation of scratch and one launch fewer (the
+    sums are finished by the launch that adds the product's pieces).  None where that does not go as the operands lie: any case that the
+    two calls bring into another form first, refuse, or run on other kernels."""
+    dtype = x.dtype
+    if (type(grad) is not torch.Tensor or type(x) is not torch.Tensor or dtype not in _SIXTEEN_BIT or grad.dtype is not dtype or grad.dim() != 2
+            or x.dim() != 2 or not grad.is_cuda or x.device != grad.device or weight_dtype not in (torch.float32, torch.float16, torch.bfloat16)
+            or not SparseSemiStructuredTensor._PANEL_LAYOUT):
+        return None
+    cfg = _DTYPE_TO_SEMI_STRUCTURED_SPARSE_CONFIG[dtype]
+    tokens, m = grad.shape
+    n = x.shape[1]
+    (g0, g1), (x0, x1) = grad.stride(), x.stride()
+    if (x.shape[0] != tokens or m < cfg.sparse_min_rows or m % cfg.sparse_min_rows or tokens < cfg.sparse_min_cols or tokens % cfg.sparse_min_cols
+            or n <= 64 or n % 8 or g1 != 1 or g0 < m or g0 % 8 or x1 != 1 or x0 < n or x0 % 8 or x0 > 1 << 23 or (grad.data_ptr() | x.data_ptr()) % 16):
+        return None
+    space = _GRAD_SPACE.get((m, n, tokens))
+    if space is None:
+        space = _GRAD_SPACE[(m, n, tokens)] = N.lib().tf24_mvue_weight_grad_workspace_bytes(m, n, tokens)
+    device = grad.device
+    rand = _next_philox_state(device)
+    if isinstance(rand, tuple):
+        mode, words = N.PRUNE_MVUE_SEEDED, (ctypes.c_uint64 * 2)(rand[0] & (2 ** 64 - 1), rand[1] & (2 ** 64 - 1))
+        rand_at = ctypes.addressof(words)            # read by the library during the call
+    else:
+        mode, rand_at = N.PRUNE_MVUE_SEEDED_DEVICE, rand.data_ptr()
+    dw = torch.empty((m, n), dtype=weight_dtype, device=device)
+    db = torch.empty((m,), dtype=sums_dtype or dtype, device=device)
+    workspace = torch.empty(space, dtype=torch.uint8, device=device)
+    N.check(N.lib().tf24_mvue_weight_grad(grad.data_ptr(), g0, x.data_ptr(), x0, N.dtype_code(dtype), m, n, tokens, mode, rand_at, dw.data_ptr(),
+                                          N.dtype_code(weight_dtype), db.data_ptr(), N.dtype_code(db.dtype), workspace.data_ptr(), space, N.stream_ptr()))
+    return dw, db

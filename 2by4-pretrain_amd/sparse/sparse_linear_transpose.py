@@ -14,7 +14,7 @@ import torch
 import torch.nn.functional as F
 from torch import autograd, nn
 
-from .semi_structured import (SparseSemiStructuredTensor, _dense_times_sparse_t, _spmm, to_sparse_semi_structured,
+from .semi_structured import (SparseSemiStructuredTensor, _dense_times_sparse_t, _mvue_weight_gradient, _spmm, to_sparse_semi_structured,
                               to_sparse_semi_structured_pair, to_sparse_semi_structured_with_row_sums)
 from .transposable_semi_structured import TransposableSparse, transposable_mask_
 
@@ -84,13 +84,20 @@ class sparse_linear_transpose(autograd.Function):
         if needs[1]:
             if input.dim() != 2:
                 input = input.view(-1, input.shape[-1])
+            both = None
             if needs[4]:
+                sums_dtype = torch.float32 if ctx.bias_dtype == torch.float32 else None
+                both = _mvue_weight_gradient(grad_output, input, ctx.weight_dtype, sums_dtype)
+            if both is not None:
+                grad_weight, grad_bias = both
+            elif needs[4]:
                 # MVUE24(dY^T) and grad_bias = dY.sum(0) (README.md:193-197) from one read of dY
                 grad_sparse, grad_bias = to_sparse_semi_structured_with_row_sums(
-                    grad_output.t(), MVUE24=True, dtype=grad_output.dtype, sums_dtype=torch.float32 if ctx.bias_dtype == torch.float32 else None)
+                    grad_output.t(), MVUE24=True, dtype=grad_output.dtype, sums_dtype=sums_dtype)
             else:
                 grad_sparse = to_sparse_semi_structured(grad_output.t(), MVUE24=True, dtype=grad_output.dtype)
-            grad_weight = _spmm(grad_sparse, input, True, out_dtype=ctx.weight_dtype)
+            if both is None:
+                grad_weight = _spmm(grad_sparse, input, True, out_dtype=ctx.weight_dtype)
         elif needs[4]:
             with torch.autocast(device_type="cuda", enabled=False):      # (autocast would promote the sum to float32)
                 grad_bias = grad_output.sum(0)

@@ -391,6 +391,18 @@ int tf24_linear(const void* a_values, const void* a_meta, int a_layout, int dtyp
                 const void* x, int64_t ldx, int64_t rows, void* y, int out_dtype, int64_t ldy,
                 const void* bias, float scale, int activation, void* workspace, int64_t workspace_bytes, void* stream);
 int64_t tf24_spmm_workspace_bytes(int dtype, int64_t n_sparse, int64_t k, int64_t n_dense);
+/*
+ * The weight and bias gradient of the transposable 2:4 layer (the reference's sparse_linear_transpose.backward, README.md:190-200) in one call:
+ *     dw [m, n] = MVUE24(grad^T) . x,   db [m] = sum over tokens of grad,      grad [tokens, m], x [tokens, n] row-major
+ * The same bits as tf24_prune_compress_rowsum (column-major [m, tokens], panel form) followed by tf24_spmm on its result.
+ *   dtype      F16|BF16 (grad, x); dw_dtype and db_dtype F32|F16|BF16
+ *   mode, rnd  TF24_PRUNE_MVUE_SEEDED or TF24_PRUNE_MVUE_SEEDED_DEVICE and its {seed, offset}
+ *   workspace  tf24_mvue_weight_grad_workspace_bytes(m, n, tokens) bytes, 16-byte aligned
+ * Shape rules: those of the two calls (m % 32, tokens % 64, n % 8; ldg, ldx multiples of 8).
+ */
+int tf24_mvue_weight_grad(const void* grad, int64_t ldg, const void* x, int64_t ldx, int dtype, int64_t m, int64_t n, int64_t tokens, int mode,
+                          const void* rnd, void* dw, int dw_dtype, void* db, int db_dtype, void* workspace, int64_t workspace_bytes, void* stream);
+int64_t tf24_mvue_weight_grad_workspace_bytes(int64_t m, int64_t n, int64_t tokens);
 
 /*
  * GELU-GLU: the last dimension of `in` [rows, cols] holds [x | gate] (cols/2 each);

@@ -968,3 +968,39 @@ def test_grad_weight_kernel_on_many_long_tiles(cuda, tokens, m, n, dtype):
     as in the tests of the others."""
     test_grad_weight_kernel(cuda, tokens, m, n, dtype)
     test_grad_weight_kernel_is_exact_and_deterministic(cuda, tokens, m, n, dtype)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype,weight_dtype,sums_dtype", [(torch.float16, torch.float32, torch.float32), (torch.bfloat16, torch.bfloat16, None),
+                                                           (torch.float16, torch.float16, None)])
+@pytest.mark.parametrize("tokens,m,n", [(64, 32, 72), (64, 96, 200), (192, 3072, 768),            # one piece, the general kernel; one piece
+                                        (2048, 768, 1024), (12288, 768, 72), (4096, 224, 136)])    # several: square tiles, partial ones, few columns
+def test_weight_and_bias_gradient_in_one_call(cuda, dtype, weight_dtype, sums_dtype, tokens, m, n):
+    """The weight's and the bias's gradient by one call of the library are, bit for bit, those of the conversion with row sums and the
+    product with its result, also from pitched views; and the generator moves on alike."""
+    import sparse
+    from sparse.semi_structured import _mvue_weight_gradient, _spmm
+    g = torch.Generator(device=cuda).manual_seed(tokens + m + n)
+    grad = torch.randn(tokens, m + 8, device=cuda, generator=g).to(dtype)
+    x = torch.randn(tokens, n + 16, device=cuda, generator=g).to(dtype)
+    for dy, at in ((grad[:, :m], x[:, :n]), (grad[:, :m].contiguous(), x[:, 8:n + 8].contiguous())):
+        torch.manual_seed(7)
+        s, sums = sparse.to_sparse_semi_structured_with_row_sums(dy.t(), MVUE24=True, dtype=dtype, sums_dtype=sums_dtype)
+        want = _spmm(s, at, True, out_dtype=weight_dtype)
+        after = torch.cuda.default_generators[torch.cuda.current_device()].get_offset()
+        torch.manual_seed(7)
+        dw, db = _mvue_weight_gradient(dy, at, weight_dtype, sums_dtype)
+        assert dw.dtype == weight_dtype and dw.equal(want) and db.dtype == sums.dtype and db.equal(sums)
+        assert torch.cuda.default_generators[torch.cuda.current_device()].get_offset() == after
+
+
+@pytest.mark.gpu
+def test_weight_gradient_in_one_call_is_left_to_the_two(cuda):
+    """Operands that the two calls bring into another form first, refuse or run on other kernels."""
+    from sparse.semi_structured import _mvue_weight_gradient
+    y, x = torch.zeros(128, 64, device=cuda, dtype=torch.float16), torch.zeros(128, 128, device=cuda, dtype=torch.float16)
+    assert _mvue_weight_gradient(y, x, torch.float32, None) is not None
+    for dy, at in ((y[:96], x[:96]), (y[:, :48], x), (y, x[:, :64]), (y, x[:, :100]), (y, x[:64]), (y.t().contiguous().t(), x), (y, x.t().contiguous().t()),
+                   (y.float(), x.float()), (y.bfloat16(), x), (y, torch.zeros(128, 132, device=cuda, dtype=torch.float16)[:, :128]),
+                   (torch.zeros(128 * 64 + 1, device=cuda, dtype=torch.float16)[1:].view(128, 64), x), (torch.nn.Parameter(y), x)):
+        assert _mvue_weight_gradient(dy, at, torch.float32, None) is None
