@@ -1441,13 +1441,15 @@ int launch_tiled(const void* av, const void* am, int64_t n_sparse, int64_t k, co
 // make NaN of an infinite activation.  The full batches are straight-line code and only the last one tests its panels,
 // which is also the faster form (with a test of zeros in every panel 1600 x 6400 fp16 against one column takes 8.5 us, with
 // a choice of the two forms in every batch 9.3, this way 7.8).
-// Up to 16 columns: spmm_few.  17 to 64 (spmm_narrow): a block owns 16 rows, its up to four waves each take a
+// Up to 16 columns, and from kFewPanels panels on up to 32: spmm_few.  Others (spmm_narrow): a block owns 16 rows, its up to four waves each take a
 // share of the k range, read their dense fragments, NB of 16 columns, from global memory (64 contiguous bytes from
 // each of the 16 dense rows, twice) and meet in LDS at the end (added in wave order).  Bound by latency, a few loads deep, at
 // short k and by the requests of the dense fragments at long k: 3072 x 768 bf16 against 37 columns 8.9 us on 256 x 64 tiles,
 // of which there are 12, and 5.4 us here.
 // ------------------------------------------------------------------------------------------
 constexpr int kNarrowWaves = 4;
+// us on spmm_narrow and on spmm_few, 24 columns fp16: 2048 x 512 (8 panels) 3.7 and 3.8, 640 x 640 3.8 and 4.1, 3072 x 768 4.4 and 4.1, 1600 x 1600 6.0 and 4.8
+constexpr int64_t kFewPanels = 12;
 template <typename T, typename OutT, bool C_JMAJOR, int NB>
 __global__ void __launch_bounds__(64 * kNarrowWaves)
 spmm_narrow(const uint8_t* __restrict__ a_values, const uint8_t* __restrict__ a_meta, int64_t n_sparse, int64_t k,
@@ -1552,7 +1554,7 @@ spmm_narrow(const uint8_t* __restrict__ a_values, const uint8_t* __restrict__ a_
   }
 }
 
-// Up to 16 dense columns (NC = 8 or 16): a block owns 16 sparse rows, its NW waves each take a share of the k range and meet in LDS at the
+// Up to 32 dense columns (NC = 8, 16 or 32): a block owns 16 sparse rows, its NW waves each take a share of the k range and meet in LDS at the
 // end (added in wave order).  Bound by the one pass over the compressed operand (50.7 MB of fp16 11008 x 4096, 7.9 us at the rate of a copy) and
 // what a launch, its first loads and its last store take beside it (768 x 768: 2.8 us).  A wave keeps two chunks of 8 panels in flight, in
 // registers; nothing it loads comes from the dense operand but each of the columns there are once, 1 KB a chunk, handed to the fragments
@@ -1563,17 +1565,22 @@ spmm_narrow(const uint8_t* __restrict__ a_values, const uint8_t* __restrict__ a_
 // us before and now, fp16, operands from memory, one column: 11008 x 4096 12.5 and 10.6, 8192 x 8192 17.7 and 14.0, 4096 x 11008 12.8 and 11.3,
 // 4096 x 4096 6.6 and 5.7, 768 x 3072 5.3 and 4.0; eight: 12.8 and 11.7, 17.8 and 15.8, 14.5 and 12.8, 7.0 and 6.1.  Chunks of
 // 16 panels 11008 x 4096 13.6, 8192 x 8192 15.1; two row blocks a wave 12.2 and 15.1 (against 16 columns 14.6 and 16.5, here 14.1 and 19.1).
+// 24 columns, before on fragments from memory or on 256 x 64 tiles and two launches: 4096 x 4096 12.7 and 8.5, 4096 x 8192 15.0 and 13.2, 10240 x 2048
+// 13.3 and 10.3, 768 x 3072 8.6 and 6.9; two row blocks a wave there 9.9, 20.2, 11.3, 9.3; 64 columns of 4096 x 4096 on four fragments 13.8 for 14.9, but of
+// 8192 x 8192 33 for 23.
 template <typename T, typename OutT, bool C_JMAJOR, int NC, int NW>
 __global__ void __launch_bounds__(64 * NW)
 spmm_few(const uint8_t* __restrict__ a_values, const uint8_t* __restrict__ a_meta, int64_t n_sparse, int64_t k,
          const uint8_t* __restrict__ b, int64_t ldb_bytes, int64_t n_dense,
          OutT* __restrict__ c, int64_t ldc, const OutT* __restrict__ bias, float scale, int act) {
   constexpr int KSTEP = mma16<T>::KSTEP;
-  constexpr int CH = 8;                               // panels per chunk: a lane brings one 16-byte piece of each dense column
+  constexpr int NB = (NC + 15) / 16, CHAINS = NB == 1 ? 2 : 1;                    // fragments of 16 columns; instructions in a row that do not wait on each other
+  constexpr int CH = NB == 1 ? 8 : 4;                 // panels per chunk
+  constexpr int COLS = 8 / CH, LOADS = NC / COLS;     // a load of the wave brings 16 bytes a lane, the chunk of COLS dense columns
   constexpr bool PAIR = sizeof(T) == 2;               // two words of metadata per row and panel (8-bit values: four, one for each lane of a row)
   using acc_t = typename mma16<T>::acc_t;
   __shared__ __attribute__((aligned(16))) uint8_t s_b[NW][CH * NC * 128];
-  __shared__ acc_t s_acc[NW - 1][64];
+  __shared__ acc_t s_acc[NW - 1][NB][64];
   const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int64_t blocks16 = n_sparse / 16, per_xcd = (blocks16 + 7) / 8;           // (workgroup ids are dealt to the XCDs round-robin)
@@ -1587,12 +1594,20 @@ spmm_few(const uint8_t* __restrict__ a_values, const uint8_t* __restrict__ a_met
   // the wave's chunk of the dense operand: [panel][column][128 bytes], the 16-byte pieces of a column XOR-swizzled by column / 2, so that
   // the 16 lanes that read one piece position of 16 columns hit different banks
   uint8_t* const sb = s_b[wave];
-  const int colr = li < n_dense ? li : (int)n_dense - 1;
-  const int rd_lo = colr * 128 + ((lk ^ ((colr >> 1) & 7)) * 16), rd_hi = colr * 128 + (((lk + 4) ^ ((colr >> 1) & 7)) * 16);
-  acc_t acc[2];
+  int rd_lo[NB], rd_hi[NB];
+  acc_t acc[NB][CHAINS];
 #pragma unroll
-  for (int r = 0; r < 4; r++) { acc[0][r] = 0; acc[1][r] = 0; }
-  int4v af[2][CH], breg[NC];
+  for (int f = 0; f < NB; f++) {
+    const int col = min(f * 16 + li, (int)n_dense - 1);         // (of a column past the last nothing is stored)
+    rd_lo[f] = col * 128 + ((lk ^ ((col >> 1) & 7)) * 16);
+    rd_hi[f] = col * 128 + (((lk + 4) ^ ((col >> 1) & 7)) * 16);
+#pragma unroll
+    for (int h = 0; h < CHAINS; h++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) acc[f][h][r] = 0;
+  }
+  const int b_col = lane / (CH * 8), b_panel = lane / 8 % CH, b_piece = lane & 7;
+  int4v af[2][CH], breg[LOADS];
   uint32_t words[2][PAIR ? CH / 2 : CH];
   auto load_a = [&](int set, int p) __attribute__((always_inline)) {
 #pragma unroll
@@ -1604,15 +1619,17 @@ spmm_few(const uint8_t* __restrict__ a_values, const uint8_t* __restrict__ a_met
     }
   };
   auto load_b = [&](int p) __attribute__((always_inline)) {
-    const int64_t at = (int64_t)min(p + (lane >> 3), p_end - 1) * 128 + (lane & 7) * 16;
+    const int64_t at = (int64_t)min(p + b_panel, p_end - 1) * 128 + b_piece * 16;
 #pragma unroll
-    for (int j = 0; j < NC; j++)
-      if (j < n_dense) breg[j] = *reinterpret_cast<const int4v*>(b + j * ldb_bytes + at);
+    for (int j = 0; j < LOADS; j++)
+      if (j * COLS < n_dense) breg[j] = *reinterpret_cast<const int4v*>(b + (COLS == 1 ? j : min((int64_t)(j * COLS + b_col), n_dense - 1)) * ldb_bytes + at);
   };
   auto store_b = [&]() __attribute__((always_inline)) {
 #pragma unroll
-    for (int j = 0; j < NC; j++)
-      if (j < n_dense) *reinterpret_cast<int4v*>(sb + ((lane >> 3) * NC + j) * 128 + (((lane & 7) ^ ((j >> 1) & 7)) * 16)) = breg[j];
+    for (int j = 0; j < LOADS; j++) {
+      const int col = j * COLS + b_col;
+      if (j * COLS < n_dense) *reinterpret_cast<int4v*>(sb + (b_panel * NC + col) * 128 + ((b_piece ^ ((col >> 1) & 7)) * 16)) = breg[j];
+    }
   };
   auto index_of = [&](int set, int u) __attribute__((always_inline)) {
     if constexpr (PAIR) {
@@ -1626,10 +1643,14 @@ spmm_few(const uint8_t* __restrict__ a_values, const uint8_t* __restrict__ a_met
     }
   };
   auto multiply_panel = [&](int set, int u) __attribute__((always_inline)) {
-    const int4v lo = *reinterpret_cast<const int4v*>(sb + u * NC * 128 + rd_lo);
-    const int4v hi = *reinterpret_cast<const int4v*>(sb + u * NC * 128 + rd_hi);
-    const int8v bfrag = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-    acc[u & 1] = mma16<T>::template run<0>(af[set][u], bfrag, acc[u & 1], index_of(set, u));
+    const int idx = index_of(set, u);
+#pragma unroll
+    for (int f = 0; f < NB; f++) {
+      const int4v lo = *reinterpret_cast<const int4v*>(sb + u * NC * 128 + rd_lo[f]);
+      const int4v hi = *reinterpret_cast<const int4v*>(sb + u * NC * 128 + rd_hi[f]);
+      const int8v bfrag = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+      acc[f][u % CHAINS] = mma16<T>::template run<0>(af[set][u], bfrag, acc[f][u % CHAINS], idx);
+    }
   };
   auto multiply = [&](int set, int p) __attribute__((always_inline)) {
     if (p + CH <= p_end) {
@@ -1660,30 +1681,42 @@ spmm_few(const uint8_t* __restrict__ a_values, const uint8_t* __restrict__ a_met
       }
     }
   }
-  acc_t sum = acc[0] + acc[1];
-  if (wave > 0) s_acc[wave - 1][lane] = sum;
+#pragma unroll
+  for (int f = 0; f < NB; f++) {
+    if constexpr (CHAINS == 2) acc[f][0] += acc[f][CHAINS - 1];
+    if (wave > 0) s_acc[wave - 1][f][lane] = acc[f][0];
+  }
   __syncthreads();
-  if (wave > 0 || li >= n_dense) return;
-#pragma unroll
-  for (int w = 1; w < NW; w++) sum += s_acc[w - 1][lane];
+  if (wave > 0) return;
   const int64_t row = i0 + lk * 4;           // D layout: column l%16, rows 4*(l/16) + r
-  OutT o[4];
 #pragma unroll
-  for (int r = 0; r < 4; r++) o[r] = to_out<OutT>(finish_value(sum[r], scale, bias, row + r, act));
-  if constexpr (C_JMAJOR) {
-    *reinterpret_cast<Pack<OutT, 4>*>(c + (int64_t)li * ldc + row) = *reinterpret_cast<Pack<OutT, 4>*>(o);
-  } else {
+  for (int f = 0; f < NB; f++) {
+    const int64_t col = f * 16 + li;
+    if (col >= n_dense) continue;
+    acc_t sum = acc[f][0];
 #pragma unroll
-    for (int r = 0; r < 4; r++) c[(row + r) * ldc + li] = o[r];
+    for (int w = 1; w < NW; w++) sum += s_acc[w - 1][f][lane];
+    OutT o[4];
+#pragma unroll
+    for (int r = 0; r < 4; r++) o[r] = to_out<OutT>(finish_value(sum[r], scale, bias, row + r, act));
+    if constexpr (C_JMAJOR) {
+      *reinterpret_cast<Pack<OutT, 4>*>(c + col * ldc + row) = *reinterpret_cast<Pack<OutT, 4>*>(o);
+    } else {
+#pragma unroll
+      for (int r = 0; r < 4; r++) c[(row + r) * ldc + col] = o[r];
+    }
   }
 }
 
-// Waves that share a row block: some 1400 to 2000 waves in all, and six panels for each of them, or two.  us with 2, 4 and 8, fp16, one column:
+// Waves that share a row block: some 1400 to 2000 waves in all, and six panels for each of them, or two; from 17 columns on, where a wave's
+// chunks are shorter, three.  us with 2, 4 and 8, fp16, one column:
 // 11008 x 4096 (688 row blocks) 10.6, 11.0 and 12.7; 8192 x 8192 (512) 14.0, 14.3 and 15.8; 6144 x 4096 (384) 7.9, 7.8 and 8.6;
-// 4096 x 11008 (256) 13.9, 11.4 and 11.3; 768 x 3072 (48) 4.7, 4.3 and 4.0; 3072 x 768 (192, 12 panels) 2.96, 3.03 and 3.6.
-inline int few_waves(int64_t blocks, int64_t npanels) {
-  int waves = blocks <= 256 ? 8 : blocks < 512 ? 4 : 2;
-  while (waves > 2 && npanels < 6 * waves) waves /= 2;
+// 4096 x 11008 (256) 13.9, 11.4 and 11.3; 768 x 3072 (48) 4.7, 4.3 and 4.0; 3072 x 768 (192, 12 panels) 2.96, 3.03 and 3.6.  24 columns:
+// 11008 x 1024 6.7, 7.6 and 12.2; 8192 x 2048 9.4, 8.0 and 9.4; 4096 x 2048 8.0, 6.2 and 5.5; 768 x 768 against 32 5.1, 4.2 and 4.9.
+inline int few_waves(int64_t blocks, int64_t npanels, int64_t n_dense) {
+  const bool many = n_dense > 16;
+  int waves = blocks <= 256 ? 8 : blocks < 512 || (many && blocks == 512) ? 4 : 2;
+  while (waves > 2 && npanels < (many ? 3 : 6) * waves) waves /= 2;
   return waves;
 }
 
@@ -1692,15 +1725,17 @@ inline int few_waves(int64_t blocks, int64_t npanels) {
 // 12.3 -> 7.8 and 11.5 -> 9.2) and some further where there are rows for k pieces of the tiled kernel to be small, but not many (of
 // 4096 x 11008 17.3 -> 13.0 and 17.4 -> 14.7, of 2048 x 11008 14.3 -> 13.0 with 16); beyond, nine or ten from 512 row blocks on (9 and 16 of 8192 x 16384
 // 31.3 -> 30.3 and 31.2 -> 34.7, of 11008 x 16384 42.4 -> 40.3 and 42.7 -> 48.4, but 16 of 768 x 11008 11.8 -> 12.5 and of 512 x 16384 13.4 -> 15.7).
-// More on spmm_narrow, whose fragments cost requests with every panel of every block, so it depends on the panels: 32 columns of 4096 x 2048
-// 10.3 -> 7.7; 64 of 4096 x 1536 13.5 -> 9.4, of
-// 2304 x 768 9.0 -> 6.5, but of 2304 x 2048 10.7 -> 11.2.  With two blocks to a compute unit (6144 rows): 48 of k = 768
-// 9.0 -> 8.0 and of 1536 13.7 -> 12.5, 64 of k = 768 9.1 -> 9.6.  With three (12288 rows) 17 and 32 columns of 16 panels 10.4 -> 8.1 and 10.0, 32 of
-// 24 panels 13.5 -> 14.1; with four (16384 rows) 32 of 16 panels 10.5 -> 12.1.
-inline int64_t narrow_columns(int64_t n_sparse, int64_t npanels) {
+// 17 to 32 on spmm_few as well, which reads them once for every row block: up to 32 panels (24 of 10240 x 2048 13.3 -> 10.3, 32 of 16384 x 1024
+// 11.8 -> 8.3, but of 20480 x 2048 17.0 -> 21.4), of 8-bit values from 512 row blocks on up to 16, which have twice the metadata (11008 x 2048 9.8 -> 8.3, but
+// 11008 x 4096 14.3 -> 16.5); 64 up to two blocks to a compute unit (24 of 6144 x 4096 13.1 -> 12.2, 32 of 8192 x 4096 15.2 -> 13.7, of 256 x 4096 8.4 -> 7.5,
+// but of 11008 x 4096 17.2 -> 19) and 128 with neither more than one nor few (32 of 4096 x 8192 15.0 -> 14.7, of 1600 x 6400 12.4 -> 12.0, but of
+// 512 x 8192 10.5 -> 12.5; 24 of 4096 x 11008 17.5 -> 17.8).  33 to 64 on spmm_narrow, whose fragments cost requests with every panel of every
+// block: 64 of 4096 x 1536 13.5 -> 9.4, of 2304 x 768 9.0 -> 6.5, but of 2304 x 2048 10.7 -> 11.2.  With two blocks to a compute unit (6144 rows):
+// 48 of k = 768 9.0 -> 8.0 and of 1536 13.7 -> 12.5, 64 of k = 768 9.1 -> 9.6.
+inline int64_t narrow_columns(int64_t n_sparse, int64_t npanels, bool eight_bit) {
   const int64_t blocks = n_sparse / 16;
-  if (blocks <= 512 && npanels <= 32) return npanels > 24 ? 32 : blocks <= 256 ? 64 : 48;
-  if (blocks <= 768 && npanels <= 16) return 32;
+  if (blocks <= 512 && npanels <= 24) return blocks <= 256 ? 64 : 48;
+  if ((blocks <= 1024 && npanels <= (eight_bit && blocks > 512 ? 16 : 32)) || (blocks <= 512 && npanels <= 64) || (blocks >= 96 && blocks <= 256 && npanels <= 128)) return 32;
   if (npanels <= 128 || (blocks >= 96 && blocks <= 256 && npanels <= 192)) return 16;
   return blocks >= 512 ? 10 : 8;
 }
@@ -1710,8 +1745,8 @@ int launch_narrow(const void* av, const void* am, int64_t n_sparse, int64_t k, c
                   void* c, int c_layout, int64_t ldc, const void* bias, float scale, int act, hipStream_t s) {
   dim3 grid((unsigned)(n_sparse / 16));
   const int64_t blocks = n_sparse / 16, npanels = k * (int64_t)sizeof(T) / 128;
-  if (n_dense <= 16) {
-    const int nw = few_waves(blocks, npanels);
+  if (n_dense <= 16 || (n_dense <= 32 && npanels >= kFewPanels)) {
+    const int nw = few_waves(blocks, npanels, n_dense);
     auto go = [&](auto jmajor, auto nc, auto nwc) {
       hipLaunchKernelGGL((spmm_few<T, OutT, decltype(jmajor)::value, decltype(nc)::value, decltype(nwc)::value>), dim3((unsigned)((blocks + 7) / 8 * 8)),
                          dim3(64 * decltype(nwc)::value), 0, s,
@@ -1724,7 +1759,9 @@ int launch_narrow(const void* av, const void* am, int64_t n_sparse, int64_t k, c
       else go(jmajor, nc, std::integral_constant<int, 2>{});
     };
     auto go_nc = [&](auto jmajor) {
-      if (n_dense <= 8) go_nw(jmajor, std::integral_constant<int, 8>{}); else go_nw(jmajor, std::integral_constant<int, 16>{});
+      if (n_dense <= 8) go_nw(jmajor, std::integral_constant<int, 8>{});
+      else if (n_dense <= 16) go_nw(jmajor, std::integral_constant<int, 16>{});
+      else go_nw(jmajor, std::integral_constant<int, 32>{});
     };
     if (c_layout == TF24_COL_MAJOR) go_nc(std::true_type{}); else go_nc(std::false_type{});
     return check_launch("tf24_spmm");
@@ -1774,7 +1811,7 @@ int dispatch_out(int out_dtype, const void* av, const void* am, int a_layout, in
   // few dense columns: one pass over the compressed operand (narrow_columns), also up to 16 when the tiled kernel cannot cut k
   // into pieces (no workspace), which it needs to fill the chip
   const bool narrow = panel && b_layout == TF24_ROW_MAJOR &&
-                      (n_dense <= narrow_columns(n_sparse, k * (int64_t)sizeof(T) / 128) || (n_dense <= 16 && !(slim && workspace)));
+                      (n_dense <= narrow_columns(n_sparse, k * (int64_t)sizeof(T) / 128, sizeof(T) == 1) || (n_dense <= 16 && !(slim && workspace)));
   if constexpr (std::is_same<T, i8_t>::value) {        // integer product: int32 accumulators, results and bias
     if (narrow) return launch_narrow<T, int32_t>(av, am, n_sparse, k, b, ldb, n_dense, c, c_layout, ldc, bias, scale, act, s);
     if (slim) return launch_tiled<T, int32_t, SlimCfg>(av, am, n_sparse, k, b, b_layout, ldb, n_dense, c, c_layout, ldc, bias, scale, act, workspace, workspace_bytes, s);

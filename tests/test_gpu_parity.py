@@ -1255,7 +1255,7 @@ def test_few_dense_columns(cuda, dtype, n, panels):
                                       (1056, 25), (6144, 49), (8160, 31),                     # four
                                       (32, 48), (1568, 49), (4096, 131), (1536, 191),         # eight, shares of one chunk and of several, odd ones
                                       (8192, 129), (10272, 18)])                              # two again
-def test_one_to_sixteen_rows(cuda, dtype, n, panels):
+def test_one_to_thirty_two_rows(cuda, dtype, n, panels):
     """Few rows against a weight whose row blocks are shared by two, four and eight waves, in whole and partial chunks of panels: exact
     on small integers, the row behind the last stays as it was."""
     import sparse
@@ -1264,7 +1264,7 @@ def test_one_to_sixteen_rows(cuda, dtype, n, panels):
     g = torch.Generator(device=cuda).manual_seed(n + panels)
     s = sparse.to_sparse_semi_structured(torch.randint(-2, 3, (n, k), device=cuda, generator=g).float(), dtype=dtype)
     dense = s.to_dense().float()
-    for rows in (1, 2, 3, 7, 8, 9, 10, 15, 16):
+    for rows in (1, 2, 3, 7, 8, 9, 10, 15, 16, 17, 24, 25, 31, 32):
         x = torch.randint(-2, 3, (rows, k), device=cuda, generator=g).to(dtype)
         y = torch.full((rows + 1, n), 77, dtype=torch.float32, device=cuda)
         N.check(N.lib().tf24_linear(s._store_values.data_ptr(), s._store_meta.data_ptr(), N.COMPRESSED_PANEL, N.operand_code(dtype), n, k, x.data_ptr(), k, rows,
