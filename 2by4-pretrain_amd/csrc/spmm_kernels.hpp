@@ -1042,15 +1042,16 @@ spmm_pipe(const uint8_t* __restrict__ a_values, const uint8_t* __restrict__ a_me
 
 // Second pass of a split-K product: a block handles one eighth of a tile (the accumulator groups
 // `slab` of one ti), same lane -> element mapping as spmm_pipe; sums the `splits` partial tiles
-// (float32, or int32 for int8 operands) and applies scale / bias / activation / conversion.  Blocks past the tiles finish the row
-// sums that a weight gradient's conversion left (`sums`; a launch of their own takes 4 to 5 us).
-template <typename Acc4, typename OutT, bool C_JMAJOR, typename C>
+// (float32, or int32 for int8 operands) and applies scale / bias / activation / conversion.  SUMS: blocks past the tiles finish the
+// row sums that a weight gradient's conversion left (a launch of their own takes 4 to 5 us; in a kernel of its own because the LDS that it
+// takes costs the others 0.3 us).
+template <typename Acc4, typename OutT, bool C_JMAJOR, typename C, bool SUMS>
 __global__ void __launch_bounds__(C::THREADS)
 spmm_reduce_splits(const float* __restrict__ partial, int splits, int tiles_i, int tiles_j, int64_t n_sparse, int64_t n_dense,
                    OutT* __restrict__ c, int64_t ldc, const OutT* __restrict__ bias, float scale, int act, RowSums sums) {
   const int ntiles = tiles_i * tiles_j;
   const int tile = blockIdx.x;
-  if constexpr (C::THREADS >= 256) {
+  if constexpr (SUMS) {
     if (tile >= ntiles) {
       row_sums_of_block(sums, (int64_t)(tile - ntiles) * gridDim.y + blockIdx.y);       // (past the last row: none)
       return;
@@ -1415,15 +1416,19 @@ int launch_tiled(const void* av, const void* am, int64_t n_sparse, int64_t k, co
   launch_tail();
   if (splits > 1) {
     constexpr int GROUPS = C::TI * C::TJ * 4;                                      // one accumulator group of the tile per block
-    RowSums rows{};
-    if (C::THREADS >= 256 && sums) { rows = *sums; sums->partial = nullptr; }      // (finished here)
-    dim3 rgrid((unsigned)(tiles_i * tiles_j + (rows.blocks() + GROUPS - 1) / GROUPS), GROUPS);
-    if (jm)
-      hipLaunchKernelGGL((spmm_reduce_splits<typename mma32<T>::acc4_t, OutT, true, C>), rgrid, dim3(C::THREADS), 0, s, (const float*)workspace, splits, tiles_i, tiles_j,
-                         n_sparse, n_dense, (OutT*)c, ldc, (const OutT*)bias, scale, act, rows);
-    else
-      hipLaunchKernelGGL((spmm_reduce_splits<typename mma32<T>::acc4_t, OutT, false, C>), rgrid, dim3(C::THREADS), 0, s, (const float*)workspace, splits, tiles_i, tiles_j,
-                         n_sparse, n_dense, (OutT*)c, ldc, (const OutT*)bias, scale, act, rows);
+    auto reduce = [&](auto c_jmajor, auto with_sums, const RowSums& rows) {
+      hipLaunchKernelGGL((spmm_reduce_splits<typename mma32<T>::acc4_t, OutT, decltype(c_jmajor)::value, C, decltype(with_sums)::value>),
+                         dim3((unsigned)(tiles_i * tiles_j + (rows.blocks() + GROUPS - 1) / GROUPS), GROUPS), dim3(C::THREADS), 0, s, (const float*)workspace, splits,
+                         tiles_i, tiles_j, n_sparse, n_dense, (OutT*)c, ldc, (const OutT*)bias, scale, act, rows);
+    };
+    if (jm) {
+      reduce(std::true_type{}, std::false_type{}, RowSums{});
+    } else if (!sums) {
+      reduce(std::false_type{}, std::false_type{}, RowSums{});
+    } else if constexpr (sizeof(T) == 2 && (std::is_same<C, TiledCfg>::value || SQUARE)) {
+      reduce(std::false_type{}, std::true_type{}, *sums);
+      sums->partial = nullptr;                                                    // (finished here)
+    }
   }
   return check_launch("tf24_spmm");
 }
