@@ -61,6 +61,7 @@ int64_t workspace_bytes(int64_t n_sparse, int64_t k, int64_t n_dense) {
                                                                        piece_bytes<T, SquareCfg>(n_sparse, k, n_dense, true)) : 0;
   if (n_dense <= narrow_columns(n_sparse, k * (int64_t)sizeof(T) / 128, sizeof(T) == 1)) return strided;
   return std::max(strided, n_dense <= SlimCfg::BJ ? piece_bytes<T, SlimCfg>(n_sparse, k, n_dense, false)
+                           : takes_small<T>(n_sparse, k, n_dense, (int64_t)1 << 40) ? piece_bytes<T, SmallCfg>(n_sparse, k, n_dense, false)
                            : takes_mid<T>(n_sparse, k, n_dense, (int64_t)1 << 40) ? piece_bytes<T, MidCfg>(n_sparse, k, n_dense, false)
                                                                                   : piece_bytes<T, TiledCfg>(n_sparse, k, n_dense, false));
 }

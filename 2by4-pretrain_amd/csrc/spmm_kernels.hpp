@@ -308,7 +308,7 @@ template <> struct mma32<i8_t> {
   }
 };
 
-template <int WAVES_J_, int TJ_, int TI_ = 4>
+template <int WAVES_J_, int TJ_, int TI_ = 4, int RING_ = 3>
 struct TileCfgT {
   static constexpr int WAVES_I = 2, WAVES_J = WAVES_J_;
   static constexpr int NW = WAVES_I * WAVES_J;
@@ -316,8 +316,9 @@ struct TileCfgT {
   static constexpr int TI = TI_, TJ = TJ_;       // 32x32 instructions per wave
   static constexpr int WI = 32 * TI, WJ = 32 * TJ;
   static constexpr int BI = WI * WAVES_I, BJ = WJ * WAVES_J;
-  static_assert((BI == 256 && (BJ == 256 || BJ == 192 || BJ == 128 || BJ == 64)) || (BJ == 192 && (BI == 192 || BI == 384)),
-                "stage buffers are sized for 256-row tiles of 256, 192, 128 or 64 columns and for 192-column tiles of 192 or 384 rows");
+  static constexpr int RING = RING_;             // stage buffers
+  static_assert((BI == 128 && BJ == 128) || (BI == 256 && (BJ == 256 || BJ == 192 || BJ == 128 || BJ == 64)) || (BJ == 192 && (BI == 192 || BI == 384)),
+                "stage buffers are sized for 256-row tiles of 256, 192, 128 or 64 columns, 192-column tiles of 192 or 384 rows and 128 x 128 ones");
   static constexpr int KB = 128;                 // bytes of dense k per row per stage
   static constexpr int STEPS = KB / 64;          // instruction steps per stage
   static constexpr int A_ROW = KB / 2;           // LDS bytes per row per stage: compressed values
@@ -369,6 +370,14 @@ static_assert(kRotateMinStages - 2 - (7 * kRotateMinStages >> 3) >= 1, "the firs
 using SlimCfg = TileCfgT<1, 2>;
 // 256 x 128 tiles, four waves: dense operands of 65 to 128 columns
 using MidCfg = TileCfgT<2, 2>;
+// 128 x 128 tiles, four waves (wave tile 64 x 64, 64 accumulators), where there is at most one for each compute unit (takes_small).  A product
+// of one round takes as long as its tile: prologue, stages one after the other, output pass.  Here that is 4.6 us and 0.21 to 0.3 a stage, against 5.6 and
+// 0.33 with 256 x 128 tiles, and with k in pieces a tile has half the partial sums to write.  What bounds it: a stage
+// moves 25 KB into LDS and 48 KB out of it to the registers for 0.12 us of matrix instructions.  Four stage buffers instead of three (a
+// stage is that much shorter, and its copies take no less time to arrive): us with 3, 4, 5 and 6 of them 3072 x 768 against
+// 952 columns 7.9, 7.6, 7.9, 8.1; 1824 x 2048 against 704 13.1, 11.8, 12.2, 12.4; 6144 x 4096 against 424 24.6, 21.5, -, 21.9.
+// (256 x 64 tiles are no faster with four.)
+using SmallCfg = TileCfgT<2, 2, 2, 4>;
 
 // ACTS: the kernel is built twice, for launches without an activation (output pass: plain or bias only) and with one
 // (bias or zeros, then ReLU, SiLU or GELU); with all five passes in one kernel the compiler no longer keeps the
@@ -402,10 +411,10 @@ spmm_pipe(const uint8_t* __restrict__ a_values, const uint8_t* __restrict__ a_me
   static_assert(MW * MWAVES == MCOPIES || C::BI != 256, "metadata copies must divide among the waves");
   static_assert(M_DWORD || C::BI == 256, "full runs are 256 rows");
   constexpr bool M_HALF_MAJOR = ES == 1;
-  // one stage buffer = [A values | B | A metadata]; three of them rotate
+  // one stage buffer = [A values | B | A metadata]; C::RING (three or four) of them rotate
   constexpr int A_STAGE = C::BI * C::A_ROW, B_STAGE = C::BJ * C::B_ROW, M_STAGE = C::BI * M_ROW;
   constexpr int B_AT = A_STAGE, M_AT = A_STAGE + B_STAGE, STAGE_BYTES = A_STAGE + B_STAGE + M_STAGE;
-  __shared__ __attribute__((aligned(1024))) uint8_t smem[3 * STAGE_BYTES];
+  __shared__ __attribute__((aligned(1024))) uint8_t smem[C::RING * STAGE_BYTES];
 
   // ---- XCD-aware work assignment.  A unit of work is (k-split, tile); units are ordered split-major
   // so that the units resident on an XCD belong to the same k range and share operand rows in L2.
@@ -712,15 +721,33 @@ spmm_pipe(const uint8_t* __restrict__ a_values, const uint8_t* __restrict__ a_me
   };
   static_assert(C::STEPS == 2, "the pipeline below is written for two instruction steps per stage");
   static_assert(!PERSIST || C_JMAJOR, "chained tiles rely on the wait inside the j-major output passes");
-  auto stage_barrier = [&](bool more) {          // B(st+1): only this wave's copies of stage st+2 may still fly
+  constexpr int LEAD = C::RING - 1;              // stages that the copies run ahead
+  static_assert(LEAD == 2 || (!PERSIST && MWAVES == C::NW), "longer rings: tiles that are not chained, the same copies in every wave");
+  auto stage_barrier = [&](bool more) {          // B(st+1): only this wave's copies of the stages from st+2 on may still fly
     if (!more) wait_copies_and_barrier<0, true>();
-    else if (MWAVES == C::NW || has_meta) wait_copies_and_barrier<NCOPY, true>();
+    else if (MWAVES == C::NW || has_meta) wait_copies_and_barrier<NCOPY * (LEAD - 1), true>();
     else wait_copies_and_barrier<NCOPY - MW, true>();
+  };
+  auto last_barrier = [&](int left) {            // the same where `left` stages follow st+1
+    if constexpr (LEAD == 2) stage_barrier(left > 0);
+    else if (left >= LEAD - 1) wait_copies_and_barrier<NCOPY * (LEAD - 1), true>();
+    else if (LEAD > 4 && left == 3) wait_copies_and_barrier<NCOPY * 3, true>();
+    else if (LEAD > 3 && left == 2) wait_copies_and_barrier<NCOPY * 2, true>();
+    else if (left == 1) wait_copies_and_barrier<NCOPY, true>();
+    else wait_copies_and_barrier<0, true>();
   };
 
   issue(smem_at);
-  if (nstages > 1) issue(smem_at + STAGE_BYTES);
-  uint32_t cur = 0, nxt = STAGE_BYTES, fre = 2 * STAGE_BYTES;   // buffers of stage st, st+1, st+2 (= st-1)
+#pragma unroll
+  for (int ahead = 1; ahead < LEAD; ahead++)
+    if (nstages > ahead) issue(smem_at + ahead * STAGE_BYTES);
+  uint32_t cur = 0, nxt = STAGE_BYTES, fre = LEAD * STAGE_BYTES;   // buffers of stage st, st+1, st+LEAD (= st-1)
+  auto turn = [&]() {                            // to the next stage's
+    const uint32_t t = cur;
+    cur = nxt;
+    nxt = LEAD == 2 ? fre : nxt == LEAD * STAGE_BYTES ? 0 : nxt + STAGE_BYTES;
+    fre = t;
+  };
   // PERSIST (nstages >= 4, no k pieces): the workgroup walks its tiles in one pipeline.  The copies of
   // the next tile's first two stages are issued during the last two stages of the current one, into
   // the two buffers those stages leave free; the output pass then stages through the third (the last
@@ -737,10 +764,10 @@ spmm_pipe(const uint8_t* __restrict__ a_values, const uint8_t* __restrict__ a_me
   // copies of stage s + 1 before it waits -- if one copy of stage s were still in flight, all of those
   // would be too, more than the NCOPY operations the wait allows.
   if (PERSIST && chained) wait_reads_and_barrier();
-  else stage_barrier(nstages > 1);
+  else last_barrier(nstages - 1);
   // stage 0: nothing to multiply yet
   {
-    const bool more = PERSIST || 2 < nstages;      // (chained tiles have four stages at least)
+    const bool more = PERSIST || LEAD < nstages;      // (chained tiles have four stages at least)
 #pragma unroll
     for (int n = 0; n < N_READS; n++) read_one(0, n, cur, 0);
     if (more) {
@@ -750,7 +777,8 @@ spmm_pipe(const uint8_t* __restrict__ a_values, const uint8_t* __restrict__ a_me
     mma_step(0, 1, more, smem_at + fre, true, cur, 1);
     if (more) next_stage();
     if (PERSIST && chained) wait_reads_and_barrier();
-    else stage_barrier(more);
+    else if (LEAD == 2) stage_barrier(more);
+    else last_barrier(nstages - 2);
   }
   // stage st: behind B(st), register set 1 holds the last step of stage st-1
   int st = 1;
@@ -760,9 +788,9 @@ spmm_pipe(const uint8_t* __restrict__ a_values, const uint8_t* __restrict__ a_me
   // tile, us on operands that change, then and now: fp16 3072 x 768 against 12288 columns 44.8 and 43.0 on 8-wave tiles, 55 and 40 on
   // 256 x 192 ones; 2048 x 512 24.3 and 22.7; 6400 x 1600 against 6000 77.4 and 76.1; 11008 x 4096 against 8192 352.5 and 350.9.)
   has_next = false;
-  for (int lim = nstages - 2 - rot;;) {
+  for (int lim = nstages - LEAD - rot;;) {
     for (; st < lim; st++) {
-      const uint32_t t = cur; cur = nxt; nxt = fre; fre = t;
+      turn();
       mma_step(1, 0, true, smem_at + fre, true, cur, 0);
       mma_step(0, 1, true, smem_at + fre, true, cur, 1);
       next_stage();
@@ -784,10 +812,11 @@ spmm_pipe(const uint8_t* __restrict__ a_values, const uint8_t* __restrict__ a_me
     lim = nstages;
   }
   for (; st < nstages; st++) {                       // the last two stages of the last tile
-    const uint32_t t = cur; cur = nxt; nxt = fre; fre = t;
+    turn();
     mma_step(1, 0, false, 0, true, cur, 0);
     mma_step(0, 1, false, 0, true, cur, 1);
-    stage_barrier(false);
+    if constexpr (LEAD == 2) stage_barrier(false);
+    else last_barrier(nstages - 2 - st);
   }
   // ---- bias: every lane fetches the bias of WI/64 of its wave's rows here, one instruction step ahead of the
   // output pass, which hands them round the wave through LDS.  (Fetched per element inside the pass -- 128 two-byte
@@ -1112,6 +1141,7 @@ spmm_reduce_splits(const float* __restrict__ partial, int splits, int tiles_i, i
 // eight pieces, 10.5 in nine and more; 480 x 2816 against 321 11.7 in five, 13.2 in nine.
 // Rounds of more than 208 blocks scatter: 4096 x 11008 against 257 to 305 columns 29.4 to 34.6 us in five pieces = 240 blocks,
 // 29.8 to 30.8 in four.
+// A stage of the smallest tiles takes longer the more units are busy (FULL_US) and the more both operands are (MEMORY_US a MB).
 // The constants are least-squares fits, per tile configuration, to 25 000 timings of 1 to 16 pieces over fp16 and fp8 weights from
 // 256 x 768 to 20480 x 11008 (6 to 512 stages) and 16 to 3072 dense columns.  The pieces chosen this way are within 1 % of
 // the best ones on average and within 4 to 6 % for 19 in 20 (a fixed 192 / tiles of them: 5, 18 and 9 % off for the three
@@ -1121,10 +1151,11 @@ spmm_reduce_splits(const float* __restrict__ partial, int splits, int tiles_i, i
 // A k-contiguous product of at most kShortStages stages is not cut: the reduction's launch and workspace are 4 us of host time,
 // which bounds such calls one after the other (linear of 96 rows with 256 x 1536: 14.6 us a call in one piece, 18.5 in
 // eight; alone 33.0 and 30.3 us, on the GPU 12.9 and 8.6).
-struct PieceCost { double call_us, stage_us, split_us, piece_us, partial_us, operand_us; };
+struct PieceCost { double call_us, stage_us, split_us, piece_us, partial_us, operand_us, full_us = 0.0, memory_us = 0.0; };
 template <typename C>
 constexpr PieceCost piece_cost(bool k_strided) {
-  return std::is_same<C, SlimCfg>::value ? PieceCost{5.1, 0.37, 1.8, 0.0, 0.48, 0.113}
+  return std::is_same<C, SmallCfg>::value ? PieceCost{4.63, 0.212, 1.86, 0.0, 0.545, 0.0, 0.025, 0.0013}
+         : std::is_same<C, SlimCfg>::value ? PieceCost{5.1, 0.37, 1.8, 0.0, 0.48, 0.113}
          : std::is_same<C, MidCfg>::value ? PieceCost{5.6, 0.33, 2.1, 0.1, 0.45, 0.0}
          : std::is_same<C, SquareCfg>::value ? PieceCost{7.3, 0.40, 1.15, 0.0, 0.40, 0.0}
          : k_strided ? PieceCost{7.1, 0.55, 1.15, 0.0, 0.42, 0.0} : PieceCost{6.9, 0.50, 3.3, 0.0, 0.385, 0.0};
@@ -1138,8 +1169,10 @@ Pieces choose_pieces(int64_t n_sparse, int64_t k, int64_t n_dense, int64_t works
   const int64_t stages = k * (int64_t)sizeof(T) / C::KB;
   const double operand_us = (double)(n_sparse * k * (int64_t)sizeof(T)) * (9.0 / 16.0) * 1e-6 * cost.operand_us;
   const double partial_us = (double)(tiles_i * C::BI * ((n_dense + 31) / 32 * 32)) * 4e-6 * cost.partial_us;     // of one piece
+  const double memory_us = ((double)(n_sparse * k) * (9.0 / 16.0) + (double)(n_dense * k)) * (double)sizeof(T) * 1e-6 * cost.memory_us;
   auto us = [&](int64_t p) {
-    const double one = cost.call_us + std::max((double)((stages + p - 1) / p) * cost.stage_us, operand_us);
+    const double stage_us = cost.stage_us + (double)(p * tiles) / 256.0 * cost.full_us + memory_us;
+    const double one = cost.call_us + std::max((double)((stages + p - 1) / p) * stage_us, operand_us);
     if (p == 1) return one;
     return (one + cost.split_us + (double)p * (cost.piece_us + partial_us) + (p > 8 ? 0.5 : 0.0)) * (p * tiles > 208 ? 1.02 : 1.0);
   };
@@ -1161,6 +1194,21 @@ bool takes_mid(int64_t n_sparse, int64_t k, int64_t n_dense, int64_t workspace_b
   if (((n_sparse + MidCfg::BI - 1) / MidCfg::BI) * ((n_dense + MidCfg::BJ - 1) / MidCfg::BJ) > 256) return false;
   return n_dense < TiledCfg::BJ || choose_pieces<T, TiledCfg>(n_sparse, k, n_dense, workspace_bytes, false).us >=
                                        0.95 * choose_pieces<T, MidCfg>(n_sparse, k, n_dense, workspace_bytes, false).us;
+}
+
+// More than 64 columns (k-contiguous) take 128 x 128 tiles where one round of the compute units holds them and the estimate for them is below that of
+// the tiles above.  Of 220 products of 256 to 12288 rows, 2 to 320 stages and 72 to 4008 columns (fp16 and e4m3) 200 take them, 15 % less time
+// on average over all; the choice is 0.5 % off the better one on average, 9 % at worst but for one product.  us, then and now: fp16 768 x 768 against
+// 160 columns 8.6 and 6.8, 3072 x 768 against 952 9.2 and 7.6, 1600 x 1600 against 1792 13.4 and 10.8, 4096 x 4096 against 128 16.0 and
+// 14.4, against 512 23.1 and 20.7, 6144 x 4096 against 424 28.9 and 21.5; e4m3 8192 x 8192 against 480 41.6 and 28.2.  The other way round, where
+// the operands no longer fit the caches: 5824 x 10176 against 328 47 and 63, 2048 x 20480 against 760 57 and 81.  More than one round:
+// 5120 x 1280 against 840 (280 tiles) 13.1 and 16.3 with two tiles to a unit.
+template <typename T>
+bool takes_small(int64_t n_sparse, int64_t k, int64_t n_dense, int64_t workspace_bytes) {
+  if (n_dense <= SlimCfg::BJ || ((n_sparse + SmallCfg::BI - 1) / SmallCfg::BI) * ((n_dense + SmallCfg::BJ - 1) / SmallCfg::BJ) > 256) return false;
+  const double others = takes_mid<T>(n_sparse, k, n_dense, workspace_bytes) ? choose_pieces<T, MidCfg>(n_sparse, k, n_dense, workspace_bytes, false).us
+                                                                           : choose_pieces<T, TiledCfg>(n_sparse, k, n_dense, workspace_bytes, false).us;
+  return choose_pieces<T, SmallCfg>(n_sparse, k, n_dense, workspace_bytes, false).us < others;
 }
 
 // Rounds of the compute units that so many tiles take (each XCD has an eighth of both).
@@ -1810,8 +1858,9 @@ int dispatch_out(int out_dtype, const void* av, const void* am, int a_layout, in
   // the tiled kernel reads a k-strided dense operand through transposing LDS reads (16-bit types only)
   // (also for a narrow dense operand: with its k pieces the tiled kernel beats the general one from 8 columns on)
   const bool tiled = panel && (b_layout == TF24_ROW_MAJOR || sizeof(T) == 2) && n_sparse >= 64;
-  // up to 64 dense columns: the tiled kernel on 256 x 64 tiles; more: 256 x 128 or 256 x 256 tiles (takes_mid)
+  // up to 64 dense columns: the tiled kernel on 256 x 64 tiles; more: 128 x 128 (takes_small), 256 x 128 or 256 x 256 tiles (takes_mid)
   const bool slim = tiled && b_layout == TF24_ROW_MAJOR && n_dense <= SlimCfg::BJ;
+  const bool small = tiled && b_layout == TF24_ROW_MAJOR && takes_small<T>(n_sparse, k, n_dense, workspace ? workspace_bytes : 0);
   const bool mid = tiled && b_layout == TF24_ROW_MAJOR && takes_mid<T>(n_sparse, k, n_dense, workspace ? workspace_bytes : 0);
   // few dense columns: one pass over the compressed operand (narrow_columns), also up to 16 when the tiled kernel cannot cut k
   // into pieces (no workspace), which it needs to fill the chip
@@ -1820,6 +1869,7 @@ int dispatch_out(int out_dtype, const void* av, const void* am, int a_layout, in
   if constexpr (std::is_same<T, i8_t>::value) {        // integer product: int32 accumulators, results and bias
     if (narrow) return launch_narrow<T, int32_t>(av, am, n_sparse, k, b, ldb, n_dense, c, c_layout, ldc, bias, scale, act, s);
     if (slim) return launch_tiled<T, int32_t, SlimCfg>(av, am, n_sparse, k, b, b_layout, ldb, n_dense, c, c_layout, ldc, bias, scale, act, workspace, workspace_bytes, s);
+    if (small) return launch_tiled<T, int32_t, SmallCfg>(av, am, n_sparse, k, b, b_layout, ldb, n_dense, c, c_layout, ldc, bias, scale, act, workspace, workspace_bytes, s);
     if (mid) return launch_tiled<T, int32_t, MidCfg>(av, am, n_sparse, k, b, b_layout, ldb, n_dense, c, c_layout, ldc, bias, scale, act, workspace, workspace_bytes, s);
     if (tiled) return launch_tiled<T, int32_t, TiledCfg>(av, am, n_sparse, k, b, b_layout, ldb, n_dense, c, c_layout, ldc, bias, scale, act, workspace, workspace_bytes, s);
     return launch_general<T, int32_t>(av, am, a_layout, n_sparse, k, b, b_layout, ldb, n_dense, c, c_layout, ldc, bias, scale, act, s);
@@ -1836,6 +1886,13 @@ int dispatch_out(int out_dtype, const void* av, const void* am, int a_layout, in
       case TF24_F16: return launch_tiled<T, f16_t, SlimCfg>(av, am, n_sparse, k, b, b_layout, ldb, n_dense, c, c_layout, ldc, bias, scale, act, workspace, workspace_bytes, s);
       case TF24_BF16: return launch_tiled<T, bf16_t, SlimCfg>(av, am, n_sparse, k, b, b_layout, ldb, n_dense, c, c_layout, ldc, bias, scale, act, workspace, workspace_bytes, s);
       case TF24_F32: return launch_tiled<T, float, SlimCfg>(av, am, n_sparse, k, b, b_layout, ldb, n_dense, c, c_layout, ldc, bias, scale, act, workspace, workspace_bytes, s);
+    }
+  }
+  if (small) {
+    switch (out_dtype) {
+      case TF24_F16: return launch_tiled<T, f16_t, SmallCfg>(av, am, n_sparse, k, b, b_layout, ldb, n_dense, c, c_layout, ldc, bias, scale, act, workspace, workspace_bytes, s);
+      case TF24_BF16: return launch_tiled<T, bf16_t, SmallCfg>(av, am, n_sparse, k, b, b_layout, ldb, n_dense, c, c_layout, ldc, bias, scale, act, workspace, workspace_bytes, s);
+      case TF24_F32: return launch_tiled<T, float, SmallCfg>(av, am, n_sparse, k, b, b_layout, ldb, n_dense, c, c_layout, ldc, bias, scale, act, workspace, workspace_bytes, s);
     }
   }
   if (mid) {

@@ -1272,6 +1272,39 @@ def test_one_to_thirty_two_rows(cuda, dtype, n, panels):
         assert y[:rows].equal(x.float() @ dense.t()) and bool((y[rows:] == 77).all()), rows
 
 
+SMALL_TILES = [(64, 1, 65), (96, 2, 127), (128, 3, 128), (160, 4, 129), (288, 5, 200), (32 * 35, 6, 255), (992, 7, 1000), (640, 8, 4001),
+               (1024, 12, 300), (4096, 28, 72), (2080, 27, 1900),                                # one piece of k: around the four stage buffers, and long
+               (96, 29, 66), (1184, 30, 136), (672, 64, 520), (160, 77, 1345), (1600, 100, 250)]    # pieces
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float8_e4m3fn, torch.int8])
+@pytest.mark.parametrize("n,stages,rows", SMALL_TILES)
+def test_tiles_of_128_square(cuda, dtype, n, stages, rows):
+    """Rows and columns that do not fill their last tile, one stage and more, whole and in pieces, either order of the results, with bias
+    and without: exact on small integers, the row behind the last stays as it was."""
+    import sparse
+    from sparse import _native as N
+    k = stages * 128 // torch.empty(0, dtype=dtype).element_size()
+    code, wide = N.operand_code(dtype), torch.int32 if dtype == torch.int8 else torch.float32
+    g = torch.Generator(device=cuda).manual_seed(n + stages + rows)
+    s = sparse.to_sparse_semi_structured(torch.randint(-2, 3, (n, k), device=cuda, generator=g).to(torch.int8 if dtype == torch.int8 else torch.float32), dtype=dtype)
+    x = torch.randint(-2, 3, (rows, k), device=cuda, generator=g).to(dtype)
+    want = x.float() @ s.to_dense().float().t()                   # (whole numbers below 2**24)
+    ws = torch.empty(max(N.lib().tf24_spmm_workspace_bytes(code, n, k, rows), 16), dtype=torch.uint8, device=cuda)
+    for out_dtype in (wide,) if dtype == torch.int8 else (wide, torch.float16):
+        bias = torch.randint(-4, 5, (n,), device=cuda, generator=g).to(out_dtype)
+        for b in (None, bias):
+            y = torch.full((rows + 1, n), 77, dtype=out_dtype, device=cuda)
+            N.check(N.lib().tf24_linear(s._store_values.data_ptr(), s._store_meta.data_ptr(), N.COMPRESSED_PANEL, code, n, k, x.data_ptr(), k, rows, y.data_ptr(),
+                                        N.operand_code(out_dtype), n, None if b is None else b.data_ptr(), 1.0, N.ACT_NONE, ws.data_ptr(), ws.numel(), N.stream_ptr()))
+            assert y[:rows].equal((want + (0 if b is None else b.float())).to(out_dtype)) and bool((y[rows:] == 77).all()), (out_dtype, b is None)
+    if rows % (8 if dtype == torch.float16 else 16) == 0:
+        yt = torch.full((n, rows), 77, dtype=wide, device=cuda)
+        N.check(N.lib().tf24_spmm(s._store_values.data_ptr(), s._store_meta.data_ptr(), N.COMPRESSED_PANEL, code, n, k, x.data_ptr(), N.ROW_MAJOR, k, rows,
+                                  yt.data_ptr(), N.operand_code(wide), N.ROW_MAJOR, rows, None, 1.0, N.ACT_NONE, ws.data_ptr(), ws.numel(), N.stream_ptr()))
+        assert yt.equal(want.t().to(wide))
+
+
 @pytest.mark.parametrize("dtype,special", [(F16, float("inf")), (BF16, float("-inf")), (E5M2, float("inf")), (E4M3, float("nan"))])
 @pytest.mark.parametrize("n,panels", [(768, 12), (512, 11), (256, 5), (4096, 22), (1024, 37), (8192, 17), (8224, 3), (10240, 43)])
 def test_few_dense_columns_special_values(cuda, dtype, special, n, panels):

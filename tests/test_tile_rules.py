@@ -6,7 +6,7 @@ import subprocess
 
 import pytest
 
-from test_gpu_parity import NOT_TALL, SHORT, SQUARE, SQUARE_STRIDED, STAGE_ORDER, TALL
+from test_gpu_parity import NOT_TALL, SHORT, SMALL_TILES, SQUARE, SQUARE_STRIDED, STAGE_ORDER, TALL
 from test_gpu_training import MANY_LONG
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -42,6 +42,11 @@ extern "C" int tiles_of_16_bits(int64_t n_sparse, int64_t n_dense, int stages, i
   const tf24::TileRows rows = tf24::full_rounds(n_sparse, n_dense, stages, cu_slots);
   return (int)tf24::choose_tiles(n_sparse, n_dense, stages, rows, true, cu_slots, true) + (rows.tail_rows ? 100 : 0);
 }
+extern "C" int small(int64_t n_sparse, int64_t n_dense, int stages, int bytes) {
+  const int64_t ws = (int64_t)1 << 40;
+  if (bytes == 1) return tf24::takes_small<tf24::e4m3_t>(n_sparse, (int64_t)stages * 128, n_dense, ws) * tf24::choose_pieces<tf24::e4m3_t, tf24::SmallCfg>(n_sparse, (int64_t)stages * 128, n_dense, ws, false).count;
+  return tf24::takes_small<tf24::f16_t>(n_sparse, (int64_t)stages * 64, n_dense, ws) * tf24::choose_pieces<tf24::f16_t, tf24::SmallCfg>(n_sparse, (int64_t)stages * 64, n_dense, ws, false).count;
+}
 extern "C" int rotate_from() { return tf24::kRotateMinStages; }
 """)
     subprocess.run([build.HIPCC, *build.FLAGS, "--offload-host-only", "-shared", str(src), "-o", str(lib)], check=True, capture_output=True)
@@ -51,7 +56,24 @@ extern "C" int rotate_from() { return tf24::kRotateMinStages; }
     handle.tiles_of_16_bits.argtypes = [ctypes.c_int64, ctypes.c_int64, ctypes.c_int, ctypes.c_int]
     handle.strided.argtypes = [ctypes.c_int64, ctypes.c_int64, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int]
     handle.strided_pieces.argtypes = [ctypes.c_int64, ctypes.c_int64, ctypes.c_int]
+    handle.small.argtypes = [ctypes.c_int64, ctypes.c_int64, ctypes.c_int, ctypes.c_int]
     return handle
+
+
+@pytest.mark.parametrize("n,stages,columns,small", [
+    # measured apart (us on the other tiles, on 128 x 128 ones)
+    (768, 12, 160, 1), (3072, 12, 952, 1), (4096, 64, 128, 1), (6144, 64, 424, 1),              # 8.6 6.8, 9.2 7.6, 16.0 14.4, 28.9 21.5
+    (5824, 159, 328, 0), (9024, 163, 272, 0), (2048, 320, 760, 0),                              # 47 63, 60 72, 57 81
+    (5120, 20, 840, 0), (768, 12, 64, 0)])                                                      # two rounds of them; the narrowest tiles
+def test_small_tiles_where_they_are_the_faster_ones(rules, n, stages, columns, small):
+    assert bool(rules.small(n, columns, stages, 2)) == small
+
+
+@pytest.mark.parametrize("n,stages,columns", SMALL_TILES)
+def test_products_tested_on_the_gpu_take_small_tiles(rules, n, stages, columns):
+    for size in (1, 2):
+        assert bool(rules.small(n, columns, stages, size))
+        assert stages <= 28 or rules.small(n, columns, stages, size) > 1
 
 
 @pytest.mark.parametrize("n,stages,columns,square", [
