@@ -317,8 +317,8 @@ struct TileCfgT {
   static constexpr int WI = 32 * TI, WJ = 32 * TJ;
   static constexpr int BI = WI * WAVES_I, BJ = WJ * WAVES_J;
   static constexpr int RING = RING_;             // stage buffers
-  static_assert((BI == 128 && BJ == 128) || (BI == 256 && (BJ == 256 || BJ == 192 || BJ == 128 || BJ == 64)) || (BJ == 192 && (BI == 192 || BI == 384)),
-                "stage buffers are sized for 256-row tiles of 256, 192, 128 or 64 columns, 192-column tiles of 192 or 384 rows and 128 x 128 ones");
+  static_assert(((BI == 128 || BI == 192) && BJ == 128) || (BI == 256 && (BJ == 256 || BJ == 192 || BJ == 128 || BJ == 64)) || (BJ == 192 && (BI == 192 || BI == 384)),
+                "stage buffers are sized for 256-row tiles of 256, 192, 128 or 64 columns, 192-column tiles of 192 or 384 rows and 128-column tiles of 128 or 192 rows");
   static constexpr int KB = 128;                 // bytes of dense k per row per stage
   static constexpr int STEPS = KB / 64;          // instruction steps per stage
   static constexpr int A_ROW = KB / 2;           // LDS bytes per row per stage: compressed values
@@ -378,6 +378,9 @@ using MidCfg = TileCfgT<2, 2>;
 // 952 columns 7.9, 7.6, 7.9, 8.1; 1824 x 2048 against 704 13.1, 11.8, 12.2, 12.4; 6144 x 4096 against 424 24.6, 21.5, -, 21.9.
 // (256 x 64 tiles are no faster with four.)
 using SmallCfg = TileCfgT<2, 2, 2, 4>;
+// 192 x 128 tiles, four waves (wave tile 96 x 64), four stage buffers: products that these cover in one round of the compute units and 128 x 128
+// tiles do not (takes_lower)
+using LowerCfg = TileCfgT<2, 2, 3, 4>;
 
 // ACTS: the kernel is built twice, for launches without an activation (output pass: plain or bias only) and with one
 // (bias or zeros, then ReLU, SiLU or GELU); with all five passes in one kernel the compiler no longer keeps the
@@ -1211,6 +1214,22 @@ bool takes_small(int64_t n_sparse, int64_t k, int64_t n_dense, int64_t workspace
   return choose_pieces<T, SmallCfg>(n_sparse, k, n_dense, workspace_bytes, false).us < others;
 }
 
+// Between the two: a product whose 128 x 128 tiles are more than one round of the compute units and whose 192 x 128 ones are not takes the latter instead of
+// 256 x 128 ones.  It is in one piece (more than half a round of any of these tiles), so again its time is that of a tile, with 3/4 of the stages' work.
+// From 20 stages on (below, the longer ring and the third of the rounds that the wider tiles leave empty weigh as much: 60 products, us on 256 x 128
+// and on these tiles 2304 x 768 against 2368 columns 10.6 and 11.3, 768 x 768 against 6048 9.6 and 9.3) up to 176 (operands that no longer
+// fit the caches: 172 stages 4096 x 11008 against 936 70.2 and 66.0, 189 5952 x 12096 against 784 95 and 100).  Between them 37 of 39 products are
+// faster and two within 2 %, 9 % less time on average: 3840 x 1280 against 1040 13.6 and 12.4, 6144 x 4096 against 736 34.1 and 30.1, 11008 x 4096 against
+// 336 40.7 and 32.6, 2048 x 8192 against 2928 79.7 and 65.7; e4m3 12288 x 4096 against 320 17.7 and 16.3.
+constexpr int64_t kLowerMinStages = 20, kLowerMaxStages = 176;
+template <typename T>
+bool takes_lower(int64_t n_sparse, int64_t k, int64_t n_dense, int64_t workspace_bytes) {
+  const int64_t columns = (n_dense + LowerCfg::BJ - 1) / LowerCfg::BJ;
+  const int64_t stages = k * (int64_t)sizeof(T) / LowerCfg::KB;
+  return stages >= kLowerMinStages && stages <= kLowerMaxStages && n_dense > LowerCfg::BJ && ((n_sparse + SmallCfg::BI - 1) / SmallCfg::BI) * columns > 256 &&
+         ((n_sparse + LowerCfg::BI - 1) / LowerCfg::BI) * columns <= 256 && takes_mid<T>(n_sparse, k, n_dense, workspace_bytes);
+}
+
 // Rounds of the compute units that so many tiles take (each XCD has an eighth of both).
 inline int64_t tile_rounds(int64_t tiles, int64_t cu_slots) { return ((tiles + 7) / 8 + cu_slots - 1) / cu_slots; }
 
@@ -1353,7 +1372,7 @@ int launch_tiled(const void* av, const void* am, int64_t n_sparse, int64_t k, co
   }
   int tiles_i = (int)((n_sparse + C::BI - 1) / C::BI);
   const int tiles_j = (int)((n_dense + C::BJ - 1) / C::BJ);
-  const int splits = workspace ? choose_pieces<T, C>(n_sparse, k, n_dense, workspace_bytes, b_layout == TF24_COL_MAJOR).count : 1;
+  const int splits = workspace && !std::is_same<C, LowerCfg>::value ? choose_pieces<T, C>(n_sparse, k, n_dense, workspace_bytes, b_layout == TF24_COL_MAJOR).count : 1;
   const int stages = (int)(k * (int64_t)sizeof(T) / C::KB);
   int tail_rows = 0;
   if constexpr (std::is_same<C, TiledCfg>::value) {
@@ -1858,9 +1877,10 @@ int dispatch_out(int out_dtype, const void* av, const void* am, int a_layout, in
   // the tiled kernel reads a k-strided dense operand through transposing LDS reads (16-bit types only)
   // (also for a narrow dense operand: with its k pieces the tiled kernel beats the general one from 8 columns on)
   const bool tiled = panel && (b_layout == TF24_ROW_MAJOR || sizeof(T) == 2) && n_sparse >= 64;
-  // up to 64 dense columns: the tiled kernel on 256 x 64 tiles; more: 128 x 128 (takes_small), 256 x 128 or 256 x 256 tiles (takes_mid)
+  // up to 64 dense columns: the tiled kernel on 256 x 64 tiles; more: 128 x 128 (takes_small), 192 x 128 (takes_lower), 256 x 128 or 256 x 256 tiles (takes_mid)
   const bool slim = tiled && b_layout == TF24_ROW_MAJOR && n_dense <= SlimCfg::BJ;
   const bool small = tiled && b_layout == TF24_ROW_MAJOR && takes_small<T>(n_sparse, k, n_dense, workspace ? workspace_bytes : 0);
+  const bool lower = tiled && b_layout == TF24_ROW_MAJOR && takes_lower<T>(n_sparse, k, n_dense, workspace ? workspace_bytes : 0);
   const bool mid = tiled && b_layout == TF24_ROW_MAJOR && takes_mid<T>(n_sparse, k, n_dense, workspace ? workspace_bytes : 0);
   // few dense columns: one pass over the compressed operand (narrow_columns), also up to 16 when the tiled kernel cannot cut k
   // into pieces (no workspace), which it needs to fill the chip
@@ -1870,6 +1890,7 @@ int dispatch_out(int out_dtype, const void* av, const void* am, int a_layout, in
     if (narrow) return launch_narrow<T, int32_t>(av, am, n_sparse, k, b, ldb, n_dense, c, c_layout, ldc, bias, scale, act, s);
     if (slim) return launch_tiled<T, int32_t, SlimCfg>(av, am, n_sparse, k, b, b_layout, ldb, n_dense, c, c_layout, ldc, bias, scale, act, workspace, workspace_bytes, s);
     if (small) return launch_tiled<T, int32_t, SmallCfg>(av, am, n_sparse, k, b, b_layout, ldb, n_dense, c, c_layout, ldc, bias, scale, act, workspace, workspace_bytes, s);
+    if (lower) return launch_tiled<T, int32_t, LowerCfg>(av, am, n_sparse, k, b, b_layout, ldb, n_dense, c, c_layout, ldc, bias, scale, act, workspace, workspace_bytes, s);
     if (mid) return launch_tiled<T, int32_t, MidCfg>(av, am, n_sparse, k, b, b_layout, ldb, n_dense, c, c_layout, ldc, bias, scale, act, workspace, workspace_bytes, s);
     if (tiled) return launch_tiled<T, int32_t, TiledCfg>(av, am, n_sparse, k, b, b_layout, ldb, n_dense, c, c_layout, ldc, bias, scale, act, workspace, workspace_bytes, s);
     return launch_general<T, int32_t>(av, am, a_layout, n_sparse, k, b, b_layout, ldb, n_dense, c, c_layout, ldc, bias, scale, act, s);
@@ -1893,6 +1914,13 @@ int dispatch_out(int out_dtype, const void* av, const void* am, int a_layout, in
       case TF24_F16: return launch_tiled<T, f16_t, SmallCfg>(av, am, n_sparse, k, b, b_layout, ldb, n_dense, c, c_layout, ldc, bias, scale, act, workspace, workspace_bytes, s);
       case TF24_BF16: return launch_tiled<T, bf16_t, SmallCfg>(av, am, n_sparse, k, b, b_layout, ldb, n_dense, c, c_layout, ldc, bias, scale, act, workspace, workspace_bytes, s);
       case TF24_F32: return launch_tiled<T, float, SmallCfg>(av, am, n_sparse, k, b, b_layout, ldb, n_dense, c, c_layout, ldc, bias, scale, act, workspace, workspace_bytes, s);
+    }
+  }
+  if (lower) {
+    switch (out_dtype) {
+      case TF24_F16: return launch_tiled<T, f16_t, LowerCfg>(av, am, n_sparse, k, b, b_layout, ldb, n_dense, c, c_layout, ldc, bias, scale, act, workspace, workspace_bytes, s);
+      case TF24_BF16: return launch_tiled<T, bf16_t, LowerCfg>(av, am, n_sparse, k, b, b_layout, ldb, n_dense, c, c_layout, ldc, bias, scale, act, workspace, workspace_bytes, s);
+      case TF24_F32: return launch_tiled<T, float, LowerCfg>(av, am, n_sparse, k, b, b_layout, ldb, n_dense, c, c_layout, ldc, bias, scale, act, workspace, workspace_bytes, s);
     }
   }
   if (mid) {

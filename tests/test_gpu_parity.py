@@ -1275,11 +1275,12 @@ def test_one_to_thirty_two_rows(cuda, dtype, n, panels):
 SMALL_TILES = [(64, 1, 65), (96, 2, 127), (128, 3, 128), (160, 4, 129), (288, 5, 200), (32 * 35, 6, 255), (992, 7, 1000), (640, 8, 4001),
                (1024, 12, 300), (4096, 28, 72), (2080, 27, 1900),                                # one piece of k: around the four stage buffers, and long
                (96, 29, 66), (1184, 30, 136), (672, 64, 520), (160, 77, 1345), (1600, 100, 250)]    # pieces
+LOWER_TILES = [(320, 20, 11001), (960, 21, 4208), (992, 23, 4297), (4128, 22, 1001), (11008, 20, 304), (1184, 40, 3584), (2048, 176, 2176)]    # 192 x 128
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.float8_e4m3fn, torch.int8])
-@pytest.mark.parametrize("n,stages,rows", SMALL_TILES)
-def test_tiles_of_128_square(cuda, dtype, n, stages, rows):
+@pytest.mark.parametrize("n,stages,rows", SMALL_TILES + LOWER_TILES)
+def test_tiles_of_128_columns(cuda, dtype, n, stages, rows):
     """Rows and columns that do not fill their last tile, one stage and more, whole and in pieces, either order of the results, with bias
     and without: exact on small integers, the row behind the last stays as it was."""
     import sparse

@@ -6,7 +6,7 @@ import subprocess
 
 import pytest
 
-from test_gpu_parity import NOT_TALL, SHORT, SMALL_TILES, SQUARE, SQUARE_STRIDED, STAGE_ORDER, TALL
+from test_gpu_parity import LOWER_TILES, NOT_TALL, SHORT, SMALL_TILES, SQUARE, SQUARE_STRIDED, STAGE_ORDER, TALL
 from test_gpu_training import MANY_LONG
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -47,6 +47,10 @@ extern "C" int small(int64_t n_sparse, int64_t n_dense, int stages, int bytes) {
   if (bytes == 1) return tf24::takes_small<tf24::e4m3_t>(n_sparse, (int64_t)stages * 128, n_dense, ws) * tf24::choose_pieces<tf24::e4m3_t, tf24::SmallCfg>(n_sparse, (int64_t)stages * 128, n_dense, ws, false).count;
   return tf24::takes_small<tf24::f16_t>(n_sparse, (int64_t)stages * 64, n_dense, ws) * tf24::choose_pieces<tf24::f16_t, tf24::SmallCfg>(n_sparse, (int64_t)stages * 64, n_dense, ws, false).count;
 }
+extern "C" int lower(int64_t n_sparse, int64_t n_dense, int stages, int bytes) {
+  return bytes == 1 ? tf24::takes_lower<tf24::e4m3_t>(n_sparse, (int64_t)stages * 128, n_dense, (int64_t)1 << 40)
+                    : tf24::takes_lower<tf24::f16_t>(n_sparse, (int64_t)stages * 64, n_dense, (int64_t)1 << 40);
+}
 extern "C" int rotate_from() { return tf24::kRotateMinStages; }
 """)
     subprocess.run([build.HIPCC, *build.FLAGS, "--offload-host-only", "-shared", str(src), "-o", str(lib)], check=True, capture_output=True)
@@ -56,7 +60,7 @@ extern "C" int rotate_from() { return tf24::kRotateMinStages; }
     handle.tiles_of_16_bits.argtypes = [ctypes.c_int64, ctypes.c_int64, ctypes.c_int, ctypes.c_int]
     handle.strided.argtypes = [ctypes.c_int64, ctypes.c_int64, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int]
     handle.strided_pieces.argtypes = [ctypes.c_int64, ctypes.c_int64, ctypes.c_int]
-    handle.small.argtypes = [ctypes.c_int64, ctypes.c_int64, ctypes.c_int, ctypes.c_int]
+    handle.small.argtypes = handle.lower.argtypes = [ctypes.c_int64, ctypes.c_int64, ctypes.c_int, ctypes.c_int]
     return handle
 
 
@@ -67,6 +71,16 @@ extern "C" int rotate_from() { return tf24::kRotateMinStages; }
     (5120, 20, 840, 0), (768, 12, 64, 0)])                                                      # two rounds of them; the narrowest tiles
 def test_small_tiles_where_they_are_the_faster_ones(rules, n, stages, columns, small):
     assert bool(rules.small(n, columns, stages, 2)) == small
+
+
+@pytest.mark.parametrize("n,stages,columns,lower", [
+    # measured apart (us on 256 x 128 tiles, on 192 x 128 ones)
+    (3840, 20, 1040, 1), (6144, 64, 736, 1), (11008, 64, 336, 1), (2048, 128, 2928, 1),         # 13.6 12.4, 34.1 30.1, 40.7 32.6, 79.7 65.7
+    (2304, 12, 2368, 0), (5952, 189, 784, 0), (4096, 64, 512, 0), (4096, 64, 1536, 0)]          # 10.6 11.3, 95 100; 128 x 128; two rounds
+    + [(*case, 1) for case in LOWER_TILES])
+def test_lower_tiles_where_they_are_the_faster_ones(rules, n, stages, columns, lower):
+    for size in (1, 2):
+        assert rules.lower(n, columns, stages, size) == lower and not (lower and rules.small(n, columns, stages, size))
 
 
 @pytest.mark.parametrize("n,stages,columns", SMALL_TILES)
