@@ -60,7 +60,9 @@ int64_t workspace_bytes(int64_t n_sparse, int64_t k, int64_t n_dense) {
   const int64_t strided = sizeof(T) == 2 && n_dense % 8 == 0 ? std::max(piece_bytes<T, TiledCfg>(n_sparse, k, n_dense, true),
                                                                        piece_bytes<T, SquareCfg>(n_sparse, k, n_dense, true)) : 0;
   if (n_dense <= narrow_columns(n_sparse, k * (int64_t)sizeof(T) / 128, sizeof(T) == 1)) return strided;
-  return std::max(strided, n_dense <= SlimCfg::BJ ? piece_bytes<T, SlimCfg>(n_sparse, k, n_dense, false)
+  const bool tall_slim = n_dense <= SlimCfg::BJ && takes_tall_slim(n_sparse, k * (int64_t)sizeof(T) / SlimCfg::KB);
+  return std::max(strided, tall_slim ? piece_bytes<T, TallSlimCfg>(n_sparse, k, n_dense, false)
+                           : n_dense <= SlimCfg::BJ ? piece_bytes<T, SlimCfg>(n_sparse, k, n_dense, false)
                            : takes_small<T>(n_sparse, k, n_dense, (int64_t)1 << 40) ? piece_bytes<T, SmallCfg>(n_sparse, k, n_dense, false)
                            : takes_mid<T>(n_sparse, k, n_dense, (int64_t)1 << 40) ? piece_bytes<T, MidCfg>(n_sparse, k, n_dense, false)
                                                                                   : piece_bytes<T, TiledCfg>(n_sparse, k, n_dense, false));

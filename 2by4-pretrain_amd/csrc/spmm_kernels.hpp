@@ -317,8 +317,8 @@ struct TileCfgT {
   static constexpr int WI = 32 * TI, WJ = 32 * TJ;
   static constexpr int BI = WI * WAVES_I, BJ = WJ * WAVES_J;
   static constexpr int RING = RING_;             // stage buffers
-  static_assert(((BI == 128 || BI == 192) && BJ == 128) || (BI == 256 && (BJ == 256 || BJ == 192 || BJ == 128 || BJ == 64)) || (BJ == 192 && (BI == 192 || BI == 384)),
-                "stage buffers are sized for 256-row tiles of 256, 192, 128 or 64 columns, 192-column tiles of 192 or 384 rows and 128-column tiles of 128 or 192 rows");
+  static_assert((BI == 128 && BJ == 64) || ((BI == 128 || BI == 192) && BJ == 128) || (BI == 256 && (BJ == 256 || BJ == 192 || BJ == 128 || BJ == 64)) || (BJ == 192 && (BI == 192 || BI == 384)),
+                "stage buffers are sized for 256-row tiles of 256, 192, 128 or 64 columns, 192-column tiles of 192 or 384 rows, 128-column tiles of 128 or 192 and 64-column tiles of 128");
   static constexpr int KB = 128;                 // bytes of dense k per row per stage
   static constexpr int STEPS = KB / 64;          // instruction steps per stage
   static constexpr int A_ROW = KB / 2;           // LDS bytes per row per stage: compressed values
@@ -365,9 +365,17 @@ using TallCfg = TileCfgT<2, 3, 6>;
 constexpr int kWave4MinStages = 32;
 constexpr int kRotateMinStages = 56;
 static_assert(kRotateMinStages - 2 - (7 * kRotateMinStages >> 3) >= 1, "the first three stages of a tile are copied before the order wraps");
-// 256 x 64 tiles, two waves: for dense operands of at most 64 columns (a few dozen tokens), where a
-// 256-wide tile would copy and multiply clamped columns.  26 KB per stage, two blocks per CU.
-using SlimCfg = TileCfgT<1, 2>;
+// 128 x 64 tiles, four waves (wave tile 64 x 32, 32 accumulators), four stage buffers: for dense operands of at most 64 columns (a few dozen
+// tokens), where a wider tile would copy and multiply clamped columns.  17 KB per stage, two blocks per CU.  These products are short: the pass
+// over the compressed operand takes a few us, and the rest is the launch, the first stage's way from memory, one stage after the other and the sum of the
+// pieces.  us on 256 x 64 tiles of two waves with three buffers, on these of two waves, of four, each with its best number of pieces:
+// fp16 4096 x 4096 against 64 columns 13.5, 12.1, 11.1; 8192 x 8192 against 64 23.1, 21.1, 20.8; 4096 x 11008 against 40 18.9, 16.2, 15.7;
+// 5120 x 1280 against 64 11.9, 8.9, 7.2; e4m3 4096 x 4096 against 64 11.5, 10.4, 9.6.  Of 100 products of 128 to 20480 rows, 2 to
+// 512 stages and 8 to 64 columns 97 are faster, 17 % on average over all; the others 3840 x 1280 against 8 columns 4.8 and 5.2, 11072 x 12352 against
+// 56 (87 rows of tiles: two pieces fill the units less well than five of 44 did) 38.6 and 40.2.
+using SlimCfg = TileCfgT<2, 1, 2, 4>;
+// 256 x 64 tiles, two waves, three stage buffers: the same for tall weights (takes_tall_slim)
+using TallSlimCfg = TileCfgT<1, 2>;
 // 256 x 128 tiles, four waves: dense operands of 65 to 128 columns
 using MidCfg = TileCfgT<2, 2>;
 // 128 x 128 tiles, four waves (wave tile 64 x 64, 64 accumulators), where there is at most one for each compute unit (takes_small).  A product
@@ -376,7 +384,6 @@ using MidCfg = TileCfgT<2, 2>;
 // moves 25 KB into LDS and 48 KB out of it to the registers for 0.12 us of matrix instructions.  Four stage buffers instead of three (a
 // stage is that much shorter, and its copies take no less time to arrive): us with 3, 4, 5 and 6 of them 3072 x 768 against
 // 952 columns 7.9, 7.6, 7.9, 8.1; 1824 x 2048 against 704 13.1, 11.8, 12.2, 12.4; 6144 x 4096 against 424 24.6, 21.5, -, 21.9.
-// (256 x 64 tiles are no faster with four.)
 using SmallCfg = TileCfgT<2, 2, 2, 4>;
 // 192 x 128 tiles, four waves (wave tile 96 x 64), four stage buffers: products that these cover in one round of the compute units and 128 x 128
 // tiles do not (takes_lower)
@@ -1158,7 +1165,8 @@ struct PieceCost { double call_us, stage_us, split_us, piece_us, partial_us, ope
 template <typename C>
 constexpr PieceCost piece_cost(bool k_strided) {
   return std::is_same<C, SmallCfg>::value ? PieceCost{4.63, 0.212, 1.86, 0.0, 0.545, 0.0, 0.025, 0.0013}
-         : std::is_same<C, SlimCfg>::value ? PieceCost{5.1, 0.37, 1.8, 0.0, 0.48, 0.113}
+         : std::is_same<C, SlimCfg>::value ? PieceCost{3.96, 0.172, 1.99, 0.0, 0.511, 0.136, 0.0, 0.0008}
+         : std::is_same<C, TallSlimCfg>::value ? PieceCost{5.1, 0.37, 1.8, 0.0, 0.48, 0.113}
          : std::is_same<C, MidCfg>::value ? PieceCost{5.6, 0.33, 2.1, 0.1, 0.45, 0.0}
          : std::is_same<C, SquareCfg>::value ? PieceCost{7.3, 0.40, 1.15, 0.0, 0.40, 0.0}
          : k_strided ? PieceCost{7.1, 0.55, 1.15, 0.0, 0.42, 0.0} : PieceCost{6.9, 0.50, 3.3, 0.0, 0.385, 0.0};
@@ -1185,6 +1193,11 @@ Pieces choose_pieces(int64_t n_sparse, int64_t k, int64_t n_dense, int64_t works
     if (us(p) < best.us) best = {(int)p, us(p)};
   return best;
 }
+
+// At most 64 columns against a weight of more than 128 rows of 128 x 64 tiles, which leave no room for two pieces: from 64 stages on the 256 x 64
+// tiles, which do.  us on 128 x 64 and on 256 x 64 tiles: fp16 16416 x 8192 against 64 columns 43.3 and 38.5, 20480 x 8192 43.5 and 46.0, 16416 x 4096 23.7
+// and 25.9, fewer stages e4m3 20480 x 4096 13.9 and 20.7.
+inline bool takes_tall_slim(int64_t n_sparse, int64_t stages) { return n_sparse > 128 * SlimCfg::BI && stages >= 64; }
 
 // A k-contiguous dense operand of more than 64 columns takes 256 x 128 tiles up to 128 columns, and beyond that where they fit one
 // round of the 256 compute units: they reach twice as many of them as 256 x 256 tiles, which are then the faster ones only with
@@ -1516,8 +1529,8 @@ int launch_tiled(const void* av, const void* am, int64_t n_sparse, int64_t k, co
 // Up to 16 columns, and from kFewPanels panels on up to 32: spmm_few.  Others (spmm_narrow): a block owns 16 rows, its up to four waves each take a
 // share of the k range, read their dense fragments, NB of 16 columns, from global memory (64 contiguous bytes from
 // each of the 16 dense rows, twice) and meet in LDS at the end (added in wave order).  Bound by latency, a few loads deep, at
-// short k and by the requests of the dense fragments at long k: 3072 x 768 bf16 against 37 columns 8.9 us on 256 x 64 tiles,
-// of which there are 12, and 5.4 us here.
+// short k and by the requests of the dense fragments at long k: 3072 x 768 bf16 against 37 columns 5.7 us on 128 x 64 tiles,
+// of which there are 24, and 5.0 us here.
 // ------------------------------------------------------------------------------------------
 constexpr int kNarrowWaves = 4;
 // us on spmm_narrow and on spmm_few, 24 columns fp16: 2048 x 512 (8 panels) 3.7 and 3.8, 640 x 640 3.8 and 4.1, 3072 x 768 4.4 and 4.1, 1600 x 1600 6.0 and 4.8
@@ -1792,23 +1805,21 @@ inline int few_waves(int64_t blocks, int64_t npanels, int64_t n_dense) {
   return waves;
 }
 
-// Up to how many dense columns the narrow kernels are the faster ones; us on float16 operands, tiled -> narrow:
-// 16 on spmm_few up to 128 panels (9 and 16 columns of 4096 x 8192 14.9 -> 9.9 and 15.0 -> 11.0, of 6144 x 6144 15.0 -> 12.2 and 14.1, of 1600 x 6400
-// 12.3 -> 7.8 and 11.5 -> 9.2) and some further where there are rows for k pieces of the tiled kernel to be small, but not many (of
-// 4096 x 11008 17.3 -> 13.0 and 17.4 -> 14.7, of 2048 x 11008 14.3 -> 13.0 with 16); beyond, nine or ten from 512 row blocks on (9 and 16 of 8192 x 16384
-// 31.3 -> 30.3 and 31.2 -> 34.7, of 11008 x 16384 42.4 -> 40.3 and 42.7 -> 48.4, but 16 of 768 x 11008 11.8 -> 12.5 and of 512 x 16384 13.4 -> 15.7).
-// 17 to 32 on spmm_few as well, which reads them once for every row block: up to 32 panels (24 of 10240 x 2048 13.3 -> 10.3, 32 of 16384 x 1024
-// 11.8 -> 8.3, but of 20480 x 2048 17.0 -> 21.4), of 8-bit values from 512 row blocks on up to 16, which have twice the metadata (11008 x 2048 9.8 -> 8.3, but
-// 11008 x 4096 14.3 -> 16.5); 64 up to two blocks to a compute unit (24 of 6144 x 4096 13.1 -> 12.2, 32 of 8192 x 4096 15.2 -> 13.7, of 256 x 4096 8.4 -> 7.5,
-// but of 11008 x 4096 17.2 -> 19) and 128 with neither more than one nor few (32 of 4096 x 8192 15.0 -> 14.7, of 1600 x 6400 12.4 -> 12.0, but of
-// 512 x 8192 10.5 -> 12.5; 24 of 4096 x 11008 17.5 -> 17.8).  33 to 64 on spmm_narrow, whose fragments cost requests with every panel of every
-// block: 64 of 4096 x 1536 13.5 -> 9.4, of 2304 x 768 9.0 -> 6.5, but of 2304 x 2048 10.7 -> 11.2.  With two blocks to a compute unit (6144 rows):
-// 48 of k = 768 9.0 -> 8.0 and of 1536 13.7 -> 12.5, 64 of k = 768 9.1 -> 9.6.
+// Up to how many dense columns the narrow kernels are the faster ones; of 200 products, us narrow and on 128 x 64 tiles (float16 if not said otherwise):
+// 9 to 16 on spmm_few up to 128 panels (16 columns of 5120 x 1280 6.0 and 7.2, of 2560 x 2304 6.0 and 7.9, of 4096 x 4096 e4m3 7.3 and 9.7, of
+// 3168 x 5504 9.3 and 10.0), 72 where fewer than 96 row blocks leave compute units without one (of 1888 x 4352 7.3 and 8.4, but of 736 x 5120 8.7 and 8.1), and some
+// further with neither many nor few (of 4096 x 11008 14.6 and 14.8).
+// 17 to 32, whose fragments cost requests with every panel of every block, up to 64 panels and one block to a compute unit (24 of 4096 x 4096 8.6 and
+// 9.5, 32 of 4096 x 1792 5.6 and 8.7, of 1024 x 4096 7.9 and 7.7; with more panels 24 of 1600 x 6400 10.9 and 8.9, 32 of 4096 x 8192 14.7 and 13.1), with
+// two blocks 32 panels, of 8-bit values, which have twice the metadata, 16 (24 of 6048 x 2112 8.6 and 9.3, 32 of 5120 x 1280 7.6 and 7.3, but of 6144 x 4096
+// 13.5 and 10.8, of 5696 x 2816 e4m3 9.2 and 8.0); with more blocks none (32 of 9824 x 448 6.0 and 5.0, of 14688 x 1856 12.5 and 9.1).
+// 33 to 48 on spmm_narrow up to 24 panels and one block (40 of 2304 x 768 4.9 and 5.7, 48 of 960 x 1472 7.5 and 7.7, but of 4320 x 1216 11.1 and 7.1); to 64 up
+// to nine panels (64 of 1088 x 320 5.1 and 5.0, but of 2304 x 768 6.0 and 5.8, of 3840 x 1280 9.1 and 7.4).  A weight of less than 64 rows takes no tiles.
 inline int64_t narrow_columns(int64_t n_sparse, int64_t npanels, bool eight_bit) {
   const int64_t blocks = n_sparse / 16;
-  if (blocks <= 512 && npanels <= 24) return blocks <= 256 ? 64 : 48;
-  if ((blocks <= 1024 && npanels <= (eight_bit && blocks > 512 ? 16 : 32)) || (blocks <= 512 && npanels <= 64) || (blocks >= 96 && blocks <= 256 && npanels <= 128)) return 32;
-  if (npanels <= 128 || (blocks >= 96 && blocks <= 256 && npanels <= 192)) return 16;
+  if (blocks <= 256 && npanels <= 24) return npanels <= 9 || n_sparse < 64 ? 64 : 48;
+  if (npanels <= (blocks <= 256 ? 64 : blocks > 512 ? 0 : eight_bit ? 16 : 32)) return 32;
+  if (npanels <= (blocks < 96 ? 72 : blocks <= 256 ? 192 : 128)) return 16;
   return blocks >= 512 ? 10 : 8;
 }
 
@@ -1877,8 +1888,9 @@ int dispatch_out(int out_dtype, const void* av, const void* am, int a_layout, in
   // the tiled kernel reads a k-strided dense operand through transposing LDS reads (16-bit types only)
   // (also for a narrow dense operand: with its k pieces the tiled kernel beats the general one from 8 columns on)
   const bool tiled = panel && (b_layout == TF24_ROW_MAJOR || sizeof(T) == 2) && n_sparse >= 64;
-  // up to 64 dense columns: the tiled kernel on 256 x 64 tiles; more: 128 x 128 (takes_small), 192 x 128 (takes_lower), 256 x 128 or 256 x 256 tiles (takes_mid)
+  // up to 64 dense columns: the tiled kernel on 128 x 64 tiles (or 256 x 64: takes_tall_slim); more: 128 x 128 (takes_small), 192 x 128 (takes_lower), 256 x 128 or 256 x 256 tiles (takes_mid)
   const bool slim = tiled && b_layout == TF24_ROW_MAJOR && n_dense <= SlimCfg::BJ;
+  const bool tall_slim = slim && takes_tall_slim(n_sparse, k * (int64_t)sizeof(T) / SlimCfg::KB);
   const bool small = tiled && b_layout == TF24_ROW_MAJOR && takes_small<T>(n_sparse, k, n_dense, workspace ? workspace_bytes : 0);
   const bool lower = tiled && b_layout == TF24_ROW_MAJOR && takes_lower<T>(n_sparse, k, n_dense, workspace ? workspace_bytes : 0);
   const bool mid = tiled && b_layout == TF24_ROW_MAJOR && takes_mid<T>(n_sparse, k, n_dense, workspace ? workspace_bytes : 0);
@@ -1888,6 +1900,7 @@ int dispatch_out(int out_dtype, const void* av, const void* am, int a_layout, in
                       (n_dense <= narrow_columns(n_sparse, k * (int64_t)sizeof(T) / 128, sizeof(T) == 1) || (n_dense <= 16 && !(slim && workspace)));
   if constexpr (std::is_same<T, i8_t>::value) {        // integer product: int32 accumulators, results and bias
     if (narrow) return launch_narrow<T, int32_t>(av, am, n_sparse, k, b, ldb, n_dense, c, c_layout, ldc, bias, scale, act, s);
+    if (tall_slim) return launch_tiled<T, int32_t, TallSlimCfg>(av, am, n_sparse, k, b, b_layout, ldb, n_dense, c, c_layout, ldc, bias, scale, act, workspace, workspace_bytes, s);
     if (slim) return launch_tiled<T, int32_t, SlimCfg>(av, am, n_sparse, k, b, b_layout, ldb, n_dense, c, c_layout, ldc, bias, scale, act, workspace, workspace_bytes, s);
     if (small) return launch_tiled<T, int32_t, SmallCfg>(av, am, n_sparse, k, b, b_layout, ldb, n_dense, c, c_layout, ldc, bias, scale, act, workspace, workspace_bytes, s);
     if (lower) return launch_tiled<T, int32_t, LowerCfg>(av, am, n_sparse, k, b, b_layout, ldb, n_dense, c, c_layout, ldc, bias, scale, act, workspace, workspace_bytes, s);
@@ -1900,6 +1913,13 @@ int dispatch_out(int out_dtype, const void* av, const void* am, int a_layout, in
       case TF24_F16: return launch_narrow<T, f16_t>(av, am, n_sparse, k, b, ldb, n_dense, c, c_layout, ldc, bias, scale, act, s);
       case TF24_BF16: return launch_narrow<T, bf16_t>(av, am, n_sparse, k, b, ldb, n_dense, c, c_layout, ldc, bias, scale, act, s);
       case TF24_F32: return launch_narrow<T, float>(av, am, n_sparse, k, b, ldb, n_dense, c, c_layout, ldc, bias, scale, act, s);
+    }
+  }
+  if (tall_slim) {
+    switch (out_dtype) {
+      case TF24_F16: return launch_tiled<T, f16_t, TallSlimCfg>(av, am, n_sparse, k, b, b_layout, ldb, n_dense, c, c_layout, ldc, bias, scale, act, workspace, workspace_bytes, s);
+      case TF24_BF16: return launch_tiled<T, bf16_t, TallSlimCfg>(av, am, n_sparse, k, b, b_layout, ldb, n_dense, c, c_layout, ldc, bias, scale, act, workspace, workspace_bytes, s);
+      case TF24_F32: return launch_tiled<T, float, TallSlimCfg>(av, am, n_sparse, k, b, b_layout, ldb, n_dense, c, c_layout, ldc, bias, scale, act, workspace, workspace_bytes, s);
     }
   }
   if (slim) {

@@ -240,9 +240,9 @@ def test_product_from_reference_ordered_metadata(cuda, dtype, n, k, j):
 
 @pytest.mark.parametrize("dtype,n,k,j,sparse_first", [
     (torch.float16, 96, 256, 8, False),            # one-pass kernel for a few dense columns
-    (torch.float16, 352, 640, 48, False),          # 256 x 64 tiles
-    (torch.bfloat16, 352, 640, 120, False),        # 256 x 128 tiles
-    (torch.float16, 352, 640, 296, False),         # 256 x 128 tiles, several columns of them
+    (torch.float16, 352, 640, 48, False),          # 128 x 64 tiles
+    (torch.bfloat16, 352, 640, 120, False),        # 128 x 128 tiles
+    (torch.float16, 352, 640, 296, False),         # 128 x 128 tiles, several columns of them
     (torch.float16, 768, 320, 12288, False),       # 256 x 256 tiles, one workgroup per tile
     (torch.float8_e4m3fn, 768, 640, 12288, False),
     (torch.float16, 352, 640, 296, True),          # i-major output, k strided dense operand

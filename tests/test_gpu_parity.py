@@ -971,7 +971,7 @@ def test_int8_spmm_extreme_values(cuda):
 @pytest.mark.parametrize("k", [512, 4096])
 def test_spmm_narrow_dense_operand(cuda, dtype, m, k):
     """A handful of dense columns against a tall sparse operand: 8 columns take the one-pass kernel,
-    up to 64 and up to 128 the tiled kernel on 256 x 64 and 256 x 128 tiles (with k pieces, whose
+    up to 64 and up to 128 the tiled kernel on 128 x 64 and 128 x 128 tiles (with k pieces, whose
     partial tiles only cover the live 32-column slabs); every operand position and layout."""
     import sparse
     n = 320
@@ -1276,11 +1276,15 @@ SMALL_TILES = [(64, 1, 65), (96, 2, 127), (128, 3, 128), (160, 4, 129), (288, 5,
                (1024, 12, 300), (4096, 28, 72), (2080, 27, 1900),                                # one piece of k: around the four stage buffers, and long
                (96, 29, 66), (1184, 30, 136), (672, 64, 520), (160, 77, 1345), (1600, 100, 250)]    # pieces
 LOWER_TILES = [(320, 20, 11001), (960, 21, 4208), (992, 23, 4297), (4128, 22, 1001), (11008, 20, 304), (1184, 40, 3584), (2048, 176, 2176)]    # 192 x 128
+MID_TILES = [(4128, 5, 1104), (320, 19, 11001)]                                                  # 256 x 128
+SLIM_TILES = [(4128, 1, 33), (8224, 2, 17), (8224, 3, 64), (5120, 4, 49), (8224, 5, 24), (8224, 6, 32), (8224, 7, 63), (96, 25, 49), (160, 28, 40),    # 128 x 64
+              (96, 29, 64), (1184, 67, 24), (672, 100, 33), (160, 77, 17), (64, 129, 16),          # in pieces
+              (16416, 64, 40), (16416, 66, 63)]                                                        # 256 x 64
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.float8_e4m3fn, torch.int8])
-@pytest.mark.parametrize("n,stages,rows", SMALL_TILES + LOWER_TILES)
-def test_tiles_of_128_columns(cuda, dtype, n, stages, rows):
+@pytest.mark.parametrize("n,stages,rows", SMALL_TILES + LOWER_TILES + MID_TILES + SLIM_TILES)
+def test_tiles_of_64_and_128_columns(cuda, dtype, n, stages, rows):
     """Rows and columns that do not fill their last tile, one stage and more, whole and in pieces, either order of the results, with bias
     and without: exact on small integers, the row behind the last stays as it was."""
     import sparse
@@ -1299,11 +1303,11 @@ def test_tiles_of_128_columns(cuda, dtype, n, stages, rows):
             N.check(N.lib().tf24_linear(s._store_values.data_ptr(), s._store_meta.data_ptr(), N.COMPRESSED_PANEL, code, n, k, x.data_ptr(), k, rows, y.data_ptr(),
                                         N.operand_code(out_dtype), n, None if b is None else b.data_ptr(), 1.0, N.ACT_NONE, ws.data_ptr(), ws.numel(), N.stream_ptr()))
             assert y[:rows].equal((want + (0 if b is None else b.float())).to(out_dtype)) and bool((y[rows:] == 77).all()), (out_dtype, b is None)
-    if rows % (8 if dtype == torch.float16 else 16) == 0:
-        yt = torch.full((n, rows), 77, dtype=wide, device=cuda)
+    for out_dtype in ((wide, torch.float16)[:1 + (dtype != torch.int8)] if rows % (8 if dtype == torch.float16 else 16) == 0 else ()):
+        yt = torch.full((n, rows), 77, dtype=out_dtype, device=cuda)
         N.check(N.lib().tf24_spmm(s._store_values.data_ptr(), s._store_meta.data_ptr(), N.COMPRESSED_PANEL, code, n, k, x.data_ptr(), N.ROW_MAJOR, k, rows,
-                                  yt.data_ptr(), N.operand_code(wide), N.ROW_MAJOR, rows, None, 1.0, N.ACT_NONE, ws.data_ptr(), ws.numel(), N.stream_ptr()))
-        assert yt.equal(want.t().to(wide))
+                                  yt.data_ptr(), N.operand_code(out_dtype), N.ROW_MAJOR, rows, None, 1.0, N.ACT_NONE, ws.data_ptr(), ws.numel(), N.stream_ptr()))
+        assert yt.equal(want.t().to(out_dtype)), out_dtype
 
 
 @pytest.mark.parametrize("dtype,special", [(F16, float("inf")), (BF16, float("-inf")), (E5M2, float("inf")), (E4M3, float("nan"))])

@@ -222,7 +222,7 @@ def test_parameters_that_overlap_take_turns():
 
 
 def test_pieces_of_products_with_few_columns():
-    """Pieces of k, read off the scratch that a product asks for (float32 partial tiles of 256 x 64, k-strided 256 x 256): their
+    """Pieces of k, read off the scratch that a product asks for (float32 partial tiles, 256 x 64 or two of 128 x 64, k-strided 256 x 256): their
     blocks fit one round of 256 compute units, partial tiles count for the columns that the dense operand
     reaches, and one pass over the weight asks for none."""
     from sparse import _native as N

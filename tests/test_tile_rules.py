@@ -6,7 +6,7 @@ import subprocess
 
 import pytest
 
-from test_gpu_parity import LOWER_TILES, NOT_TALL, SHORT, SMALL_TILES, SQUARE, SQUARE_STRIDED, STAGE_ORDER, TALL
+from test_gpu_parity import LOWER_TILES, MID_TILES, NOT_TALL, SHORT, SLIM_TILES, SMALL_TILES, SQUARE, SQUARE_STRIDED, STAGE_ORDER, TALL
 from test_gpu_training import MANY_LONG
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -51,6 +51,10 @@ extern "C" int lower(int64_t n_sparse, int64_t n_dense, int stages, int bytes) {
   return bytes == 1 ? tf24::takes_lower<tf24::e4m3_t>(n_sparse, (int64_t)stages * 128, n_dense, (int64_t)1 << 40)
                     : tf24::takes_lower<tf24::f16_t>(n_sparse, (int64_t)stages * 64, n_dense, (int64_t)1 << 40);
 }
+extern "C" int mid(int64_t n_sparse, int64_t n_dense, int stages) {
+  return tf24::takes_mid<tf24::f16_t>(n_sparse, (int64_t)stages * 64, n_dense, (int64_t)1 << 40);
+}
+extern "C" int64_t narrow(int64_t n_sparse, int64_t panels, int eight_bit) { return tf24::narrow_columns(n_sparse, panels, eight_bit); }
 extern "C" int rotate_from() { return tf24::kRotateMinStages; }
 """)
     subprocess.run([build.HIPCC, *build.FLAGS, "--offload-host-only", "-shared", str(src), "-o", str(lib)], check=True, capture_output=True)
@@ -61,7 +65,27 @@ extern "C" int rotate_from() { return tf24::kRotateMinStages; }
     handle.strided.argtypes = [ctypes.c_int64, ctypes.c_int64, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int]
     handle.strided_pieces.argtypes = [ctypes.c_int64, ctypes.c_int64, ctypes.c_int]
     handle.small.argtypes = handle.lower.argtypes = [ctypes.c_int64, ctypes.c_int64, ctypes.c_int, ctypes.c_int]
+    handle.mid.argtypes = [ctypes.c_int64, ctypes.c_int64, ctypes.c_int]
+    handle.narrow.argtypes = [ctypes.c_int64, ctypes.c_int64, ctypes.c_int]
+    handle.narrow.restype = ctypes.c_int64
     return handle
+
+
+@pytest.mark.parametrize("n,panels,columns,narrow", [
+    # measured apart (us on the kernels for few columns, on 128 x 64 tiles)
+    (5120, 20, 16, 1), (4096, 64, 24, 1), (4096, 28, 32, 1), (2304, 12, 40, 1), (4096, 172, 16, 1),     # 6.0 7.2, 8.6 9.5, 5.6 8.7, 4.9 5.7, 14.6 14.8
+    (736, 80, 16, 0), (1600, 100, 24, 0), (6144, 64, 32, 0), (9824, 7, 32, 0), (4320, 19, 48, 0), (3840, 20, 64, 0)])    # 8.7 8.1, 10.9 8.9, 13.5 10.8, 6.0 5.0, 11.1 7.1, 9.1 7.4
+def test_kernels_for_few_columns_where_they_are_the_faster_ones(rules, n, panels, columns, narrow):
+    assert (columns <= rules.narrow(n, panels, 0)) == narrow
+
+
+@pytest.mark.parametrize("n,stages,columns", SLIM_TILES + MID_TILES)
+def test_products_tested_on_the_gpu_take_the_tiles_of_64_and_128_columns(rules, n, stages, columns):
+    for size in (1, 2):
+        if columns <= 64:
+            assert columns > rules.narrow(n, stages, size == 1)
+        else:
+            assert rules.mid(n, columns, stages) and not rules.small(n, columns, stages, size) and not rules.lower(n, columns, stages, size)
 
 
 @pytest.mark.parametrize("n,stages,columns,small", [
