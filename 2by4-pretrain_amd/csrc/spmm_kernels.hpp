@@ -336,12 +336,12 @@ using TiledCfg = TileCfgT<4, 2>;
 // fp16 products of 8192 x 4096 x 11008 (more on boxes with less power headroom), 2.8 to 4.6 % on the fp8 product of
 // 16384 x 8192 x 8192.  With few stages per tile the longer prologue and output pass of a
 // 4-wave workgroup cost more than that (12 stages: 8 % slower; 24: equal; 32: 0.6 to 1.3 % faster), so only chained
-// tiles of kWave4MinStages or more stages take this form.
+// tiles of kWave4MinStages or more stages take this form (256 x 192 and 384 x 192 tiles: choose_short).
 using Wave4Cfg = TileCfgT<2, 4>;
 // 256 x 192 tiles in the 4-wave form (wave tile 128 x 96): a tile costs 0.89 of a 256 x 256 one, so where the
 // narrower tiles need no more rounds of the compute units than the wide ones, every round is that much shorter
 // (W[1600, 6400] against 12288 tokens: 336 wide tiles or 448 narrow ones, two rounds either way, 147 against 165 us;
-// W[11008, 4096] against 2048 tokens alike).  Long chained tiles only, like the 4-wave form itself.
+// W[11008, 4096] against 2048 tokens alike).  Below kWave4MinStages stages choose_short decides.
 using Wave4Cfg192 = TileCfgT<2, 3>;
 // 192 x 192 tiles in the 4-wave form (wave tile 96 x 96, 144 accumulators): where rounds of the compute units fill better with
 // them (takes_square).  A stage takes 0.53 us against 0.93 of a 256 x 256 one for 0.5625 of its work, but 0.67 against 1.0 at the
@@ -376,7 +376,7 @@ static_assert(kRotateMinStages - 2 - (7 * kRotateMinStages >> 3) >= 1, "the firs
 using SlimCfg = TileCfgT<2, 1, 2, 4>;
 // 256 x 64 tiles, two waves, three stage buffers: the same for tall weights (takes_tall_slim)
 using TallSlimCfg = TileCfgT<1, 2>;
-// 256 x 128 tiles, four waves: dense operands of 65 to 128 columns
+// 256 x 128 tiles, four waves: products that these cover in one round of the compute units and the smaller tiles below do not (takes_mid)
 using MidCfg = TileCfgT<2, 2>;
 // 128 x 128 tiles, four waves (wave tile 64 x 64, 64 accumulators), where there is at most one for each compute unit (takes_small).  A product
 // of one round takes as long as its tile: prologue, stages one after the other, output pass.  Here that is 4.6 us and 0.21 to 0.3 a stage, against 5.6 and
