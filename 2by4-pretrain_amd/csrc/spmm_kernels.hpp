@@ -1501,13 +1501,18 @@ int launch_tiled(const void* av, const void* am, int64_t n_sparse, int64_t k, co
                          dim3((unsigned)(tiles_i * tiles_j + (rows.blocks() + GROUPS - 1) / GROUPS), GROUPS), dim3(C::THREADS), 0, s, (const float*)workspace, splits,
                          tiles_i, tiles_j, n_sparse, n_dense, (OutT*)c, ldc, (const OutT*)bias, scale, act, rows);
     };
-    if (jm) {
-      reduce(std::true_type{}, std::false_type{}, RowSums{});
-    } else if (!sums) {
-      reduce(std::false_type{}, std::false_type{}, RowSums{});
-    } else if constexpr (sizeof(T) == 2 && (std::is_same<C, TiledCfg>::value || SQUARE)) {
-      reduce(std::false_type{}, std::true_type{}, *sums);
-      sums->partial = nullptr;                                                    // (finished here)
+    // The row sums go with the tiles that a weight gradient takes; from any other product they come back as they are, and the caller finishes them.
+    bool added = false;
+    if constexpr (sizeof(T) == 2 && (std::is_same<C, TiledCfg>::value || SQUARE)) {
+      if (sums && !jm) {
+        reduce(std::false_type{}, std::true_type{}, *sums);
+        sums->partial = nullptr;                                                  // (finished here)
+        added = true;
+      }
+    }
+    if (!added) {
+      if (jm) reduce(std::true_type{}, std::false_type{}, RowSums{});
+      else reduce(std::false_type{}, std::false_type{}, RowSums{});
     }
   }
   return check_launch("tf24_spmm");
