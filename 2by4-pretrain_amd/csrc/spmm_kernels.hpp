@@ -1648,7 +1648,7 @@ spmm_narrow(const uint8_t* __restrict__ a_values, const uint8_t* __restrict__ a_
 // end (added in wave order).  Bound by the one pass over the compressed operand (50.7 MB of fp16 11008 x 4096, 7.9 us at the rate of a copy) and
 // what a launch, its first loads and its last store take beside it (768 x 768: 2.8 us).  A wave keeps two chunks of 8 panels in flight, in
 // registers; nothing it loads comes from the dense operand but each of the columns there are once, 1 KB a chunk, handed to the fragments
-// through LDS of its own (no barrier: the LDS accesses of a wave execute in order).  Read as fragments from memory the dense operand costs
+// through LDS of its own (no barrier: wave_lds_fence).  Read as fragments from memory the dense operand costs
 // twice the sparse one's requests, and a compute unit takes 64 bytes of them a clock; shared by the waves of a block, 16 panels between two
 // barriers, it leaves a third of the compute units without a block.  The metadata of two panels are one load of a word per lane,
 // brought to their lanes by swaps of rows.  Adjacent row blocks, which share the lines of their metadata, are dealt to the same XCD.
@@ -1715,11 +1715,13 @@ spmm_few(const uint8_t* __restrict__ a_values, const uint8_t* __restrict__ a_met
       if (j * COLS < n_dense) breg[j] = *reinterpret_cast<const int4v*>(b + (COLS == 1 ? j : min((int64_t)(j * COLS + b_col), n_dense - 1)) * ldb_bytes + at);
   };
   auto store_b = [&]() __attribute__((always_inline)) {
+    wave_lds_fence();                                 // behind the reads of the chunk before
 #pragma unroll
     for (int j = 0; j < LOADS; j++) {
       const int col = j * COLS + b_col;
       if (j * COLS < n_dense) *reinterpret_cast<int4v*>(sb + (b_panel * NC + col) * 128 + ((b_piece ^ ((col >> 1) & 7)) * 16)) = breg[j];
     }
+    wave_lds_fence();
   };
   auto index_of = [&](int set, int u) __attribute__((always_inline)) {
     if constexpr (PAIR) {

@@ -97,3 +97,33 @@ def test_compression_by_magnitude_streams_its_loads_only(tmp_path):
         loads, stores = re.findall(r"global_load_dwordx4.*", body), re.findall(r"global_store_dwordx2.*", body)
         assert loads and all(line.endswith(" nt") for line in loads), (kernel, loads)
         assert stores and not any(line.endswith(" nt") for line in stores), (kernel, stores)
+
+
+@pytest.mark.parametrize("columns,waves", [(8, 2), (16, 4), (32, 8)])
+def test_lanes_that_exchange_data_through_lds_are_ordered(tmp_path, columns, waves):
+    """What a wave of the kernel for few columns writes to its slice of LDS and what other lanes read there are ordered by a fence, either way
+    round, in the code as it is optimised."""
+    spec = importlib.util.spec_from_file_location("tf24_build", os.path.join(ROOT, "2by4-pretrain_amd", "build.py"))
+    build = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(build)
+    if not os.path.exists(build.HIPCC):
+        pytest.skip("no hipcc")
+    src, out = tmp_path / "few.hip", tmp_path / "few.ll"
+    src.write_text(f"""#include "spmm_kernels.hpp"
+void few() {{
+  hipLaunchKernelGGL((tf24::spmm_few<tf24::f16_t, tf24::f16_t, true, {columns}, {waves}>), dim3(1), dim3({64 * waves}), 0, 0, nullptr, nullptr, 16, 64, nullptr, 64, 1,
+                     nullptr, 16, nullptr, 1.0f, 0);
+}}
+""")
+    subprocess.run([build.HIPCC, *build.FLAGS, "--offload-device-only", "-S", "-emit-llvm", str(src), "-o", str(out)], check=True, capture_output=True)
+    last, fenced, changes = None, True, 0
+    for line in out.read_text().splitlines():
+        if "fence syncscope(\"wavefront\")" in line:
+            fenced = True
+        elif "addrspace(3)" in line and ("store <4 x i32>" in line or "load <4 x i32>" in line):       # (the partial sums are floats)
+            access = "store" if "store <4 x i32>" in line else "load"
+            if last not in (None, access):
+                assert fenced, line
+                changes += 1
+            last, fenced = access, False
+    assert changes >= 3
