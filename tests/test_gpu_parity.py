@@ -1310,6 +1310,38 @@ def test_tiles_of_64_and_128_columns(cuda, dtype, n, stages, rows):
         assert yt.equal(want.t().to(out_dtype)), out_dtype
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float8_e4m3fn, torch.int8])
+@pytest.mark.parametrize("n,stages,rows", [(64, 1, 65), (160, 4, 129), (1184, 30, 136), (672, 64, 520), (2080, 27, 1900),          # 128 x 128 tiles, whole and in pieces
+                                           (320, 20, 11001), (1184, 40, 3584),                                                  # 192 x 128
+                                           (8224, 3, 64), (96, 25, 49), (160, 28, 40), (672, 100, 33)])                         # 128 x 64
+def test_tiles_of_64_and_128_columns_with_activation(cuda, dtype, n, stages, rows):
+    """The kernels with an activation, a bias in the results' type and in float32, and as much scratch as asked for, half of it (fewer
+    pieces) and none: exact on small integers, the row behind the last stays as it was."""
+    import sparse
+    from sparse import _native as N
+    k = stages * 128 // torch.empty(0, dtype=dtype).element_size()
+    code, out_dtype = N.operand_code(dtype), torch.int32 if dtype == torch.int8 else torch.float16 if dtype == torch.float8_e4m3fn else dtype
+    g = torch.Generator(device=cuda).manual_seed(n + stages + rows)
+    s = sparse.to_sparse_semi_structured(torch.randint(-2, 3, (n, k), device=cuda, generator=g).to(torch.int8 if dtype == torch.int8 else torch.float32), dtype=dtype)
+    x = torch.randint(-2, 3, (rows, k), device=cuda, generator=g).to(dtype)
+    bias = torch.randint(-4, 5, (n,), device=cuda, generator=g)
+    want = (x.float() @ s.to_dense().float().t() + bias).clamp_min(0).to(out_dtype)                  # (whole numbers below 2**24)
+    asked = N.lib().tf24_spmm_workspace_bytes(code, n, k, rows)
+    ws = torch.empty(max(asked, 16), dtype=torch.uint8, device=cuda)
+    for b, flag in [(bias.to(out_dtype), 0)] + ([(bias.float(), N.BIAS_F32)] if out_dtype != torch.int32 else []):
+        for scratch in {asked, asked // 2 // 16 * 16, 0}:
+            y = torch.full((rows + 1, n), 77, dtype=out_dtype, device=cuda)
+            N.check(N.lib().tf24_linear(s._store_values.data_ptr(), s._store_meta.data_ptr(), N.COMPRESSED_PANEL, code, n, k, x.data_ptr(), k, rows, y.data_ptr(),
+                                        N.operand_code(out_dtype), n, b.data_ptr(), 1.0, N.ACT_RELU | flag, ws.data_ptr() if scratch else None, scratch, N.stream_ptr()))
+            assert y[:rows].equal(want) and bool((y[rows:] == 77).all()), (flag, scratch)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float8_e4m3fn])
+@pytest.mark.parametrize("n,panels", [(4096, 64), (4096, 65), (512, 32), (512, 33), (6144, 32), (8192, 16), (8192, 17)])      # shares of whole chunks (8 panels, 4 from 17 rows on), and one panel more
+def test_one_to_thirty_two_rows_at_the_edges_of_chunks(cuda, dtype, n, panels):
+    test_one_to_thirty_two_rows(cuda, dtype, n, panels)
+
+
 @pytest.mark.parametrize("dtype,special", [(F16, float("inf")), (BF16, float("-inf")), (E5M2, float("inf")), (E4M3, float("nan"))])
 @pytest.mark.parametrize("n,panels", [(768, 12), (512, 11), (256, 5), (4096, 22), (1024, 37), (8192, 17), (8224, 3), (10240, 43)])
 def test_few_dense_columns_special_values(cuda, dtype, special, n, panels):
