@@ -1531,7 +1531,7 @@ int launch_tiled(const void* av, const void* am, int64_t n_sparse, int64_t k, co
 // make NaN of an infinite activation.  The full batches are straight-line code and only the last one tests its panels,
 // which is also the faster form (with a test of zeros in every panel 1600 x 6400 fp16 against one column takes 8.5 us, with
 // a choice of the two forms in every batch 9.3, this way 7.8).
-// Up to 16 columns, and from kFewPanels panels on up to 32: spmm_few.  Others (spmm_narrow): a block owns 16 rows, its up to four waves each take a
+// Up to 32 columns mostly (takes_few): spmm_few.  Others (spmm_narrow): a block owns 16 rows, its up to four waves each take a
 // share of the k range, read their dense fragments, NB of 16 columns, from global memory (64 contiguous bytes from
 // each of the 16 dense rows, twice) and meet in LDS at the end (added in wave order).  Bound by latency, a few loads deep, at
 // short k and by the requests of the dense fragments at long k: 3072 x 768 bf16 against 37 columns 5.7 us on 128 x 64 tiles,
@@ -1547,7 +1547,7 @@ spmm_narrow(const uint8_t* __restrict__ a_values, const uint8_t* __restrict__ a_
             OutT* __restrict__ c, int64_t ldc, const OutT* __restrict__ bias, float scale, int act) {
   constexpr int KSTEP = mma16<T>::KSTEP;     // dense k per panel = per instruction
   constexpr int M_ROW = KSTEP / 8;           // metadata bytes per row per panel
-  constexpr int BATCH = NB == 2 ? 4 : 2;     // panels per load batch; two batches are in flight
+  constexpr int BATCH = NB == 1 ? 8 : NB == 2 ? 4 : 2;          // panels per load batch; two batches are in flight
   using acc_t = typename mma16<T>::acc_t;
   __shared__ acc_t s_acc[kNarrowWaves][NB][64];
   const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
@@ -1830,12 +1830,22 @@ inline int64_t narrow_columns(int64_t n_sparse, int64_t npanels, bool eight_bit)
   return blocks >= 512 ? 10 : 8;
 }
 
+// Whether so many columns (up to narrow_columns) take spmm_few.  9 to 16 of a short k do not where one block a compute unit is all there is: a wave
+// has its dense columns brought in whole chunks of 8 panels, 16 loads of which most are of no use.  us before spmm_few, on it, and on
+// spmm_narrow again, 16 columns: fp16 256 x 256 (4 panels) 2.88, 3.36, 2.88, 2144 x 256 3.13, 3.42, 3.13; e4m3 864 x 384 3.04, 3.42, 3.04; with more
+// blocks spmm_few is as fast (6016 x 256 3.7) or faster, with 8 panels alike (3.2).
+constexpr int64_t kShortPanels = 8;
+inline bool takes_few(int64_t blocks, int64_t npanels, int64_t n_dense) {
+  if (n_dense <= 16) return n_dense <= 8 || blocks > 256 || npanels >= kShortPanels;
+  return n_dense <= 32 && npanels >= kFewPanels;
+}
+
 template <typename T, typename OutT>
 int launch_narrow(const void* av, const void* am, int64_t n_sparse, int64_t k, const void* b, int64_t ldb, int64_t n_dense,
                   void* c, int c_layout, int64_t ldc, const void* bias, float scale, int act, hipStream_t s) {
   dim3 grid((unsigned)(n_sparse / 16));
   const int64_t blocks = n_sparse / 16, npanels = k * (int64_t)sizeof(T) / 128;
-  if (n_dense <= 16 || (n_dense <= 32 && npanels >= kFewPanels)) {
+  if (takes_few(blocks, npanels, n_dense)) {
     const int nw = few_waves(blocks, npanels, n_dense);
     auto go = [&](auto jmajor, auto nc, auto nwc) {
       hipLaunchKernelGGL((spmm_few<T, OutT, decltype(jmajor)::value, decltype(nc)::value, decltype(nwc)::value>), dim3((unsigned)((blocks + 7) / 8 * 8)),
@@ -1863,7 +1873,8 @@ int launch_narrow(const void* av, const void* am, int64_t n_sparse, int64_t k, c
                        (const uint8_t*)am, n_sparse, k, (const uint8_t*)b, ldb * (int64_t)sizeof(T), n_dense, (OutT*)c, ldc, (const OutT*)bias, scale, act);
   };
   auto go_nb = [&](auto jmajor) {
-    if (n_dense <= 32) go(jmajor, std::integral_constant<int, 2>{});
+    if (n_dense <= 16) go(jmajor, std::integral_constant<int, 1>{});
+    else if (n_dense <= 32) go(jmajor, std::integral_constant<int, 2>{});
     else if (n_dense <= 48) go(jmajor, std::integral_constant<int, 3>{});
     else go(jmajor, std::integral_constant<int, 4>{});
   };

@@ -1342,6 +1342,12 @@ def test_one_to_thirty_two_rows_at_the_edges_of_chunks(cuda, dtype, n, panels):
     test_one_to_thirty_two_rows(cuda, dtype, n, panels)
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float8_e4m3fn])
+@pytest.mark.parametrize("n,panels", [(32, 1), (256, 4), (2144, 5), (4096, 7), (4128, 7), (4096, 8)])
+def test_one_to_thirty_two_rows_of_a_short_k(cuda, dtype, n, panels):
+    test_one_to_thirty_two_rows(cuda, dtype, n, panels)
+
+
 @pytest.mark.parametrize("dtype,special", [(F16, float("inf")), (BF16, float("-inf")), (E5M2, float("inf")), (E4M3, float("nan"))])
 @pytest.mark.parametrize("n,panels", [(768, 12), (512, 11), (256, 5), (4096, 22), (1024, 37), (8192, 17), (8224, 3), (10240, 43)])
 def test_few_dense_columns_special_values(cuda, dtype, special, n, panels):

@@ -2,6 +2,7 @@
 import ctypes
 import importlib.util
 import os
+import re
 import subprocess
 
 import pytest
@@ -23,7 +24,7 @@ def launches(tmp_path_factory):
 #include <string>
 static std::string made;                                 // the kernels launched, one a line
 #undef hipLaunchKernelGGL
-#define hipLaunchKernelGGL(kernel, grid, block, ...) (made += std::string(#kernel) + "\\n", (void)(grid), (void)(block))
+#define hipLaunchKernelGGL(kernel, grid, block, ...) (made += std::string(#kernel) + " in " + __PRETTY_FUNCTION__ + "\\n", (void)(grid), (void)(block))
 #include "spmm_kernels.hpp"
 namespace tf24 {
 int check_launch(const char*) { return 0; }
@@ -40,6 +41,18 @@ static int with_sums(int64_t n_sparse, int64_t n_dense, int64_t stages, int b_la
 extern "C" int small_with_sums(int64_t n, int64_t j, int64_t stages, int64_t scratch) { return with_sums<tf24::SmallCfg>(n, j, stages, TF24_ROW_MAJOR, scratch); }
 extern "C" int mid_with_sums(int64_t n, int64_t j, int64_t stages, int64_t scratch) { return with_sums<tf24::MidCfg>(n, j, stages, TF24_ROW_MAJOR, scratch); }
 extern "C" int wide_with_sums(int64_t n, int64_t j, int64_t stages, int64_t scratch) { return with_sums<tf24::TiledCfg>(n, j, stages, TF24_COL_MAJOR, scratch); }
+// the product of a weight of n rows and j rows of activations (linear), its scratch as asked for
+template <typename T>
+static void linear(int64_t n, int64_t j, int64_t stages) {
+  const int64_t k = stages * 128 / (int64_t)sizeof(T);
+  tf24::dispatch_out<T>(TF24_F16, (void*)256, (void*)256, TF24_COMPRESSED_PANEL, n, k, (void*)256, TF24_ROW_MAJOR, k, j, (void*)256, TF24_COL_MAJOR, n, nullptr, 1.0f, 0, (void*)256,
+                        (int64_t)1 << 40, nullptr, nullptr);
+}
+extern "C" void product(int bytes, int64_t n, int64_t j, int64_t stages) {
+  made.clear();
+  if (bytes == 1) linear<tf24::e4m3_t>(n, j, stages);
+  else linear<tf24::f16_t>(n, j, stages);
+}
 extern "C" const char* launched() { return made.c_str(); }
 """)
     res = subprocess.run([build.HIPCC, *build.FLAGS, "--offload-host-only", "-shared", str(src), "-o", str(lib)], capture_output=True, text=True)
@@ -47,6 +60,7 @@ extern "C" const char* launched() { return made.c_str(); }
     handle = ctypes.CDLL(str(lib))
     for f in (handle.small_with_sums, handle.mid_with_sums, handle.wide_with_sums):
         f.argtypes = [ctypes.c_int64] * 4
+    handle.product.argtypes = [ctypes.c_int] + [ctypes.c_int64] * 3
     handle.launched.restype = ctypes.c_char_p
     return handle
 
@@ -61,3 +75,26 @@ def test_a_product_in_pieces_is_added_whoever_finishes_the_row_sums(launches, ti
     made = launches.launched().decode().splitlines()
     assert ["spmm_reduce_splits" in line for line in made] == ([False, True] if pieces else [False]), made
     assert finished == (pieces and tiles == "wide")
+
+
+def kernels_of(launches, size, n, columns, stages):
+    """The names of the kernels that such a product launches, tiles by their rows and columns."""
+    launches.product(size, n, columns, stages)
+    names = []
+    for line in launches.launched().decode().splitlines():
+        name = line[1:line.index("<")]
+        tile = re.search(r"\bC = (?:tf24::)?(?:\(anonymous namespace\)::)?TileCfgT<([^>]*)>", line)
+        if tile:
+            waves_j, tj, ti = [int(v) for v in tile.group(1).split(",")][:3]
+            name += f" {64 * ti}x{32 * waves_j * tj}"
+        names.append(name)
+    return names
+
+
+@pytest.mark.parametrize("size,n,panels,columns,kernel", [
+    # us before spmm_few, on it, and on spmm_narrow again
+    (2, 256, 4, 16, "spmm_narrow"), (2, 2144, 4, 16, "spmm_narrow"), (1, 864, 3, 16, "spmm_narrow"), (1, 928, 6, 16, "spmm_narrow"),      # 2.88 3.36 2.88, 3.13 3.42 3.13, 3.04 3.42 3.04, 3.14 3.49 3.15
+    (2, 4096, 7, 9, "spmm_narrow"),
+    (2, 256, 4, 8, "spmm_few"), (2, 2144, 8, 16, "spmm_few"), (2, 6016, 4, 14, "spmm_few"), (2, 4096, 28, 32, "spmm_few"), (2, 2304, 11, 32, "spmm_narrow")])
+def test_short_products_of_few_columns(launches, size, n, panels, columns, kernel):
+    assert kernels_of(launches, size, n, columns, panels) == [kernel]
