@@ -1801,14 +1801,16 @@ spmm_few(const uint8_t* __restrict__ a_values, const uint8_t* __restrict__ a_met
 }
 
 // Waves that share a row block: some 1400 to 2000 waves in all, and six panels for each of them, or two; from 17 columns on, where a wave's
-// chunks are shorter, three.  us with 2, 4 and 8, fp16, one column:
+// chunks are of four panels, so many that one chunk holds a wave's share: a second one, begun for a panel or two, costs half as much again with 16-bit values and
+// up to all of it with 8-bit ones.  us in four waves and in eight, 17 panels: fp16 3072 x 1088 against 26 columns 5.7 and 5.0, e4m3 3008 x 2176 against 30 8.7 and 5.3; 20
+// panels: e4m3 2912 x 2560 against 31 9.4 and 5.6 (before spmm_few 5.2, 5.3, 6.1).  us with 2, 4 and 8, fp16, one column:
 // 11008 x 4096 (688 row blocks) 10.6, 11.0 and 12.7; 8192 x 8192 (512) 14.0, 14.3 and 15.8; 6144 x 4096 (384) 7.9, 7.8 and 8.6;
 // 4096 x 11008 (256) 13.9, 11.4 and 11.3; 768 x 3072 (48) 4.7, 4.3 and 4.0; 3072 x 768 (192, 12 panels) 2.96, 3.03 and 3.6.  24 columns:
 // 11008 x 1024 6.7, 7.6 and 12.2; 8192 x 2048 9.4, 8.0 and 9.4; 4096 x 2048 8.0, 6.2 and 5.5; 768 x 768 against 32 5.1, 4.2 and 4.9.
 inline int few_waves(int64_t blocks, int64_t npanels, int64_t n_dense) {
   const bool many = n_dense > 16;
-  int waves = blocks <= 256 ? 8 : blocks < 512 || (many && blocks == 512) ? 4 : 2;
-  while (waves > 2 && npanels < (many ? 3 : 6) * waves) waves /= 2;
+  int waves = blocks <= 256 ? 8 : many || blocks < 512 ? 4 : 2;
+  while (waves > 2 && (many ? npanels <= 2 * waves : npanels < 6 * waves)) waves /= 2;
   return waves;
 }
 
@@ -1818,14 +1820,16 @@ inline int few_waves(int64_t blocks, int64_t npanels, int64_t n_dense) {
 // further with neither many nor few (of 4096 x 11008 14.6 and 14.8).
 // 17 to 32, whose fragments cost requests with every panel of every block, up to 64 panels and one block to a compute unit (24 of 4096 x 4096 8.6 and
 // 9.5, 32 of 4096 x 1792 5.6 and 8.7, of 1024 x 4096 7.9 and 7.7; with more panels 24 of 1600 x 6400 10.9 and 8.9, 32 of 4096 x 8192 14.7 and 13.1), with
-// two blocks 32 panels, of 8-bit values, which have twice the metadata, 16 (24 of 6048 x 2112 8.6 and 9.3, 32 of 5120 x 1280 7.6 and 7.3, but of 6144 x 4096
-// 13.5 and 10.8, of 5696 x 2816 e4m3 9.2 and 8.0); with more blocks none (32 of 9824 x 448 6.0 and 5.0, of 14688 x 1856 12.5 and 9.1).
+// two blocks 32 panels, of 8-bit values, which have twice the metadata, 16, and up to 24 columns 32 of them on spmm_narrow (24 of 6048 x 2112 8.6 and 9.3, 32 of
+// 5120 x 1280 7.6 and 7.3, but of 6144 x 4096 13.5 and 10.8; e4m3 19 of 7520 x 3840 8.9 and 11.6, 20 of 6496 x 3072 8.6 and 9.7, but 30 of 5728 x 2432 8.4 and 7.7);
+// with more blocks none (32 of 9824 x 448 6.0 and 5.0, of 14688 x 1856 12.5 and 9.1).
 // 33 to 48 on spmm_narrow up to 24 panels and one block (40 of 2304 x 768 4.9 and 5.7, 48 of 960 x 1472 7.5 and 7.7, but of 4320 x 1216 11.1 and 7.1); to 64 up
 // to nine panels (64 of 1088 x 320 5.1 and 5.0, but of 2304 x 768 6.0 and 5.8, of 3840 x 1280 9.1 and 7.4).  A weight of less than 64 rows takes no tiles.
 inline int64_t narrow_columns(int64_t n_sparse, int64_t npanels, bool eight_bit) {
   const int64_t blocks = n_sparse / 16;
   if (blocks <= 256 && npanels <= 24) return npanels <= 9 || n_sparse < 64 ? 64 : 48;
   if (npanels <= (blocks <= 256 ? 64 : blocks > 512 ? 0 : eight_bit ? 16 : 32)) return 32;
+  if (eight_bit && blocks <= 512 && npanels <= 32) return 24;
   if (npanels <= (blocks < 96 ? 72 : blocks <= 256 ? 192 : 128)) return 16;
   return blocks >= 512 ? 10 : 8;
 }
@@ -1833,11 +1837,12 @@ inline int64_t narrow_columns(int64_t n_sparse, int64_t npanels, bool eight_bit)
 // Whether so many columns (up to narrow_columns) take spmm_few.  9 to 16 of a short k do not where one block a compute unit is all there is: a wave
 // has its dense columns brought in whole chunks of 8 panels, 16 loads of which most are of no use.  us before spmm_few, on it, and on
 // spmm_narrow again, 16 columns: fp16 256 x 256 (4 panels) 2.88, 3.36, 2.88, 2144 x 256 3.13, 3.42, 3.13; e4m3 864 x 384 3.04, 3.42, 3.04; with more
-// blocks spmm_few is as fast (6016 x 256 3.7) or faster, with 8 panels alike (3.2).
+// blocks spmm_few is as fast (6016 x 256 3.7) or faster, with 8 panels alike (3.2).  17 to 32: from kFewPanels panels on, of 8-bit values against more than one
+// block a compute unit, whose share of a wave is then more than one chunk, up to 16 (24 columns of e4m3 5696 x 2816 9.2, on spmm_narrow 8.6).
 constexpr int64_t kShortPanels = 8;
-inline bool takes_few(int64_t blocks, int64_t npanels, int64_t n_dense) {
+inline bool takes_few(int64_t blocks, int64_t npanels, int64_t n_dense, bool eight_bit) {
   if (n_dense <= 16) return n_dense <= 8 || blocks > 256 || npanels >= kShortPanels;
-  return n_dense <= 32 && npanels >= kFewPanels;
+  return n_dense <= 32 && npanels >= kFewPanels && !(eight_bit && blocks > 256 && npanels > 16);
 }
 
 template <typename T, typename OutT>
@@ -1845,7 +1850,7 @@ int launch_narrow(const void* av, const void* am, int64_t n_sparse, int64_t k, c
                   void* c, int c_layout, int64_t ldc, const void* bias, float scale, int act, hipStream_t s) {
   dim3 grid((unsigned)(n_sparse / 16));
   const int64_t blocks = n_sparse / 16, npanels = k * (int64_t)sizeof(T) / 128;
-  if (takes_few(blocks, npanels, n_dense)) {
+  if (takes_few(blocks, npanels, n_dense, sizeof(T) == 1)) {
     const int nw = few_waves(blocks, npanels, n_dense);
     auto go = [&](auto jmajor, auto nc, auto nwc) {
       hipLaunchKernelGGL((spmm_few<T, OutT, decltype(jmajor)::value, decltype(nc)::value, decltype(nwc)::value>), dim3((unsigned)((blocks + 7) / 8 * 8)),

@@ -2,7 +2,6 @@
 import ctypes
 import importlib.util
 import os
-import re
 import subprocess
 
 import pytest
@@ -24,7 +23,9 @@ def launches(tmp_path_factory):
 #include <string>
 static std::string made;                                 // the kernels launched, one a line
 #undef hipLaunchKernelGGL
-#define hipLaunchKernelGGL(kernel, grid, block, ...) (made += std::string(#kernel) + " in " + __PRETTY_FUNCTION__ + "\\n", (void)(grid), (void)(block))
+struct C { static constexpr int BI = 0, BJ = 0; };        // for launches outside of a function that has tiles of that name
+#define hipLaunchKernelGGL(kernel, grid, block, ...) \\
+  (made += std::string(#kernel) + " " + std::to_string(C::BI) + "x" + std::to_string(C::BJ) + "\\n", (void)(grid), (void)(block))
 #include "spmm_kernels.hpp"
 namespace tf24 {
 int check_launch(const char*) { return 0; }
@@ -53,6 +54,7 @@ extern "C" void product(int bytes, int64_t n, int64_t j, int64_t stages) {
   if (bytes == 1) linear<tf24::e4m3_t>(n, j, stages);
   else linear<tf24::f16_t>(n, j, stages);
 }
+extern "C" int waves(int64_t blocks, int64_t panels, int64_t columns) { return tf24::few_waves(blocks, panels, columns); }
 extern "C" const char* launched() { return made.c_str(); }
 """)
     res = subprocess.run([build.HIPCC, *build.FLAGS, "--offload-host-only", "-shared", str(src), "-o", str(lib)], capture_output=True, text=True)
@@ -61,6 +63,7 @@ extern "C" const char* launched() { return made.c_str(); }
     for f in (handle.small_with_sums, handle.mid_with_sums, handle.wide_with_sums):
         f.argtypes = [ctypes.c_int64] * 4
     handle.product.argtypes = [ctypes.c_int] + [ctypes.c_int64] * 3
+    handle.waves.argtypes = [ctypes.c_int64] * 3
     handle.launched.restype = ctypes.c_char_p
     return handle
 
@@ -80,15 +83,7 @@ def test_a_product_in_pieces_is_added_whoever_finishes_the_row_sums(launches, ti
 def kernels_of(launches, size, n, columns, stages):
     """The names of the kernels that such a product launches, tiles by their rows and columns."""
     launches.product(size, n, columns, stages)
-    names = []
-    for line in launches.launched().decode().splitlines():
-        name = line[1:line.index("<")]
-        tile = re.search(r"\bC = (?:tf24::)?(?:\(anonymous namespace\)::)?TileCfgT<([^>]*)>", line)
-        if tile:
-            waves_j, tj, ti = [int(v) for v in tile.group(1).split(",")][:3]
-            name += f" {64 * ti}x{32 * waves_j * tj}"
-        names.append(name)
-    return names
+    return [line[1:line.index("<")] + line[line.rindex(" "):].replace(" 0x0", "") for line in launches.launched().decode().splitlines()]
 
 
 @pytest.mark.parametrize("size,n,panels,columns,kernel", [
@@ -98,3 +93,20 @@ def kernels_of(launches, size, n, columns, stages):
     (2, 256, 4, 8, "spmm_few"), (2, 2144, 8, 16, "spmm_few"), (2, 6016, 4, 14, "spmm_few"), (2, 4096, 28, 32, "spmm_few"), (2, 2304, 11, 32, "spmm_narrow")])
 def test_short_products_of_few_columns(launches, size, n, panels, columns, kernel):
     assert kernels_of(launches, size, n, columns, panels) == [kernel]
+
+
+@pytest.mark.parametrize("panels,columns,blocks,waves", [
+    # one chunk of four panels holds a wave's share from 17 columns on, up to the most waves
+    (12, 17, 192, 4), (16, 32, 192, 4), (17, 26, 192, 8), (23, 25, 256, 8), (24, 32, 256, 8), (64, 32, 256, 8), (17, 24, 300, 4), (32, 32, 512, 4), (12, 20, 257, 4),
+    (12, 1, 192, 2), (24, 16, 192, 4), (48, 8, 256, 8), (64, 1, 384, 4), (128, 1, 512, 2), (64, 8, 688, 2)])
+def test_waves_that_share_a_row_block(launches, panels, columns, blocks, waves):
+    assert launches.waves(blocks, panels, columns) == waves
+
+
+@pytest.mark.parametrize("n,panels,columns,kernel", [
+    # e4m3 values of more than one row block a compute unit: us on spmm_narrow and on 128 x 64 tiles
+    (7520, 30, 19, "spmm_narrow"), (6496, 24, 20, "spmm_narrow"), (5056, 32, 24, "spmm_narrow"),      # 8.9 11.6, 8.6 9.7, 9.4 9.6
+    (5728, 19, 30, "spmm_pipe 128x64"), (5728, 33, 20, "spmm_pipe 128x64"),                            # 8.4 7.7
+    (5728, 16, 30, "spmm_few"), (8224, 12, 17, "spmm_pipe 128x64"), (3008, 17, 30, "spmm_few")])
+def test_8_bit_products_of_17_to_32_columns(launches, n, panels, columns, kernel):
+    assert kernels_of(launches, 1, n, columns, panels)[0] == kernel
