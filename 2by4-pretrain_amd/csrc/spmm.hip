@@ -60,7 +60,11 @@ int64_t workspace_bytes(int64_t n_sparse, int64_t k, int64_t n_dense) {
   const int64_t strided = sizeof(T) == 2 && n_dense % 8 == 0 ? std::max(piece_bytes<T, TiledCfg>(n_sparse, k, n_dense, true),
                                                                        piece_bytes<T, SquareCfg>(n_sparse, k, n_dense, true)) : 0;
   if (n_dense <= narrow_columns(n_sparse, k * (int64_t)sizeof(T) / 128, sizeof(T) == 1)) return strided;
-  const bool tall_slim = n_dense <= SlimCfg::BJ && takes_tall_slim(n_sparse, k * (int64_t)sizeof(T) / SlimCfg::KB);
+  // (for weights of 129 to 168 rows of 128 x 64 tiles the scratch of the 256 x 64 ones from 64 stages on, also where the product is the faster in one
+  // piece of the former and leaves it alone: sizes that programs hold for a weight stay what they were)
+  const int64_t rows = (n_sparse + SlimCfg::BI - 1) / SlimCfg::BI, stages = k * (int64_t)sizeof(T) / SlimCfg::KB;
+  if (n_dense <= SlimCfg::BJ && rows > 128 && rows <= 168 && stages >= 64) return std::max(strided, piece_bytes<T, TallSlimCfg>(n_sparse, k, n_dense, false));
+  const bool tall_slim = n_dense <= SlimCfg::BJ && takes_tall_slim(n_sparse, stages, sizeof(T) == 1);
   return std::max(strided, tall_slim ? piece_bytes<T, TallSlimCfg>(n_sparse, k, n_dense, false)
                            : n_dense <= SlimCfg::BJ ? piece_bytes<T, SlimCfg>(n_sparse, k, n_dense, false)
                            : takes_small<T>(n_sparse, k, n_dense, (int64_t)1 << 40) ? piece_bytes<T, SmallCfg>(n_sparse, k, n_dense, false)

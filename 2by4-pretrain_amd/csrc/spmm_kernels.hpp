@@ -371,8 +371,8 @@ static_assert(kRotateMinStages - 2 - (7 * kRotateMinStages >> 3) >= 1, "the firs
 // pieces.  us on 256 x 64 tiles of two waves with three buffers, on these of two waves, of four, each with its best number of pieces:
 // fp16 4096 x 4096 against 64 columns 13.5, 12.1, 11.1; 8192 x 8192 against 64 23.1, 21.1, 20.8; 4096 x 11008 against 40 18.9, 16.2, 15.7;
 // 5120 x 1280 against 64 11.9, 8.9, 7.2; e4m3 4096 x 4096 against 64 11.5, 10.4, 9.6.  Of 100 products of 128 to 20480 rows, 2 to
-// 512 stages and 8 to 64 columns 97 are faster, 17 % on average over all; the others 3840 x 1280 against 8 columns 4.8 and 5.2, 11072 x 12352 against
-// 56 (87 rows of tiles: two pieces fill the units less well than five of 44 did) 38.6 and 40.2.
+// 512 stages and 8 to 64 columns 97 are faster, 17 % on average over all (3840 x 1280 against 8 columns would be 4.8 and 5.2, but takes spmm_few); of weights of
+// 85 to 98 rows of tiles some are slower, whose two pieces fill the units less well than four or five of half as many did: 11072 x 12352 against 56 38.6 and 40.2.
 using SlimCfg = TileCfgT<2, 1, 2, 4>;
 // 256 x 64 tiles, two waves, three stage buffers: the same for tall weights (takes_tall_slim)
 using TallSlimCfg = TileCfgT<1, 2>;
@@ -1194,10 +1194,24 @@ Pieces choose_pieces(int64_t n_sparse, int64_t k, int64_t n_dense, int64_t works
   return best;
 }
 
-// At most 64 columns against a weight of more than 128 rows of 128 x 64 tiles, which leave no room for two pieces: from 64 stages on the 256 x 64
-// tiles, which do.  us on 128 x 64 and on 256 x 64 tiles: fp16 16416 x 8192 against 64 columns 43.3 and 38.5, 20480 x 8192 43.5 and 46.0, 16416 x 4096 23.7
-// and 25.9, fewer stages e4m3 20480 x 4096 13.9 and 20.7.
-inline bool takes_tall_slim(int64_t n_sparse, int64_t stages) { return n_sparse > 128 * SlimCfg::BI && stages >= 64; }
+// At most 64 columns: whether 256 x 64 tiles instead of 128 x 64 ones, of which a compute unit holds two of either.  By the rows of 128 x 64 tiles there are
+// (620 products of 129 to 2112 of them and 2 to 256 stages, fp16 and e4m3; us on 128 x 64 and on 256 x 64 tiles, operands from memory):
+// 129 to 168: the former are one piece of k (two are slower throughout: 1.02 to 1.7 times), of the latter there is room for three.  That pays where k is long, the
+// longer the more of the units one piece fills: fp16 16416 x 8192 against 64 columns 43.3 and 38.5, 18880 x 14336 77.9 and 63.0, but 16416 x 4096 23.7 and 25.9,
+// 20480 x 8192 43.5 and 46.0.  (With the weight in the caches it pays some 80 stages later: e4m3 18912 x 18944 35.4 and 41.9, from memory 51.4 and 47.7.)
+// 169 to 256: 128 x 64 throughout, 1.1 to 1.5 times as fast (28544 x 4032 25.7 and 40.1).
+// 257 to 512: units with two tiles of the one kind beside units with one, or one of the other kind each: fp16 32832 x 5056 58.2 and 53.7, e4m3 34560 x 11136
+// 67.2 and 56.5, 62592 x 768 15.6 and 13.9, but under 12 stages no better (47584 x 192 5.9 and 6.5; 36128 x 576 10.2 and 9.7, from the caches 6.3 and 7.9).
+// Beyond that the rounds are full with either, and the smaller tiles are the faster ones (e4m3 by a fifth) unless the others' last round is
+// three quarters full or more and the values are of 16 bits: fp16 114976 x 320 13.4 and 11.4, 128256 x 2048 63.9 and 59.0, 247104 x 320 28.7 and 25.3.
+constexpr int64_t kTallSlimMinStages = 12;
+inline bool takes_tall_slim(int64_t n_sparse, int64_t stages, bool eight_bit) {
+  const int64_t rows = (n_sparse + SlimCfg::BI - 1) / SlimCfg::BI;
+  if (rows <= 128) return false;
+  if (rows <= 256) return rows <= 168 && stages >= 100 + (rows - 128) * 5 / 2;
+  if (rows <= 512) return stages >= kTallSlimMinStages;
+  return !eight_bit && (rows - 1) % 1024 >= 768;
+}
 
 // A k-contiguous dense operand of more than 64 columns takes 256 x 128 tiles up to 128 columns, and beyond that where they fit one
 // round of the 256 compute units: they reach twice as many of them as 256 x 256 tiles, which are then the faster ones only with
@@ -1913,7 +1927,7 @@ int dispatch_out(int out_dtype, const void* av, const void* am, int a_layout, in
   const bool tiled = panel && (b_layout == TF24_ROW_MAJOR || sizeof(T) == 2) && n_sparse >= 64;
   // up to 64 dense columns: the tiled kernel on 128 x 64 tiles (or 256 x 64: takes_tall_slim); more: 128 x 128 (takes_small), 192 x 128 (takes_lower), 256 x 128 or 256 x 256 tiles (takes_mid)
   const bool slim = tiled && b_layout == TF24_ROW_MAJOR && n_dense <= SlimCfg::BJ;
-  const bool tall_slim = slim && takes_tall_slim(n_sparse, k * (int64_t)sizeof(T) / SlimCfg::KB);
+  const bool tall_slim = slim && takes_tall_slim(n_sparse, k * (int64_t)sizeof(T) / SlimCfg::KB, sizeof(T) == 1);
   const bool small = tiled && b_layout == TF24_ROW_MAJOR && takes_small<T>(n_sparse, k, n_dense, workspace ? workspace_bytes : 0);
   const bool lower = tiled && b_layout == TF24_ROW_MAJOR && takes_lower<T>(n_sparse, k, n_dense, workspace ? workspace_bytes : 0);
   const bool mid = tiled && b_layout == TF24_ROW_MAJOR && takes_mid<T>(n_sparse, k, n_dense, workspace ? workspace_bytes : 0);

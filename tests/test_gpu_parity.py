@@ -1342,6 +1342,15 @@ def test_one_to_thirty_two_rows_at_the_edges_of_chunks(cuda, dtype, n, panels):
     test_one_to_thirty_two_rows(cuda, dtype, n, panels)
 
 
+TALL_SLIM_TILES = [(16416, 102, 40), (17440, 133, 63), (32800, 12, 33), (33056, 13, 64)]       # 256 x 64, in pieces and whole (test_launches.py)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float8_e4m3fn, torch.int8])
+@pytest.mark.parametrize("n,stages,rows", TALL_SLIM_TILES + [(98336, 1, 17), (16416, 101, 64)])
+def test_tiles_of_64_columns_of_tall_weights(cuda, dtype, n, stages, rows):
+    test_tiles_of_64_and_128_columns(cuda, dtype, n, stages, rows)
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.float8_e4m3fn])
 @pytest.mark.parametrize("n,panels", [(32, 1), (256, 4), (2144, 5), (4096, 7), (4128, 7), (4096, 8)])
 def test_one_to_thirty_two_rows_of_a_short_k(cuda, dtype, n, panels):

@@ -6,6 +6,8 @@ import subprocess
 
 import pytest
 
+from test_gpu_parity import TALL_SLIM_TILES
+
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 
@@ -110,3 +112,25 @@ def test_waves_that_share_a_row_block(launches, panels, columns, blocks, waves):
     (5728, 16, 30, "spmm_few"), (8224, 12, 17, "spmm_pipe 128x64"), (3008, 17, 30, "spmm_few")])
 def test_8_bit_products_of_17_to_32_columns(launches, n, panels, columns, kernel):
     assert kernels_of(launches, 1, n, columns, panels)[0] == kernel
+
+
+@pytest.mark.parametrize("n,stages,columns", TALL_SLIM_TILES)
+def test_products_tested_on_the_gpu_take_the_tall_tiles(launches, n, stages, columns):
+    for size in (1, 2):
+        assert kernels_of(launches, size, n, columns, stages) == ["spmm_pipe 256x64"] + ["spmm_reduce_splits 256x64"] * (n < 32768)
+
+
+@pytest.mark.parametrize("size,n,stages,tall", [
+    # us on 128 x 64 and on 256 x 64 tiles
+    (2, 16416, 64, 0), (2, 20480, 128, 0), (1, 20480, 64, 0), (2, 32000, 64, 0), (1, 28480, 65, 0), (2, 28544, 63, 0),    # 23.7 25.9, 43.5 46.0, 31.4 46.1, 25.7 40.1
+    (2, 16416, 128, 1), (2, 18880, 224, 1), (2, 16416, 102, 1), (2, 16416, 101, 0), (2, 16384, 256, 0),                  # 43.3 38.5, 77.9 63.0
+    (2, 21504, 200, 1), (2, 21536, 512, 0),                                                                              # three pieces, two
+    (2, 32832, 79, 1), (1, 34560, 87, 1), (2, 62592, 12, 1), (2, 47584, 3, 0), (2, 50304, 12, 1), (2, 65536, 11, 0),      # 58.2 53.7, 67.2 56.5, 15.6 13.9, 5.9 6.5
+    (2, 73984, 33, 0), (1, 114976, 12, 0), (2, 114976, 5, 1), (2, 128256, 32, 1), (2, 151936, 64, 0), (2, 247104, 5, 1)])  # 13.4 11.4, 63.9 59.0, 28.7 25.3
+def test_tiles_of_64_columns_of_tall_weights(launches, size, n, stages, tall):
+    made = kernels_of(launches, size, n, 64, stages)
+    assert made[0] == ("spmm_pipe 256x64" if tall else "spmm_pipe 128x64")
+    if tall and n <= 21504:
+        assert made[1:] == ["spmm_reduce_splits 256x64"]                     # in pieces, which is what these tiles are for
+    elif n >= 16416:
+        assert len(made) == 1
