@@ -1228,17 +1228,25 @@ bool takes_mid(int64_t n_sparse, int64_t k, int64_t n_dense, int64_t workspace_b
 
 // More than 64 columns (k-contiguous) take 128 x 128 tiles where one round of the compute units holds them and the estimate for them is below that of
 // the tiles above.  Of 220 products of 256 to 12288 rows, 2 to 320 stages and 72 to 4008 columns (fp16 and e4m3) 200 take them, 15 % less time
-// on average over all; the choice is 0.5 % off the better one on average, 9 % at worst but for one product.  us, then and now: fp16 768 x 768 against
+// on average over all; the choice is 0.5 % off the better one on average.  us, then and now: fp16 768 x 768 against
 // 160 columns 8.6 and 6.8, 3072 x 768 against 952 9.2 and 7.6, 1600 x 1600 against 1792 13.4 and 10.8, 4096 x 4096 against 128 16.0 and
 // 14.4, against 512 23.1 and 20.7, 6144 x 4096 against 424 28.9 and 21.5; e4m3 8192 x 8192 against 480 41.6 and 28.2.  The other way round, where
 // the operands no longer fit the caches: 5824 x 10176 against 328 47 and 63, 2048 x 20480 against 760 57 and 81.  More than one round:
 // 5120 x 1280 against 840 (280 tiles) 13.1 and 16.3 with two tiles to a unit.
+// The estimates are of operands in the caches.  From memory a stage of these tiles takes 0.4 us, whatever their number (three stages are under way, for
+// 1.2 us), so one piece of a long k is the slower way where the others' is cut: of 450 such products those above kColdPart times the others' estimate lose 8 %
+// on average over both operands from memory, the weight alone and neither; us there on the other tiles and on these fp16 1600 x 6400 against 1296 columns 33.9, 34.7,
+// 30.3 and 44.1, 38.9, 30.4, e4m3 4096 x 11008 against 457 30.7, 29.5, 25.2 and 40.5, 32.4, 27.5.  Those below it gain 4, 13 and 15 %, a sixth of them for a loss from
+// memory: 1024 x 4096 against 1455 25.2, 20.6, 20.5 and 30.5, 19.6, 19.6.
+constexpr double kColdStageUs = 0.4, kColdPart = 1.35;
 template <typename T>
 bool takes_small(int64_t n_sparse, int64_t k, int64_t n_dense, int64_t workspace_bytes) {
   if (n_dense <= SlimCfg::BJ || ((n_sparse + SmallCfg::BI - 1) / SmallCfg::BI) * ((n_dense + SmallCfg::BJ - 1) / SmallCfg::BJ) > 256) return false;
-  const double others = takes_mid<T>(n_sparse, k, n_dense, workspace_bytes) ? choose_pieces<T, MidCfg>(n_sparse, k, n_dense, workspace_bytes, false).us
-                                                                           : choose_pieces<T, TiledCfg>(n_sparse, k, n_dense, workspace_bytes, false).us;
-  return choose_pieces<T, SmallCfg>(n_sparse, k, n_dense, workspace_bytes, false).us < others;
+  const Pieces others = takes_mid<T>(n_sparse, k, n_dense, workspace_bytes) ? choose_pieces<T, MidCfg>(n_sparse, k, n_dense, workspace_bytes, false)
+                                                                           : choose_pieces<T, TiledCfg>(n_sparse, k, n_dense, workspace_bytes, false);
+  const Pieces small = choose_pieces<T, SmallCfg>(n_sparse, k, n_dense, workspace_bytes, false);
+  const double cold_us = piece_cost<SmallCfg>(false).call_us + kColdStageUs * (double)(k * (int64_t)sizeof(T) / SmallCfg::KB);
+  return small.us < others.us && !(small.count == 1 && others.count > 1 && cold_us > kColdPart * others.us);
 }
 
 // Between the two: a product whose 128 x 128 tiles are more than one round of the compute units and whose 192 x 128 ones are not takes the latter instead of

@@ -134,3 +134,11 @@ def test_tiles_of_64_columns_of_tall_weights(launches, size, n, stages, tall):
         assert made[1:] == ["spmm_reduce_splits 256x64"]                     # in pieces, which is what these tiles are for
     elif n >= 16416:
         assert len(made) == 1
+
+
+@pytest.mark.parametrize("size,n,stages,columns,tiles", [
+    # us with the operands from memory on the tiles that k is cut for, on 128 x 128 ones in one piece
+    (2, 1600, 100, 1296, "256x128"), (2, 4480, 91, 447, "256x128"), (2, 1280, 80, 1430, "256x128"), (1, 4096, 86, 457, "256x128"),      # 33.9 44.1, 31.2 42.1, 31.2 38.0, 30.7 40.5
+    (2, 1024, 64, 1696, "128x128"), (2, 4096, 64, 512, "128x128"), (2, 640, 40, 1034, "128x128"), (2, 1600, 100, 250, "128x128")])       # one piece of either, short, and cut itself
+def test_one_piece_of_a_long_k_on_128_x_128_tiles(launches, size, n, stages, columns, tiles):
+    assert kernels_of(launches, size, n, columns, stages)[0] == "spmm_pipe " + tiles
