@@ -996,7 +996,7 @@ def test_spmm_narrow_dense_operand(cuda, dtype, m, k):
 @pytest.mark.parametrize("n,k", [(320, 1024), (8192, 1408 * 2)])
 def test_spmm_16_columns_without_workspace(cuda, dtype, n, k):
     """Through the C ABI with no workspace the tiled kernel cannot cut k into pieces, and 16 dense
-    columns take the one-pass kernel (four waves that split k at 320 rows, the LDS-shared form at 8192)."""
+    columns take the one-pass kernel (spmm_few, two waves a row block)."""
     import sparse
     from sparse import _native as N
     m = 16
@@ -1023,10 +1023,9 @@ def test_spmm_16_columns_without_workspace(cuda, dtype, n, k):
 @pytest.mark.parametrize("n", [8192, 10272])
 @pytest.mark.parametrize("dtype", [F16, E4M3])
 def test_spmm_narrow_one_wave_per_block(cuda, dtype, n, panels):
-    """Many sparse rows and few dense columns: the one-pass kernel whose waves own one 16-row block each
-    and share the dense operand through LDS (two blocks per workgroup at 8192 rows, four at 10272, where
-    the last workgroup has two idle waves and 16 columns also take this kernel; fewer rows split k over
-    four waves: test_spmm_narrow_dense_operand); k not a multiple of the 16-panel chunks."""
+    """Many sparse rows and few dense columns: the one-pass kernel whose blocks own 16 rows, two waves each
+    (fewer rows: test_spmm_narrow_dense_operand), with a share of k of no or one panel, of a chunk of eight and a
+    panel more, and of one and three more."""
     import sparse
     k, m = panels * (64 if dtype == F16 else 128), 16      # 1 panel, one chunk + 1, 22 panels
     w, x = _small_ints((n, k), 131, -2, 3).to(dtype), _small_ints((m, k), 132, -2, 3).to(dtype)
@@ -1277,9 +1276,9 @@ SMALL_TILES = [(64, 1, 65), (96, 2, 127), (128, 3, 128), (160, 4, 129), (288, 5,
                (96, 29, 66), (1184, 30, 136), (672, 64, 520), (160, 77, 1345), (1600, 100, 250)]    # pieces
 LOWER_TILES = [(320, 20, 11001), (960, 21, 4208), (992, 23, 4297), (4128, 22, 1001), (11008, 20, 304), (1184, 40, 3584), (2048, 176, 2176)]    # 192 x 128
 MID_TILES = [(4128, 5, 1104), (320, 19, 11001)]                                                  # 256 x 128
-SLIM_TILES = [(4128, 1, 33), (8224, 2, 17), (8224, 3, 64), (5120, 4, 49), (8224, 5, 24), (8224, 6, 32), (8224, 7, 63), (96, 25, 49), (160, 28, 40),    # 128 x 64
+SLIM_TILES = [(4128, 1, 33), (8224, 2, 17), (8224, 3, 64), (5120, 4, 49), (8224, 5, 24), (8224, 6, 32), (8224, 7, 63), (96, 25, 49), (160, 28, 40),    # 128 x 64, whole
               (96, 29, 64), (1184, 67, 24), (672, 100, 33), (160, 77, 17), (64, 129, 16),          # in pieces
-              (16416, 64, 40), (16416, 66, 63)]                                                        # 256 x 64
+              (16416, 64, 40), (16416, 66, 63)]                                                        # whole, where only 256 x 64 tiles could be cut
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.float8_e4m3fn, torch.int8])

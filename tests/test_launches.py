@@ -6,7 +6,7 @@ import subprocess
 
 import pytest
 
-from test_gpu_parity import TALL_SLIM_TILES
+from test_gpu_parity import SLIM_TILES, TALL_SLIM_TILES
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
@@ -142,3 +142,21 @@ def test_tiles_of_64_columns_of_tall_weights(launches, size, n, stages, tall):
     (2, 1024, 64, 1696, "128x128"), (2, 4096, 64, 512, "128x128"), (2, 640, 40, 1034, "128x128"), (2, 1600, 100, 250, "128x128")])       # one piece of either, short, and cut itself
 def test_one_piece_of_a_long_k_on_128_x_128_tiles(launches, size, n, stages, columns, tiles):
     assert kernels_of(launches, size, n, columns, stages)[0] == "spmm_pipe " + tiles
+
+
+@pytest.mark.parametrize("n,stages,columns", SLIM_TILES)
+def test_products_tested_on_the_gpu_take_128_x_64_tiles_in_pieces_or_whole(launches, n, stages, columns):
+    """In pieces from 29 stages on, but the tallest weights of the list."""
+    for size in (1, 2):
+        made = kernels_of(launches, size, n, columns, stages)
+        assert made == ["spmm_pipe 128x64"] + ["spmm_reduce_splits 128x64"] * (stages >= 29 and n < 16384)
+
+
+def test_pieces_fit_one_round_of_compute_units():
+    """Read off the scratch that a product asks for, in partial tiles of the size that it takes: whole pieces, of no more tiles than there are units."""
+    from sparse import _native as N
+    for n, k, columns, rows in ((11008, 11008, 48, 128), (5120, 32768, 32, 128), (12288, 16384, 64, 128), (17408, 32768, 64, 256), (33024, 11008, 64, 256)):
+        tile, tiles = rows * 64 * 4, -(-n // rows)
+        blocks, rest = divmod(N.lib().tf24_spmm_workspace_bytes(N.E4M3, n, k, columns), tile)
+        assert rest == 0 and blocks <= 256 and blocks % tiles == 0 and blocks != tiles, (n, k)
+        assert (blocks > 0) == (n < 32768), (n, k)
