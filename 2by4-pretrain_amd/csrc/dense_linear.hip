@@ -248,7 +248,7 @@ dense_linear(const uint8_t* __restrict__ w, int64_t ldw, const uint8_t* __restri
       point_at(next_i0, next_j0);
       lim = nstages;
     }
-    for (; st < nstages; st++) {                                 // the last two stages of the last tile
+    for (; st < nstages; st++) {                                 // the last stages of the last tile
       rotate();
       mma_step(1, 0, false, 0, true, cur, 0);
       mma_step(0, 1, false, 0, true, cur, 1);
@@ -271,10 +271,12 @@ dense_linear(const uint8_t* __restrict__ w, int64_t ldw, const uint8_t* __restri
 #pragma unroll
     for (int q = 0; q < 2; q++)
       if (q * 64 + lane < 96) bias_lds[q * 64 + lane] = to_float(T{(uint16_t)bias_w[q]});
+    wave_lds_fence();
     uint8_t* stage = smem + cur + wave * SLICE;
     auto chunk_at = [](int row, int ch) { return row * 192 + (ch ^ ((row >> 2) & 3)) * 16; };
 #pragma unroll
     for (int tp = 0; tp < kFrags / 2; tp++) {                    // 32 columns (t)
+      if (tp > 0) wave_lds_fence();                              // behind the reads of the piece before
 #pragma unroll
       for (int ti = 0; ti < kFrags; ti++) {
         const float4v add = *reinterpret_cast<const float4v*>(bias_lds + ti * 16 + lq * 4);
@@ -287,6 +289,7 @@ dense_linear(const uint8_t* __restrict__ w, int64_t ldw, const uint8_t* __restri
         }
       }
       if (tp == 0 && has_next) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");     // the next tile's first two stages
+      wave_lds_fence();
 #pragma unroll
       for (int it = 0; it < 6; it++) {
         const uint32_t piece = it * 64 + lane;

@@ -45,15 +45,6 @@ __device__ __forceinline__ void wait_copies_and_barrier() {
 __device__ __forceinline__ void wait_reads_and_barrier() {
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
-// Between what the lanes of one wave write to LDS and what others of its lanes read there, either way round: no instruction, the LDS accesses of a
-// wave execute in order.  It keeps the compiler to that order, to which the accesses of one lane at different addresses have none (a scheduling barrier
-// binds the instruction scheduler, not the passes before it).
-__device__ __forceinline__ void wave_lds_fence() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // compute units of the current device (looked up once per device; the cache is a table of atomics: two threads
 // that meet on an empty entry both look the value up and store the same number)
 inline int compute_units() {

@@ -376,7 +376,8 @@ prune_compress_row_mag16_panel(const In* __restrict__ dense, int64_t ld, int64_t
     const uint32_t w = quad_bytes(mbyte);
     words[it] = w;
   }
-  // lane l' of store instruction i takes row l'/16, unit 16 i + l'%16 (LDS accesses of one wave execute in order: no barrier)
+  // lane l' of store instruction i takes row l'/16, unit 16 i + l'%16
+  wave_lds_fence();
 #pragma unroll
   for (int i = 0; i < 4; i++) {
     const int r = lane >> 4, u = 16 * i + (lane & 15);

@@ -127,8 +127,8 @@ extern "C" int tf24_linear(const void* a_values, const void* a_meta, int a_layou
                         TF24_COL_MAJOR, ldy, bias, scale, activation, workspace, workspace_bytes, stream);
 }
 
-// ---- the weight gradient of the transposable layer: MVUE24(dY^T) . X and the row sums of dY^T, three launches (conversion, product in pieces
-// of the token axis, their sum with the row sums) and one workspace.
+// ---- the weight gradient of the transposable layer: MVUE24(dY^T) . X and the row sums of dY^T, three launches and one workspace: conversion, product in
+// pieces of the token axis, their sum with the row sums; of a product in one piece the row sums are the third launch (some 4 us).
 namespace tf24 {
 namespace {
 struct GradSpace { int64_t meta, partial, pieces, pieces_bytes, total; };          // offsets behind the compressed values

@@ -509,6 +509,16 @@ __device__ __forceinline__ Pack<Out, 4> from_float4(float a0, float b0, bool fin
   return o;
 }
 
+// ---------------------------------------------------------------- LDS within a wave
+// Between what the lanes of one wave write to LDS and what others of its lanes read there, either way round: no instruction, the LDS accesses of a
+// wave execute in order.  It keeps the compiler to that order, to which the accesses of one lane at different addresses have none (a scheduling barrier
+// binds the instruction scheduler, not the passes before it).
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // ---------------------------------------------------------------- row sums
 // out[r] = sum over column blocks of partial[b * m + r], one rounding to out's type (F32 | F16 | BF16): what is left to do behind a
 // conversion that also adds the rows of its matrix, 128 columns at a time.

@@ -127,3 +127,36 @@ void few() {{
                 changes += 1
             last, fenced = access, False
     assert changes >= 3
+
+
+def test_dense_products_and_conversions_order_the_lanes_that_exchange_data_through_lds(tmp_path):
+    """The staged results of the dense product's output pass, and what the panel conversion exchanges: between writes to LDS and reads of it, either way
+    round, stands a fence or a barrier's clobber in the code as it is optimised."""
+    spec = importlib.util.spec_from_file_location("tf24_build", os.path.join(ROOT, "2by4-pretrain_amd", "build.py"))
+    build = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(build)
+    if not os.path.exists(build.HIPCC):
+        pytest.skip("no hipcc")
+    for source, wanted in (("dense_linear.hip", "dense_linear"), ("prune_compress.hip", "mag16_panel")):
+        out = tmp_path / "out.ll"
+        subprocess.run([build.HIPCC, *build.FLAGS, "--offload-device-only", "-S", "-emit-llvm", os.path.join(build.CSRC, source), "-o", str(out)], check=True, capture_output=True)
+        found, inside = 0, False
+        for line in out.read_text().splitlines():
+            label = re.match(r"(\d+):.*; preds = (.*)", line)
+            if line.startswith("define "):
+                inside, last, ordered, changes, block = wanted in line, None, True, 0, None
+            elif label:
+                if block is not None and f"%{block}" not in label.group(2).split(", "):
+                    last, ordered = None, True                               # not entered from the block above it
+                block = label.group(1)
+            elif line == "}" and inside:
+                found, inside = found + (changes > 0), False
+            elif inside and (line.lstrip().startswith("fence ") or "~{memory}" in line):
+                ordered = True
+            elif inside and "addrspace(3)" in line and (" store " in line or re.search(r" load (<\d x i\d+>|i64|i32)", line)):      # (pieces as they are stored; not the bias)
+                access = "store" if " store " in line else "load"
+                if last not in (None, access):
+                    assert ordered, (wanted, line)
+                    changes += 1
+                last, ordered = access, False
+        assert found >= 3, wanted
