@@ -1857,14 +1857,15 @@ inline int64_t narrow_columns(int64_t n_sparse, int64_t npanels, bool eight_bit)
   return blocks >= 512 ? 10 : 8;
 }
 
-// Whether so many columns (up to narrow_columns) take spmm_few.  9 to 16 of a short k do not where one block a compute unit is all there is: a wave
+// Whether so many columns (up to narrow_columns) take spmm_few.  9 to 16 of a short k do not with up to two blocks a compute unit: a wave
 // has its dense columns brought in whole chunks of 8 panels, 16 loads of which most are of no use.  us before spmm_few, on it, and on
-// spmm_narrow again, 16 columns: fp16 256 x 256 (4 panels) 2.88, 3.36, 2.88, 2144 x 256 3.13, 3.42, 3.13; e4m3 864 x 384 3.04, 3.42, 3.04; with more
-// blocks spmm_few is as fast (6016 x 256 3.7) or faster, with 8 panels alike (3.2).  17 to 32: from kFewPanels panels on, of 8-bit values against more than one
+// spmm_narrow again, 16 columns: fp16 256 x 256 (4 panels) 2.88, 3.36, 2.88, 2144 x 256 3.13, 3.42, 3.13; e4m3 864 x 384 3.04, 3.42, 3.04; with two blocks a unit
+// from memory alike (6016 x 256 3.7), from the caches 3.3, 3.7, 3.3; with more spmm_few is the faster one by a fifth, with 8 panels
+// as fast (3.2).  17 to 32: from kFewPanels panels on, of 8-bit values against more than one
 // block a compute unit, whose share of a wave is then more than one chunk, up to 16 (24 columns of e4m3 5696 x 2816 9.2, on spmm_narrow 8.6).
 constexpr int64_t kShortPanels = 8;
 inline bool takes_few(int64_t blocks, int64_t npanels, int64_t n_dense, bool eight_bit) {
-  if (n_dense <= 16) return n_dense <= 8 || blocks > 256 || npanels >= kShortPanels;
+  if (n_dense <= 16) return n_dense <= 8 || blocks > 512 || npanels >= kShortPanels;
   return n_dense <= 32 && npanels >= kFewPanels && !(eight_bit && blocks > 256 && npanels > 16);
 }
 

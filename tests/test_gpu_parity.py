@@ -1351,7 +1351,7 @@ def test_tiles_of_64_columns_of_tall_weights(cuda, dtype, n, stages, rows):
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.float8_e4m3fn])
-@pytest.mark.parametrize("n,panels", [(32, 1), (256, 4), (2144, 5), (4096, 7), (4128, 7), (4096, 8)])
+@pytest.mark.parametrize("n,panels", [(32, 1), (256, 4), (2144, 5), (4096, 7), (4128, 7), (8192, 7), (8224, 7), (4096, 8)])
 def test_one_to_thirty_two_rows_of_a_short_k(cuda, dtype, n, panels):
     test_one_to_thirty_two_rows(cuda, dtype, n, panels)
 

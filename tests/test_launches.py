@@ -91,8 +91,8 @@ def kernels_of(launches, size, n, columns, stages):
 @pytest.mark.parametrize("size,n,panels,columns,kernel", [
     # us before spmm_few, on it, and on spmm_narrow again
     (2, 256, 4, 16, "spmm_narrow"), (2, 2144, 4, 16, "spmm_narrow"), (1, 864, 3, 16, "spmm_narrow"), (1, 928, 6, 16, "spmm_narrow"),      # 2.88 3.36 2.88, 3.13 3.42 3.13, 3.04 3.42 3.04, 3.14 3.49 3.15
-    (2, 4096, 7, 9, "spmm_narrow"),
-    (2, 256, 4, 8, "spmm_few"), (2, 2144, 8, 16, "spmm_few"), (2, 6016, 4, 14, "spmm_few"), (2, 4096, 28, 32, "spmm_few"), (2, 2304, 11, 32, "spmm_narrow")])
+    (2, 4096, 7, 9, "spmm_narrow"), (2, 6016, 4, 14, "spmm_narrow"), (1, 4832, 5, 16, "spmm_narrow"),                                    # 3.3 3.7 3.3 (from the caches)
+    (2, 256, 4, 8, "spmm_few"), (2, 2144, 8, 16, "spmm_few"), (2, 8224, 4, 16, "spmm_few"), (2, 4096, 28, 32, "spmm_few"), (2, 2304, 11, 32, "spmm_narrow")])
 def test_short_products_of_few_columns(launches, size, n, panels, columns, kernel):
     assert kernels_of(launches, size, n, columns, panels) == [kernel]
 
