@@ -921,7 +921,7 @@ spmm_pipe(const uint8_t* __restrict__ a_values, const uint8_t* __restrict__ a_me
     // instruction (streaming stores: the tile is not read again by this kernel and should not
     // displace operand lines in L2).  LDS accesses of one wave execute in order, so the passes need
     // no barrier between them.  (No wave_lds_fence either: with one around every piece 256 x 192 tiles take 13 accumulator
-    // registers more, and the training step at 12288 tokens, whose products are of 12 stages, 1 % longer.)
+    // registers more, and 3072 x 768 against 12288 columns and 5120 x 1280 against 4416, of 12 and 20 stages, 1 to 3 % longer.)
     if constexpr (C_JMAJOR && sizeof(OutT) == 2) {
       uint8_t* stage = smem + cur + wave * SLICE;
       constexpr int CHUNKS = PASS_TI * 4;                       // 16-byte chunks of a row of the piece

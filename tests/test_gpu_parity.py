@@ -1350,6 +1350,15 @@ def test_tiles_of_64_columns_of_tall_weights(cuda, dtype, n, stages, rows):
     test_tiles_of_64_and_128_columns(cuda, dtype, n, stages, rows)
 
 
+MID_PIECES = [(1600, 100, 1297), (4096, 86, 457), (608, 101, 3408)]       # 256 x 128, in pieces (test_launches.py)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float8_e4m3fn, torch.int8])
+@pytest.mark.parametrize("n,stages,rows", MID_PIECES)
+def test_tiles_of_128_columns_in_pieces(cuda, dtype, n, stages, rows):
+    test_tiles_of_64_and_128_columns(cuda, dtype, n, stages, rows)
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.float8_e4m3fn])
 @pytest.mark.parametrize("n,panels", [(32, 1), (256, 4), (2144, 5), (4096, 7), (4128, 7), (8192, 7), (8224, 7), (4096, 8)])
 def test_one_to_thirty_two_rows_of_a_short_k(cuda, dtype, n, panels):

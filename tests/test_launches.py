@@ -6,7 +6,7 @@ import subprocess
 
 import pytest
 
-from test_gpu_parity import SLIM_TILES, TALL_SLIM_TILES
+from test_gpu_parity import MID_PIECES, SLIM_TILES, TALL_SLIM_TILES
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
@@ -112,6 +112,12 @@ def test_waves_that_share_a_row_block(launches, panels, columns, blocks, waves):
     (5728, 16, 30, "spmm_few"), (8224, 12, 17, "spmm_pipe 128x64"), (3008, 17, 30, "spmm_few")])
 def test_8_bit_products_of_17_to_32_columns(launches, n, panels, columns, kernel):
     assert kernels_of(launches, 1, n, columns, panels)[0] == kernel
+
+
+@pytest.mark.parametrize("n,stages,columns", MID_PIECES)
+def test_products_tested_on_the_gpu_take_256_x_128_tiles_in_pieces(launches, n, stages, columns):
+    for size in (1, 2):
+        assert kernels_of(launches, size, n, columns, stages) == ["spmm_pipe 256x128", "spmm_reduce_splits 256x128"]
 
 
 @pytest.mark.parametrize("n,stages,columns", TALL_SLIM_TILES)
