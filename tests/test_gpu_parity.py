@@ -1350,7 +1350,7 @@ def test_tiles_of_64_columns_of_tall_weights(cuda, dtype, n, stages, rows):
     test_tiles_of_64_and_128_columns(cuda, dtype, n, stages, rows)
 
 
-MID_PIECES = [(1600, 100, 1297), (4096, 86, 457), (608, 101, 3408)]       # 256 x 128, in pieces (test_launches.py)
+MID_PIECES = [(1600, 100, 1297), (4096, 86, 457), (1280, 80, 1432)]       # 256 x 128, in pieces (test_launches.py)
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.float8_e4m3fn, torch.int8])
